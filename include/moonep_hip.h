@@ -127,6 +127,17 @@ int mep_plan_warm(const int32_t* tpe_RE, const int32_t* topk_SK, int rank, int S
                   void* stream);
 
 /*
+ * mep_plan_warm for a plan that has no duplicate groups yet: dup_counts [2] comes out as
+ * zeros (what a plan is read as before mep_build_dedup has filled it), which saves its
+ * owner a launch of its own to clear two words.
+ */
+int mep_plan_fresh(const int32_t* tpe_RE, const int32_t* topk_SK, int rank, int S, int K, int E,
+                   int R, int token_padding, int NvS, int32_t* dst, int32_t* cu_seqlens,
+                   int32_t* experts_to_copy, int32_t* zero_fill, int32_t* remote_stats,
+                   int32_t* dup_counts, void* scratch, size_t scratch_bytes, const void* warm,
+                   size_t warm_bytes, void* stream);
+
+/*
  * The same planner for ranks rank0 .. rank0+nranks-1 in one launch (one GPU
  * standing in for several ranks).  topk is [nranks,S,K]; dst, cu_seqlens,
  * zero_fill and remote_stats gain a leading [nranks] dimension;
@@ -359,6 +370,16 @@ int mep_transpose_bf16(const void* src, void* dst, int batch, int rows, int cols
 int mep_swiglu_bwd(const void* dh, const void* gate_pre, const void* up_pre, const float* row_scale,
                    const int32_t* cu_seqlens, int G, void* dgate, void* dup, void* hs, float* dscale,
                    int M, int N, void* stream);
+
+/*
+ * One launch that copies up to two device ranges: `bytes` at src (16-byte aligned, a multiple
+ * of 16) and `words` 4-byte words at src_w; either may be absent (size 0).  What stages a
+ * rank's shard and its weight slots out of or into the communication buffers where a caller
+ * does not work on the views (reference moonep/api.py:815, :1094: tensor copies).  The ranges
+ * must not overlap.
+ */
+int mep_copy_shard(void* dst, const void* src, size_t bytes, void* dst_w, const void* src_w,
+                   size_t words, void* stream);
 
 #ifdef __cplusplus
 }

@@ -15,6 +15,7 @@ LIB_PATH = os.path.join(_HERE, "libmoonep_hip.so")
 
 _lock = threading.Lock()
 _lib = None
+_host = None
 
 # combine modes / dispatch flags (include/moonep_hip.h)
 COMBINE_PRIMARIES = 0
@@ -41,6 +42,7 @@ _SIGNATURES = {
     "mep_plan_scratch_bytes": (_sz, [_i, _i, _i, _i, _i]),
     "mep_plan": (_i, [_p, _p, _i, _i, _i, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _sz, _p]),
     "mep_plan_warm": (_i, [_p, _p, _i, _i, _i, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _sz, _p, _sz, _p]),
+    "mep_plan_fresh": (_i, [_p, _p, _i, _i, _i, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _sz, _p, _sz, _p]),
     "mep_plan_ranks": (_i, [_p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _sz, _p]),
     "mep_dispatch": (_i, [_p, _p, _p, _p, _p, _i64, _p, _i64, _i, _i, _i, _i, _i, _i, _i, _i,
                           C.c_uint, _p]),
@@ -55,6 +57,7 @@ _SIGNATURES = {
     "mep_prefetch_pull": (_i, [_i, C.POINTER(_p), C.POINTER(_i64), C.POINTER(_p), C.POINTER(_i64),
                                C.POINTER(_i64), _p, _i, _i, _i, _p]),
     "mep_grad_reduce": (_i, [_p, _p, _i64, _p, _i, _i, _i, _i64, C.c_uint, _p]),
+    "mep_copy_shard": (_i, [_p, _p, _sz, _p, _p, _sz, _p]),
     "mep_set_gemm_row_tile": (_i, [_i]),
     "mep_grouped_gemm_nt": (_i, [_p, _p, _p, _p, _i, _p, _p, _i, _i, _i, _i, _p]),
     "mep_grouped_swiglu_nt": (_i, [_p, _p, _p, _p, _i, _p, _p, _p, _i, _i, _i, _p]),
@@ -101,6 +104,21 @@ def lib():
                     raise RuntimeError(f"mep_init failed: {handle.mep_strerror(rc).decode()} (code {rc})")
                 _lib = handle
     return _lib
+
+
+def host():
+    """The native host side of the Buffer operators (``_host.so``, built with the library);
+    raises RuntimeError when it has not been built."""
+    global _host
+    if _host is None:
+        lib()
+        try:
+            from . import _host as module
+        except ImportError as exc:
+            raise RuntimeError(f"{_HERE}/_host.so cannot be loaded ({exc}): build it with "
+                               "`python -m moonep_amd.build`") from exc
+        _host = module
+    return _host
 
 
 def init_device() -> None:

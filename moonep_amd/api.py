@@ -58,24 +58,40 @@ import logging
 import os
 import threading
 import warnings
-import weakref
 
 import torch
 
+from . import _lib
 from .combine import launch_combine, launch_combine_prologue  # noqa: F401
 from .dispatch import (check_dispatch_inputs, launch_build_dedup, launch_dispatch,  # noqa: F401
                        launch_dispatch_epilogue)
 from .grad_reduce import launch_grad_reduce
-from .planning import (MoonEPCommPlan, allocate_launch_scratch, allocate_planning_outputs,
-                       launch_planning, launch_planning_all_ranks)
+from .planning import (MoonEPCommPlan, _check_dedup_encoding_bounds, allocate_launch_scratch,
+                       allocate_planning_outputs, launch_planning, launch_planning_all_ranks, plan_scratch)
 from .prefetch import _ELEM_TYPES, launch_prefetch
 
 logger = logging.getLogger(__name__)
 
 
 def _lib_init_device() -> None:
-    from . import _lib
     _lib.init_device()
+
+
+def _native_context(ctx: dict, comm_stream):
+    """What csrc/host.cpp keeps for a Buffer, or None where its plain case never holds: rank
+    threads that meet inside the operators, or sizes beyond the plan's encodings."""
+    world = ctx["world"]
+    if world.host_threads:
+        return None
+    try:
+        _check_dedup_encoding_bounds(ctx)
+    except AssertionError:
+        return None
+    scratch = plan_scratch(ctx)
+    keys = ("S", "H", "K", "E", "R", "NvS", "NvS_padded", "rank", "token_padding", "meta_chunk_padded", "WEIGHTS_OFF",
+            "hidden_buf", "meta_buf", "hidden_buf_local", "weights_buf_local")
+    return _lib.host().context({**{k: ctx[k] for k in keys}, "plan_scratch": scratch}, MoonEPCommPlan,
+                               world._no_map_token, comm_stream, torch.cuda.Event)
 
 
 def _align_up(x: int, alignment: int) -> int:
@@ -209,9 +225,8 @@ class EmulatedWorld:
         self.host_threads = bool(host_threads) and R > 1
         self._barrier = threading.Barrier(R) if self.host_threads else None
         self._arrived = [None] * R             # per rank: event recorded on arrival
-        # dup_counts tensors of plans without a duplicate map, by id (a tensor's == is
-        # elementwise, so a WeakSet cannot hold them)
-        self._no_dedup = weakref.WeakValueDictionary()
+        # what the dup_counts tensor of a plan without a duplicate map of this world is marked with
+        self._no_map_token = object()
 
     def matches(self, S, H, K, E, R, token_padding) -> bool:
         return (self.S, self.H, self.K, self.E, self.R, self.token_padding) == \
@@ -274,10 +289,10 @@ class EmulatedWorld:
 
     # -- plans without a duplicate map ----------------------------------------------
     def mark_no_dedup(self, plan: MoonEPCommPlan) -> None:
-        self._no_dedup[id(plan.dup_counts)] = plan.dup_counts
+        plan.dup_counts._no_dup_map_in = self._no_map_token
 
     def has_dedup(self, plan: MoonEPCommPlan) -> bool:
-        return self._no_dedup.get(id(plan.dup_counts)) is not plan.dup_counts
+        return getattr(plan.dup_counts, "_no_dup_map_in", None) is not self._no_map_token
 
 
 def _create_context(S: int, H: int, K: int, E: int, num_ep_ranks: int, num_sms=None,
@@ -364,7 +379,6 @@ def _limited_stream(device: int, num_cus: int):
     import atexit
     import ctypes
 
-    from . import _lib
     key = (int(device), int(num_cus))
     with _LIMITED_LOCK:
         if key not in _LIMITED_STREAMS:
@@ -381,7 +395,6 @@ def _limited_stream(device: int, num_cus: int):
 def _release_limited_streams() -> None:
     """Wait for the device(s) and destroy every CU-masked stream this process made.
     Runs at interpreter exit; may also be called once no Buffer with ``num_sms`` is in use."""
-    from . import _lib
     with _LIMITED_LOCK:
         streams = dict(_LIMITED_STREAMS)
         _LIMITED_STREAMS.clear()
@@ -415,12 +428,14 @@ class Buffer:
         self._limited_stream = None      # raw handle of a CU-masked comm stream, if any
         self._inflight = []              # (event, tensors) of asynchronous work on such a stream
         self._destroyed = False
+        self._native = None              # csrc/host.cpp's context: the plain case of every operator
         self._ctx = _create_context(S, H, K, E, num_ep_ranks, num_sms=num_sms,
                                     token_padding=token_padding, group=group, rank=rank,
                                     world=world)
         # default priority on purpose: mixed stream priorities are not used on this hardware
         if num_sms is None:
             self._comm_stream = torch.cuda.Stream(device=int(self._ctx["device"]))
+            self._native = _native_context(self._ctx, self._comm_stream)
         else:
             # an explicit num_sms: every kernel of this Buffer runs on that many CUs
             self._limited_stream, self._comm_stream = _limited_stream(
@@ -457,6 +472,7 @@ class Buffer:
             if world is not None:
                 world.attached -= 1
             self._ctx.clear()
+        self._native = None
         self._ctx = None
         self._comm_stream = None
         self._limited_stream = None      # the stream itself is shared (see _limited_stream)
@@ -626,6 +642,12 @@ class Buffer:
         ``topk_experts_sk[R, S, K]`` to get this rank's duplicate groups too.
         Returns ``(hidden_nvsh, route_weights_nvs, cu_seqlens, plan[, event])``.
         """
+        # a shared world takes copies only in the cases _check_copy_mode lets through
+        if self._native is not None and (zero_copy or self._ctx["world"].attached == 1):
+            res = _lib.host().dispatch(self._native, hidden_sh, route_weights_sk, topk_experts_sk, tokens_per_expert,
+                                       plan, bool(async_finish), bool(zero_copy), bool(router_weights_zero_copy))
+            if res is not None:
+                return res
         ctx = self._require_ctx()
         # the inputs are checked before any kernel (the planner's cache warming
         # included) reads them
@@ -685,6 +707,13 @@ class Buffer:
                         up_scale_prefetch_buffer=None, down_scale_prefetch_buffer=None):
         """Push this rank's expert weights selected by ``plan`` into every
         rank's prefetch slots (reference moonep/api.py:853-984)."""
+        if self._native is not None:
+            done = _lib.host().prefetch(
+                self._native, plan, bool(async_finish), local_gate_weight, local_up_weight, local_down_weight,
+                gate_prefetch_buffer, up_prefetch_buffer, down_prefetch_buffer, local_gate_scale, local_up_scale,
+                local_down_scale, gate_scale_prefetch_buffer, up_scale_prefetch_buffer, down_scale_prefetch_buffer)
+            if done is not None:
+                return done if async_finish else None
         ctx = self._require_ctx()
         assert isinstance(plan, MoonEPCommPlan), "Buffer.prefetch_weight: plan is required"
         R = int(ctx["R"])
@@ -720,6 +749,11 @@ class Buffer:
         token-major ``[S, H]``; gather the route weights back to ``[S, K]``
         (reference moonep/api.py:986-1119).
         Returns ``(hidden_sh, route_weights_sk | None, event | None)``."""
+        if self._native is not None and (zero_copy or self._ctx["world"].attached == 1):
+            res = _lib.host().combine(self._native, plan, hidden_nvsh, route_weights_nvs, bool(async_finish),
+                                      bool(zero_copy), bool(router_weights_zero_copy))
+            if res is not None:
+                return res
         ctx = self._require_ctx()
         assert isinstance(plan, MoonEPCommPlan), "Buffer.combine: plan is required"
         self._check_copy_mode(ctx, zero_copy, "combine")
@@ -773,6 +807,12 @@ class Buffer:
         "reduce" for every rank before "clear" for any -- a rank's clear wipes slots that
         hold *other* ranks' experts -- so "both" is refused there; ranks on the host
         threads of a ``host_threads`` world meet at a rendezvous between the halves."""
+        if self._native is not None and phase == "both" and \
+                (self._ctx["world"].attached == 1 or self._ctx["R"] == 1):
+            done = _lib.host().reduce_grad(self._native, plan, bool(async_finish), local_gate_grad, local_up_grad,
+                                           local_down_grad, gate_reduce_buffer, up_reduce_buffer, down_reduce_buffer)
+            if done is not None:
+                return done if async_finish else None
         ctx = self._require_ctx()
         R = int(ctx["R"])
         epn = int(ctx["E"]) // R

@@ -1,0 +1,532 @@
+// Host side of the Buffer operators: argument checks, output allocation and launches of one
+// call in native code (module moonep_amd._host).
+//
+// An operator of a small batch is bound by the host: through Python and ctypes a decode step
+// (8 tokens, dispatch + combine) took 63 us for 22 us of GPU work -- nine allocations, fifteen
+// shape checks and four launches, a microsecond or more each.  Here a plan's eight tensors are
+// views of ONE allocation, and the checks cost nanoseconds.
+//
+// Every function returns None, with nothing launched, when the call is not the plain case it
+// handles (a failed check, a world with host threads, ...): the Python body of the operator
+// then runs and raises what it always raised, or does the rarer work.
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <c10/hip/HIPStream.h>
+#include <hip/hip_runtime.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <initializer_list>
+#include <memory>
+#include <vector>
+
+#include "../../include/moonep_hip.h"
+
+namespace {
+
+struct Names {
+  PyObject *dst, *etc, *zfr, *stats, *dup_groups, *dup_loffs, *dup_counts, *N, *R, *E, *NvS, *K, *no_map, *record;
+} nm;
+
+// what a Buffer keeps from one call to the next
+struct Ctx {
+  int S, H, K, E, R, epn, NvS, rank, tp;
+  int64_t N, wslot_stride;
+  at::Tensor hidden_buf, meta_buf, hidden_local, weights_local, scratch;
+  c10::Stream comm = c10::Stream(c10::Stream::UNSAFE, c10::Device(c10::kCPU), 0);
+  hipStream_t comm_raw = nullptr;
+  hipEvent_t order = nullptr;
+  PyObject *plan_type = nullptr, *hidden_local_py = nullptr, *no_map_token = nullptr, *event_type = nullptr,
+           *comm_py = nullptr, *empty = nullptr;
+  PyObject *py_N = nullptr, *py_R = nullptr, *py_E = nullptr, *py_NvS = nullptr, *py_K = nullptr;
+  ~Ctx() {
+    for (PyObject* o : {plan_type, hidden_local_py, no_map_token, event_type, comm_py, empty, py_N, py_R, py_E,
+                        py_NvS, py_K})
+      Py_XDECREF(o);
+    if (order) (void)hipEventDestroy(order);
+  }
+};
+
+const char* kCapsule = "moonep_amd._host.Ctx";
+
+void free_ctx(PyObject* cap) { delete (Ctx*)PyCapsule_GetPointer(cap, kCapsule); }
+
+Ctx* ctx_of(PyObject* cap) { return (Ctx*)PyCapsule_GetPointer(cap, kCapsule); }
+
+// the C ABI's return code as the exception the Python binding raises
+bool failed(int rc, const char* what) {
+  if (rc == 0) return false;
+  PyErr_Format(PyExc_RuntimeError, "%s failed: %s (code %d)", what, mep_strerror(rc), rc);
+  return true;
+}
+
+const at::Tensor* tensor(PyObject* o) { return THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr; }
+
+bool is(const at::Tensor& t, at::ScalarType dt, const Ctx& c) {
+  return t.scalar_type() == dt && t.device() == c.hidden_buf.device() && t.is_contiguous();
+}
+
+bool shape(const at::Tensor& t, std::initializer_list<int64_t> s) {
+  return t.sizes() == c10::IntArrayRef(s.begin(), s.size());
+}
+
+bool aligned(const void* p) { return ((uintptr_t)p & 15) == 0; }
+
+// a dense tensor of `sizes` at element `offset` of a storage
+at::Tensor view_of(const at::Tensor& base, caffe2::TypeMeta dtype, int64_t offset, c10::IntArrayRef sizes) {
+  at::Tensor t = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(base.storage()), base.key_set(), dtype);
+  c10::TensorImpl* impl = t.unsafeGetTensorImpl();
+  impl->set_storage_offset(offset);
+  impl->set_sizes_contiguous(sizes);
+  return t;
+}
+
+PyObject* new_none() { Py_RETURN_NONE; }
+
+// ---- asynchronous calls: the work goes to the communication stream -----------------------
+struct Async {
+  Ctx& c;
+  bool on;
+  hipStream_t stream;
+  Async(Ctx& ctx, bool async) : c(ctx), on(async) {
+    if (on && !c.comm_raw) {  // asked for by the first asynchronous call: the answer makes the stream exist
+      PyObject* o = PyObject_GetAttrString(c.comm_py, "cuda_stream");
+      c.comm_raw = o ? (hipStream_t)PyLong_AsVoidPtr(o) : nullptr;
+      Py_XDECREF(o);
+    }
+    stream = on ? c.comm_raw : c10::hip::getCurrentHIPStream(c.hidden_buf.device().index()).stream();
+  }
+  // after the caller's work; the allocator must not reuse what the stream still works on
+  bool begin(std::initializer_list<const at::Tensor*> used) {
+    if (!on) return true;
+    if (PyErr_Occurred()) return false;
+    const c10::StorageImpl* seen[24];
+    int n = 0;
+    for (const at::Tensor* t : used) {
+      if (!t || !t->defined()) continue;
+      const c10::StorageImpl* s = t->storage().unsafeGetStorageImpl();
+      bool dup = false;
+      for (int i = 0; i < n; ++i) dup |= seen[i] == s;
+      if (dup) continue;
+      if (n < 24) seen[n++] = s;
+      t->record_stream(c.comm);
+    }
+    hipStream_t main = c10::hip::getCurrentHIPStream(c.hidden_buf.device().index()).stream();
+    hipError_t e = c.order ? hipSuccess : hipEventCreateWithFlags(&c.order, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipEventRecord(c.order, main);
+    if (e == hipSuccess) e = hipStreamWaitEvent(c.comm_raw, c.order, 0);
+    return !failed((int)e, "ordering the communication stream");
+  }
+  // a new reference to the completion event
+  PyObject* end() {
+    PyObject* ev = PyObject_CallNoArgs(c.event_type);
+    if (!ev) return nullptr;
+    PyObject* r = PyObject_CallMethodOneArg(ev, nm.record, c.comm_py);
+    if (!r) { Py_DECREF(ev); return nullptr; }
+    Py_DECREF(r);
+    return ev;
+  }
+};
+
+// an ordering event is shared by a Buffer's calls: under stream capture the Python body makes its own
+bool capturing(const Ctx& c) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  hipStream_t s = c10::hip::getCurrentHIPStream(c.hidden_buf.device().index()).stream();
+  return hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+}
+
+// ---- plans -------------------------------------------------------------------------------
+struct Plan {
+  at::Tensor dst, etc, zfr, stats, dup_groups, dup_loffs, dup_counts;
+};
+
+const at::Tensor* attr_tensor(PyObject* plan, PyObject* name, std::vector<PyObject*>& hold) {
+  PyObject* o = PyObject_GetAttr(plan, name);
+  if (!o) { PyErr_Clear(); return nullptr; }
+  hold.push_back(o);
+  return tensor(o);
+}
+
+bool attr_is(PyObject* plan, PyObject* name, int64_t want) {
+  PyObject* o = PyObject_GetAttr(plan, name);
+  if (!o) { PyErr_Clear(); return false; }
+  const long long v = PyLong_Check(o) ? PyLong_AsLongLong(o) : -1;
+  Py_DECREF(o);
+  if (v == -1 && PyErr_Occurred()) PyErr_Clear();
+  return v == want;
+}
+
+// the tensors of a caller's plan, checked as a dispatch checks them; false: let Python look
+bool read_plan(const Ctx& c, PyObject* plan, Plan* p) {
+  if ((PyObject*)Py_TYPE(plan) != c.plan_type) return false;
+  if (!attr_is(plan, nm.N, c.N) || !attr_is(plan, nm.R, c.R) || !attr_is(plan, nm.K, c.K) ||
+      !attr_is(plan, nm.NvS, c.NvS))
+    return false;
+  std::vector<PyObject*> hold;
+  hold.reserve(8);
+  const at::Tensor* t[7];
+  PyObject* names[7] = {nm.dst, nm.etc, nm.zfr, nm.stats, nm.dup_groups, nm.dup_loffs, nm.dup_counts};
+  bool ok = true;
+  for (int i = 0; i < 7; ++i) {
+    t[i] = attr_tensor(plan, names[i], hold);
+    ok = ok && t[i] && is(*t[i], at::kInt, c);
+  }
+  ok = ok && shape(*t[0], {c.N}) && shape(*t[1], {c.R, c.epn}) && shape(*t[2], {2 * c.epn, 2}) &&
+       shape(*t[3], {2}) && shape(*t[4], {c.NvS, 3}) && shape(*t[5], {c.NvS}) && shape(*t[6], {2});
+  if (ok) *p = Plan{*t[0], *t[1], *t[2], *t[3], *t[4], *t[5], *t[6]};
+  for (PyObject* o : hold) Py_DECREF(o);
+  return ok;
+}
+
+// a MoonEPCommPlan whose tensors are already known to be right (its __post_init__ checks nothing new)
+PyObject* wrap_plan(const Ctx& c, const Plan& p) {
+  PyTypeObject* type = (PyTypeObject*)c.plan_type;
+  PyObject* plan = type->tp_new(type, c.empty, nullptr);
+  if (!plan) return nullptr;
+  auto set = [&](PyObject* name, PyObject* value, bool own) {  // the slots themselves: the class is frozen
+    const int rc = value ? PyObject_GenericSetAttr(plan, name, value) : -1;
+    if (own) Py_XDECREF(value);
+    return rc == 0;
+  };
+  PyObject* counts = THPVariable_Wrap(p.dup_counts);
+  bool ok = counts != nullptr;
+  // the other ranks' routing is unknown: the plan has no duplicate map of this world
+  if (ok && c.R > 1) ok = PyObject_SetAttr(counts, nm.no_map, c.no_map_token) == 0;
+  ok = ok && set(nm.dst, THPVariable_Wrap(p.dst), true) && set(nm.etc, THPVariable_Wrap(p.etc), true) &&
+       set(nm.zfr, THPVariable_Wrap(p.zfr), true) && set(nm.stats, THPVariable_Wrap(p.stats), true) &&
+       set(nm.dup_groups, THPVariable_Wrap(p.dup_groups), true) &&
+       set(nm.dup_loffs, THPVariable_Wrap(p.dup_loffs), true) && set(nm.dup_counts, counts, false) &&
+       set(nm.N, c.py_N, false) && set(nm.R, c.py_R, false) && set(nm.E, c.py_E, false) &&
+       set(nm.NvS, c.py_NvS, false) && set(nm.K, c.py_K, false);
+  Py_XDECREF(counts);
+  if (!ok) { Py_DECREF(plan); return nullptr; }
+  return plan;
+}
+
+// every tensor of a fresh plan and its cu_seqlens as views of one block (64-byte starts)
+at::Tensor new_plan(const Ctx& c, Plan* p, at::Tensor* cu) {
+  int64_t at_int = 0;
+  auto take = [&](int64_t n) { const int64_t o = at_int; at_int += (n + 15) & ~(int64_t)15; return o; };
+  const int64_t o_dst = take(c.N), o_cu = take(2 * c.epn), o_etc = take((int64_t)c.R * c.epn),
+                o_zfr = take(4 * c.epn), o_stats = take(2), o_counts = take(2), o_groups = take(3 * (int64_t)c.NvS),
+                o_loffs = take(c.NvS);
+  at::Tensor block = at::empty({at_int}, c.meta_buf.options());
+  auto v = [&](int64_t o, std::initializer_list<int64_t> s) {
+    return view_of(block, block.dtype(), o, c10::IntArrayRef(s.begin(), s.size()));
+  };
+  *p = Plan{v(o_dst, {c.N}), v(o_etc, {c.R, c.epn}), v(o_zfr, {2 * c.epn, 2}), v(o_stats, {2}),
+            v(o_groups, {c.NvS, 3}), v(o_loffs, {c.NvS}), v(o_counts, {2})};
+  *cu = v(o_cu, {2 * c.epn});
+  return block;
+}
+
+template <class T>
+T* ptr(const at::Tensor& t) { return t.defined() ? (T*)t.data_ptr() : nullptr; }
+
+// ---- dispatch(ctx, hidden, weights, topk, tpe, plan, async, zero_copy, weights_zero_copy) ----
+PyObject* py_dispatch(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 9) { PyErr_SetString(PyExc_TypeError, "dispatch takes 9 arguments"); return nullptr; }
+  Ctx* cp = ctx_of(args[0]);
+  if (!cp) return nullptr;
+  Ctx& c = *cp;
+  const at::Tensor* hidden = tensor(args[1]);
+  const at::Tensor* w = args[2] == Py_None ? nullptr : tensor(args[2]);
+  if (!hidden || !is(*hidden, at::kBFloat16, c) || !shape(*hidden, {c.S, c.H}) || !aligned(hidden->data_ptr()))
+    return new_none();
+  if (args[2] != Py_None && (!w || !is(*w, at::kFloat, c) || !shape(*w, {c.S, c.K}))) return new_none();
+  const bool async = args[6] == Py_True, zero_copy = args[7] == Py_True, w_zero_copy = args[8] == Py_True;
+  if (async && capturing(c)) return new_none();
+  const bool fresh = args[5] == Py_None;
+  const at::Tensor *topk = nullptr, *tpe = nullptr;
+  Plan plan;
+  at::Tensor cu;
+  if (fresh) {
+    topk = tensor(args[3]);
+    tpe = tensor(args[4]);
+    if (!topk || !is(*topk, at::kInt, c) || topk->dim() == 3 || topk->numel() != c.N) return new_none();
+    if (!tpe || !is(*tpe, at::kInt, c) || tpe->dim() != 2 || !shape(*tpe, {c.R, c.E})) return new_none();
+    new_plan(c, &plan, &cu);
+  } else if (!read_plan(c, args[5], &plan)) {
+    return new_none();
+  }
+  at::Tensor out = zero_copy ? c.hidden_local : at::empty({c.NvS, c.H}, c.hidden_buf.options());
+  at::Tensor w_local = view_of(c.weights_local, caffe2::TypeMeta::Make<float>(), c.weights_local.storage_offset(), {c.NvS});
+  at::Tensor w_out;
+  if (w) w_out = w_zero_copy ? w_local : at::empty({c.NvS}, c.hidden_buf.options().dtype(at::kFloat));
+
+  Async as(c, async);
+  if (!as.begin({hidden, w, &out, &w_out, &plan.dst, &plan.etc, &plan.zfr, &plan.stats, &plan.dup_groups,
+                 &plan.dup_loffs, &plan.dup_counts, topk, tpe, &cu}))
+    return nullptr;
+  if (fresh) {
+    const int rc = mep_plan_fresh(ptr<int>(*tpe), ptr<int>(*topk), c.rank, c.S, c.K, c.E, c.R, c.tp, c.NvS,
+                                  ptr<int>(plan.dst), ptr<int>(cu), ptr<int>(plan.etc), ptr<int>(plan.zfr),
+                                  ptr<int>(plan.stats), ptr<int>(plan.dup_counts), ptr<void>(c.scratch),
+                                  c.scratch.defined() ? c.scratch.nbytes() : 0, hidden->data_ptr(),
+                                  hidden->nbytes(), as.stream);
+    if (failed(rc, "mep_plan")) return nullptr;
+  }
+  int rc = mep_dispatch(hidden->data_ptr(), w ? ptr<float>(*w) : nullptr, ptr<int>(plan.dst), ptr<int>(plan.zfr),
+                        c.hidden_buf.data_ptr(), c.NvS, w ? ptr<float>(c.meta_buf) : nullptr, c.wslot_stride,
+                        c.rank, c.S, c.H, c.K, c.R, c.epn, c.NvS, c.tp, MEP_DISPATCH_WRITE_DUPS, as.stream);
+  if (failed(rc, "mep_dispatch")) return nullptr;
+  const bool copy_w = w && !w_zero_copy;
+  if (!zero_copy || copy_w) {
+    rc = mep_copy_shard(zero_copy ? nullptr : out.data_ptr(), zero_copy ? nullptr : c.hidden_local.data_ptr(),
+                        zero_copy ? 0 : out.nbytes(), copy_w ? w_out.data_ptr() : nullptr,
+                        copy_w ? w_local.data_ptr() : nullptr, copy_w ? (size_t)c.NvS : 0, as.stream);
+    if (failed(rc, "mep_copy_shard")) return nullptr;
+  }
+  PyObject* event = nullptr;
+  if (async && !(event = as.end())) return nullptr;
+  PyObject* res = PyTuple_New(async ? 5 : 4);
+  PyObject* py_out;
+  if (zero_copy) { py_out = c.hidden_local_py; Py_INCREF(py_out); }
+  else py_out = THPVariable_Wrap(out);
+  PyObject* py_plan;
+  if (fresh) py_plan = wrap_plan(c, plan);
+  else { py_plan = args[5]; Py_INCREF(py_plan); }
+  if (!res || !py_out || !py_plan) { Py_XDECREF(res); Py_XDECREF(py_out); Py_XDECREF(py_plan); Py_XDECREF(event); return nullptr; }
+  PyTuple_SET_ITEM(res, 0, py_out);
+  PyTuple_SET_ITEM(res, 1, w ? THPVariable_Wrap(w_out) : new_none());
+  PyTuple_SET_ITEM(res, 2, fresh ? THPVariable_Wrap(cu) : new_none());
+  PyTuple_SET_ITEM(res, 3, py_plan);
+  if (async) PyTuple_SET_ITEM(res, 4, event);
+  return res;
+  END_HANDLE_TH_ERRORS
+}
+
+// ---- combine(ctx, plan, hidden, weights, async, zero_copy, weights_zero_copy) ----------------
+PyObject* py_combine(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 7) { PyErr_SetString(PyExc_TypeError, "combine takes 7 arguments"); return nullptr; }
+  Ctx* cp = ctx_of(args[0]);
+  if (!cp) return nullptr;
+  Ctx& c = *cp;
+  Plan plan;
+  const at::Tensor* hidden = tensor(args[2]);
+  const at::Tensor* w = args[3] == Py_None ? nullptr : tensor(args[3]);
+  if (!read_plan(c, args[1], &plan)) return new_none();
+  if (!hidden || !is(*hidden, at::kBFloat16, c) || !shape(*hidden, {c.NvS, c.H}) || !aligned(hidden->data_ptr()))
+    return new_none();
+  if (args[3] != Py_None && (!w || !is(*w, at::kFloat, c) || !shape(*w, {c.NvS}))) return new_none();
+  const bool async = args[4] == Py_True, zero_copy = args[5] == Py_True, w_zero_copy = args[6] == Py_True;
+  const bool copy_h = hidden->data_ptr() != c.hidden_local.data_ptr();
+  const bool copy_w = w && w->data_ptr() != c.weights_local.data_ptr();
+  if ((zero_copy && copy_h) || (w_zero_copy && copy_w)) return new_none();
+  if (async && capturing(c)) return new_none();
+  at::Tensor out = at::empty({c.S, c.H}, c.hidden_buf.options());
+  at::Tensor out_w;
+  if (w) out_w = at::empty({c.S, c.K}, c.hidden_buf.options().dtype(at::kFloat));
+  Async as(c, async);
+  if (!as.begin({&out, &plan.dst, &plan.etc, &plan.zfr, &plan.stats, &plan.dup_groups, &plan.dup_loffs,
+                 &plan.dup_counts, hidden, w, &out_w}))
+    return nullptr;
+  int rc;
+  if (copy_h || copy_w) {
+    rc = mep_copy_shard(copy_h ? c.hidden_local.data_ptr() : nullptr, copy_h ? hidden->data_ptr() : nullptr,
+                        copy_h ? hidden->nbytes() : 0, copy_w ? c.weights_local.data_ptr() : nullptr,
+                        copy_w ? w->data_ptr() : nullptr, copy_w ? (size_t)c.NvS : 0, as.stream);
+    if (failed(rc, "mep_copy_shard")) return nullptr;
+  }
+  rc = mep_combine(c.hidden_buf.data_ptr(), c.NvS, w ? ptr<float>(c.meta_buf) : nullptr, c.wslot_stride,
+                   ptr<int>(plan.dst), out.data_ptr(), w ? ptr<float>(out_w) : nullptr, c.S, c.H, c.K, c.R, c.NvS,
+                   MEP_COMBINE_TWO_LEVEL, as.stream);
+  if (failed(rc, "mep_combine")) return nullptr;
+  PyObject* event = async ? as.end() : new_none();
+  if (!event) return nullptr;
+  PyObject* res = PyTuple_New(3);
+  if (!res) { Py_DECREF(event); return nullptr; }
+  PyTuple_SET_ITEM(res, 0, THPVariable_Wrap(out));
+  PyTuple_SET_ITEM(res, 1, w ? THPVariable_Wrap(out_w) : new_none());
+  PyTuple_SET_ITEM(res, 2, event);
+  return res;
+  END_HANDLE_TH_ERRORS
+}
+
+// ---- weights and gradients: (this rank's tensor, all-rank pool) pairs ------------------------
+// dense [epn, ...] and [R, epn, ...], blocks of the pool 16-byte aligned and inside the storage
+bool pair_ok(const Ctx& c, const at::Tensor* local, const at::Tensor* pool) {
+  if (!local || !pool || local->device() != c.hidden_buf.device() || pool->device() != c.hidden_buf.device())
+    return false;
+  const int64_t d = local->dim();
+  if (d < 2 || local->scalar_type() != pool->scalar_type() || !local->is_contiguous() || pool->dim() != d + 1)
+    return false;
+  if (local->size(0) != c.epn || pool->size(0) != c.R) return false;
+  int64_t dense = 1;
+  for (int64_t i = d; i >= 1; --i) {
+    if (pool->size(i) != local->size(i - 1) || pool->stride(i) != dense) return false;
+    dense *= pool->size(i);
+  }
+  const int64_t width = pool->element_size(), stride = pool->stride(0);
+  if (dense <= 0 || stride < dense || (stride * width) % 16 != 0 || stride * width >= ((int64_t)1 << 40)) return false;
+  if (!aligned(pool->data_ptr()) || !aligned(local->data_ptr())) return false;
+  return (pool->storage_offset() + stride * (c.R - 1) + dense) * width <= (int64_t)pool->storage().nbytes();
+}
+
+bool matrix_ok(const at::Tensor& t) { return t.dim() == 3 && t.size(1) % 128 == 0 && t.size(2) % 128 == 0; }
+
+// plan.experts_to_copy, or undefined
+at::Tensor slot_table(const Ctx& c, PyObject* plan) {
+  at::Tensor etc;
+  if ((PyObject*)Py_TYPE(plan) != c.plan_type) return etc;
+  PyObject* o = PyObject_GetAttr(plan, nm.etc);
+  if (!o) { PyErr_Clear(); return etc; }
+  const at::Tensor* t = tensor(o);
+  if (t && is(*t, at::kInt, c) && shape(*t, {c.R, c.epn})) etc = *t;
+  Py_DECREF(o);
+  return etc;
+}
+
+// prefetch(ctx, plan, async, 3 x local, 3 x pool, 3 x local scale, 3 x scale pool) -> True | event
+PyObject* py_prefetch(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 15) { PyErr_SetString(PyExc_TypeError, "prefetch takes 15 arguments"); return nullptr; }
+  Ctx* cp = ctx_of(args[0]);
+  if (!cp) return nullptr;
+  Ctx& c = *cp;
+  const bool async = args[2] == Py_True;
+  at::Tensor etc = slot_table(c, args[1]);
+  if (!etc.defined() || (async && capturing(c))) return new_none();
+  const void* src[6];
+  void* dst[6];
+  int64_t stride[6], bytes[6];
+  const at::Tensor* t[12] = {};
+  int given = 0;
+  for (int i = 9; i < 15; ++i) given += args[i] != Py_None;
+  if (given != 0 && given != 6) return new_none();
+  const int m = given ? 6 : 3;
+  for (int i = 0; i < m; ++i) {
+    const bool scale = i >= 3;
+    const at::Tensor* l = tensor(args[(scale ? 9 : 3) + i % 3]);
+    const at::Tensor* p = tensor(args[(scale ? 12 : 6) + i % 3]);
+    if (!pair_ok(c, l, p)) return new_none();
+    const at::ScalarType dt = l->scalar_type();
+    if (!scale) {
+      if (!matrix_ok(*l)) return new_none();
+      if (dt != at::kBFloat16 && dt != at::kChar && dt != at::kByte) return new_none();
+      if (i > 0 && dt != t[0]->scalar_type()) return new_none();
+      if (given && dt != at::kByte) return new_none();
+    } else if (dt != at::kByte) {
+      return new_none();
+    }
+    t[i] = l; t[6 + i] = p;
+    src[i] = l->data_ptr(); dst[i] = p->data_ptr();
+    stride[i] = p->stride(0) * p->element_size();
+    bytes[i] = (int64_t)(l->nbytes() / c.epn);
+    if (scale && bytes[i] % (128 * 128) != 0) return new_none();
+  }
+  Async as(c, async);
+  if (!as.begin({&etc, t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], t[9], t[10], t[11]})) return nullptr;
+  const int rc = mep_prefetch(m, src, dst, stride, bytes, ptr<int>(etc), c.rank, c.epn, c.R, as.stream);
+  if (failed(rc, "mep_prefetch")) return nullptr;
+  if (async) return as.end();
+  Py_RETURN_TRUE;
+  END_HANDLE_TH_ERRORS
+}
+
+// reduce_grad(ctx, plan, async, 3 x local, 3 x pool) -> True | event
+PyObject* py_reduce(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 9) { PyErr_SetString(PyExc_TypeError, "reduce_grad takes 9 arguments"); return nullptr; }
+  Ctx* cp = ctx_of(args[0]);
+  if (!cp) return nullptr;
+  Ctx& c = *cp;
+  const bool async = args[2] == Py_True;
+  at::Tensor etc = slot_table(c, args[1]);
+  if (!etc.defined() || (async && capturing(c))) return new_none();
+  const at::Tensor *l[3], *p[3];
+  for (int i = 0; i < 3; ++i) {
+    l[i] = tensor(args[3 + i]);
+    p[i] = tensor(args[6 + i]);
+    if (!pair_ok(c, l[i], p[i]) || l[i]->scalar_type() != at::kFloat || !matrix_ok(*l[i])) return new_none();
+  }
+  Async as(c, async);
+  if (!as.begin({&etc, l[0], l[1], l[2], p[0], p[1], p[2]})) return nullptr;
+  for (int i = 0; i < 3; ++i) {
+    const int rc = mep_grad_reduce(ptr<float>(*l[i]), ptr<float>(*p[i]), p[i]->stride(0), ptr<int>(etc), c.rank, c.epn,
+                                   c.R, l[i]->size(1) * l[i]->size(2), 0, as.stream);
+    if (failed(rc, "mep_grad_reduce")) return nullptr;
+  }
+  if (async) return as.end();
+  Py_RETURN_TRUE;
+  END_HANDLE_TH_ERRORS
+}
+
+// ---- context(ctx dict, plan type, no-map token, comm stream, event type) ----------------------
+PyObject* py_context(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 5 || !PyDict_Check(args[0])) { PyErr_SetString(PyExc_TypeError, "context takes 5 arguments"); return nullptr; }
+  PyObject* d = args[0];
+  bool ok = true;
+  auto num = [&](const char* key) -> int64_t {
+    PyObject* o = PyDict_GetItemString(d, key);  // borrowed
+    const int64_t v = o ? PyLong_AsLongLong(o) : -1;
+    ok = ok && o && !PyErr_Occurred();
+    return v;
+  };
+  auto tens = [&](const char* key) -> at::Tensor {
+    PyObject* o = PyDict_GetItemString(d, key);
+    const at::Tensor* t = o ? tensor(o) : nullptr;
+    return t ? *t : at::Tensor();
+  };
+  auto cptr = std::make_unique<Ctx>();
+  Ctx& c = *cptr;
+  c.S = (int)num("S"); c.H = (int)num("H"); c.K = (int)num("K"); c.E = (int)num("E"); c.R = (int)num("R");
+  c.NvS = (int)num("NvS"); c.rank = (int)num("rank"); c.tp = (int)num("token_padding");
+  c.N = (int64_t)c.S * c.K;
+  c.wslot_stride = num("meta_chunk_padded");
+  if (!ok) { PyErr_Clear(); return new_none(); }
+  c.epn = c.E / c.R;
+  c.hidden_buf = tens("hidden_buf"); c.meta_buf = tens("meta_buf");
+  c.hidden_local = tens("hidden_buf_local"); c.weights_local = tens("weights_buf_local");
+  c.scratch = tens("plan_scratch");
+  // the launches below address the weight slots at the start of a meta chunk and shards NvS rows apart
+  if (!c.hidden_buf.defined() || !c.meta_buf.defined() || !c.hidden_local.defined() || !c.weights_local.defined() ||
+      num("WEIGHTS_OFF") != 0 || num("NvS_padded") != c.NvS || c.H % 8 != 0)
+    return new_none();
+  auto keep = [](PyObject* o) { Py_INCREF(o); return o; };
+  c.plan_type = keep(args[1]);
+  c.no_map_token = keep(args[2]);
+  c.comm_py = keep(args[3]);
+  c.event_type = keep(args[4]);
+  c.hidden_local_py = keep(PyDict_GetItemString(d, "hidden_buf_local"));
+  c.empty = PyTuple_New(0);
+  c.py_N = PyLong_FromLongLong(c.N); c.py_R = PyLong_FromLong(c.R); c.py_E = PyLong_FromLong(c.E);
+  c.py_NvS = PyLong_FromLong(c.NvS); c.py_K = PyLong_FromLong(c.K);
+  auto stream_num = [&](const char* key) -> int64_t {
+    PyObject* o = PyObject_GetAttrString(args[3], key);
+    const int64_t v = o ? PyLong_AsLongLong(o) : 0;
+    Py_XDECREF(o);
+    return v;
+  };
+  c.comm = c10::Stream::unpack3(stream_num("stream_id"), (c10::DeviceIndex)stream_num("device_index"),
+                                (c10::DeviceType)stream_num("device_type"));
+  if (PyErr_Occurred()) return nullptr;
+  PyObject* cap = PyCapsule_New(cptr.get(), kCapsule, free_ctx);
+  if (cap) cptr.release();
+  return cap;
+  END_HANDLE_TH_ERRORS
+}
+
+#define MEP_FAST(f) (PyCFunction)(void (*)(void)) f, METH_FASTCALL, nullptr
+PyMethodDef kMethods[] = {{"context", MEP_FAST(py_context)},
+                          {"dispatch", MEP_FAST(py_dispatch)},
+                          {"combine", MEP_FAST(py_combine)},
+                          {"prefetch", MEP_FAST(py_prefetch)},
+                          {"reduce_grad", MEP_FAST(py_reduce)},
+                          {nullptr, nullptr, 0, nullptr}};
+PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_host", "native host side of the Buffer operators", -1, kMethods,
+                       nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__host(void) {
+  auto s = [](const char* t) { return PyUnicode_InternFromString(t); };
+  nm = Names{s("dst"), s("experts_to_copy"), s("zero_fill_ranges"), s("remote_stats"), s("dup_groups"),
+             s("dup_loffs"), s("dup_counts"), s("N"), s("R"), s("E"), s("NvS"), s("K"), s("_no_dup_map_in"),
+             s("record")};
+  return PyModule_Create(&kModule);
+}

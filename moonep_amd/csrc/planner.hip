@@ -38,6 +38,7 @@ struct PlanArgs {
   int* etc;          // [R, epn]
   int* zero_fill;    // [nranks, 2*epn, 2]
   int* remote_stats; // [nranks, 2]
+  int* dup_counts;   // [2] set to zero (a fresh plan has no duplicate groups yet), or null
   int* scratch;      // alloc/base tables when they do not fit in LDS
   int rank0, S, K, E, R, epn, tp, NvS, tok_per_wg;
   // optional: a byte range the workgroups beyond `groups` read once, so that it
@@ -552,6 +553,7 @@ __global__ __launch_bounds__(NT) void plan_kernel(PlanArgs a) {
   if (writer && tid == 0) {
     a.remote_stats[2 * blockIdx.y] = s_nrem[rank];
     a.remote_stats[2 * blockIdx.y + 1] = s_stat1[rank];
+    if (a.dup_counts) { a.dup_counts[0] = 0; a.dup_counts[1] = 0; }
   }
 }
 
@@ -607,8 +609,8 @@ extern "C" size_t mep_plan_scratch_bytes(int S, int K, int E, int R, int nranks)
 namespace {
 int plan_launch(const int32_t* tpe_RE, const int32_t* topk_nSK, int rank0, int nranks, int S, int K,
                 int E, int R, int token_padding, int NvS, int32_t* dst, int32_t* cu_seqlens,
-                int32_t* experts_to_copy, int32_t* zero_fill, int32_t* remote_stats, void* scratch,
-                size_t scratch_bytes, const void* warm, size_t warm_bytes, void* stream) {
+                int32_t* experts_to_copy, int32_t* zero_fill, int32_t* remote_stats, int32_t* dup_counts,
+                void* scratch, size_t scratch_bytes, const void* warm, size_t warm_bytes, void* stream) {
   MEP_REQUIRE(tpe_RE && topk_nSK && dst && cu_seqlens && experts_to_copy && zero_fill &&
                   remote_stats, MEP_ERR_INVALID_ARG);
   MEP_REQUIRE(S > 0 && K > 0 && E > 0 && R > 0 && token_padding > 0 && NvS > 0, MEP_ERR_INVALID_ARG);
@@ -629,6 +631,7 @@ int plan_launch(const int32_t* tpe_RE, const int32_t* topk_nSK, int rank0, int n
   PlanArgs a;
   a.tpe = tpe_RE; a.topk = topk_nSK; a.dst = dst; a.cu_seqlens = cu_seqlens;
   a.etc = experts_to_copy; a.zero_fill = zero_fill; a.remote_stats = remote_stats;
+  a.dup_counts = dup_counts;
   a.scratch = (int*)scratch;
   a.rank0 = rank0; a.S = S; a.K = K; a.E = E; a.R = R; a.epn = E / R; a.tp = token_padding;
   a.NvS = NvS; a.tok_per_wg = c.tok_per_wg;
@@ -690,7 +693,7 @@ extern "C" int mep_plan_ranks(const int32_t* tpe_RE, const int32_t* topk_nSK, in
                               int32_t* remote_stats, void* scratch, size_t scratch_bytes,
                               void* stream) {
   return plan_launch(tpe_RE, topk_nSK, rank0, nranks, S, K, E, R, token_padding, NvS, dst, cu_seqlens,
-                     experts_to_copy, zero_fill, remote_stats, scratch, scratch_bytes, nullptr, 0,
+                     experts_to_copy, zero_fill, remote_stats, nullptr, scratch, scratch_bytes, nullptr, 0,
                      stream);
 }
 
@@ -701,7 +704,19 @@ extern "C" int mep_plan_warm(const int32_t* tpe_RE, const int32_t* topk_SK, int 
                              const void* warm, size_t warm_bytes, void* stream) {
   MEP_REQUIRE(!warm || (uintptr_t)warm % 16 == 0, MEP_ERR_ALIGNMENT);
   return plan_launch(tpe_RE, topk_SK, rank, 1, S, K, E, R, token_padding, NvS, dst, cu_seqlens,
-                     experts_to_copy, zero_fill, remote_stats, scratch, scratch_bytes, warm,
+                     experts_to_copy, zero_fill, remote_stats, nullptr, scratch, scratch_bytes, warm,
+                     warm_bytes, stream);
+}
+
+extern "C" int mep_plan_fresh(const int32_t* tpe_RE, const int32_t* topk_SK, int rank, int S, int K,
+                              int E, int R, int token_padding, int NvS, int32_t* dst,
+                              int32_t* cu_seqlens, int32_t* experts_to_copy, int32_t* zero_fill,
+                              int32_t* remote_stats, int32_t* dup_counts, void* scratch,
+                              size_t scratch_bytes, const void* warm, size_t warm_bytes, void* stream) {
+  MEP_REQUIRE(dup_counts, MEP_ERR_INVALID_ARG);
+  MEP_REQUIRE(!warm || (uintptr_t)warm % 16 == 0, MEP_ERR_ALIGNMENT);
+  return plan_launch(tpe_RE, topk_SK, rank, 1, S, K, E, R, token_padding, NvS, dst, cu_seqlens,
+                     experts_to_copy, zero_fill, remote_stats, dup_counts, scratch, scratch_bytes, warm,
                      warm_bytes, stream);
 }
 
