@@ -381,6 +381,27 @@ int mep_swiglu_bwd(const void* dh, const void* gate_pre, const void* up_pre, con
 int mep_copy_shard(void* dst, const void* src, size_t bytes, void* dst_w, const void* src_w,
                    size_t words, void* stream);
 
+/*
+ * The expert FFN of one rank's rows in one call: y = slots * (silu(rows gate^T) * (rows up^T)) down^T
+ * per group (the two products of mep_grouped_swiglu_nt and mep_grouped_gemm_nt), and its backward
+ * (mep_grouped_gemm_nn, mep_swiglu_bwd, mep_grouped_gemm_dual_nn, three mep_grouped_gemm_wgrad_tn).
+ * The rows of y and drows beyond the last group come out as zeros; those of the intermediate
+ * buffers (act, gate_pre, up_pre [M,H'], dh) do not.
+ *   gate, up [G,H',H]; down [G,H,H']; slots [M] or NULL; gate_pre, up_pre: NULL where no backward
+ *   pass follows; dh, dgate, dup, hs [M,H'] scratch of the backward; dslots [M], NULL iff slots is;
+ *   wgrads: host array of three fp32 outputs (gate, up [.,H',H], down [.,H,H']) for the groups
+ *   below `split`, wgrads_from_split for the others; skip_empty_from as for mep_grouped_gemm_wgrad
+ * H and H' multiples of 256, G even, M a multiple of 128.
+ */
+int mep_ffn_forward(const void* rows, const float* slots, const int32_t* cu_seqlens, int G, const void* gate,
+                    const void* up, const void* down, void* act, void* gate_pre, void* up_pre, void* y, int M,
+                    int H, int Hp, void* stream);
+int mep_ffn_backward(const void* dy, const void* rows, const float* slots, const int32_t* cu_seqlens, int G,
+                     const void* gate, const void* up, const void* down, const void* gate_pre, const void* up_pre,
+                     void* dh, void* dgate, void* dup, void* hs, float* dslots, void* drows, float* const* wgrads,
+                     float* const* wgrads_from_split, int split, int M, int H, int Hp, int skip_empty_from,
+                     void* stream);
+
 #ifdef __cplusplus
 }
 #endif

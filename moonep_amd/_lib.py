@@ -66,6 +66,9 @@ _SIGNATURES = {
     "mep_grouped_gemm_dual_nn": (_i, [_p, _p, _p, _p, _p, _i, _p, _i, _i, _i, _p]),
     "mep_grouped_gemm_wgrad": (_i, [_p, _p, _p, _i, _p, _i, _i, _i64, _i, _p]),
     "mep_grouped_gemm_wgrad_tn": (_i, [_p, _p, _p, _i, _p, _i, _i, _i64, _i, _p]),
+    "mep_ffn_forward": (_i, [_p, _p, _p, _i, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _p]),
+    "mep_ffn_backward": (_i, [_p, _p, _p, _p, _i, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, C.POINTER(_p),
+                              C.POINTER(_p), _i, _i, _i, _i, _i, _p]),
     "mep_transpose_bf16": (_i, [_p, _p, _i, _i, _i, _p]),
     "mep_swiglu_bwd": (_i, [_p, _p, _p, _p, _p, _i, _p, _p, _p, _p, _i, _i, _p]),
 }

@@ -57,8 +57,10 @@ struct GemmArgs {
   uint16_t* Cu;        // swiglu: up pre-activation [M,N] or null
   float* Cf;           // wgrad: [G,M,N] fp32
   int64_t ld;          // row stride of A and B in elements (K, or the row count for wgrad)
-  int panel;           // row tiles of a long group that share a sweep over the weight tiles
   int skip_from;       // wgrad: groups g >= skip_from without rows are left unwritten
+  float* Cf2;          // wgrad: the groups from `split` on go here
+  int split;
+  bool zero_tail;      // row-tiled: the rows of C beyond the last group come out as zeros
 };
 
 enum { kModeScale = 0, kModeSwiglu = 1, kModeDual = 2, kModeWgrad = 3 };
@@ -80,6 +82,16 @@ __device__ __forceinline__ mep_bf16x8 mep_tr_pair(const char* lo, const char* hi
   const mep_s16x4 y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) mep_s16x4*)hi);
   const mep_s16x8 z = __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7);
   return __builtin_bit_cast(mep_bf16x8, z);
+}
+
+// rows of C beyond the last group, zeroed by `parts` workgroups of `threads` threads
+__device__ __forceinline__ void zero_tail_rows(const GemmArgs& a, int part, int parts, int threads) {
+  const int first = a.cu[a.G - 1];
+  const size_t bytes = (size_t)(a.M - first) * a.N * 2;  // N is a multiple of 128
+  char* base = (char*)(a.C + (size_t)first * a.N);
+  const mep_u4 zero = {0u, 0u, 0u, 0u};
+  for (size_t o = ((size_t)part * threads + threadIdx.x) * 16; o < bytes; o += (size_t)parts * threads * 16)
+    mep_st16_stream(base + o, zero);
 }
 
 // Producer / consumer waves.  Two producer waves stream the tiles from global
@@ -127,7 +139,12 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_nt_kernel(GemmAr
   const int total = MODE == kModeWgrad ? per_group * a.G : per_group;
   const int per_xcd = (total + 7) >> 3;
   const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
-  if (idx >= per_xcd) return;
+  if (idx >= per_xcd) {
+    // no tile: these workgroups are at least as many as the tiles that the unused rows would have
+    if (MODE != kModeWgrad && a.zero_tail)
+      zero_tail_rows(a, (idx - per_xcd) * 8 + xcd, ((int)(gridDim.x >> 3) - per_xcd) * 8, kGemmThreads);
+    return;
+  }
   int tg = 0, mt, nt;
   if (MODE == kModeWgrad) {
     if ((mtiles & 7) == 0) {
@@ -167,15 +184,15 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_nt_kernel(GemmAr
       }
     }
     if (tg < 0) return;  // cannot happen: L0 < total
-    // a long group goes in panels of a.panel row tiles (its weights are then read once per
-    // panel, its rows once per 32 / a.panel weight tiles)
+    // a long group goes in panels of kPanel row tiles (its weights are then read once per
+    // panel, its rows once per 32 / kPanel weight tiles)
     const int h = end_tiles - beg_tiles;
     const int local = L0 - beg_tiles * a.ntiles;
-    const int panel = local / (a.panel * a.ntiles);
-    const int within = local - panel * (a.panel * a.ntiles);
-    const int ph = min(a.panel, h - panel * a.panel);
+    const int panel = local / (kPanel * a.ntiles);
+    const int within = local - panel * (kPanel * a.ntiles);
+    const int ph = min(kPanel, h - panel * kPanel);
     nt = within / ph;
-    mt = beg_tiles + panel * a.panel + (within - nt * ph);
+    mt = beg_tiles + panel * kPanel + (within - nt * ph);
   }
   const int m0 = mt * kBM;
   constexpr int kCols = SWIGLU ? kBN / 2 : kBN;  // output columns per tile
@@ -344,238 +361,95 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_nt_kernel(GemmAr
 }
 
 // ---------------------------------------------------------------------------
-// Row-tiled products on tiles of 256 (or 128) rows x 256 weight rows.  These
-// kernels are bound by the lines they load, and a 256 x 256 tile needs a third
-// fewer of them per flop than a 128 x 256 one.  Groups end on multiples of 128
-// rows, so a group of h row blocks is covered by h / 2 tiles of 256 rows and,
-// if h is odd, one of 128 (a 256-row tile padded to the next group would load
-// and multiply as much again as it saves).  Eight waves of 128 x 64, all of
-// them load: every wave moves eight of the 64 one-KB pieces of a K step
-// straight into the other of two 64 KB LDS stages before it multiplies the
-// current one; one barrier per step.  (K in steps of 32 through a ring of four
-// 32 KB stages keeps the request stream going where two stages stop it at
-// every step, but asks for every line twice, half by half, and was 12 %
-// slower: what bounds the loads is the number of requests.)  A tile of 128
-// rows loads no rows for the upper four waves' half and those waves only take
-// part in the loads.
-// Tile list as in the kernel above: group by group, weight tile by weight
-// tile, the group's row tiles fastest; XCD x walks the x-th eighth.
+// The products of long groups and the weight gradient: 256 x 256 output tiles, K in steps of
+// 64, 8 waves of 128 x 64 (two on every SIMD), one workgroup per CU.
+//
+// What bounds it: latency of the loads first (a step's 64 KB arrive 1.8 us after they were asked
+// for when the chip is busy, and its matrix instructions take 0.9), then the matrix cores at the
+// clock their power leaves.  Hence
+//  * loads go straight into LDS, half an operand's tile (16 KB) at a time, into five slots per
+//    operand that are taken in turn: a half tile is asked for as soon as the one that had the slot
+//    five turns before has been read, four of a step's eight half-phases -- two K steps -- before
+//    it is wanted, and 64 to 96 KB per CU are in flight at every moment (the whole LDS of a CU is
+//    these slots);
+//  * s_waitcnt vmcnt(n) waits for the half tiles the next phase reads and leaves the rest in
+//    flight.  Neither a workgroup fence nor the compiler's transposing LDS read may stand in the
+//    loop: both wait for every load straight into LDS (that alone made the [K, N] forms 20 %
+//    slower);
+//  * a K step has two phases, rows 0 .. 127 and 128 .. 255 of the tile: read fragments and issue
+//    loads | barrier | 16 matrix instructions | barrier.  The waves 4 .. 7 run one barrier behind
+//    the waves 0 .. 3, so on every SIMD one wave multiplies while the other reads (without the
+//    shift 14 % slower; four phases of 8 instructions 2 % slower);
+//  * workgroups are persistent and walk the tile list as one stream of K steps: the next tile's
+//    loads are on their way while this one is finished and stored (10 % for K = 2048).
+// Groups end on multiples of 128 rows: a group of h 128-row blocks is h / 2 tiles and, if h is
+// odd, one of 128 rows whose second phase has no matrix instructions.
+//
+// Measured at 34 560 rows in 33 groups, H = 7168, H' = 2048 (us, before -> now; before: one
+// 256-row kernel with two LDS stages that drained its loads every step, wgrad likewise, dy * down
+// on 128 x 256 tiles): SwiGLU 2046 -> 1700, down 1150 -> 930, dy * down 1255 -> 887, dual
+// 2310 -> 1735, weight gradient 1555 -> 1285 (1.1 GB of fp32 zeroes for unused groups included);
+// 1.09 .. 1.19 PFLOP/s, where the library's dense product of such sizes reaches 1.16 .. 1.42.
+//
+// LDS layouts.  Operand rows along K: 128 bytes per row and step, 16-byte vector q of row r at
+// position q ^ (r & 7) ^ ((r >> 3) & 1): sixteen consecutive lanes cover all banks.  Operands
+// given as [K, columns] (weights of the input gradients, activations of the weight gradient): 64
+// rows of 256 bytes, vector v of row k at v ^ 4 (k & 3), read with transposing LDS reads (four
+// rows of 32 bytes per sixteen lanes): two such blocks side by side cover all banks.
 // ---------------------------------------------------------------------------
-constexpr int kT2Rows = 256;
-constexpr int kT2Stage = (kT2Rows + kBN) * kRowBytes;  // 64 KB
-constexpr int kT2Threads = 512;
-constexpr int kT2Panel = 8;  // row tiles of a long group that share a sweep over the weight tiles (4: 2-3 % slower at 3-6 per group)
-constexpr int kT2BOff = kT2Rows * kRowBytes;           // weight rows follow the 256 rows of the row tile
+constexpr int kPT = 256;                  // tile edge
+constexpr int kPPanel = 8;                // row tiles of a long group that share a sweep over the weight tiles
+constexpr int kPThreads = 512;
+constexpr int kPHalf = 128 * kRowBytes;   // 16 KB: half of one operand's tile of a K step
+constexpr int kPSlots = 5;                // of each operand
+constexpr int kPOperand = kPSlots * kPHalf;
+constexpr int kPLds = 2 * kPOperand;      // 160 KB
 
-template <int MODE, bool BKN>
-__global__ __launch_bounds__(kT2Threads, 1) void grouped_gemm256_kernel(GemmArgs a) {
-  constexpr bool SWIGLU = MODE == kModeSwiglu;
-  static_assert(MODE == kModeScale || MODE == kModeSwiglu || MODE == kModeDual, "row-tiled products only");
-  static_assert(!BKN || !SWIGLU, "[K, N] weights: plain and dual products only");
-  extern __shared__ __attribute__((aligned(1024))) char gsm[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-
-  // ---- tile list: group g has (h + 1) / 2 row tiles, h = its 128-row blocks
-  int total_rt = 0;
-  for (int c = 0; c < a.G; c += 64) {
-    const int gi = c + lane;
-    const int end = gi < a.G ? a.cu[gi] : 0;
-    const int beg = (gi > 0 && gi < a.G) ? a.cu[gi - 1] : 0;
-    const int t = gi < a.G ? ((end - beg) / kBM + 1) >> 1 : 0;
-    total_rt += __shfl(mep_wave_incl_scan(t), 63);
-  }
-  const int total = total_rt * a.ntiles;
-  const int per_xcd = (total + 7) >> 3;
-  const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
-  if (idx >= per_xcd) return;
-  const int L0 = xcd * per_xcd + idx;
-  if (L0 >= total) return;
-  int g = -1, m0 = 0, nt = 0;
-  bool tall = true;
-  {
-    int carry = 0;
-    for (int c = 0; c < a.G && g < 0; c += 64) {
-      const int gi = c + lane;
-      const int end = gi < a.G ? a.cu[gi] : 0;
-      const int beg = (gi > 0 && gi < a.G) ? a.cu[gi - 1] : 0;
-      const int t = gi < a.G ? ((end - beg) / kBM + 1) >> 1 : 0;
-      const int incl = carry + mep_wave_incl_scan(t);
-      const uint64_t m = __ballot(gi < a.G && incl * a.ntiles > L0);
-      if (m) {
-        const int src = __ffsll((unsigned long long)m) - 1;
-        g = c + src;
-        const int hs = __shfl(t, src), first = __shfl(incl - t, src);
-        const int gbeg = __shfl(beg, src), gend = __shfl(end, src);
-        const int local = L0 - first * a.ntiles;
-        // a long group goes in panels of a.panel row tiles
-        const int panel = local / (a.panel * a.ntiles);
-        const int within = local - panel * (a.panel * a.ntiles);
-        const int ph = min(a.panel, hs - panel * a.panel);
-        nt = within / ph;
-        m0 = gbeg + (panel * a.panel + (within - nt * ph)) * kT2Rows;
-        tall = m0 + kT2Rows <= gend;
-      }
-      carry = __shfl(incl, 63);
-    }
-  }
-  if (g < 0) return;  // cannot happen: L0 < total
-  constexpr int kCols = SWIGLU ? kBN / 2 : kBN;  // output columns per tile
-  const int n0 = nt * kCols;
-  const int KT1 = a.K / kBK;
-  const int KT = MODE == kModeDual ? 2 * KT1 : KT1;
-  const size_t K = (size_t)a.ld;
-
-  // ---- loads.  Piece j (0 .. 63) is rows 8j .. 8j+7 of the stage (the row tile, then the
-  // weight tile); wave w moves the pieces 8w .. 8w+7, so the waves 0-3 load rows and the waves
-  // 4-7 weights.  Lane (r, kv) fetches vector kv ^ r ^ (j & 1) of its row into slot (r, kv).
-  // [K, N] weights: weight piece jb holds the K rows 2 jb and 2 jb + 1 of the step, lane
-  // (lk, lv) fetches vector lv ^ 2 ((2 jb + lk) & 3) of its row.
-  const bool loads_rows = wave < 4;
-  const bool idle_loader = !tall && (wave == 2 || wave == 3);  // rows 128 .. 255 of a 128-row tile
-  const uint16_t* src[8];
-  size_t kstep;         // elements per K step
-  ptrdiff_t delta = 0;  // distance to the second pair (dual), elements
-  {
-    const int r = lane >> 3, kv = lane & 7, lk = lane >> 5, lv = lane & 31;
-    const size_t goff = (size_t)g * a.N * K;
-    kstep = (BKN && !loads_rows) ? (size_t)kBK * a.N : (size_t)kBK;
-    if (MODE == kModeDual) delta = loads_rows ? a.A2 - a.A : a.B2 - a.B;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int j = wave * 8 + q;
-      if (loads_rows) {
-        const int row = 8 * j + r;
-        src[q] = a.A + (size_t)(m0 + (idle_loader ? 0 : row)) * K + ((kv ^ r ^ (q & 1)) * 8);
-      } else if (BKN) {
-        const int jb = j - 32;
-        src[q] = a.B + goff + (size_t)(2 * jb + lk) * a.N + n0 + ((lv ^ ((2 * (q & 1) + lk) << 1)) * 8);
-      } else {
-        const int rb = 8 * (j - 32) + r;  // 0 .. 255
-        const uint16_t* base = (SWIGLU && rb >= kBN / 2) ? a.B2 : a.B;
-        const int nrow = SWIGLU ? n0 + (rb & (kBN / 2 - 1)) : n0 + rb;
-        src[q] = base + goff + (size_t)nrow * K + ((kv ^ r ^ (q & 1)) * 8);
-      }
-    }
-  }
-  auto issue = [&](int kt, int stage) {
-    if (idle_loader) return;
-    ptrdiff_t off = (ptrdiff_t)((size_t)kt * kstep);
-    if (MODE == kModeDual && kt >= KT1) off = (ptrdiff_t)((size_t)(kt - KT1) * kstep) + delta;
-    char* base = gsm + stage * kT2Stage + wave * 8 * 1024;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[q] + off),
-                                       (__attribute__((address_space(3))) void*)(base + q * 1024), 16, 0, 0);
-    }
-  };
-
-  // ---- consumers: 2 x 4 waves, 128 x 64 each
-  const int wm = wave & 1, wn = wave >> 1;
-  const bool works = tall || wm == 0;
-  mep_f32x16 acc[4][2];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
-  const int l31 = lane & 31, half = lane >> 5;
-  const int sw = (lane & 7) ^ ((lane >> 3) & 1);
-  const int oa = (128 * wm + l31) * kRowBytes;
-  const int ob0 = kT2BOff + (SWIGLU ? 32 * wn + l31 : 64 * wn + l31) * kRowBytes;
-  const int ob1 = ob0 + (SWIGLU ? kBN / 2 : 32) * kRowBytes;
-  const int ts = lane & 15, tb = (lane >> 4) & 1;
-  const int okn0 = kT2BOff + (8 * half + (ts >> 2)) * (kBN * 2) +
-                   (((8 * wn + 2 * tb + ((ts & 3) >> 1)) ^ ((ts >> 2) << 1)) * 16) + (ts & 1) * 8;
-  const int okn1 = kT2BOff + (8 * half + (ts >> 2)) * (kBN * 2) +
-                   (((8 * wn + 4 + 2 * tb + ((ts & 3) >> 1)) ^ ((ts >> 2) << 1)) * 16) + (ts & 1) * 8;
-
-  issue(0, 0);
-  mep_wait_vmcnt<0>();
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-  for (int kt = 0; kt < KT; ++kt) {
-    const int st = kt & 1;
-    if (kt + 1 < KT) issue(kt + 1, st ^ 1);
-    const char* sb = gsm + st * kT2Stage;
-    if (works) {
-#pragma unroll
-      for (int ks = 0; ks < kBK / 16; ++ks) {
-        const int col = ((2 * ks + half) ^ sw) * 16;
-        mep_bf16x8 fa[4], fb[2];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) fa[i] = *(const mep_bf16x8*)(sb + oa + i * 32 * kRowBytes + col);
-        if (BKN) {
-          const int step = ks * 16 * (kBN * 2);
-          fb[0] = mep_tr_pair(sb + okn0 + step, sb + okn0 + step + 4 * (kBN * 2));
-          fb[1] = mep_tr_pair(sb + okn1 + step, sb + okn1 + step + 4 * (kBN * 2));
-        } else {
-          fb[0] = *(const mep_bf16x8*)(sb + ob0 + col);
-          fb[1] = *(const mep_bf16x8*)(sb + ob1 + col);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
-      }
-    }
-    mep_wait_vmcnt<0>();  // the next stage has landed
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_s_barrier();  // ... for everyone, and everyone is done with this one
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-  }
-  if (!works) return;
-
-  // ---- epilogue.  acc[i][j][v]: row 128 wm + 32 i + 8 (v / 4) + 4 (lane / 32) + v % 4,
-  // column lane % 32 of the j-th 32-wide block
-  const int ldc = a.N;
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int m = m0 + 128 * wm + 32 * i + 8 * (v >> 2) + 4 * half + (v & 3);
-      if (SWIGLU) {
-        const int n = n0 + 32 * wn + l31;
-        const float res = mep_silu(acc[i][0][v]) * acc[i][1][v];
-        a.C[(size_t)m * ldc + n] = (uint16_t)mep_f32_to_bf16_bits(res);
-        if (a.Cg) a.Cg[(size_t)m * ldc + n] = (uint16_t)mep_f32_to_bf16_bits(acc[i][0][v]);
-        if (a.Cu) a.Cu[(size_t)m * ldc + n] = (uint16_t)mep_f32_to_bf16_bits(acc[i][1][v]);
-      } else {
-        const float sc = (MODE == kModeScale && a.scale) ? a.scale[m] : 1.0f;
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const int n = n0 + 64 * wn + 32 * j + l31;
-          a.C[(size_t)m * ldc + n] = (uint16_t)mep_f32_to_bf16_bits(sc * acc[i][j][v]);
-        }
-      }
-    }
+__device__ __forceinline__ const char* mep_uniform(const char* p) {
+  const uint64_t v = (uint64_t)p;
+  return (const char*)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) |
+                       (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v));
 }
 
-// ---------------------------------------------------------------------------
-// Weight gradient on 256 x 256 tiles.  The weight gradient is bound by the
-// lines its tiles load (a K loop of only rows / 64 steps, both operands
-// activations): a 256 x 256 tile needs a third fewer lines per flop than a
-// 128 x 256 one, and both output dimensions are multiples of 256 for the
-// shapes of an expert.  Eight waves of 128 x 64 (128 accumulator registers),
-// all of them load: every wave moves eight of the 64 one-KB pieces of a K step
-// straight into the other of two 64 KB LDS stages before it multiplies the
-// current one; one barrier per step.
-//
-// Tile map: the dimension with more tiles is cut into eight slices, one per
-// XCD (mirrored for odd groups, so that 28 tiles give every XCD 3 + 4), and
-// every XCD takes its slice of every group, two neighbouring groups at a time
-// (pairing every local expert with a slot instead, so that the zeroes of unused
-// slots are written beside the products, was 8 % slower): all XCDs
-// finish together whatever the groups' lengths, and the tiles an XCD runs at
-// one time are one group's slice times the whole other dimension -- each line
-// they load is wanted by 3 to 8 of them.
-// ---------------------------------------------------------------------------
-constexpr int kW2T = 256;                       // tile edge
-constexpr int kW2Stage = 2 * kW2T * kRowBytes;  // 64 KB: 256 rows of each operand
-constexpr int kW2Threads = 512;
+// 16 bytes per lane straight into LDS: lane offsets voff from a uniform base
+__device__ __forceinline__ void mep_load_lds16(const char* base, uint32_t voff, uint32_t soff, char* lds) {
+  __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, -1, 0x00020000);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, soff, 0, 0);
+}
+template <int VM>
+__device__ __forceinline__ void mep_wait_vm_lgkm0() {
+  __builtin_amdgcn_s_waitcnt((VM & 15) | (7 << 4) | ((VM >> 4) << 14));
+}
 
+__device__ __forceinline__ void mep_bar() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// two floats as bf16, rounded to nearest even by the hardware conversion
+__device__ __forceinline__ uint32_t mep_cvt_bf16x2(float lo, float hi) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  const f32x2 v = {lo, hi};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+}
+
+// Four K rows of a column block, transposed (see mep_tr_pair).  As an instruction of its own: in
+// front of the builtin the compiler waits for every load straight into LDS that is in flight.  The
+// result is there after the next wait for lgkmcnt(0); nothing may touch it before.
+template <class T>
+__device__ __forceinline__ void mep_tr_issue(T& x, uint32_t lds, int offset) {
+  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(x) : "v"(lds), "n"(offset));
+}
+
+// Tile list of the weight gradient: the dimension with more tiles is cut into eight slices, one
+// per XCD (mirrored for odd groups, so that 28 tiles give every XCD 3 + 4), and every XCD takes
+// its slice of every group, two neighbouring groups at a time: all XCDs finish together whatever
+// the groups' lengths, and the tiles an XCD runs at one time are one group's slice times the whole
+// other dimension -- each line they load is wanted by 3 to 8 of them.
 struct Wgrad2Map {
   int sliced, other;  // tiles of the sliced and of the other dimension
   bool slice_m;       // the sliced dimension is the output row
@@ -584,154 +458,382 @@ struct Wgrad2Map {
   __host__ __device__ int pair_count(int x) const { return (size(x) + size(7 - x)) * other; }
 };
 
-// TN: the operands are given as the forward and backward passes hold them, X1 [rows, Ma] and
-// X2 [rows, Nb] (a K step is then 64 rows of 512 bytes of each in LDS, read with the transposing
-// LDS loads of the [K, N] weight form above); otherwise as transposed copies [Ma, rows], [Nb, rows].
-template <bool TN>
-__global__ __launch_bounds__(kW2Threads, 1) void wgrad256_kernel(GemmArgs a, Wgrad2Map map) {
-  extern __shared__ __attribute__((aligned(1024))) char gsm[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
-  const int per_pair = map.pair_count(xcd);
-  if (per_pair == 0 || idx >= per_pair * (a.G >> 1)) return;
-  const int pair = idx / per_pair;
-  int local = idx - pair * per_pair;
-  const int n_even = map.size(xcd) * map.other;
-  int g = 2 * pair, xe = xcd;
-  if (local >= n_even) { local -= n_even; g += 1; xe = 7 - xcd; }
-  const int sz = map.size(xe);
-  const int u = local / sz, sl = map.lo(xe) + (local - u * sz);
-  const int m0 = (map.slice_m ? sl : u) * kW2T, n0 = (map.slice_m ? u : sl) * kW2T;
-  const int kbeg = g > 0 ? a.cu[g - 1] : 0;
-  const int KT = (a.cu[g] - kbeg) / kBK;
-  const size_t ld = (size_t)a.ld;
-
-  // ---- loads: piece j (0 .. 63) is rows 8j .. 8j+7 of the stage (output rows, then output
-  // columns); wave w moves the pieces 8w .. 8w+7; lane (r, kv) fetches vector
-  // kv ^ r ^ (j & 1) of its row into slot (r, kv).  TN: piece jp of an operand's half of the
-  // stage is the K rows 2 jp and 2 jp + 1 of the step (256 columns = 512 bytes each); lane
-  // (lk, lv) fetches vector lv ^ 2 ((2 jp + lk) & 3) of its row.
-  const int r = lane >> 3, kv = lane & 7;
-  const uint16_t* src[8];
-  size_t kstep;  // elements per K step
-  if (TN) {
-    const int lk = lane >> 5, lv = lane & 31;
-    const bool first = wave < 4;  // the waves 0-3 load X1, the waves 4-7 X2
-    const size_t pitch = first ? (size_t)a.M : (size_t)a.N;
-    const uint16_t* base = (first ? a.A + m0 : a.B + n0) + (size_t)kbeg * pitch;
-    kstep = (size_t)kBK * pitch;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int jp = (wave & 3) * 8 + q;
-      src[q] = base + (size_t)(2 * jp + lk) * pitch + ((lv ^ ((2 * (q & 1) + lk) << 1)) * 8);
-    }
-  } else {
-    kstep = kBK;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int j = wave * 8 + q;
-      const int row = 8 * j + r;  // 0 .. 511
-      const uint16_t* base = row < kW2T ? a.A + (size_t)(m0 + row) * ld : a.B + (size_t)(n0 + row - kW2T) * ld;
-      src[q] = base + kbeg + ((kv ^ r ^ (q & 1)) * 8);
+// The tiles of one workgroup, in order.  XCD x (workgroups x, x + 8, ...) walks a contiguous
+// eighth of the list, its workgroups in turn, so the tiles that run on an XCD at one time are
+// neighbours in the list.  Row-tiled products: the list goes group by group, inside a group weight
+// tile by weight tile, the group's row tiles fastest; a long group in panels of kPPanel row tiles
+// (its weights are read once per panel, its rows once per 32 / kPPanel weight tiles).  From round
+// to round a workgroup moves on by one place, so that the short last tiles of the groups do not
+// all go to the same ones.
+template <int MODE>
+struct PTiles {
+  const GemmArgs& a;
+  const Wgrad2Map& map;
+  int xcd, w, nw, count, first_item, r;  // this workgroup among the XCD's, tiles of the XCD, round
+  int c0, carry, cbeg;                   // row-tiled: 64 groups, one per lane; tiles and row before them
+  int incl, end;                         // tiles up to and including the group, its end
+  int g, m0, n0, kbeg, KT;
+  bool tall;
+  __device__ __forceinline__ PTiles(const GemmArgs& a_, const Wgrad2Map& map_) : a(a_), map(map_) {
+    xcd = blockIdx.x & 7; w = blockIdx.x >> 3; nw = gridDim.x >> 3; r = 0;
+    tall = true; kbeg = 0; KT = 0; g = 0; m0 = 0; n0 = 0;
+    if (MODE == kModeWgrad) {
+      count = map.pair_count(xcd) * (a.G >> 1);
+    } else {
+      int total_rt = 0;
+      for (int c = 0; c < a.G; c += 64) {
+        chunk(c);
+        total_rt += __shfl(incl, 63);
+      }
+      const int total = total_rt * a.ntiles;
+      const int per_xcd = (total + 7) >> 3;
+      first_item = xcd * per_xcd;
+      count = min(per_xcd, total - first_item);
+      count = __builtin_amdgcn_readfirstlane(count);
+      chunk(0);
+      carry = 0;
     }
   }
-  auto issue = [&](int kt, int stage) {
-    char* base = gsm + stage * kW2Stage + wave * 8 * 1024;
+  __device__ __forceinline__ void chunk(int c) {
+    c0 = c;
+    const int gi = c + (int)(threadIdx.x & 63);
+    end = gi < a.G ? a.cu[gi] : 0;
+    int beg = (gi > 0 && gi < a.G) ? a.cu[gi - 1] : 0;
+    asm volatile("" : "+v"(end), "+v"(beg));  // the loads end here, not inside the main loop
+    cbeg = __builtin_amdgcn_readfirstlane(beg);
+    incl = mep_wave_incl_scan(gi < a.G ? ((end - beg) / kBM + 1) >> 1 : 0);
+  }
+  // the next tile with work; false: no more
+  __device__ __forceinline__ bool next() {
+    for (;;) {
+      int rot = w + r;
+      rot -= rot / nw * nw;
+      const int item = r * nw + rot;
+      if (r * nw >= count) return false;
+      ++r;
+      if (item >= count) continue;
+      if (MODE == kModeWgrad) {
+        const int per_pair = map.pair_count(xcd);
+        const int pair = item / per_pair;
+        int local = item - pair * per_pair;
+        const int n_even = map.size(xcd) * map.other;
+        g = 2 * pair;
+        int xe = xcd;
+        if (local >= n_even) { local -= n_even; g += 1; xe = 7 - xcd; }
+        const int sz = map.size(xe);
+        const int u = local / sz, sl = map.lo(xe) + (local - u * sz);
+        m0 = (map.slice_m ? sl : u) * kPT; n0 = (map.slice_m ? u : sl) * kPT;
+        typedef const __attribute__((address_space(4))) int* cptr;
+        kbeg = g > 0 ? ((cptr)a.cu)[g - 1] : 0;
+        KT = (((cptr)a.cu)[g] - kbeg) / kBK;
+        if (KT == 0 && g >= a.skip_from) continue;
+        return true;
+      }
+      return find(item);
+    }
+  }
+  __device__ __forceinline__ bool find(int item) {
+    const int L0 = first_item + item;
+    for (;;) {
+      const uint64_t m = __ballot((carry + incl) * a.ntiles > L0);
+      if (m) {
+        const int src = __ffsll((unsigned long long)m) - 1;
+        g = c0 + src;
+        const int before = src > 0 ? __builtin_amdgcn_readlane(incl, src - 1) : 0;
+        const int hs = __builtin_amdgcn_readlane(incl, src) - before, first = carry + before;
+        const int gbeg = src > 0 ? __builtin_amdgcn_readlane(end, src - 1) : cbeg;
+        const int gend = __builtin_amdgcn_readlane(end, src);
+        const int local = L0 - first * a.ntiles;
+        const int panel = local / (kPPanel * a.ntiles);
+        const int within = local - panel * (kPPanel * a.ntiles);
+        const int ph = min(kPPanel, hs - panel * kPPanel);
+        const int nt = within / ph;
+        m0 = gbeg + (panel * kPPanel + (within - nt * ph)) * kPT;
+        n0 = nt * (MODE == kModeSwiglu ? kBN / 2 : kBN);
+        tall = m0 + kPT <= gend;
+        KT = MODE == kModeDual ? 2 * (a.K / kBK) : a.K / kBK;
+        return true;
+      }
+      carry += __builtin_amdgcn_readlane(incl, 63);
+      if (c0 + 64 >= a.G) return false;
+      chunk(c0 + 64);
+    }
+  }
+};
+
+// AT, BT: the operand is given as [K, columns].  SCALED: scale mode with row scales.
+template <int MODE, bool AT, bool BT, bool SCALED = false>
+__global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad2Map map) {
+  constexpr bool SWIGLU = MODE == kModeSwiglu, DUAL = MODE == kModeDual, WGRAD = MODE == kModeWgrad;
+  extern __shared__ __attribute__((aligned(1024))) char gsm[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l31 = lane & 31, half = lane >> 5;
+
+  // ---- loads: a cursor over (tile, K step)
+  const size_t ldA = AT ? (size_t)a.M : (size_t)a.ld, ldB = BT ? (size_t)a.N : (size_t)a.ld;
+  const size_t stepA = AT ? kBK * ldA * 2 : kBK * 2, stepB = BT ? kBK * ldB * 2 : kBK * 2;
+  const int KT1 = WGRAD ? 0 : a.K / kBK;
+  PTiles<MODE> ld(a, map);
+  const char *pA, *pB, *pB1;
+  uint32_t halfA, halfB;
+  int kl = 0;
+  auto stand = [&](int pair) {  // the pointers at the first K step of the cursor's tile (of its second pair)
+    const size_t goff = WGRAD ? (size_t)ld.kbeg * (BT ? ldB : 1) : (size_t)ld.g * a.N * a.K;
+    const size_t offA = AT ? (size_t)ld.kbeg * ldA + ld.m0 : (size_t)ld.m0 * ldA + (WGRAD ? ld.kbeg : 0);
+    const size_t offB = goff + (BT ? (size_t)ld.n0 : (size_t)ld.n0 * ldB);
+    pA = mep_uniform((const char*)((pair ? a.A2 : a.A) + offA));
+    pB = mep_uniform((const char*)((pair ? a.B2 : a.B) + offB));
+    pB1 = SWIGLU ? mep_uniform((const char*)(a.B2 + offB)) : pB;
+    halfA = __builtin_amdgcn_readfirstlane(ld.tall ? (AT ? 256u : (uint32_t)(128 * ldA * 2)) : 0u);
+    halfB = SWIGLU ? 0u : (BT ? 256u : (uint32_t)(128 * ldB * 2));
+  };
+  bool more = true;
+  do { more = ld.next(); } while (more && ld.KT == 0);
+  if (more) stand(0);
+  auto advance = [&]() {
+    if (!more) return;
+    if (kl + 1 < ld.KT) {
+      ++kl;
+      if (DUAL && kl == KT1) { stand(1); return; }
+      pA += stepA; pB += stepB; pB1 += stepB;
+      return;
+    }
+    do { more = ld.next(); } while (more && ld.KT == 0);
+    if (more) { kl = 0; stand(0); }  // otherwise the last step is loaded again, for nobody
+  };
+  uint32_t vA[2], vB[2];
+  {
+    const int r = lane >> 3, kv = lane & 7, lk = lane >> 4, lv = lane & 15;
 #pragma unroll
-    for (int q = 0; q < 8; ++q)
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[q] + (size_t)kt * kstep),
-                                       (__attribute__((address_space(3))) void*)(base + q * 1024), 16, 0, 0);
+    for (int q = 0; q < 2; ++q) {
+      const int j = 2 * wave + q;
+      vA[q] = AT ? (uint32_t)((4 * j + lk) * ldA * 2 + ((lv ^ (lk << 2)) * 16)) : (uint32_t)((8 * j + r) * ldA * 2 + ((kv ^ r ^ q) * 16));
+      vB[q] = BT ? (uint32_t)((4 * j + lk) * ldB * 2 + ((lv ^ (lk << 2)) * 16)) : (uint32_t)((8 * j + r) * ldB * 2 + ((kv ^ r ^ q) * 16));
+    }
+  }
+  // slots are taken in turn: where the next half tile of each operand is written and read
+  int wA = 0, wB = kPOperand, rA = 0, rB = kPOperand;
+  auto turn = [](int& slot, int first) { slot = slot == first + (kPSlots - 1) * kPHalf ? first : slot + kPHalf; };
+  char* lds_w = gsm + wave * 2048;
+  auto issueA = [&](int h) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) mep_load_lds16(pA, vA[q], h ? halfA : 0u, lds_w + wA + q * 1024);
+    turn(wA, 0);
+  };
+  auto issueB = [&](int h) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) mep_load_lds16(h ? pB1 : pB, vB[q], h ? halfB : 0u, lds_w + wB + q * 1024);
+    turn(wB, kPOperand);
   };
 
-  float* cf = a.Cf + (size_t)g * a.M * a.N;
-  if (KT == 0 && g >= a.skip_from) return;  // an unused slot whose gradient nobody reads
-  if (KT == 0) {
-    // a group without rows: its gradient is zero -- whole 1 KB rows of the
-    // tile per wave instruction instead of the accumulators' two 128-byte pieces
-    typedef float f32x4 __attribute__((ext_vector_type(4)));
-    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-    for (int row = wave; row < kW2T; row += kW2Threads / 64)
-      __builtin_nontemporal_store(zero, (f32x4*)(cf + (size_t)(m0 + row) * a.N + n0) + lane);
-    return;
-  }
-  const int wm = wave & 1, wn = wave >> 1;  // 2 x 4 waves, 128 x 64 each
-  mep_f32x16 acc[4][2];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
-  const int l31 = lane & 31, half = lane >> 5;
+  // ---- fragments
+  const int wm = wave >> 2, wn = wave & 3;
   const int sw = (lane & 7) ^ ((lane >> 3) & 1);
-  const int oa = (128 * wm + l31) * kRowBytes, ob = (kW2T + 64 * wn + l31) * kRowBytes;
-  // TN: lane s of a block of sixteen reads 8 bytes of K row 8 half + s / 4 (+ 4 for the second
-  // read, + 16 per MFMA step) at the columns c + 16 (block & 1) + 4 (s & 3) of a 32-column block
-  // that starts at column c of its operand's half of the stage
   const int ts = lane & 15, tb = (lane >> 4) & 1;
-  const int otn = (8 * half + (ts >> 2)) * (kW2T * 2) + (ts & 1) * 8;
-  const int vtn = 2 * tb + ((ts & 3) >> 1), xtn = (ts >> 2) << 1;
-
-  issue(0, 0);
-  mep_wait_vmcnt<0>();
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-  for (int kt = 0; kt < KT; ++kt) {
-    const int st = kt & 1;
-    if (kt + 1 < KT) issue(kt + 1, st ^ 1);
-    const char* sb = gsm + st * kW2Stage;
+  int adA[4], adB[4];
 #pragma unroll
-    for (int ks = 0; ks < kBK / 16; ++ks) {
-      const int col = ((2 * ks + half) ^ sw) * 16;
-      mep_bf16x8 fa[4], fb[2];
-      if (TN) {
-        // block i (32 columns = 4 vectors) moves the vector index by 4 i; the XOR with xtn
-        // (0, 2, 4 or 6) touches the bits 1 and 2 only, so 4 i is added before it
-        const int step = ks * 16 * (kW2T * 2);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int o = otn + step + (((16 * wm + 4 * i + vtn) ^ xtn) * 16);
-          fa[i] = mep_tr_pair(sb + o, sb + o + 4 * (kW2T * 2));
-        }
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const int o = kW2T * kRowBytes + otn + step + (((8 * wn + 4 * j + vtn) ^ xtn) * 16);
-          fb[j] = mep_tr_pair(sb + o, sb + o + 4 * (kW2T * 2));
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) fa[i] = *(const mep_bf16x8*)(sb + oa + i * 32 * kRowBytes + col);
-#pragma unroll
-        for (int j = 0; j < 2; ++j) fb[j] = *(const mep_bf16x8*)(sb + ob + j * 32 * kRowBytes + col);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
-    }
-    mep_wait_vmcnt<0>();  // the next stage has landed
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_s_barrier();  // ... for everyone, and everyone is done with this one
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  for (int ks = 0; ks < 4; ++ks) {
+    const int col = ((2 * ks + half) ^ sw) * 16;
+    adA[ks] = (64 * wm + l31) * kRowBytes + col;
+    adB[ks] = (32 * wn + l31) * kRowBytes + col;
   }
-
-  // ---- epilogue: acc[i][j][v] is row 128 wm + 32 i + 8 (v / 4) + 4 (lane / 32) + v % 4,
-  // column 64 wn + 32 j + lane % 32; streaming stores (see the 128 x 256 kernel)
+  const int lds0 = (int)(uintptr_t)(__attribute__((address_space(3))) char*)gsm;
+  const int trow = lds0 + (8 * half + (ts >> 2)) * 256 + (ts & 1) * 8;
+  const int tvec = 2 * tb + ((ts & 3) >> 1);
+  if (AT) {
+    adA[0] = trow + (((8 * wm + tvec) ^ ((ts >> 2) << 2)) * 16);
+    adA[1] = adA[0] ^ 64;
+  }
+  if (BT) adB[0] = trow + (((4 * wn + tvec) ^ ((ts >> 2) << 2)) * 16);
+  mep_bf16x8 fa[2][4], fb0[4], fb1[4];
+  mep_s16x4 ta[2][4][2], tb0[4][2], tb1[4][2];  // transposed reads until they have arrived
+  auto readA = [&]() {
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+    for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int m = m0 + 128 * wm + 32 * i + 8 * (v >> 2) + 4 * half + (v & 3);
+      for (int i = 0; i < 2; ++i) {
+        if (AT) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
-        __builtin_nontemporal_store(acc[i][j][v], &cf[(size_t)m * a.N + n0 + 64 * wn + 32 * j + l31]);
+          for (int u = 0; u < 2; ++u) mep_tr_issue(ta[i][ks][u], adA[i] + rA, ks * 4096 + u * 1024);
+        } else {
+          fa[i][ks] = *(const mep_bf16x8*)(gsm + (adA[ks] + rA) + i * 32 * kRowBytes);
+        }
+      }
+    turn(rA, 0);
+  };
+  auto readB = [&](mep_bf16x8* fb, mep_s16x4 (*tbw)[2]) {
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      if (BT) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) mep_tr_issue(tbw[ks][u], adB[0] + rB, ks * 4096 + u * 1024);
+      } else {
+        fb[ks] = *(const mep_bf16x8*)(gsm + (adB[ks] + rB));
+      }
     }
+    turn(rB, kPOperand);
+  };
+  auto join = [](const mep_s16x4* t) {
+    return __builtin_bit_cast(mep_bf16x8, __builtin_shufflevector(t[0], t[1], 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+  auto gotA = [&]() {  // after the wait
+    if (!AT) return;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        asm volatile("" : "+v"(ta[i][ks][0]), "+v"(ta[i][ks][1]));
+        fa[i][ks] = join(ta[i][ks]);
+      }
+  };
+  auto gotB = [&](mep_bf16x8* fb, mep_s16x4 (*tbw)[2]) {
+    if (!BT) return;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      asm volatile("" : "+v"(tbw[ks][0]), "+v"(tbw[ks][1]));
+      fb[ks] = join(tbw[ks]);
+    }
+  };
+  mep_f32x16 acc[2][2][2];
+  auto mm = [&](int hA) {
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        acc[hA][0][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i][ks], fb0[ks], acc[hA][0][i], 0, 0, 0);
+        acc[hA][1][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i][ks], fb1[ks], acc[hA][1][i], 0, 0, 0);
+      }
+    __builtin_amdgcn_s_setprio(0);
+  };
+
+  // ---- prologue: the first two K steps
+  PTiles<MODE> cp(a, map);
+  if (more) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      issueA(0); issueB(0); issueB(1); issueA(1);
+      advance();
+    }
+    mep_wait_vmcnt<10>();
+    mep_bar();
+    if (wave >= 4) mep_bar();
+  }
+  bool any = false;
+  while (cp.next()) {
+    const int g = cp.g, m0 = cp.m0, n0 = cp.n0, KT = cp.KT;
+    const bool tall = cp.tall;
+    float* cf = !WGRAD ? nullptr
+                : (g < a.split ? a.Cf + (size_t)g * a.M * a.N : a.Cf2 + (size_t)(g - a.split) * a.M * a.N);
+    if (WGRAD && KT == 0) {  // a group without rows: whole 1 KB rows of zeroes per wave instruction
+      typedef float f32x4 __attribute__((ext_vector_type(4)));
+      const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+      for (int row = wave; row < kPT; row += 8)
+        __builtin_nontemporal_store(zero, (f32x4*)(cf + (size_t)(m0 + row) * a.N + n0) + lane);
+      continue;
+    }
+    any = true;
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int y = 0; y < 2; ++y)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) acc[x][y][i][v] = 0.0f;
+    // The scales of this wave's rows, one per lane: asked for here, in order before the tile's
+    // loads, and there by the epilogue (a load the compiler knows would be waited for there, and
+    // with it every load of the next tile).
+    float scl0 = 1.0f, scl1 = 1.0f;
+    if (SCALED) {
+      const float* sp = a.scale + m0 + 64 * wm + lane;
+      asm volatile("global_load_dword %0, %1, off" : "=v"(scl0) : "v"(sp));
+      asm volatile("global_load_dword %0, %1, off" : "=v"(scl1) : "v"(sp + (tall ? 128 : 0)));
+    }
+    for (int kt = 0; kt < KT; ++kt) {
+      readA();
+      readB(fb0, tb0);
+      readB(fb1, tb1);
+      issueA(0);
+      issueB(0);
+      mep_wait_vm_lgkm0<12>();
+      gotA();
+      gotB(fb0, tb0);
+      gotB(fb1, tb1);
+      mep_bar();
+      mm(0);
+      mep_bar();
+
+      readA();
+      issueB(1);
+      issueA(1);
+      advance();
+      mep_wait_vm_lgkm0<10>();
+      gotA();
+      mep_bar();
+      if (tall) mm(1);
+      mep_bar();
+    }
+
+    if (SCALED) {
+      if (KT < 4) mep_wait_vmcnt<0>();  // too few loads after them for the loop to have waited
+      asm volatile("" : "+v"(scl0), "+v"(scl1));
+    }
+    // ---- epilogue: acc[x][y][i][v] is row 128 x + 64 wm + 32 i + 8 (v / 4) + 4 half + v % 4,
+    // column 128 y + 32 wn + l31
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      if (x == 1 && !tall) break;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int m = m0 + 128 * x + 64 * wm + 32 * i + 4 * half;
+        if (WGRAD) {
+          float* out = cf + (size_t)m * a.N + n0 + 32 * wn + l31;
+#pragma unroll
+          for (int v = 0; v < 16; ++v)
+#pragma unroll
+            for (int y = 0; y < 2; ++y)
+              __builtin_nontemporal_store(acc[x][y][i][v], out + (size_t)(8 * (v >> 2) + (v & 3)) * a.N + 128 * y);
+        } else {
+          // bf16: two rows of a column pair at a time -- the even lane of a pair stores both
+          // columns of the first row, the odd lane both of the second
+          int at0 = 16 * half;
+          asm volatile("" : "+v"(at0));  // addresses made here, not kept in registers across the main loop
+          const bool odd = lane & 1;
+          const uint32_t sel = odd ? 0x03020706u : 0x05040100u;
+          const size_t first = (size_t)(m + odd) * a.N + n0 + 32 * wn + (l31 & ~1);
+          auto put = [&](uint16_t* c, int v, int col, float v0, float v1) {
+            const uint32_t w = mep_cvt_bf16x2(v0, v1);
+            const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0xB1, 0xf, 0xf, true);  // the pair's other lane
+            *(uint32_t*)(c + first + (size_t)(8 * (v >> 2) + (v & 3)) * a.N + col) = __builtin_amdgcn_perm(o, w, sel);
+          };
+#pragma unroll
+          for (int v = 0; v < 16; v += 2) {
+            const float g0 = acc[x][0][i][v], g1 = acc[x][0][i][v + 1], u0 = acc[x][1][i][v], u1 = acc[x][1][i][v + 1];
+            if (SWIGLU) {
+              put(a.C, v, 0, mep_silu(g0) * u0, mep_silu(g1) * u1);
+              if (a.Cg) put(a.Cg, v, 0, g0, g1);
+              if (a.Cu) put(a.Cu, v, 0, u0, u1);
+            } else if (SCALED) {
+              const int at = at0 + 4 * (32 * i + 8 * (v >> 2) + (v & 3));
+              const float s0 = __int_as_float(__builtin_amdgcn_ds_bpermute(at, __float_as_int(x ? scl1 : scl0)));
+              const float s1 = __int_as_float(__builtin_amdgcn_ds_bpermute(at + 4, __float_as_int(x ? scl1 : scl0)));
+              put(a.C, v, 0, s0 * g0, s1 * g1);
+              put(a.C, v, 128, s0 * u0, s1 * u1);
+            } else {
+              put(a.C, v, 0, g0, g1);
+              put(a.C, v, 128, u0, u1);
+            }
+          }
+        }
+      }
+    }
+  }
+  if (any && wave < 4) mep_bar();
+  mep_wait_vmcnt<0>();  // the loads of steps nobody wanted write LDS, too
+  if (!WGRAD && a.zero_tail) zero_tail_rows(a, blockIdx.x, gridDim.x, kPThreads);
 }
-
-
 // ---------------------------------------------------------------------------
 // [batch, rows, cols] -> [batch, cols, rows] of 2-byte elements through a
 // 64 x 64 LDS tile (rows and cols multiples of 64): 128-byte reads and writes.
@@ -825,30 +927,35 @@ __global__ __launch_bounds__(256) void swiglu_bwd_kernel(SwigluBwdArgs a) {
   }
 }
 
-// launch of the 256-row-tile kernel: the grid covers the most row tiles the groups can need
-// ((M / 128 + G) / 2, when every group has an odd number of 128-row blocks)
+// persistent workgroups: one per CU, fewer when there are fewer tiles (a multiple of the 8 XCDs)
+unsigned pp_grid(int64_t tiles_per_xcd) {
+  const int cus = mep_device_cu_count();
+  const int64_t per_xcd = (cus > 0 ? cus : 256) / 8;
+  return 8 * (unsigned)(tiles_per_xcd < per_xcd ? tiles_per_xcd : per_xcd);
+}
+
 template <int MODE, bool BKN>
-int gemm256_launch(const GemmArgs& a0, hipStream_t st) {
-  GemmArgs a = a0;
-  a.panel = kT2Panel;
-  const int64_t row_tiles = ((int64_t)a.M / kBM + a.G + 1) / 2;
-  const int64_t total = row_tiles * a.ntiles;
+int gemm_pp_launch(const GemmArgs& a, hipStream_t st) {
+  // the most row tiles the groups can need: every group has an odd number of 128-row blocks
+  const int64_t total = ((int64_t)a.M / kBM + a.G + 1) / 2 * a.ntiles;
   MEP_REQUIRE(total > 0 && total < (1 << 30), MEP_ERR_UNSUPPORTED);
-  const int per_xcd = (int)((total + 7) / 8);
-  const size_t lds = 2 * (size_t)kT2Stage;
+  // lane offsets inside a tile are 32 bits
+  MEP_REQUIRE((int64_t)kPT * 2 * (a.K > a.N ? a.K : a.N) < ((int64_t)1 << 31), MEP_ERR_UNSUPPORTED);
   const int irc = mep_ensure_init();  // the LDS opt-in of this kernel, once per device
   if (irc != MEP_OK) return irc;
-  hipLaunchKernelGGL((grouped_gemm256_kernel<MODE, BKN>), dim3(per_xcd * 8), dim3(kT2Threads), lds, st, a);
+  const dim3 grid(pp_grid((total + 7) / 8)), block(kPThreads);
+  if (MODE == kModeScale && a.scale)
+    hipLaunchKernelGGL((gemm_pp_kernel<MODE, false, BKN, MODE == kModeScale>), grid, block, kPLds, st, a, Wgrad2Map{});
+  else
+    hipLaunchKernelGGL((gemm_pp_kernel<MODE, false, BKN>), grid, block, kPLds, st, a, Wgrad2Map{});
   return mep_launch_status();
 }
 
 // 144 KB of dynamic LDS: opted in by mep_init_gemm_kernels
 template <int MODE, bool BKN = false>
-int gemm_launch(const GemmArgs& a0, int64_t total, hipStream_t st) {
-  GemmArgs a = a0;
-  a.panel = kPanel;
+int gemm_launch(const GemmArgs& a, int64_t total, hipStream_t st) {
   MEP_REQUIRE(total > 0 && total < (1 << 30), MEP_ERR_UNSUPPORTED);
-  const int per_xcd = (int)((total + 7) / 8);
+  const int per_xcd = (int)((total + 7) / 8) + (a.zero_tail ? 1 : 0);
   const size_t lds = (size_t)kStages * kStage;
   const int irc = mep_ensure_init();
   if (irc != MEP_OK) return irc;
@@ -856,11 +963,11 @@ int gemm_launch(const GemmArgs& a0, int64_t total, hipStream_t st) {
   return mep_launch_status();
 }
 
-// launch of the 256 x 256 weight gradient (a.M, a.N multiples of 256, a.G even)
+// weight gradient on 256 x 256 tiles (a.M, a.N multiples of 256, a.G even)
 template <bool TN>
-int wgrad256_launch(const GemmArgs& a, hipStream_t st) {
+int wgrad_pp_launch(const GemmArgs& a, hipStream_t st) {
   Wgrad2Map map;
-  const int mt = a.M / kW2T, nt = a.N / kW2T;
+  const int mt = a.M / kPT, nt = a.N / kPT;
   map.slice_m = mt >= nt;
   map.sliced = map.slice_m ? mt : nt;
   map.other = map.slice_m ? nt : mt;
@@ -868,10 +975,10 @@ int wgrad256_launch(const GemmArgs& a, hipStream_t st) {
   for (int x = 0; x < 8; ++x) per_pair = per_pair > map.pair_count(x) ? per_pair : map.pair_count(x);
   const int64_t per_xcd = (int64_t)per_pair * (a.G / 2);
   MEP_REQUIRE(per_xcd > 0 && per_xcd < (1 << 27), MEP_ERR_UNSUPPORTED);
-  const size_t lds = 2 * (size_t)kW2Stage;
+  MEP_REQUIRE((int64_t)kPT * 2 * (TN ? (a.M > a.N ? a.M : a.N) : a.ld) < ((int64_t)1 << 31), MEP_ERR_UNSUPPORTED);
   const int irc = mep_ensure_init();
   if (irc != MEP_OK) return irc;
-  hipLaunchKernelGGL(wgrad256_kernel<TN>, dim3((unsigned)(per_xcd * 8)), dim3(kW2Threads), lds, st, a, map);
+  hipLaunchKernelGGL((gemm_pp_kernel<kModeWgrad, TN, TN>), dim3(pp_grid(per_xcd)), dim3(kPThreads), kPLds, st, a, map);
   return mep_launch_status();
 }
 
@@ -896,41 +1003,76 @@ GemmArgs nt_args(const void* A, const void* B, const void* B2, const int32_t* cu
   return a;
 }
 
-// Which row tiling: 256-row tiles load a third fewer lines per flop, but with two 64 KB
-// stages their loads drain at every K step, and there are half as many tiles to spread over
-// the CUs.  Measured at 34 688 rows, H = 7168, H' = 2048: 5-8 % faster where a launch has at
-// least eight of them per CU (SwiGLU, down, the dual input gradient), 12 % slower at five
-// (dy * down, 2048 output columns).
+// Which tiles.  The 256 x 256 kernel is the faster one wherever its tiles are filled.  Where the
+// groups have about one 128-row block each (decode batches: the padding alone fills it) half of
+// its matrix work and of its LDS would be idle, and the 128 x 256 kernel streams the weights
+// better (64 tokens, 16 experts of 4096 x 2048: SwiGLU 152 against 168 us; 512 tokens: 226
+// against 198).  The rows of the groups are only known on the device; M less the padding that
+// G groups can have at token_padding = 128 is what the rows of the G / 2 local experts fill.
 // mep_set_gemm_row_tile(128 or 256) forces one (tests run both on small shapes).
 std::atomic<int> g_forced_row_tile{0};
 
-static bool use_256_row_tiles(const GemmArgs& a) {
+static bool use_256_tiles(const GemmArgs& a) {
   const int forced = g_forced_row_tile.load(std::memory_order_relaxed);
   if (forced) return forced == 256;
-  const int cus = mep_device_cu_count();
-  return (int64_t)(a.M / kT2Rows) * a.ntiles >= 8 * (int64_t)(cus > 0 ? cus : 256);
+  return 2 * ((int64_t)a.M - (int64_t)(kBM - 1) * a.G) >= (int64_t)kBM * a.G;
+}
+
+// C = rows x weights for the modes that tile the rows; BKN: weights as [K, N]
+template <int MODE, bool BKN>
+int row_tiled(const GemmArgs& a, hipStream_t st) {
+  if (use_256_tiles(a)) return gemm_pp_launch<MODE, BKN>(a, st);
+  return gemm_launch<MODE, BKN>(a, (int64_t)a.mtiles * a.ntiles, st);
 }
 
 int gemm_nt_forward(const void* A, const void* B, const void* B_up, const int32_t* cu, int G, void* C,
                     void* C_gate, void* C_up, const float* row_scale, int M, int N, int K, int swiglu,
-                    void* stream) {
+                    bool zero_tail, void* stream) {
   const int cols = swiglu ? kBN / 2 : kBN;
   const int rc = check_nt_shapes(A, B, cu, C, M, N, K, G, cols);
   if (rc != MEP_OK) return rc;
   MEP_REQUIRE(!swiglu || (B_up && !row_scale), MEP_ERR_INVALID_ARG);
   MEP_REQUIRE(swiglu || (!C_gate && !C_up), MEP_ERR_INVALID_ARG);
   MEP_REQUIRE(((uintptr_t)A % 16 == 0) && ((uintptr_t)B % 16 == 0) && ((uintptr_t)B_up % 16 == 0) &&
-                  ((uintptr_t)C % 2 == 0) && ((uintptr_t)C_gate % 2 == 0) && ((uintptr_t)C_up % 2 == 0),
+                  ((uintptr_t)C % 4 == 0) && ((uintptr_t)C_gate % 4 == 0) && ((uintptr_t)C_up % 4 == 0),
               MEP_ERR_ALIGNMENT);
   GemmArgs a = nt_args(A, B, B_up, cu, C, row_scale, M, N, K, G, cols);
   a.Cg = (uint16_t*)C_gate;
   a.Cu = (uint16_t*)C_up;
-  const int64_t total = (int64_t)a.mtiles * a.ntiles;
-  if (use_256_row_tiles(a))
-    return swiglu ? gemm256_launch<kModeSwiglu, false>(a, (hipStream_t)stream)
-                  : gemm256_launch<kModeScale, false>(a, (hipStream_t)stream);
-  return swiglu ? gemm_launch<kModeSwiglu>(a, total, (hipStream_t)stream)
-                : gemm_launch<kModeScale>(a, total, (hipStream_t)stream);
+  a.zero_tail = zero_tail;
+  return swiglu ? row_tiled<kModeSwiglu, false>(a, (hipStream_t)stream)
+                : row_tiled<kModeScale, false>(a, (hipStream_t)stream);
+}
+
+// input gradients: weights as [K, N], one or two pairs
+int gemm_nn(const void* A1, const void* B1, const void* A2, const void* B2, const int32_t* cu, int G, void* C,
+            const float* row_scale, int M, int N, int K, bool zero_tail, void* stream) {
+  const int rc = check_nt_shapes(A1, B1, cu, C, M, N, K, G, kBN);
+  if (rc != MEP_OK) return rc;
+  MEP_REQUIRE(2 * (int64_t)K < ((int64_t)1 << 30), MEP_ERR_UNSUPPORTED);
+  MEP_REQUIRE(((uintptr_t)A1 % 16 == 0) && ((uintptr_t)B1 % 16 == 0) && ((uintptr_t)A2 % 16 == 0) &&
+                  ((uintptr_t)B2 % 16 == 0) && ((uintptr_t)C % 4 == 0), MEP_ERR_ALIGNMENT);
+  GemmArgs a = nt_args(A1, B1, B2, cu, C, row_scale, M, N, K, G, kBN);
+  a.A2 = (const uint16_t*)A2;
+  a.zero_tail = zero_tail;
+  return A2 ? row_tiled<kModeDual, true>(a, (hipStream_t)stream) : row_tiled<kModeScale, true>(a, (hipStream_t)stream);
+}
+
+// weight gradient from the activations as they are; the groups from `split` on go to C2
+int wgrad_tn(const void* X1, const void* X2, const int32_t* cu, int G, float* C, float* C2, int split, int Ma, int Nb,
+             int64_t rows, int skip_empty_from, void* stream) {
+  MEP_REQUIRE(X1 && X2 && cu && C && C2, MEP_ERR_INVALID_ARG);
+  MEP_REQUIRE(Ma > 0 && Nb > 0 && G > 0 && rows > 0 && skip_empty_from >= 0, MEP_ERR_INVALID_ARG);
+  MEP_REQUIRE(Ma % kPT == 0 && Nb % kPT == 0 && G % 2 == 0 && rows % kBM == 0, MEP_ERR_UNSUPPORTED);
+  MEP_REQUIRE((int64_t)(Ma > Nb ? Ma : Nb) * rows < ((int64_t)1 << 40), MEP_ERR_UNSUPPORTED);
+  MEP_REQUIRE(((uintptr_t)X1 % 16 == 0) && ((uintptr_t)X2 % 16 == 0) && ((uintptr_t)C % 16 == 0) &&
+                  ((uintptr_t)C2 % 16 == 0), MEP_ERR_ALIGNMENT);
+  GemmArgs a{};
+  a.A = (const uint16_t*)X1; a.B = (const uint16_t*)X2; a.cu = cu; a.Cf = C; a.Cf2 = C2; a.split = split;
+  a.M = Ma; a.N = Nb; a.K = 0; a.G = G;
+  a.ld = rows;
+  a.skip_from = skip_empty_from;
+  return wgrad_pp_launch<true>(a, (hipStream_t)stream);
 }
 
 template <class Kern>
@@ -946,7 +1088,7 @@ int opt_in_lds(Kern kern, size_t bytes) {
 // for the current device, made once from mep_init (never from a launch, which may be
 // under stream capture).
 int mep_init_gemm_kernels() {
-  const size_t ring = (size_t)kStages * kStage, two = 2 * (size_t)kT2Stage, w2 = 2 * (size_t)kW2Stage;
+  const size_t ring = (size_t)kStages * kStage;
   int rc = MEP_OK;
 #define MEP_OPT(k, b) if (rc == MEP_OK) rc = opt_in_lds(k, b)
   MEP_OPT((grouped_gemm_nt_kernel<kModeScale, false>), ring);
@@ -955,13 +1097,15 @@ int mep_init_gemm_kernels() {
   MEP_OPT((grouped_gemm_nt_kernel<kModeWgrad, false>), ring);
   MEP_OPT((grouped_gemm_nt_kernel<kModeScale, true>), ring);
   MEP_OPT((grouped_gemm_nt_kernel<kModeDual, true>), ring);
-  MEP_OPT((grouped_gemm256_kernel<kModeScale, false>), two);
-  MEP_OPT((grouped_gemm256_kernel<kModeSwiglu, false>), two);
-  MEP_OPT((grouped_gemm256_kernel<kModeDual, false>), two);
-  MEP_OPT((grouped_gemm256_kernel<kModeScale, true>), two);
-  MEP_OPT((grouped_gemm256_kernel<kModeDual, true>), two);
-  MEP_OPT(wgrad256_kernel<false>, w2);
-  MEP_OPT(wgrad256_kernel<true>, w2);
+  MEP_OPT((gemm_pp_kernel<kModeScale, false, false>), kPLds);
+  MEP_OPT((gemm_pp_kernel<kModeScale, false, false, true>), kPLds);
+  MEP_OPT((gemm_pp_kernel<kModeSwiglu, false, false>), kPLds);
+  MEP_OPT((gemm_pp_kernel<kModeDual, false, false>), kPLds);
+  MEP_OPT((gemm_pp_kernel<kModeScale, false, true>), kPLds);
+  MEP_OPT((gemm_pp_kernel<kModeScale, false, true, true>), kPLds);
+  MEP_OPT((gemm_pp_kernel<kModeDual, false, true>), kPLds);
+  MEP_OPT((gemm_pp_kernel<kModeWgrad, false, false>), kPLds);
+  MEP_OPT((gemm_pp_kernel<kModeWgrad, true, true>), kPLds);
 #undef MEP_OPT
   return rc;
 }
@@ -976,13 +1120,13 @@ extern "C" int mep_grouped_gemm_nt(const void* A, const void* B, const void* B_u
                                    const int32_t* cu_seqlens, int G, void* C,
                                    const float* row_scale, int M, int N, int K, int swiglu,
                                    void* stream) {
-  return gemm_nt_forward(A, B, B_up, cu_seqlens, G, C, nullptr, nullptr, row_scale, M, N, K, swiglu, stream);
+  return gemm_nt_forward(A, B, B_up, cu_seqlens, G, C, nullptr, nullptr, row_scale, M, N, K, swiglu, false, stream);
 }
 
 extern "C" int mep_grouped_swiglu_nt(const void* A, const void* B_gate, const void* B_up,
                                      const int32_t* cu_seqlens, int G, void* C_act, void* C_gate,
                                      void* C_up, int M, int N, int K, void* stream) {
-  return gemm_nt_forward(A, B_gate, B_up, cu_seqlens, G, C_act, C_gate, C_up, nullptr, M, N, K, 1, stream);
+  return gemm_nt_forward(A, B_gate, B_up, cu_seqlens, G, C_act, C_gate, C_up, nullptr, M, N, K, 1, false, stream);
 }
 
 extern "C" int mep_grouped_gemm_dual_nt(const void* A1, const void* B1, const void* A2, const void* B2,
@@ -993,21 +1137,15 @@ extern "C" int mep_grouped_gemm_dual_nt(const void* A1, const void* B1, const vo
   MEP_REQUIRE(A2 && B2, MEP_ERR_INVALID_ARG);
   MEP_REQUIRE(2 * (int64_t)K < ((int64_t)1 << 30), MEP_ERR_UNSUPPORTED);
   MEP_REQUIRE(((uintptr_t)A1 % 16 == 0) && ((uintptr_t)B1 % 16 == 0) && ((uintptr_t)A2 % 16 == 0) &&
-                  ((uintptr_t)B2 % 16 == 0) && ((uintptr_t)C % 2 == 0), MEP_ERR_ALIGNMENT);
+                  ((uintptr_t)B2 % 16 == 0) && ((uintptr_t)C % 4 == 0), MEP_ERR_ALIGNMENT);
   GemmArgs a = nt_args(A1, B1, B2, cu_seqlens, C, nullptr, M, N, K, G, kBN);
   a.A2 = (const uint16_t*)A2;
-  if (use_256_row_tiles(a)) return gemm256_launch<kModeDual, false>(a, (hipStream_t)stream);
-  return gemm_launch<kModeDual>(a, (int64_t)a.mtiles * a.ntiles, (hipStream_t)stream);
+  return row_tiled<kModeDual, false>(a, (hipStream_t)stream);
 }
 
 extern "C" int mep_grouped_gemm_nn(const void* A, const void* B, const int32_t* cu_seqlens, int G, void* C,
                                    const float* row_scale, int M, int N, int K, void* stream) {
-  const int rc = check_nt_shapes(A, B, cu_seqlens, C, M, N, K, G, kBN);
-  if (rc != MEP_OK) return rc;
-  MEP_REQUIRE(((uintptr_t)A % 16 == 0) && ((uintptr_t)B % 16 == 0) && ((uintptr_t)C % 2 == 0), MEP_ERR_ALIGNMENT);
-  GemmArgs a = nt_args(A, B, nullptr, cu_seqlens, C, row_scale, M, N, K, G, kBN);
-  if (use_256_row_tiles(a)) return gemm256_launch<kModeScale, true>(a, (hipStream_t)stream);
-  return gemm_launch<kModeScale, true>(a, (int64_t)a.mtiles * a.ntiles, (hipStream_t)stream);
+  return gemm_nn(A, B, nullptr, nullptr, cu_seqlens, G, C, row_scale, M, N, K, false, stream);
 }
 
 extern "C" int mep_grouped_gemm_dual_nn(const void* A1, const void* B1, const void* A2, const void* B2,
@@ -1016,13 +1154,7 @@ extern "C" int mep_grouped_gemm_dual_nn(const void* A1, const void* B1, const vo
   const int rc = check_nt_shapes(A1, B1, cu_seqlens, C, M, N, K, G, kBN);
   if (rc != MEP_OK) return rc;
   MEP_REQUIRE(A2 && B2, MEP_ERR_INVALID_ARG);
-  MEP_REQUIRE(2 * (int64_t)K < ((int64_t)1 << 30), MEP_ERR_UNSUPPORTED);
-  MEP_REQUIRE(((uintptr_t)A1 % 16 == 0) && ((uintptr_t)B1 % 16 == 0) && ((uintptr_t)A2 % 16 == 0) &&
-                  ((uintptr_t)B2 % 16 == 0) && ((uintptr_t)C % 2 == 0), MEP_ERR_ALIGNMENT);
-  GemmArgs a = nt_args(A1, B1, B2, cu_seqlens, C, nullptr, M, N, K, G, kBN);
-  a.A2 = (const uint16_t*)A2;
-  if (use_256_row_tiles(a)) return gemm256_launch<kModeDual, true>(a, (hipStream_t)stream);
-  return gemm_launch<kModeDual, true>(a, (int64_t)a.mtiles * a.ntiles, (hipStream_t)stream);
+  return gemm_nn(A1, B1, A2, B2, cu_seqlens, G, C, nullptr, M, N, K, false, stream);
 }
 
 extern "C" int mep_grouped_gemm_wgrad(const void* At, const void* Bt, const int32_t* cu_seqlens, int G,
@@ -1039,8 +1171,10 @@ extern "C" int mep_grouped_gemm_wgrad(const void* At, const void* Bt, const int3
   a.ld = ld;
   MEP_REQUIRE(skip_empty_from >= 0, MEP_ERR_INVALID_ARG);
   a.skip_from = skip_empty_from;
-  if (Ma % kW2T == 0 && Nb % kW2T == 0 && G % 2 == 0 && (uintptr_t)C % 16 == 0)  // an expert's shapes: 256 x 256 tiles
-    return wgrad256_launch<false>(a, (hipStream_t)stream);
+  a.split = G;
+  // an expert's shapes: 256 x 256 tiles (whose lane offsets are 32 bits)
+  if (Ma % kPT == 0 && Nb % kPT == 0 && G % 2 == 0 && (uintptr_t)C % 16 == 0 && ld < ((int64_t)1 << 22))
+    return wgrad_pp_launch<false>(a, (hipStream_t)stream);
   a.mtiles = Ma / kBM;
   a.ntiles = Nb / kBN;
   return gemm_launch<kModeWgrad>(a, (int64_t)a.mtiles * a.ntiles * G, (hipStream_t)stream);
@@ -1049,19 +1183,34 @@ extern "C" int mep_grouped_gemm_wgrad(const void* At, const void* Bt, const int3
 extern "C" int mep_grouped_gemm_wgrad_tn(const void* X1, const void* X2, const int32_t* cu_seqlens, int G,
                                          float* C, int Ma, int Nb, int64_t rows, int skip_empty_from,
                                          void* stream) {
-  MEP_REQUIRE(X1 && X2 && cu_seqlens && C, MEP_ERR_INVALID_ARG);
-  MEP_REQUIRE(Ma > 0 && Nb > 0 && G > 0 && rows > 0, MEP_ERR_INVALID_ARG);
-  MEP_REQUIRE(Ma % kW2T == 0 && Nb % kW2T == 0 && G % 2 == 0 && rows % kBM == 0, MEP_ERR_UNSUPPORTED);
-  MEP_REQUIRE((int64_t)(Ma > Nb ? Ma : Nb) * rows < ((int64_t)1 << 40), MEP_ERR_UNSUPPORTED);
-  MEP_REQUIRE(((uintptr_t)X1 % 16 == 0) && ((uintptr_t)X2 % 16 == 0) && ((uintptr_t)C % 16 == 0),
-              MEP_ERR_ALIGNMENT);
-  GemmArgs a{};
-  a.A = (const uint16_t*)X1; a.B = (const uint16_t*)X2; a.cu = cu_seqlens; a.Cf = C;
-  a.M = Ma; a.N = Nb; a.K = 0; a.G = G;
-  a.ld = rows;
-  MEP_REQUIRE(skip_empty_from >= 0, MEP_ERR_INVALID_ARG);
-  a.skip_from = skip_empty_from;
-  return wgrad256_launch<true>(a, (hipStream_t)stream);
+  return wgrad_tn(X1, X2, cu_seqlens, G, C, C, G, Ma, Nb, rows, skip_empty_from, stream);
+}
+
+extern "C" int mep_ffn_forward(const void* rows, const float* slots, const int32_t* cu_seqlens, int G, const void* gate,
+                               const void* up, const void* down, void* act, void* gate_pre, void* up_pre, void* y,
+                               int M, int H, int Hp, void* stream) {
+  const int rc = gemm_nt_forward(rows, gate, up, cu_seqlens, G, act, gate_pre, up_pre, nullptr, M, Hp, H, 1, false, stream);
+  if (rc != MEP_OK) return rc;
+  return gemm_nt_forward(act, down, nullptr, cu_seqlens, G, y, nullptr, nullptr, slots, M, H, Hp, 0, true, stream);
+}
+
+extern "C" int mep_ffn_backward(const void* dy, const void* rows, const float* slots, const int32_t* cu_seqlens, int G,
+                                const void* gate, const void* up, const void* down, const void* gate_pre,
+                                const void* up_pre, void* dh, void* dgate, void* dup, void* hs, float* dslots,
+                                void* drows, float* const* wgrads, float* const* wgrads_from_split, int split, int M,
+                                int H, int Hp, int skip_empty_from, void* stream) {
+  MEP_REQUIRE(gate && up && wgrads && wgrads_from_split && drows, MEP_ERR_INVALID_ARG);
+  MEP_REQUIRE((slots == nullptr) == (dslots == nullptr), MEP_ERR_INVALID_ARG);
+  // gradient of the unscaled activation: dy * down[g], down[g] is [H, H'] = [K, N]
+  int rc = gemm_nn(dy, down, nullptr, nullptr, cu_seqlens, G, dh, nullptr, M, Hp, H, false, stream);
+  if (rc == MEP_OK) rc = mep_swiglu_bwd(dh, gate_pre, up_pre, slots, cu_seqlens, G, dgate, dup, hs, dslots, M, Hp, stream);
+  if (rc == MEP_OK) rc = gemm_nn(dgate, gate, dup, up, cu_seqlens, G, drows, nullptr, M, H, Hp, true, stream);
+  const void* x1[3] = {dgate, dup, dy};
+  const void* x2[3] = {rows, rows, hs};
+  for (int i = 0; i < 3 && rc == MEP_OK; ++i)
+    rc = wgrad_tn(x1[i], x2[i], cu_seqlens, G, wgrads[i], wgrads_from_split[i], split, i < 2 ? Hp : H, i < 2 ? H : Hp,
+                  M, skip_empty_from, stream);
+  return rc;
 }
 
 extern "C" int mep_transpose_bf16(const void* src, void* dst, int batch, int rows, int cols, void* stream) {

@@ -1,4 +1,4 @@
-// Host side of the Buffer operators: argument checks, output allocation and launches of one
+// Host side of the Buffer operators and of the expert FFN: argument checks, output allocation and launches of one
 // call in native code (module moonep_amd._host).
 //
 // An operator of a small batch is bound by the host: through Python and ctypes a decode step
@@ -12,6 +12,7 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime.h>
 #include <torch/csrc/Exceptions.h>
@@ -455,6 +456,112 @@ PyObject* py_reduce(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// ---- the expert FFN --------------------------------------------------------------------------
+struct Ffn {
+  const at::Tensor *rows, *slots = nullptr, *cu, *gate, *up, *down;
+  int M, H, Hp, G;
+  at::TensorOptions bf16, f32;
+  hipStream_t stream;
+};
+
+bool dense(const at::Tensor* t, at::ScalarType dt, const at::Tensor& like) {
+  return t && t->scalar_type() == dt && t->device() == like.device() && t->is_contiguous() && aligned(t->data_ptr());
+}
+
+// args: rows, slots, cu, gate, up, down, token_padding
+bool read_ffn(PyObject* const* args, Ffn* f) {
+  f->rows = tensor(args[0]);
+  if (!f->rows || !f->rows->is_cuda() || !dense(f->rows, at::kBFloat16, *f->rows) || f->rows->dim() != 2) return false;
+  const at::Tensor& x = *f->rows;
+  f->cu = tensor(args[2]); f->gate = tensor(args[3]); f->up = tensor(args[4]); f->down = tensor(args[5]);
+  if (!f->cu || f->cu->scalar_type() != at::kInt || !f->cu->is_contiguous() || f->cu->dim() != 1 ||
+      f->cu->device() != x.device())
+    return false;
+  if (!dense(f->gate, at::kBFloat16, x) || !dense(f->up, at::kBFloat16, x) || !dense(f->down, at::kBFloat16, x)) return false;
+  const int64_t M = x.size(0), H = x.size(1), G = f->cu->numel();
+  if (f->gate->dim() != 3 || M % 128 != 0 || H % 256 != 0 || M <= 0 || M > INT32_MAX || H > (1 << 20) || G <= 0) return false;
+  const int64_t Hp = f->gate->size(1);
+  if (Hp % 128 != 0 || Hp <= 0 || Hp > (1 << 20)) return false;
+  if (!shape(*f->gate, {G, Hp, H}) || !shape(*f->up, {G, Hp, H}) || !shape(*f->down, {G, H, Hp})) return false;
+  if (args[1] != Py_None) {
+    f->slots = tensor(args[1]);
+    if (!dense(f->slots, at::kFloat, x) || f->slots->numel() != M) return false;
+  }
+  if (!PyLong_CheckExact(args[6])) return false;
+  const long tp = PyLong_AsLong(args[6]);
+  if (tp <= 0 || tp % 128 != 0) { PyErr_Clear(); return false; }
+  if (x.device().index() != c10::hip::current_device()) return false;
+  f->M = (int)M; f->H = (int)H; f->Hp = (int)Hp; f->G = (int)G;
+  f->bf16 = x.options(); f->f32 = x.options().dtype(at::kFloat);
+  f->stream = c10::hip::getCurrentHIPStream(x.device().index()).stream();
+  return true;
+}
+
+// ffn_forward(rows, slots, cu, gate, up, down, token_padding, train) -> y | (y, (gate_pre, up_pre))
+PyObject* py_ffn_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 8) { PyErr_SetString(PyExc_TypeError, "ffn_forward takes 8 arguments"); return nullptr; }
+  Ffn f;
+  if (!read_ffn(args, &f)) return new_none();
+  const bool train = args[7] == Py_True;
+  at::Tensor y = at::empty({f.M, f.H}, f.bf16), act = at::empty({f.M, f.Hp}, f.bf16), gp, up;
+  if (train) { gp = at::empty({f.M, f.Hp}, f.bf16); up = at::empty({f.M, f.Hp}, f.bf16); }
+  const int rc = mep_ffn_forward(f.rows->data_ptr(), f.slots ? ptr<float>(*f.slots) : nullptr, ptr<int>(*f.cu), f.G,
+                                 f.gate->data_ptr(), f.up->data_ptr(), f.down->data_ptr(), act.data_ptr(),
+                                 ptr<void>(gp), ptr<void>(up), y.data_ptr(), f.M, f.H, f.Hp, f.stream);
+  if (failed(rc, "mep_ffn_forward")) return nullptr;
+  if (!train) return THPVariable_Wrap(y);
+  return Py_BuildValue("(N(NN))", THPVariable_Wrap(y), THPVariable_Wrap(gp), THPVariable_Wrap(up));
+  END_HANDLE_TH_ERRORS
+}
+
+// ffn_backward(rows, slots, cu, gate, up, down, token_padding, dy, gate_pre, up_pre, skip_unused,
+//              own, from_slots): own and from_slots are tuples of three fp32 tensors for the
+//              weight gradients of the lower and the upper half of the groups, or None
+//   -> (drows, dslots, dgate, dup, ddown), the last three None where own is given
+PyObject* py_ffn_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 13) { PyErr_SetString(PyExc_TypeError, "ffn_backward takes 13 arguments"); return nullptr; }
+  Ffn f;
+  if (!read_ffn(args, &f)) return new_none();
+  const at::Tensor *dy = tensor(args[7]), *gp = tensor(args[8]), *up = tensor(args[9]);
+  if (!dense(dy, at::kBFloat16, *f.rows) || !dense(gp, at::kBFloat16, *f.rows) || !dense(up, at::kBFloat16, *f.rows) ||
+      !shape(*dy, {f.M, f.H}) || !shape(*gp, {f.M, f.Hp}) || !shape(*up, {f.M, f.Hp}))
+    return new_none();
+  if (f.Hp % 256 != 0 || f.G % 2 != 0) return new_none();
+  const bool skip = args[10] == Py_True, given = args[11] != Py_None;
+  float *w[3], *w2[3];
+  at::Tensor dw[3];
+  for (int i = 0; i < 3; ++i) {
+    const int64_t a = i < 2 ? f.Hp : f.H, b = i < 2 ? f.H : f.Hp;
+    if (given) {
+      if (!PyTuple_Check(args[11]) || PyTuple_GET_SIZE(args[11]) != 3 || !PyTuple_Check(args[12]) ||
+          PyTuple_GET_SIZE(args[12]) != 3)
+        return new_none();
+      const at::Tensor *o = tensor(PyTuple_GET_ITEM(args[11], i)), *s = tensor(PyTuple_GET_ITEM(args[12], i));
+      if (!dense(o, at::kFloat, *f.rows) || !dense(s, at::kFloat, *f.rows) || !shape(*o, {f.G / 2, a, b}) ||
+          !shape(*s, {f.G / 2, a, b}))
+        return new_none();
+      w[i] = ptr<float>(*o); w2[i] = ptr<float>(*s);
+    } else {
+      dw[i] = at::empty({f.G, a, b}, f.f32);
+      w[i] = ptr<float>(dw[i]); w2[i] = w[i] + (int64_t)(f.G / 2) * a * b;
+    }
+  }
+  at::Tensor drows = at::empty({f.M, f.H}, f.bf16), dslots, dh = at::empty({f.M, f.Hp}, f.bf16),
+             dg = at::empty({f.M, f.Hp}, f.bf16), du = at::empty({f.M, f.Hp}, f.bf16), hs = at::empty({f.M, f.Hp}, f.bf16);
+  if (f.slots) dslots = at::empty({f.M}, f.f32);
+  const int rc = mep_ffn_backward(dy->data_ptr(), f.rows->data_ptr(), f.slots ? ptr<float>(*f.slots) : nullptr,
+                                  ptr<int>(*f.cu), f.G, f.gate->data_ptr(), f.up->data_ptr(), f.down->data_ptr(),
+                                  gp->data_ptr(), up->data_ptr(), dh.data_ptr(), dg.data_ptr(), du.data_ptr(),
+                                  hs.data_ptr(), ptr<float>(dslots), drows.data_ptr(), w, w2, f.G / 2, f.M, f.H, f.Hp,
+                                  skip ? f.G / 2 : f.G, f.stream);
+  if (failed(rc, "mep_ffn_backward")) return nullptr;
+  auto give = [](const at::Tensor& t) { return t.defined() ? THPVariable_Wrap(t) : new_none(); };
+  return Py_BuildValue("(NNNNN)", give(drows), give(dslots), give(dw[0]), give(dw[1]), give(dw[2]));
+  END_HANDLE_TH_ERRORS
+}
+
 // ---- context(ctx dict, plan type, no-map token, comm stream, event type) ----------------------
 PyObject* py_context(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -517,6 +624,8 @@ PyMethodDef kMethods[] = {{"context", MEP_FAST(py_context)},
                           {"combine", MEP_FAST(py_combine)},
                           {"prefetch", MEP_FAST(py_prefetch)},
                           {"reduce_grad", MEP_FAST(py_reduce)},
+                          {"ffn_forward", MEP_FAST(py_ffn_forward)},
+                          {"ffn_backward", MEP_FAST(py_ffn_backward)},
                           {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_host", "native host side of the Buffer operators", -1, kMethods,
                        nullptr, nullptr, nullptr, nullptr};

@@ -73,6 +73,10 @@ def grouped_ffn_hip(rows, slots, cu_seqlens, gate_t, up_t, down, *, token_paddin
     weights (or None), cu_seqlens [2*epn]; gate_t/up_t [2*epn,H',H], down
     [2*epn,H,H'].  Rows outside every group come out as zeros.  ``token_padding``:
     that of the Buffer whose plan produced ``cu_seqlens`` (a multiple of 128)."""
+    y = _lib.host().ffn_forward(rows, slots, cu_seqlens, gate_t, up_t, down, token_padding, False)
+    if y is not None:
+        return y
+    # a shape that only the pieces take, or an argument they refuse
     hmid = launch_grouped_gemm_nt(rows, gate_t, cu_seqlens, up_weights=up_t,
                                   token_padding=token_padding)
     return launch_grouped_gemm_nt(hmid, down, cu_seqlens, row_scale=slots,
@@ -266,6 +270,9 @@ def launch_swiglu_bwd(dh, gate_pre, up_pre, row_scale, cu_seqlens, outs=None):
 def grouped_ffn_hip_forward(rows, slots, cu_seqlens, gate_t, up_t, down, *, token_padding: int = 128):
     """Forward for training: -> (y, saved) where ``saved`` is what
     ``grouped_ffn_hip_backward`` needs (the two pre-activations)."""
+    res = _lib.host().ffn_forward(rows, slots, cu_seqlens, gate_t, up_t, down, token_padding, True)
+    if res is not None:
+        return res
     act, gp, up = launch_grouped_swiglu(rows, gate_t, up_t, cu_seqlens, token_padding=token_padding)
     y = launch_grouped_gemm_nt(act, down, cu_seqlens, row_scale=slots, token_padding=token_padding)
     return y, (gp, up)
@@ -283,6 +290,10 @@ def grouped_ffn_hip_backward(dy, rows, slots, cu_seqlens, gate_t, up_t, down, sa
     hold no expert, which ``launch_grad_reduce`` never reads."""
     gp, up = saved
     dy = dy.contiguous()
+    res = _lib.host().ffn_backward(rows, slots, cu_seqlens, gate_t, up_t, down, token_padding, dy, gp, up,
+                                   bool(skip_unused_slots), None, None)
+    if res is not None:
+        return res
     # gradient of the unscaled activation: dy @ down[g], down[g] is [H, H'] = [K, N]
     dh = launch_grouped_gemm_nn(dy, down, cu_seqlens, token_padding=token_padding)
     dg, du, hs, dslots = launch_swiglu_bwd(dh, gp, up, slots, cu_seqlens)
