@@ -391,16 +391,53 @@ int mep_copy_shard(void* dst, const void* src, size_t bytes, void* dst_w, const 
  *   pass follows; dh, dgate, dup, hs [M,H'] scratch of the backward; dslots [M], NULL iff slots is;
  *   wgrads: host array of three fp32 outputs (gate, up [.,H',H], down [.,H,H']) for the groups
  *   below `split`, wgrads_from_split for the others; skip_empty_from as for mep_grouped_gemm_wgrad
- * H and H' multiples of 256, G even, M a multiple of 128.
+ * H and H' multiples of 256, G even, M a multiple of 128.  With nranks > 1 every tensor has that
+ * many ranks' blocks behind each other (cu_seqlens [nranks, G] counting from a rank's first row,
+ * weights [nranks, G, ..], gradients [nranks, split, ..] and [nranks, G - split, ..]).
  */
 int mep_ffn_forward(const void* rows, const float* slots, const int32_t* cu_seqlens, int G, const void* gate,
-                    const void* up, const void* down, void* act, void* gate_pre, void* up_pre, void* y, int M,
-                    int H, int Hp, void* stream);
+                    const void* up, const void* down, void* act, void* gate_pre, void* up_pre, void* y,
+                    int nranks, int M, int H, int Hp, void* stream);
 int mep_ffn_backward(const void* dy, const void* rows, const float* slots, const int32_t* cu_seqlens, int G,
                      const void* gate, const void* up, const void* down, const void* gate_pre, const void* up_pre,
                      void* dh, void* dgate, void* dup, void* hs, float* dslots, void* drows, float* const* wgrads,
-                     float* const* wgrads_from_split, int split, int M, int H, int Hp, int skip_empty_from,
-                     void* stream);
+                     float* const* wgrads_from_split, int split, int nranks, int M, int H, int Hp,
+                     int skip_empty_from, void* stream);
+
+/*
+ * The group's ranks in one launch, for one GPU that plays all of them: the operators above with a
+ * leading rank dimension on every per-rank tensor (tokens [n,S,H], weights [n,S,K], dst [n,S*K],
+ * zero_fill [n,2*epn,2], outputs likewise; duplicate groups [n,NvS,3] / [n,NvS] / [n,2]).
+ *   mep_dispatch_ranks: with cu_seqlens [n,2*epn] the rows and weight slots behind a rank's last
+ *     group are zeroed like its padding (so every row of its shard is written); NULL: they are not
+ *   mep_build_dedup_ranks: workspace of nranks times mep_dedup_scratch_bytes
+ *   mep_grad_reduce_batch: up to three projections at once; for several ranks (local_grad
+ *     [n,epn,..]) only the summing half (flags == MEP_REDUCE_NO_CLEAR)
+ */
+int mep_dispatch_ranks(const void* hidden_nSH, const float* w_nSK, const int32_t* dst, const int32_t* zero_fill,
+                       const int32_t* cu_seqlens, void* shards, int64_t shard_stride_rows, float* wslots,
+                       int64_t wslot_stride, int rank0, int nranks, int S, int H, int K, int R, int epn, int NvS,
+                       int token_padding, unsigned flags, void* stream);
+int mep_build_dedup_ranks(const int32_t* dst_RN, int rank0, int nranks, int S, int K, int R, int NvS,
+                          int32_t* dup_groups, int32_t* dup_loffs, int32_t* dup_counts, void* workspace,
+                          size_t workspace_bytes, void* stream);
+int mep_combine_ranks(const void* shards, int64_t shard_stride_rows, const float* wslots, int64_t wslot_stride,
+                      const int32_t* dst, void* out_nSH, float* out_nSK, int nranks, int S, int H, int K, int R,
+                      int NvS, int mode, void* stream);
+int mep_prefetch_pull_ranks(int ntensors, const void* const* owners, const int64_t* owner_stride_bytes,
+                            void* const* pool, const int64_t* rank_stride_bytes, const int64_t* bytes_per_expert,
+                            const int32_t* experts_to_copy, int rank0, int nranks, int epn, int R, void* stream);
+int mep_grad_reduce_batch(int ntensors, float* const* local_grad, float* const* reduce_pool,
+                          const int64_t* rank_stride_elems, const int64_t* elems_per_expert,
+                          const int32_t* experts_to_copy, int rank0, int nranks, int epn, int R, unsigned flags,
+                          void* stream);
+
+/*
+ * fp32 -> bf16 (round to nearest even) of up to six tensors of `nranks` dense blocks each, into
+ * blocks dst_rank_stride elements apart (compute views: a rank's local experts before its slots).
+ */
+int mep_cast_bf16(int ntensors, const float* const* src, void* const* dst, const int64_t* elems_per_rank,
+                  const int64_t* dst_rank_stride, int nranks, void* stream);
 
 #ifdef __cplusplus
 }

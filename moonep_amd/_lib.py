@@ -66,9 +66,18 @@ _SIGNATURES = {
     "mep_grouped_gemm_dual_nn": (_i, [_p, _p, _p, _p, _p, _i, _p, _i, _i, _i, _p]),
     "mep_grouped_gemm_wgrad": (_i, [_p, _p, _p, _i, _p, _i, _i, _i64, _i, _p]),
     "mep_grouped_gemm_wgrad_tn": (_i, [_p, _p, _p, _i, _p, _i, _i, _i64, _i, _p]),
-    "mep_ffn_forward": (_i, [_p, _p, _p, _i, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _p]),
+    "mep_ffn_forward": (_i, [_p, _p, _p, _i, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _p]),
     "mep_ffn_backward": (_i, [_p, _p, _p, _p, _i, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, C.POINTER(_p),
-                              C.POINTER(_p), _i, _i, _i, _i, _i, _p]),
+                              C.POINTER(_p), _i, _i, _i, _i, _i, _i, _p]),
+    "mep_dispatch_ranks": (_i, [_p, _p, _p, _p, _p, _p, _i64, _p, _i64, _i, _i, _i, _i, _i, _i, _i, _i, _i,
+                                C.c_uint, _p]),
+    "mep_build_dedup_ranks": (_i, [_p, _i, _i, _i, _i, _i, _i, _p, _p, _p, _p, _sz, _p]),
+    "mep_combine_ranks": (_i, [_p, _i64, _p, _i64, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _p]),
+    "mep_prefetch_pull_ranks": (_i, [_i, C.POINTER(_p), C.POINTER(_i64), C.POINTER(_p), C.POINTER(_i64),
+                                     C.POINTER(_i64), _p, _i, _i, _i, _i, _p]),
+    "mep_grad_reduce_batch": (_i, [_i, C.POINTER(_p), C.POINTER(_p), C.POINTER(_i64), C.POINTER(_i64), _p, _i, _i,
+                                   _i, _i, C.c_uint, _p]),
+    "mep_cast_bf16": (_i, [_i, C.POINTER(_p), C.POINTER(_p), C.POINTER(_i64), C.POINTER(_i64), _i, _p]),
     "mep_transpose_bf16": (_i, [_p, _p, _i, _i, _i, _p]),
     "mep_swiglu_bwd": (_i, [_p, _p, _p, _p, _p, _i, _p, _p, _p, _p, _i, _i, _p]),
 }

@@ -42,14 +42,15 @@ __global__ __launch_bounds__(kBlock) void combine_kernel(CombineArgs a) {
   const int K = a.K;
   const size_t row_bytes = (size_t)a.H * 2;
   int dv = 0;
-  if (lane < K) dv = a.dst[(size_t)s * K + lane];
+  const size_t sy = (size_t)blockIdx.y * a.S + s;  // blockIdx.y: one of several ranks behind each other
+  if (lane < K) dv = a.dst[sy * K + lane];
   const int raw = dv < 0 ? -dv - 1 : dv;
   const int drank = raw / a.NvS;
   const int loff = raw - drank * a.NvS;
   const bool valid = lane < K && drank < a.R;
   float wk = 0.0f;  // route weight of entry `lane`, read from its slot
   if (a.wslots && valid) wk = a.wslots[(size_t)drank * a.wslot_stride + loff];
-  if (a.out_sk && part == 0 && lane < K) a.out_sk[(size_t)s * K + lane] = wk;
+  if (a.out_sk && part == 0 && lane < K) a.out_sk[sy * K + lane] = wk;
   const uint64_t off = ((uint64_t)drank * (uint64_t)a.shard_stride_rows + (uint64_t)loff) * row_bytes;
   const uint32_t off_lo = (uint32_t)off, off_hi = (uint32_t)(off >> 32);
   const bool primary = valid && dv >= 0;
@@ -58,7 +59,7 @@ __global__ __launch_bounds__(kBlock) void combine_kernel(CombineArgs a) {
   const int nvec = a.H / 8;
   const int c0 = part * CH * 64 + lane;  // this lane's first 16-byte vector
   const char* base = (const char*)a.shards + (size_t)c0 * 16;
-  char* orow = (char*)a.out + (size_t)s * row_bytes + (size_t)c0 * 16;
+  char* orow = (char*)a.out + sy * row_bytes + (size_t)c0 * 16;
 
   float acc[CH][8];
 #pragma unroll
@@ -170,23 +171,21 @@ __global__ __launch_bounds__(kBlock) void combine_kernel(CombineArgs a) {
 }
 
 template <int CH, bool EXACT, bool TWO>
-void launch_combine(const CombineArgs& a0, hipStream_t st) {
+void launch_combine(const CombineArgs& a0, int nranks, hipStream_t st) {
   CombineArgs a = a0;
   const int nvec = a.H / 8;
   a.parts = (nvec + CH * 64 - 1) / (CH * 64);
   const int64_t waves = (int64_t)a.S * a.parts;
-  dim3 grid((unsigned)((waves + kWavesPerBlock - 1) / kWavesPerBlock));
+  dim3 grid((unsigned)((waves + kWavesPerBlock - 1) / kWavesPerBlock), nranks);
   hipLaunchKernelGGL((combine_kernel<CH, EXACT, TWO>), grid, dim3(kBlock), 0, st, a);
 }
 
-}  // namespace
-
-extern "C" int mep_combine(const void* shards, int64_t shard_stride_rows, const float* wslots,
-                           int64_t wslot_stride, const int32_t* dst, void* out_SH, float* out_SK,
-                           int S, int H, int K, int R, int NvS, int mode, void* stream) {
+int combine_launch(const void* shards, int64_t shard_stride_rows, const float* wslots,
+                   int64_t wslot_stride, const int32_t* dst, void* out_SH, float* out_SK, int nranks,
+                   int S, int H, int K, int R, int NvS, int mode, void* stream) {
   MEP_REQUIRE(shards && dst && out_SH, MEP_ERR_INVALID_ARG);
   MEP_REQUIRE(!out_SK || wslots, MEP_ERR_INVALID_ARG);
-  MEP_REQUIRE(S > 0 && H > 0 && K > 0 && R > 0 && NvS > 0, MEP_ERR_INVALID_ARG);
+  MEP_REQUIRE(S > 0 && H > 0 && K > 0 && R > 0 && NvS > 0 && nranks > 0 && nranks <= R, MEP_ERR_INVALID_ARG);
   MEP_REQUIRE(mode >= MEP_COMBINE_PRIMARIES && mode <= MEP_COMBINE_WEIGHTED, MEP_ERR_INVALID_ARG);
   MEP_REQUIRE(mode != MEP_COMBINE_WEIGHTED || wslots, MEP_ERR_INVALID_ARG);
   MEP_REQUIRE(K <= 32, MEP_ERR_UNSUPPORTED);
@@ -205,13 +204,29 @@ extern "C" int mep_combine(const void* shards, int64_t shard_stride_rows, const 
   if (mode == MEP_COMBINE_TWO_LEVEL) {
     // two accumulator sets: narrow tiles keep the register count low and more
     // waves resident (88.6 us with 2-chunk tiles vs 90.0 with 7 at H = 7168)
-    if (nvec % (2 * 64) == 0) launch_combine<2, true, true>(a, st);
-    else launch_combine<2, false, true>(a, st);
+    if (nvec % (2 * 64) == 0) launch_combine<2, true, true>(a, nranks, st);
+    else launch_combine<2, false, true>(a, nranks, st);
   } else {
-    if (nvec % (14 * 64) == 0) launch_combine<14, true, false>(a, st);
-    else if (nvec % (8 * 64) == 0) launch_combine<8, true, false>(a, st);
-    else if (nvec % (4 * 64) == 0) launch_combine<4, true, false>(a, st);
-    else launch_combine<2, false, false>(a, st);
+    if (nvec % (14 * 64) == 0) launch_combine<14, true, false>(a, nranks, st);
+    else if (nvec % (8 * 64) == 0) launch_combine<8, true, false>(a, nranks, st);
+    else if (nvec % (4 * 64) == 0) launch_combine<4, true, false>(a, nranks, st);
+    else launch_combine<2, false, false>(a, nranks, st);
   }
   return mep_launch_status();
+}
+
+}  // namespace
+
+extern "C" int mep_combine(const void* shards, int64_t shard_stride_rows, const float* wslots,
+                           int64_t wslot_stride, const int32_t* dst, void* out_SH, float* out_SK,
+                           int S, int H, int K, int R, int NvS, int mode, void* stream) {
+  return combine_launch(shards, shard_stride_rows, wslots, wslot_stride, dst, out_SH, out_SK, 1, S, H, K, R, NvS,
+                        mode, stream);
+}
+
+extern "C" int mep_combine_ranks(const void* shards, int64_t shard_stride_rows, const float* wslots,
+                                 int64_t wslot_stride, const int32_t* dst, void* out_nSH, float* out_nSK,
+                                 int nranks, int S, int H, int K, int R, int NvS, int mode, void* stream) {
+  return combine_launch(shards, shard_stride_rows, wslots, wslot_stride, dst, out_nSH, out_nSK, nranks, S, H, K, R,
+                        NvS, mode, stream);
 }

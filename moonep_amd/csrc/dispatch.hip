@@ -23,6 +23,10 @@ struct DispatchArgs {
   int64_t shard_stride_rows, wslot_stride;
   int rank, S, H, K, R, NvS, groups, tok_blocks, zblocks, zblocks_per_group;
   unsigned flags;
+  // blockIdx.y is one of several ranks whose inputs lie behind each other; with `cu` ([2*epn] a
+  // rank: padded ends of its groups) the slots behind the last group are zeroed like padding
+  const int* cu;
+  int cu_len, tail_blocks;
 };
 
 // One wave per (token, k) copy: it reads the token row (the K waves of a token
@@ -42,14 +46,14 @@ __global__ __launch_bounds__(kBlock) void dispatch_kernel(DispatchArgs a) {
     const int64_t gw = (int64_t)(blockIdx.x - a.zblocks) * kWavesPerBlock + wave;  // flat (token, k) index
     if (gw >= (int64_t)a.S * a.K) return;
     const int s = (int)(gw / a.K);
-    const int dv = a.dst[gw];
+    const int dv = a.dst[(size_t)blockIdx.y * a.S * a.K + gw];
     const int raw = dv < 0 ? -dv - 1 : dv;
     const int drank = raw / a.NvS;
     const int loff = raw - drank * a.NvS;
     if (drank >= a.R) return;  // never write outside the shards
-    if (a.w && lane == 0) a.wslots[(size_t)drank * a.wslot_stride + loff] = a.w[gw];
+    if (a.w && lane == 0) a.wslots[(size_t)drank * a.wslot_stride + loff] = a.w[(size_t)blockIdx.y * a.S * a.K + gw];
     if (dv < 0 && !(a.flags & MEP_DISPATCH_WRITE_DUPS)) return;
-    const char* src = (const char*)a.hidden + (size_t)s * row_bytes + (size_t)lane * 16;
+    const char* src = (const char*)a.hidden + ((size_t)blockIdx.y * a.S + s) * row_bytes + (size_t)lane * 16;
     char* row = (char*)a.shards +
                 ((uint64_t)drank * (uint64_t)a.shard_stride_rows + (uint64_t)loff) * row_bytes +
                 (size_t)lane * 16;
@@ -74,12 +78,21 @@ __global__ __launch_bounds__(kBlock) void dispatch_kernel(DispatchArgs a) {
     return;
   }
   // ---- zero-fill of this rank's padding rows (and their weight slots) -----
-  const int zb = blockIdx.x;
-  const int g = zb / a.zblocks_per_group;
-  const int part = zb - g * a.zblocks_per_group;
-  if (g >= a.groups) return;
-  const int pad_start = a.zero_fill[2 * g];
-  int n_pad = a.zero_fill[2 * g + 1];
+  const int rank = a.rank + blockIdx.y;
+  int zb = blockIdx.x, parts = a.zblocks_per_group, pad_start, n_pad;
+  if (zb < a.tail_blocks) {
+    pad_start = a.cu[(size_t)blockIdx.y * a.cu_len + a.cu_len - 1];
+    n_pad = a.NvS - pad_start;
+    parts = a.tail_blocks;
+  } else {
+    zb -= a.tail_blocks;
+    const int g = zb / parts;
+    zb -= g * parts;
+    if (g >= a.groups) return;
+    const int* zf = a.zero_fill + (size_t)blockIdx.y * 2 * a.groups + 2 * g;
+    pad_start = zf[0];
+    n_pad = zf[1];
+  }
   if (n_pad <= 0 || pad_start < 0) return;
   if ((int64_t)pad_start + n_pad > a.NvS) n_pad = a.NvS - pad_start;
   // The padding rows of a group are one contiguous byte range: the group's workgroups fill it
@@ -88,14 +101,14 @@ __global__ __launch_bounds__(kBlock) void dispatch_kernel(DispatchArgs a) {
   // costs a third more).
   const mep_u4 zero = {0u, 0u, 0u, 0u};
   char* base = (char*)a.shards +
-               ((uint64_t)a.rank * (uint64_t)a.shard_stride_rows + (uint64_t)pad_start) * row_bytes;
+               ((uint64_t)rank * (uint64_t)a.shard_stride_rows + (uint64_t)pad_start) * row_bytes;
   const size_t region = (size_t)n_pad * row_bytes;              // a multiple of 16 (H % 8 == 0)
-  const size_t step = (size_t)a.zblocks_per_group * kBlock * 16;
-  for (size_t off = ((size_t)part * kBlock + threadIdx.x) * 16; off < region; off += step)
+  const size_t step = (size_t)parts * kBlock * 16;
+  for (size_t off = ((size_t)zb * kBlock + threadIdx.x) * 16; off < region; off += step)
     mep_st16_stream(base + off, zero);
-  if (a.w && part == 0)
+  if (a.w && zb == 0)
     for (int j = threadIdx.x; j < n_pad; j += kBlock)
-      a.wslots[(size_t)a.rank * a.wslot_stride + pad_start + j] = 0.0f;
+      a.wslots[(size_t)rank * a.wslot_stride + pad_start + j] = 0.0f;
 }
 
 // ---------------------------------------------------------------------------
@@ -111,6 +124,15 @@ struct DedupArgs {
   int rank, S, K, R, NvS, ntok, nblk;
   int vec;         // rows of dst can be read as 16-byte vectors
 };
+
+// blockIdx.y is one of several destination ranks whose outputs lie behind each other
+__device__ __forceinline__ DedupArgs dedup_rank(DedupArgs a) {
+  const size_t y = blockIdx.y;
+  a.rank += (int)y;
+  a.dup_groups += y * 3 * a.NvS; a.dup_loffs += y * a.NvS; a.dup_counts += 2 * y;
+  a.blk_sums += y * 2 * a.nblk;
+  return a;
+}
 
 constexpr int kDedupBlock = 256;
 
@@ -143,7 +165,8 @@ __device__ __forceinline__ void dedup_block_sums(int g, int d, int* s_g, int* s_
   __syncthreads();
 }
 
-__global__ __launch_bounds__(kDedupBlock) void dedup_count_kernel(DedupArgs a) {
+__global__ __launch_bounds__(kDedupBlock) void dedup_count_kernel(DedupArgs a0) {
+  const DedupArgs a = dedup_rank(a0);
   __shared__ int s_g[kDedupBlock / 64], s_d[kDedupBlock / 64];
   const int t = blockIdx.x * kDedupBlock + threadIdx.x;
   int nd = 0;
@@ -159,7 +182,8 @@ __global__ __launch_bounds__(kDedupBlock) void dedup_count_kernel(DedupArgs a) {
   }
 }
 
-__global__ __launch_bounds__(kDedupBlock) void dedup_emit_kernel(DedupArgs a) {
+__global__ __launch_bounds__(kDedupBlock) void dedup_emit_kernel(DedupArgs a0) {
+  const DedupArgs a = dedup_rank(a0);
   __shared__ int s_g[kDedupBlock / 64], s_d[kDedupBlock / 64];
   const int t = blockIdx.x * kDedupBlock + threadIdx.x;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -327,25 +351,25 @@ void dup_launch_shape(int NvS, int max_cus, dim3* grid, dim3* block) {
 
 }  // namespace
 
-extern "C" int mep_dispatch(const void* hidden_SH, const float* w_SK, const int32_t* dst,
-                            const int32_t* zero_fill, void* shards, int64_t shard_stride_rows,
-                            float* wslots, int64_t wslot_stride, int rank, int S, int H, int K,
-                            int R, int epn, int NvS, int token_padding, unsigned flags,
-                            void* stream) {
-  MEP_REQUIRE(hidden_SH && dst && shards, MEP_ERR_INVALID_ARG);
-  MEP_REQUIRE((w_SK == nullptr) == (wslots == nullptr), MEP_ERR_INVALID_ARG);
+namespace {
+int dispatch_launch(const void* hidden, const float* w, const int32_t* dst, const int32_t* zero_fill,
+                    const int32_t* cu, void* shards, int64_t shard_stride_rows, float* wslots,
+                    int64_t wslot_stride, int rank, int nranks, int S, int H, int K, int R, int epn, int NvS,
+                    int token_padding, unsigned flags, void* stream) {
+  MEP_REQUIRE(hidden && dst && shards, MEP_ERR_INVALID_ARG);
+  MEP_REQUIRE((w == nullptr) == (wslots == nullptr), MEP_ERR_INVALID_ARG);
   MEP_REQUIRE(S > 0 && H > 0 && K > 0 && R > 0 && epn > 0 && NvS > 0 && token_padding > 0,
               MEP_ERR_INVALID_ARG);
-  MEP_REQUIRE(rank >= 0 && rank < R, MEP_ERR_INVALID_ARG);
+  MEP_REQUIRE(nranks > 0 && rank >= 0 && rank + nranks <= R, MEP_ERR_INVALID_ARG);
   MEP_REQUIRE(K <= 32, MEP_ERR_UNSUPPORTED);
   // an entry decodes as (raw / NvS, raw % NvS); raw = R*NvS (rank R) marks an entry nobody copies
   MEP_REQUIRE((int64_t)R * NvS <= INT32_MAX, MEP_ERR_UNSUPPORTED);
   MEP_REQUIRE(H % 8 == 0, MEP_ERR_UNSUPPORTED);  // 16-byte row vectors (reference dispatch.py:901)
   MEP_REQUIRE(shard_stride_rows >= NvS && (!wslots || wslot_stride >= NvS), MEP_ERR_INVALID_ARG);
-  MEP_REQUIRE(((uintptr_t)hidden_SH % 16 == 0) && ((uintptr_t)shards % 16 == 0), MEP_ERR_ALIGNMENT);
+  MEP_REQUIRE(((uintptr_t)hidden % 16 == 0) && ((uintptr_t)shards % 16 == 0), MEP_ERR_ALIGNMENT);
   const bool zf = zero_fill && !(flags & MEP_DISPATCH_NO_ZERO_FILL);
   DispatchArgs a;
-  a.hidden = (const uint16_t*)hidden_SH; a.w = w_SK; a.dst = dst; a.zero_fill = zero_fill;
+  a.hidden = (const uint16_t*)hidden; a.w = w; a.dst = dst; a.zero_fill = zero_fill;
   a.shards = (uint16_t*)shards; a.wslots = wslots;
   a.shard_stride_rows = shard_stride_rows; a.wslot_stride = wslot_stride;
   a.rank = rank; a.S = S; a.H = H; a.K = K; a.R = R; a.NvS = NvS; a.flags = flags;
@@ -357,8 +381,11 @@ extern "C" int mep_dispatch(const void* hidden_SH, const float* w_SK, const int3
   a.zblocks_per_group = zpg;
   const int zblocks = (zf && token_padding > 1) ? a.groups * zpg : 0;
   if (zblocks == 0) a.groups = 0;
-  a.zblocks = zblocks;
-  dim3 grid(a.tok_blocks + zblocks);
+  a.cu = cu;
+  a.cu_len = 2 * epn;
+  a.tail_blocks = cu ? 64 : 0;
+  a.zblocks = zblocks + a.tail_blocks;
+  dim3 grid(a.tok_blocks + a.zblocks, nranks);
   hipStream_t st = (hipStream_t)stream;
   // rows that are a whole number of 1-KiB wave tiles (H % 512 == 0, up to H = 8192) pass
   // through registers in one go; any other H % 8 == 0 takes the strided loop
@@ -375,6 +402,25 @@ extern "C" int mep_dispatch(const void* hidden_SH, const float* w_SK, const int3
     default: hipLaunchKernelGGL(dispatch_kernel<0>, grid, dim3(kBlock), 0, st, a); break;
   }
   return mep_launch_status();
+}
+}  // namespace
+
+extern "C" int mep_dispatch(const void* hidden_SH, const float* w_SK, const int32_t* dst,
+                            const int32_t* zero_fill, void* shards, int64_t shard_stride_rows,
+                            float* wslots, int64_t wslot_stride, int rank, int S, int H, int K,
+                            int R, int epn, int NvS, int token_padding, unsigned flags,
+                            void* stream) {
+  return dispatch_launch(hidden_SH, w_SK, dst, zero_fill, nullptr, shards, shard_stride_rows, wslots, wslot_stride,
+                         rank, 1, S, H, K, R, epn, NvS, token_padding, flags, stream);
+}
+
+extern "C" int mep_dispatch_ranks(const void* hidden_nSH, const float* w_nSK, const int32_t* dst,
+                                  const int32_t* zero_fill, const int32_t* cu_seqlens, void* shards,
+                                  int64_t shard_stride_rows, float* wslots, int64_t wslot_stride, int rank0,
+                                  int nranks, int S, int H, int K, int R, int epn, int NvS, int token_padding,
+                                  unsigned flags, void* stream) {
+  return dispatch_launch(hidden_nSH, w_nSK, dst, zero_fill, cu_seqlens, shards, shard_stride_rows, wslots,
+                         wslot_stride, rank0, nranks, S, H, K, R, epn, NvS, token_padding, flags, stream);
 }
 
 extern "C" size_t mep_dedup_scratch_bytes(int S, int R) {
@@ -432,13 +478,13 @@ extern "C" int mep_build_dedup_static(const int32_t* dst_RN, int rank, int S, in
                          kStaticDedupBytes, stream);
 }
 
-extern "C" int mep_build_dedup(const int32_t* dst_RN, int rank, int S, int K, int R, int NvS,
-                               int32_t* dup_groups, int32_t* dup_loffs, int32_t* dup_counts,
-                               void* workspace, size_t workspace_bytes, void* stream) {
+namespace {
+int dedup_launch(const int32_t* dst_RN, int rank, int nranks, int S, int K, int R, int NvS, int32_t* dup_groups,
+                 int32_t* dup_loffs, int32_t* dup_counts, void* workspace, size_t workspace_bytes, void* stream) {
   MEP_REQUIRE(dst_RN && dup_groups && dup_loffs && dup_counts, MEP_ERR_INVALID_ARG);
-  MEP_REQUIRE(S > 0 && K > 0 && R > 0 && NvS > 0 && rank >= 0 && rank < R, MEP_ERR_INVALID_ARG);
+  MEP_REQUIRE(S > 0 && K > 0 && R > 0 && NvS > 0 && nranks > 0 && rank >= 0 && rank + nranks <= R, MEP_ERR_INVALID_ARG);
   MEP_REQUIRE((int64_t)S * R < INT32_MAX && (int64_t)R * NvS <= INT32_MAX, MEP_ERR_UNSUPPORTED);
-  MEP_REQUIRE(workspace && workspace_bytes >= mep_dedup_scratch_bytes(S, R), MEP_ERR_SCRATCH);
+  MEP_REQUIRE(workspace && workspace_bytes >= nranks * mep_dedup_scratch_bytes(S, R), MEP_ERR_SCRATCH);
   DedupArgs a;
   a.dst = dst_RN; a.dup_groups = dup_groups; a.dup_loffs = dup_loffs; a.dup_counts = dup_counts;
   a.rank = rank; a.S = S; a.K = K; a.R = R; a.NvS = NvS;
@@ -447,9 +493,24 @@ extern "C" int mep_build_dedup(const int32_t* dst_RN, int rank, int S, int K, in
   a.blk_sums = (int*)workspace;
   a.vec = (K % 4 == 0) && ((uintptr_t)dst_RN % 16 == 0);
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(dedup_count_kernel, dim3(a.nblk), dim3(kDedupBlock), 0, st, a);
-  hipLaunchKernelGGL(dedup_emit_kernel, dim3(a.nblk), dim3(kDedupBlock), 0, st, a);
+  hipLaunchKernelGGL(dedup_count_kernel, dim3(a.nblk, nranks), dim3(kDedupBlock), 0, st, a);
+  hipLaunchKernelGGL(dedup_emit_kernel, dim3(a.nblk, nranks), dim3(kDedupBlock), 0, st, a);
   return mep_launch_status();
+}
+}  // namespace
+
+extern "C" int mep_build_dedup(const int32_t* dst_RN, int rank, int S, int K, int R, int NvS,
+                               int32_t* dup_groups, int32_t* dup_loffs, int32_t* dup_counts,
+                               void* workspace, size_t workspace_bytes, void* stream) {
+  return dedup_launch(dst_RN, rank, 1, S, K, R, NvS, dup_groups, dup_loffs, dup_counts, workspace, workspace_bytes,
+                      stream);
+}
+
+extern "C" int mep_build_dedup_ranks(const int32_t* dst_RN, int rank0, int nranks, int S, int K, int R, int NvS,
+                                     int32_t* dup_groups, int32_t* dup_loffs, int32_t* dup_counts,
+                                     void* workspace, size_t workspace_bytes, void* stream) {
+  return dedup_launch(dst_RN, rank0, nranks, S, K, R, NvS, dup_groups, dup_loffs, dup_counts, workspace,
+                      workspace_bytes, stream);
 }
 
 extern "C" int mep_dispatch_epilogue(void* shard, const int32_t* dup_groups,

@@ -61,6 +61,9 @@ struct GemmArgs {
   float* Cf2;          // wgrad: the groups from `split` on go here
   int split;
   bool zero_tail;      // row-tiled: the rows of C beyond the last group come out as zeros
+  // the 256 x 256 kernel takes the groups of several ranks at once: Gr groups per rank, whose rows
+  // start at rank_rows * rank (cu counts from there)
+  int Gr, rank_rows;
 };
 
 enum { kModeScale = 0, kModeSwiglu = 1, kModeDual = 2, kModeWgrad = 3 };
@@ -84,14 +87,23 @@ __device__ __forceinline__ mep_bf16x8 mep_tr_pair(const char* lo, const char* hi
   return __builtin_bit_cast(mep_bf16x8, z);
 }
 
-// rows of C beyond the last group, zeroed by `parts` workgroups of `threads` threads
+// rows of C beyond a rank's last group, zeroed by `parts` workgroups of `threads` threads
 __device__ __forceinline__ void zero_tail_rows(const GemmArgs& a, int part, int parts, int threads) {
-  const int first = a.cu[a.G - 1];
-  const size_t bytes = (size_t)(a.M - first) * a.N * 2;  // N is a multiple of 128
-  char* base = (char*)(a.C + (size_t)first * a.N);
   const mep_u4 zero = {0u, 0u, 0u, 0u};
-  for (size_t o = ((size_t)part * threads + threadIdx.x) * 16; o < bytes; o += (size_t)parts * threads * 16)
-    mep_st16_stream(base + o, zero);
+  for (int r = 0; (r + 1) * a.Gr <= a.G; ++r) {
+    const int first = a.cu[(r + 1) * a.Gr - 1];
+    const size_t bytes = (size_t)(a.rank_rows - first) * a.N * 2;  // N is a multiple of 128
+    char* base = (char*)(a.C + ((size_t)r * a.rank_rows + first) * a.N);
+    for (size_t o = ((size_t)part * threads + threadIdx.x) * 16; o < bytes; o += (size_t)parts * threads * 16)
+      mep_st16_stream(base + o, zero);
+  }
+}
+
+// first row / end row of group gi
+__device__ __forceinline__ int group_end(const GemmArgs& a, int gi) { return gi / a.Gr * a.rank_rows + a.cu[gi]; }
+__device__ __forceinline__ int group_beg(const GemmArgs& a, int gi) {
+  const int r = gi / a.Gr;
+  return r * a.rank_rows + (gi > r * a.Gr ? a.cu[gi - 1] : 0);
 }
 
 // Producer / consumer waves.  Two producer waves stream the tiles from global
@@ -470,8 +482,8 @@ struct PTiles {
   const GemmArgs& a;
   const Wgrad2Map& map;
   int xcd, w, nw, count, first_item, r;  // this workgroup among the XCD's, tiles of the XCD, round
-  int c0, carry, cbeg;                   // row-tiled: 64 groups, one per lane; tiles and row before them
-  int incl, end;                         // tiles up to and including the group, its end
+  int c0, carry;             // row-tiled: 64 groups, one per lane; tiles before them
+  int incl, end, blocks;     // tiles up to and including the group, its end, its 128-row blocks
   int g, m0, n0, kbeg, KT;
   bool tall;
   __device__ __forceinline__ PTiles(const GemmArgs& a_, const Wgrad2Map& map_) : a(a_), map(map_) {
@@ -497,11 +509,11 @@ struct PTiles {
   __device__ __forceinline__ void chunk(int c) {
     c0 = c;
     const int gi = c + (int)(threadIdx.x & 63);
-    end = gi < a.G ? a.cu[gi] : 0;
-    int beg = (gi > 0 && gi < a.G) ? a.cu[gi - 1] : 0;
+    end = gi < a.G ? group_end(a, gi) : 0;
+    int beg = gi < a.G ? group_beg(a, gi) : 0;
     asm volatile("" : "+v"(end), "+v"(beg));  // the loads end here, not inside the main loop
-    cbeg = __builtin_amdgcn_readfirstlane(beg);
-    incl = mep_wave_incl_scan(gi < a.G ? ((end - beg) / kBM + 1) >> 1 : 0);
+    blocks = (end - beg) / kBM;
+    incl = mep_wave_incl_scan((blocks + 1) >> 1);
   }
   // the next tile with work; false: no more
   __device__ __forceinline__ bool next() {
@@ -523,10 +535,12 @@ struct PTiles {
         const int sz = map.size(xe);
         const int u = local / sz, sl = map.lo(xe) + (local - u * sz);
         m0 = (map.slice_m ? sl : u) * kPT; n0 = (map.slice_m ? u : sl) * kPT;
-        typedef const __attribute__((address_space(4))) int* cptr;
-        kbeg = g > 0 ? ((cptr)a.cu)[g - 1] : 0;
-        KT = (((cptr)a.cu)[g] - kbeg) / kBK;
-        if (KT == 0 && g >= a.skip_from) continue;
+        typedef const __attribute__((address_space(4))) int* cptr;  // scalar loads
+        const int rank = g / a.Gr, l = g - rank * a.Gr;
+        const int first = l > 0 ? ((cptr)a.cu)[g - 1] : 0;
+        KT = (((cptr)a.cu)[g] - first) / kBK;
+        kbeg = rank * a.rank_rows + first;
+        if (KT == 0 && l >= a.skip_from) continue;
         return true;
       }
       return find(item);
@@ -541,8 +555,8 @@ struct PTiles {
         g = c0 + src;
         const int before = src > 0 ? __builtin_amdgcn_readlane(incl, src - 1) : 0;
         const int hs = __builtin_amdgcn_readlane(incl, src) - before, first = carry + before;
-        const int gbeg = src > 0 ? __builtin_amdgcn_readlane(end, src - 1) : cbeg;
         const int gend = __builtin_amdgcn_readlane(end, src);
+        const int gbeg = gend - __builtin_amdgcn_readlane(blocks, src) * kBM;
         const int local = L0 - first * a.ntiles;
         const int panel = local / (kPPanel * a.ntiles);
         const int within = local - panel * (kPPanel * a.ntiles);
@@ -723,8 +737,13 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
   while (cp.next()) {
     const int g = cp.g, m0 = cp.m0, n0 = cp.n0, KT = cp.KT;
     const bool tall = cp.tall;
-    float* cf = !WGRAD ? nullptr
-                : (g < a.split ? a.Cf + (size_t)g * a.M * a.N : a.Cf2 + (size_t)(g - a.split) * a.M * a.N);
+    float* cf = nullptr;
+    if (WGRAD) {
+      const int rank = g / a.Gr, l = g - rank * a.Gr;
+      const size_t mn = (size_t)a.M * a.N;
+      cf = l < a.split ? a.Cf + ((size_t)rank * a.split + l) * mn
+                       : a.Cf2 + ((size_t)rank * (a.Gr - a.split) + l - a.split) * mn;
+    }
     if (WGRAD && KT == 0) {  // a group without rows: whole 1 KB rows of zeroes per wave instruction
       typedef float f32x4 __attribute__((ext_vector_type(4)));
       const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
@@ -872,14 +891,15 @@ __global__ __launch_bounds__(256) void transpose16_kernel(const uint16_t* __rest
 struct SwigluBwdArgs {
   const uint16_t* dh; const uint16_t* gate; const uint16_t* up; const float* scale; const int* cu;
   uint16_t* dgate; uint16_t* dup; uint16_t* hs; float* dscale;
-  int M, N, G;
+  int M, N, G, rank_rows;  // G groups and rank_rows rows per rank
 };
 
 __global__ __launch_bounds__(256) void swiglu_bwd_kernel(SwigluBwdArgs a) {
   const int lane = threadIdx.x & 63;
   const int m = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (m >= a.M) return;
-  const bool live = m < a.cu[a.G - 1];
+  const int rank = m / a.rank_rows;
+  const bool live = m - rank * a.rank_rows < a.cu[(rank + 1) * a.G - 1];
   const float s = a.scale ? a.scale[m] : 1.0f;
   const size_t row = (size_t)m * a.N;
   float dot = 0.0f;
@@ -1000,7 +1020,18 @@ GemmArgs nt_args(const void* A, const void* B, const void* B2, const int32_t* cu
   a.mtiles = M / kBM;
   a.ntiles = N / cols_per_tile;
   a.ld = K;
+  a.Gr = G;
+  a.rank_rows = M;
   return a;
+}
+
+// the arguments of one rank's product made those of `nranks` ranks' whose operands lie behind each other
+bool for_ranks(GemmArgs& a, int nranks) {
+  if (nranks < 1 || (int64_t)a.M * nranks > INT32_MAX || (int64_t)a.G * nranks > INT32_MAX) return false;
+  a.M *= nranks;
+  a.G *= nranks;
+  a.mtiles *= nranks;
+  return true;
 }
 
 // Which tiles.  The 256 x 256 kernel is the faster one wherever its tiles are filled.  Where the
@@ -1013,6 +1044,7 @@ GemmArgs nt_args(const void* A, const void* B, const void* B2, const int32_t* cu
 std::atomic<int> g_forced_row_tile{0};
 
 static bool use_256_tiles(const GemmArgs& a) {
+  if (a.G != a.Gr) return true;  // several ranks
   const int forced = g_forced_row_tile.load(std::memory_order_relaxed);
   if (forced) return forced == 256;
   return 2 * ((int64_t)a.M - (int64_t)(kBM - 1) * a.G) >= (int64_t)kBM * a.G;
@@ -1027,7 +1059,7 @@ int row_tiled(const GemmArgs& a, hipStream_t st) {
 
 int gemm_nt_forward(const void* A, const void* B, const void* B_up, const int32_t* cu, int G, void* C,
                     void* C_gate, void* C_up, const float* row_scale, int M, int N, int K, int swiglu,
-                    bool zero_tail, void* stream) {
+                    bool zero_tail, void* stream, int nranks = 1) {
   const int cols = swiglu ? kBN / 2 : kBN;
   const int rc = check_nt_shapes(A, B, cu, C, M, N, K, G, cols);
   if (rc != MEP_OK) return rc;
@@ -1040,13 +1072,14 @@ int gemm_nt_forward(const void* A, const void* B, const void* B_up, const int32_
   a.Cg = (uint16_t*)C_gate;
   a.Cu = (uint16_t*)C_up;
   a.zero_tail = zero_tail;
+  if (!for_ranks(a, nranks)) return MEP_ERR_UNSUPPORTED;
   return swiglu ? row_tiled<kModeSwiglu, false>(a, (hipStream_t)stream)
                 : row_tiled<kModeScale, false>(a, (hipStream_t)stream);
 }
 
 // input gradients: weights as [K, N], one or two pairs
 int gemm_nn(const void* A1, const void* B1, const void* A2, const void* B2, const int32_t* cu, int G, void* C,
-            const float* row_scale, int M, int N, int K, bool zero_tail, void* stream) {
+            const float* row_scale, int M, int N, int K, bool zero_tail, void* stream, int nranks = 1) {
   const int rc = check_nt_shapes(A1, B1, cu, C, M, N, K, G, kBN);
   if (rc != MEP_OK) return rc;
   MEP_REQUIRE(2 * (int64_t)K < ((int64_t)1 << 30), MEP_ERR_UNSUPPORTED);
@@ -1055,12 +1088,13 @@ int gemm_nn(const void* A1, const void* B1, const void* A2, const void* B2, cons
   GemmArgs a = nt_args(A1, B1, B2, cu, C, row_scale, M, N, K, G, kBN);
   a.A2 = (const uint16_t*)A2;
   a.zero_tail = zero_tail;
+  if (!for_ranks(a, nranks)) return MEP_ERR_UNSUPPORTED;
   return A2 ? row_tiled<kModeDual, true>(a, (hipStream_t)stream) : row_tiled<kModeScale, true>(a, (hipStream_t)stream);
 }
 
 // weight gradient from the activations as they are; the groups from `split` on go to C2
 int wgrad_tn(const void* X1, const void* X2, const int32_t* cu, int G, float* C, float* C2, int split, int Ma, int Nb,
-             int64_t rows, int skip_empty_from, void* stream) {
+             int64_t rows, int skip_empty_from, void* stream, int nranks = 1) {
   MEP_REQUIRE(X1 && X2 && cu && C && C2, MEP_ERR_INVALID_ARG);
   MEP_REQUIRE(Ma > 0 && Nb > 0 && G > 0 && rows > 0 && skip_empty_from >= 0, MEP_ERR_INVALID_ARG);
   MEP_REQUIRE(Ma % kPT == 0 && Nb % kPT == 0 && G % 2 == 0 && rows % kBM == 0, MEP_ERR_UNSUPPORTED);
@@ -1069,9 +1103,12 @@ int wgrad_tn(const void* X1, const void* X2, const int32_t* cu, int G, float* C,
                   ((uintptr_t)C2 % 16 == 0), MEP_ERR_ALIGNMENT);
   GemmArgs a{};
   a.A = (const uint16_t*)X1; a.B = (const uint16_t*)X2; a.cu = cu; a.Cf = C; a.Cf2 = C2; a.split = split;
-  a.M = Ma; a.N = Nb; a.K = 0; a.G = G;
+  a.M = Ma; a.N = Nb; a.K = 0; a.G = G * nranks;
   a.ld = rows;
+  a.Gr = G;
+  a.rank_rows = (int)rows;
   a.skip_from = skip_empty_from;
+  MEP_REQUIRE(rows * nranks <= INT32_MAX, MEP_ERR_UNSUPPORTED);
   return wgrad_pp_launch<true>(a, (hipStream_t)stream);
 }
 
@@ -1172,6 +1209,7 @@ extern "C" int mep_grouped_gemm_wgrad(const void* At, const void* Bt, const int3
   MEP_REQUIRE(skip_empty_from >= 0, MEP_ERR_INVALID_ARG);
   a.skip_from = skip_empty_from;
   a.split = G;
+  a.Gr = G;
   // an expert's shapes: 256 x 256 tiles (whose lane offsets are 32 bits)
   if (Ma % kPT == 0 && Nb % kPT == 0 && G % 2 == 0 && (uintptr_t)C % 16 == 0 && ld < ((int64_t)1 << 22))
     return wgrad_pp_launch<false>(a, (hipStream_t)stream);
@@ -1186,30 +1224,58 @@ extern "C" int mep_grouped_gemm_wgrad_tn(const void* X1, const void* X2, const i
   return wgrad_tn(X1, X2, cu_seqlens, G, C, C, G, Ma, Nb, rows, skip_empty_from, stream);
 }
 
+namespace {
+int swiglu_bwd_launch(const void* dh, const void* gate_pre, const void* up_pre, const float* row_scale,
+                      const int32_t* cu_seqlens, int G, void* dgate, void* dup, void* hs, float* dscale, int M, int N,
+                      int rank_rows, void* stream) {
+  MEP_REQUIRE(dh && gate_pre && up_pre && cu_seqlens && dgate && dup && hs, MEP_ERR_INVALID_ARG);
+  MEP_REQUIRE(M > 0 && N > 0 && G > 0, MEP_ERR_INVALID_ARG);
+  MEP_REQUIRE(N % 8 == 0, MEP_ERR_UNSUPPORTED);
+  MEP_REQUIRE(((uintptr_t)dh % 16 == 0) && ((uintptr_t)gate_pre % 16 == 0) && ((uintptr_t)up_pre % 16 == 0) &&
+                  ((uintptr_t)dgate % 16 == 0) && ((uintptr_t)dup % 16 == 0) && ((uintptr_t)hs % 16 == 0),
+              MEP_ERR_ALIGNMENT);
+  SwigluBwdArgs a;
+  a.dh = (const uint16_t*)dh; a.gate = (const uint16_t*)gate_pre; a.up = (const uint16_t*)up_pre;
+  a.scale = row_scale; a.cu = cu_seqlens;
+  a.dgate = (uint16_t*)dgate; a.dup = (uint16_t*)dup; a.hs = (uint16_t*)hs; a.dscale = dscale;
+  a.M = M; a.N = N; a.G = G; a.rank_rows = rank_rows;
+  hipLaunchKernelGGL(swiglu_bwd_kernel, dim3((M + 3) / 4), dim3(256), 0, (hipStream_t)stream, a);
+  return mep_launch_status();
+}
+}  // namespace
+
+extern "C" int mep_swiglu_bwd(const void* dh, const void* gate_pre, const void* up_pre,
+                              const float* row_scale, const int32_t* cu_seqlens, int G, void* dgate,
+                              void* dup, void* hs, float* dscale, int M, int N, void* stream) {
+  return swiglu_bwd_launch(dh, gate_pre, up_pre, row_scale, cu_seqlens, G, dgate, dup, hs, dscale, M, N, M, stream);
+}
+
 extern "C" int mep_ffn_forward(const void* rows, const float* slots, const int32_t* cu_seqlens, int G, const void* gate,
                                const void* up, const void* down, void* act, void* gate_pre, void* up_pre, void* y,
-                               int M, int H, int Hp, void* stream) {
-  const int rc = gemm_nt_forward(rows, gate, up, cu_seqlens, G, act, gate_pre, up_pre, nullptr, M, Hp, H, 1, false, stream);
+                               int nranks, int M, int H, int Hp, void* stream) {
+  const int rc = gemm_nt_forward(rows, gate, up, cu_seqlens, G, act, gate_pre, up_pre, nullptr, M, Hp, H, 1, false, stream, nranks);
   if (rc != MEP_OK) return rc;
-  return gemm_nt_forward(act, down, nullptr, cu_seqlens, G, y, nullptr, nullptr, slots, M, H, Hp, 0, true, stream);
+  return gemm_nt_forward(act, down, nullptr, cu_seqlens, G, y, nullptr, nullptr, slots, M, H, Hp, 0, true, stream, nranks);
 }
 
 extern "C" int mep_ffn_backward(const void* dy, const void* rows, const float* slots, const int32_t* cu_seqlens, int G,
                                 const void* gate, const void* up, const void* down, const void* gate_pre,
                                 const void* up_pre, void* dh, void* dgate, void* dup, void* hs, float* dslots,
-                                void* drows, float* const* wgrads, float* const* wgrads_from_split, int split, int M,
-                                int H, int Hp, int skip_empty_from, void* stream) {
+                                void* drows, float* const* wgrads, float* const* wgrads_from_split, int split,
+                                int nranks, int M, int H, int Hp, int skip_empty_from, void* stream) {
   MEP_REQUIRE(gate && up && wgrads && wgrads_from_split && drows, MEP_ERR_INVALID_ARG);
   MEP_REQUIRE((slots == nullptr) == (dslots == nullptr), MEP_ERR_INVALID_ARG);
   // gradient of the unscaled activation: dy * down[g], down[g] is [H, H'] = [K, N]
-  int rc = gemm_nn(dy, down, nullptr, nullptr, cu_seqlens, G, dh, nullptr, M, Hp, H, false, stream);
-  if (rc == MEP_OK) rc = mep_swiglu_bwd(dh, gate_pre, up_pre, slots, cu_seqlens, G, dgate, dup, hs, dslots, M, Hp, stream);
-  if (rc == MEP_OK) rc = gemm_nn(dgate, gate, dup, up, cu_seqlens, G, drows, nullptr, M, H, Hp, true, stream);
+  MEP_REQUIRE(nranks > 0 && (int64_t)M * nranks <= INT32_MAX && (int64_t)G * nranks <= INT32_MAX, MEP_ERR_UNSUPPORTED);
+  int rc = gemm_nn(dy, down, nullptr, nullptr, cu_seqlens, G, dh, nullptr, M, Hp, H, false, stream, nranks);
+  if (rc == MEP_OK)
+    rc = swiglu_bwd_launch(dh, gate_pre, up_pre, slots, cu_seqlens, G, dgate, dup, hs, dslots, M * nranks, Hp, M, stream);
+  if (rc == MEP_OK) rc = gemm_nn(dgate, gate, dup, up, cu_seqlens, G, drows, nullptr, M, H, Hp, true, stream, nranks);
   const void* x1[3] = {dgate, dup, dy};
   const void* x2[3] = {rows, rows, hs};
   for (int i = 0; i < 3 && rc == MEP_OK; ++i)
     rc = wgrad_tn(x1[i], x2[i], cu_seqlens, G, wgrads[i], wgrads_from_split[i], split, i < 2 ? Hp : H, i < 2 ? H : Hp,
-                  M, skip_empty_from, stream);
+                  M, skip_empty_from, stream, nranks);
   return rc;
 }
 
@@ -1223,20 +1289,3 @@ extern "C" int mep_transpose_bf16(const void* src, void* dst, int batch, int row
   return mep_launch_status();
 }
 
-extern "C" int mep_swiglu_bwd(const void* dh, const void* gate_pre, const void* up_pre,
-                              const float* row_scale, const int32_t* cu_seqlens, int G, void* dgate,
-                              void* dup, void* hs, float* dscale, int M, int N, void* stream) {
-  MEP_REQUIRE(dh && gate_pre && up_pre && cu_seqlens && dgate && dup && hs, MEP_ERR_INVALID_ARG);
-  MEP_REQUIRE(M > 0 && N > 0 && G > 0, MEP_ERR_INVALID_ARG);
-  MEP_REQUIRE(N % 8 == 0, MEP_ERR_UNSUPPORTED);
-  MEP_REQUIRE(((uintptr_t)dh % 16 == 0) && ((uintptr_t)gate_pre % 16 == 0) && ((uintptr_t)up_pre % 16 == 0) &&
-                  ((uintptr_t)dgate % 16 == 0) && ((uintptr_t)dup % 16 == 0) && ((uintptr_t)hs % 16 == 0),
-              MEP_ERR_ALIGNMENT);
-  SwigluBwdArgs a;
-  a.dh = (const uint16_t*)dh; a.gate = (const uint16_t*)gate_pre; a.up = (const uint16_t*)up_pre;
-  a.scale = row_scale; a.cu = cu_seqlens;
-  a.dgate = (uint16_t*)dgate; a.dup = (uint16_t*)dup; a.hs = (uint16_t*)hs; a.dscale = dscale;
-  a.M = M; a.N = N; a.G = G;
-  hipLaunchKernelGGL(swiglu_bwd_kernel, dim3((M + 3) / 4), dim3(256), 0, (hipStream_t)stream, a);
-  return mep_launch_status();
-}

@@ -446,11 +446,14 @@ PyObject* py_reduce(PyObject*, PyObject* const* args, Py_ssize_t n) {
   }
   Async as(c, async);
   if (!as.begin({&etc, l[0], l[1], l[2], p[0], p[1], p[2]})) return nullptr;
+  float *lp[3], *pp[3];
+  int64_t stride[3], elems[3];
   for (int i = 0; i < 3; ++i) {
-    const int rc = mep_grad_reduce(ptr<float>(*l[i]), ptr<float>(*p[i]), p[i]->stride(0), ptr<int>(etc), c.rank, c.epn,
-                                   c.R, l[i]->size(1) * l[i]->size(2), 0, as.stream);
-    if (failed(rc, "mep_grad_reduce")) return nullptr;
+    lp[i] = ptr<float>(*l[i]); pp[i] = ptr<float>(*p[i]);
+    stride[i] = p[i]->stride(0); elems[i] = l[i]->size(1) * l[i]->size(2);
   }
+  const int rc = mep_grad_reduce_batch(3, lp, pp, stride, elems, ptr<int>(etc), c.rank, 1, c.epn, c.R, 0, as.stream);
+  if (failed(rc, "mep_grad_reduce")) return nullptr;
   if (async) return as.end();
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
@@ -459,9 +462,19 @@ PyObject* py_reduce(PyObject*, PyObject* const* args, Py_ssize_t n) {
 // ---- the expert FFN --------------------------------------------------------------------------
 struct Ffn {
   const at::Tensor *rows, *slots = nullptr, *cu, *gate, *up, *down;
-  int M, H, Hp, G;
+  int n, M, H, Hp, G;  // ranks, rows and groups of a rank
+  bool many;           // every tensor has a leading rank dimension
   at::TensorOptions bf16, f32;
   hipStream_t stream;
+  // shape of a tensor with `s` per rank
+  c10::SmallVector<int64_t, 5> per_rank(std::initializer_list<int64_t> s) const {
+    c10::SmallVector<int64_t, 5> v;
+    if (many) v.push_back(n);
+    v.append(s.begin(), s.end());
+    return v;
+  }
+  bool of(const at::Tensor& t, std::initializer_list<int64_t> s) const { return t.sizes() == c10::IntArrayRef(per_rank(s)); }
+  at::Tensor make(std::initializer_list<int64_t> s, const at::TensorOptions& o) const { return at::empty(per_rank(s), o); }
 };
 
 bool dense(const at::Tensor* t, at::ScalarType dt, const at::Tensor& like) {
@@ -471,27 +484,33 @@ bool dense(const at::Tensor* t, at::ScalarType dt, const at::Tensor& like) {
 // args: rows, slots, cu, gate, up, down, token_padding
 bool read_ffn(PyObject* const* args, Ffn* f) {
   f->rows = tensor(args[0]);
-  if (!f->rows || !f->rows->is_cuda() || !dense(f->rows, at::kBFloat16, *f->rows) || f->rows->dim() != 2) return false;
+  if (!f->rows || !f->rows->is_cuda() || !dense(f->rows, at::kBFloat16, *f->rows)) return false;
   const at::Tensor& x = *f->rows;
+  if (x.dim() != 2 && x.dim() != 3) return false;
+  f->many = x.dim() == 3;
+  const int d = f->many;
   f->cu = tensor(args[2]); f->gate = tensor(args[3]); f->up = tensor(args[4]); f->down = tensor(args[5]);
-  if (!f->cu || f->cu->scalar_type() != at::kInt || !f->cu->is_contiguous() || f->cu->dim() != 1 ||
+  if (!f->cu || f->cu->scalar_type() != at::kInt || !f->cu->is_contiguous() || f->cu->dim() != 1 + d ||
       f->cu->device() != x.device())
     return false;
   if (!dense(f->gate, at::kBFloat16, x) || !dense(f->up, at::kBFloat16, x) || !dense(f->down, at::kBFloat16, x)) return false;
-  const int64_t M = x.size(0), H = x.size(1), G = f->cu->numel();
-  if (f->gate->dim() != 3 || M % 128 != 0 || H % 256 != 0 || M <= 0 || M > INT32_MAX || H > (1 << 20) || G <= 0) return false;
-  const int64_t Hp = f->gate->size(1);
+  const int64_t n = d ? x.size(0) : 1, M = x.size(d), H = x.size(d + 1), G = f->cu->size(d);
+  if (f->gate->dim() != 3 + d || M % 128 != 0 || H % 256 != 0 || n <= 0 || M <= 0 || n * M > INT32_MAX ||
+      H > (1 << 20) || G <= 0)
+    return false;
+  const int64_t Hp = f->gate->size(1 + d);
   if (Hp % 128 != 0 || Hp <= 0 || Hp > (1 << 20)) return false;
-  if (!shape(*f->gate, {G, Hp, H}) || !shape(*f->up, {G, Hp, H}) || !shape(*f->down, {G, H, Hp})) return false;
+  f->n = (int)n; f->M = (int)M; f->H = (int)H; f->Hp = (int)Hp; f->G = (int)G;
+  if (d && f->cu->size(0) != n) return false;
+  if (!f->of(*f->gate, {G, Hp, H}) || !f->of(*f->up, {G, Hp, H}) || !f->of(*f->down, {G, H, Hp})) return false;
   if (args[1] != Py_None) {
     f->slots = tensor(args[1]);
-    if (!dense(f->slots, at::kFloat, x) || f->slots->numel() != M) return false;
+    if (!dense(f->slots, at::kFloat, x) || f->slots->numel() != n * M) return false;
   }
   if (!PyLong_CheckExact(args[6])) return false;
   const long tp = PyLong_AsLong(args[6]);
   if (tp <= 0 || tp % 128 != 0) { PyErr_Clear(); return false; }
   if (x.device().index() != c10::hip::current_device()) return false;
-  f->M = (int)M; f->H = (int)H; f->Hp = (int)Hp; f->G = (int)G;
   f->bf16 = x.options(); f->f32 = x.options().dtype(at::kFloat);
   f->stream = c10::hip::getCurrentHIPStream(x.device().index()).stream();
   return true;
@@ -504,11 +523,11 @@ PyObject* py_ffn_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   Ffn f;
   if (!read_ffn(args, &f)) return new_none();
   const bool train = args[7] == Py_True;
-  at::Tensor y = at::empty({f.M, f.H}, f.bf16), act = at::empty({f.M, f.Hp}, f.bf16), gp, up;
-  if (train) { gp = at::empty({f.M, f.Hp}, f.bf16); up = at::empty({f.M, f.Hp}, f.bf16); }
+  at::Tensor y = f.make({f.M, f.H}, f.bf16), act = f.make({f.M, f.Hp}, f.bf16), gp, up;
+  if (train) { gp = f.make({f.M, f.Hp}, f.bf16); up = f.make({f.M, f.Hp}, f.bf16); }
   const int rc = mep_ffn_forward(f.rows->data_ptr(), f.slots ? ptr<float>(*f.slots) : nullptr, ptr<int>(*f.cu), f.G,
                                  f.gate->data_ptr(), f.up->data_ptr(), f.down->data_ptr(), act.data_ptr(),
-                                 ptr<void>(gp), ptr<void>(up), y.data_ptr(), f.M, f.H, f.Hp, f.stream);
+                                 ptr<void>(gp), ptr<void>(up), y.data_ptr(), f.n, f.M, f.H, f.Hp, f.stream);
   if (failed(rc, "mep_ffn_forward")) return nullptr;
   if (!train) return THPVariable_Wrap(y);
   return Py_BuildValue("(N(NN))", THPVariable_Wrap(y), THPVariable_Wrap(gp), THPVariable_Wrap(up));
@@ -519,6 +538,7 @@ PyObject* py_ffn_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
 //              own, from_slots): own and from_slots are tuples of three fp32 tensors for the
 //              weight gradients of the lower and the upper half of the groups, or None
 //   -> (drows, dslots, dgate, dup, ddown), the last three None where own is given
+// Both take several ranks' tensors with a leading rank dimension (the backward with own given).
 PyObject* py_ffn_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (n != 13) { PyErr_SetString(PyExc_TypeError, "ffn_backward takes 13 arguments"); return nullptr; }
@@ -526,10 +546,10 @@ PyObject* py_ffn_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (!read_ffn(args, &f)) return new_none();
   const at::Tensor *dy = tensor(args[7]), *gp = tensor(args[8]), *up = tensor(args[9]);
   if (!dense(dy, at::kBFloat16, *f.rows) || !dense(gp, at::kBFloat16, *f.rows) || !dense(up, at::kBFloat16, *f.rows) ||
-      !shape(*dy, {f.M, f.H}) || !shape(*gp, {f.M, f.Hp}) || !shape(*up, {f.M, f.Hp}))
+      !f.of(*dy, {f.M, f.H}) || !f.of(*gp, {f.M, f.Hp}) || !f.of(*up, {f.M, f.Hp}))
     return new_none();
-  if (f.Hp % 256 != 0 || f.G % 2 != 0) return new_none();
   const bool skip = args[10] == Py_True, given = args[11] != Py_None;
+  if (f.Hp % 256 != 0 || f.G % 2 != 0 || (f.many && !given)) return new_none();
   float *w[3], *w2[3];
   at::Tensor dw[3];
   for (int i = 0; i < 3; ++i) {
@@ -539,8 +559,8 @@ PyObject* py_ffn_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
           PyTuple_GET_SIZE(args[12]) != 3)
         return new_none();
       const at::Tensor *o = tensor(PyTuple_GET_ITEM(args[11], i)), *s = tensor(PyTuple_GET_ITEM(args[12], i));
-      if (!dense(o, at::kFloat, *f.rows) || !dense(s, at::kFloat, *f.rows) || !shape(*o, {f.G / 2, a, b}) ||
-          !shape(*s, {f.G / 2, a, b}))
+      if (!dense(o, at::kFloat, *f.rows) || !dense(s, at::kFloat, *f.rows) || !f.of(*o, {f.G / 2, a, b}) ||
+          !f.of(*s, {f.G / 2, a, b}))
         return new_none();
       w[i] = ptr<float>(*o); w2[i] = ptr<float>(*s);
     } else {
@@ -548,13 +568,13 @@ PyObject* py_ffn_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
       w[i] = ptr<float>(dw[i]); w2[i] = w[i] + (int64_t)(f.G / 2) * a * b;
     }
   }
-  at::Tensor drows = at::empty({f.M, f.H}, f.bf16), dslots, dh = at::empty({f.M, f.Hp}, f.bf16),
-             dg = at::empty({f.M, f.Hp}, f.bf16), du = at::empty({f.M, f.Hp}, f.bf16), hs = at::empty({f.M, f.Hp}, f.bf16);
-  if (f.slots) dslots = at::empty({f.M}, f.f32);
+  at::Tensor drows = f.make({f.M, f.H}, f.bf16), dslots, dh = f.make({f.M, f.Hp}, f.bf16),
+             dg = f.make({f.M, f.Hp}, f.bf16), du = f.make({f.M, f.Hp}, f.bf16), hs = f.make({f.M, f.Hp}, f.bf16);
+  if (f.slots) dslots = f.make({f.M}, f.f32);
   const int rc = mep_ffn_backward(dy->data_ptr(), f.rows->data_ptr(), f.slots ? ptr<float>(*f.slots) : nullptr,
                                   ptr<int>(*f.cu), f.G, f.gate->data_ptr(), f.up->data_ptr(), f.down->data_ptr(),
                                   gp->data_ptr(), up->data_ptr(), dh.data_ptr(), dg.data_ptr(), du.data_ptr(),
-                                  hs.data_ptr(), ptr<float>(dslots), drows.data_ptr(), w, w2, f.G / 2, f.M, f.H, f.Hp,
+                                  hs.data_ptr(), ptr<float>(dslots), drows.data_ptr(), w, w2, f.G / 2, f.n, f.M, f.H, f.Hp,
                                   skip ? f.G / 2 : f.G, f.stream);
   if (failed(rc, "mep_ffn_backward")) return nullptr;
   auto give = [](const at::Tensor& t) { return t.defined() ? THPVariable_Wrap(t) : new_none(); };

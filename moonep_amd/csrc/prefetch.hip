@@ -268,11 +268,13 @@ struct PullArgs {
   int ntensors, rank, epn, R;
 };
 
+// blockIdx.y is one of several ranks that are filled in one launch.
 // The occupied slots of `rank` form the work list (slot b <- expert etc[rank, b]); persistent
 // workgroups walk (tensor, occupied slot, tile) in the tile layout of the push kernel, the
 // next tile's loads issued before the current tile's stores.  LDS: slot[epn], expert[epn], n.
 __global__ __launch_bounds__(kBlock) void prefetch_pull_kernel(PullArgs a) {
   extern __shared__ int smem[];
+  const int rank = a.rank + blockIdx.y;
   int* s_slot = smem;
   int* s_exp = smem + a.epn;
   int* s_n = s_exp + a.epn;
@@ -281,7 +283,7 @@ __global__ __launch_bounds__(kBlock) void prefetch_pull_kernel(PullArgs a) {
     int n = 0;
     for (int c = 0; c < a.epn; c += 64) {
       const int b = c + lane;
-      const int e = b < a.epn ? a.etc[a.rank * a.epn + b] : -1;
+      const int e = b < a.epn ? a.etc[rank * a.epn + b] : -1;
       const bool ok = e >= 0 && e < a.R * a.epn;
       const uint64_t m = __ballot(ok);
       if (ok) {
@@ -325,7 +327,7 @@ __global__ __launch_bounds__(kBlock) void prefetch_pull_kernel(PullArgs a) {
   };
   auto store = [&](const Tile& p, const mep_u4* v) {
     const int64_t bytes = a.st[p.ti].bytes;
-    char* dst = a.pool[p.ti] + (int64_t)a.rank * a.rank_stride[p.ti] + (int64_t)p.b * bytes + p.off;
+    char* dst = a.pool[p.ti] + (int64_t)rank * a.rank_stride[p.ti] + (int64_t)p.b * bytes + p.off;
     if (p.whole) {
 #pragma unroll
       for (int i = 0; i < kVecPerThread; ++i) mep_st16_through(dst + (int64_t)i * p.step, v[i]);
@@ -419,6 +421,39 @@ __global__ __launch_bounds__(kBlock) void copy_kernel(CopyArgs a) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// fp32 master weights -> bf16 compute views: one launch for all projections,
+// eight elements per thread and step (two 16-byte loads, one store), bound by
+// HBM.  A rank's block of the destination may be followed by other memory (its
+// prefetch slots), hence the two rank strides.
+// ---------------------------------------------------------------------------
+struct CastArgs {
+  const float* src[kMaxTensors];
+  uint16_t* dst[kMaxTensors];
+  int64_t elems[kMaxTensors];       // of a rank's block, a multiple of 8
+  int64_t dst_stride[kMaxTensors];  // elements between ranks' blocks of dst; src is dense
+};
+
+__global__ __launch_bounds__(kBlock) void cast_kernel(CastArgs a) {
+  const int ti = blockIdx.z;
+  const float* src = a.src[ti] + (int64_t)blockIdx.y * a.elems[ti];
+  uint16_t* dst = a.dst[ti] + (int64_t)blockIdx.y * a.dst_stride[ti];
+  const int64_t n = a.elems[ti], step = (int64_t)gridDim.x * kBlock * 8;
+  auto pack = [](mep_u4 x, mep_u4 y) {
+    auto f = [](uint32_t v) { return __uint_as_float(v); };
+    return mep_u4{mep_pack_bf16(f(x[0]), f(x[1])), mep_pack_bf16(f(x[2]), f(x[3])),
+                  mep_pack_bf16(f(y[0]), f(y[1])), mep_pack_bf16(f(y[2]), f(y[3]))};
+  };
+  int64_t i = ((int64_t)blockIdx.x * kBlock + threadIdx.x) * 8;
+  for (; i + step < n; i += 2 * step) {  // two steps' loads in flight
+    const mep_u4 x0 = mep_ld16_stream(src + i), y0 = mep_ld16_stream(src + i + 4);
+    const mep_u4 x1 = mep_ld16_stream(src + i + step), y1 = mep_ld16_stream(src + i + step + 4);
+    mep_st16(dst + i, pack(x0, y0));
+    mep_st16(dst + i + step, pack(x1, y1));
+  }
+  if (i < n) mep_st16(dst + i, pack(mep_ld16_stream(src + i), mep_ld16_stream(src + i + 4)));
+}
+
 struct ReduceArgs {
   float* local_grad;
   float* pool;
@@ -427,6 +462,27 @@ struct ReduceArgs {
   const int* etc;
   int rank, epn, R;
   unsigned flags;       // MEP_REDUCE_*
+};
+
+constexpr int kMaxReduce = 3;
+
+// One launch sums several projections, one after the other with all workgroups on each (all at
+// once was 17 % slower: three times as many streams), over one slot table; a launch per projection
+// ends and begins with a few microseconds in which only part of the chip has work.  blockIdx.y is
+// the rank, for a caller that plays several.
+struct ReduceBatch {
+  float* local_grad[kMaxReduce];
+  float* pool[kMaxReduce];
+  int64_t rank_stride[kMaxReduce];
+  int64_t elems[kMaxReduce];
+  const int* etc;
+  int ntensors, rank0, epn, R;  // local_grad: a block of epn experts per rank
+  unsigned flags;
+  __device__ __forceinline__ ReduceArgs of(int t) const {
+    const int r = blockIdx.y;
+    return ReduceArgs{local_grad[t] + (int64_t)r * epn * elems[t], pool[t], rank_stride[t], elems[t],
+                      etc, rank0 + r, epn, R, flags};
+  }
 };
 
 typedef float mep_f4 __attribute__((ext_vector_type(4)));
@@ -455,32 +511,9 @@ __device__ __forceinline__ void clear_tile(const ReduceArgs& a, const SpreadTile
 //    as tiles of the spread layout, cost 7-16 % more time; separate short fill
 //    workgroups beside the summing ones are as fast but the host cannot know
 //    how many to launch.)
-__global__ __launch_bounds__(kBlock) void grad_reduce_kernel(ReduceArgs a) {
-  extern __shared__ int smem[];
+__device__ __forceinline__ void reduce_tensor(const ReduceArgs& a, const SlotTable& t, const int* occ, int64_t* sbase,
+                                              int n_active, int n_clear) {
   const SpreadTiles rt(a.elems * 4);
-  SlotTable t;
-  t.carve(smem, a.R, a.epn);
-  int* occ = smem + slot_table_ints(a.R, a.epn);  // [epn] own slots holding foreign experts, [1] their number
-  int64_t* sbase = (int64_t*)(smem + ((slot_table_ints(a.R, a.epn) + a.epn + 2) & ~1));  // [R*epn] byte offset in the pool of list entry i
-  if (threadIdx.x < 64) {
-    const int lane = threadIdx.x;
-    const int lo = a.rank * a.epn;
-    int n = 0;
-    for (int c = 0; c < a.epn; c += 64) {
-      const int b = c + lane;
-      const int e = b < a.epn ? a.etc[a.rank * a.epn + b] : -1;
-      // a clear-only call zeroes every occupied own slot as pieces
-      const bool foreign = e >= 0 && ((a.flags & MEP_REDUCE_CLEAR_ONLY) ||
-                                      (unsigned)(e - lo) >= (unsigned)a.epn);
-      const uint64_t m = __ballot(foreign);
-      if (foreign) occ[n + __popcll(m & mep_lanes_lt())] = b;
-      n += __popcll(m);
-    }
-    if (lane == 0) occ[a.epn] = n;
-  }
-  t.build<true>(a.etc, a.rank, a.R, a.epn);  // ends with a workgroup barrier
-  const int n_active = (a.flags & MEP_REDUCE_CLEAR_ONLY) ? 0 : t.misc[0];
-  const int n_clear = (a.flags & MEP_REDUCE_NO_CLEAR) ? 0 : occ[a.epn];
   const bool clear_as_read = a.flags == 0;  // own slots holding own experts, zeroed by their reader
   // where each entry of the slot lists starts in the pool, so that a tile only adds its offset
   for (int i = threadIdx.x; i < t.off[a.epn]; i += kBlock) {
@@ -626,6 +659,38 @@ __global__ __launch_bounds__(kBlock) void grad_reduce_kernel(ReduceArgs a) {
   }
 }
 
+__global__ __launch_bounds__(kBlock) void grad_reduce_kernel(ReduceBatch batch) {
+  extern __shared__ int smem[];
+  const ReduceArgs a = batch.of(0);
+  SlotTable t;
+  t.carve(smem, a.R, a.epn);
+  int* occ = smem + slot_table_ints(a.R, a.epn);  // [epn] own slots holding foreign experts, [1] their number
+  int64_t* sbase = (int64_t*)(smem + ((slot_table_ints(a.R, a.epn) + a.epn + 2) & ~1));  // [R*epn] byte offset in the pool of list entry i
+  if (threadIdx.x < 64) {
+    const int lane = threadIdx.x;
+    const int lo = a.rank * a.epn;
+    int n = 0;
+    for (int c = 0; c < a.epn; c += 64) {
+      const int b = c + lane;
+      const int e = b < a.epn ? a.etc[a.rank * a.epn + b] : -1;
+      // a clear-only call zeroes every occupied own slot as pieces
+      const bool foreign = e >= 0 && ((a.flags & MEP_REDUCE_CLEAR_ONLY) ||
+                                      (unsigned)(e - lo) >= (unsigned)a.epn);
+      const uint64_t m = __ballot(foreign);
+      if (foreign) occ[n + __popcll(m & mep_lanes_lt())] = b;
+      n += __popcll(m);
+    }
+    if (lane == 0) occ[a.epn] = n;
+  }
+  t.build<true>(a.etc, a.rank, a.R, a.epn);  // ends with a workgroup barrier
+  const int n_active = (a.flags & MEP_REDUCE_CLEAR_ONLY) ? 0 : t.misc[0];
+  const int n_clear = (a.flags & MEP_REDUCE_NO_CLEAR) ? 0 : occ[a.epn];
+  for (int i = 0; i < batch.ntensors; ++i) {
+    if (i > 0) __syncthreads();  // sbase of the tensor before is no longer read
+    reduce_tensor(batch.of(i), t, occ, sbase, n_active, n_clear);
+  }
+}
+
 }  // namespace
 
 extern "C" int mep_prefetch(int ntensors, const void* const* local, void* const* pool,
@@ -666,15 +731,14 @@ extern "C" int mep_prefetch(int ntensors, const void* const* local, void* const*
   return mep_launch_status();
 }
 
-extern "C" int mep_prefetch_pull(int ntensors, const void* const* owners,
-                                 const int64_t* owner_stride_bytes, void* const* pool,
-                                 const int64_t* rank_stride_bytes, const int64_t* bytes_per_expert,
-                                 const int32_t* experts_to_copy, int rank, int epn, int R,
-                                 void* stream) {
+namespace {
+int pull_launch(int ntensors, const void* const* owners, const int64_t* owner_stride_bytes, void* const* pool,
+                const int64_t* rank_stride_bytes, const int64_t* bytes_per_expert, const int32_t* experts_to_copy,
+                int rank, int nranks, int epn, int R, void* stream) {
   MEP_REQUIRE(owners && owner_stride_bytes && pool && rank_stride_bytes && bytes_per_expert &&
                   experts_to_copy, MEP_ERR_INVALID_ARG);
   MEP_REQUIRE(ntensors > 0 && ntensors <= kMaxTensors, MEP_ERR_INVALID_ARG);
-  MEP_REQUIRE(epn > 0 && R > 0 && rank >= 0 && rank < R, MEP_ERR_INVALID_ARG);
+  MEP_REQUIRE(epn > 0 && R > 0 && nranks > 0 && rank >= 0 && rank + nranks <= R, MEP_ERR_INVALID_ARG);
   const size_t lds = (2 * (size_t)epn + 1) * sizeof(int);
   MEP_REQUIRE(lds <= 64 * 1024, MEP_ERR_UNSUPPORTED);
   PullArgs a;
@@ -699,9 +763,29 @@ extern "C" int mep_prefetch_pull(int ntensors, const void* const* owners,
   MEP_REQUIRE(all_tiles * epn < ((int64_t)1 << 31), MEP_ERR_UNSUPPORTED);
   const int cus = mep_device_cu_count();
   int64_t blocks = 2 * (int64_t)(cus > 0 ? cus : 256);
+  blocks = (blocks + nranks - 1) / nranks;
   if (all_tiles * epn < blocks) blocks = all_tiles * epn;
-  hipLaunchKernelGGL(prefetch_pull_kernel, dim3((unsigned)blocks), dim3(kBlock), lds, (hipStream_t)stream, a);
+  hipLaunchKernelGGL(prefetch_pull_kernel, dim3((unsigned)blocks, nranks), dim3(kBlock), lds, (hipStream_t)stream, a);
   return mep_launch_status();
+}
+}  // namespace
+
+extern "C" int mep_prefetch_pull(int ntensors, const void* const* owners,
+                                 const int64_t* owner_stride_bytes, void* const* pool,
+                                 const int64_t* rank_stride_bytes, const int64_t* bytes_per_expert,
+                                 const int32_t* experts_to_copy, int rank, int epn, int R,
+                                 void* stream) {
+  return pull_launch(ntensors, owners, owner_stride_bytes, pool, rank_stride_bytes, bytes_per_expert,
+                     experts_to_copy, rank, 1, epn, R, stream);
+}
+
+extern "C" int mep_prefetch_pull_ranks(int ntensors, const void* const* owners,
+                                       const int64_t* owner_stride_bytes, void* const* pool,
+                                       const int64_t* rank_stride_bytes, const int64_t* bytes_per_expert,
+                                       const int32_t* experts_to_copy, int rank0, int nranks, int epn, int R,
+                                       void* stream) {
+  return pull_launch(ntensors, owners, owner_stride_bytes, pool, rank_stride_bytes, bytes_per_expert,
+                     experts_to_copy, rank0, nranks, epn, R, stream);
 }
 
 extern "C" int mep_copy_shard(void* dst, const void* src, size_t bytes, void* dst_w, const void* src_w,
@@ -728,17 +812,29 @@ int mep_init_stream_kernels() {
   return MEP_OK;
 }
 
-extern "C" int mep_grad_reduce(float* local_grad, float* reduce_pool, int64_t rank_stride_elems,
-                               const int32_t* experts_to_copy, int rank, int epn, int R,
-                               int64_t elems_per_expert, unsigned flags, void* stream) {
+namespace {
+int reduce_launch(int ntensors, float* const* local_grad, float* const* reduce_pool,
+                  const int64_t* rank_stride_elems, const int64_t* elems_per_expert, const int32_t* experts_to_copy,
+                  int rank0, int nranks, int epn, int R, unsigned flags, void* stream) {
   MEP_REQUIRE(flags <= MEP_REDUCE_CLEAR_ONLY, MEP_ERR_INVALID_ARG);  // the two flags exclude each other
-  MEP_REQUIRE(local_grad && reduce_pool && experts_to_copy, MEP_ERR_INVALID_ARG);
-  MEP_REQUIRE(epn > 0 && R > 0 && rank >= 0 && rank < R && elems_per_expert > 0,
-              MEP_ERR_INVALID_ARG);
-  MEP_REQUIRE(elems_per_expert % 4 == 0, MEP_ERR_UNSUPPORTED);
-  MEP_REQUIRE(rank_stride_elems >= elems_per_expert * epn, MEP_ERR_INVALID_ARG);
-  MEP_REQUIRE(rank_stride_elems % 4 == 0 && (uintptr_t)local_grad % 16 == 0 &&
-                  (uintptr_t)reduce_pool % 16 == 0, MEP_ERR_ALIGNMENT);
+  MEP_REQUIRE(ntensors > 0 && ntensors <= kMaxReduce && local_grad && reduce_pool && rank_stride_elems &&
+                  elems_per_expert && experts_to_copy, MEP_ERR_INVALID_ARG);
+  MEP_REQUIRE(epn > 0 && R > 0 && nranks > 0 && rank0 >= 0 && rank0 + nranks <= R, MEP_ERR_INVALID_ARG);
+  // several ranks at once read each other's slots: only the summing half may run for them
+  MEP_REQUIRE(nranks == 1 || flags == MEP_REDUCE_NO_CLEAR, MEP_ERR_INVALID_ARG);
+  ReduceBatch a{};
+  int64_t tiles = 0;
+  for (int i = 0; i < ntensors; ++i) {
+    MEP_REQUIRE(local_grad[i] && reduce_pool[i] && elems_per_expert[i] > 0, MEP_ERR_INVALID_ARG);
+    MEP_REQUIRE(elems_per_expert[i] % 4 == 0, MEP_ERR_UNSUPPORTED);
+    MEP_REQUIRE(rank_stride_elems[i] >= elems_per_expert[i] * epn, MEP_ERR_INVALID_ARG);
+    MEP_REQUIRE(rank_stride_elems[i] % 4 == 0 && (uintptr_t)local_grad[i] % 16 == 0 &&
+                    (uintptr_t)reduce_pool[i] % 16 == 0, MEP_ERR_ALIGNMENT);
+    a.local_grad[i] = local_grad[i]; a.pool[i] = reduce_pool[i];
+    a.rank_stride[i] = rank_stride_elems[i]; a.elems[i] = elems_per_expert[i];
+    const SpreadTiles rt(elems_per_expert[i] * 4);
+    if (rt.tiles > tiles) tiles = rt.tiles;
+  }
   // slot table + own foreign-held slots + a pool offset per list entry
   const size_t lds = slot_table_bytes(R, epn) + ((size_t)epn + 2) * sizeof(int) +
                      (size_t)R * epn * sizeof(int64_t) + 8;
@@ -747,13 +843,52 @@ extern "C" int mep_grad_reduce(float* local_grad, float* reduce_pool, int64_t ra
     const int irc = mep_ensure_init();
     if (irc != MEP_OK) return irc;
   }
-  ReduceArgs a{local_grad, reduce_pool, rank_stride_elems, elems_per_expert, experts_to_copy,
-               rank, epn, R, flags};
-  const SpreadTiles rt(elems_per_expert * 4);
+  a.etc = experts_to_copy; a.ntensors = ntensors; a.rank0 = rank0; a.epn = epn; a.R = R; a.flags = flags;
   const int cus = mep_device_cu_count();
   // persistent workgroups, two per CU (the kernel halves that when it has slots to fill);
   // three or four per CU lose 3-7 % on a table with many slots
-  const int blocks = stream_blocks(rt.tiles, R, epn, 2 * (cus > 0 ? cus : 256));
-  hipLaunchKernelGGL(grad_reduce_kernel, dim3(blocks), dim3(kBlock), lds, (hipStream_t)stream, a);
+  int64_t cap = 2 * (int64_t)(cus > 0 ? cus : 256) / nranks;
+  if (cap < 1) cap = 1;
+  const int blocks = stream_blocks(tiles, R, epn, cap);
+  hipLaunchKernelGGL(grad_reduce_kernel, dim3(blocks, nranks), dim3(kBlock), lds, (hipStream_t)stream, a);
+  return mep_launch_status();
+}
+}  // namespace
+
+extern "C" int mep_grad_reduce(float* local_grad, float* reduce_pool, int64_t rank_stride_elems,
+                               const int32_t* experts_to_copy, int rank, int epn, int R,
+                               int64_t elems_per_expert, unsigned flags, void* stream) {
+  return reduce_launch(1, &local_grad, &reduce_pool, &rank_stride_elems, &elems_per_expert, experts_to_copy, rank, 1,
+                       epn, R, flags, stream);
+}
+
+extern "C" int mep_grad_reduce_batch(int ntensors, float* const* local_grad, float* const* reduce_pool,
+                                     const int64_t* rank_stride_elems, const int64_t* elems_per_expert,
+                                     const int32_t* experts_to_copy, int rank0, int nranks, int epn, int R,
+                                     unsigned flags, void* stream) {
+  return reduce_launch(ntensors, local_grad, reduce_pool, rank_stride_elems, elems_per_expert, experts_to_copy, rank0,
+                       nranks, epn, R, flags, stream);
+}
+
+extern "C" int mep_cast_bf16(int ntensors, const float* const* src, void* const* dst, const int64_t* elems_per_rank,
+                             const int64_t* dst_rank_stride, int nranks, void* stream) {
+  MEP_REQUIRE(ntensors > 0 && ntensors <= kMaxTensors && src && dst && elems_per_rank && dst_rank_stride && nranks > 0,
+              MEP_ERR_INVALID_ARG);
+  CastArgs a{};
+  int64_t most = 0;
+  for (int i = 0; i < ntensors; ++i) {
+    MEP_REQUIRE(src[i] && dst[i] && elems_per_rank[i] > 0 && dst_rank_stride[i] >= elems_per_rank[i], MEP_ERR_INVALID_ARG);
+    MEP_REQUIRE(elems_per_rank[i] % 8 == 0 && dst_rank_stride[i] % 8 == 0 && nranks <= 65535, MEP_ERR_UNSUPPORTED);
+    MEP_REQUIRE((uintptr_t)src[i] % 16 == 0 && (uintptr_t)dst[i] % 16 == 0, MEP_ERR_ALIGNMENT);
+    a.src[i] = src[i]; a.dst[i] = (uint16_t*)dst[i];
+    a.elems[i] = elems_per_rank[i]; a.dst_stride[i] = dst_rank_stride[i];
+    if (elems_per_rank[i] > most) most = elems_per_rank[i];
+  }
+  const int cus = mep_device_cu_count();
+  int64_t blocks = 8 * (int64_t)(cus > 0 ? cus : 256) / (ntensors * nranks);
+  const int64_t want = (most / 8 + kBlock - 1) / kBlock;
+  if (blocks > want) blocks = want;
+  if (blocks < 1) blocks = 1;
+  hipLaunchKernelGGL(cast_kernel, dim3((unsigned)blocks, nranks, ntensors), dim3(kBlock), 0, (hipStream_t)stream, a);
   return mep_launch_status();
 }

@@ -15,18 +15,21 @@ reference gets from its cross-rank barriers.
 
 ``group_expert_ffn_hip`` is the expert stage of the layer on the matrix cores,
 forward and backward: the compute views of every rank (its local experts, then
-its prefetch slots filled by one ``launch_prefetch_pull``), the grouped SwiGLU FFN
-of every rank, and in backward the grouped input / weight gradient GEMMs followed
-by ``reduce_grad`` in fp32 -- no PyTorch GEMM on either pass.
+its prefetch slots pulled from their owners), the grouped SwiGLU FFN of every rank's
+groups, and in backward the grouped input / weight gradient GEMMs followed by
+``reduce_grad`` in fp32 -- no PyTorch GEMM on either pass.
 """
 
 from __future__ import annotations
 
+import ctypes as C
+
 import torch
 
-from . import ffn
+from . import _lib, ffn
 from .api import Buffer, EmulatedWorld
 from .grad_reduce import launch_grad_reduce
+from .planning import MoonEPCommPlan, launch_planning_all_ranks
 from .prefetch import launch_prefetch_pull
 
 
@@ -54,44 +57,109 @@ class EmulatedGroup:
             b.destroy()
 
 
+# Every operator below is one launch for the whole group (csrc: the *_ranks entry points).  The rows
+# go straight into the tensor that the experts (or autograd) own and come straight out of it: on one
+# GPU that tensor can be the destination of a dispatch and the source of a combine itself, so
+# neither the shards of the world nor a copy into or out of them is needed.
+
+def _group_ctx(group):
+    return group.buffers[0]._require_ctx()
+
+
+def _dispatch_all(group, x_all, w_all, dst_all, zero_fill, cu):
+    """Rows ``[R,NvS,H]`` (+ slots ``[R,NvS]``) of every rank; every row is written."""
+    ctx, R = _group_ctx(group), group.R
+    # without the groups' ends (plans of another origin) the rows behind them are cleared first
+    make = torch.empty if cu is not None else torch.zeros
+    rows = make(R, group.NvS, group.H, dtype=torch.bfloat16, device=x_all.device)
+    slots = None if w_all is None else make(R, group.NvS, dtype=torch.float32, device=x_all.device)
+    rc = _lib.lib().mep_dispatch_ranks(
+        x_all.data_ptr(), _lib.ptr(w_all), dst_all.data_ptr(), zero_fill.data_ptr(), _lib.ptr(cu), rows.data_ptr(),
+        group.NvS, _lib.ptr(slots), group.NvS, 0, R, group.S, group.H, group.K, R, group.epn, group.NvS,
+        int(ctx["token_padding"]), _lib.DISPATCH_WRITE_DUPS, _lib.current_stream())
+    _lib.check(rc, "mep_dispatch_ranks")
+    return rows, slots
+
+
+def _combine_all(group, rows, slots, dst_all):
+    """Token-major sums ``[R,S,H]`` (+ slots gathered back to ``[R,S,K]``) of every rank."""
+    _group_ctx(group)
+    R, S, K = group.R, group.S, group.K
+    out = torch.empty(R, S, group.H, dtype=torch.bfloat16, device=rows.device)
+    w = None if slots is None else torch.empty(R, S, K, dtype=torch.float32, device=rows.device)
+    rc = _lib.lib().mep_combine_ranks(
+        rows.data_ptr(), group.NvS, _lib.ptr(slots), group.NvS, dst_all.data_ptr(), out.data_ptr(), _lib.ptr(w), R,
+        S, group.H, K, R, group.NvS, _lib.COMBINE_TWO_LEVEL, _lib.current_stream())
+    _lib.check(rc, "mep_combine_ranks")
+    return out, w
+
+
+def _group_plans(group, topk_all, tpe):
+    """Plans of every rank from one planner launch and one duplicate-group build: tensors with a
+    leading rank dimension and the per-rank plans as views of them."""
+    ctx, R, NvS, epn = _group_ctx(group), group.R, group.NvS, group.epn
+    dst, cu, etc, zfr, stats = launch_planning_all_ranks(ctx, topk_all, tpe)
+    i32 = dict(dtype=torch.int32, device=dst.device)
+    groups, loffs, counts = torch.empty(R, NvS, 3, **i32), torch.empty(R, NvS, **i32), torch.empty(R, 2, **i32)
+    n = R * _lib.lib().mep_dedup_scratch_bytes(group.S, R)
+    work = torch.empty(n, dtype=torch.uint8, device=dst.device)
+    rc = _lib.lib().mep_build_dedup_ranks(dst.data_ptr(), 0, R, group.S, group.K, R, NvS, groups.data_ptr(),
+                                          loffs.data_ptr(), counts.data_ptr(), work.data_ptr(), n, _lib.current_stream())
+    _lib.check(rc, "mep_build_dedup_ranks")
+    plans = [MoonEPCommPlan(dst=dst[r], experts_to_copy=etc, zero_fill_ranges=zfr[r], remote_stats=stats[r],
+                            dup_groups=groups[r], dup_loffs=loffs[r], dup_counts=counts[r], N=group.S * group.K,
+                            R=R, E=group.E, NvS=NvS, K=group.K) for r in range(R)]
+    return plans, _PlanTensors(dst, zfr, cu)
+
+
+class _PlanTensors:
+    """A group's plans with a leading rank dimension: dst [R,N], zero_fill [R,2*epn,2], cu [R,2*epn]."""
+
+    def __init__(self, dst, zero_fill, cu):
+        self.dst, self.zero_fill, self.cu = dst, zero_fill, cu
+
+
+def _plan_tensors(group, plans):
+    """The stacked tensors of ``plans``: those they are views of, where a group's own dispatch made
+    them, else stacked here (the groups' ends are then not known)."""
+    own = getattr(group, "_last_tensors", None)
+    if own is not None and len(plans) == group.R and all(
+            p.dst.data_ptr() == own.dst[r].data_ptr() for r, p in enumerate(plans)):
+        return own
+    return _PlanTensors(torch.stack([p.dst for p in plans]), torch.stack([p.zero_fill_ranges for p in plans]), None)
+
+
+def _check_group_tokens(group, x_all, w_all):
+    R, S, H, K = group.R, group.S, group.H, group.K
+    assert x_all.dtype == torch.bfloat16 and x_all.is_cuda and tuple(x_all.shape) == (R, S, H), (
+        f"tokens must be bf16 [R={R}, S={S}, H={H}] on the GPU, got {tuple(x_all.shape)} {x_all.dtype}")
+    if w_all is not None:
+        assert w_all.dtype == torch.float32 and tuple(w_all.shape) == (R, S, K) and w_all.device == x_all.device, (
+            f"route weights must be fp32 [R={R}, S={S}, K={K}], got {tuple(w_all.shape)} {w_all.dtype}")
+
+
 class _GroupDispatch(torch.autograd.Function):
     """tokens [R,S,H] (+ weights [R,S,K]) -> rows [R,NvS,H] (+ slots [R,NvS])."""
 
     @staticmethod
     def forward(ctx, group, x_all, w_all, topk_all, tpe):
-        R = group.R
-        group.world.hidden_buf.zero_()
-        group.world.meta_buf.zero_()
-        plans, cus = [], []
-        for r in range(R):
-            _, _, cu, plan = group.buffers[r].dispatch(
-                x_all[r].contiguous(), None if w_all is None else w_all[r].contiguous(),
-                topk_all, tpe, zero_copy=True, router_weights_zero_copy=True)
-            plans.append(plan)
-            cus.append(cu)
-        ctx.group, ctx.plans, ctx.has_w = group, plans, w_all is not None
-        group.last_plans, group.last_cu_seqlens = plans, torch.stack(cus)
-        hidden = group.shards().clone()
-        slots = group.weight_slots().clone() if w_all is not None else None
-        ctx.mark_non_differentiable(group.last_cu_seqlens)
-        return hidden, slots, group.last_cu_seqlens
+        _check_group_tokens(group, x_all, w_all)
+        plans, t = _group_plans(group, topk_all, tpe)
+        rows, slots = _dispatch_all(group, x_all.contiguous(), None if w_all is None else w_all.contiguous(),
+                                    t.dst, t.zero_fill, t.cu)
+        ctx.group, ctx.t, ctx.has_w = group, t, w_all is not None
+        group.last_plans, group.last_cu_seqlens, group._last_tensors = plans, t.cu, t
+        ctx.mark_non_differentiable(t.cu)
+        return rows, slots, t.cu
 
     @staticmethod
-    def backward(ctx, g_hidden, g_slots, _g_cu):
-        group = ctx.group
-        group.shards().copy_(g_hidden.to(torch.bfloat16))
+    def backward(ctx, g_rows, g_slots, _g_cu):
+        slots = None
         if ctx.has_w:
-            group.weight_slots().copy_(g_slots if g_slots is not None else 0.0)
-        gx, gw = [], []
-        for r in range(group.R):
-            b = group.buffers[r]
-            out, w_back, _ = b.combine(
-                plan=ctx.plans[r], hidden_nvsh=b.hidden_nvsh_buffer_view,
-                route_weights_nvs=b.router_weight_buffer_view if ctx.has_w else None,
-                zero_copy=True, router_weights_zero_copy=True)
-            gx.append(out)
-            gw.append(w_back)
-        return (None, torch.stack(gx), torch.stack(gw) if ctx.has_w else None, None, None)
+            slots = (torch.zeros(g_rows.shape[:2], dtype=torch.float32, device=g_rows.device) if g_slots is None
+                     else g_slots.float().contiguous())
+        gx, gw = _combine_all(ctx.group, g_rows.to(torch.bfloat16).contiguous(), slots, ctx.t.dst)
+        return None, gx, gw, None, None
 
 
 class _GroupCombine(torch.autograd.Function):
@@ -99,23 +167,14 @@ class _GroupCombine(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, group, plans, y_all):
-        group.shards().copy_(y_all.to(torch.bfloat16))
-        outs = []
-        for r in range(group.R):
-            b = group.buffers[r]
-            out, _, _ = b.combine(plan=plans[r], hidden_nvsh=b.hidden_nvsh_buffer_view, zero_copy=True)
-            outs.append(out)
-        ctx.group, ctx.plans = group, plans
-        return torch.stack(outs)
+        ctx.group, ctx.t = group, _plan_tensors(group, plans)
+        assert tuple(y_all.shape) == (group.R, group.NvS, group.H)
+        return _combine_all(group, y_all.to(torch.bfloat16).contiguous(), None, ctx.t.dst)[0]
 
     @staticmethod
     def backward(ctx, g_out):
-        group = ctx.group
-        group.world.hidden_buf.zero_()
-        for r in range(group.R):
-            group.buffers[r].dispatch(g_out[r].to(torch.bfloat16).contiguous(), plan=ctx.plans[r],
-                                      zero_copy=True)
-        return None, None, group.shards().clone()
+        t, g = ctx.t, g_out.to(torch.bfloat16).contiguous()
+        return None, None, _dispatch_all(ctx.group, g, None, t.dst, t.zero_fill, t.cu)[0]
 
 
 class _GroupPrefetch(torch.autograd.Function):
@@ -152,55 +211,90 @@ class _GroupExpertFFN(torch.autograd.Function):
 
     fp32 master weights in the orientation the kernels read: gate / up
     [R, epn, H', H], down [R, epn, H, H'].  Forward: bf16 compute views (local
-    experts, then the prefetch slots filled by ``launch_prefetch_pull``), then per rank
-    the fused gate/up GEMM and the down GEMM with the route weight applied.
-    Backward: the grouped gradient GEMMs per rank, then ``launch_grad_reduce``
-    sums every slot's fp32 weight gradient into its owner's."""
+    experts, then the prefetch slots), then the fused gate/up GEMM and the down
+    GEMM with the route weight applied, each one launch over the groups of all
+    ranks (a rank's own have too few tiles to fill the GPU).  Backward: the
+    grouped gradient GEMMs, then every slot's fp32 weight gradient is summed
+    into its owner's."""
 
     @staticmethod
     def forward(ctx, group, experts_to_copy, cu_all, rows_all, slots_all, gate_m, up_m, down_m):
-        R, tp = group.R, group.world.token_padding
-        local = [m.detach().to(torch.bfloat16).contiguous() for m in (gate_m, up_m, down_m)]
-        pools = [torch.zeros_like(t) for t in local]
-        for r in range(R):     # a rank's slots filled from all owners in one launch
-            launch_prefetch_pull(tuple(local), tuple(pools), experts_to_copy, rank=r)
-        views = [torch.cat([l, p], dim=1) for l, p in zip(local, pools)]      # [R, 2*epn, ...]
-        outs, saved = [], []
-        for r in range(R):
-            y, keep = ffn.grouped_ffn_hip_forward(rows_all[r], None if slots_all is None else slots_all[r],
-                                                  cu_all[r], views[0][r], views[1][r], views[2][r],
-                                                  token_padding=tp)
-            outs.append(y)
-            saved.append(keep)
-        ctx.group, ctx.etc, ctx.cu_all, ctx.views, ctx.saved = group, experts_to_copy, cu_all, views, saved
-        ctx.rows_all, ctx.slots_all = rows_all, slots_all
-        return torch.stack(outs)
+        tp = group.world.token_padding
+        views = _fill_views(group, experts_to_copy, (gate_m, up_m, down_m))              # [R, 2*epn, ...]
+        args = (rows_all.contiguous(), None if slots_all is None else slots_all.contiguous(), cu_all.contiguous(), *views)
+        res = _lib.host().ffn_forward(*args, tp, True)
+        ctx.native = res is not None
+        if not ctx.native:     # sizes that only the single products take: rank by rank
+            each = [ffn.grouped_ffn_hip_forward(*_of_rank(args, r), token_padding=tp) for r in range(group.R)]
+            res = torch.stack([y for y, _ in each]), [keep for _, keep in each]
+        ctx.group, ctx.etc, ctx.args, ctx.saved = group, experts_to_copy, args, res[1]
+        return res[0]
 
     @staticmethod
     def backward(ctx, g_out):
-        group = ctx.group
+        group, args = ctx.group, ctx.args
         R, epn, tp = group.R, group.epn, group.world.token_padding
         g_out = g_out.to(torch.bfloat16).contiguous()
-        drows, dslots, dw = [], [], ([], [], [])
-        for r in range(R):
-            res = ffn.grouped_ffn_hip_backward(
-                g_out[r], ctx.rows_all[r], None if ctx.slots_all is None else ctx.slots_all[r],
-                ctx.cu_all[r], ctx.views[0][r], ctx.views[1][r], ctx.views[2][r], ctx.saved[r],
-                token_padding=tp, skip_unused_slots=True)   # grad reduce reads occupied slots only
-            drows.append(res[0])
-            dslots.append(res[1])
-            for acc, g in zip(dw, res[2:]):
-                acc.append(g)                                                   # [2*epn, ...] fp32
-        grads = []
-        for per_rank in dw:
-            full = torch.stack(per_rank)                                        # [R, 2*epn, ...]
-            own = full[:, :epn].contiguous()
-            slots = full[:, epn:].contiguous()
-            for r in range(R):     # every rank reads before any rank would clear: summing half only
-                launch_grad_reduce(own[r], slots, ctx.etc, rank=r, phase="reduce")
-            grads.append(own)
-        return (None, None, None, torch.stack(drows),
-                None if ctx.slots_all is None else torch.stack(dslots), *grads)
+        # every rank's weight gradients in fp32: its local experts' and its slots' (the latter are
+        # read for occupied slots only, so those of unused ones are left unwritten)
+        own, slots = (tuple(torch.empty(R, epn, *v.shape[2:], dtype=torch.float32, device=v.device) for v in args[3:])
+                      for _ in range(2))
+        res = _lib.host().ffn_backward(*args, tp, g_out, *ctx.saved, True, own, slots) if ctx.native else None
+        if res is not None:
+            drows, dslots = res[:2]
+        else:
+            drows, dslots = [], []
+            for r in range(R):
+                keep = [t[r] for t in ctx.saved] if ctx.native else ctx.saved[r]
+                g = ffn.grouped_ffn_hip_backward(g_out[r], *_of_rank(args, r), keep, token_padding=tp,
+                                                 skip_unused_slots=True)
+                drows.append(g[0])
+                dslots.append(g[1])
+                for o, s, full in zip(own, slots, g[2:]):
+                    o[r].copy_(full[:epn])
+                    s[r].copy_(full[epn:])
+            drows = torch.stack(drows)
+            dslots = None if args[1] is None else torch.stack(dslots)
+        # every rank reads before any rank would clear: summing half only
+        arr_p, arr_i = C.c_void_p * 3, C.c_int64 * 3
+        elems = [int(v.shape[2]) * int(v.shape[3]) for v in args[3:]]
+        rc = _lib.lib().mep_grad_reduce_batch(
+            3, arr_p(*[t.data_ptr() for t in own]), arr_p(*[t.data_ptr() for t in slots]),
+            arr_i(*[epn * n for n in elems]), arr_i(*elems), ctx.etc.data_ptr(), 0, R, epn, R, _lib.REDUCE_NO_CLEAR,
+            _lib.current_stream())
+        _lib.check(rc, "mep_grad_reduce_batch")
+        return (None, None, None, drows, dslots, *own)
+
+
+def _of_rank(args, r):
+    return [None if t is None else t[r] for t in args]
+
+
+def _fill_views(group, experts_to_copy, masters):
+    """bf16 compute views ``[R, 2*epn, ...]`` of the three projections: every rank's local experts
+    rounded from the masters, its occupied slots copied from their owners (one launch each).  Slots
+    that hold no expert are left as they are: no row goes there."""
+    R, epn = group.R, group.epn
+    assert experts_to_copy.dtype == torch.int32 and experts_to_copy.is_contiguous() and \
+        tuple(experts_to_copy.shape) == (R, epn), f"experts_to_copy must be int32 [R={R}, epn={epn}]"
+    for m in masters:
+        assert m.dim() == 4 and tuple(m.shape[:2]) == (R, epn), f"masters must be [R={R}, epn={epn}, ., .]"
+    views = [torch.empty(R, 2 * epn, *m.shape[2:], dtype=torch.bfloat16, device=m.device) for m in masters]
+    per = [int(m.shape[2]) * int(m.shape[3]) for m in masters]
+    assert all(n % 8 == 0 for n in per)
+    arr_p, arr_i = C.c_void_p * 3, C.c_int64 * 3
+    lib, st = _lib.lib(), _lib.current_stream()
+    dense = [m.detach().float().contiguous() for m in masters]
+    rc = lib.mep_cast_bf16(3, arr_p(*[m.data_ptr() for m in dense]), arr_p(*[v.data_ptr() for v in views]),
+                           arr_i(*[epn * n for n in per]), arr_i(*[2 * epn * n for n in per]), R, st)
+    _lib.check(rc, "mep_cast_bf16")
+    rank_bytes = arr_i(*[4 * epn * n for n in per])
+    rc = lib.mep_prefetch_pull_ranks(
+        3, arr_p(*[v.data_ptr() for v in views]), rank_bytes,
+        arr_p(*[v.data_ptr() + 2 * epn * n for v, n in zip(views, per)]), rank_bytes, arr_i(*[2 * n for n in per]),
+        experts_to_copy.data_ptr(), 0, R, epn, R, st)
+    _lib.check(rc, "mep_prefetch_pull_ranks")
+    return views
 
 
 def group_expert_ffn_hip(group, experts_to_copy, cu_all, rows_all, slots_all, gate_m, up_m, down_m):

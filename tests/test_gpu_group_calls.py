@@ -1,0 +1,100 @@
+"""The whole-group launches (mep_*_ranks, mep_grad_reduce_batch, mep_cast_bf16 behind
+moonep_amd.moe) against the per-rank operators on the same inputs: the same bits.  Sizes: rows
+that are no whole wave tiles, paddings with and without rows behind the last group, one expert per
+rank, projections of different sizes."""
+
+import pytest
+import torch
+
+from moonep_amd import Buffer, EmulatedWorld, moe, routing
+from moonep_amd.grad_reduce import launch_grad_reduce
+from moonep_amd.prefetch import launch_prefetch_pull
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("R,epn,S,K,H,tp,sigma", [
+    (2, 1, 1, 1, 8, 1, 0.0),            # the smallest: no padding, one entry per rank
+    (4, 3, 37, 3, 136, 16, 1.0),        # H no multiple of 512
+    (8, 4, 64, 8, 512, 128, 2.0),       # skewed: slots in use, long tails behind the last group
+])
+def test_dispatch_and_combine_of_a_group(cuda, R, epn, S, K, H, tp, sigma):
+    E = R * epn
+    print(f"group R={R} epn={epn} S={S} K={K} H={H}", flush=True)
+    topk = torch.stack([routing.popularity_biased(S, K, E, R, r, sigma, seed=3) for r in range(R)])
+    tpe = routing.tokens_per_expert(topk, E).to(cuda)
+    topk = topk.to(cuda)
+    g = torch.Generator().manual_seed(R + S)
+    x = torch.randn(R, S, H, generator=g).to(torch.bfloat16).to(cuda)
+    w = torch.rand(R, S, K, generator=g).to(cuda)
+    group = moe.EmulatedGroup(S, H, K, E, R, token_padding=tp)
+    rows, slots, cu, plans = moe.group_dispatch(group, x, w, topk, tpe)
+
+    world = EmulatedWorld(S, H, K, E, R, tp)
+    world.hidden_buf.zero_()
+    world.meta_buf.zero_()
+    bufs = [Buffer(S, H, K, E, R, token_padding=tp, rank=r, world=world) for r in range(R)]
+    mine = [bufs[r].dispatch(x[r], w[r], topk, tpe, zero_copy=True, router_weights_zero_copy=True) for r in range(R)]
+    for r in range(R):
+        p, q = plans[r], mine[r][3]
+        assert torch.equal(rows[r], bufs[r].hidden_nvsh_buffer_view)
+        assert torch.equal(slots[r], bufs[r].router_weight_buffer_view)
+        assert torch.equal(cu[r], mine[r][2])
+        n, d = (int(v) for v in q.dup_counts)
+        assert torch.equal(p.dup_counts, q.dup_counts)
+        assert torch.equal(p.dup_groups[:n], q.dup_groups[:n]) and torch.equal(p.dup_loffs[:d], q.dup_loffs[:d])
+        for a, b in ((p.dst, q.dst), (p.experts_to_copy, q.experts_to_copy), (p.remote_stats, q.remote_stats),
+                     (p.zero_fill_ranges, q.zero_fill_ranges)):
+            assert torch.equal(a, b)
+    out = moe.group_combine(group, plans, rows)
+    stacked = moe.group_combine(group, [m[3] for m in mine], rows)     # plans of another origin
+    for r in range(R):
+        want = bufs[r].combine(mine[r][3], bufs[r].hidden_nvsh_buffer_view, zero_copy=True)[0]
+        assert torch.equal(out[r], want) and torch.equal(stacked[r], want)
+    for b in (group, *bufs):
+        b.destroy()
+
+
+@pytest.mark.parametrize("R,epn,shapes", [(2, 2, ((128, 128), (128, 256), (256, 128))), (4, 5, ((256, 256),) * 3)])
+def test_views_and_gradient_sums_of_a_group(cuda, R, epn, shapes):
+    g = torch.Generator().manual_seed(R * epn)
+    etc = torch.full((R, epn), -1, dtype=torch.int32)
+    for d in range(R):
+        for b in range(epn - 1):
+            etc[d, b] = int(torch.randint(0, R * epn, (1,), generator=g))
+    etc = etc.to(cuda)
+
+    class Group:
+        pass
+
+    group = Group()
+    group.R, group.epn = R, epn
+    master = [torch.randn(R, epn, *s, generator=g).to(cuda) for s in shapes]
+    views = moe._fill_views(group, etc, master)
+    for m, v in zip(master, views):
+        local = m.to(torch.bfloat16)
+        pool = torch.zeros_like(local)
+        for r in range(R):
+            launch_prefetch_pull((local,) * 3, (pool,) * 3, etc, rank=r)
+        assert torch.equal(v[:, :epn], local)
+        for d, b in (etc >= 0).nonzero().tolist():
+            assert torch.equal(v[d, epn + b], pool[d, b])
+    # sums: one launch for all projections and ranks against one per projection and rank
+    import ctypes as C
+
+    from moonep_amd import _lib
+    own = [torch.randn(R, epn, *s, generator=g).to(cuda) for s in shapes]
+    pool = [torch.randn(R, epn, *s, generator=g).to(cuda) for s in shapes]
+    want = [t.clone() for t in own]
+    for o, p in zip(want, pool):
+        for r in range(R):
+            launch_grad_reduce(o[r], p, etc, rank=r, phase="reduce")
+    arr_p, arr_i = C.c_void_p * 3, C.c_int64 * 3
+    n = [a * b for a, b in shapes]
+    rc = _lib.lib().mep_grad_reduce_batch(3, arr_p(*[t.data_ptr() for t in own]), arr_p(*[t.data_ptr() for t in pool]),
+                                          arr_i(*[epn * k for k in n]), arr_i(*n), etc.data_ptr(), 0, R, epn, R,
+                                          _lib.REDUCE_NO_CLEAR, _lib.current_stream())
+    assert rc == 0
+    torch.cuda.synchronize()
+    for a, b in zip(own, want):
+        assert torch.equal(a, b)
