@@ -8,6 +8,7 @@ namespace {
 
 constexpr int kWavesPerBlock = 4;
 constexpr int kBlock = kWavesPerBlock * MEP_WAVE;
+constexpr int64_t kFewPieces = 6144;
 
 struct CombineArgs {
   const uint16_t* shards;
@@ -50,7 +51,6 @@ __global__ __launch_bounds__(kBlock) void combine_kernel(CombineArgs a) {
   const bool valid = lane < K && drank < a.R;
   float wk = 0.0f;  // route weight of entry `lane`, read from its slot
   if (a.wslots && valid) wk = a.wslots[(size_t)drank * a.wslot_stride + loff];
-  if (a.out_sk && part == 0 && lane < K) a.out_sk[sy * K + lane] = wk;
   const uint64_t off = ((uint64_t)drank * (uint64_t)a.shard_stride_rows + (uint64_t)loff) * row_bytes;
   const uint32_t off_lo = (uint32_t)off, off_hi = (uint32_t)(off >> 32);
   const bool primary = valid && dv >= 0;
@@ -168,6 +168,87 @@ __global__ __launch_bounds__(kBlock) void combine_kernel(CombineArgs a) {
       else mep_st16_through(orow + (size_t)i * 1024, o);
     }
   }
+  // last: the rows need not wait for the loads of the weights
+  if (a.out_sk && part == 0 && lane < K) a.out_sk[sy * K + lane] = wk;
+}
+
+// Two-level mode for few tokens (K <= KM): what bounds it is the chain of memory latencies of one
+// wave -- the kernel above asks for a row when the one before has been added, and nothing else runs
+// on the CU to fill the wait.  Here a wave takes one 1-KiB piece of a token, asks for all K rows
+// at once and then sums them from registers in the same order; the route weights are stored last,
+// so that no row waits for their loads.
+template <int KM>
+__global__ __launch_bounds__(MEP_WAVE) void combine_few_kernel(CombineArgs a) {
+  const int lane = threadIdx.x;
+  const int s = blockIdx.x / a.parts;
+  const int part = blockIdx.x - s * a.parts;
+  const int K = a.K;
+  const size_t row_bytes = (size_t)a.H * 2;
+  const size_t sy = (size_t)blockIdx.y * a.S + s;
+  const int dv = lane < K ? a.dst[sy * K + lane] : 0;
+  const int raw = dv < 0 ? -dv - 1 : dv;
+  const int drank = raw / a.NvS;
+  const int loff = raw - drank * a.NvS;
+  const bool valid = lane < K && drank < a.R;
+  // an entry that is skipped reads the first row of the shards, for nobody
+  const uint64_t off = valid ? ((uint64_t)drank * (uint64_t)a.shard_stride_rows + (uint64_t)loff) * row_bytes : 0;
+  const uint32_t off_lo = (uint32_t)off, off_hi = (uint32_t)(off >> 32);
+  const bool primary = valid && dv >= 0;
+  const uint32_t prim_mask = (uint32_t)__ballot(primary);
+  const int c = part * 64 + lane;  // this lane's 16-byte vector of the row
+  const bool inside = c < a.H / 8;
+  const char* base = (const char*)a.shards + (inside ? (size_t)c * 16 : 0);
+  mep_u4 v[KM];
+#pragma unroll
+  for (int k = 0; k < KM; ++k) {
+    const int kk = k < K ? k : K - 1;
+    const uint64_t o = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(off_hi, kk) << 32) |
+                       (uint32_t)__builtin_amdgcn_readlane(off_lo, kk);
+    v[k] = mep_ld16_stream(base + o);
+  }
+  float wk = 0.0f;
+  if (a.wslots && part == 0 && valid) wk = a.wslots[(size_t)drank * a.wslot_stride + loff];
+  // members of the group that entry k leads, as in the kernel above
+  uint32_t members[KM];
+#pragma unroll
+  for (int k = 0; k < KM; ++k) {
+    const int dk = __builtin_amdgcn_readlane(drank, k);
+    members[k] = (uint32_t)__ballot(valid && !primary && drank == dk && lane > k);
+  }
+  float acc[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) acc[j] = 0.0f;
+#pragma unroll
+  for (int k = 0; k < KM; ++k) {
+    if (!(prim_mask >> k & 1)) continue;
+    if (members[k] == 0) {
+      acc8(acc, v[k]);
+      continue;
+    }
+    float grp[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) grp[j] = 0.0f;
+    acc8(grp, v[k]);
+#pragma unroll
+    for (int m = k + 1; m < KM; ++m)
+      if (members[k] >> m & 1) acc8(grp, v[m]);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[j] += mep_round_bf16(grp[j]);
+  }
+  if (inside) {
+    mep_u4 o;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] = mep_pack_bf16(acc[2 * j], acc[2 * j + 1]);
+    mep_st16_stream((char*)a.out + sy * row_bytes + (size_t)c * 16, o);
+  }
+  if (a.out_sk && part == 0 && lane < K) a.out_sk[sy * K + lane] = wk;
+}
+
+template <int KM>
+void launch_combine_few(const CombineArgs& a0, int nranks, hipStream_t st) {
+  CombineArgs a = a0;
+  a.parts = (a.H / 8 + 63) / 64;
+  hipLaunchKernelGGL((combine_few_kernel<KM>), dim3((unsigned)((int64_t)a.S * a.parts), nranks), dim3(MEP_WAVE), 0, st, a);
 }
 
 template <int CH, bool EXACT, bool TWO>
@@ -202,6 +283,15 @@ int combine_launch(const void* shards, int64_t shard_stride_rows, const float* w
   hipStream_t st = (hipStream_t)stream;
   const int nvec = H / 8;
   if (mode == MEP_COMBINE_TWO_LEVEL) {
+    // Few tokens: up to six waves of one 1-KiB piece per SIMD (of 1024) all rows at once beat rows
+    // in turn -- 64 pieces (8 tokens, H = 4096, K = 8) 3.4 against 5.2 us, 4096 6.9 against 9.5,
+    // 6144 (K = 6) 9.1 against 10.2; 8192 13.7 against 13.6, 12288 (K = 6) 15.7 against 14.9.
+    const int64_t pieces = (int64_t)nranks * S * ((nvec + 63) / 64);
+    if (K <= 8 && pieces <= kFewPieces) {
+      if (K <= 4) launch_combine_few<4>(a, nranks, st);
+      else launch_combine_few<8>(a, nranks, st);
+      return mep_launch_status();
+    }
     // two accumulator sets: narrow tiles keep the register count low and more
     // waves resident (88.6 us with 2-chunk tiles vs 90.0 with 7 at H = 7168)
     if (nvec % (2 * 64) == 0) launch_combine<2, true, true>(a, nranks, st);
