@@ -3,28 +3,34 @@
 // padded end offsets in cu_seqlens (device memory, as the planner wrote them);
 // group g multiplies by its own weight matrix B[g] stored [N,K] (K
 // contiguous), so C = A * B[g]^T needs no transposition on either operand.
+// With token_padding a multiple of 128 a block of 128 rows never straddles two
+// groups.
 //
-// Workgroup: 640 threads on a 128 x 256 tile of (rows x weight rows), K in
-// steps of 64: two producer waves stream the tile slices from global memory
-// straight into a ring of three LDS stages, eight consumer waves own 64 x 64
-// of the tile each as 2 x 2 MFMA 32x32x16 accumulators.  With token_padding a
-// multiple of 128 a row tile never straddles two groups.  The kernel is bound
-// by the L2 (its channels are ~75 % busy at 0.8 PFLOP/s), i.e. by tile bytes
-// per flop.
-// Four kinds of launch share the main loop:
+// Four kinds of product:
 //   scale  : C[m,n] = bf16(row_scale[m] * acc)               (down projection)
-//   swiglu : C[m,n] = bf16(silu(A*Bg^T) * (A*Bu^T))           (gate/up fused;
-//            the tile holds 128 gate rows and the same 128 up rows; the two
-//            pre-activations can be stored beside it for the backward pass)
+//   swiglu : C[m,n] = bf16(silu(A*Bg^T) * (A*Bu^T))           (gate/up fused)
 //   dual   : C = bf16(A*B[g]^T + A2*B2[g]^T): the K loop runs over both pairs
 //            (input gradient of the gate/up pair)
 //   wgrad  : C[g] = At[:, rows of g] * Bt[:, rows of g]^T in fp32: the K range
-//            of a tile is the row range of its group (weight gradients from
-//            transposed activations)
-// Tiles are handed out so that the workgroups running at one time on an XCD
-// (one L2) work on the same 8 row tiles and neighbouring weight tiles.
+//            of a tile is the row range of its group (weight gradients)
+// Three kernels:
+//   gemm_pp_kernel         256 x 256 tiles, long groups, every kind
+//   gemm_stream_kernel     128 rows x up to 288 weight rows, forward products of
+//                          groups of about one block: bound by the weights' bytes
+//   grouped_gemm_nt_kernel 128 x 256 tiles: backward products of such groups, and
+//                          weight gradients that are no multiples of 256
+//
+// grouped_gemm_nt_kernel: workgroups of 640 threads on a 128 x 256 tile of (rows
+// x weight rows), K in steps of 64: two producer waves stream the tile slices
+// from global memory straight into a ring of three LDS stages, eight consumer
+// waves own 64 x 64 of the tile each as 2 x 2 MFMA 32x32x16 accumulators.  It is
+// bound by the L2 (its channels are ~75 % busy at 0.8 PFLOP/s), i.e. by tile
+// bytes per flop.  Tiles are handed out so that the workgroups running at one
+// time on an XCD (one L2) work on the same 8 row tiles and neighbouring weight
+// tiles.
 #include "mep_common.h"
 
+#include <algorithm>
 #include <atomic>
 
 namespace {
@@ -127,7 +133,7 @@ __device__ __forceinline__ int group_beg(const GemmArgs& a, int gi) {
 // banks once.
 template <int MODE, bool BKN = false>
 __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_nt_kernel(GemmArgs a) {
-  constexpr bool SWIGLU = MODE == kModeSwiglu;
+  static_assert(MODE == kModeDual || (MODE == kModeScale ? BKN : MODE == kModeWgrad), "the products that need it");
   static_assert(!BKN || MODE == kModeScale || MODE == kModeDual, "[K, N] weights: plain and dual products only");
   static_assert(kProducers == 2, "the lane offsets of the pieces assume that a producer wave's pieces share a parity");
   extern __shared__ __attribute__((aligned(1024))) char gsm[];
@@ -207,8 +213,7 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_nt_kernel(GemmAr
     mt = beg_tiles + panel * kPanel + (within - nt * ph);
   }
   const int m0 = mt * kBM;
-  constexpr int kCols = SWIGLU ? kBN / 2 : kBN;  // output columns per tile
-  const int n0 = nt * kCols;
+  const int n0 = nt * kBN;
   const int g = tg;
 
   // K steps of this tile and where its K range starts in a row
@@ -240,7 +245,7 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_nt_kernel(GemmAr
     const int lk = lane >> 5, lv = lane & 31;
     const size_t lane_off_kn = (size_t)lk * a.N + (size_t)((lv ^ ((2 * (p & 1) + lk) << 1)) * 8) + n0;
     const uint16_t* Bp0 = BKN ? a.B + goff + lane_off_kn : a.B + goff + (size_t)n0 * K + lane_off;
-    const uint16_t* Bp1 = SWIGLU ? a.B2 + goff + (size_t)n0 * K + lane_off : Bp0 + (size_t)(kBN / 2) * K;
+    const uint16_t* Bp1 = Bp0 + (size_t)(kBN / 2) * K;
     // dual: the second half of the K loop reads the second pair
     const uint16_t* Aq = MODE == kModeDual ? a.A2 + (size_t)m0 * K + lane_off : Ap;
     const uint16_t* Bq0 = MODE != kModeDual ? Bp0
@@ -294,8 +299,8 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_nt_kernel(GemmAr
 
   // operand rows of this lane inside a stage (weight rows follow the kBM rows)
   const int arow = 64 * wm + (lane & 31);
-  const int brow0 = kBM + (SWIGLU ? 32 * wn + (lane & 31) : 64 * wn + (lane & 31));
-  const int brow1 = SWIGLU ? brow0 + kBN / 2 : brow0 + 32;
+  const int brow0 = kBM + 64 * wn + (lane & 31);
+  const int brow1 = brow0 + 32;
   const int sw = (lane & 7) ^ ((lane >> 3) & 1);  // (row & 7) ^ ((row >> 3) & 1) of every operand row of this lane
   const int half = lane >> 5;   // which 8 of the 16 K values of an MFMA step
   const int oa0 = arow * kRowBytes, oa1 = (arow + 32) * kRowBytes;
@@ -349,13 +354,7 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_nt_kernel(GemmAr
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
       const int m = m0 + 64 * wm + 32 * i + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-      if (SWIGLU) {
-        const int n = n0 + 32 * wn + (lane & 31);
-        const float res = mep_silu(acc[i][0][v]) * acc[i][1][v];
-        a.C[(size_t)m * ldc + n] = (uint16_t)mep_f32_to_bf16_bits(res);
-        if (a.Cg) a.Cg[(size_t)m * ldc + n] = (uint16_t)mep_f32_to_bf16_bits(acc[i][0][v]);
-        if (a.Cu) a.Cu[(size_t)m * ldc + n] = (uint16_t)mep_f32_to_bf16_bits(acc[i][1][v]);
-      } else if (MODE == kModeWgrad) {
+      if (MODE == kModeWgrad) {
 #pragma unroll
         for (int j = 0; j < 2; ++j)
           // streaming stores: 58 MB of output per group passing through L2 as ordinary
@@ -423,10 +422,14 @@ __device__ __forceinline__ const char* mep_uniform(const char* p) {
                        (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v));
 }
 
-// 16 bytes per lane straight into LDS: lane offsets voff from a uniform base
-__device__ __forceinline__ void mep_load_lds16(const char* base, uint32_t voff, uint32_t soff, char* lds) {
-  __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, -1, 0x00020000);
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, soff, 0, 0);
+constexpr int kNontemporal = 2;  // cache policy of a buffer load
+
+// 16 bytes per lane straight into LDS: lane offsets voff from a uniform base.  bytes = 0: nothing
+// is read (every offset is past the end) and the lanes' LDS vectors come out undefined.
+template <int AUX = 0>
+__device__ __forceinline__ void mep_load_lds16(const char* base, uint32_t voff, uint32_t soff, char* lds, int bytes = -1) {
+  __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes, 0x00020000);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, soff, 0, AUX);
 }
 template <int VM>
 __device__ __forceinline__ void mep_wait_vm_lgkm0() {
@@ -854,6 +857,197 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
   if (!WGRAD && a.zero_tail) zero_tail_rows(a, blockIdx.x, gridDim.x, kPThreads);
 }
 // ---------------------------------------------------------------------------
+// Forward products of groups of about one 128-row block (decode batches): every weight is read
+// once and its bytes are the time, 805 MB for 16 experts of 4096 x 2048.
+//
+// A unit is 32 weight rows (SwiGLU: 16 gate rows and the same 16 up rows) times one 128-row block.
+// Tiles are 128 rows x one to nine units, so that the tiles of all blocks fill the CUs evenly
+// however many groups have rows (whole 128 x 256 tiles leave 17 blocks of 4096 weight rows with
+// 272 tiles for 256 CUs: a second round for sixteen of them) and the rows come from L2 once for up
+// to 288 weight rows.  A K step of 64 is 16 KB of rows and 4 KB a unit; the whole LDS holds D of
+// them, D - 1 on their way (72 KB of weights per CU at nine units) while one is multiplied, with
+// one barrier a step.  8 waves: 32 rows each, every other unit.  All of a step's fragments are
+// asked for before the next loads are issued (behind them they waited: 78 against 54 us where a
+// tile has one or two units); weights are loaded nontemporal, so that the rows stay in L2 (183
+// against 202 us at 17 blocks).  K goes up in every tile as in the other kernels: the order of a
+// sum does not depend on where its tile lies.  (Workgroups that start at different K steps, and
+// so do not all read the same column of rows of one pitch, took 168 us.)
+//
+// The tiles of a block divide its units evenly and are as many as fill whole rounds of the grid:
+// cut where a CU's even share of the list ends, a tile in two blocks ran its K loop twice with
+// half the weights in flight (17 blocks: 209 us).
+//
+// Measured, FFN forward of 64 tokens, K = 8, experts of 4096 x 2048, E = 128 on 8 ranks, before
+// (128 x 256 tiles) -> now: 16 blocks 200 -> 168 us, 17 blocks 290 -> 183 us (4.7 TB/s of
+// weights), 18 blocks (two rounds) 323 -> 216 us; 7168 x 2048, 33 blocks 720 -> 582 us.
+// ---------------------------------------------------------------------------
+constexpr int kSThreads = 512;
+constexpr int kSUnits = 9;                 // most units of a tile
+constexpr int kSA = kBM * kRowBytes;       // 16 KB
+constexpr int kSUnit = 32 * kRowBytes;     // 4 KB
+constexpr int kSLds = 160 * 1024;
+
+template <int MODE, int NU>
+__device__ __forceinline__ void stream_tile(const GemmArgs& a, char* gsm, int m0, int g, int unit0) {
+  constexpr bool SWIGLU = MODE == kModeSwiglu;
+  constexpr int kStageBytes = kSA + NU * kSUnit;
+  constexpr int D = kSLds / kStageBytes < 8 ? kSLds / kStageBytes : 8;
+  constexpr int kHi = (NU + 1) / 2, kLo = NU / 2;  // units of the waves 0 .. 3 and 4 .. 7; as many pieces to load
+  static_assert(D >= 3 && (D - 1) * (2 + kHi) < 64, "the loads on their way must fit the 6-bit counter");
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l31 = lane & 31, half = lane >> 5;
+  const int rb = wave & 3, uh = wave >> 2;
+  const bool lower = wave < 4;
+  const size_t ld = (size_t)a.K * 2;
+  const int KT = a.K / kBK;
+
+  // ---- loads.  A wave brings the row pieces 2 wave, 2 wave + 1 and the weight pieces wave + 8 i
+  // (1 KB: 8 rows of 128 bytes); vector q of LDS row r lies at q ^ (r & 7) ^ ((r >> 3) & 1)
+  const int r = lane >> 3, kv = lane & 7;
+  const char* pA = mep_uniform((const char*)a.A + (size_t)(m0 + 16 * wave) * ld);
+  const uint16_t* mat = SWIGLU && (wave >> 1 & 1) ? a.B2 : a.B;
+  const int row0 = SWIGLU ? 16 * (unit0 + (wave >> 2)) + 8 * (wave & 1) : 32 * unit0 + 8 * wave;
+  const char* pB = mep_uniform((const char*)mat + ((size_t)g * a.N + row0) * ld);
+  const uint32_t strideB = (uint32_t)((SWIGLU ? 32 : 64) * ld);
+  uint32_t vA[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) vA[q] = (uint32_t)((8 * q + r) * ld + ((kv ^ r ^ q) * 16));
+  const uint32_t vB = (uint32_t)(r * ld + ((kv ^ r ^ (wave & 1)) * 16));
+  int kl = 0, ws = 0, rs = 0;
+  auto issue = [&]() {
+    const int bytes = __builtin_amdgcn_readfirstlane(kl < KT ? -1 : 0);  // past the last step: counted, but nothing is read
+    char* slot = gsm + ws;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) mep_load_lds16(pA, vA[q], 0, slot + (2 * wave + q) * 1024, bytes);
+#pragma unroll
+    for (int i = 0; i < kLo; ++i) mep_load_lds16<kNontemporal>(pB, vB, i * strideB, slot + kSA + (wave + 8 * i) * 1024, bytes);
+    if (kHi > kLo && lower) mep_load_lds16<kNontemporal>(pB, vB, kLo * strideB, slot + kSA + (wave + 8 * kLo) * 1024, bytes);
+    pA += kRowBytes; pB += kRowBytes;
+    ++kl;
+    ws = ws == (D - 1) * kStageBytes ? 0 : ws + kStageBytes;
+  };
+#pragma unroll
+  for (int k = 0; k < D - 1; ++k) issue();
+
+  mep_f32x16 acc[kHi];
+#pragma unroll
+  for (int i = 0; i < kHi; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[i][v] = 0.0f;
+  const int sw = (lane & 7) ^ ((lane >> 3) & 1);
+  int ad[4];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) ad[ks] = l31 * kRowBytes + ((2 * ks + half) ^ sw) * 16;
+
+  for (int kt = 0; kt < KT; ++kt) {
+    // this wave's part of step kt is there; after the barrier everybody's, and the slot of the
+    // step before has been read by all
+    if (kHi == kLo || lower) mep_wait_vm_lgkm0<(D - 2) * (2 + kHi)>();
+    else mep_wait_vm_lgkm0<(D - 2) * (2 + kLo)>();
+    mep_bar();
+    const char* sa = gsm + rs + rb * 32 * kRowBytes;
+    const char* sb = gsm + rs + kSA + uh * kSUnit;
+    mep_bf16x8 fa[4], fb[4][kHi];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      fa[ks] = *(const mep_bf16x8*)(sa + ad[ks]);
+#pragma unroll
+      for (int i = 0; i < kHi; ++i)  // one more than the upper waves multiply, where NU is odd
+        fb[ks][i] = *(const mep_bf16x8*)(sb + ad[ks] + (i < kLo || lower ? 2 * i * kSUnit : 0));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    issue();
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+#pragma unroll
+      for (int i = 0; i < kLo; ++i)
+        acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[ks], fb[ks][i], acc[i], 0, 0, 0);
+      if (kHi > kLo && lower)
+        acc[kHi - 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[ks], fb[ks][kHi - 1], acc[kHi - 1], 0, 0, 0);
+    }
+    rs = rs == (D - 1) * kStageBytes ? 0 : rs + kStageBytes;
+  }
+  mep_wait_vm_lgkm0<0>();  // the loads past the last step write LDS, too
+  mep_bar();               // the next tile may be loaded
+
+  // ---- epilogue: acc[i][v] is row 32 rb + 8 (v / 4) + 4 half + v % 4, weight row l31 of unit 2 i + uh
+  const int m = m0 + 32 * rb + 4 * half;
+#pragma unroll
+  for (int i = 0; i < kHi; ++i) {
+    if (i >= kLo && !lower) break;
+    const int unit = unit0 + 2 * i + uh;
+    if (SWIGLU) {
+      // gate in the lanes 0 .. 15 of a half wave, up in 16 .. 31: the first take the rows of
+      // v = 0 .. 7, the others of v = 8 .. 15, and hand each other what they lack
+      const bool up = l31 >= 16;
+      const size_t first = (size_t)(m + (up ? 16 : 0)) * a.N + 16 * unit + (l31 & 15);
+#pragma unroll
+      for (int v = 0; v < 8; ++v) {
+        const float mine = up ? acc[i][v + 8] : acc[i][v];
+        const float other = __shfl_xor(up ? acc[i][v] : acc[i][v + 8], 16);
+        const float gv = up ? other : mine, uv = up ? mine : other;
+        const size_t o = first + (size_t)(8 * (v >> 2) + (v & 3)) * a.N;
+        a.C[o] = (uint16_t)mep_f32_to_bf16_bits(mep_silu(gv) * uv);
+        if (a.Cg) a.Cg[o] = (uint16_t)mep_f32_to_bf16_bits(gv);
+        if (a.Cu) a.Cu[o] = (uint16_t)mep_f32_to_bf16_bits(uv);
+      }
+    } else {
+      uint16_t* c = a.C + (size_t)m * a.N + 32 * unit + l31;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int dr = 8 * (v >> 2) + (v & 3);
+        const float sc = a.scale ? a.scale[m + dr] : 1.0f;
+        c[(size_t)dr * a.N] = (uint16_t)mep_f32_to_bf16_bits(sc * acc[i][v]);
+      }
+    }
+  }
+}
+
+template <int MODE>
+__global__ __launch_bounds__(kSThreads, 2) void gemm_stream_kernel(GemmArgs a) {
+  extern __shared__ __attribute__((aligned(1024))) char gsm[];
+  const int per_block = a.N / (MODE == kModeSwiglu ? 16 : 32);
+  const int blocks = min(a.mtiles, a.cu[a.G - 1] / kBM);
+  // `per` tiles of a block: as many as make the tiles of all blocks whole rounds of the grid
+  const int least = (per_block + kSUnits - 1) / kSUnits;
+  const int rounds = (blocks * least + (int)gridDim.x - 1) / (int)gridDim.x;
+  const int per = min(per_block, rounds * (int)gridDim.x / max(blocks, 1));
+  // neighbours in the list on one XCD: a block's rows, and the weights of a group of two blocks
+  const int nw = gridDim.x >> 3;
+  const int p = (int)(blockIdx.x & 7) * nw + (int)(blockIdx.x >> 3);
+  const int total = blocks * per;
+  const int end = (int)((int64_t)total * (p + 1) / (int)gridDim.x);
+  for (int t = (int)((int64_t)total * p / (int)gridDim.x); t < end; ++t) {
+    const int mt = t / per, tl = t - mt * per;
+    const int unit0 = tl * per_block / per;
+    const int n = (tl + 1) * per_block / per - unit0;
+    // the group of this block: the first whose padded end lies beyond it
+    int g = -1;
+    for (int c = 0; c < a.G && g < 0; c += 64) {
+      const int gi = c + (int)(threadIdx.x & 63);
+      const uint64_t mask = __ballot(gi < a.G && a.cu[gi] > mt * kBM);
+      if (mask) g = c + __ffsll((unsigned long long)mask) - 1;
+    }
+    g = __builtin_amdgcn_readfirstlane(g);
+    if (g < 0) break;  // cannot happen: the block lies below the last end
+    const int m0 = mt * kBM;
+    switch (n) {
+      case 1: stream_tile<MODE, 1>(a, gsm, m0, g, unit0); break;
+      case 2: stream_tile<MODE, 2>(a, gsm, m0, g, unit0); break;
+      case 3: stream_tile<MODE, 3>(a, gsm, m0, g, unit0); break;
+      case 4: stream_tile<MODE, 4>(a, gsm, m0, g, unit0); break;
+      case 5: stream_tile<MODE, 5>(a, gsm, m0, g, unit0); break;
+      case 6: stream_tile<MODE, 6>(a, gsm, m0, g, unit0); break;
+      case 7: stream_tile<MODE, 7>(a, gsm, m0, g, unit0); break;
+      case 8: stream_tile<MODE, 8>(a, gsm, m0, g, unit0); break;
+      default: stream_tile<MODE, 9>(a, gsm, m0, g, unit0); break;
+    }
+  }
+  if (a.zero_tail) zero_tail_rows(a, blockIdx.x, gridDim.x, kSThreads);
+}
+
+// ---------------------------------------------------------------------------
 // [batch, rows, cols] -> [batch, cols, rows] of 2-byte elements through a
 // 64 x 64 LDS tile (rows and cols multiples of 64): 128-byte reads and writes.
 // ---------------------------------------------------------------------------
@@ -983,6 +1177,18 @@ int gemm_launch(const GemmArgs& a, int64_t total, hipStream_t st) {
   return mep_launch_status();
 }
 
+template <int MODE>
+int gemm_stream_launch(const GemmArgs& a, hipStream_t st) {
+  const int64_t units = (int64_t)a.mtiles * (a.N / (MODE == kModeSwiglu ? 16 : 32));
+  MEP_REQUIRE(units > 0 && units < ((int64_t)1 << 30), MEP_ERR_UNSUPPORTED);
+  // offsets inside a tile are 32 bits
+  MEP_REQUIRE((int64_t)32 * kSUnits * 2 * a.K < ((int64_t)1 << 31), MEP_ERR_UNSUPPORTED);
+  const int irc = mep_ensure_init();
+  if (irc != MEP_OK) return irc;
+  hipLaunchKernelGGL((gemm_stream_kernel<MODE>), dim3(pp_grid((units + 7) / 8)), dim3(kSThreads), kSLds, st, a);
+  return mep_launch_status();
+}
+
 // weight gradient on 256 x 256 tiles (a.M, a.N multiples of 256, a.G even)
 template <bool TN>
 int wgrad_pp_launch(const GemmArgs& a, hipStream_t st) {
@@ -1034,27 +1240,40 @@ bool for_ranks(GemmArgs& a, int nranks) {
   return true;
 }
 
-// Which tiles.  The 256 x 256 kernel is the faster one wherever its tiles are filled.  Where the
-// groups have about one 128-row block each (decode batches: the padding alone fills it) half of
-// its matrix work and of its LDS would be idle, and the 128 x 256 kernel streams the weights
-// better (64 tokens, 16 experts of 4096 x 2048: SwiGLU 152 against 168 us; 512 tokens: 226
-// against 198).  The rows of the groups are only known on the device; M less the padding that
-// G groups can have at token_padding = 128 is what the rows of the G / 2 local experts fill.
-// mep_set_gemm_row_tile(128 or 256) forces one (tests run both on small shapes).
+// Which kernel.  The rows of the groups are only known on the device; M less the padding that G
+// groups can have at token_padding = 128 is about what the rows fill.
+// mep_set_gemm_row_tile(128 or 256) forces one side (tests run both on small shapes).
 std::atomic<int> g_forced_row_tile{0};
 
-static bool use_256_tiles(const GemmArgs& a) {
+bool use_256_tiles(const GemmArgs& a, bool forward) {
   if (a.G != a.Gr) return true;  // several ranks
   const int forced = g_forced_row_tile.load(std::memory_order_relaxed);
   if (forced) return forced == 256;
-  return 2 * ((int64_t)a.M - (int64_t)(kBM - 1) * a.G) >= (int64_t)kBM * a.G;
+  const int64_t rows = std::max((int64_t)a.M - (int64_t)(kBM - 1) * a.G, (int64_t)0);
+  // products of the backward pass: 256-row tiles unless half of their matrix work would be padding
+  if (!forward) return 2 * rows >= (int64_t)kBM * a.G;
+  // Forward products: what a K step costs either kernel.  The local experts (half of the groups)
+  // and a slot or two have rows, the last block of each about half filled.  A round of 256 x 256
+  // tiles takes 1.57 us a step whether it is full or not; the streaming kernel 0.21 us for each
+  // unit of 128 x 32 that a CU has.  Measured (FFN forward, us, streaming / 256 x 256): experts of
+  // 4096 x 2048, E = 128, K = 8: 64 tokens 183 / 289, 256 245 .. 277 / 301; 512 404 / 302;
+  // 7168 x 2048, E = 256: 256 tokens 597 / 738, 512 800 / 765; 1024 x 512, E = 64: 512 tokens
+  // 44 / 51, 1024 76 / 53; 512 x 256, E = 16, K = 4, 2048 tokens: 34 / 40.
+  const int64_t cus = std::max(mep_device_cu_count(), 8);
+  const int64_t active = a.G / 2 + 1;
+  const int64_t blocks = std::max(active, rows / kBM + a.G / 4);
+  const int64_t row_tiles = std::max(active, blocks / 2 + a.G / 8);
+  const int64_t rounds = (row_tiles * a.ntiles + cus - 1) / cus;
+  return 1570 * rounds * cus < 210 * blocks * 8 * a.ntiles;  // a tile is eight units wide
 }
 
 // C = rows x weights for the modes that tile the rows; BKN: weights as [K, N]
 template <int MODE, bool BKN>
 int row_tiled(const GemmArgs& a, hipStream_t st) {
-  if (use_256_tiles(a)) return gemm_pp_launch<MODE, BKN>(a, st);
-  return gemm_launch<MODE, BKN>(a, (int64_t)a.mtiles * a.ntiles, st);
+  constexpr bool forward = !BKN && (MODE == kModeScale || MODE == kModeSwiglu);
+  if (use_256_tiles(a, forward)) return gemm_pp_launch<MODE, BKN>(a, st);
+  if constexpr (forward) return gemm_stream_launch<MODE>(a, st);
+  else return gemm_launch<MODE, BKN>(a, (int64_t)a.mtiles * a.ntiles, st);
 }
 
 int gemm_nt_forward(const void* A, const void* B, const void* B_up, const int32_t* cu, int G, void* C,
@@ -1128,8 +1347,8 @@ int mep_init_gemm_kernels() {
   const size_t ring = (size_t)kStages * kStage;
   int rc = MEP_OK;
 #define MEP_OPT(k, b) if (rc == MEP_OK) rc = opt_in_lds(k, b)
-  MEP_OPT((grouped_gemm_nt_kernel<kModeScale, false>), ring);
-  MEP_OPT((grouped_gemm_nt_kernel<kModeSwiglu, false>), ring);
+  MEP_OPT((gemm_stream_kernel<kModeScale>), kSLds);
+  MEP_OPT((gemm_stream_kernel<kModeSwiglu>), kSLds);
   MEP_OPT((grouped_gemm_nt_kernel<kModeDual, false>), ring);
   MEP_OPT((grouped_gemm_nt_kernel<kModeWgrad, false>), ring);
   MEP_OPT((grouped_gemm_nt_kernel<kModeScale, true>), ring);
