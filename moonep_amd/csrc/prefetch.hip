@@ -12,6 +12,8 @@
 // serialises a thread's loads.
 #include "mep_common.h"
 
+#include <algorithm>
+
 namespace {
 
 constexpr int kBlock = 256;
@@ -432,26 +434,86 @@ struct CastArgs {
   uint16_t* dst[kMaxTensors];
   int64_t elems[kMaxTensors];       // of a rank's block, a multiple of 8
   int64_t dst_stride[kMaxTensors];  // elements between ranks' blocks of dst; src is dense
+  int ntensors, nranks;
 };
 
+// fp32 -> bf16: 4 bytes read and 2 written an element, bound by HBM.  One walk over all tensors'
+// and ranks' blocks in order, two workgroups per CU, the next tile's loads ahead of the current
+// stores.  A tile is 256 threads x kCastVec vectors of four floats kCastStep apart (the layout of
+// the streams below); a pair of lanes exchanges halves of two packed vectors, so that loads and
+// stores are 16 bytes a lane and whole lines a wave.
+// Measured, three projections of 8 ranks x 8 experts of 2048 x 1024 (2.4 GB): 383 us, 6.3 TB/s;
+// 464 us with all 24 blocks walked at once and 32 bytes per thread.  Vectors 4 KiB apart 409, plain
+// stores 432, stores written through 398, eight workgroups per CU 412.
+constexpr int kCastVec = 4;
+constexpr int64_t kCastStep = 32768;              // bytes of the source
+constexpr int64_t kCastSpan = kCastStep * kCastVec;  // a group of kCastStep / 4 KiB tiles
+
 __global__ __launch_bounds__(kBlock) void cast_kernel(CastArgs a) {
-  const int ti = blockIdx.z;
-  const float* src = a.src[ti] + (int64_t)blockIdx.y * a.elems[ti];
-  uint16_t* dst = a.dst[ti] + (int64_t)blockIdx.y * a.dst_stride[ti];
-  const int64_t n = a.elems[ti], step = (int64_t)gridDim.x * kBlock * 8;
-  auto pack = [](mep_u4 x, mep_u4 y) {
-    auto f = [](uint32_t v) { return __uint_as_float(v); };
-    return mep_u4{mep_pack_bf16(f(x[0]), f(x[1])), mep_pack_bf16(f(x[2]), f(x[3])),
-                  mep_pack_bf16(f(y[0]), f(y[1])), mep_pack_bf16(f(y[2]), f(y[3]))};
-  };
-  int64_t i = ((int64_t)blockIdx.x * kBlock + threadIdx.x) * 8;
-  for (; i + step < n; i += 2 * step) {  // two steps' loads in flight
-    const mep_u4 x0 = mep_ld16_stream(src + i), y0 = mep_ld16_stream(src + i + 4);
-    const mep_u4 x1 = mep_ld16_stream(src + i + step), y1 = mep_ld16_stream(src + i + step + 4);
-    mep_st16(dst + i, pack(x0, y0));
-    mep_st16(dst + i + step, pack(x1, y1));
+  constexpr int kTilesPerSpan = (int)(kCastStep / (kBlock * 16));
+  auto f = [](uint32_t v) { return __uint_as_float(v); };
+  const bool odd = threadIdx.x & 1;
+  for (int ti = 0; ti < a.ntensors; ++ti) {
+    const int64_t n = a.elems[ti], spans = n * 4 / kCastSpan, tiles = spans * kTilesPerSpan;
+    const int64_t all = tiles * a.nranks;
+    auto src_of = [&](int64_t t, int64_t* o) {
+      const int64_t r = t / tiles, l = t - r * tiles;
+      const int64_t span = l / kTilesPerSpan;
+      const int64_t off = span * kCastSpan + (l - span * kTilesPerSpan) * (kBlock * 16) + threadIdx.x * 16;
+      *o = r * a.dst_stride[ti] * 2 + off / 2;
+      return (const char*)a.src[ti] + r * n * 4 + off;
+    };
+    mep_u4 v[kCastVec], nx[kCastVec];
+    int64_t o, no;
+    int64_t t = blockIdx.x;
+    if (t < all) {
+      const char* p = src_of(t, &o);
+#pragma unroll
+      for (int i = 0; i < kCastVec; ++i) v[i] = mep_ld16_stream(p + i * kCastStep);
+    }
+    for (; t < all; t += gridDim.x) {
+      const bool more = t + gridDim.x < all;
+      if (more) {
+        const char* p = src_of(t + gridDim.x, &no);
+#pragma unroll
+        for (int i = 0; i < kCastVec; ++i) nx[i] = mep_ld16_stream(p + i * kCastStep);
+      }
+      char* d = (char*)a.dst[ti] + o;
+#pragma unroll
+      for (int i = 0; i < kCastVec; i += 2) {
+        // own halves of vector i and i + 1; the even lane keeps i and takes the odd lane's i
+        uint32_t q[2][2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          q[e][0] = mep_pack_bf16(f(v[i + e][0]), f(v[i + e][1]));
+          q[e][1] = mep_pack_bf16(f(v[i + e][2]), f(v[i + e][3]));
+        }
+        mep_u4 w;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const uint32_t give = odd ? q[0][j] : q[1][j];
+          const uint32_t got = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)give, 0xB1, 0xf, 0xf, true);
+          w[j] = odd ? got : q[0][j];
+          w[2 + j] = odd ? q[1][j] : got;
+        }
+        char* at = d + (odd ? (i + 1) * (kCastStep / 2) - 8 : i * (kCastStep / 2));
+        mep_st16_stream(at, w);
+      }
+#pragma unroll
+      for (int i = 0; i < kCastVec; ++i) v[i] = nx[i];
+      o = no;
+    }
+    // what the spans leave of every rank's block: eight floats per thread
+    const int64_t rest0 = spans * (kCastSpan / 4), rest = (n - rest0) / 8;
+    for (int64_t u = (int64_t)blockIdx.x * kBlock + threadIdx.x; u < rest * a.nranks; u += (int64_t)gridDim.x * kBlock) {
+      const int64_t r = u / rest, i = rest0 + (u - r * rest) * 8;
+      const float* s = a.src[ti] + r * n + i;
+      const mep_u4 x = mep_ld16_stream(s), y = mep_ld16_stream(s + 4);
+      mep_st16(a.dst[ti] + r * a.dst_stride[ti] + i,
+               mep_u4{mep_pack_bf16(f(x[0]), f(x[1])), mep_pack_bf16(f(x[2]), f(x[3])),
+                      mep_pack_bf16(f(y[0]), f(y[1])), mep_pack_bf16(f(y[2]), f(y[3]))});
+    }
   }
-  if (i < n) mep_st16(dst + i, pack(mep_ld16_stream(src + i), mep_ld16_stream(src + i + 4)));
 }
 
 struct ReduceArgs {
@@ -884,11 +946,11 @@ extern "C" int mep_cast_bf16(int ntensors, const float* const* src, void* const*
     a.elems[i] = elems_per_rank[i]; a.dst_stride[i] = dst_rank_stride[i];
     if (elems_per_rank[i] > most) most = elems_per_rank[i];
   }
+  a.ntensors = ntensors;
+  a.nranks = nranks;
   const int cus = mep_device_cu_count();
-  int64_t blocks = 8 * (int64_t)(cus > 0 ? cus : 256) / (ntensors * nranks);
-  const int64_t want = (most / 8 + kBlock - 1) / kBlock;
-  if (blocks > want) blocks = want;
-  if (blocks < 1) blocks = 1;
-  hipLaunchKernelGGL(cast_kernel, dim3((unsigned)blocks, nranks, ntensors), dim3(kBlock), 0, (hipStream_t)stream, a);
+  const int64_t want = (most * nranks / 8 + kBlock - 1) / kBlock;
+  const int64_t blocks = std::min<int64_t>(2 * (int64_t)(cus > 0 ? cus : 256), want);
+  hipLaunchKernelGGL(cast_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, (hipStream_t)stream, a);
   return mep_launch_status();
 }
