@@ -70,6 +70,7 @@ struct GemmArgs {
   // the 256 x 256 kernel takes the groups of several ranks at once: Gr groups per rank, whose rows
   // start at rank_rows * rank (cu counts from there)
   int Gr, rank_rows;
+  int width, rounds;  // 256 x 256 and streaming kernel: workgroups of an XCD that work at one time, tiles of one
 };
 
 enum { kModeScale = 0, kModeSwiglu = 1, kModeDual = 2, kModeWgrad = 3 };
@@ -391,8 +392,9 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_nt_kernel(GemmAr
 //    loads | barrier | 16 matrix instructions | barrier.  The waves 4 .. 7 run one barrier behind
 //    the waves 0 .. 3, so on every SIMD one wave multiplies while the other reads (without the
 //    shift 14 % slower; four phases of 8 instructions 2 % slower);
-//  * workgroups are persistent and walk the tile list as one stream of K steps: the next tile's
-//    loads are on their way while this one is finished and stored (10 % for K = 2048).
+//  * a workgroup walks its tiles as one stream of K steps: the next tile's loads are on their way
+//    while this one is finished and stored (10 % for K = 2048).  It takes kPSteps steps, then
+//    leaves its CU to the next one (see there).
 // Groups end on multiples of 128 rows: a group of h 128-row blocks is h / 2 tiles and, if h is
 // odd, one of 128 rows whose second phase has no matrix instructions.
 //
@@ -415,6 +417,15 @@ constexpr int kPHalf = 128 * kRowBytes;   // 16 KB: half of one operand's tile o
 constexpr int kPSlots = 5;                // of each operand
 constexpr int kPOperand = kPSlots * kPHalf;
 constexpr int kPLds = 2 * kPOperand;      // 160 KB
+// K steps of a workgroup, about 200 us.  With one share of the whole list per CU a kernel that holds
+// 32 CUs beside the product (Buffer(num_sms=32) while the FFN runs on a stream of its own) left 32
+// shares waiting until others had ended, and a communication kernel asked for meanwhile waited for
+// the whole product.  Beside dispatch and combine on 32 CUs, us, one share -> 128 steps: forward of
+// S = 4096, 7168 x 2048, E = 256 3364 -> 2930, forward and backward of S = 4096, 4096 x 2048, E = 128
+// 7177 -> 5900 (64 steps 2940 / 5600, 224 steps 3130 / 6130).  With the whole chip 2661 -> 2636 and
+// 4816 -> 4824, a layer of small experts 2481 -> 2502 (64 steps: 2 % slower): a change of workgroups
+// costs some 4 us, and their shares end more evenly.
+constexpr int kPSteps = 128;
 
 __device__ __forceinline__ const char* mep_uniform(const char* p) {
   const uint64_t v = (uint64_t)p;
@@ -474,8 +485,8 @@ struct Wgrad2Map {
 };
 
 // The tiles of one workgroup, in order.  XCD x (workgroups x, x + 8, ...) walks a contiguous
-// eighth of the list, its workgroups in turn, so the tiles that run on an XCD at one time are
-// neighbours in the list.  Row-tiled products: the list goes group by group, inside a group weight
+// eighth of the list, `width` workgroups in turn for `rounds` tiles each, then the next ones, so the
+// tiles that run on an XCD at one time are neighbours in the list.  Row-tiled products: the list goes group by group, inside a group weight
 // tile by weight tile, the group's row tiles fastest; a long group in panels of kPPanel row tiles
 // (its weights are read once per panel, its rows once per 32 / kPPanel weight tiles).  From round
 // to round a workgroup moves on by one place, so that the short last tiles of the groups do not
@@ -484,13 +495,14 @@ template <int MODE>
 struct PTiles {
   const GemmArgs& a;
   const Wgrad2Map& map;
-  int xcd, w, nw, count, first_item, r;  // this workgroup among the XCD's, tiles of the XCD, round
+  int xcd, w, nw, count, first_item, r, last;  // this workgroup among the XCD's, tiles of the XCD, rounds
   int c0, carry;             // row-tiled: 64 groups, one per lane; tiles before them
   int incl, end, blocks;     // tiles up to and including the group, its end, its 128-row blocks
   int g, m0, n0, kbeg, KT;
   bool tall;
   __device__ __forceinline__ PTiles(const GemmArgs& a_, const Wgrad2Map& map_) : a(a_), map(map_) {
-    xcd = blockIdx.x & 7; w = blockIdx.x >> 3; nw = gridDim.x >> 3; r = 0;
+    xcd = blockIdx.x & 7; nw = a.width; w = (int)(blockIdx.x >> 3) % nw;
+    r = (int)(blockIdx.x >> 3) / nw * a.rounds; last = r + a.rounds;
     tall = true; kbeg = 0; KT = 0; g = 0; m0 = 0; n0 = 0;
     if (MODE == kModeWgrad) {
       count = map.pair_count(xcd) * (a.G >> 1);
@@ -505,7 +517,7 @@ struct PTiles {
       first_item = xcd * per_xcd;
       count = min(per_xcd, total - first_item);
       count = __builtin_amdgcn_readfirstlane(count);
-      chunk(0);
+      if (a.G > 64) chunk(0);
       carry = 0;
     }
   }
@@ -524,7 +536,7 @@ struct PTiles {
       int rot = w + r;
       rot -= rot / nw * nw;
       const int item = r * nw + rot;
-      if (r * nw >= count) return false;
+      if (r >= last || r * nw >= count) return false;
       ++r;
       if (item >= count) continue;
       if (MODE == kModeWgrad) {
@@ -591,6 +603,7 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
   const size_t stepA = AT ? kBK * ldA * 2 : kBK * 2, stepB = BT ? kBK * ldB * 2 : kBK * 2;
   const int KT1 = WGRAD ? 0 : a.K / kBK;
   PTiles<MODE> ld(a, map);
+  PTiles<MODE> cp = ld;  // the tiles as they are multiplied; the groups' ends are read once for both
   const char *pA, *pB, *pB1;
   uint32_t halfA, halfB;
   int kl = 0;
@@ -725,7 +738,6 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
   };
 
   // ---- prologue: the first two K steps
-  PTiles<MODE> cp(a, map);
   if (more) {
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
@@ -886,6 +898,7 @@ constexpr int kSUnits = 9;                 // most units of a tile
 constexpr int kSA = kBM * kRowBytes;       // 16 KB
 constexpr int kSUnit = 32 * kRowBytes;     // 4 KB
 constexpr int kSLds = 160 * 1024;
+constexpr int kSParts = 2;                 // workgroups that share what a CU does
 
 template <int MODE, int NU>
 __device__ __forceinline__ void stream_tile(const GemmArgs& a, char* gsm, int m0, int g, int unit0) {
@@ -1009,16 +1022,20 @@ __global__ __launch_bounds__(kSThreads, 2) void gemm_stream_kernel(GemmArgs a) {
   extern __shared__ __attribute__((aligned(1024))) char gsm[];
   const int per_block = a.N / (MODE == kModeSwiglu ? 16 : 32);
   const int blocks = min(a.mtiles, a.cu[a.G - 1] / kBM);
-  // `per` tiles of a block: as many as make the tiles of all blocks whole rounds of the grid
+  // `per` tiles of a block: as many as make the tiles of all blocks whole rounds of the CUs
   const int least = (per_block + kSUnits - 1) / kSUnits;
-  const int rounds = (blocks * least + (int)gridDim.x - 1) / (int)gridDim.x;
-  const int per = min(per_block, rounds * (int)gridDim.x / max(blocks, 1));
-  // neighbours in the list on one XCD: a block's rows, and the weights of a group of two blocks
-  const int nw = gridDim.x >> 3;
-  const int p = (int)(blockIdx.x & 7) * nw + (int)(blockIdx.x >> 3);
+  const int width = 8 * a.width;
+  const int rounds = (blocks * least + width - 1) / width;
+  const int per = min(per_block, rounds * width / max(blocks, 1));
+  // neighbours in the list on one XCD: a block's rows, and the weights of a group of two blocks.
+  // The tiles of a share alternate between kSParts workgroups: where a kernel beside holds some
+  // of the CUs, the second half of what could not start there goes to whoever is done first (FFN
+  // forward of 64 tokens at 18 blocks beside 32 held CUs: 463 -> 367 us; alone 233 either way).
+  const int q = blockIdx.x >> 3;
+  const int p = (int)(blockIdx.x & 7) * a.width + q % a.width;
   const int total = blocks * per;
-  const int end = (int)((int64_t)total * (p + 1) / (int)gridDim.x);
-  for (int t = (int)((int64_t)total * p / (int)gridDim.x); t < end; ++t) {
+  const int end = (int)((int64_t)total * (p + 1) / width);
+  for (int t = (int)((int64_t)total * p / width) + q / a.width; t < end; t += kSParts) {
     const int mt = t / per, tl = t - mt * per;
     const int unit0 = tl * per_block / per;
     const int n = (tl + 1) * per_block / per - unit0;
@@ -1141,15 +1158,21 @@ __global__ __launch_bounds__(256) void swiglu_bwd_kernel(SwigluBwdArgs a) {
   }
 }
 
-// persistent workgroups: one per CU, fewer when there are fewer tiles (a multiple of the 8 XCDs)
-unsigned pp_grid(int64_t tiles_per_xcd) {
+// The grid of a kernel whose workgroups take a CU each, for at most `tiles` tiles per XCD of about
+// `steps` K steps: one workgroup per CU at one time (fewer where there are fewer tiles), each for
+// kPSteps steps.
+unsigned pp_split(GemmArgs& a, int64_t tiles, int64_t steps) {
   const int cus = mep_device_cu_count();
-  const int64_t per_xcd = (cus > 0 ? cus : 256) / 8;
-  return 8 * (unsigned)(tiles_per_xcd < per_xcd ? tiles_per_xcd : per_xcd);
+  const int64_t width = std::min<int64_t>(tiles, std::max(cus > 0 ? cus / 8 : 32, 1));
+  const int64_t rounds = (tiles + width - 1) / width;
+  steps = std::max<int64_t>(steps, 1);
+  a.width = (int)width;
+  a.rounds = (int)std::min(rounds, std::max<int64_t>((kPSteps + steps / 2) / steps, 1));
+  return 8 * (unsigned)(width * ((rounds + a.rounds - 1) / a.rounds));
 }
 
 template <int MODE, bool BKN>
-int gemm_pp_launch(const GemmArgs& a, hipStream_t st) {
+int gemm_pp_launch(GemmArgs a, hipStream_t st) {
   // the most row tiles the groups can need: every group has an odd number of 128-row blocks
   const int64_t total = ((int64_t)a.M / kBM + a.G + 1) / 2 * a.ntiles;
   MEP_REQUIRE(total > 0 && total < (1 << 30), MEP_ERR_UNSUPPORTED);
@@ -1157,7 +1180,7 @@ int gemm_pp_launch(const GemmArgs& a, hipStream_t st) {
   MEP_REQUIRE((int64_t)kPT * 2 * (a.K > a.N ? a.K : a.N) < ((int64_t)1 << 31), MEP_ERR_UNSUPPORTED);
   const int irc = mep_ensure_init();  // the LDS opt-in of this kernel, once per device
   if (irc != MEP_OK) return irc;
-  const dim3 grid(pp_grid((total + 7) / 8)), block(kPThreads);
+  const dim3 grid(pp_split(a, (total + 7) / 8, (int64_t)a.K / kBK * (MODE == kModeDual ? 2 : 1))), block(kPThreads);
   if (MODE == kModeScale && a.scale)
     hipLaunchKernelGGL((gemm_pp_kernel<MODE, false, BKN, MODE == kModeScale>), grid, block, kPLds, st, a, Wgrad2Map{});
   else
@@ -1178,20 +1201,22 @@ int gemm_launch(const GemmArgs& a, int64_t total, hipStream_t st) {
 }
 
 template <int MODE>
-int gemm_stream_launch(const GemmArgs& a, hipStream_t st) {
+int gemm_stream_launch(GemmArgs a, hipStream_t st) {
   const int64_t units = (int64_t)a.mtiles * (a.N / (MODE == kModeSwiglu ? 16 : 32));
   MEP_REQUIRE(units > 0 && units < ((int64_t)1 << 30), MEP_ERR_UNSUPPORTED);
   // offsets inside a tile are 32 bits
   MEP_REQUIRE((int64_t)32 * kSUnits * 2 * a.K < ((int64_t)1 << 31), MEP_ERR_UNSUPPORTED);
   const int irc = mep_ensure_init();
   if (irc != MEP_OK) return irc;
-  hipLaunchKernelGGL((gemm_stream_kernel<MODE>), dim3(pp_grid((units + 7) / 8)), dim3(kSThreads), kSLds, st, a);
+  const int cus = mep_device_cu_count();
+  a.width = (int)std::min<int64_t>((units + 7) / 8, std::max(cus > 0 ? cus / 8 : 32, 1));
+  hipLaunchKernelGGL((gemm_stream_kernel<MODE>), dim3(8 * a.width * kSParts), dim3(kSThreads), kSLds, st, a);
   return mep_launch_status();
 }
 
 // weight gradient on 256 x 256 tiles (a.M, a.N multiples of 256, a.G even)
 template <bool TN>
-int wgrad_pp_launch(const GemmArgs& a, hipStream_t st) {
+int wgrad_pp_launch(GemmArgs a, hipStream_t st) {
   Wgrad2Map map;
   const int mt = a.M / kPT, nt = a.N / kPT;
   map.slice_m = mt >= nt;
@@ -1204,7 +1229,10 @@ int wgrad_pp_launch(const GemmArgs& a, hipStream_t st) {
   MEP_REQUIRE((int64_t)kPT * 2 * (TN ? (a.M > a.N ? a.M : a.N) : a.ld) < ((int64_t)1 << 31), MEP_ERR_UNSUPPORTED);
   const int irc = mep_ensure_init();
   if (irc != MEP_OK) return irc;
-  hipLaunchKernelGGL((gemm_pp_kernel<kModeWgrad, TN, TN>), dim3(pp_grid(per_xcd)), dim3(kPThreads), kPLds, st, a, map);
+  // about half of the groups have rows
+  const int64_t steps = 2 * (a.rank_rows ? a.rank_rows : a.ld) / kBK / a.Gr;
+  hipLaunchKernelGGL((gemm_pp_kernel<kModeWgrad, TN, TN>), dim3(pp_split(a, per_xcd, steps)), dim3(kPThreads), kPLds, st, a,
+                     map);
   return mep_launch_status();
 }
 
