@@ -277,6 +277,7 @@ int mep_grad_reduce(float* local_grad, float* reduce_pool, int64_t rank_stride_e
  *   swiglu == 0: C = bf16(row_scale[m] * acc), row_scale [M] fp32 or NULL;
  *   swiglu != 0: C = bf16(silu(A*B[g]^T) * (A*B_up[g]^T)), B_up [G,N,K].
  * Rows at or beyond cu_seqlens[G-1] are not written.
+ * A and B on 16-byte boundaries, C on any element (so for every product below with a bf16 C).
  * M % 128 == 0, K % 64 == 0, N % 256 == 0 (N % 128 == 0 with swiglu).
  */
 int mep_grouped_gemm_nt(const void* A, const void* B, const void* B_up, const int32_t* cu_seqlens,

@@ -94,15 +94,20 @@ __device__ __forceinline__ mep_bf16x8 mep_tr_pair(const char* lo, const char* hi
   return __builtin_bit_cast(mep_bf16x8, z);
 }
 
+// bf16 outputs start at any element: stores of two and of eight of them at two-byte addresses (one
+// instruction each at any address; the reads keep their 16 bytes)
+typedef uint32_t mep_u1_any __attribute__((aligned(2)));
+typedef uint32_t mep_u4_any __attribute__((ext_vector_type(4), aligned(2)));
+
 // rows of C beyond a rank's last group, zeroed by `parts` workgroups of `threads` threads
 __device__ __forceinline__ void zero_tail_rows(const GemmArgs& a, int part, int parts, int threads) {
-  const mep_u4 zero = {0u, 0u, 0u, 0u};
+  const mep_u4_any zero = {0u, 0u, 0u, 0u};
   for (int r = 0; (r + 1) * a.Gr <= a.G; ++r) {
     const int first = a.cu[(r + 1) * a.Gr - 1];
     const size_t bytes = (size_t)(a.rank_rows - first) * a.N * 2;  // N is a multiple of 128
     char* base = (char*)(a.C + ((size_t)r * a.rank_rows + first) * a.N);
     for (size_t o = ((size_t)part * threads + threadIdx.x) * 16; o < bytes; o += (size_t)parts * threads * 16)
-      mep_st16_stream(base + o, zero);
+      __builtin_nontemporal_store(zero, (mep_u4_any*)(base + o));
   }
 }
 
@@ -840,7 +845,7 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
           auto put = [&](uint16_t* c, int v, int col, float v0, float v1) {
             const uint32_t w = mep_cvt_bf16x2(v0, v1);
             const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0xB1, 0xf, 0xf, true);  // the pair's other lane
-            *(uint32_t*)(c + first + (size_t)(8 * (v >> 2) + (v & 3)) * a.N + col) = __builtin_amdgcn_perm(o, w, sel);
+            *(mep_u1_any*)(c + first + (size_t)(8 * (v >> 2) + (v & 3)) * a.N + col) = __builtin_amdgcn_perm(o, w, sel);
           };
 #pragma unroll
           for (int v = 0; v < 16; v += 2) {
@@ -1313,7 +1318,7 @@ int gemm_nt_forward(const void* A, const void* B, const void* B_up, const int32_
   MEP_REQUIRE(!swiglu || (B_up && !row_scale), MEP_ERR_INVALID_ARG);
   MEP_REQUIRE(swiglu || (!C_gate && !C_up), MEP_ERR_INVALID_ARG);
   MEP_REQUIRE(((uintptr_t)A % 16 == 0) && ((uintptr_t)B % 16 == 0) && ((uintptr_t)B_up % 16 == 0) &&
-                  ((uintptr_t)C % 4 == 0) && ((uintptr_t)C_gate % 4 == 0) && ((uintptr_t)C_up % 4 == 0),
+                  ((uintptr_t)C % 2 == 0) && ((uintptr_t)C_gate % 2 == 0) && ((uintptr_t)C_up % 2 == 0),
               MEP_ERR_ALIGNMENT);
   GemmArgs a = nt_args(A, B, B_up, cu, C, row_scale, M, N, K, G, cols);
   a.Cg = (uint16_t*)C_gate;
@@ -1331,7 +1336,7 @@ int gemm_nn(const void* A1, const void* B1, const void* A2, const void* B2, cons
   if (rc != MEP_OK) return rc;
   MEP_REQUIRE(2 * (int64_t)K < ((int64_t)1 << 30), MEP_ERR_UNSUPPORTED);
   MEP_REQUIRE(((uintptr_t)A1 % 16 == 0) && ((uintptr_t)B1 % 16 == 0) && ((uintptr_t)A2 % 16 == 0) &&
-                  ((uintptr_t)B2 % 16 == 0) && ((uintptr_t)C % 4 == 0), MEP_ERR_ALIGNMENT);
+                  ((uintptr_t)B2 % 16 == 0) && ((uintptr_t)C % 2 == 0), MEP_ERR_ALIGNMENT);
   GemmArgs a = nt_args(A1, B1, B2, cu, C, row_scale, M, N, K, G, kBN);
   a.A2 = (const uint16_t*)A2;
   a.zero_tail = zero_tail;
@@ -1421,7 +1426,7 @@ extern "C" int mep_grouped_gemm_dual_nt(const void* A1, const void* B1, const vo
   MEP_REQUIRE(A2 && B2, MEP_ERR_INVALID_ARG);
   MEP_REQUIRE(2 * (int64_t)K < ((int64_t)1 << 30), MEP_ERR_UNSUPPORTED);
   MEP_REQUIRE(((uintptr_t)A1 % 16 == 0) && ((uintptr_t)B1 % 16 == 0) && ((uintptr_t)A2 % 16 == 0) &&
-                  ((uintptr_t)B2 % 16 == 0) && ((uintptr_t)C % 4 == 0), MEP_ERR_ALIGNMENT);
+                  ((uintptr_t)B2 % 16 == 0) && ((uintptr_t)C % 2 == 0), MEP_ERR_ALIGNMENT);
   GemmArgs a = nt_args(A1, B1, B2, cu_seqlens, C, nullptr, M, N, K, G, kBN);
   a.A2 = (const uint16_t*)A2;
   return row_tiled<kModeDual, false>(a, (hipStream_t)stream);
