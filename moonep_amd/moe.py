@@ -106,10 +106,13 @@ def _group_plans(group, topk_all, tpe):
     rc = _lib.lib().mep_build_dedup_ranks(dst.data_ptr(), 0, R, group.S, group.K, R, NvS, groups.data_ptr(),
                                           loffs.data_ptr(), counts.data_ptr(), work.data_ptr(), n, _lib.current_stream())
     _lib.check(rc, "mep_build_dedup_ranks")
+    t = _PlanTensors(dst, zfr, cu)
     plans = [MoonEPCommPlan(dst=dst[r], experts_to_copy=etc, zero_fill_ranges=zfr[r], remote_stats=stats[r],
                             dup_groups=groups[r], dup_loffs=loffs[r], dup_counts=counts[r], N=group.S * group.K,
                             R=R, E=group.E, NvS=NvS, K=group.K) for r in range(R)]
-    return plans, _PlanTensors(dst, zfr, cu)
+    for p in plans:
+        p.dst._group_tensors = t
+    return plans, t
 
 
 class _PlanTensors:
@@ -120,13 +123,17 @@ class _PlanTensors:
 
 
 def _plan_tensors(group, plans):
-    """The stacked tensors of ``plans``: those they are views of, where a group's own dispatch made
-    them, else stacked here (the groups' ends are then not known)."""
-    own = getattr(group, "_last_tensors", None)
-    if own is not None and len(plans) == group.R and all(
-            p.dst.data_ptr() == own.dst[r].data_ptr() for r, p in enumerate(plans)):
+    """The stacked tensors of ``plans``: those they are views of, where a whole-group dispatch made
+    them (any of those in flight: the plans carry them), else stacked here; the groups' ends are
+    known to the former only."""
+    own = getattr(plans[0].dst, "_group_tensors", None)
+    # `own` holds its memory, so an equal address is the same memory
+    if own is None or len(plans) != group.R or any(
+            p.dst.data_ptr() != own.dst[r].data_ptr() for r, p in enumerate(plans)):
+        return _PlanTensors(torch.stack([p.dst for p in plans]), torch.stack([p.zero_fill_ranges for p in plans]), None)
+    if all(p.zero_fill_ranges.data_ptr() == own.zero_fill[r].data_ptr() for r, p in enumerate(plans)):
         return own
-    return _PlanTensors(torch.stack([p.dst for p in plans]), torch.stack([p.zero_fill_ranges for p in plans]), None)
+    return _PlanTensors(own.dst, torch.stack([p.zero_fill_ranges for p in plans]), own.cu)
 
 
 def _check_group_tokens(group, x_all, w_all):
@@ -148,7 +155,7 @@ class _GroupDispatch(torch.autograd.Function):
         rows, slots = _dispatch_all(group, x_all.contiguous(), None if w_all is None else w_all.contiguous(),
                                     t.dst, t.zero_fill, t.cu)
         ctx.group, ctx.t, ctx.has_w = group, t, w_all is not None
-        group.last_plans, group.last_cu_seqlens, group._last_tensors = plans, t.cu, t
+        group.last_plans, group.last_cu_seqlens = plans, t.cu
         ctx.mark_non_differentiable(t.cu)
         return rows, slots, t.cu
 

@@ -98,3 +98,56 @@ def test_views_and_gradient_sums_of_a_group(cuda, R, epn, shapes):
     torch.cuda.synchronize()
     for a, b in zip(own, want):
         assert torch.equal(a, b)
+
+
+def _routed(cuda, R, E, S, K, H, seed):
+    topk = torch.stack([routing.popularity_biased(S, K, E, R, r, 1.0, seed=seed) for r in range(R)])
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(R, S, H, generator=g).to(torch.bfloat16).to(cuda).requires_grad_()
+    return x, topk.to(cuda), routing.tokens_per_expert(topk, E).to(cuda)
+
+
+def test_two_dispatches_of_a_group_in_flight(cuda, monkeypatch):
+    """Micro-batches: the first one's combine and its backward work from the first one's plans."""
+    R, epn, S, K, H, tp = 4, 2, 21, 3, 136, 16
+    group = moe.EmulatedGroup(S, H, K, R * epn, R, token_padding=tp)
+    batches = [_routed(cuda, R, R * epn, S, K, H, seed) for seed in (1, 2)]
+    gout = torch.randn(R, S, H, device=cuda).to(torch.bfloat16)
+
+    def finish(x, rows, plans):
+        out = moe.group_combine(group, plans, rows * 2)
+        return (out.detach(), *torch.autograd.grad(out, (rows, x), gout))
+
+    want = []
+    for x, topk, tpe in batches:
+        rows, _, cu, plans = moe.group_dispatch(group, x, None, topk, tpe)
+        want.append(finish(x, rows, plans))
+    seen = []
+    run = moe._dispatch_all
+    monkeypatch.setattr(moe, "_dispatch_all", lambda *a: seen.append(a[3:]) or run(*a))
+    flying = [moe.group_dispatch(group, x, None, topk, tpe) for x, topk, tpe in batches]
+    del seen[:]
+    for (x, _, _), (rows, _, cu, plans), w in zip(batches, flying, want):
+        for a, b in zip(finish(x, rows, list(plans)), w):
+            assert torch.equal(a, b)
+        dst, zero_fill, ends = seen.pop()
+        # the plans' own tensors, nothing stacked, and the groups' ends known
+        assert dst.data_ptr() == plans[0].dst.data_ptr() and zero_fill.data_ptr() == plans[0].zero_fill_ranges.data_ptr()
+        assert ends is not None and torch.equal(ends, cu)
+    group.destroy()
+
+
+def test_combine_of_a_group_takes_the_ranges_of_the_plans_it_is_given(cuda):
+    import dataclasses
+    R, epn, S, K, H, tp = 4, 2, 21, 3, 136, 16
+    group = moe.EmulatedGroup(S, H, K, R * epn, R, token_padding=tp)
+    x, topk, tpe = _routed(cuda, R, R * epn, S, K, H, 1)
+    _, _, _, plans = moe.group_dispatch(group, x, None, topk, tpe)
+    other = [dataclasses.replace(p, zero_fill_ranges=p.zero_fill_ranges * 0) for p in plans]
+    t = moe._plan_tensors(group, other)
+    assert torch.equal(t.zero_fill, torch.zeros_like(t.zero_fill)) and t.dst.data_ptr() == plans[0].dst.data_ptr()
+    cloned = moe._plan_tensors(group, [p.clone() for p in plans])
+    assert torch.equal(cloned.dst, t.dst) and cloned.cu is None
+    turned = moe._plan_tensors(group, plans[::-1])
+    assert torch.equal(turned.dst, t.dst.flip(0))
+    group.destroy()
