@@ -45,14 +45,41 @@ class EmulatedGroup:
         self.NvS = self.world.NvS
         lay = self.world.layout
         self._mcp = lay["meta_chunk_padded"]
+        # what the last whole-group operator dispatched or combined, until somebody asks for it in
+        # the world's shards: rows [R,NvS,H]; slots [R,NvS], or 0.0 after a dispatch without weights
+        self._rows = self._slots = None
+
+    def _note(self, rows, slots=None):
+        self._rows = rows.detach()     # its own tensor: a reference to the caller's would keep the graph alive
+        if slots is not None:
+            self._slots = slots.detach() if isinstance(slots, torch.Tensor) else slots
 
     def shards(self) -> torch.Tensor:
-        return self.world.hidden_buf.view(self.R, self.NvS, self.H)
+        """Every rank's shard ``[R, NvS, H]`` as the last whole-group operator saw it: the rows that
+        ``group_dispatch`` wrote, or those that ``group_combine`` (or the backward pass of either)
+        read or wrote.  It is the memory that the group's Buffers work on; the operators work on
+        tensors of their own, and the rows are copied here by this call."""
+        view = self.world.hidden_buf.view(self.R, self.NvS, self.H)
+        if self._rows is not None:
+            self._rows.record_stream(torch.cuda.current_stream())   # may be another than the operator's
+            view.copy_(self._rows)
+            self._rows = None
+        return view
 
     def weight_slots(self) -> torch.Tensor:
-        return self.world.meta_buf.view(self.R, self._mcp)[:, :self.NvS].view(torch.float32)
+        """Every rank's route-weight slots ``[R, NvS]``, likewise; zeros after a dispatch without weights."""
+        view = self.world.meta_buf.view(self.R, self._mcp)[:, :self.NvS].view(torch.float32)
+        if self._slots is not None:
+            if isinstance(self._slots, torch.Tensor):
+                self._slots.record_stream(torch.cuda.current_stream())
+                view.copy_(self._slots)
+            else:
+                view.zero_()
+            self._slots = None
+        return view
 
     def destroy(self):
+        self._rows = self._slots = None
         for b in self.buffers:
             b.destroy()
 
@@ -69,6 +96,7 @@ def _group_ctx(group):
 def _dispatch_all(group, x_all, w_all, dst_all, zero_fill, cu):
     """Rows ``[R,NvS,H]`` (+ slots ``[R,NvS]``) of every rank; every row is written."""
     ctx, R = _group_ctx(group), group.R
+    group._rows = None     # its memory is free for the new rows
     # without the groups' ends (plans of another origin) the rows behind them are cleared first
     make = torch.empty if cu is not None else torch.zeros
     rows = make(R, group.NvS, group.H, dtype=torch.bfloat16, device=x_all.device)
@@ -155,6 +183,7 @@ class _GroupDispatch(torch.autograd.Function):
         rows, slots = _dispatch_all(group, x_all.contiguous(), None if w_all is None else w_all.contiguous(),
                                     t.dst, t.zero_fill, t.cu)
         ctx.group, ctx.t, ctx.has_w = group, t, w_all is not None
+        group._note(rows, 0.0 if slots is None else slots)
         group.last_plans, group.last_cu_seqlens = plans, t.cu
         ctx.mark_non_differentiable(t.cu)
         return rows, slots, t.cu
@@ -165,7 +194,9 @@ class _GroupDispatch(torch.autograd.Function):
         if ctx.has_w:
             slots = (torch.zeros(g_rows.shape[:2], dtype=torch.float32, device=g_rows.device) if g_slots is None
                      else g_slots.float().contiguous())
-        gx, gw = _combine_all(ctx.group, g_rows.to(torch.bfloat16).contiguous(), slots, ctx.t.dst)
+        rows = g_rows.to(torch.bfloat16).contiguous()
+        ctx.group._note(rows, slots)
+        gx, gw = _combine_all(ctx.group, rows, slots, ctx.t.dst)
         return None, gx, gw, None, None
 
 
@@ -176,12 +207,16 @@ class _GroupCombine(torch.autograd.Function):
     def forward(ctx, group, plans, y_all):
         ctx.group, ctx.t = group, _plan_tensors(group, plans)
         assert tuple(y_all.shape) == (group.R, group.NvS, group.H)
-        return _combine_all(group, y_all.to(torch.bfloat16).contiguous(), None, ctx.t.dst)[0]
+        rows = y_all.to(torch.bfloat16).contiguous()
+        group._note(rows)
+        return _combine_all(group, rows, None, ctx.t.dst)[0]
 
     @staticmethod
     def backward(ctx, g_out):
         t, g = ctx.t, g_out.to(torch.bfloat16).contiguous()
-        return None, None, _dispatch_all(ctx.group, g, None, t.dst, t.zero_fill, t.cu)[0]
+        rows = _dispatch_all(ctx.group, g, None, t.dst, t.zero_fill, t.cu)[0]
+        ctx.group._note(rows)
+        return None, None, rows
 
 
 class _GroupPrefetch(torch.autograd.Function):

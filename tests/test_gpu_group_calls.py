@@ -151,3 +151,27 @@ def test_combine_of_a_group_takes_the_ranges_of_the_plans_it_is_given(cuda):
     turned = moe._plan_tensors(group, plans[::-1])
     assert torch.equal(turned.dst, t.dst.flip(0))
     group.destroy()
+
+
+def test_shards_of_a_group_hold_what_its_operators_worked_on(cuda):
+    R, epn, S, K, H, tp = 4, 2, 21, 3, 136, 16
+    group = moe.EmulatedGroup(S, H, K, R * epn, R, token_padding=tp)
+    x, topk, tpe = _routed(cuda, R, R * epn, S, K, H, 1)
+    w = torch.rand(R, S, K, device=cuda)
+    rows, slots, _, plans = moe.group_dispatch(group, x, w, topk, tpe)
+    assert torch.equal(group.shards(), rows) and torch.equal(group.weight_slots(), slots)
+    assert group.shards().data_ptr() == group.buffers[0].hidden_nvsh_buffer_view.data_ptr()
+    # what a rank's own Buffer makes of them
+    one = group.buffers[1].combine(plans[1], group.buffers[1].hidden_nvsh_buffer_view, zero_copy=True)[0]
+    y = rows * 2
+    out = moe.group_combine(group, plans, y)
+    assert torch.equal(group.shards(), y.detach()) and torch.equal(group.weight_slots(), slots)
+    assert torch.equal(out[1], one * 2)      # doubled throughout: every rounding is the same
+    g_y, = torch.autograd.grad(out, y, torch.ones_like(out), retain_graph=True)
+    assert torch.equal(group.shards(), g_y)
+    g_rows = torch.randn(R, group.NvS, H, device=cuda).to(torch.bfloat16)
+    torch.autograd.grad(rows, x, g_rows)
+    assert torch.equal(group.shards(), g_rows)
+    rows, none, _, _ = moe.group_dispatch(group, x, None, topk, tpe)
+    assert none is None and torch.equal(group.shards(), rows) and not group.weight_slots().any()
+    group.destroy()
