@@ -20,6 +20,7 @@
 
 #include <initializer_list>
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "../../include/moonep_hip.h"
@@ -38,6 +39,7 @@ struct Ctx {
   c10::Stream comm = c10::Stream(c10::Stream::UNSAFE, c10::Device(c10::kCPU), 0);
   hipStream_t comm_raw = nullptr;
   hipEvent_t order = nullptr;
+  std::mutex order_mutex;  // record and wait of `order` belong together
   PyObject *plan_type = nullptr, *hidden_local_py = nullptr, *no_map_token = nullptr, *event_type = nullptr,
            *comm_py = nullptr, *empty = nullptr;
   PyObject *py_N = nullptr, *py_R = nullptr, *py_E = nullptr, *py_NvS = nullptr, *py_K = nullptr;
@@ -62,6 +64,8 @@ bool failed(int rc, const char* what) {
   return true;
 }
 
+const char* const kOrdering = "ordering the communication stream";
+
 const at::Tensor* tensor(PyObject* o) { return THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr; }
 
 bool is(const at::Tensor& t, at::ScalarType dt, const Ctx& c) {
@@ -85,6 +89,13 @@ at::Tensor view_of(const at::Tensor& base, caffe2::TypeMeta dtype, int64_t offse
 
 PyObject* new_none() { Py_RETURN_NONE; }
 
+// Other Python threads run meanwhile: an allocation may wait for the device and a launch for a place
+// in a full queue.  Nothing of Python may be touched inside.
+struct NoGil {
+  PyThreadState* state = PyEval_SaveThread();
+  ~NoGil() { PyEval_RestoreThread(state); }
+};
+
 // ---- asynchronous calls: the work goes to the communication stream -----------------------
 struct Async {
   Ctx& c;
@@ -95,13 +106,13 @@ struct Async {
       PyObject* o = PyObject_GetAttrString(c.comm_py, "cuda_stream");
       c.comm_raw = o ? (hipStream_t)PyLong_AsVoidPtr(o) : nullptr;
       Py_XDECREF(o);
+      if (PyErr_Occurred()) throw python_error();
     }
     stream = on ? c.comm_raw : c10::hip::getCurrentHIPStream(c.hidden_buf.device().index()).stream();
   }
   // after the caller's work; the allocator must not reuse what the stream still works on
-  bool begin(std::initializer_list<const at::Tensor*> used) {
-    if (!on) return true;
-    if (PyErr_Occurred()) return false;
+  int begin(std::initializer_list<const at::Tensor*> used) {
+    if (!on) return MEP_OK;
     const c10::StorageImpl* seen[24];
     int n = 0;
     for (const at::Tensor* t : used) {
@@ -114,10 +125,11 @@ struct Async {
       t->record_stream(c.comm);
     }
     hipStream_t main = c10::hip::getCurrentHIPStream(c.hidden_buf.device().index()).stream();
+    std::lock_guard<std::mutex> lock(c.order_mutex);
     hipError_t e = c.order ? hipSuccess : hipEventCreateWithFlags(&c.order, hipEventDisableTiming);
     if (e == hipSuccess) e = hipEventRecord(c.order, main);
     if (e == hipSuccess) e = hipStreamWaitEvent(c.comm_raw, c.order, 0);
-    return !failed((int)e, "ordering the communication stream");
+    return (int)e;
   }
   // a new reference to the completion event
   PyObject* end() {
@@ -248,38 +260,44 @@ PyObject* py_dispatch(PyObject*, PyObject* const* args, Py_ssize_t n) {
     tpe = tensor(args[4]);
     if (!topk || !is(*topk, at::kInt, c) || topk->dim() == 3 || topk->numel() != c.N) return new_none();
     if (!tpe || !is(*tpe, at::kInt, c) || tpe->dim() != 2 || !shape(*tpe, {c.R, c.E})) return new_none();
-    new_plan(c, &plan, &cu);
   } else if (!read_plan(c, args[5], &plan)) {
     return new_none();
   }
-  at::Tensor out = zero_copy ? c.hidden_local : at::empty({c.NvS, c.H}, c.hidden_buf.options());
-  at::Tensor w_local = view_of(c.weights_local, caffe2::TypeMeta::Make<float>(), c.weights_local.storage_offset(), {c.NvS});
-  at::Tensor w_out;
-  if (w) w_out = w_zero_copy ? w_local : at::empty({c.NvS}, c.hidden_buf.options().dtype(at::kFloat));
-
   Async as(c, async);
-  if (!as.begin({hidden, w, &out, &w_out, &plan.dst, &plan.etc, &plan.zfr, &plan.stats, &plan.dup_groups,
-                 &plan.dup_loffs, &plan.dup_counts, topk, tpe, &cu}))
-    return nullptr;
-  if (fresh) {
-    const int rc = mep_plan_fresh(ptr<int>(*tpe), ptr<int>(*topk), c.rank, c.S, c.K, c.E, c.R, c.tp, c.NvS,
-                                  ptr<int>(plan.dst), ptr<int>(cu), ptr<int>(plan.etc), ptr<int>(plan.zfr),
-                                  ptr<int>(plan.stats), ptr<int>(plan.dup_counts), ptr<void>(c.scratch),
-                                  c.scratch.defined() ? c.scratch.nbytes() : 0, hidden->data_ptr(),
-                                  hidden->nbytes(), as.stream);
-    if (failed(rc, "mep_plan")) return nullptr;
-  }
-  int rc = mep_dispatch(hidden->data_ptr(), w ? ptr<float>(*w) : nullptr, ptr<int>(plan.dst), ptr<int>(plan.zfr),
+  at::Tensor out, w_out;
+  const char* what = kOrdering;
+  int rc;
+  {
+    NoGil other_threads;
+    if (fresh) new_plan(c, &plan, &cu);
+    out = zero_copy ? c.hidden_local : at::empty({c.NvS, c.H}, c.hidden_buf.options());
+    at::Tensor w_local = view_of(c.weights_local, caffe2::TypeMeta::Make<float>(), c.weights_local.storage_offset(), {c.NvS});
+    if (w) w_out = w_zero_copy ? w_local : at::empty({c.NvS}, c.hidden_buf.options().dtype(at::kFloat));
+    rc = as.begin({hidden, w, &out, &w_out, &plan.dst, &plan.etc, &plan.zfr, &plan.stats, &plan.dup_groups,
+                   &plan.dup_loffs, &plan.dup_counts, topk, tpe, &cu});
+    if (rc == MEP_OK && fresh) {
+      what = "mep_plan";
+      rc = mep_plan_fresh(ptr<int>(*tpe), ptr<int>(*topk), c.rank, c.S, c.K, c.E, c.R, c.tp, c.NvS,
+                          ptr<int>(plan.dst), ptr<int>(cu), ptr<int>(plan.etc), ptr<int>(plan.zfr),
+                          ptr<int>(plan.stats), ptr<int>(plan.dup_counts), ptr<void>(c.scratch),
+                          c.scratch.defined() ? c.scratch.nbytes() : 0, hidden->data_ptr(),
+                          hidden->nbytes(), as.stream);
+    }
+    if (rc == MEP_OK) {
+      what = "mep_dispatch";
+      rc = mep_dispatch(hidden->data_ptr(), w ? ptr<float>(*w) : nullptr, ptr<int>(plan.dst), ptr<int>(plan.zfr),
                         c.hidden_buf.data_ptr(), c.NvS, w ? ptr<float>(c.meta_buf) : nullptr, c.wslot_stride,
                         c.rank, c.S, c.H, c.K, c.R, c.epn, c.NvS, c.tp, MEP_DISPATCH_WRITE_DUPS, as.stream);
-  if (failed(rc, "mep_dispatch")) return nullptr;
-  const bool copy_w = w && !w_zero_copy;
-  if (!zero_copy || copy_w) {
-    rc = mep_copy_shard(zero_copy ? nullptr : out.data_ptr(), zero_copy ? nullptr : c.hidden_local.data_ptr(),
-                        zero_copy ? 0 : out.nbytes(), copy_w ? w_out.data_ptr() : nullptr,
-                        copy_w ? w_local.data_ptr() : nullptr, copy_w ? (size_t)c.NvS : 0, as.stream);
-    if (failed(rc, "mep_copy_shard")) return nullptr;
+    }
+    const bool copy_w = w && !w_zero_copy;
+    if (rc == MEP_OK && (!zero_copy || copy_w)) {
+      what = "mep_copy_shard";
+      rc = mep_copy_shard(zero_copy ? nullptr : out.data_ptr(), zero_copy ? nullptr : c.hidden_local.data_ptr(),
+                          zero_copy ? 0 : out.nbytes(), copy_w ? w_out.data_ptr() : nullptr,
+                          copy_w ? w_local.data_ptr() : nullptr, copy_w ? (size_t)c.NvS : 0, as.stream);
+    }
   }
+  if (failed(rc, what)) return nullptr;
   PyObject* event = nullptr;
   if (async && !(event = as.end())) return nullptr;
   PyObject* res = PyTuple_New(async ? 5 : 4);
@@ -318,24 +336,30 @@ PyObject* py_combine(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const bool copy_w = w && w->data_ptr() != c.weights_local.data_ptr();
   if ((zero_copy && copy_h) || (w_zero_copy && copy_w)) return new_none();
   if (async && capturing(c)) return new_none();
-  at::Tensor out = at::empty({c.S, c.H}, c.hidden_buf.options());
-  at::Tensor out_w;
-  if (w) out_w = at::empty({c.S, c.K}, c.hidden_buf.options().dtype(at::kFloat));
   Async as(c, async);
-  if (!as.begin({&out, &plan.dst, &plan.etc, &plan.zfr, &plan.stats, &plan.dup_groups, &plan.dup_loffs,
-                 &plan.dup_counts, hidden, w, &out_w}))
-    return nullptr;
+  at::Tensor out, out_w;
+  const char* what = kOrdering;
   int rc;
-  if (copy_h || copy_w) {
-    rc = mep_copy_shard(copy_h ? c.hidden_local.data_ptr() : nullptr, copy_h ? hidden->data_ptr() : nullptr,
-                        copy_h ? hidden->nbytes() : 0, copy_w ? c.weights_local.data_ptr() : nullptr,
-                        copy_w ? w->data_ptr() : nullptr, copy_w ? (size_t)c.NvS : 0, as.stream);
-    if (failed(rc, "mep_copy_shard")) return nullptr;
+  {
+    NoGil other_threads;
+    out = at::empty({c.S, c.H}, c.hidden_buf.options());
+    if (w) out_w = at::empty({c.S, c.K}, c.hidden_buf.options().dtype(at::kFloat));
+    rc = as.begin({&out, &plan.dst, &plan.etc, &plan.zfr, &plan.stats, &plan.dup_groups, &plan.dup_loffs,
+                   &plan.dup_counts, hidden, w, &out_w});
+    if (rc == MEP_OK && (copy_h || copy_w)) {
+      what = "mep_copy_shard";
+      rc = mep_copy_shard(copy_h ? c.hidden_local.data_ptr() : nullptr, copy_h ? hidden->data_ptr() : nullptr,
+                          copy_h ? hidden->nbytes() : 0, copy_w ? c.weights_local.data_ptr() : nullptr,
+                          copy_w ? w->data_ptr() : nullptr, copy_w ? (size_t)c.NvS : 0, as.stream);
+    }
+    if (rc == MEP_OK) {
+      what = "mep_combine";
+      rc = mep_combine(c.hidden_buf.data_ptr(), c.NvS, w ? ptr<float>(c.meta_buf) : nullptr, c.wslot_stride,
+                       ptr<int>(plan.dst), out.data_ptr(), w ? ptr<float>(out_w) : nullptr, c.S, c.H, c.K, c.R, c.NvS,
+                       MEP_COMBINE_TWO_LEVEL, as.stream);
+    }
   }
-  rc = mep_combine(c.hidden_buf.data_ptr(), c.NvS, w ? ptr<float>(c.meta_buf) : nullptr, c.wslot_stride,
-                   ptr<int>(plan.dst), out.data_ptr(), w ? ptr<float>(out_w) : nullptr, c.S, c.H, c.K, c.R, c.NvS,
-                   MEP_COMBINE_TWO_LEVEL, as.stream);
-  if (failed(rc, "mep_combine")) return nullptr;
+  if (failed(rc, what)) return nullptr;
   PyObject* event = async ? as.end() : new_none();
   if (!event) return nullptr;
   PyObject* res = PyTuple_New(3);
@@ -420,9 +444,17 @@ PyObject* py_prefetch(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (scale && bytes[i] % (128 * 128) != 0) return new_none();
   }
   Async as(c, async);
-  if (!as.begin({&etc, t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], t[9], t[10], t[11]})) return nullptr;
-  const int rc = mep_prefetch(m, src, dst, stride, bytes, ptr<int>(etc), c.rank, c.epn, c.R, as.stream);
-  if (failed(rc, "mep_prefetch")) return nullptr;
+  const char* what = kOrdering;
+  int rc;
+  {
+    NoGil other_threads;
+    rc = as.begin({&etc, t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], t[9], t[10], t[11]});
+    if (rc == MEP_OK) {
+      what = "mep_prefetch";
+      rc = mep_prefetch(m, src, dst, stride, bytes, ptr<int>(etc), c.rank, c.epn, c.R, as.stream);
+    }
+  }
+  if (failed(rc, what)) return nullptr;
   if (async) return as.end();
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
@@ -445,15 +477,23 @@ PyObject* py_reduce(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (!pair_ok(c, l[i], p[i]) || l[i]->scalar_type() != at::kFloat || !matrix_ok(*l[i])) return new_none();
   }
   Async as(c, async);
-  if (!as.begin({&etc, l[0], l[1], l[2], p[0], p[1], p[2]})) return nullptr;
   float *lp[3], *pp[3];
   int64_t stride[3], elems[3];
   for (int i = 0; i < 3; ++i) {
     lp[i] = ptr<float>(*l[i]); pp[i] = ptr<float>(*p[i]);
     stride[i] = p[i]->stride(0); elems[i] = l[i]->size(1) * l[i]->size(2);
   }
-  const int rc = mep_grad_reduce_batch(3, lp, pp, stride, elems, ptr<int>(etc), c.rank, 1, c.epn, c.R, 0, as.stream);
-  if (failed(rc, "mep_grad_reduce")) return nullptr;
+  const char* what = kOrdering;
+  int rc;
+  {
+    NoGil other_threads;
+    rc = as.begin({&etc, l[0], l[1], l[2], p[0], p[1], p[2]});
+    if (rc == MEP_OK) {
+      what = "mep_grad_reduce";
+      rc = mep_grad_reduce_batch(3, lp, pp, stride, elems, ptr<int>(etc), c.rank, 1, c.epn, c.R, 0, as.stream);
+    }
+  }
+  if (failed(rc, what)) return nullptr;
   if (async) return as.end();
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
@@ -523,11 +563,17 @@ PyObject* py_ffn_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   Ffn f;
   if (!read_ffn(args, &f)) return new_none();
   const bool train = args[7] == Py_True;
-  at::Tensor y = f.make({f.M, f.H}, f.bf16), act = f.make({f.M, f.Hp}, f.bf16), gp, up;
-  if (train) { gp = f.make({f.M, f.Hp}, f.bf16); up = f.make({f.M, f.Hp}, f.bf16); }
-  const int rc = mep_ffn_forward(f.rows->data_ptr(), f.slots ? ptr<float>(*f.slots) : nullptr, ptr<int>(*f.cu), f.G,
-                                 f.gate->data_ptr(), f.up->data_ptr(), f.down->data_ptr(), act.data_ptr(),
-                                 ptr<void>(gp), ptr<void>(up), y.data_ptr(), f.n, f.M, f.H, f.Hp, f.stream);
+  at::Tensor y, gp, up;
+  int rc;
+  {
+    NoGil other_threads;
+    y = f.make({f.M, f.H}, f.bf16);
+    at::Tensor act = f.make({f.M, f.Hp}, f.bf16);
+    if (train) { gp = f.make({f.M, f.Hp}, f.bf16); up = f.make({f.M, f.Hp}, f.bf16); }
+    rc = mep_ffn_forward(f.rows->data_ptr(), f.slots ? ptr<float>(*f.slots) : nullptr, ptr<int>(*f.cu), f.G,
+                         f.gate->data_ptr(), f.up->data_ptr(), f.down->data_ptr(), act.data_ptr(),
+                         ptr<void>(gp), ptr<void>(up), y.data_ptr(), f.n, f.M, f.H, f.Hp, f.stream);
+  }
   if (failed(rc, "mep_ffn_forward")) return nullptr;
   if (!train) return THPVariable_Wrap(y);
   return Py_BuildValue("(N(NN))", THPVariable_Wrap(y), THPVariable_Wrap(gp), THPVariable_Wrap(up));
@@ -563,19 +609,27 @@ PyObject* py_ffn_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
           !f.of(*s, {f.G / 2, a, b}))
         return new_none();
       w[i] = ptr<float>(*o); w2[i] = ptr<float>(*s);
-    } else {
+    }
+  }
+  at::Tensor drows, dslots;
+  int rc;
+  {
+    NoGil other_threads;
+    for (int i = 0; i < 3 && !given; ++i) {
+      const int64_t a = i < 2 ? f.Hp : f.H, b = i < 2 ? f.H : f.Hp;
       dw[i] = at::empty({f.G, a, b}, f.f32);
       w[i] = ptr<float>(dw[i]); w2[i] = w[i] + (int64_t)(f.G / 2) * a * b;
     }
+    drows = f.make({f.M, f.H}, f.bf16);
+    at::Tensor dh = f.make({f.M, f.Hp}, f.bf16), dg = f.make({f.M, f.Hp}, f.bf16), du = f.make({f.M, f.Hp}, f.bf16),
+               hs = f.make({f.M, f.Hp}, f.bf16);
+    if (f.slots) dslots = f.make({f.M}, f.f32);
+    rc = mep_ffn_backward(dy->data_ptr(), f.rows->data_ptr(), f.slots ? ptr<float>(*f.slots) : nullptr,
+                          ptr<int>(*f.cu), f.G, f.gate->data_ptr(), f.up->data_ptr(), f.down->data_ptr(),
+                          gp->data_ptr(), up->data_ptr(), dh.data_ptr(), dg.data_ptr(), du.data_ptr(),
+                          hs.data_ptr(), ptr<float>(dslots), drows.data_ptr(), w, w2, f.G / 2, f.n, f.M, f.H, f.Hp,
+                          skip ? f.G / 2 : f.G, f.stream);
   }
-  at::Tensor drows = f.make({f.M, f.H}, f.bf16), dslots, dh = f.make({f.M, f.Hp}, f.bf16),
-             dg = f.make({f.M, f.Hp}, f.bf16), du = f.make({f.M, f.Hp}, f.bf16), hs = f.make({f.M, f.Hp}, f.bf16);
-  if (f.slots) dslots = f.make({f.M}, f.f32);
-  const int rc = mep_ffn_backward(dy->data_ptr(), f.rows->data_ptr(), f.slots ? ptr<float>(*f.slots) : nullptr,
-                                  ptr<int>(*f.cu), f.G, f.gate->data_ptr(), f.up->data_ptr(), f.down->data_ptr(),
-                                  gp->data_ptr(), up->data_ptr(), dh.data_ptr(), dg.data_ptr(), du.data_ptr(),
-                                  hs.data_ptr(), ptr<float>(dslots), drows.data_ptr(), w, w2, f.G / 2, f.n, f.M, f.H, f.Hp,
-                                  skip ? f.G / 2 : f.G, f.stream);
   if (failed(rc, "mep_ffn_backward")) return nullptr;
   auto give = [](const at::Tensor& t) { return t.defined() ? THPVariable_Wrap(t) : new_none(); };
   return Py_BuildValue("(NNNNN)", give(drows), give(dslots), give(dw[0]), give(dw[1]), give(dw[2]));
