@@ -3,8 +3,8 @@
 //
 // An operator of a small batch is bound by the host: through Python and ctypes a decode step
 // (8 tokens, dispatch + combine) took 63 us for 22 us of GPU work -- nine allocations, fifteen
-// shape checks and four launches, a microsecond or more each.  Here a plan's eight tensors are
-// views of ONE allocation, and the checks cost nanoseconds.
+// shape checks and four launches, a microsecond or more each.  Here a plan's eight tensors take four
+// allocations past the dispatcher, and the checks cost nanoseconds.
 //
 // Every function returns None, with nothing launched, when the call is not the plain case it
 // handles (a failed check, a world with host threads, ...): the Python body of the operator
@@ -217,21 +217,43 @@ PyObject* wrap_plan(const Ctx& c, const Plan& p) {
   return plan;
 }
 
-// every tensor of a fresh plan and its cu_seqlens as views of one block (64-byte starts)
-at::Tensor new_plan(const Ctx& c, Plan* p, at::Tensor* cu) {
+// A dense int32 tensor of its own from the allocator that meta_buf came from, past the dispatcher.
+struct NewInts {
+  const at::Tensor& like;
+  c10::Allocator* from;
+  explicit NewInts(const Ctx& c) : like(c.meta_buf), from(c.meta_buf.storage().allocator()) {
+    if (c10::hip::current_device() != like.device().index()) from = nullptr;  // at::empty looks after that
+  }
+  at::Tensor operator()(std::initializer_list<int64_t> s) const {
+    const c10::IntArrayRef sizes(s.begin(), s.size());
+    if (!from) return at::empty(sizes, like.options());
+    const size_t bytes = (size_t)c10::multiply_integers(sizes) * sizeof(int);
+    at::Tensor t = at::detail::make_tensor<c10::TensorImpl>(
+        c10::Storage(c10::make_intrusive<c10::StorageImpl>(c10::StorageImpl::use_byte_size_t(), bytes, from->allocate(bytes),
+                                                           from, /*resizable=*/true)),
+        like.key_set(), like.dtype());
+    t.unsafeGetTensorImpl()->set_sizes_contiguous(sizes);
+    return t;
+  }
+};
+
+// A fresh plan and its cu_seqlens.  The small tensors are views of one block of a few KB (64-byte
+// starts), those that grow with the tokens own their memory, so that what a caller keeps holds
+// nothing large besides.  (Dispatch + combine of 8 tokens, host time: all eight in one block 16.9 us, so 17.5, each
+// on its own 18.2.)
+void new_plan(const Ctx& c, Plan* p, at::Tensor* cu) {
+  const NewInts make(c);
   int64_t at_int = 0;
   auto take = [&](int64_t n) { const int64_t o = at_int; at_int += (n + 15) & ~(int64_t)15; return o; };
-  const int64_t o_dst = take(c.N), o_cu = take(2 * c.epn), o_etc = take((int64_t)c.R * c.epn),
-                o_zfr = take(4 * c.epn), o_stats = take(2), o_counts = take(2), o_groups = take(3 * (int64_t)c.NvS),
-                o_loffs = take(c.NvS);
-  at::Tensor block = at::empty({at_int}, c.meta_buf.options());
+  const int64_t o_cu = take(2 * c.epn), o_etc = take((int64_t)c.R * c.epn), o_zfr = take(4 * c.epn), o_stats = take(2),
+                o_counts = take(2);
+  const at::Tensor block = make({at_int});
   auto v = [&](int64_t o, std::initializer_list<int64_t> s) {
     return view_of(block, block.dtype(), o, c10::IntArrayRef(s.begin(), s.size()));
   };
-  *p = Plan{v(o_dst, {c.N}), v(o_etc, {c.R, c.epn}), v(o_zfr, {2 * c.epn, 2}), v(o_stats, {2}),
-            v(o_groups, {c.NvS, 3}), v(o_loffs, {c.NvS}), v(o_counts, {2})};
+  *p = Plan{make({c.N}), v(o_etc, {c.R, c.epn}), v(o_zfr, {2 * c.epn, 2}), v(o_stats, {2}), make({c.NvS, 3}),
+            make({c.NvS}), v(o_counts, {2})};
   *cu = v(o_cu, {2 * c.epn});
-  return block;
 }
 
 template <class T>

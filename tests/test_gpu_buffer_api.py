@@ -310,3 +310,24 @@ def test_single_rank_group(cuda):
     want, _ = oo.combine(sh, None, torch.from_numpy(rp.dst), K1, mode="two_level")
     assert torch.equal(out.cpu().view(torch.int16), want.view(torch.int16))
     b.destroy()
+
+
+def test_what_is_kept_of_a_plan_holds_nothing_large_besides(cuda):
+    """A caller that keeps one tensor of a dispatch keeps its bytes (and a few KB), not the plan's."""
+    s, k = 2048, 8
+    topk = (torch.arange(s * k, dtype=torch.int32, device=cuda) % E).view(s, k)
+    tpe = torch.bincount(topk.flatten(), minlength=E).to(torch.int32).repeat(R, 1)
+    x = torch.zeros(s, 64, dtype=torch.bfloat16, device=cuda)
+    buf = Buffer(s, 64, k, E, R, token_padding=TP, rank=1)
+    fields = ("dst", "experts_to_copy", "zero_fill_ranges", "remote_stats", "dup_groups", "dup_loffs", "dup_counts")
+    buf.dispatch(x, None, topk, tpe, zero_copy=True)
+    torch.cuda.synchronize()
+    for name in (*fields, "cu_seqlens"):
+        before = torch.cuda.memory_allocated()
+        _, _, cu, plan = buf.dispatch(x, None, topk, tpe, zero_copy=True)
+        kept = cu if name == "cu_seqlens" else getattr(plan, name)
+        del cu, plan
+        assert torch.cuda.memory_allocated() - before <= kept.nbytes + 4096, name
+        del kept
+        assert torch.cuda.memory_allocated() == before, name
+    buf.destroy()
