@@ -12,6 +12,7 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -34,10 +35,10 @@ def build_host(verbose: bool = True) -> str:
     from torch.utils.cpp_extension import include_paths, library_paths
 
     out = os.path.join(HERE, "_host.so")
-    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-w",
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-Wextra",
            "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__=1",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-           *[f"-I{p}" for p in (*include_paths("cuda"), sysconfig.get_path("include"))],
+           *[f"-isystem{p}" for p in (*include_paths("cuda"), sysconfig.get_path("include"))],
            os.path.join(CSRC, "host.cpp"), "-o", out,
            *[f"-L{p}" for p in (*library_paths("cuda"), HERE)],
            "-lmoonep_hip", "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip", "-lamdhip64",
@@ -48,12 +49,48 @@ def build_host(verbose: bool = True) -> str:
     return out
 
 
+def gemm_assembly(out: str, wait: bool = True):
+    """The compiler's gfx950 assembly of grouped_gemm.hip, with the library's flags."""
+    hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+    cmd = [hipcc, *[f for f in FLAGS if f != "-shared"], "--cuda-device-only", "-S",
+           os.path.join(CSRC, "grouped_gemm.hip"), "-o", out]
+    proc = subprocess.Popen(cmd, stderr=subprocess.DEVNULL)      # the library's build shows the warnings
+    if wait and proc.wait():
+        raise subprocess.CalledProcessError(proc.returncode, cmd)
+    return proc
+
+
+def check_gemm_waits(path: str) -> int:
+    """Loads whose waits are counted by hand; raises where the compiler touches one before its wait."""
+    from . import asm_waits
+
+    with open(path) as f:
+        faults, followed = asm_waits.check(f.read())
+    if faults or not followed:
+        raise RuntimeError("grouped_gemm.hip as this compiler builds it is not safe to run: " +
+                           ("; ".join(faults[:8]) or "no load in an asm statement was found"))
+    return followed
+
+
 def build(verbose: bool = True) -> str:
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     cmd = [hipcc, *FLAGS, *[os.path.join(CSRC, s) for s in SOURCES], "-o", LIB]
     if verbose:
         print(" ".join(cmd), flush=True)
-    subprocess.run(cmd, check=True)
+    with tempfile.TemporaryDirectory() as tmp:
+        assembly = os.path.join(tmp, "grouped_gemm.s")
+        beside = gemm_assembly(assembly, wait=False)
+        try:
+            subprocess.run(cmd, check=True)
+        finally:
+            failed = beside.wait()
+        if failed:
+            raise subprocess.CalledProcessError(failed, beside.args)
+        try:
+            check_gemm_waits(assembly)
+        except RuntimeError:
+            os.remove(LIB)
+            raise
     build_host(verbose)
     return LIB
 

@@ -470,7 +470,9 @@ __device__ __forceinline__ uint32_t mep_cvt_bf16x2(float lo, float hi) {
 
 // Four K rows of a column block, transposed (see mep_tr_pair).  As an instruction of its own: in
 // front of the builtin the compiler waits for every load straight into LDS that is in flight.  The
-// result is there after the next wait for lgkmcnt(0); nothing may touch it before.
+// result is there after the next wait for lgkmcnt(0); nothing may touch it before.  The compiler does
+// not know that: the build reads its assembly and fails where a register of a load in an asm
+// statement is touched before its wait, or where anything is spilled (moonep_amd/asm_waits.py).
 template <class T>
 __device__ __forceinline__ void mep_tr_issue(T& x, uint32_t lds, int offset) {
   asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(x) : "v"(lds), "n"(offset));
@@ -717,7 +719,7 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
     for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        asm volatile("" : "+v"(ta[i][ks][0]), "+v"(ta[i][ks][1]));
+        asm volatile("; arrived %0 %1" : "+v"(ta[i][ks][0]), "+v"(ta[i][ks][1]));
         fa[i][ks] = join(ta[i][ks]);
       }
   };
@@ -725,7 +727,7 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
     if (!BT) return;
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
-      asm volatile("" : "+v"(tbw[ks][0]), "+v"(tbw[ks][1]));
+      asm volatile("; arrived %0 %1" : "+v"(tbw[ks][0]), "+v"(tbw[ks][1]));
       fb[ks] = join(tbw[ks]);
     }
   };
@@ -757,6 +759,7 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
   while (cp.next()) {
     const int g = cp.g, m0 = cp.m0, n0 = cp.n0, KT = cp.KT;
     const bool tall = cp.tall;
+    if (SCALED) __builtin_assume(KT > 0);
     float* cf = nullptr;
     if (WGRAD) {
       const int rank = g / a.Gr, l = g - rank * a.Gr;
@@ -816,8 +819,8 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
     }
 
     if (SCALED) {
-      if (KT < 4) mep_wait_vmcnt<0>();  // too few loads after them for the loop to have waited
-      asm volatile("" : "+v"(scl0), "+v"(scl1));
+      mep_wait_vmcnt<8>();  // a K step's loads came after them; the next phase would wait for as many
+      asm volatile("; arrived %0 %1" : "+v"(scl0), "+v"(scl1));
     }
     // ---- epilogue: acc[x][y][i][v] is row 128 x + 64 wm + 32 i + 8 (v / 4) + 4 half + v % 4,
     // column 128 y + 32 wn + l31
