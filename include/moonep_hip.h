@@ -79,7 +79,9 @@ int mep_init(void);
  * for (moonep/api.py:438-451, README.md:13: communication on 32 SMs beside the
  * expert GEMMs): every mep_* call takes a stream, so launching the path on such
  * a stream bounds all of its kernels at once, whatever their grids.  Default
- * priority.  mep_stream_cu_census records, per workgroup of a small probe
+ * priority.  The runtime makes it a stream that is ordered with the null stream
+ * (it takes no flags): what should run beside it belongs on a stream made with
+ * hipStreamNonBlocking.  mep_stream_cu_census records, per workgroup of a small probe
  * kernel, which CU it ran on (XCC id << 16 | HW_ID bits 8..15): for checking.
  */
 int mep_stream_create_limited(int num_cus, void** stream_out);

@@ -45,6 +45,8 @@ One GPU stands in for the R expert-parallel ranks.  What that changes:
   compute units: the comm stream is created with a CU mask and all operators
   (synchronous ones too, the caller's stream then waits for them) launch on
   it -- the reference's "communication on 32 SMs beside the expert GEMMs".
+  The runtime orders a CU-masked stream with the null stream, which is torch's
+  default stream: GEMMs that should run beside it go on a ``torch.cuda.Stream``.
   Left at ``None`` the kernels use the whole GPU on the caller's stream;
 * ``inter_rank_sync`` selects whether a threaded world's rendezvous are taken;
   ``enable_pdl`` and ``comm_stream_priority`` are validated like the reference

@@ -286,6 +286,11 @@ int combine_launch(const void* shards, int64_t shard_stride_rows, const float* w
     // Few tokens: up to six waves of one 1-KiB piece per SIMD (of 1024) all rows at once beat rows
     // in turn -- 64 pieces (8 tokens, H = 4096, K = 8) 3.4 against 5.2 us, 4096 6.9 against 9.5,
     // 6144 (K = 6) 9.1 against 10.2; 8192 13.7 against 13.6, 12288 (K = 6) 15.7 against 14.9.
+    // The same line on a stream of fewer CUs, where more waves queue for each: on 16, 32, 64 and
+    // 128 CUs this form is the faster one at K = 8 for every number of pieces (6144: 69 against 76,
+    // 36 / 41, 21 / 23, 12.8 / 14.0), level or faster at K = 4, and at K = 6 between 25 % faster
+    // (below 512 pieces) and 7 % slower (3072 on 64 CUs 11.2 / 10.5; 6144 on 16 CUs 65 / 62), so the
+    // rule asks neither for the device nor for the stream.
     const int64_t pieces = (int64_t)nranks * S * ((nvec + 63) / 64);
     if (K <= 8 && pieces <= kFewPieces) {
       if (K <= 4) launch_combine_few<4>(a, nranks, st);

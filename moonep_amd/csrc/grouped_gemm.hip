@@ -399,15 +399,18 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_nt_kernel(GemmAr
 //    shift 14 % slower; four phases of 8 instructions 2 % slower);
 //  * a workgroup walks its tiles as one stream of K steps: the next tile's loads are on their way
 //    while this one is finished and stored (10 % for K = 2048).  It takes kPSteps steps, then
-//    leaves its CU to the next one (see there).
+//    leaves its CU to the next one (see there).  The forward products also fetch less from HBM that
+//    way, 7.4 GB instead of 9.2 (operands 6.3): an XCD's workgroups drift apart over a long walk,
+//    and lines that several tiles share leave L2 in between.
 // Groups end on multiples of 128 rows: a group of h 128-row blocks is h / 2 tiles and, if h is
 // odd, one of 128 rows whose second phase has no matrix instructions.
 //
-// Measured at 34 560 rows in 33 groups, H = 7168, H' = 2048 (us, before -> now; before: one
+// Measured at 34 688 rows in 33 groups, H = 7168, H' = 2048 (us, before -> now; before: one
 // 256-row kernel with two LDS stages that drained its loads every step, wgrad likewise, dy * down
-// on 128 x 256 tiles): SwiGLU 2046 -> 1700, down 1150 -> 930, dy * down 1255 -> 887, dual
-// 2310 -> 1735, weight gradient 1555 -> 1285 (1.1 GB of fp32 zeroes for unused groups included);
-// 1.09 .. 1.19 PFLOP/s, where the library's dense product of such sizes reaches 1.16 .. 1.42.
+// on 128 x 256 tiles): SwiGLU 2046 -> 1705, down 1150 -> 915, dy * down 1255 -> 894, dual
+// 2310 -> 1728, weight gradient 1555 -> 1314 (1.1 GB of fp32 zeroes for unused groups included);
+// 1.11 .. 1.19 PFLOP/s for the products that tile the rows, where the library's dense product of as
+// many rows reaches 1.32 at 2048 columns and 1.49 .. 1.52 at 4096.
 //
 // LDS layouts.  Operand rows along K: 128 bytes per row and step, 16-byte vector q of row r at
 // position q ^ (r & 7) ^ ((r >> 3) & 1): sixteen consecutive lanes cover all banks.  Operands
