@@ -4,6 +4,7 @@ plan reuse vs zero-copy give the same bits; a world of R Buffers sharing the
 emulated shards reproduces the all-rank result of the oracle; bad inputs raise
 the reference's assertions; the whole chain replays from a HIP graph."""
 
+import gc
 import numpy as np
 import pytest
 import torch
@@ -322,6 +323,7 @@ def test_what_is_kept_of_a_plan_holds_nothing_large_besides(cuda):
     fields = ("dst", "experts_to_copy", "zero_fill_ranges", "remote_stats", "dup_groups", "dup_loffs", "dup_counts")
     buf.dispatch(x, None, topk, tpe, zero_copy=True)
     torch.cuda.synchronize()
+    gc.collect()
     for name in (*fields, "cu_seqlens"):
         before = torch.cuda.memory_allocated()
         _, _, cu, plan = buf.dispatch(x, None, topk, tpe, zero_copy=True)
@@ -329,5 +331,5 @@ def test_what_is_kept_of_a_plan_holds_nothing_large_besides(cuda):
         del cu, plan
         assert torch.cuda.memory_allocated() - before <= kept.nbytes + 4096, name
         del kept
-        assert torch.cuda.memory_allocated() == before, name
+        assert torch.cuda.memory_allocated() <= before, name
     buf.destroy()
