@@ -5,6 +5,7 @@ emulated shards reproduces the all-rank result of the oracle; bad inputs raise
 the reference's assertions; the whole chain replays from a HIP graph."""
 
 import gc
+
 import numpy as np
 import pytest
 import torch
