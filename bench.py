@@ -732,7 +732,7 @@ def bench_ffn(seed, steps):
         "rows_in_groups": used, "NvS": NvS, "groups": G, "maxvio": mv, "backward": bw,
         "swiglu_gate_up_us": t1, "swiglu_gate_up_TFLOPs": f1 / t1 / 1e6,
         "down_us": t2, "down_TFLOPs": f2 / t2 / 1e6,
-        "roofline": {"bound": "mfma", "kernel": "gemm_pp_kernel (SwiGLU gate/up + down)",
+        "roofline": {"bound": "mfma", "kernel": "gemm_wide_kernel (SwiGLU gate/up + down)",
                      "achieved": (f1 + f2) / (t1 + t2) / 1e6, "peak": peak, "unit": "TFLOP/s",
                      "frac": (f1 + f2) / (t1 + t2) / 1e6 / peak,
                      "traffic": measured_traffic("grouped_gemm_forward")[0]},

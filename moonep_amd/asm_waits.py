@@ -1,6 +1,6 @@
 """Loads in asm statements against the waits that make their results valid, in the compiler's assembly.
 
-``gemm_pp_kernel`` issues some loads from asm statements, because for a load that the compiler knows it
+The 256 x 256 GEMM kernels issue some loads from asm statements, because for a load that the compiler knows it
 also waits for every younger one.  To the compiler such a result is there at once: it may copy, spill
 or read the register anywhere behind the statement.  The waits are counted by hand, and the statement
 ``; arrived %0 ..`` says from where on the result may be used.  ``check`` follows every path from such
@@ -17,6 +17,7 @@ from collections import deque
 _FUNCTION = re.compile(r"^(\S+):\s*; @\1")
 _LABEL = re.compile(r"^(\.\w+):")
 _REGS = re.compile(r"\bv(?:(\d+)|\[(\d+):(\d+)\])(?!\w)")
+_ACC = re.compile(r"\ba(?:\d+|\[\d+:\d+\])(?!\w)")
 _MOST = 63      # the largest count that s_waitcnt vmcnt can name
 
 
@@ -113,12 +114,31 @@ def _follow(name, body, labels, start):
     return faults
 
 
+def _accumulators(name, body):
+    """Faults around matrix instructions in asm statements."""
+    faults = []
+    if not any(ins.in_asm and ins.op.startswith("v_mfma") for ins in body):
+        return faults
+    waited = []     # the registers that VALU instructions wrote in the last two issue slots
+    for ins in body:
+        if not ins.in_asm and _ACC.search(ins.text):
+            faults.append(f"{name}: line {ins.line}: `{ins.text}` touches an accumulation register")
+        if ins.op.startswith("v_mfma") and any(ins.regs & regs for regs in waited):
+            faults.append(f"{name}: line {ins.line}: `{ins.text}` too early after the VALU write of an operand")
+        slots = int(ins.text.split()[1]) + 1 if ins.op == "s_nop" else 0 if ins.arrived else 1
+        valu = ins.op.startswith("v_") and not ins.op.startswith("v_mfma")
+        written = _registers(ins.text.split(",")[0]) if valu else set()
+        waited = ([*waited, written] + [set()] * (slots - 1))[-2:] if slots else waited
+    return faults
+
+
 def check(assembly, kernels=("gemm_",)):
     """(faults, loads followed) of the functions whose names hold one of ``kernels``."""
     faults, followed = [], 0
     for name, (body, labels) in functions(assembly).items():
         if not any(k in name for k in kernels):
             continue
+        faults += _accumulators(name, body)
         for i, ins in enumerate(body):
             if ins.in_asm and (ins.op.startswith("ds_read") or ins.vmem) and not ins.text.endswith(" lds"):
                 followed += 1

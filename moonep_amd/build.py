@@ -18,7 +18,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libmoonep_hip.so")
 SOURCES = ["capi.hip", "planner.hip", "dispatch.hip", "combine.hip", "prefetch.hip",
-           "grouped_gemm.hip"]
+           "grouped_gemm.hip", "gemm_wide.hip"]
+GEMM_SOURCES = ["grouped_gemm.hip", "gemm_wide.hip"]    # loads in asm statements, waits counted by hand
 FLAGS = [
     "-O3", "-std=c++17", "--offload-arch=gfx950", "-fPIC", "-shared",
     "-Wall", "-Wno-unused-function",
@@ -49,11 +50,11 @@ def build_host(verbose: bool = True) -> str:
     return out
 
 
-def gemm_assembly(out: str, wait: bool = True):
-    """The compiler's gfx950 assembly of grouped_gemm.hip, with the library's flags."""
+def gemm_assembly(out: str, wait: bool = True, source: str = "grouped_gemm.hip"):
+    """The compiler's gfx950 assembly of a source of GEMM kernels, with the library's flags."""
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     cmd = [hipcc, *[f for f in FLAGS if f != "-shared"], "--cuda-device-only", "-S",
-           os.path.join(CSRC, "grouped_gemm.hip"), "-o", out]
+           os.path.join(CSRC, source), "-o", out]
     proc = subprocess.Popen(cmd, stderr=subprocess.DEVNULL)      # the library's build shows the warnings
     if wait and proc.wait():
         raise subprocess.CalledProcessError(proc.returncode, cmd)
@@ -67,7 +68,7 @@ def check_gemm_waits(path: str) -> int:
     with open(path) as f:
         faults, followed = asm_waits.check(f.read())
     if faults or not followed:
-        raise RuntimeError("grouped_gemm.hip as this compiler builds it is not safe to run: " +
+        raise RuntimeError("the GEMM kernels as this compiler builds them are not safe to run: " +
                            ("; ".join(faults[:8]) or "no load in an asm statement was found"))
     return followed
 
@@ -78,16 +79,19 @@ def build(verbose: bool = True) -> str:
     if verbose:
         print(" ".join(cmd), flush=True)
     with tempfile.TemporaryDirectory() as tmp:
-        assembly = os.path.join(tmp, "grouped_gemm.s")
-        beside = gemm_assembly(assembly, wait=False)
+        beside = []
+        for source in GEMM_SOURCES:
+            path = os.path.join(tmp, source + ".s")
+            beside.append((path, gemm_assembly(path, wait=False, source=source)))
         try:
             subprocess.run(cmd, check=True)
         finally:
-            failed = beside.wait()
+            failed = [proc for _, proc in beside if proc.wait()]
         if failed:
-            raise subprocess.CalledProcessError(failed, beside.args)
+            raise subprocess.CalledProcessError(failed[0].returncode, failed[0].args)
         try:
-            check_gemm_waits(assembly)
+            for path, _ in beside:
+                check_gemm_waits(path)
         except RuntimeError:
             os.remove(LIB)
             raise

@@ -13,8 +13,11 @@
 //            (input gradient of the gate/up pair)
 //   wgrad  : C[g] = At[:, rows of g] * Bt[:, rows of g]^T in fp32: the K range
 //            of a tile is the row range of its group (weight gradients)
-// Three kernels:
-//   gemm_pp_kernel         256 x 256 tiles, long groups, every kind
+// Four kernels:
+//   gemm_wide_kernel       (gemm_wide.hip) 256 x 256 tiles, long groups: the products that
+//                          tile the rows
+//   gemm_pp_kernel         256 x 256 tiles: weight gradients, and the other products where
+//                          few of the CUs get a tile
 //   gemm_stream_kernel     128 rows x up to 288 weight rows, forward products of
 //                          groups of about one block: bound by the weights' bytes
 //   grouped_gemm_nt_kernel 128 x 256 tiles: backward products of such groups, and
@@ -28,19 +31,15 @@
 // bytes per flop.  Tiles are handed out so that the workgroups running at one
 // time on an XCD (one L2) work on the same 8 row tiles and neighbouring weight
 // tiles.
-#include "mep_common.h"
+#include "grouped_gemm.h"
 
 #include <algorithm>
 #include <atomic>
 
 namespace {
 
-typedef __bf16 mep_bf16x8 __attribute__((ext_vector_type(8)));
-typedef float mep_f32x16 __attribute__((ext_vector_type(16)));
+using namespace mep_gemm;
 
-constexpr int kBM = 128, kBN = 256, kBK = 64;  // rows, weight rows, K per step of a tile
-constexpr int kRowBytes = kBK * 2;             // an LDS row is one 128-byte slice, no padding
-constexpr int kATile = kBM * kRowBytes, kBTile = kBN * kRowBytes;
 constexpr int kStage = kATile + kBTile;        // 48 KB
 constexpr int kStages = 3;
 constexpr int kConsumers = 8, kProducers = 2;  // waves
@@ -50,72 +49,12 @@ constexpr int kPanel = 8;  // row tiles of a long group that share a sweep over 
 constexpr int kPiecesPerProducer = (kBM + kBN) / 8 / kProducers;  // 24
 static_assert(2 * kPiecesPerProducer < 64, "two steps of loads must fit the 6-bit load counter");
 
-struct GemmArgs {
-  const uint16_t* A;   // [M,K]
-  const uint16_t* B;   // [G,N,K]
-  const uint16_t* B2;  // [G,N,K] up weights (swiglu) or null
-  const int* cu;       // [G] padded end row of each group
-  uint16_t* C;         // [M,N]
-  const float* scale;  // [M] or null
-  int M, N, K, G, mtiles, ntiles;
-  const uint16_t* A2;  // dual: rows of the second K segment [M,K]
-  uint16_t* Cg;        // swiglu: gate pre-activation [M,N] or null
-  uint16_t* Cu;        // swiglu: up pre-activation [M,N] or null
-  float* Cf;           // wgrad: [G,M,N] fp32
-  int64_t ld;          // row stride of A and B in elements (K, or the row count for wgrad)
-  int skip_from;       // wgrad: groups g >= skip_from without rows are left unwritten
-  float* Cf2;          // wgrad: the groups from `split` on go here
-  int split;
-  bool zero_tail;      // row-tiled: the rows of C beyond the last group come out as zeros
-  // the 256 x 256 kernel takes the groups of several ranks at once: Gr groups per rank, whose rows
-  // start at rank_rows * rank (cu counts from there)
-  int Gr, rank_rows;
-  int width, rounds;  // 256 x 256 and streaming kernel: workgroups of an XCD that work at one time, tiles of one
-};
-
-enum { kModeScale = 0, kModeSwiglu = 1, kModeDual = 2, kModeWgrad = 3 };
-
-__device__ __forceinline__ float mep_silu(float x) { return x / (1.0f + __expf(-x)); }
-
-// s_waitcnt vmcnt(n) alone (expcnt and lgkmcnt left at "do not wait")
-template <int N>
-__device__ __forceinline__ void mep_wait_vmcnt() {
-  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
-
-typedef short mep_s16x4 __attribute__((ext_vector_type(4)));
-typedef short mep_s16x8 __attribute__((ext_vector_type(8)));
-
 // eight K values of one column from two transposing LDS reads (K rows k .. k+3 and k+4 .. k+7)
 __device__ __forceinline__ mep_bf16x8 mep_tr_pair(const char* lo, const char* hi) {
   const mep_s16x4 x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) mep_s16x4*)lo);
   const mep_s16x4 y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) mep_s16x4*)hi);
   const mep_s16x8 z = __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7);
   return __builtin_bit_cast(mep_bf16x8, z);
-}
-
-// bf16 outputs start at any element: stores of two and of eight of them at two-byte addresses (one
-// instruction each at any address; the reads keep their 16 bytes)
-typedef uint32_t mep_u1_any __attribute__((aligned(2)));
-typedef uint32_t mep_u4_any __attribute__((ext_vector_type(4), aligned(2)));
-
-// rows of C beyond a rank's last group, zeroed by `parts` workgroups of `threads` threads
-__device__ __forceinline__ void zero_tail_rows(const GemmArgs& a, int part, int parts, int threads) {
-  const mep_u4_any zero = {0u, 0u, 0u, 0u};
-  for (int r = 0; (r + 1) * a.Gr <= a.G; ++r) {
-    const int first = a.cu[(r + 1) * a.Gr - 1];
-    const size_t bytes = (size_t)(a.rank_rows - first) * a.N * 2;  // N is a multiple of 128
-    char* base = (char*)(a.C + ((size_t)r * a.rank_rows + first) * a.N);
-    for (size_t o = ((size_t)part * threads + threadIdx.x) * 16; o < bytes; o += (size_t)parts * threads * 16)
-      __builtin_nontemporal_store(zero, (mep_u4_any*)(base + o));
-  }
-}
-
-// first row / end row of group gi
-__device__ __forceinline__ int group_end(const GemmArgs& a, int gi) { return gi / a.Gr * a.rank_rows + a.cu[gi]; }
-__device__ __forceinline__ int group_beg(const GemmArgs& a, int gi) {
-  const int r = gi / a.Gr;
-  return r * a.rank_rows + (gi > r * a.Gr ? a.cu[gi - 1] : 0);
 }
 
 // Producer / consumer waves.  Two producer waves stream the tiles from global
@@ -418,8 +357,6 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_nt_kernel(GemmAr
 // rows of 256 bytes, vector v of row k at v ^ 4 (k & 3), read with transposing LDS reads (four
 // rows of 32 bytes per sixteen lanes): two such blocks side by side cover all banks.
 // ---------------------------------------------------------------------------
-constexpr int kPT = 256;                  // tile edge
-constexpr int kPPanel = 8;                // row tiles of a long group that share a sweep over the weight tiles
 constexpr int kPThreads = 512;
 constexpr int kPHalf = 128 * kRowBytes;   // 16 KB: half of one operand's tile of a K step
 constexpr int kPSlots = 5;                // of each operand
@@ -435,175 +372,11 @@ constexpr int kPLds = 2 * kPOperand;      // 160 KB
 // costs some 4 us, and their shares end more evenly.
 constexpr int kPSteps = 128;
 
-__device__ __forceinline__ const char* mep_uniform(const char* p) {
-  const uint64_t v = (uint64_t)p;
-  return (const char*)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) |
-                       (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v));
-}
-
-constexpr int kNontemporal = 2;  // cache policy of a buffer load
-
-// 16 bytes per lane straight into LDS: lane offsets voff from a uniform base.  bytes = 0: nothing
-// is read (every offset is past the end) and the lanes' LDS vectors come out undefined.
-template <int AUX = 0>
-__device__ __forceinline__ void mep_load_lds16(const char* base, uint32_t voff, uint32_t soff, char* lds, int bytes = -1) {
-  __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes, 0x00020000);
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, soff, 0, AUX);
-}
-template <int VM>
-__device__ __forceinline__ void mep_wait_vm_lgkm0() {
-  __builtin_amdgcn_s_waitcnt((VM & 15) | (7 << 4) | ((VM >> 4) << 14));
-}
-
-__device__ __forceinline__ void mep_bar() {
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-}
-
-// two floats as bf16, rounded to nearest even by the hardware conversion
-__device__ __forceinline__ uint32_t mep_cvt_bf16x2(float lo, float hi) {
-  typedef float f32x2 __attribute__((ext_vector_type(2)));
-  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-  const f32x2 v = {lo, hi};
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
-}
-
-// Four K rows of a column block, transposed (see mep_tr_pair).  As an instruction of its own: in
-// front of the builtin the compiler waits for every load straight into LDS that is in flight.  The
-// result is there after the next wait for lgkmcnt(0); nothing may touch it before.  The compiler does
-// not know that: the build reads its assembly and fails where a register of a load in an asm
-// statement is touched before its wait, or where anything is spilled (moonep_amd/asm_waits.py).
-template <class T>
-__device__ __forceinline__ void mep_tr_issue(T& x, uint32_t lds, int offset) {
-  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(x) : "v"(lds), "n"(offset));
-}
-
-// Tile list of the weight gradient: the dimension with more tiles is cut into eight slices, one
-// per XCD (mirrored for odd groups, so that 28 tiles give every XCD 3 + 4), and every XCD takes
-// its slice of every group, two neighbouring groups at a time: all XCDs finish together whatever
-// the groups' lengths, and the tiles an XCD runs at one time are one group's slice times the whole
-// other dimension -- each line they load is wanted by 3 to 8 of them.
-struct Wgrad2Map {
-  int sliced, other;  // tiles of the sliced and of the other dimension
-  bool slice_m;       // the sliced dimension is the output row
-  __host__ __device__ int lo(int x) const { return x * sliced / 8; }
-  __host__ __device__ int size(int x) const { return (x + 1) * sliced / 8 - x * sliced / 8; }
-  __host__ __device__ int pair_count(int x) const { return (size(x) + size(7 - x)) * other; }
-};
-
-// The tiles of one workgroup, in order.  XCD x (workgroups x, x + 8, ...) walks a contiguous
-// eighth of the list, `width` workgroups in turn for `rounds` tiles each, then the next ones, so the
-// tiles that run on an XCD at one time are neighbours in the list.  Row-tiled products: the list goes group by group, inside a group weight
-// tile by weight tile, the group's row tiles fastest; a long group in panels of kPPanel row tiles
-// (its weights are read once per panel, its rows once per 32 / kPPanel weight tiles).  From round
-// to round a workgroup moves on by one place, so that the short last tiles of the groups do not
-// all go to the same ones.
-template <int MODE>
-struct PTiles {
-  const GemmArgs& a;
-  const Wgrad2Map& map;
-  int xcd, w, nw, count, first_item, r, last;  // this workgroup among the XCD's, tiles of the XCD, rounds
-  int c0, carry;             // row-tiled: 64 groups, one per lane; tiles before them
-  int incl, end, blocks;     // tiles up to and including the group, its end, its 128-row blocks
-  int g, m0, n0, kbeg, KT;
-  bool tall;
-  __device__ __forceinline__ PTiles(const GemmArgs& a_, const Wgrad2Map& map_) : a(a_), map(map_) {
-    xcd = blockIdx.x & 7; nw = a.width; w = (int)(blockIdx.x >> 3) % nw;
-    r = (int)(blockIdx.x >> 3) / nw * a.rounds; last = r + a.rounds;
-    tall = true; kbeg = 0; KT = 0; g = 0; m0 = 0; n0 = 0;
-    if (MODE == kModeWgrad) {
-      count = map.pair_count(xcd) * (a.G >> 1);
-    } else {
-      int total_rt = 0;
-      for (int c = 0; c < a.G; c += 64) {
-        chunk(c);
-        total_rt += __shfl(incl, 63);
-      }
-      const int total = total_rt * a.ntiles;
-      const int per_xcd = (total + 7) >> 3;
-      first_item = xcd * per_xcd;
-      count = min(per_xcd, total - first_item);
-      count = __builtin_amdgcn_readfirstlane(count);
-      if (a.G > 64) chunk(0);
-      carry = 0;
-    }
-  }
-  __device__ __forceinline__ void chunk(int c) {
-    c0 = c;
-    const int gi = c + (int)(threadIdx.x & 63);
-    end = gi < a.G ? group_end(a, gi) : 0;
-    int beg = gi < a.G ? group_beg(a, gi) : 0;
-    asm volatile("" : "+v"(end), "+v"(beg));  // the loads end here, not inside the main loop
-    blocks = (end - beg) / kBM;
-    incl = mep_wave_incl_scan((blocks + 1) >> 1);
-  }
-  // the next tile with work; false: no more
-  __device__ __forceinline__ bool next() {
-    for (;;) {
-      int rot = w + r;
-      rot -= rot / nw * nw;
-      const int item = r * nw + rot;
-      if (r >= last || r * nw >= count) return false;
-      ++r;
-      if (item >= count) continue;
-      if (MODE == kModeWgrad) {
-        const int per_pair = map.pair_count(xcd);
-        const int pair = item / per_pair;
-        int local = item - pair * per_pair;
-        const int n_even = map.size(xcd) * map.other;
-        g = 2 * pair;
-        int xe = xcd;
-        if (local >= n_even) { local -= n_even; g += 1; xe = 7 - xcd; }
-        const int sz = map.size(xe);
-        const int u = local / sz, sl = map.lo(xe) + (local - u * sz);
-        m0 = (map.slice_m ? sl : u) * kPT; n0 = (map.slice_m ? u : sl) * kPT;
-        typedef const __attribute__((address_space(4))) int* cptr;  // scalar loads
-        const int rank = g / a.Gr, l = g - rank * a.Gr;
-        const int first = l > 0 ? ((cptr)a.cu)[g - 1] : 0;
-        KT = (((cptr)a.cu)[g] - first) / kBK;
-        kbeg = rank * a.rank_rows + first;
-        if (KT == 0 && l >= a.skip_from) continue;
-        return true;
-      }
-      return find(item);
-    }
-  }
-  __device__ __forceinline__ bool find(int item) {
-    const int L0 = first_item + item;
-    for (;;) {
-      const uint64_t m = __ballot((carry + incl) * a.ntiles > L0);
-      if (m) {
-        const int src = __ffsll((unsigned long long)m) - 1;
-        g = c0 + src;
-        const int before = src > 0 ? __builtin_amdgcn_readlane(incl, src - 1) : 0;
-        const int hs = __builtin_amdgcn_readlane(incl, src) - before, first = carry + before;
-        const int gend = __builtin_amdgcn_readlane(end, src);
-        const int gbeg = gend - __builtin_amdgcn_readlane(blocks, src) * kBM;
-        const int local = L0 - first * a.ntiles;
-        const int panel = local / (kPPanel * a.ntiles);
-        const int within = local - panel * (kPPanel * a.ntiles);
-        const int ph = min(kPPanel, hs - panel * kPPanel);
-        const int nt = within / ph;
-        m0 = gbeg + (panel * kPPanel + (within - nt * ph)) * kPT;
-        n0 = nt * (MODE == kModeSwiglu ? kBN / 2 : kBN);
-        tall = m0 + kPT <= gend;
-        KT = MODE == kModeDual ? 2 * (a.K / kBK) : a.K / kBK;
-        return true;
-      }
-      carry += __builtin_amdgcn_readlane(incl, 63);
-      if (c0 + 64 >= a.G) return false;
-      chunk(c0 + 64);
-    }
-  }
-};
-
 // AT, BT: the operand is given as [K, columns].  SCALED: scale mode with row scales.
 template <int MODE, bool AT, bool BT, bool SCALED = false>
 __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad2Map map) {
-  constexpr bool SWIGLU = MODE == kModeSwiglu, DUAL = MODE == kModeDual, WGRAD = MODE == kModeWgrad;
+  constexpr bool DUAL = MODE == kModeDual, WGRAD = MODE == kModeWgrad;
+  static_assert(MODE != kModeSwiglu, "gemm_wide_kernel has it");
   extern __shared__ __attribute__((aligned(1024))) char gsm[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l31 = lane & 31, half = lane >> 5;
@@ -614,7 +387,7 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
   const int KT1 = WGRAD ? 0 : a.K / kBK;
   PTiles<MODE> ld(a, map);
   PTiles<MODE> cp = ld;  // the tiles as they are multiplied; the groups' ends are read once for both
-  const char *pA, *pB, *pB1;
+  const char *pA, *pB;
   uint32_t halfA, halfB;
   int kl = 0;
   auto stand = [&](int pair) {  // the pointers at the first K step of the cursor's tile (of its second pair)
@@ -623,9 +396,8 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
     const size_t offB = goff + (BT ? (size_t)ld.n0 : (size_t)ld.n0 * ldB);
     pA = mep_uniform((const char*)((pair ? a.A2 : a.A) + offA));
     pB = mep_uniform((const char*)((pair ? a.B2 : a.B) + offB));
-    pB1 = SWIGLU ? mep_uniform((const char*)(a.B2 + offB)) : pB;
     halfA = __builtin_amdgcn_readfirstlane(ld.tall ? (AT ? 256u : (uint32_t)(128 * ldA * 2)) : 0u);
-    halfB = SWIGLU ? 0u : (BT ? 256u : (uint32_t)(128 * ldB * 2));
+    halfB = BT ? 256u : (uint32_t)(128 * ldB * 2);
   };
   bool more = true;
   do { more = ld.next(); } while (more && ld.KT == 0);
@@ -635,7 +407,7 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
     if (kl + 1 < ld.KT) {
       ++kl;
       if (DUAL && kl == KT1) { stand(1); return; }
-      pA += stepA; pB += stepB; pB1 += stepB;
+      pA += stepA; pB += stepB;
       return;
     }
     do { more = ld.next(); } while (more && ld.KT == 0);
@@ -662,7 +434,7 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
   };
   auto issueB = [&](int h) {
 #pragma unroll
-    for (int q = 0; q < 2; ++q) mep_load_lds16(h ? pB1 : pB, vB[q], h ? halfB : 0u, lds_w + wB + q * 1024);
+    for (int q = 0; q < 2; ++q) mep_load_lds16(pB, vB[q], h ? halfB : 0u, lds_w + wB + q * 1024);
     turn(wB, kPOperand);
   };
 
@@ -856,11 +628,7 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
 #pragma unroll
           for (int v = 0; v < 16; v += 2) {
             const float g0 = acc[x][0][i][v], g1 = acc[x][0][i][v + 1], u0 = acc[x][1][i][v], u1 = acc[x][1][i][v + 1];
-            if (SWIGLU) {
-              put(a.C, v, 0, mep_silu(g0) * u0, mep_silu(g1) * u1);
-              if (a.Cg) put(a.Cg, v, 0, g0, g1);
-              if (a.Cu) put(a.Cu, v, 0, u0, u1);
-            } else if (SCALED) {
+            if (SCALED) {
               const int at = at0 + 4 * (32 * i + 8 * (v >> 2) + (v & 3));
               const float s0 = __int_as_float(__builtin_amdgcn_ds_bpermute(at, __float_as_int(x ? scl1 : scl0)));
               const float s1 = __int_as_float(__builtin_amdgcn_ds_bpermute(at + 4, __float_as_int(x ? scl1 : scl0)));
@@ -1182,8 +950,16 @@ unsigned pp_split(GemmArgs& a, int64_t tiles, int64_t steps) {
   return 8 * (unsigned)(width * ((rounds + a.rounds - 1) / a.rounds));
 }
 
+// about how many 256-row tiles the groups have: rows / 128 blocks are filled, about half of the
+// groups (the local experts) and a slot or two have rows
+int64_t row_tiles_256(const GemmArgs& a) {
+  const int64_t rows = std::max((int64_t)a.M - (int64_t)(kBM - 1) * a.G, (int64_t)0);
+  const int64_t blocks = std::max<int64_t>(a.G / 2 + 1, rows / kBM + a.G / 4);
+  return std::max<int64_t>(a.G / 2 + 1, blocks / 2 + a.G / 8);
+}
+
 template <int MODE, bool BKN>
-int gemm_pp_launch(GemmArgs a, hipStream_t st) {
+int gemm_256_launch(GemmArgs a, hipStream_t st) {
   // the most row tiles the groups can need: every group has an odd number of 128-row blocks
   const int64_t total = ((int64_t)a.M / kBM + a.G + 1) / 2 * a.ntiles;
   MEP_REQUIRE(total > 0 && total < (1 << 30), MEP_ERR_UNSUPPORTED);
@@ -1191,12 +967,24 @@ int gemm_pp_launch(GemmArgs a, hipStream_t st) {
   MEP_REQUIRE((int64_t)kPT * 2 * (a.K > a.N ? a.K : a.N) < ((int64_t)1 << 31), MEP_ERR_UNSUPPORTED);
   const int irc = mep_ensure_init();  // the LDS opt-in of this kernel, once per device
   if (irc != MEP_OK) return irc;
-  const dim3 grid(pp_split(a, (total + 7) / 8, (int64_t)a.K / kBK * (MODE == kModeDual ? 2 : 1))), block(kPThreads);
-  if (MODE == kModeScale && a.scale)
-    hipLaunchKernelGGL((gemm_pp_kernel<MODE, false, BKN, MODE == kModeScale>), grid, block, kPLds, st, a, Wgrad2Map{});
-  else
-    hipLaunchKernelGGL((gemm_pp_kernel<MODE, false, BKN>), grid, block, kPLds, st, a, Wgrad2Map{});
-  return mep_launch_status();
+  const unsigned grid = pp_split(a, (total + 7) / 8, (int64_t)a.K / kBK * (MODE == kModeDual ? 2 : 1));
+  // Where at most a quarter of the CUs get a tile, the time is that of one tile, whose steps wait for
+  // loads that come from HBM: two waves on a SIMD hide more of that than one.  us, gemm_pp_kernel /
+  // gemm_wide_kernel, 64 tiles of 1024 columns: dy * down K = 2048 40.7 / 43.0, K = 7168 117 / 125;
+  // down 40.2 / 40.3, 119 / 120; both pairs 74.2 / 74.1, 247 / 241; at 128 tiles 131 / 132, 131 / 125 and
+  // 271 / 248, at 256 184 / 179, 185 / 174 and 369 / 343.  SwiGLU is faster on the wide kernel down to 32
+  // tiles (48.9 / 41.7, 119 / 116).
+  if constexpr (MODE != kModeSwiglu) {
+    if (4 * row_tiles_256(a) * a.ntiles <= std::max(mep_device_cu_count(), 8)) {
+      if (MODE == kModeScale && a.scale)
+        hipLaunchKernelGGL((gemm_pp_kernel<MODE, false, BKN, MODE == kModeScale>), dim3(grid), dim3(kPThreads), kPLds, st, a,
+                           Wgrad2Map{});
+      else
+        hipLaunchKernelGGL((gemm_pp_kernel<MODE, false, BKN>), dim3(grid), dim3(kPThreads), kPLds, st, a, Wgrad2Map{});
+      return mep_launch_status();
+    }
+  }
+  return mep_launch_gemm_wide(MODE, BKN, a, grid, st);
 }
 
 // 144 KB of dynamic LDS: opted in by mep_init_gemm_kernels
@@ -1299,10 +1087,8 @@ bool use_256_tiles(const GemmArgs& a, bool forward) {
   // 7168 x 2048, E = 256: 256 tokens 597 / 738, 512 800 / 765; 1024 x 512, E = 64: 512 tokens
   // 44 / 51, 1024 76 / 53; 512 x 256, E = 16, K = 4, 2048 tokens: 34 / 40.
   const int64_t cus = std::max(mep_device_cu_count(), 8);
-  const int64_t active = a.G / 2 + 1;
-  const int64_t blocks = std::max(active, rows / kBM + a.G / 4);
-  const int64_t row_tiles = std::max(active, blocks / 2 + a.G / 8);
-  const int64_t rounds = (row_tiles * a.ntiles + cus - 1) / cus;
+  const int64_t blocks = std::max<int64_t>(a.G / 2 + 1, rows / kBM + a.G / 4);
+  const int64_t rounds = (row_tiles_256(a) * a.ntiles + cus - 1) / cus;
   return 1570 * rounds * cus < 210 * blocks * 8 * a.ntiles;  // a tile is eight units wide
 }
 
@@ -1310,7 +1096,7 @@ bool use_256_tiles(const GemmArgs& a, bool forward) {
 template <int MODE, bool BKN>
 int row_tiled(const GemmArgs& a, hipStream_t st) {
   constexpr bool forward = !BKN && (MODE == kModeScale || MODE == kModeSwiglu);
-  if (use_256_tiles(a, forward)) return gemm_pp_launch<MODE, BKN>(a, st);
+  if (use_256_tiles(a, forward)) return gemm_256_launch<MODE, BKN>(a, st);
   if constexpr (forward) return gemm_stream_launch<MODE>(a, st);
   else return gemm_launch<MODE, BKN>(a, (int64_t)a.mtiles * a.ntiles, st);
 }
@@ -1394,7 +1180,6 @@ int mep_init_gemm_kernels() {
   MEP_OPT((grouped_gemm_nt_kernel<kModeDual, true>), ring);
   MEP_OPT((gemm_pp_kernel<kModeScale, false, false>), kPLds);
   MEP_OPT((gemm_pp_kernel<kModeScale, false, false, true>), kPLds);
-  MEP_OPT((gemm_pp_kernel<kModeSwiglu, false, false>), kPLds);
   MEP_OPT((gemm_pp_kernel<kModeDual, false, false>), kPLds);
   MEP_OPT((gemm_pp_kernel<kModeScale, false, true>), kPLds);
   MEP_OPT((gemm_pp_kernel<kModeScale, false, true, true>), kPLds);
@@ -1402,7 +1187,7 @@ int mep_init_gemm_kernels() {
   MEP_OPT((gemm_pp_kernel<kModeWgrad, false, false>), kPLds);
   MEP_OPT((gemm_pp_kernel<kModeWgrad, true, true>), kPLds);
 #undef MEP_OPT
-  return rc;
+  return rc == MEP_OK ? mep_init_gemm_wide_kernels() : rc;
 }
 
 extern "C" int mep_set_gemm_row_tile(int rows) {
