@@ -166,6 +166,18 @@ int mep_dispatch(const void* hidden_SH, const float* w_SK, const int32_t* dst,
                  int token_padding, unsigned flags, void* stream);
 
 /*
+ * mep_plan_fresh, with the tokens as what it warms the cache for, and mep_dispatch with
+ * MEP_DISPATCH_WRITE_DUPS behind it.  A call that has few bytes to move runs as one kernel: the
+ * planner's workgroups copy the rows.  Same results, bit for bit.
+ */
+int mep_dispatch_fresh(const int32_t* tpe_RE, const int32_t* topk_SK, const void* hidden_SH,
+                       const float* w_SK, int rank, int S, int H, int K, int E, int R,
+                       int token_padding, int NvS, int32_t* dst, int32_t* cu_seqlens,
+                       int32_t* experts_to_copy, int32_t* zero_fill, int32_t* remote_stats,
+                       int32_t* dup_counts, void* shards, int64_t shard_stride_rows, float* wslots,
+                       int64_t wslot_stride, void* scratch, size_t scratch_bytes, void* stream);
+
+/*
  * Destination-side duplicate groups of `rank` from all ranks' dst.
  * Replaces the dedup builder warps of DispatchKernel (reference
  * moonep/dispatch.py:502-681).  Output order is deterministic (source rank,

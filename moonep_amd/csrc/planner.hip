@@ -26,7 +26,9 @@
 //      duplicates of a token on one rank found along DPP rows; store
 #include "mep_common.h"
 
+#include <algorithm>
 #include <atomic>
+#include <type_traits>
 
 namespace {
 
@@ -49,6 +51,17 @@ struct PlanArgs {
   int groups;        // workgroups per rank that plan
 };
 
+// What the planning workgroups of a small call copy themselves (mep_dispatch's arguments)
+struct CopyArgs {
+  const uint16_t* hidden;  // [S,H] bf16
+  const float* w;          // [S,K] or null
+  uint16_t* shards;
+  float* wslots;
+  int64_t shard_stride_rows, wslot_stride;
+  int H;
+};
+struct NoCopy {};
+
 // LDS layout in ints (must match plan_lds_bytes on the host)
 template <int NT>
 struct PlanLds {
@@ -59,11 +72,19 @@ struct PlanLds {
   static constexpr int FIXED = NT;
 };
 
+// COPY: plan and dispatch of a call with few bytes to move, in one launch.  Apart they are two
+// chains of latencies behind each other (8 tokens at H = 4096: planner 5.7 us, dispatch 5.7 us, of
+// which 3 are 16 MB of padding rows zeroed, and the host's second launch); the plan is in every
+// workgroup's LDS, so each, on a CU of its own, goes on with its tokens' rows and a share of the
+// padding.  A work item of a wave is 4 KB of a row.
+//
 // RC, KC: the number of ranks and top-k as compile-time constants (0: taken
 // from the arguments); the planner is a chain of dependent instructions, and
 // a kernel that knows them drops the loops, clamps and alternative paths
-template <int NT, bool kLdsTables, int RC = 0, int KC = 0>
-__global__ __launch_bounds__(NT) void plan_kernel(PlanArgs a) {
+template <int NT, bool kLdsTables, int RC = 0, int KC = 0, class Copy = NoCopy>
+__global__ __launch_bounds__(NT) void plan_kernel(PlanArgs a, Copy copy) {
+  constexpr bool COPY = !std::is_same_v<Copy, NoCopy>;
+  static_assert(!COPY || kLdsTables, "small calls only");
   using L = PlanLds<NT>;
   constexpr int NW = L::NW;
   constexpr int W4 = L::W4;
@@ -89,6 +110,7 @@ __global__ __launch_bounds__(NT) void plan_kernel(PlanArgs a) {
                         : a.scratch + (size_t)(blockIdx.y * a.groups + blockIdx.x) * 2 * E * R;
   int* alloc = tbl;            // [E,R] tokens of expert e landing on rank d
   int* base = tbl + E * R;     // [E,R] first slot of e on d, as an encoded dst
+  int* s_pad = base + E * R;   // COPY: [2*epn] first padding row, [2*epn] padding rows up to and with the group
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -117,7 +139,7 @@ __global__ __launch_bounds__(NT) void plan_kernel(PlanArgs a) {
   const int rank = a.rank0 + blockIdx.y;
   const bool writer = blockIdx.x == 0;  // one workgroup per rank stores the small outputs
   const int* topk = a.topk + (size_t)blockIdx.y * N;
-  const int t0 = blockIdx.x * a.tok_per_wg;
+  const int t0 = COPY ? min((int)blockIdx.x * a.tok_per_wg, a.S) : blockIdx.x * a.tok_per_wg;
   const int t1 = min(t0 + a.tok_per_wg, a.S);
   const int e0 = t0 * K;
   const int n = (t1 - t0) * K;  // <= NT
@@ -188,6 +210,20 @@ __global__ __launch_bounds__(NT) void plan_kernel(PlanArgs a) {
   };
   int4 ha[4], hb[6], hc[6];
   if (count_a) hist_load(ha, v0, hb1, ta, NA);
+  // COPY, several tokens a workgroup: the first 128 KB of them are on their way into its L2 meanwhile
+  // (tokens that come from HBM, 1024 at H = 4096: 23.1 -> 21.4 us; where there is one it costs 0.4 us)
+  constexpr int WARM = COPY ? 8 : 1;
+  mep_u4 warm[WARM];
+  int warm_vecs = 0;
+  if constexpr (COPY) {
+    if (a.tok_per_wg > 1) {
+      warm_vecs = (t1 - t0) * (copy.H / 8);
+      const mep_u4* rows = (const mep_u4*)copy.hidden + (size_t)t0 * (copy.H / 8);
+#pragma unroll
+      for (int u = 0; u < WARM; ++u)
+        if (tid + u * NT < warm_vecs) warm[u] = rows[tid + u * NT];
+    }
+  }
 
   for (int i = tid; i < R; i += NT) {
     s_gt[i] = 0; s_from[i] = -1; s_quota[i] = 0; s_stat1[i] = 0; s_nrem[i] = 0;
@@ -430,7 +466,7 @@ __global__ __launch_bounds__(NT) void plan_kernel(PlanArgs a) {
     const bool mine = writer && d == rank;
     int* cu = a.cu_seqlens + (size_t)blockIdx.y * 2 * epn;
     int* zf = a.zero_fill + (size_t)blockIdx.y * 4 * epn;
-    int running = 0;
+    int running = 0, padding = 0;
     for (int c = 0; c < 2 * epn; c += 64) {
       const int g = c + lane;
       int eid = -1, cnt = 0;
@@ -447,6 +483,12 @@ __global__ __launch_bounds__(NT) void plan_kernel(PlanArgs a) {
         zf[2 * g] = padded > cnt ? start + cnt : 0;
         zf[2 * g + 1] = padded - cnt;
       }
+      if constexpr (COPY)
+        if (d == rank) {
+          const int incl_pad = padding + mep_wave_incl_scan(padded - cnt);
+          if (g < 2 * epn) { s_pad[g] = start + cnt; s_pad[2 * epn + g] = incl_pad; }
+          padding = __builtin_amdgcn_readlane(incl_pad, 63);
+        }
       running += __builtin_amdgcn_readlane(incl, 63);
     }
   }
@@ -555,6 +597,82 @@ __global__ __launch_bounds__(NT) void plan_kernel(PlanArgs a) {
     a.remote_stats[2 * blockIdx.y + 1] = s_stat1[rank];
     if (a.dup_counts) { a.dup_counts[0] = 0; a.dup_counts[1] = 0; }
   }
+  if constexpr (COPY) {
+    const size_t row_bytes = (size_t)copy.H * 2;
+    if (warm_vecs > 0) {  // a comparison that guards a sleep keeps those loads
+      mep_u4 x = {0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int u = 0; u < WARM; ++u)
+        if (tid + u * NT < warm_vecs) x ^= warm[u];
+      if ((x[0] ^ x[1]) == 0x9e3779b9u && (x[2] ^ x[3]) == 0x7f4a7c15u) __builtin_amdgcn_s_sleep(1);
+    }
+    // ---- the rows and weights of this workgroup's entries
+    if (16 % K != 0) __syncthreads();  // s_cd has been read
+    s_cd[tid] = dv;
+    // (a count table that does not belong to the routing makes slots of any value: none outside the shards)
+    const unsigned slots = (unsigned)(R * NvS);
+    if (tid < n && copy.w && (unsigned)dv < slots)
+      copy.wslots[(size_t)(dv / NvS) * copy.wslot_stride + dv % NvS] = copy.w[e0 + tid];
+    __syncthreads();
+    const int pieces = (int)((row_bytes + 4095) >> 12);
+    for (int i = wave; i < n * pieces; i += NW) {
+      const int en = i / pieces, piece = i - en * pieces;
+      const int raw = __builtin_amdgcn_readfirstlane(s_cd[en]);
+      if ((unsigned)raw >= slots) continue;  // an invalid expert's
+      const int drank = raw / NvS;
+      const size_t off = (size_t)piece * 4096 + lane * 16;
+      const char* src = (const char*)copy.hidden + (size_t)((e0 + en) / K) * row_bytes + off;
+      char* to = (char*)copy.shards + ((uint64_t)drank * (uint64_t)copy.shard_stride_rows + (uint64_t)(raw - drank * NvS)) * row_bytes + off;
+      mep_u4 v[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (off + q * 1024 < row_bytes) v[q] = mep_ld16(src + q * 1024);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (off + q * 1024 < row_bytes) mep_st16_stream(to + q * 1024, v[q]);
+    }
+    // ---- this rank's padding rows (consecutive waves consecutive pieces) and their weight slots
+    const mep_u4 zero = {0u, 0u, 0u, 0u};
+    char* own = (char*)copy.shards + (uint64_t)rank * (uint64_t)copy.shard_stride_rows * row_bytes;
+    const int* upto = s_pad + 2 * epn;
+    const int rows = mep_imax(0, mep_imin(upto[2 * epn - 1], NvS));
+    // padding row r is row r + off of the shard in the group whose running count is the first beyond
+    // it; 128 groups two to a lane
+    int up[2], of[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int g = 64 * c + lane;
+      up[c] = g < 2 * epn ? upto[g] : 0;
+      of[c] = g < 2 * epn ? s_pad[g] - (g > 0 ? upto[g - 1] : 0) : 0;
+    }
+    const int stride = gridDim.x * NW, dr = stride / pieces, dp = stride - dr * pieces;
+    int r = (int)(blockIdx.x * NW + wave) / pieces, piece = (int)(blockIdx.x * NW + wave) - r * pieces;
+    while (r < rows) {
+      int at = -1;
+      const uint64_t m0 = __ballot(up[0] > r), m1 = __ballot(up[1] > r);
+      if (m0) at = r + __builtin_amdgcn_readlane(of[0], __ffsll((unsigned long long)m0) - 1);
+      else if (m1) at = r + __builtin_amdgcn_readlane(of[1], __ffsll((unsigned long long)m1) - 1);
+      else
+        for (int g = 128; g < 2 * epn && at < 0; ++g)
+          if (upto[g] > r) at = s_pad[g] + r - upto[g - 1];
+      if ((unsigned)at < (unsigned)NvS) {
+        const size_t off = (size_t)piece * 4096 + lane * 16;
+        char* to = own + (size_t)at * row_bytes + off;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (off + q * 1024 < row_bytes) mep_st16_stream(to + q * 1024, zero);
+      }
+      r += dr;
+      piece += dp;
+      if (piece >= pieces) { piece -= pieces; ++r; }
+    }
+    if (copy.w)
+      for (int g = blockIdx.x; g < 2 * epn; g += gridDim.x) {
+        const int pad = upto[g] - (g > 0 ? upto[g - 1] : 0);
+        for (int j = tid; j < pad; j += NT)
+          if ((unsigned)(s_pad[g] + j) < (unsigned)NvS) copy.wslots[(size_t)rank * copy.wslot_stride + s_pad[g] + j] = 0.0f;
+      }
+  }
 }
 
 size_t plan_lds_bytes(int nt, int E, int R, bool lds_tables) {
@@ -607,10 +725,56 @@ extern "C" size_t mep_plan_scratch_bytes(int S, int K, int E, int R, int nranks)
 }
 
 namespace {
+
+// Compile-time variants for the usual expert-parallel widths, with top-8 routing and any.  Planner
+// alone at R = 8, K = 8: 7.3 us against 8.8 us for the generic kernel; plan and dispatch of 8 to 333
+// tokens at H = 1024, generic -> R known: R = 2 8.7 -> 7.3, R = 4, K = 6 9.8 -> 8.4, R = 8, K = 4 9.4 -> 7.7,
+// R = 16, K = 4 11.7 -> 9.9.
+#define MEP_PLAN_VARIANT(R, K, LAUNCH) \
+  do {                                 \
+    if ((K) == 8 && (R) == 8) LAUNCH(8, 8);        \
+    else if ((K) == 8 && (R) == 4) LAUNCH(4, 8);   \
+    else if ((K) == 8 && (R) == 16) LAUNCH(16, 8); \
+    else if ((R) == 2) LAUNCH(2, 0);               \
+    else if ((R) == 4) LAUNCH(4, 0);               \
+    else if ((R) == 8) LAUNCH(8, 0);               \
+    else if ((R) == 16) LAUNCH(16, 0);             \
+    else LAUNCH(0, 0);                             \
+  } while (0)
+
+size_t plan_copy_lds_bytes(const PlanConfig& c, int epn) { return c.lds_bytes + 4 * (size_t)epn * sizeof(int); }
+
+// Calls whose copies are no more than this plan and dispatch in one launch.  us, two launches -> one,
+// tokens in the cache (from HBM): 8 tokens at H = 4096, E = 128 11.1 -> 10.5 (10.4 -> 9.9), 512 at 7168, E = 256
+// 26.5 -> 24.2 (26.2 -> 24.3), 1024 at 4096 22.6 -> 21.3 (22.3 -> 21.4); above it the two meet: 1024 at 7168
+// 33.1 -> 32.9 (33.0 -> 33.5), 2048 at 7168 56.8 -> 57.8 (57.1 -> 60.6).  The most padding, 8 tokens at 7168,
+// E = 256 (58 MB of it): 15.8 -> 15.8.  And the host has one launch less: Buffer.dispatch and combine of 8
+// tokens 14.4 -> 13.0.
+constexpr int64_t kCopyMost = (int64_t)64 << 20;
+
+int plan_copy_launch(PlanArgs a, const CopyArgs& copy, const PlanConfig& c, hipStream_t st) {
+  // a workgroup per CU where there are 16 KB for each, of as many tokens as it can resolve
+  const int cus = mep_device_cu_count();
+  if (cus <= 0) return MEP_ERR_INVALID_ARG;
+  const int64_t rows = (int64_t)a.S * a.K + (int64_t)2 * a.epn * (a.tp - 1);  // with the most padding
+  const int64_t want = (rows * copy.H * 2 + 16383) / 16384;
+  const int groups = (int)std::max<int64_t>(c.groups, std::min<int64_t>(want, cus));
+  a.tok_per_wg = (a.S + groups - 1) / groups;
+  a.groups = groups;
+  a.warm = nullptr;
+  a.warm_vecs = 0;
+  const size_t lds = plan_copy_lds_bytes(c, a.epn);
+#define MEP_PLAN_COPY(RC, KC) hipLaunchKernelGGL((plan_kernel<1024, true, RC, KC, CopyArgs>), dim3(groups), dim3(1024), lds, st, a, copy)
+  MEP_PLAN_VARIANT(a.R, a.K, MEP_PLAN_COPY);
+#undef MEP_PLAN_COPY
+  return mep_launch_status();
+}
+
 int plan_launch(const int32_t* tpe_RE, const int32_t* topk_nSK, int rank0, int nranks, int S, int K,
                 int E, int R, int token_padding, int NvS, int32_t* dst, int32_t* cu_seqlens,
                 int32_t* experts_to_copy, int32_t* zero_fill, int32_t* remote_stats, int32_t* dup_counts,
-                void* scratch, size_t scratch_bytes, const void* warm, size_t warm_bytes, void* stream) {
+                void* scratch, size_t scratch_bytes, const void* warm, size_t warm_bytes, void* stream,
+                const CopyArgs* copy = nullptr) {
   MEP_REQUIRE(tpe_RE && topk_nSK && dst && cu_seqlens && experts_to_copy && zero_fill &&
                   remote_stats, MEP_ERR_INVALID_ARG);
   MEP_REQUIRE(S > 0 && K > 0 && E > 0 && R > 0 && token_padding > 0 && NvS > 0, MEP_ERR_INVALID_ARG);
@@ -636,6 +800,8 @@ int plan_launch(const int32_t* tpe_RE, const int32_t* topk_nSK, int rank0, int n
   a.rank0 = rank0; a.S = S; a.K = K; a.E = E; a.R = R; a.epn = E / R; a.tp = token_padding;
   a.NvS = NvS; a.tok_per_wg = c.tok_per_wg;
   a.groups = c.groups;
+  hipStream_t st = (hipStream_t)stream;
+  if (copy) return plan_copy_launch(a, *copy, c, st);
   a.warm = (const char*)warm;
   // never more than half of the 256 MB last-level cache: beyond that the read
   // only delays the planner and evicts itself
@@ -655,25 +821,18 @@ int plan_launch(const int32_t* tpe_RE, const int32_t* topk_nSK, int rank0, int n
     warm_groups = (int)(want < cap ? want : cap);
   }
   dim3 grid(c.groups + warm_groups, nranks);
-  hipStream_t st = (hipStream_t)stream;
-  // compile-time variants for the usual expert-parallel widths with top-8 routing
-  // (7.3 us against 8.8 us for the generic kernel at R = 8)
-  if (c.nt == 1024 && K == 8 && R == 8) {
-    hipLaunchKernelGGL((plan_kernel<1024, true, 8, 8>), grid, dim3(1024), c.lds_bytes, st, a);
-  } else if (c.nt == 1024 && K == 8 && R == 4) {
-    hipLaunchKernelGGL((plan_kernel<1024, true, 4, 8>), grid, dim3(1024), c.lds_bytes, st, a);
-  } else if (c.nt == 1024 && K == 8 && R == 16) {
-    hipLaunchKernelGGL((plan_kernel<1024, true, 16, 8>), grid, dim3(1024), c.lds_bytes, st, a);
-  } else if (c.nt == 1024) {
-    hipLaunchKernelGGL((plan_kernel<1024, true>), grid, dim3(1024), c.lds_bytes, st, a);
+  if (c.nt == 1024) {
+#define MEP_PLAN(RC, KC) hipLaunchKernelGGL((plan_kernel<1024, true, RC, KC>), grid, dim3(1024), c.lds_bytes, st, a, NoCopy{})
+    MEP_PLAN_VARIANT(R, K, MEP_PLAN);
+#undef MEP_PLAN
   } else if (c.lds_tables) {
-    hipLaunchKernelGGL((plan_kernel<256, true>), grid, dim3(256), c.lds_bytes, st, a);
+    hipLaunchKernelGGL((plan_kernel<256, true>), grid, dim3(256), c.lds_bytes, st, a, NoCopy{});
   } else {
     if (c.opt_in) {  // more dynamic LDS than the default limit: opted in by mep_init_planner_kernels
       const int irc = mep_ensure_init();
       if (irc != MEP_OK) return irc;
     }
-    hipLaunchKernelGGL((plan_kernel<256, false>), grid, dim3(256), c.lds_bytes, st, a);
+    hipLaunchKernelGGL((plan_kernel<256, false>), grid, dim3(256), c.lds_bytes, st, a, NoCopy{});
   }
   return mep_launch_status();
 }
@@ -718,6 +877,33 @@ extern "C" int mep_plan_fresh(const int32_t* tpe_RE, const int32_t* topk_SK, int
   return plan_launch(tpe_RE, topk_SK, rank, 1, S, K, E, R, token_padding, NvS, dst, cu_seqlens,
                      experts_to_copy, zero_fill, remote_stats, dup_counts, scratch, scratch_bytes, warm,
                      warm_bytes, stream);
+}
+
+extern "C" int mep_dispatch_fresh(const int32_t* tpe_RE, const int32_t* topk_SK, const void* hidden_SH,
+                                  const float* w_SK, int rank, int S, int H, int K, int E, int R,
+                                  int token_padding, int NvS, int32_t* dst, int32_t* cu_seqlens,
+                                  int32_t* experts_to_copy, int32_t* zero_fill, int32_t* remote_stats,
+                                  int32_t* dup_counts, void* shards, int64_t shard_stride_rows, float* wslots,
+                                  int64_t wslot_stride, void* scratch, size_t scratch_bytes, void* stream) {
+  MEP_REQUIRE(dup_counts && hidden_SH && shards && (w_SK == nullptr) == (wslots == nullptr), MEP_ERR_INVALID_ARG);
+  MEP_REQUIRE(((uintptr_t)hidden_SH % 16 == 0) && ((uintptr_t)shards % 16 == 0), MEP_ERR_ALIGNMENT);
+  MEP_REQUIRE(H > 0 && H % 8 == 0, MEP_ERR_UNSUPPORTED);
+  MEP_REQUIRE(R > 0 && E > 0 && E % R == 0 && token_padding > 0, MEP_ERR_INVALID_ARG);
+  MEP_REQUIRE(shard_stride_rows >= NvS && (!wslots || wslot_stride >= NvS), MEP_ERR_INVALID_ARG);
+  const int epn = E / R;
+  PlanConfig c;
+  if (S > 0 && K > 0 && K <= 32 && (int64_t)S * K * H * 2 <= kCopyMost && plan_config(S, K, E, R, &c) == MEP_OK &&
+      c.nt == 1024 && plan_copy_lds_bytes(c, epn) <= kLdsDefaultLimit) {
+    const CopyArgs copy{(const uint16_t*)hidden_SH, w_SK, (uint16_t*)shards, wslots, shard_stride_rows, wslot_stride, H};
+    return plan_launch(tpe_RE, topk_SK, rank, 1, S, K, E, R, token_padding, NvS, dst, cu_seqlens, experts_to_copy,
+                       zero_fill, remote_stats, dup_counts, scratch, scratch_bytes, nullptr, 0, stream, &copy);
+  }
+  const int rc = plan_launch(tpe_RE, topk_SK, rank, 1, S, K, E, R, token_padding, NvS, dst, cu_seqlens, experts_to_copy,
+                             zero_fill, remote_stats, dup_counts, scratch, scratch_bytes, hidden_SH,
+                             (size_t)S * H * 2, stream);
+  if (rc != MEP_OK) return rc;
+  return mep_dispatch(hidden_SH, w_SK, dst, zero_fill, shards, shard_stride_rows, wslots, wslot_stride, rank, S, H, K, R,
+                      epn, NvS, token_padding, MEP_DISPATCH_WRITE_DUPS, stream);
 }
 
 extern "C" int mep_plan(const int32_t* tpe_RE, const int32_t* topk_SK, int rank, int S, int K,

@@ -1,0 +1,103 @@
+"""Plan and dispatch of a small call in one kernel against the two kernels one after the other: every
+output and every byte of the shards the same (plans, copies and zeroes: nothing is rounded)."""
+
+import pytest
+import torch
+
+from moonep_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+
+# S, H, K, E, R, rank, token_padding: one token and more tokens than CUs, rows of 16 bytes and of no whole KB,
+# every compile-time number of ranks and others, more than 64 and more than 128 groups, no padding, both sides
+# of the largest call that is one kernel (64 MiB of copies)
+CASES = [(1, 8, 1, 1, 1, 0, 1), (3, 24, 2, 8, 2, 1, 16), (8, 4096, 8, 128, 8, 4, 128), (33, 520, 6, 96, 4, 3, 64),
+         (300, 2880, 8, 64, 4, 0, 7), (257, 1032, 8, 64, 16, 15, 128), (700, 512, 4, 96, 24, 11, 16), (90, 640, 3, 160, 2, 1, 32),
+         (64, 256, 5, 60, 3, 2, 128), (1024, 256, 2, 16, 8, 7, 128), (1100, 64, 32, 128, 8, 3, 64), (40, 7168, 8, 288, 2, 0, 128),
+         (1024, 4096, 8, 128, 8, 1, 128), (1025, 4096, 8, 128, 8, 1, 128)]
+
+
+@pytest.mark.parametrize("weights", [True, False])
+@pytest.mark.parametrize("S,H,K,E,R,rank,tp", CASES)
+def test_one_launch_is_two(cuda, S, H, K, E, R, rank, tp, weights):
+    print(f"S={S} H={H} K={K} E={E} R={R} rank={rank} tp={tp}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(S + H)
+    epn = E // R
+    NvS = -(-(S * K + (tp - 1) * 2 * epn) // tp) * tp
+    skew = torch.randn(E, device=cuda, generator=g) * 0.5
+    topk = torch.topk(torch.randn(R, S, E, device=cuda, generator=g) + skew, min(K, E), dim=-1)[1].to(torch.int32)
+    counts = torch.zeros(R, E, dtype=torch.int32, device=cuda)
+    counts.scatter_add_(1, topk.reshape(R, -1).long(), torch.ones(R, S * K, dtype=torch.int32, device=cuda))
+    mine = topk[rank].contiguous()
+    if S > 30:      # ids that no expert has: entries nobody copies
+        flat = mine.view(-1)
+        for at, bad in ((5, -1), (S * K // 2, E), (S * K - 1, 2**31 - 1)):
+            counts[rank, int(flat[at])] -= 1
+            flat[at] = bad
+    x = torch.randn(S, H, device=cuda, generator=g).to(torch.bfloat16)
+    w = torch.rand(S, K, device=cuda, generator=g) if weights else None
+    stride, wstride = NvS + 3, NvS + 5
+    lib, p, s = _lib.lib(), _lib.ptr, _lib.current_stream()
+    got = []
+    for fused in (False, True):
+        ints = [torch.full(shape, -7, dtype=torch.int32, device=cuda)
+                for shape in ((S * K,), (2 * epn,), (R, epn), (2 * epn, 2), (2,), (2,))]
+        shards = torch.full((R, stride, H), 7.0, dtype=torch.bfloat16, device=cuda)
+        slots = torch.full((R, wstride), 7.0, device=cuda) if weights else None
+        scratch = torch.empty(max(int(lib.mep_plan_scratch_bytes(S, K, E, R, 1)), 16), dtype=torch.uint8, device=cuda)
+        dst, cu, etc, zf, stats, dup = map(p, ints)
+        if fused:
+            rc = lib.mep_dispatch_fresh(p(counts), p(mine), p(x), p(w), rank, S, H, K, E, R, tp, NvS, dst, cu, etc, zf, stats, dup,
+                                        p(shards), stride, p(slots), wstride, p(scratch), scratch.numel(), s)
+        else:
+            rc = lib.mep_plan_fresh(p(counts), p(mine), rank, S, K, E, R, tp, NvS, dst, cu, etc, zf, stats, dup, p(scratch),
+                                    scratch.numel(), None, 0, s)
+            _lib.check(rc, "mep_plan_fresh")
+            rc = lib.mep_dispatch(p(x), p(w), dst, zf, p(shards), stride, p(slots), wstride, rank, S, H, K, R, epn, NvS, tp,
+                                  _lib.DISPATCH_WRITE_DUPS, s)
+        _lib.check(rc, "dispatch")
+        got.append([*ints, shards.view(torch.int16), *([slots] if weights else [])])
+    torch.cuda.synchronize()
+    for i, (a, b) in enumerate(zip(*got)):
+        assert torch.equal(a, b), i
+    assert bool((got[1][6] != torch.tensor(7.0, dtype=torch.bfloat16).view(torch.int16).item()).any())
+
+
+def test_replayed_from_a_graph(cuda):
+    """No state is left between launches: replays give what an eager call gives."""
+    S, H, K, E, R, tp = 24, 1024, 8, 64, 8, 64
+    epn = E // R
+    NvS = -(-(S * K + (tp - 1) * 2 * epn) // tp) * tp
+    g = torch.Generator(device="cuda").manual_seed(3)
+    topk = torch.topk(torch.randn(R, S, E, device=cuda, generator=g), K, dim=-1)[1].to(torch.int32)
+    counts = torch.zeros(R, E, dtype=torch.int32, device=cuda)
+    counts.scatter_add_(1, topk.reshape(R, -1).long(), torch.ones(R, S * K, dtype=torch.int32, device=cuda))
+    mine, x = topk[2].contiguous(), torch.randn(S, H, device=cuda, generator=g).to(torch.bfloat16)
+    ints = [torch.empty(n, dtype=torch.int32, device=cuda) for n in (S * K, 2 * epn, E, 4 * epn, 2, 2)]
+    shards = torch.zeros(R, NvS, H, dtype=torch.bfloat16, device=cuda)
+    lib, p = _lib.lib(), _lib.ptr
+
+    def call():
+        _lib.check(lib.mep_dispatch_fresh(p(counts), p(mine), p(x), None, 2, S, H, K, E, R, tp, NvS, *map(p, ints), p(shards), NvS,
+                                          None, 0, None, 0, _lib.current_stream()), "mep_dispatch_fresh")
+
+    call()
+    torch.cuda.synchronize()
+    want = [t.clone() for t in (*ints, shards)]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    for _ in range(4):
+        for t in (*ints, shards):
+            t.fill_(5)
+        graph.replay()
+        torch.cuda.synchronize()
+        keep = want[-1] != 0
+        assert all(torch.equal(a, b) for a, b in zip(ints, want))
+        assert torch.equal(shards[keep], want[-1][keep])
+
+
+def test_argument_checks(cuda):
+    lib = _lib.lib()
+    assert lib.mep_dispatch_fresh(*([None] * 4), 0, 4, 64, 2, 8, 2, 8, 64, *([None] * 7), 0, None, 0, None, 0, None) == -1
