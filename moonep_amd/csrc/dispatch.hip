@@ -23,6 +23,7 @@ struct DispatchArgs {
   int64_t shard_stride_rows, wslot_stride;
   int rank, S, H, K, R, NvS, groups, tok_blocks, zblocks, zblocks_per_group;
   unsigned flags;
+  bool through;  // zeroes are written through
   // blockIdx.y is one of several ranks whose inputs lie behind each other; with `cu` ([2*epn] a
   // rank: padded ends of its groups) the slots behind the last group are zeroed like padding
   const int* cu;
@@ -104,8 +105,10 @@ __global__ __launch_bounds__(kBlock) void dispatch_kernel(DispatchArgs a) {
                ((uint64_t)rank * (uint64_t)a.shard_stride_rows + (uint64_t)pad_start) * row_bytes;
   const size_t region = (size_t)n_pad * row_bytes;              // a multiple of 16 (H % 8 == 0)
   const size_t step = (size_t)parts * kBlock * 16;
-  for (size_t off = ((size_t)zb * kBlock + threadIdx.x) * 16; off < region; off += step)
-    mep_st16_stream(base + off, zero);
+  for (size_t off = ((size_t)zb * kBlock + threadIdx.x) * 16; off < region; off += step) {
+    if (a.through) mep_st16_through(base + off, zero);
+    else mep_st16_stream(base + off, zero);
+  }
   if (a.w && zb == 0)
     for (int j = threadIdx.x; j < n_pad; j += kBlock)
       a.wslots[(size_t)rank * a.wslot_stride + pad_start + j] = 0.0f;
@@ -381,6 +384,7 @@ int dispatch_launch(const void* hidden, const float* w, const int32_t* dst, cons
   a.zblocks_per_group = zpg;
   const int zblocks = (zf && token_padding > 1) ? a.groups * zpg : 0;
   if (zblocks == 0) a.groups = 0;
+  a.through = mep_zero_through((int64_t)nranks * S * K, (int64_t)nranks * 2 * epn * (token_padding - 1), H);
   a.cu = cu;
   a.cu_len = 2 * epn;
   a.tail_blocks = cu ? 64 : 0;

@@ -200,4 +200,16 @@ __device__ __forceinline__ void mep_st16(void* p, mep_u4 v) {
   *(mep_u4*)p = v;
 }
 
+// Whether a dispatch zeroes padding rows with stores written through: where they are nearly all it
+// writes, and where there are few copies and more zeroes than the L2s hold.  Elsewhere the hint keeps
+// what the combine behind it reads and what the next call writes.  Both sides (hint -> through), us of
+// dispatch + combine: 8 tokens at H = 7168, K = 8, 32 groups 14.8 -> 13.8, 16 at 2880, K = 6, 48 groups
+// 12.3 -> 11.7, 100 at 4096 14.0 -> 14.3, 333 at 2880 17.6 -> 18.8; 512 at 7168, K = 8, 64 groups
+// 38.6 -> 36.7; 4096 at 7168 with a saved plan and three Buffers in turn 185 -> 193.  `padding`: the most
+// rows that there can be.
+static inline bool mep_zero_through(int64_t copies, int64_t padding, int64_t H) {
+  constexpr int64_t MiB = (int64_t)1 << 20;
+  return 16 * copies <= padding || (copies * H * 2 <= 64 * MiB && (copies + padding) * H * 2 > 96 * MiB);
+}
+
 #endif  // __HIPCC__

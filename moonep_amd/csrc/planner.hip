@@ -59,6 +59,8 @@ struct CopyArgs {
   float* wslots;
   int64_t shard_stride_rows, wslot_stride;
   int H;
+  int zero_from;  // first workgroup that zeroes padding
+  bool through;   // ... with stores written through
 };
 struct NoCopy {};
 
@@ -110,7 +112,7 @@ __global__ __launch_bounds__(NT) void plan_kernel(PlanArgs a, Copy copy) {
                         : a.scratch + (size_t)(blockIdx.y * a.groups + blockIdx.x) * 2 * E * R;
   int* alloc = tbl;            // [E,R] tokens of expert e landing on rank d
   int* base = tbl + E * R;     // [E,R] first slot of e on d, as an encoded dst
-  int* s_pad = base + E * R;   // COPY: [2*epn] first padding row, [2*epn] padding rows up to and with the group
+  int* s_pad = base + E * R;   // COPY: [2*epn] first padding row, [2*epn] padding rows, [2*epn] 4-KB pieces of them up to and with the group
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -485,8 +487,10 @@ __global__ __launch_bounds__(NT) void plan_kernel(PlanArgs a, Copy copy) {
       }
       if constexpr (COPY)
         if (d == rank) {
-          const int incl_pad = padding + mep_wave_incl_scan(padded - cnt);
-          if (g < 2 * epn) { s_pad[g] = start + cnt; s_pad[2 * epn + g] = incl_pad; }
+          // (bounded: counts that do not belong to the routing zero nothing outside the shard)
+          const int pad = (unsigned)(start + cnt) < (unsigned)NvS ? mep_imin(padded - cnt, NvS - start - cnt) : 0;
+          const int incl_pad = padding + mep_wave_incl_scan((int)(((uint64_t)pad * (uint64_t)copy.H * 2 + 4095) >> 12));
+          if (g < 2 * epn) { s_pad[g] = start + cnt; s_pad[2 * epn + g] = pad; s_pad[4 * epn + g] = incl_pad; }
           padding = __builtin_amdgcn_readlane(incl_pad, 63);
         }
       running += __builtin_amdgcn_readlane(incl, 63);
@@ -631,46 +635,38 @@ __global__ __launch_bounds__(NT) void plan_kernel(PlanArgs a, Copy copy) {
       for (int q = 0; q < 4; ++q)
         if (off + q * 1024 < row_bytes) mep_st16_stream(to + q * 1024, v[q]);
     }
-    // ---- this rank's padding rows (consecutive waves consecutive pieces) and their weight slots
+    // ---- this rank's padding rows (consecutive waves consecutive pieces) and their weight slots: by the
+    // workgroups without tokens where that is half of them (8 tokens at H = 4096: 10.9 -> 9.9 us, 8 at
+    // 7168 13.4 -> 12.1, 128 at 4096 9.7 -> 9.6)
     const mep_u4 zero = {0u, 0u, 0u, 0u};
     char* own = (char*)copy.shards + (uint64_t)rank * (uint64_t)copy.shard_stride_rows * row_bytes;
-    const int* upto = s_pad + 2 * epn;
-    const int rows = mep_imax(0, mep_imin(upto[2 * epn - 1], NvS));
-    // padding row r is row r + off of the shard in the group whose running count is the first beyond
-    // it; 128 groups two to a lane
-    int up[2], of[2];
+    const int* upto = s_pad + 4 * epn;
+    // 4-KB piece p lies in the first group whose running count is beyond it; 128 groups two to a lane
+    int up[2];
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const int g = 64 * c + lane;
-      up[c] = g < 2 * epn ? upto[g] : 0;
-      of[c] = g < 2 * epn ? s_pad[g] - (g > 0 ? upto[g - 1] : 0) : 0;
-    }
-    const int stride = gridDim.x * NW, dr = stride / pieces, dp = stride - dr * pieces;
-    int r = (int)(blockIdx.x * NW + wave) / pieces, piece = (int)(blockIdx.x * NW + wave) - r * pieces;
-    while (r < rows) {
-      int at = -1;
-      const uint64_t m0 = __ballot(up[0] > r), m1 = __ballot(up[1] > r);
-      if (m0) at = r + __builtin_amdgcn_readlane(of[0], __ffsll((unsigned long long)m0) - 1);
-      else if (m1) at = r + __builtin_amdgcn_readlane(of[1], __ffsll((unsigned long long)m1) - 1);
-      else
-        for (int g = 128; g < 2 * epn && at < 0; ++g)
-          if (upto[g] > r) at = s_pad[g] + r - upto[g - 1];
-      if ((unsigned)at < (unsigned)NvS) {
-        const size_t off = (size_t)piece * 4096 + lane * 16;
-        char* to = own + (size_t)at * row_bytes + off;
+    for (int c = 0; c < 2; ++c) up[c] = 64 * c + lane < 2 * epn ? upto[64 * c + lane] : 0;
+    const int z0 = copy.zero_from, npieces = upto[2 * epn - 1];
+    if ((int)blockIdx.x >= z0)
+      for (int p = ((int)blockIdx.x - z0) * NW + wave; p < npieces; p += ((int)gridDim.x - z0) * NW) {
+        const uint64_t m0 = __ballot(up[0] > p), m1 = __ballot(up[1] > p);
+        int g = m0 ? __ffsll((unsigned long long)m0) - 1 : 63 + __ffsll((unsigned long long)m1);
+        if (!(m0 | m1))
+          for (g = 128; upto[g] <= p;) ++g;
+        const int before = g > 0 ? upto[g - 1] : 0;
+        const uint64_t off = (uint64_t)(p - before) * 4096 + lane * 16, end = (uint64_t)s_pad[2 * epn + g] * row_bytes;
+        char* to = own + (uint64_t)s_pad[g] * row_bytes + off;
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-          if (off + q * 1024 < row_bytes) mep_st16_stream(to + q * 1024, zero);
+          if (off + q * 1024 < end) {
+            if (copy.through) mep_st16_through(to + q * 1024, zero);
+            else mep_st16_stream(to + q * 1024, zero);
+          }
       }
-      r += dr;
-      piece += dp;
-      if (piece >= pieces) { piece -= pieces; ++r; }
-    }
     if (copy.w)
-      for (int g = blockIdx.x; g < 2 * epn; g += gridDim.x) {
-        const int pad = upto[g] - (g > 0 ? upto[g - 1] : 0);
-        for (int j = tid; j < pad; j += NT)
-          if ((unsigned)(s_pad[g] + j) < (unsigned)NvS) copy.wslots[(size_t)rank * copy.wslot_stride + s_pad[g] + j] = 0.0f;
+      for (int g = (int)blockIdx.x - z0; g < 2 * epn; g += (int)gridDim.x - z0) {
+        if (g < 0) break;
+        for (int j = tid; j < s_pad[2 * epn + g]; j += NT)
+          copy.wslots[(size_t)rank * copy.wslot_stride + s_pad[g] + j] = 0.0f;
       }
   }
 }
@@ -742,25 +738,28 @@ namespace {
     else LAUNCH(0, 0);                             \
   } while (0)
 
-size_t plan_copy_lds_bytes(const PlanConfig& c, int epn) { return c.lds_bytes + 4 * (size_t)epn * sizeof(int); }
+size_t plan_copy_lds_bytes(const PlanConfig& c, int epn) { return c.lds_bytes + 6 * (size_t)epn * sizeof(int); }
 
 // Calls whose copies are no more than this plan and dispatch in one launch.  us, two launches -> one,
-// tokens in the cache (from HBM): 8 tokens at H = 4096, E = 128 11.1 -> 10.5 (10.4 -> 9.9), 512 at 7168, E = 256
-// 26.5 -> 24.2 (26.2 -> 24.3), 1024 at 4096 22.6 -> 21.3 (22.3 -> 21.4); above it the two meet: 1024 at 7168
+// tokens in the cache (from HBM): 8 tokens at H = 4096, E = 128 11.1 -> 9.3, 512 at 7168, E = 256
+// 26.5 -> 21.3, 1024 at 4096 22.6 -> 21.3 (22.3 -> 21.4); above it the two meet: 1024 at 7168
 // 33.1 -> 32.9 (33.0 -> 33.5), 2048 at 7168 56.8 -> 57.8 (57.1 -> 60.6).  The most padding, 8 tokens at 7168,
-// E = 256 (58 MB of it): 15.8 -> 15.8.  And the host has one launch less: Buffer.dispatch and combine of 8
+// E = 256 (58 MB of it): 15.8 -> 13.8.  And the host has one launch less: Buffer.dispatch and combine of 8
 // tokens 14.4 -> 13.0.
 constexpr int64_t kCopyMost = (int64_t)64 << 20;
 
-int plan_copy_launch(PlanArgs a, const CopyArgs& copy, const PlanConfig& c, hipStream_t st) {
+int plan_copy_launch(PlanArgs a, CopyArgs copy, const PlanConfig& c, hipStream_t st) {
   // a workgroup per CU where there are 16 KB for each, of as many tokens as it can resolve
   const int cus = mep_device_cu_count();
   if (cus <= 0) return MEP_ERR_INVALID_ARG;
-  const int64_t rows = (int64_t)a.S * a.K + (int64_t)2 * a.epn * (a.tp - 1);  // with the most padding
-  const int64_t want = (rows * copy.H * 2 + 16383) / 16384;
+  const int64_t copies = (int64_t)a.S * a.K, padding = (int64_t)2 * a.epn * (a.tp - 1);  // the most there can be
+  const int64_t want = ((copies + padding) * copy.H * 2 + 16383) / 16384;
   const int groups = (int)std::max<int64_t>(c.groups, std::min<int64_t>(want, cus));
   a.tok_per_wg = (a.S + groups - 1) / groups;
   a.groups = groups;
+  const int busy = (a.S + a.tok_per_wg - 1) / a.tok_per_wg;
+  copy.zero_from = 2 * busy <= groups ? busy : 0;
+  copy.through = mep_zero_through(copies, padding, copy.H);
   a.warm = nullptr;
   a.warm_vecs = 0;
   const size_t lds = plan_copy_lds_bytes(c, a.epn);
@@ -894,7 +893,7 @@ extern "C" int mep_dispatch_fresh(const int32_t* tpe_RE, const int32_t* topk_SK,
   PlanConfig c;
   if (S > 0 && K > 0 && K <= 32 && (int64_t)S * K * H * 2 <= kCopyMost && plan_config(S, K, E, R, &c) == MEP_OK &&
       c.nt == 1024 && plan_copy_lds_bytes(c, epn) <= kLdsDefaultLimit) {
-    const CopyArgs copy{(const uint16_t*)hidden_SH, w_SK, (uint16_t*)shards, wslots, shard_stride_rows, wslot_stride, H};
+    const CopyArgs copy{(const uint16_t*)hidden_SH, w_SK, (uint16_t*)shards, wslots, shard_stride_rows, wslot_stride, H, 0, false};
     return plan_launch(tpe_RE, topk_SK, rank, 1, S, K, E, R, token_padding, NvS, dst, cu_seqlens, experts_to_copy,
                        zero_fill, remote_stats, dup_counts, scratch, scratch_bytes, nullptr, 0, stream, &copy);
   }
