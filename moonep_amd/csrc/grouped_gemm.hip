@@ -317,8 +317,9 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_nt_kernel(GemmAr
 }
 
 // ---------------------------------------------------------------------------
-// The products of long groups and the weight gradient: 256 x 256 output tiles, K in steps of
-// 64, 8 waves of 128 x 64 (two on every SIMD), one workgroup per CU.
+// The weight gradient, and products of long groups of which few CUs get a tile (the others are
+// gemm_wide_kernel's): 256 x 256 output tiles, K in steps of 64, 8 waves of 128 x 64 (two on every
+// SIMD), one workgroup per CU.
 //
 // What bounds it: latency of the loads first (a step's 64 KB arrive 1.8 us after they were asked
 // for when the chip is busy, and its matrix instructions take 0.9), then the matrix cores at the
@@ -344,12 +345,13 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_nt_kernel(GemmAr
 // Groups end on multiples of 128 rows: a group of h 128-row blocks is h / 2 tiles and, if h is
 // odd, one of 128 rows whose second phase has no matrix instructions.
 //
-// Measured at 34 688 rows in 33 groups, H = 7168, H' = 2048 (us, before -> now; before: one
-// 256-row kernel with two LDS stages that drained its loads every step, wgrad likewise, dy * down
-// on 128 x 256 tiles): SwiGLU 2046 -> 1705, down 1150 -> 915, dy * down 1255 -> 894, dual
-// 2310 -> 1728, weight gradient 1555 -> 1314 (1.1 GB of fp32 zeroes for unused groups included);
-// 1.11 .. 1.19 PFLOP/s for the products that tile the rows, where the library's dense product of as
-// many rows reaches 1.32 at 2048 columns and 1.49 .. 1.52 at 4096.
+// Weight gradient at 34 688 rows in 33 groups, H = 7168, H' = 2048 (us, before -> now; before: one
+// 256-row kernel with two LDS stages that drained its loads every step): 1555 -> 1314 (1.1 GB of fp32
+// zeroes for unused groups included).  A step of it takes 1.9 us: 192 KB of transposing LDS reads, which
+// the LDS serves at half its rate, and 64 KB of loads into it.  gemm_wide_kernel reads 128 KB, but has
+// nothing beside its stores of fp32 and then meets the power limit: from equal (32 steps a tile) to
+// 15 % slower (8).  Stores of 16 bytes in pieces of 32, and waits that leave them in flight for the
+// first two steps of the next tile: 518 -> 550 at 33 792 rows, 4096 x 2048.
 //
 // LDS layouts.  Operand rows along K: 128 bytes per row and step, 16-byte vector q of row r at
 // position q ^ (r & 7) ^ ((r >> 3) & 1): sixteen consecutive lanes cover all banks.  Operands
