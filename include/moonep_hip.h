@@ -167,8 +167,8 @@ int mep_dispatch(const void* hidden_SH, const float* w_SK, const int32_t* dst,
 
 /*
  * mep_plan_fresh, with the tokens as what it warms the cache for, and mep_dispatch with
- * MEP_DISPATCH_WRITE_DUPS behind it.  A call that has few bytes to move runs as one kernel: the
- * planner's workgroups copy the rows.  Same results, bit for bit.
+ * MEP_DISPATCH_WRITE_DUPS behind it.  A call that has few bytes to move runs as one kernel, where
+ * the stream has the whole GPU: the planner's workgroups copy the rows.  Same results, bit for bit.
  */
 int mep_dispatch_fresh(const int32_t* tpe_RE, const int32_t* topk_SK, const void* hidden_SH,
                        const float* w_SK, int rank, int S, int H, int K, int E, int R,

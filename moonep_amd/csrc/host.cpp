@@ -302,7 +302,7 @@ PyObject* py_dispatch(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (w) w_out = w_zero_copy ? w_local : make(at::kFloat, {c.NvS});
     rc = as.begin({hidden, w, &out, &w_out, &plan.dst, &plan.etc, &plan.zfr, &plan.stats, &plan.dup_groups,
                    &plan.dup_loffs, &plan.dup_counts, topk, tpe, &cu});
-    if (rc == MEP_OK && fresh) {
+    if (rc == MEP_OK && fresh && !async) {
       what = "mep_dispatch_fresh";
       rc = mep_dispatch_fresh(ptr<int>(*tpe), ptr<int>(*topk), hidden->data_ptr(), w ? ptr<float>(*w) : nullptr, c.rank, c.S,
                               c.H, c.K, c.E, c.R, c.tp, c.NvS, ptr<int>(plan.dst), ptr<int>(cu), ptr<int>(plan.etc),
@@ -310,6 +310,16 @@ PyObject* py_dispatch(PyObject*, PyObject* const* args, Py_ssize_t n) {
                               c.hidden_buf.data_ptr(), c.NvS, w ? ptr<float>(c.meta_buf) : nullptr, c.wslot_stride,
                               ptr<void>(c.scratch), c.scratch.defined() ? c.scratch.nbytes() : 0, as.stream);
     } else if (rc == MEP_OK) {
+      // what is asynchronous runs beside kernels that hold CUs: two launches even of a small call
+      // (mep_dispatch_fresh has the figures)
+      what = "mep_plan";
+      if (fresh)
+        rc = mep_plan_fresh(ptr<int>(*tpe), ptr<int>(*topk), c.rank, c.S, c.K, c.E, c.R, c.tp, c.NvS,
+                            ptr<int>(plan.dst), ptr<int>(cu), ptr<int>(plan.etc), ptr<int>(plan.zfr),
+                            ptr<int>(plan.stats), ptr<int>(plan.dup_counts), ptr<void>(c.scratch),
+                            c.scratch.defined() ? c.scratch.nbytes() : 0, hidden->data_ptr(), hidden->nbytes(), as.stream);
+    }
+    if (rc == MEP_OK && !(fresh && !async)) {
       what = "mep_dispatch";
       rc = mep_dispatch(hidden->data_ptr(), w ? ptr<float>(*w) : nullptr, ptr<int>(plan.dst), ptr<int>(plan.zfr),
                         c.hidden_buf.data_ptr(), c.NvS, w ? ptr<float>(c.meta_buf) : nullptr, c.wslot_stride,

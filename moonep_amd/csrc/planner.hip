@@ -748,6 +748,20 @@ size_t plan_copy_lds_bytes(const PlanConfig& c, int epn) { return c.lds_bytes + 
 // tokens 14.4 -> 13.0.
 constexpr int64_t kCopyMost = (int64_t)64 << 20;
 
+// ... on a stream that has the whole GPU: a workgroup that starts when another has ended plans
+// once more.  8 tokens at H = 4096, 333 at 2880, us, one launch / two: on 32 CUs 50.3 / 16.7, 61.6 / 20.6, on 128 CUs
+// 15.3 / 14.9, 18.9 / 15.0, on 256 10.0 / 15.1, 11.8 / 14.7.  (The question takes 0.2 us of host time.)
+bool has_all_cus(hipStream_t st, int cus) {
+  uint32_t mask[32] = {};
+  if (hipExtStreamGetCUMask(st, 32, mask) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  int n = 0;
+  for (uint32_t m : mask) n += __builtin_popcount(m);
+  return n >= cus;
+}
+
 int plan_copy_launch(PlanArgs a, CopyArgs copy, const PlanConfig& c, hipStream_t st) {
   // a workgroup per CU where there are 16 KB for each, of as many tokens as it can resolve
   const int cus = mep_device_cu_count();
@@ -892,7 +906,7 @@ extern "C" int mep_dispatch_fresh(const int32_t* tpe_RE, const int32_t* topk_SK,
   const int epn = E / R;
   PlanConfig c;
   if (S > 0 && K > 0 && K <= 32 && (int64_t)S * K * H * 2 <= kCopyMost && plan_config(S, K, E, R, &c) == MEP_OK &&
-      c.nt == 1024 && plan_copy_lds_bytes(c, epn) <= kLdsDefaultLimit) {
+      c.nt == 1024 && plan_copy_lds_bytes(c, epn) <= kLdsDefaultLimit && has_all_cus((hipStream_t)stream, mep_device_cu_count())) {
     const CopyArgs copy{(const uint16_t*)hidden_SH, w_SK, (uint16_t*)shards, wslots, shard_stride_rows, wslot_stride, H, 0, false};
     return plan_launch(tpe_RE, topk_SK, rank, 1, S, K, E, R, token_padding, NvS, dst, cu_seqlens, experts_to_copy,
                        zero_fill, remote_stats, dup_counts, scratch, scratch_bytes, nullptr, 0, stream, &copy);

@@ -1,6 +1,8 @@
 """Plan and dispatch of a small call in one kernel against the two kernels one after the other: every
 output and every byte of the shards the same (plans, copies and zeroes: nothing is rounded)."""
 
+import ctypes
+
 import pytest
 import torch
 
@@ -97,6 +99,42 @@ def test_replayed_from_a_graph(cuda):
         keep = want[-1] != 0
         assert all(torch.equal(a, b) for a, b in zip(ints, want))
         assert torch.equal(shards[keep], want[-1][keep])
+
+
+def test_small_calls_beside_others_stay_two_launches(cuda):
+    """One kernel on a stream that has the whole GPU; on a part of the CUs, and asynchronously, two: each of its
+    workgroups plans, and there they run one after the other."""
+    from moonep_amd import Buffer, EmulatedWorld
+
+    S, H, K, E, R = 6, 512, 4, 32, 4
+    g = torch.Generator(device="cuda").manual_seed(5)
+    topk = torch.topk(torch.randn(S, E, device=cuda, generator=g), K, dim=-1)[1].to(torch.int32)
+    counts = torch.bincount(topk.flatten(), minlength=E).to(torch.int32).repeat(R, 1)
+    x = torch.randn(S, H, device=cuda, generator=g).to(torch.bfloat16)
+    limited = ctypes.c_void_p()
+    lib = _lib.lib()
+    _lib.check(lib.mep_stream_create_limited(32, ctypes.byref(limited)), "stream")
+    got = []
+    try:
+        for stream, wait in ((torch.cuda.current_stream(), False), (torch.cuda.ExternalStream(limited.value), False),
+                             (torch.cuda.current_stream(), True)):
+            world = EmulatedWorld(S, H, K, E, R, 64)
+            world.hidden_buf.zero_()
+            buf = Buffer(S, H, K, E, R, token_padding=64, rank=1, world=world)
+            torch.cuda.synchronize()
+            with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof, torch.cuda.stream(stream):
+                res = buf.dispatch(x, None, topk, counts, zero_copy=True, async_finish=wait)
+                torch.cuda.synchronize()
+            names = [e.key for e in prof.key_averages()]
+            assert any("CopyArgs" in n for n in names) == (not got)
+            assert any("dispatch_kernel" in n for n in names) == bool(got)
+            got.append((world.hidden_buf.clone(), res[2].clone(), res[3].dst.clone()))
+            del res, buf
+    finally:
+        torch.cuda.synchronize()
+        _lib.check(lib.mep_stream_destroy(limited), "stream")
+    for other in got[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(got[0], other))
 
 
 def test_argument_checks(cuda):
