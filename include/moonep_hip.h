@@ -169,6 +169,8 @@ int mep_dispatch(const void* hidden_SH, const float* w_SK, const int32_t* dst,
  * mep_plan_fresh, with the tokens as what it warms the cache for, and mep_dispatch with
  * MEP_DISPATCH_WRITE_DUPS behind it.  A call that has few bytes to move runs as one kernel, where
  * the stream has the whole GPU: the planner's workgroups copy the rows.  Same results, bit for bit.
+ * (That kernel waits for room on up to 128 CUs.  While another stream's kernels hold more, or all, as a
+ * large matrix product does, mep_plan_fresh and mep_dispatch, which need fewer, may be through earlier.)
  */
 int mep_dispatch_fresh(const int32_t* tpe_RE, const int32_t* topk_SK, const void* hidden_SH,
                        const float* w_SK, int rank, int S, int H, int K, int E, int R,

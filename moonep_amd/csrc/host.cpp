@@ -310,8 +310,8 @@ PyObject* py_dispatch(PyObject*, PyObject* const* args, Py_ssize_t n) {
                               c.hidden_buf.data_ptr(), c.NvS, w ? ptr<float>(c.meta_buf) : nullptr, c.wslot_stride,
                               ptr<void>(c.scratch), c.scratch.defined() ? c.scratch.nbytes() : 0, as.stream);
     } else if (rc == MEP_OK) {
-      // what is asynchronous runs beside kernels that hold CUs: two launches even of a small call
-      // (mep_dispatch_fresh has the figures)
+      // what is asynchronous runs beside kernels that hold CUs, GEMMs all of them: two launches even of a
+      // small call (has_all_cus in planner.hip has the figures)
       what = "mep_plan";
       if (fresh)
         rc = mep_plan_fresh(ptr<int>(*tpe), ptr<int>(*topk), c.rank, c.S, c.K, c.E, c.R, c.tp, c.NvS,

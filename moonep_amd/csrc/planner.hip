@@ -63,6 +63,14 @@ struct CopyArgs {
   bool through;   // ... with stores written through
 };
 struct NoCopy {};
+static_assert(sizeof(PlanArgs) % alignof(CopyArgs) == 0, "late_args<CopyArgs> reads right behind them");
+// Two planning and copying workgroups fit on a CU: 64 vector and 80 scalar registers, 64 KB of LDS.
+// Beside kernels that hold CUs none of them then waits for another to end, which would plan once
+// more.  us on a stream that has the whole GPU while 32 CUs run another stream's combine, one to a CU -> two
+// / planner and dispatch as two launches: 8 tokens at H = 4096 15.2 -> 10.4 / 13.0, 333 at 2880 13.3 -> 10.8 / 16.8,
+// 512 at 7168 32.0 -> 26.5 / 29.9, 1024 at 4096 31.6 -> 26.7 / 28.0.
+template <class Copy>
+constexpr int kPlanWavesPerSimd = std::is_same_v<Copy, NoCopy> ? 1 : 8;
 
 // LDS layout in ints (must match plan_lds_bytes on the host)
 template <int NT>
@@ -74,6 +82,15 @@ struct PlanLds {
   static constexpr int FIXED = NT;
 };
 
+// Kernel arguments read again where they are used: what is used last would sit in scalar registers
+// through all of the plan, and a wave of a workgroup that shares its CU has 80 of them.
+template <class T>
+__device__ __forceinline__ T late_args(size_t offset) {
+  auto args = (const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr() + offset;
+  asm volatile("" : "+s"(args));
+  return *(const T*)(const char*)args;
+}
+
 // COPY: plan and dispatch of a call with few bytes to move, in one launch.  Apart they are two
 // chains of latencies behind each other (8 tokens at H = 4096: planner 5.7 us, dispatch 5.7 us, of
 // which 3 are 16 MB of padding rows zeroed, and the host's second launch); the plan is in every
@@ -84,13 +101,14 @@ struct PlanLds {
 // from the arguments); the planner is a chain of dependent instructions, and
 // a kernel that knows them drops the loops, clamps and alternative paths
 template <int NT, bool kLdsTables, int RC = 0, int KC = 0, class Copy = NoCopy>
-__global__ __launch_bounds__(NT) void plan_kernel(PlanArgs a, Copy copy) {
+__global__ __launch_bounds__(NT, kPlanWavesPerSimd<Copy>) void plan_kernel(PlanArgs a, Copy copy) {
   constexpr bool COPY = !std::is_same_v<Copy, NoCopy>;
   static_assert(!COPY || kLdsTables, "small calls only");
   using L = PlanLds<NT>;
   constexpr int NW = L::NW;
   constexpr int W4 = L::W4;
   extern __shared__ int smem[];
+  const int by = COPY ? 0 : blockIdx.y;  // rank of those planned
   const int E = a.E, R = RC > 0 ? RC : a.R, epn = a.epn, tp = a.tp, NvS = a.NvS, K = KC > 0 ? KC : a.K;
   const int N = a.S * K;
   const int CAP = N;
@@ -109,7 +127,7 @@ __global__ __launch_bounds__(NT) void plan_kernel(PlanArgs a, Copy copy) {
   int* s_bal = s_nrem + R;       // [R] word 0: where counts of invalid expert ids go
   int* s_cd = s_bal + R;         // [NT] destination rank of each entry
   int* tbl = kLdsTables ? (s_cd + NT)
-                        : a.scratch + (size_t)(blockIdx.y * a.groups + blockIdx.x) * 2 * E * R;
+                        : a.scratch + (size_t)(by * a.groups + blockIdx.x) * 2 * E * R;
   int* alloc = tbl;            // [E,R] tokens of expert e landing on rank d
   int* base = tbl + E * R;     // [E,R] first slot of e on d, as an encoded dst
   int* s_pad = base + E * R;   // COPY: [2*epn] first padding row, [2*epn] padding rows, [2*epn] 4-KB pieces of them up to and with the group
@@ -117,10 +135,10 @@ __global__ __launch_bounds__(NT) void plan_kernel(PlanArgs a, Copy copy) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: roles branch on scalars
-  if ((int)blockIdx.x >= a.groups) {
+  if (!COPY && (int)blockIdx.x >= a.groups) {
     // cache warmer: plain 16-byte loads, eight in flight.  The values only feed
     // a comparison that guards a sleep, so the loads stay and nothing is written.
-    if (blockIdx.y != 0 || a.warm_vecs == 0) return;
+    if (by != 0 || a.warm_vecs == 0) return;
     const size_t nthreads = (size_t)(gridDim.x - a.groups) * NT;
     const size_t first = (size_t)(blockIdx.x - a.groups) * NT + tid;
     const mep_u4* w = (const mep_u4*)a.warm;
@@ -138,9 +156,9 @@ __global__ __launch_bounds__(NT) void plan_kernel(PlanArgs a, Copy copy) {
     if ((x[0] ^ x[1]) == 0x9e3779b9u && (x[2] ^ x[3]) == 0x7f4a7c15u) __builtin_amdgcn_s_sleep(1);
     return;
   }
-  const int rank = a.rank0 + blockIdx.y;
+  const int rank = a.rank0 + by;
   const bool writer = blockIdx.x == 0;  // one workgroup per rank stores the small outputs
-  const int* topk = a.topk + (size_t)blockIdx.y * N;
+  const int* topk = a.topk + (size_t)by * N;
   const int t0 = COPY ? min((int)blockIdx.x * a.tok_per_wg, a.S) : blockIdx.x * a.tok_per_wg;
   const int t1 = min(t0 + a.tok_per_wg, a.S);
   const int e0 = t0 * K;
@@ -212,18 +230,18 @@ __global__ __launch_bounds__(NT) void plan_kernel(PlanArgs a, Copy copy) {
   };
   int4 ha[4], hb[6], hc[6];
   if (count_a) hist_load(ha, v0, hb1, ta, NA);
-  // COPY, several tokens a workgroup: the first 128 KB of them are on their way into its L2 meanwhile
-  // (tokens that come from HBM, 1024 at H = 4096: 23.1 -> 21.4 us; where there is one it costs 0.4 us)
-  constexpr int WARM = COPY ? 8 : 1;
-  mep_u4 warm[WARM];
-  int warm_vecs = 0;
+  // COPY, several tokens a workgroup: these are on their way into its L2 meanwhile, a word of every 32 bytes
+  // of the first 64 KB (one of every 64 of 128 KB where no token is read twice).  Tokens that come from HBM,
+  // never -> so: 1024 at H = 4096 23.1 -> 21.7 us; where there is one token it costs 0.4 us.  16-byte loads, which
+  // hold eight registers instead of two through the plan, are no faster (22.1); reading 128 KB where
+  // tokens are read twice (4096 at 4096, K = 2) takes 23.8 instead of 21.5.
+  int warm[2] = {};
   if constexpr (COPY) {
-    if (a.tok_per_wg > 1) {
-      warm_vecs = (t1 - t0) * (copy.H / 8);
-      const mep_u4* rows = (const mep_u4*)copy.hidden + (size_t)t0 * (copy.H / 8);
+    const char* rows = (const char*)copy.hidden + (size_t)t0 * copy.H * 2;
 #pragma unroll
-      for (int u = 0; u < WARM; ++u)
-        if (tid + u * NT < warm_vecs) warm[u] = rows[tid + u * NT];
+    for (int u = 0; u < 2; ++u) {
+      const int word = (u * NT + tid) * (K == 1 ? 64 : 32);
+      if (a.tok_per_wg > 1 && word < (t1 - t0) * copy.H * 2) warm[u] = *(const int*)(rows + word);
     }
   }
 
@@ -439,6 +457,11 @@ __global__ __launch_bounds__(NT) void plan_kernel(PlanArgs a, Copy copy) {
 
   // ---- layout of every destination: one wave per destination -------------
   if (count_b && spread) hist_part(hc, hb2, v1, tb, NB);
+  auto outputs = [&] {
+    if constexpr (COPY) return late_args<PlanArgs>(0);
+    else return a;
+  };
+  const PlanArgs to = outputs();
   const bool tp_pow2 = (tp & (tp - 1)) == 0;
   for (int d = (wave + NW - 1) % NW; d < R; d += NW) {
     const int lo = d * epn;
@@ -463,11 +486,11 @@ __global__ __launch_bounds__(NT) void plan_kernel(PlanArgs a, Copy copy) {
     for (int b = nremote + lane; b < epn; b += 64) s_etc[lo + b] = -1;
     if (lane == 0) s_nrem[d] = nremote;
     mep_wave_sync();
-    if (writer && blockIdx.y == 0)
-      for (int b = lane; b < epn; b += 64) a.etc[lo + b] = s_etc[lo + b];
+    if (writer && by == 0)
+      for (int b = lane; b < epn; b += 64) to.etc[lo + b] = s_etc[lo + b];
     const bool mine = writer && d == rank;
-    int* cu = a.cu_seqlens + (size_t)blockIdx.y * 2 * epn;
-    int* zf = a.zero_fill + (size_t)blockIdx.y * 4 * epn;
+    int* cu = to.cu_seqlens + (size_t)by * 2 * epn;
+    int* zf = to.zero_fill + (size_t)by * 4 * epn;
     int running = 0, padding = 0;
     for (int c = 0; c < 2 * epn; c += 64) {
       const int g = c + lane;
@@ -502,7 +525,7 @@ __global__ __launch_bounds__(NT) void plan_kernel(PlanArgs a, Copy copy) {
   // An entry with an invalid expert id gets destination rank R: dispatch and
   // combine skip such entries (they never write or read outside the R shards),
   // the duplicate-group builder matches no rank to it.
-  int* dst = a.dst + (size_t)blockIdx.y * N;
+  int* dst = outputs().dst + (size_t)by * N;
   int dv = R * NvS, dest = -1;  // fits: the host requires R*NvS <= INT32_MAX
   if (e >= 0) {
     // entries of my expert in the waves before mine: one byte per wave, W4 words
@@ -597,19 +620,16 @@ __global__ __launch_bounds__(NT) void plan_kernel(PlanArgs a, Copy copy) {
   }
   if (tid < n) dst[e0 + tid] = dup ? -dv - 1 : dv;
   if (writer && tid == 0) {
-    a.remote_stats[2 * blockIdx.y] = s_nrem[rank];
-    a.remote_stats[2 * blockIdx.y + 1] = s_stat1[rank];
-    if (a.dup_counts) { a.dup_counts[0] = 0; a.dup_counts[1] = 0; }
+    const PlanArgs to = outputs();
+    to.remote_stats[2 * by] = s_nrem[rank];
+    to.remote_stats[2 * by + 1] = s_stat1[rank];
+    if (to.dup_counts) { to.dup_counts[0] = 0; to.dup_counts[1] = 0; }
   }
   if constexpr (COPY) {
+    const CopyArgs copy = late_args<CopyArgs>(sizeof(PlanArgs));
     const size_t row_bytes = (size_t)copy.H * 2;
-    if (warm_vecs > 0) {  // a comparison that guards a sleep keeps those loads
-      mep_u4 x = {0u, 0u, 0u, 0u};
 #pragma unroll
-      for (int u = 0; u < WARM; ++u)
-        if (tid + u * NT < warm_vecs) x ^= warm[u];
-      if ((x[0] ^ x[1]) == 0x9e3779b9u && (x[2] ^ x[3]) == 0x7f4a7c15u) __builtin_amdgcn_s_sleep(1);
-    }
+    for (int u = 0; u < 2; ++u) asm volatile("" : : "v"(warm[u]));  // keeps those loads, and waits for them here
     // ---- the rows and weights of this workgroup's entries
     if (16 % K != 0) __syncthreads();  // s_cd has been read
     s_cd[tid] = dv;
@@ -749,8 +769,12 @@ size_t plan_copy_lds_bytes(const PlanConfig& c, int epn) { return c.lds_bytes + 
 constexpr int64_t kCopyMost = (int64_t)64 << 20;
 
 // ... on a stream that has the whole GPU: a workgroup that starts when another has ended plans
-// once more.  8 tokens at H = 4096, 333 at 2880, us, one launch / two: on 32 CUs 50.3 / 16.7, 61.6 / 20.6, on 128 CUs
-// 15.3 / 14.9, 18.9 / 15.0, on 256 10.0 / 15.1, 11.8 / 14.7.  (The question takes 0.2 us of host time.)
+// once more.  8 tokens at H = 4096, 333 at 2880, us, one launch / two: on 32 CUs 31.6 / 16.1, 37.8 / 19.7, on 64
+// 17.3 / 12.4, 20.2 / 14.3, on 128, where two workgroups share a CU, 9.9 / 10.7, 12.4 / 12.3, on 256 9.1 / 10.9,
+// 10.0 / 11.1.  Beside kernels of other streams nothing is asked.  32 CUs held: kPlanWavesPerSimd.  All of them held
+// by GEMMs whose workgroups fill a CU, 8 to 1024 tokens: either way a call takes the 190 to 210 us until some
+// have ended, but on one pair of queues in three one launch of 8 tokens 260 to 290.  (The question takes 0.2 us
+// of host time.)
 bool has_all_cus(hipStream_t st, int cus) {
   uint32_t mask[32] = {};
   if (hipExtStreamGetCUMask(st, 32, mask) != hipSuccess) {
