@@ -14,11 +14,12 @@ pytestmark = pytest.mark.gpu
 # S, H, K, E, R, rank, token_padding: one token and more tokens than CUs, rows of 16 bytes and of no whole KB,
 # every compile-time number of ranks and others, more than 64 and more than 128 groups, no padding, padding that is
 # written through and not (workgroups without tokens, few copies beside much of it), both sides of the largest call
-# that is one kernel (64 MiB of copies)
+# that is one kernel (64 MiB of copies), and that call of many short rows and of one copy a token
 CASES = [(1, 8, 1, 1, 1, 0, 1), (3, 24, 2, 8, 2, 1, 16), (8, 4096, 8, 128, 8, 4, 128), (33, 520, 6, 96, 4, 3, 64),
          (300, 2880, 8, 64, 4, 0, 7), (257, 1032, 8, 64, 16, 15, 128), (700, 512, 4, 96, 24, 11, 16), (90, 640, 3, 160, 2, 1, 32),
          (64, 256, 5, 60, 3, 2, 128), (1024, 256, 2, 16, 8, 7, 128), (1100, 64, 32, 128, 8, 3, 64), (40, 7168, 8, 288, 2, 0, 128),
-         (600, 6144, 8, 256, 8, 2, 128), (1024, 4096, 8, 128, 8, 1, 128), (1025, 4096, 8, 128, 8, 1, 128)]
+         (600, 6144, 8, 256, 8, 2, 128), (1024, 4096, 8, 128, 8, 1, 128), (1025, 4096, 8, 128, 8, 1, 128), (8192, 512, 8, 128, 8, 3, 128), (16000, 256, 8, 64, 8, 5, 128),
+         (5000, 4096, 1, 32, 2, 0, 16)]
 
 
 @pytest.mark.parametrize("weights", [True, False])
