@@ -114,22 +114,29 @@ def _follow(name, body, labels, start):
     return faults
 
 
-def _accumulators(name, body):
+def _accumulators(name, body, labels):
     """Faults around matrix instructions in asm statements."""
-    faults = []
     if not any(ins.in_asm and ins.op.startswith("v_mfma") for ins in body):
-        return faults
-    waited = []     # the registers that VALU instructions wrote in the last two issue slots
-    for ins in body:
+        return []
+    faults = {}
+    for i, ins in enumerate(body):
         if not ins.in_asm and _ACC.search(ins.text):
-            faults.append(f"{name}: line {ins.line}: `{ins.text}` touches an accumulation register")
-        if ins.op.startswith("v_mfma") and any(ins.regs & regs for regs in waited):
-            faults.append(f"{name}: line {ins.line}: `{ins.text}` too early after the VALU write of an operand")
-        slots = int(ins.text.split()[1]) + 1 if ins.op == "s_nop" else 0 if ins.arrived else 1
-        valu = ins.op.startswith("v_") and not ins.op.startswith("v_mfma")
-        written = _registers(ins.text.split(",")[0]) if valu else set()
-        waited = ([*waited, written] + [set()] * (slots - 1))[-2:] if slots else waited
-    return faults
+            faults[i] = "touches an accumulation register"
+        if not ins.op.startswith("v_") or ins.op.startswith("v_mfma"):
+            continue
+        # a VALU write: two issue slots on every way from it, around loops too, before its register is an operand
+        written = _registers(ins.text.split(",")[0])
+        todo = [(at, 0) for at in _successors(body, labels, i)] if written else []
+        while todo:
+            at, slots = todo.pop()
+            if slots >= 2 or at >= len(body):
+                continue
+            after = body[at]
+            if after.op.startswith("v_mfma") and after.regs & written:
+                faults[at] = "too early after the VALU write of an operand"
+            slots += int(after.text.split()[1]) + 1 if after.op == "s_nop" else 0 if after.arrived else 1
+            todo.extend((n, slots) for n in _successors(body, labels, at))
+    return [f"{name}: line {body[i].line}: `{body[i].text}` {what}" for i, what in sorted(faults.items())]
 
 
 def check(assembly, kernels=("gemm_",)):
@@ -138,7 +145,7 @@ def check(assembly, kernels=("gemm_",)):
     for name, (body, labels) in functions(assembly).items():
         if not any(k in name for k in kernels):
             continue
-        faults += _accumulators(name, body)
+        faults += _accumulators(name, body, labels)
         for i, ins in enumerate(body):
             if ins.in_asm and (ins.op.startswith("ds_read") or ins.vmem) and not ins.text.endswith(" lds"):
                 followed += 1
