@@ -5,6 +5,8 @@ Sizes leave more than a quarter of the CUs a tile (below that another kernel run
 operands, fp32 sums, one rounding to bf16 (2^-9 relative): 5e-3 in the 2-norm of every 128-row block; the
 activation of a SwiGLU rounds once, too."""
 
+import ctypes
+
 import pytest
 import torch
 
@@ -75,3 +77,60 @@ def test_products(cuda, form, heights, K):
         beg = end
     for out in outs:
         assert (out[beg:] == 7.0).all()
+
+
+# row blocks of each rank's groups: ends that differ between the ranks, empty groups first, last and side by side,
+# more groups in all than a wave has lanes
+RANKS = {"three": ((3, 0, 5, 2, 0, 1), (0, 0, 1, 1, 9, 4), (7, 2, 1, 0, 0, 0)),
+         "ten": tuple(tuple((r + 3 * i) % 5 % 3 for i in range(8)) for r in range(10))}
+
+
+@pytest.mark.parametrize("slots", [True, False])
+@pytest.mark.parametrize("ranks,H,Hp", [("three", 2048, 1792), ("ten", 1024, 2304)])
+def test_groups_of_several_ranks(cuda, ranks, H, Hp, slots):
+    """The row-tiled products of an FFN's forward and backward pass of all ranks of a group: SwiGLU with saved
+    pre-activations, down (scaled and plain), dy * down and the two pairs with [K, N] weights."""
+    heights = RANKS[ranks]
+    n, G, M = len(heights), len(heights[0]), 128 * (max(map(sum, heights)) + 1)
+    print(f"{n} ranks H={H} Hp={Hp} M={M} slots={slots}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n)
+
+    def normal(*shape, scale=1.0):
+        return (torch.randn(*shape, device=cuda, generator=g) * scale).to(torch.bfloat16)
+
+    rows, dy = normal(n, M, H), normal(n, M, H)
+    gate, up, down = normal(n, G, Hp, H, scale=H ** -0.5), normal(n, G, Hp, H, scale=H ** -0.5), normal(n, G, H, Hp, scale=Hp ** -0.5)
+    cu = torch.tensor([[128 * sum(h[:i + 1]) for i in range(G)] for h in heights], dtype=torch.int32, device=cuda)
+    scale = torch.rand(n, M, device=cuda, generator=g) + 0.1 if slots else None
+    act, gate_pre, up_pre, dh, dgate, dup, hs = (torch.full((n, M, Hp), 7.0, dtype=torch.bfloat16, device=cuda) for _ in range(7))
+    y, drows = (torch.full((n, M, H), 7.0, dtype=torch.bfloat16, device=cuda) for _ in range(2))
+    dslots = torch.empty(n, M, device=cuda) if slots else None
+    split = G // 2
+    grads = [[torch.empty(n, s, *shape, device=cuda) for shape in ((Hp, H), (Hp, H), (H, Hp))] for s in (split, G - split)]
+    lib, p, s = _lib.lib(), _lib.ptr, _lib.current_stream()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        _lib.check(lib.mep_ffn_forward(p(rows), p(scale), p(cu), G, p(gate), p(up), p(down), p(act), p(gate_pre), p(up_pre), p(y),
+                                       n, M, H, Hp, s), "mep_ffn_forward")
+        _lib.check(lib.mep_ffn_backward(p(dy), p(rows), p(scale), p(cu), G, p(gate), p(up), p(down), p(gate_pre), p(up_pre), p(dh),
+                                        p(dgate), p(dup), p(hs), p(dslots), p(drows), *((ctypes.c_void_p * 3)(*map(p, t)) for t in grads),
+                                        split, n, M, H, Hp, G, s), "mep_ffn_backward")
+        torch.cuda.synchronize()
+    assert sum(e.count for e in prof.key_averages() if "gemm_wide_kernel" in e.key) == 4
+    for r in range(n):
+        ends = cu[r].tolist()
+        for i, end in enumerate(ends):
+            beg = ends[i - 1] if i else 0
+            t = slice(beg, end)
+            if end == beg:
+                continue
+            x = rows[r, t].float()
+            one, two = x @ gate[r, i].float().t(), x @ up[r, i].float().t()
+            by = scale[r, t, None] if slots else 1.0
+            checks = [(gate_pre, one), (up_pre, two), (act, torch.nn.functional.silu(one) * two),
+                      (y, act[r, t].float() @ down[r, i].float().t() * by), (dh, dy[r, t].float() @ down[r, i].float()),
+                      (drows, dgate[r, t].float() @ gate[r, i].float() + dup[r, t].float() @ up[r, i].float())]
+            for k, (out, want) in enumerate(checks):
+                d, norm = (v.view((end - beg) // 128, 128, -1, 64).square().sum((1, 3)).sqrt() for v in (out[r, t].float() - want, want))
+                assert float((d / norm).max()) < 1e-2, (r, i, k)
+        assert not y[r, ends[-1]:].any() and not drows[r, ends[-1]:].any()
+        assert (act[r, ends[-1]:] == 7.0).all() and (dh[r, ends[-1]:] == 7.0).all()
