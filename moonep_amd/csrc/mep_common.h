@@ -203,10 +203,13 @@ __device__ __forceinline__ void mep_st16(void* p, mep_u4 v) {
 // Whether a dispatch zeroes padding rows with stores written through: where they are nearly all it
 // writes, and where there are few copies and more zeroes than the L2s hold.  Elsewhere the hint keeps
 // what the combine behind it reads and what the next call writes.  Both sides (hint -> through), us of
-// dispatch + combine: 8 tokens at H = 7168, K = 8, 32 groups 14.8 -> 13.8, 16 at 2880, K = 6, 48 groups
-// 12.3 -> 11.7, 100 at 4096 14.0 -> 14.3, 333 at 2880 17.6 -> 18.8; 512 at 7168, K = 8, 64 groups
-// 38.6 -> 36.7; 4096 at 7168 with a saved plan and three Buffers in turn 185 -> 193.  `padding`: the most
-// rows that there can be.
+// dispatch + combine behind 800 MB of weights / on the same shards again / on as many shards in turn as push each other's
+// zeroes out of the last-level cache.  Planned in the same launch: 1 token at H = 4096, K = 8, 32 groups
+// 15.4 -> 14.9 / 10.9 -> 10.7 / 11.3 -> 11.0, 8 16.8 -> 16.7 / 12.2 -> 12.4 / 12.1 -> 13.1, 40 at 2880, K = 6, 96 groups
+// 18.9 -> 18.0 / 15.6 -> 14.8 / 15.7 -> 16.2, 64 at 7168, K = 8, 64 groups 25.4 -> 23.6 / 22.2 -> 21.4 / 22.0 -> 22.5, 512
+// 41.5 -> 38.2 / 38.5 -> 36.2 / 39.4 -> 35.9; kept out: 100 at 4096 13.8 -> 15.2 / 13.3 -> 15.3 (same, in turn).  With
+// a saved plan: 64 at 7168 20.7 -> 19.2 / 16.1 -> 15.8 / 15.8 -> 18.4, 512 39.3 -> 38.1; kept out: 4096 at 7168 with three
+// Buffers in turn 185 -> 193.  `padding`: the most rows that there can be.
 static inline bool mep_zero_through(int64_t copies, int64_t padding, int64_t H) {
   constexpr int64_t MiB = (int64_t)1 << 20;
   return 16 * copies <= padding || (copies * H * 2 <= 64 * MiB && (copies + padding) * H * 2 > 96 * MiB);

@@ -230,18 +230,19 @@ __global__ __launch_bounds__(NT, kPlanWavesPerSimd<Copy>) void plan_kernel(PlanA
   };
   int4 ha[4], hb[6], hc[6];
   if (count_a) hist_load(ha, v0, hb1, ta, NA);
-  // COPY, several tokens a workgroup: these are on their way into its L2 meanwhile, a word of every 32 bytes
-  // of the first 64 KB (one of every 64 of 128 KB where no token is read twice).  Tokens that come from HBM,
-  // never -> so: 1024 at H = 4096 23.1 -> 21.7 us; where there is one token it costs 0.4 us.  16-byte loads, which
-  // hold eight registers instead of two through the plan, are no faster (22.1); reading 128 KB where
-  // tokens are read twice (4096 at 4096, K = 2) takes 23.8 instead of 21.5.
+  // COPY: the workgroup's tokens are on their way into its L2 meanwhile, a word of every 32 bytes of the first
+  // 64 KB (one of every 64 of 128 KB where no token is read twice).  Tokens that come from HBM, never -> so:
+  // 1 at H = 4096 behind 800 MB of weights 11.5 -> 10.6 us, 33 13.5 -> 12.3, 1 at 7168 13.9 -> 12.4, 1024 at 4096 over eight
+  // Buffers in turn 23.1 -> 21.7; tokens in the cache +-0.1.  16-byte loads, which hold eight registers
+  // instead of two through the plan, are no faster (22.1); reading 128 KB where tokens are read twice (4096
+  // at 4096, K = 2) takes 23.8 instead of 21.5.
   int warm[2] = {};
   if constexpr (COPY) {
     const char* rows = (const char*)copy.hidden + (size_t)t0 * copy.H * 2;
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int word = (u * NT + tid) * (K == 1 ? 64 : 32);
-      if (a.tok_per_wg > 1 && word < (t1 - t0) * copy.H * 2) warm[u] = *(const int*)(rows + word);
+      if (word < (t1 - t0) * copy.H * 2) warm[u] = *(const int*)(rows + word);
     }
   }
 
