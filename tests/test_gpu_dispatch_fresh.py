@@ -104,7 +104,7 @@ def test_replayed_from_a_graph(cuda):
 
 def test_small_calls_beside_others_stay_two_launches(cuda):
     """One kernel on a stream that has the whole GPU; on a part of the CUs, and asynchronously, two: each of its
-    workgroups plans, and there they run one after the other."""
+    workgroups plans, and one that has to wait for room on a CU does so late."""
     from moonep_amd import Buffer, EmulatedWorld
 
     S, H, K, E, R = 6, 512, 4, 32, 4
