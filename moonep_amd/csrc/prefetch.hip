@@ -106,24 +106,6 @@ __host__ __device__ inline int slot_table_ints(int R, int epn) { return 2 * R * 
 
 size_t slot_table_bytes(int R, int epn) { return (size_t)slot_table_ints(R, epn) * sizeof(int); }
 
-// Grid of the reduction: persistent workgroups, each moving a 16 KiB tile per
-// step.  Each workgroup pays the table set-up, which dominates when only a few
-// experts are hosted remotely -- the common case; `cap` bounds their number.
-// The number of active experts is only known on the device, so the grid is
-// sized from the tiles of ONE expert: with `tiles` (or an even fraction of
-// them) workgroups every workgroup moves the same number of tiles whatever that
-// number is; small tensors spread over up to `epn` experts' tiles.
-int stream_blocks(int64_t tiles, int R, int epn, int64_t cap) {
-  if ((int64_t)R * epn > 1024 && cap > 2048) cap = 2048;  // large tables: set-up costs more
-  if (tiles <= 0) return 1;
-  if (8 * tiles > cap) {
-    const int64_t per_block = (tiles + cap - 1) / cap;  // tiles of an expert per workgroup
-    return (int)((tiles + per_block - 1) / per_block);
-  }
-  const int64_t all = tiles * epn;
-  return (int)(all < cap ? all : cap / tiles * tiles);
-}
-
 // Tile layout of both kernels.  A tile is 256 threads x 4 vectors of 16 bytes.
 // Where an expert's matrix allows it the four vectors of a thread lie 32 KiB
 // apart and eight tiles interleave in a 128 KiB block: a wave's consecutive
@@ -574,7 +556,7 @@ __device__ __forceinline__ void clear_tile(const ReduceArgs& a, const SpreadTile
 //    workgroups beside the summing ones are as fast but the host cannot know
 //    how many to launch.)
 __device__ __forceinline__ void reduce_tensor(const ReduceArgs& a, const SlotTable& t, const int* occ, int64_t* sbase,
-                                              int n_active, int n_clear) {
+                                              int n_active, int n_clear, int64_t before) {
   const SpreadTiles rt(a.elems * 4);
   const bool clear_as_read = a.flags == 0;  // own slots holding own experts, zeroed by their reader
   // where each entry of the slot lists starts in the pool, so that a tile only adds its offset
@@ -605,19 +587,28 @@ __device__ __forceinline__ void reduce_tensor(const ReduceArgs& a, const SlotTab
     for (int64_t p = blockIdx.x; p < pieces; p += gridDim.x) fill(p, p + 1);
     return;
   }
-  // With pieces to fill between the tiles one workgroup per CU is the faster shape (6.0 against
-  // 5.8 TB/s on a table with 8 slots per rank), without them two per CU (6.4 against 6.0): the
-  // upper half of the grid leaves when there is something to fill.
-  const int nwg = pieces > 0 ? (int)((gridDim.x + 1) / 2) : (int)gridDim.x;
+  // With pieces to fill between the tiles a long stream is faster with one workgroup per CU (a table
+  // with 8 slots per rank 6.0 against 5.8 TB/s), without them with two (6.4 against 6.0): the upper
+  // half of the grid leaves when there is something to fill.  A short one needs all of them to have
+  // enough on its way.  us, half / all, by the bytes a tensor's sums and fills touch: 22 MB 26.9 /
+  // 22.9, 37 MB 23.1 / 20.0, 235 MB 117 / 105, 245 MB 122 / 116, 470 MB 236 / 243, 700 MB 351 / 355 ..
+  // 381.
+  constexpr int64_t kLongStream = (int64_t)384 << 20;
+  const bool half = pieces > 0 && rt.bytes * (2 * n_active + t.off[a.epn] + n_clear) > kLongStream;
+  const int nwg = half ? (int)((gridDim.x + 1) / 2) : (int)gridDim.x;
   if ((int)blockIdx.x >= nwg) return;
   const int64_t q = (pieces + work - 1) / work;  // pieces that follow every tile
-  int ai = (int)(blockIdx.x / rt.tiles);
-  int64_t tile = blockIdx.x - (int64_t)ai * rt.tiles;
+  // the workgroups' turns go on from the tensor before, so that none has more than one tile more
+  // than another over all of them
+  int first = (int)blockIdx.x - (int)(before % nwg);
+  if (first < 0) first += nwg;
+  int ai = (int)(first / rt.tiles);
+  int64_t tile = first - (int64_t)ai * rt.tiles;
   // grad and first-slot vectors of the tile at hand, requested while the tile before it was
   // still being summed (a workgroup's loads then overlap its own stores)
   mep_f4 pacc[kVecPerThread], pv[kVecPerThread];
   bool ahead = false;
-  for (int64_t w = blockIdx.x; w < work; w += nwg, tile += nwg) {
+  for (int64_t w = first; w < work; w += nwg, tile += nwg) {
     while (tile >= rt.tiles) { tile -= rt.tiles; ++ai; }
     const int le = t.active[ai];
     int step;
@@ -747,9 +738,11 @@ __global__ __launch_bounds__(kBlock) void grad_reduce_kernel(ReduceBatch batch) 
   t.build<true>(a.etc, a.rank, a.R, a.epn);  // ends with a workgroup barrier
   const int n_active = (a.flags & MEP_REDUCE_CLEAR_ONLY) ? 0 : t.misc[0];
   const int n_clear = (a.flags & MEP_REDUCE_NO_CLEAR) ? 0 : occ[a.epn];
+  int64_t before = 0;  // tiles of the tensors before
   for (int i = 0; i < batch.ntensors; ++i) {
     if (i > 0) __syncthreads();  // sbase of the tensor before is no longer read
-    reduce_tensor(batch.of(i), t, occ, sbase, n_active, n_clear);
+    reduce_tensor(batch.of(i), t, occ, sbase, n_active, n_clear, before);
+    before += SpreadTiles(batch.elems[i] * 4).tiles * n_active;
   }
 }
 
@@ -907,11 +900,14 @@ int reduce_launch(int ntensors, float* const* local_grad, float* const* reduce_p
   }
   a.etc = experts_to_copy; a.ntensors = ntensors; a.rank0 = rank0; a.epn = epn; a.R = R; a.flags = flags;
   const int cus = mep_device_cu_count();
-  // persistent workgroups, two per CU (the kernel halves that when it has slots to fill);
-  // three or four per CU lose 3-7 % on a table with many slots
+  // Persistent workgroups, two per CU (the kernel halves that for a long stream with slots to fill),
+  // fewer where all experts together have fewer tiles; three or four per CU lose 3-7 % on a table with
+  // many slots.  As many as one expert has tiles, so that all took the same number of them, left most
+  // CUs idle in small ones: 16 experts of 1792 x 256, 5 hosted elsewhere, 59.4 -> 20.0 us; 4 of 1024 x
+  // 896, 3 hosted elsewhere, 42.3 -> 22.9.
   int64_t cap = 2 * (int64_t)(cus > 0 ? cus : 256) / nranks;
   if (cap < 1) cap = 1;
-  const int blocks = stream_blocks(tiles, R, epn, cap);
+  const int blocks = (int)std::min(cap, tiles * epn);
   hipLaunchKernelGGL(grad_reduce_kernel, dim3(blocks, nranks), dim3(kBlock), lds, (hipStream_t)stream, a);
   return mep_launch_status();
 }

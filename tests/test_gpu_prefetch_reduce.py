@@ -382,3 +382,37 @@ def test_grad_reduce_large_offsets(cuda):
     assert not bool(pool[0, 0].any())          # own occupied slot cleared
     assert bool((pool[0, 1] == 7.0).all())     # own free slot untouched
     assert bool((pool[2, 1] == 0.5).all())     # a peer's slot is never written
+
+
+@pytest.mark.parametrize("shapes", [
+    ((256, 384), (128, 128), (640, 256)),          # fewer tiles than workgroups: every one has at most one a tensor
+    ((1024, 896), (1024, 1024), (384, 1024)),      # turns of 512 workgroups wrap inside and between tensors
+])
+@pytest.mark.parametrize("plan", ["random", "fan_in", "empty"])
+def test_grad_reduce_batch_of_different_sizes_matches_oracle(cuda, shapes, plan):
+    """Three projections in one launch: a tensor's first tile goes to the workgroup whose turn it is
+    after the tensor before."""
+    import ctypes
+
+    from moonep_amd import _lib
+
+    print(f"grad_reduce batch {shapes} {plan}", flush=True)
+    R, epn, rank, n = 4, 8, 2, 3
+    etc = PLANS[plan](R, epn, 5)
+    g = torch.Generator().manual_seed(31)
+    local = [torch.randn(epn, *s, generator=g) for s in shapes]
+    pools = [torch.randn(R, epn, *s, generator=g) for s in shapes]
+    dev_local, dev_pools = [t.to(cuda) for t in local], [t.to(cuda) for t in pools]
+    etc_dev = etc.to(cuda)
+    rc = _lib.lib().mep_grad_reduce_batch(
+        n, (ctypes.c_void_p * n)(*[t.data_ptr() for t in dev_local]),
+        (ctypes.c_void_p * n)(*[t.data_ptr() for t in dev_pools]),
+        (ctypes.c_int64 * n)(*[int(t.stride(0)) for t in dev_pools]),
+        (ctypes.c_int64 * n)(*[s[0] * s[1] for s in shapes]),
+        etc_dev.data_ptr(), rank, 1, epn, R, 0, _lib.current_stream())
+    _lib.check(rc, "mep_grad_reduce_batch")
+    torch.cuda.synchronize()
+    for i in range(n):
+        oo.grad_reduce(local[i], pools[i], etc, rank)
+        assert torch.equal(dev_local[i].cpu().view(torch.int32), local[i].view(torch.int32)), f"sums of tensor {i}"
+        assert torch.equal(dev_pools[i].cpu().view(torch.int32), pools[i].view(torch.int32)), f"slots of tensor {i}"
