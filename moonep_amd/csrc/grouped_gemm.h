@@ -25,11 +25,10 @@ struct GemmArgs {
   const uint16_t* A2;  // dual: rows of the second K segment [M,K]
   uint16_t* Cg;        // swiglu: gate pre-activation [M,N] or null
   uint16_t* Cu;        // swiglu: up pre-activation [M,N] or null
-  float* Cf;           // wgrad: [G,M,N] fp32
+  float* Cf;           // wgrad on 128 x 256 tiles: [G,M,N] fp32
   int64_t ld;          // row stride of A and B in elements (K, or the row count for wgrad)
   int skip_from;       // wgrad: groups g >= skip_from without rows are left unwritten
-  float* Cf2;          // wgrad: the groups from `split` on go here
-  int split;
+  int split;           // wgrad: the groups of a rank from here on have an output of their own
   bool zero_tail;      // row-tiled: the rows of C beyond the last group come out as zeros
   // the 256 x 256 kernel takes the groups of several ranks at once: Gr groups per rank, whose rows
   // start at rank_rows * rank (cu counts from there)
@@ -125,17 +124,118 @@ __device__ __forceinline__ void mep_tr_issue(T& x, uint32_t lds, int offset) {
   asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(x) : "v"(lds), "n"(offset));
 }
 
-// Tile list of the weight gradient: the dimension with more tiles is cut into eight slices, one
-// per XCD (mirrored for odd groups, so that 28 tiles give every XCD 3 + 4), and every XCD takes
-// its slice of every group, two neighbouring groups at a time: all XCDs finish together whatever
-// the groups' lengths, and the tiles an XCD runs at one time are one group's slice times the whole
-// other dimension -- each line they load is wanted by 3 to 8 of them.
-struct Wgrad2Map {
-  int sliced, other;  // tiles of the sliced and of the other dimension
-  bool slice_m;       // the sliced dimension is the output row
-  __host__ __device__ int lo(int x) const { return x * sliced / 8; }
-  __host__ __device__ int size(int x) const { return (x + 1) * sliced / 8 - x * sliced / 8; }
-  __host__ __device__ int pair_count(int x) const { return (size(x) + size(7 - x)) * other; }
+// Tile list of the weight gradients.  A group's T tiles, those of a row of the longer dimension behind
+// each other, are cut into eight runs of T / 8, and XCD x takes the run (x + group) mod 8: all XCDs
+// finish together whatever the groups' lengths (slots are often empty) and however few tiles an expert
+// has, and the tiles an XCD runs at one time lie in few rows and columns of one group.  (With whole rows
+// to an XCD the 3 x 3 tiles of 768 x 768 went to four of the eight: 192 such experts on 16 ranks of 692
+// tokens, K = 8, all three products 1140 -> 654 us.)  In eight consecutive groups every XCD has T tiles,
+// and its place among them is found without a table: it walks the runs x, x + 1, ... x + 7; run v begins
+// at v T / 8, from 8 on run v - 8 counted T further.
+// Up to three products whose outputs are M x N or N x M (the projections of an expert) are one list,
+// one product behind the other.
+constexpr int kProducts = 3;
+struct WgradMap {
+  int tiles, other;   // T; tiles of the shorter dimension
+  int n;              // products
+  const uint16_t* A[kProducts];
+  const uint16_t* B[kProducts];
+  float* C[kProducts];   // [G, M, N]; the groups of a rank from a.split on go to C2
+  float* C2[kProducts];
+  int M[kProducts], N[kProducts];
+  // one of the three without an address, which would put the arguments into memory
+  template <class T>
+  __host__ __device__ static T pick(const T (&v)[kProducts], int p) { return p == 0 ? v[0] : p == 1 ? v[1] : v[2]; }
+  __host__ __device__ int begin(int v) const { return (int)((int64_t)v * tiles / 8); }
+  // an XCD's tiles of one product
+  __host__ __device__ int64_t count(int xcd, int groups) const {
+    return (int64_t)tiles * (groups >> 3) + begin(xcd + (groups & 7)) - begin(xcd);
+  }
+  // the XCD's tile `item` of a product: its group, row of the longer dimension and place in it
+  __host__ __device__ void find(int xcd, int item, int* group, int* row, int* place) const {
+    const int octet = item / tiles;
+    const int pos = item - octet * tiles + begin(xcd);
+    const int v = (8 * pos + 7) / tiles;  // the last run that begins at or before this place
+    *group = 8 * octet + v - xcd;
+    const int first = begin(v), size = begin(v + 1) - first, rows = size / other;
+    int at = pos - first;
+    if (rows * other == size) at = at % rows * other + at / rows;  // whole rows: in columns (1 % at 16 x 8 tiles)
+    at += first - (v >= 8 ? tiles : 0);
+    *row = at / other;
+    *place = at - *row * other;
+  }
+};
+
+// The tiles of one workgroup of the weight gradients, one per lane: all that their divisions and table
+// lookups need is done once, side by side, and a change of tiles reads the lane (made anew by both
+// cursors at every change they were some hundred dependent instructions: three products of 64 experts of
+// 2048 x 1024, 512 rows each, 708 -> 652 us, of 16 of 4096 x 2048, 2048 rows each, 1890 -> 1778).  As in
+// PTiles, an XCD's workgroups take `rounds` tiles each in turn, moving on by one place from round to round.
+constexpr int kListed = 64;  // most rounds
+template <bool TN>
+struct WgradTiles {
+  int a0, a1, b0, b1, c0, c1;  // addresses: first K step of the operands, first element of the output
+  int kp;                      // K steps, product
+  uint64_t left;               // the tiles to come
+  int KT, p, at;               // the present one
+  static constexpr bool tall = true;
+  __device__ __forceinline__ WgradTiles(const GemmArgs& a, const WgradMap* of) {
+    const WgradMap& map = *of;
+    const int lane = threadIdx.x & 63, xcd = blockIdx.x & 7, q = blockIdx.x >> 3;
+    const int w = q % a.width, r = q / a.width * a.rounds + lane;
+    const int per = (int)map.count(xcd, a.G);
+    int item = r * a.width + (w + r) % a.width;
+    bool live = lane < a.rounds && item < per * map.n;
+    if (!live) item = 0;
+    const int pr = (item >= per) + (item >= 2 * per);
+    item -= pr * per;
+    int g, sl, u;
+    map.find(xcd, item, &g, &sl, &u);
+    if (!live) g = 0;
+    const int rank = g / a.Gr, l = g - rank * a.Gr;
+    const int first = l > 0 ? a.cu[g - 1] : 0;
+    const int steps = (a.cu[g] - first) / kBK;
+    const int64_t kbeg = (int64_t)rank * a.rank_rows + first;
+    live = live && (steps > 0 || l < a.skip_from);
+    int64_t M = 0, N = 0;
+    uint64_t A = 0, B = 0, C = 0;
+#pragma unroll
+    for (int k = 0; k < kProducts; ++k) {
+      const uint64_t own = (uint64_t)map.C[k], other = (uint64_t)map.C2[k];
+      const uint64_t to = l < a.split ? own : other;
+      M = pr == k ? map.M[k] : M;
+      N = pr == k ? map.N[k] : N;
+      A = pr == k ? (uint64_t)map.A[k] : A;
+      B = pr == k ? (uint64_t)map.B[k] : B;
+      C = pr == k ? to : C;
+    }
+    const int64_t m0 = (M >= N ? sl : u) * kPT, n0 = (M >= N ? u : sl) * kPT;
+    A += 2 * (TN ? kbeg * M + m0 : m0 * a.ld + kbeg);
+    B += 2 * (TN ? kbeg * N + n0 : n0 * a.ld + kbeg);
+    const int64_t row = (l < a.split ? (int64_t)rank * a.split + l : (int64_t)rank * (a.Gr - a.split) + l - a.split) * M + m0;
+    C += 4 * (row * N + n0);
+    a0 = (int)(uint32_t)A; a1 = (int)(A >> 32);
+    b0 = (int)(uint32_t)B; b1 = (int)(B >> 32);
+    c0 = (int)(uint32_t)C; c1 = (int)(C >> 32);
+    kp = steps * 4 + pr;
+    left = __ballot(live);
+    KT = 0; p = 0; at = 0;
+  }
+  __device__ __forceinline__ char* lane_pointer(int lo, int hi) const {
+    return (char*)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane(hi, at) << 32) | (uint32_t)__builtin_amdgcn_readlane(lo, at));
+  }
+  __device__ __forceinline__ const char* A() const { return lane_pointer(a0, a1); }
+  __device__ __forceinline__ const char* B() const { return lane_pointer(b0, b1); }
+  __device__ __forceinline__ float* C() const { return (float*)lane_pointer(c0, c1); }
+  // the next tile to write; false: no more
+  __device__ __forceinline__ bool next() {
+    if (!left) return false;
+    at = __ffsll((unsigned long long)left) - 1;
+    left &= left - 1;
+    const int v = __builtin_amdgcn_readlane(kp, at);
+    KT = v >> 2; p = v & 3;
+    return true;
+  }
 };
 
 // The tiles of one workgroup, in order.  XCD x (workgroups x, x + 8, ...) walks a contiguous
@@ -148,32 +248,27 @@ struct Wgrad2Map {
 template <int MODE>
 struct PTiles {
   const GemmArgs& a;
-  const Wgrad2Map& map;
   int xcd, w, nw, count, first_item, r, last;  // this workgroup among the XCD's, tiles of the XCD, rounds
   int c0, carry;             // row-tiled: 64 groups, one per lane; tiles before them
   int incl, end, blocks;     // tiles up to and including the group, its end, its 128-row blocks
-  int g, m0, n0, kbeg, KT;
+  int g, m0, n0, KT;
   bool tall;
-  __device__ __forceinline__ PTiles(const GemmArgs& a_, const Wgrad2Map& map_) : a(a_), map(map_) {
+  __device__ __forceinline__ explicit PTiles(const GemmArgs& a_, const WgradMap* = nullptr) : a(a_) {
     xcd = blockIdx.x & 7; nw = a.width; w = (int)(blockIdx.x >> 3) % nw;
     r = (int)(blockIdx.x >> 3) / nw * a.rounds; last = r + a.rounds;
-    tall = true; kbeg = 0; KT = 0; g = 0; m0 = 0; n0 = 0;
-    if (MODE == kModeWgrad) {
-      count = map.pair_count(xcd) * (a.G >> 1);
-    } else {
-      int total_rt = 0;
-      for (int c = 0; c < a.G; c += 64) {
-        chunk(c);
-        total_rt += __shfl(incl, 63);
-      }
-      const int total = total_rt * a.ntiles;
-      const int per_xcd = (total + 7) >> 3;
-      first_item = xcd * per_xcd;
-      count = min(per_xcd, total - first_item);
-      count = __builtin_amdgcn_readfirstlane(count);
-      if (a.G > 64) chunk(0);
-      carry = 0;
+    tall = true; KT = 0; g = 0; m0 = 0; n0 = 0;
+    int total_rt = 0;
+    for (int c = 0; c < a.G; c += 64) {
+      chunk(c);
+      total_rt += __shfl(incl, 63);
     }
+    const int total = total_rt * a.ntiles;
+    const int per_xcd = (total + 7) >> 3;
+    first_item = xcd * per_xcd;
+    count = min(per_xcd, total - first_item);
+    count = __builtin_amdgcn_readfirstlane(count);
+    if (a.G > 64) chunk(0);
+    carry = 0;
   }
   __device__ __forceinline__ void chunk(int c) {
     c0 = c;
@@ -193,25 +288,6 @@ struct PTiles {
       if (r >= last || r * nw >= count) return false;
       ++r;
       if (item >= count) continue;
-      if (MODE == kModeWgrad) {
-        const int per_pair = map.pair_count(xcd);
-        const int pair = item / per_pair;
-        int local = item - pair * per_pair;
-        const int n_even = map.size(xcd) * map.other;
-        g = 2 * pair;
-        int xe = xcd;
-        if (local >= n_even) { local -= n_even; g += 1; xe = 7 - xcd; }
-        const int sz = map.size(xe);
-        const int u = local / sz, sl = map.lo(xe) + (local - u * sz);
-        m0 = (map.slice_m ? sl : u) * kPT; n0 = (map.slice_m ? u : sl) * kPT;
-        typedef const __attribute__((address_space(4))) int* cptr;  // scalar loads
-        const int rank = g / a.Gr, l = g - rank * a.Gr;
-        const int first = l > 0 ? ((cptr)a.cu)[g - 1] : 0;
-        KT = (((cptr)a.cu)[g] - first) / kBK;
-        kbeg = rank * a.rank_rows + first;
-        if (KT == 0 && l >= a.skip_from) continue;
-        return true;
-      }
       return find(item);
     }
   }

@@ -35,6 +35,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 
 namespace {
 
@@ -376,28 +377,51 @@ constexpr int kPSteps = 128;
 
 // AT, BT: the operand is given as [K, columns].  SCALED: scale mode with row scales.
 template <int MODE, bool AT, bool BT, bool SCALED = false>
-__global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad2Map map) {
+__global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, WgradMap map) {
   constexpr bool DUAL = MODE == kModeDual, WGRAD = MODE == kModeWgrad;
+  static_assert(!AT || WGRAD, "rows of the other products lie along K");
   static_assert(MODE != kModeSwiglu, "gemm_wide_kernel has it");
   extern __shared__ __attribute__((aligned(1024))) char gsm[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l31 = lane & 31, half = lane >> 5;
 
   // ---- loads: a cursor over (tile, K step)
-  const size_t ldA = AT ? (size_t)a.M : (size_t)a.ld, ldB = BT ? (size_t)a.N : (size_t)a.ld;
-  const size_t stepA = AT ? kBK * ldA * 2 : kBK * 2, stepB = BT ? kBK * ldB * 2 : kBK * 2;
+  // pitches; of a weight gradient's operands, [rows, M] and [rows, N], those of the product at hand
+  size_t ldA = AT ? (size_t)a.M : (size_t)a.ld, ldB = BT ? (size_t)a.N : (size_t)a.ld;
   const int KT1 = WGRAD ? 0 : a.K / kBK;
-  PTiles<MODE> ld(a, map);
-  PTiles<MODE> cp = ld;  // the tiles as they are multiplied; the groups' ends are read once for both
+  using Tiles = std::conditional_t<WGRAD, WgradTiles<AT>, PTiles<MODE>>;
+  Tiles ld(a, &map);
+  Tiles cp = ld;  // the tiles as they are multiplied; what describes them is read once for both
   const char *pA, *pB;
   uint32_t halfA, halfB;
   int kl = 0;
+  uint32_t vA[2], vB[2];
+  auto lanes = [&]() {
+    const int r = lane >> 3, kv = lane & 7, lk = lane >> 4, lv = lane & 15;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int j = 2 * wave + q;
+      vA[q] = AT ? (uint32_t)((4 * j + lk) * ldA * 2 + ((lv ^ (lk << 2)) * 16)) : (uint32_t)((8 * j + r) * ldA * 2 + ((kv ^ r ^ q) * 16));
+      vB[q] = BT ? (uint32_t)((4 * j + lk) * ldB * 2 + ((lv ^ (lk << 2)) * 16)) : (uint32_t)((8 * j + r) * ldB * 2 + ((kv ^ r ^ q) * 16));
+    }
+  };
+  if (!WGRAD) lanes();
+  int of = -1;  // weight gradient: the product that the pitches are of
   auto stand = [&](int pair) {  // the pointers at the first K step of the cursor's tile (of its second pair)
-    const size_t goff = WGRAD ? (size_t)ld.kbeg * (BT ? ldB : 1) : (size_t)ld.g * a.N * a.K;
-    const size_t offA = AT ? (size_t)ld.kbeg * ldA + ld.m0 : (size_t)ld.m0 * ldA + (WGRAD ? ld.kbeg : 0);
-    const size_t offB = goff + (BT ? (size_t)ld.n0 : (size_t)ld.n0 * ldB);
-    pA = mep_uniform((const char*)((pair ? a.A2 : a.A) + offA));
-    pB = mep_uniform((const char*)((pair ? a.B2 : a.B) + offB));
+    if constexpr (WGRAD) {
+      if (of != ld.p) {
+        of = ld.p;
+        if (AT) ldA = (size_t)WgradMap::pick(map.M, of);
+        if (BT) ldB = (size_t)WgradMap::pick(map.N, of);
+        lanes();
+      }
+      pA = ld.A();
+      pB = ld.B();
+    } else {
+      const size_t offB = (size_t)ld.g * a.N * a.K + (BT ? (size_t)ld.n0 : (size_t)ld.n0 * ldB);
+      pA = mep_uniform((const char*)((pair ? a.A2 : a.A) + (size_t)ld.m0 * ldA));
+      pB = mep_uniform((const char*)((pair ? a.B2 : a.B) + offB));
+    }
     halfA = __builtin_amdgcn_readfirstlane(ld.tall ? (AT ? 256u : (uint32_t)(128 * ldA * 2)) : 0u);
     halfB = BT ? 256u : (uint32_t)(128 * ldB * 2);
   };
@@ -409,22 +433,13 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
     if (kl + 1 < ld.KT) {
       ++kl;
       if (DUAL && kl == KT1) { stand(1); return; }
-      pA += stepA; pB += stepB;
+      pA += AT ? kBK * ldA * 2 : kBK * 2;
+      pB += BT ? kBK * ldB * 2 : kBK * 2;
       return;
     }
     do { more = ld.next(); } while (more && ld.KT == 0);
     if (more) { kl = 0; stand(0); }  // otherwise the last step is loaded again, for nobody
   };
-  uint32_t vA[2], vB[2];
-  {
-    const int r = lane >> 3, kv = lane & 7, lk = lane >> 4, lv = lane & 15;
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int j = 2 * wave + q;
-      vA[q] = AT ? (uint32_t)((4 * j + lk) * ldA * 2 + ((lv ^ (lk << 2)) * 16)) : (uint32_t)((8 * j + r) * ldA * 2 + ((kv ^ r ^ q) * 16));
-      vB[q] = BT ? (uint32_t)((4 * j + lk) * ldB * 2 + ((lv ^ (lk << 2)) * 16)) : (uint32_t)((8 * j + r) * ldB * 2 + ((kv ^ r ^ q) * 16));
-    }
-  }
   // slots are taken in turn: where the next half tile of each operand is written and read
   int wA = 0, wB = kPOperand, rA = 0, rB = kPOperand;
   auto turn = [](int& slot, int first) { slot = slot == first + (kPSlots - 1) * kPHalf ? first : slot + kPHalf; };
@@ -534,22 +549,23 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
   }
   bool any = false;
   while (cp.next()) {
-    const int g = cp.g, m0 = cp.m0, n0 = cp.n0, KT = cp.KT;
+    const int KT = cp.KT;
     const bool tall = cp.tall;
-    if (SCALED) __builtin_assume(KT > 0);
+    int m0 = 0, n0 = 0, N = a.N;
     float* cf = nullptr;
-    if (WGRAD) {
-      const int rank = g / a.Gr, l = g - rank * a.Gr;
-      const size_t mn = (size_t)a.M * a.N;
-      cf = l < a.split ? a.Cf + ((size_t)rank * a.split + l) * mn
-                       : a.Cf2 + ((size_t)rank * (a.Gr - a.split) + l - a.split) * mn;
+    if constexpr (WGRAD) {
+      cf = cp.C();
+      N = WgradMap::pick(map.N, cp.p);
+    } else {
+      m0 = cp.m0; n0 = cp.n0;
     }
+    if (SCALED) __builtin_assume(KT > 0);
     if (WGRAD && KT == 0) {  // a group without rows: whole 1 KB rows of zeroes per wave instruction
       typedef float f32x4 __attribute__((ext_vector_type(4)));
       const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
       for (int row = wave; row < kPT; row += 8)
-        __builtin_nontemporal_store(zero, (f32x4*)(cf + (size_t)(m0 + row) * a.N + n0) + lane);
+        __builtin_nontemporal_store(zero, (f32x4*)(cf + (size_t)row * N) + lane);
       continue;
     }
     any = true;
@@ -608,12 +624,12 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
       for (int i = 0; i < 2; ++i) {
         const int m = m0 + 128 * x + 64 * wm + 32 * i + 4 * half;
         if (WGRAD) {
-          float* out = cf + (size_t)m * a.N + n0 + 32 * wn + l31;
+          float* out = cf + (size_t)m * N + n0 + 32 * wn + l31;
 #pragma unroll
           for (int v = 0; v < 16; ++v)
 #pragma unroll
             for (int y = 0; y < 2; ++y)
-              __builtin_nontemporal_store(acc[x][y][i][v], out + (size_t)(8 * (v >> 2) + (v & 3)) * a.N + 128 * y);
+              __builtin_nontemporal_store(acc[x][y][i][v], out + (size_t)(8 * (v >> 2) + (v & 3)) * N + 128 * y);
         } else {
           // bf16: two rows of a column pair at a time -- the even lane of a pair stores both
           // columns of the first row, the odd lane both of the second
@@ -621,11 +637,11 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
           asm volatile("" : "+v"(at0));  // addresses made here, not kept in registers across the main loop
           const bool odd = lane & 1;
           const uint32_t sel = odd ? 0x03020706u : 0x05040100u;
-          const size_t first = (size_t)(m + odd) * a.N + n0 + 32 * wn + (l31 & ~1);
+          const size_t first = (size_t)(m + odd) * N + n0 + 32 * wn + (l31 & ~1);
           auto put = [&](uint16_t* c, int v, int col, float v0, float v1) {
             const uint32_t w = mep_cvt_bf16x2(v0, v1);
             const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0xB1, 0xf, 0xf, true);  // the pair's other lane
-            *(mep_u1_any*)(c + first + (size_t)(8 * (v >> 2) + (v & 3)) * a.N + col) = __builtin_amdgcn_perm(o, w, sel);
+            *(mep_u1_any*)(c + first + (size_t)(8 * (v >> 2) + (v & 3)) * N + col) = __builtin_amdgcn_perm(o, w, sel);
           };
 #pragma unroll
           for (int v = 0; v < 16; v += 2) {
@@ -942,13 +958,13 @@ __global__ __launch_bounds__(256) void swiglu_bwd_kernel(SwigluBwdArgs a) {
 // The grid of a kernel whose workgroups take a CU each, for at most `tiles` tiles per XCD of about
 // `steps` K steps: one workgroup per CU at one time (fewer where there are fewer tiles), each for
 // kPSteps steps.
-unsigned pp_split(GemmArgs& a, int64_t tiles, int64_t steps) {
+unsigned pp_split(GemmArgs& a, int64_t tiles, int64_t steps, int64_t most_rounds = INT32_MAX) {
   const int cus = mep_device_cu_count();
   const int64_t width = std::min<int64_t>(tiles, std::max(cus > 0 ? cus / 8 : 32, 1));
   const int64_t rounds = (tiles + width - 1) / width;
   steps = std::max<int64_t>(steps, 1);
   a.width = (int)width;
-  a.rounds = (int)std::min(rounds, std::max<int64_t>((kPSteps + steps / 2) / steps, 1));
+  a.rounds = (int)std::min({rounds, std::max<int64_t>((kPSteps + steps / 2) / steps, 1), most_rounds});
   return 8 * (unsigned)(width * ((rounds + a.rounds - 1) / a.rounds));
 }
 
@@ -980,9 +996,9 @@ int gemm_256_launch(GemmArgs a, hipStream_t st) {
     if (4 * row_tiles_256(a) * a.ntiles <= std::max(mep_device_cu_count(), 8)) {
       if (MODE == kModeScale && a.scale)
         hipLaunchKernelGGL((gemm_pp_kernel<MODE, false, BKN, MODE == kModeScale>), dim3(grid), dim3(kPThreads), kPLds, st, a,
-                           Wgrad2Map{});
+                           WgradMap{});
       else
-        hipLaunchKernelGGL((gemm_pp_kernel<MODE, false, BKN>), dim3(grid), dim3(kPThreads), kPLds, st, a, Wgrad2Map{});
+        hipLaunchKernelGGL((gemm_pp_kernel<MODE, false, BKN>), dim3(grid), dim3(kPThreads), kPLds, st, a, WgradMap{});
       return mep_launch_status();
     }
   }
@@ -1015,25 +1031,23 @@ int gemm_stream_launch(GemmArgs a, hipStream_t st) {
   return mep_launch_status();
 }
 
-// weight gradient on 256 x 256 tiles (a.M, a.N multiples of 256, a.G even)
+// weight gradients on 256 x 256 tiles (M, N multiples of 256, a.G even)
 template <bool TN>
-int wgrad_pp_launch(GemmArgs a, hipStream_t st) {
-  Wgrad2Map map;
-  const int mt = a.M / kPT, nt = a.N / kPT;
-  map.slice_m = mt >= nt;
-  map.sliced = map.slice_m ? mt : nt;
-  map.other = map.slice_m ? nt : mt;
-  int per_pair = 0;
-  for (int x = 0; x < 8; ++x) per_pair = per_pair > map.pair_count(x) ? per_pair : map.pair_count(x);
-  const int64_t per_xcd = (int64_t)per_pair * (a.G / 2);
+int wgrad_pp_launch(GemmArgs a, WgradMap map, hipStream_t st) {
+  const int m = map.M[0], n = map.N[0];
+  MEP_REQUIRE((int64_t)(m / kPT) * (n / kPT) < (1 << 24), MEP_ERR_UNSUPPORTED);
+  map.tiles = (m / kPT) * (n / kPT);
+  map.other = std::min(m, n) / kPT;
+  int64_t per_xcd = 0;
+  for (int x = 0; x < 8; ++x) per_xcd = std::max(per_xcd, map.n * map.count(x, a.G));
   MEP_REQUIRE(per_xcd > 0 && per_xcd < (1 << 27), MEP_ERR_UNSUPPORTED);
-  MEP_REQUIRE((int64_t)kPT * 2 * (TN ? (a.M > a.N ? a.M : a.N) : a.ld) < ((int64_t)1 << 31), MEP_ERR_UNSUPPORTED);
+  MEP_REQUIRE((int64_t)kPT * 2 * (TN ? (m > n ? m : n) : a.ld) < ((int64_t)1 << 31), MEP_ERR_UNSUPPORTED);
   const int irc = mep_ensure_init();
   if (irc != MEP_OK) return irc;
   // about half of the groups have rows
   const int64_t steps = 2 * (a.rank_rows ? a.rank_rows : a.ld) / kBK / a.Gr;
-  hipLaunchKernelGGL((gemm_pp_kernel<kModeWgrad, TN, TN>), dim3(pp_split(a, per_xcd, steps)), dim3(kPThreads), kPLds, st, a,
-                     map);
+  hipLaunchKernelGGL((gemm_pp_kernel<kModeWgrad, TN, TN>), dim3(pp_split(a, per_xcd, steps, kListed)), dim3(kPThreads), kPLds,
+                     st, a, map);
   return mep_launch_status();
 }
 
@@ -1138,24 +1152,40 @@ int gemm_nn(const void* A1, const void* B1, const void* A2, const void* B2, cons
   return A2 ? row_tiled<kModeDual, true>(a, (hipStream_t)stream) : row_tiled<kModeScale, true>(a, (hipStream_t)stream);
 }
 
-// weight gradient from the activations as they are; the groups from `split` on go to C2
-int wgrad_tn(const void* X1, const void* X2, const int32_t* cu, int G, float* C, float* C2, int split, int Ma, int Nb,
-             int64_t rows, int skip_empty_from, void* stream, int nranks = 1) {
-  MEP_REQUIRE(X1 && X2 && cu && C && C2, MEP_ERR_INVALID_ARG);
-  MEP_REQUIRE(Ma > 0 && Nb > 0 && G > 0 && rows > 0 && skip_empty_from >= 0, MEP_ERR_INVALID_ARG);
-  MEP_REQUIRE(Ma % kPT == 0 && Nb % kPT == 0 && G % 2 == 0 && rows % kBM == 0, MEP_ERR_UNSUPPORTED);
-  MEP_REQUIRE((int64_t)(Ma > Nb ? Ma : Nb) * rows < ((int64_t)1 << 40), MEP_ERR_UNSUPPORTED);
-  MEP_REQUIRE(((uintptr_t)X1 % 16 == 0) && ((uintptr_t)X2 % 16 == 0) && ((uintptr_t)C % 16 == 0) &&
-                  ((uintptr_t)C2 % 16 == 0), MEP_ERR_ALIGNMENT);
+// Weight gradients from the activations as they are, in one launch: n products of X1 [rows, M] and
+// X2 [rows, N], whose outputs are M x N or N x M; a rank's groups from `split` on go to C2.  As three
+// launches each of them has a start and a last round of its own: us, 48 experts of 512 x 512 with 465
+// rows each 142 -> 114, 8 of 4864 x 1536 with 1685 rows 771 -> 746, 64 of 2048 x 1024 with 512 rows 761 -> 724.
+int wgrad_tn(int n, const void* const* X1, const void* const* X2, const int32_t* cu, int G, float* const* C,
+             float* const* C2, int split, const int* M, const int* N, int64_t rows, int skip_empty_from, void* stream,
+             int nranks = 1) {
+  MEP_REQUIRE(cu && G > 0 && rows > 0 && skip_empty_from >= 0, MEP_ERR_INVALID_ARG);
+  MEP_REQUIRE(G % 2 == 0 && rows % kBM == 0 && rows * nranks <= INT32_MAX, MEP_ERR_UNSUPPORTED);
+  WgradMap map{};
+  map.n = n;
+  for (int i = 0; i < n; ++i) {
+    MEP_REQUIRE(X1[i] && X2[i] && C[i] && C2[i] && M[i] > 0 && N[i] > 0, MEP_ERR_INVALID_ARG);
+    MEP_REQUIRE(M[i] % kPT == 0 && N[i] % kPT == 0, MEP_ERR_UNSUPPORTED);
+    MEP_REQUIRE((int64_t)(M[i] > N[i] ? M[i] : N[i]) * rows < ((int64_t)1 << 40), MEP_ERR_UNSUPPORTED);
+    MEP_REQUIRE(((uintptr_t)X1[i] % 16 == 0) && ((uintptr_t)X2[i] % 16 == 0) && ((uintptr_t)C[i] % 16 == 0) &&
+                    ((uintptr_t)C2[i] % 16 == 0), MEP_ERR_ALIGNMENT);
+    MEP_REQUIRE(std::max(M[i], N[i]) == std::max(M[0], N[0]) && std::min(M[i], N[i]) == std::min(M[0], N[0]),
+                MEP_ERR_INVALID_ARG);
+    map.A[i] = (const uint16_t*)X1[i];
+    map.B[i] = (const uint16_t*)X2[i];
+    map.C[i] = C[i];
+    map.C2[i] = C2[i];
+    map.M[i] = M[i];
+    map.N[i] = N[i];
+  }
   GemmArgs a{};
-  a.A = (const uint16_t*)X1; a.B = (const uint16_t*)X2; a.cu = cu; a.Cf = C; a.Cf2 = C2; a.split = split;
-  a.M = Ma; a.N = Nb; a.K = 0; a.G = G * nranks;
+  a.cu = cu; a.split = split;
+  a.G = G * nranks;
   a.ld = rows;
   a.Gr = G;
   a.rank_rows = (int)rows;
   a.skip_from = skip_empty_from;
-  MEP_REQUIRE(rows * nranks <= INT32_MAX, MEP_ERR_UNSUPPORTED);
-  return wgrad_pp_launch<true>(a, (hipStream_t)stream);
+  return wgrad_pp_launch<true>(a, map, (hipStream_t)stream);
 }
 
 template <class Kern>
@@ -1256,8 +1286,12 @@ extern "C" int mep_grouped_gemm_wgrad(const void* At, const void* Bt, const int3
   a.split = G;
   a.Gr = G;
   // an expert's shapes: 256 x 256 tiles (whose lane offsets are 32 bits)
-  if (Ma % kPT == 0 && Nb % kPT == 0 && G % 2 == 0 && (uintptr_t)C % 16 == 0 && ld < ((int64_t)1 << 22))
-    return wgrad_pp_launch<false>(a, (hipStream_t)stream);
+  if (Ma % kPT == 0 && Nb % kPT == 0 && G % 2 == 0 && (uintptr_t)C % 16 == 0 && ld < ((int64_t)1 << 22)) {
+    WgradMap map{};
+    map.n = 1;
+    map.A[0] = a.A; map.B[0] = a.B; map.C[0] = map.C2[0] = C; map.M[0] = Ma; map.N[0] = Nb;
+    return wgrad_pp_launch<false>(a, map, (hipStream_t)stream);
+  }
   a.mtiles = Ma / kBM;
   a.ntiles = Nb / kBN;
   return gemm_launch<kModeWgrad>(a, (int64_t)a.mtiles * a.ntiles * G, (hipStream_t)stream);
@@ -1266,7 +1300,7 @@ extern "C" int mep_grouped_gemm_wgrad(const void* At, const void* Bt, const int3
 extern "C" int mep_grouped_gemm_wgrad_tn(const void* X1, const void* X2, const int32_t* cu_seqlens, int G,
                                          float* C, int Ma, int Nb, int64_t rows, int skip_empty_from,
                                          void* stream) {
-  return wgrad_tn(X1, X2, cu_seqlens, G, C, C, G, Ma, Nb, rows, skip_empty_from, stream);
+  return wgrad_tn(1, &X1, &X2, cu_seqlens, G, &C, &C, G, &Ma, &Nb, rows, skip_empty_from, stream);
 }
 
 namespace {
@@ -1318,10 +1352,10 @@ extern "C" int mep_ffn_backward(const void* dy, const void* rows, const float* s
   if (rc == MEP_OK) rc = gemm_nn(dgate, gate, dup, up, cu_seqlens, G, drows, nullptr, M, H, Hp, true, stream, nranks);
   const void* x1[3] = {dgate, dup, dy};
   const void* x2[3] = {rows, rows, hs};
-  for (int i = 0; i < 3 && rc == MEP_OK; ++i)
-    rc = wgrad_tn(x1[i], x2[i], cu_seqlens, G, wgrads[i], wgrads_from_split[i], split, i < 2 ? Hp : H, i < 2 ? H : Hp,
-                  M, skip_empty_from, stream, nranks);
-  return rc;
+  const int m[3] = {Hp, Hp, H}, n[3] = {H, H, Hp};
+  return rc == MEP_OK ? wgrad_tn(3, x1, x2, cu_seqlens, G, wgrads, wgrads_from_split, split, m, n, M, skip_empty_from,
+                                 stream, nranks)
+                      : rc;
 }
 
 extern "C" int mep_transpose_bf16(const void* src, void* dst, int batch, int rows, int cols, void* stream) {
