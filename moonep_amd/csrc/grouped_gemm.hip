@@ -18,10 +18,12 @@
 //                          tile the rows
 //   gemm_pp_kernel         256 x 256 tiles: weight gradients, and the other products where
 //                          few of the CUs get a tile
-//   gemm_stream_kernel     128 rows x up to 288 weight rows, forward products of
-//                          groups of about one block: bound by the weights' bytes
-//   grouped_gemm_nt_kernel 128 x 256 tiles: backward products of such groups, and
-//                          weight gradients that are no multiples of 256
+//   gemm_stream_kernel     128 rows x up to 288 weight rows or 256 weight columns:
+//                          forward products and input gradients of groups of about
+//                          one block, and of few tiles: bound by the weights' bytes
+//   grouped_gemm_nt_kernel 128 x 256 tiles: the sum of two products with weights
+//                          along K of such groups, and weight gradients that are no
+//                          multiples of 256
 //
 // grouped_gemm_nt_kernel: workgroups of 640 threads on a 128 x 256 tile of (rows
 // x weight rows), K in steps of 64: two producer waves stream the tile slices
@@ -50,14 +52,6 @@ constexpr int kPanel = 8;  // row tiles of a long group that share a sweep over 
 constexpr int kPiecesPerProducer = (kBM + kBN) / 8 / kProducers;  // 24
 static_assert(2 * kPiecesPerProducer < 64, "two steps of loads must fit the 6-bit load counter");
 
-// eight K values of one column from two transposing LDS reads (K rows k .. k+3 and k+4 .. k+7)
-__device__ __forceinline__ mep_bf16x8 mep_tr_pair(const char* lo, const char* hi) {
-  const mep_s16x4 x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) mep_s16x4*)lo);
-  const mep_s16x4 y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) mep_s16x4*)hi);
-  const mep_s16x8 z = __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7);
-  return __builtin_bit_cast(mep_bf16x8, z);
-}
-
 // Producer / consumer waves.  Two producer waves stream the tiles from global
 // memory straight into a ring of three LDS stages (global_load_lds, 16 bytes
 // per lane: no registers, no LDS store instructions), always two K steps
@@ -68,19 +62,9 @@ __device__ __forceinline__ mep_bf16x8 mep_tr_pair(const char* lo, const char* hi
 // sixteen rows that sixteen consecutive lanes read cover all 64 banks once (a
 // 16-byte read runs at 256 bytes per clock then; with q ^ (r & 7) alone, which
 // separates only eight rows, at half of that).
-//
-// BKN: the weights are given as [G, K, N] (the output column contiguous), as the
-// backward pass finds them -- dX = dY * W with W stored for Y = X * W^T.  A K
-// step of the weight tile is then 64 rows of 512 bytes in LDS, and a consumer
-// lane gets its eight K values of one column from two transposing LDS reads
-// (ds_read_b64_tr_b16: sixteen lanes read a 4 x 16 block, four rows of 32
-// bytes, and each receives one column of it).  The 16-byte vector v of row k
-// sits at position v ^ 2 (k & 3): the four rows of such a block then cover all
-// banks once.
-template <int MODE, bool BKN = false>
+template <int MODE>
 __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_nt_kernel(GemmArgs a) {
-  static_assert(MODE == kModeDual || (MODE == kModeScale ? BKN : MODE == kModeWgrad), "the products that need it");
-  static_assert(!BKN || MODE == kModeScale || MODE == kModeDual, "[K, N] weights: plain and dual products only");
+  static_assert(MODE == kModeDual || MODE == kModeWgrad, "the products that need it");
   static_assert(kProducers == 2, "the lane offsets of the pieces assume that a producer wave's pieces share a parity");
   extern __shared__ __attribute__((aligned(1024))) char gsm[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -185,17 +169,11 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_nt_kernel(GemmAr
     const size_t goff = MODE == kModeWgrad ? (size_t)kbeg : (size_t)g * a.N * K;
     const size_t lane_off = (size_t)r * K + ((kv ^ r ^ (p & 1)) * 8);
     const uint16_t* Ap = a.A + (size_t)m0 * K + lane_off + (MODE == kModeWgrad ? (size_t)kbeg : 0);
-    // [K, N] weights: piece jb holds the K rows 2 jb and 2 jb + 1 of the step; lane (lk, lv)
-    // fetches vector lv ^ 2 (row & 3) of row 2 jb + lk, and (2 jb + lk) & 3 = 2 (p & 1) + lk
-    // because this wave's pieces all have the parity of p
-    const int lk = lane >> 5, lv = lane & 31;
-    const size_t lane_off_kn = (size_t)lk * a.N + (size_t)((lv ^ ((2 * (p & 1) + lk) << 1)) * 8) + n0;
-    const uint16_t* Bp0 = BKN ? a.B + goff + lane_off_kn : a.B + goff + (size_t)n0 * K + lane_off;
+    const uint16_t* Bp0 = a.B + goff + (size_t)n0 * K + lane_off;
     const uint16_t* Bp1 = Bp0 + (size_t)(kBN / 2) * K;
     // dual: the second half of the K loop reads the second pair
     const uint16_t* Aq = MODE == kModeDual ? a.A2 + (size_t)m0 * K + lane_off : Ap;
-    const uint16_t* Bq0 = MODE != kModeDual ? Bp0
-                          : BKN ? a.B2 + goff + lane_off_kn : a.B2 + goff + (size_t)n0 * K + lane_off;
+    const uint16_t* Bq0 = MODE == kModeDual ? a.B2 + goff + (size_t)n0 * K + lane_off : Bp0;
     const uint16_t* Bq1 = Bq0 + (size_t)(kBN / 2) * K;
     auto issue = [&](int k0, int stage) {
       char* base = gsm + stage * kStage;
@@ -209,7 +187,6 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_nt_kernel(GemmAr
         const int j = p + q * kProducers;  // 0 .. 47
         const uint16_t* src;
         if (j < kBM / 8) src = pa + (size_t)(8 * j) * K + k0;
-        else if (BKN) src = pb0 + (size_t)(k0 + 2 * (j - kBM / 8)) * a.N;
         else if (j < kBM / 8 + kBN / 16) src = pb0 + (size_t)(8 * (j - kBM / 8)) * K + k0;
         else src = pb1 + (size_t)(8 * (j - kBM / 8 - kBN / 16)) * K + k0;
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
@@ -251,14 +228,6 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_nt_kernel(GemmAr
   const int half = lane >> 5;   // which 8 of the 16 K values of an MFMA step
   const int oa0 = arow * kRowBytes, oa1 = (arow + 32) * kRowBytes;
   const int ob0 = brow0 * kRowBytes, ob1 = brow1 * kRowBytes;
-  // [K, N] weights: lane s of a block of sixteen reads 8 bytes of row 8 half + s / 4 (+ 4 for
-  // the second read, + 16 per MFMA step) at the columns 64 wn + 32 j + 16 (block & 1) + 4 (s & 3)
-  const int ts = lane & 15, tb = (lane >> 4) & 1;
-  const int okn0 = kATile + (8 * half + (ts >> 2)) * (kBN * 2) +
-                   (((8 * wn + 2 * tb + ((ts & 3) >> 1)) ^ ((ts >> 2) << 1)) * 16) + (ts & 1) * 8;
-  const int okn1 = kATile + (8 * half + (ts >> 2)) * (kBN * 2) +
-                   (((8 * wn + 4 + 2 * tb + ((ts & 3) >> 1)) ^ ((ts >> 2) << 1)) * 16) + (ts & 1) * 8;
-
   if (any) {
     __builtin_amdgcn_s_barrier();  // stage 0 is filled
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
@@ -271,15 +240,8 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_nt_kernel(GemmAr
       const int col = ((2 * ks + half) ^ sw) * 16;
       const mep_bf16x8 a0 = *(const mep_bf16x8*)(sb + oa0 + col);
       const mep_bf16x8 a1 = *(const mep_bf16x8*)(sb + oa1 + col);
-      mep_bf16x8 b0, b1;
-      if (BKN) {
-        const int step = ks * 16 * (kBN * 2);
-        b0 = mep_tr_pair(sb + okn0 + step, sb + okn0 + step + 4 * (kBN * 2));
-        b1 = mep_tr_pair(sb + okn1 + step, sb + okn1 + step + 4 * (kBN * 2));
-      } else {
-        b0 = *(const mep_bf16x8*)(sb + ob0 + col);
-        b1 = *(const mep_bf16x8*)(sb + ob1 + col);
-      }
+      const mep_bf16x8 b0 = *(const mep_bf16x8*)(sb + ob0 + col);
+      const mep_bf16x8 b1 = *(const mep_bf16x8*)(sb + ob1 + col);
       acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, b0, acc[0][0], 0, 0, 0);
       acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, b1, acc[0][1], 0, 0, 0);
       acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b0, acc[1][0], 0, 0, 0);
@@ -307,11 +269,10 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_nt_kernel(GemmAr
           // writes evicts the operand lines the other tiles of the group still need (9 % slower)
           __builtin_nontemporal_store(acc[i][j][v], &cf[(size_t)m * ldc + n0 + 64 * wn + 32 * j + (lane & 31)]);
       } else {
-        const float sc = a.scale ? a.scale[m] : 1.0f;
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
           const int n = n0 + 64 * wn + 32 * j + (lane & 31);
-          a.C[(size_t)m * ldc + n] = (uint16_t)mep_f32_to_bf16_bits(sc * acc[i][j][v]);
+          a.C[(size_t)m * ldc + n] = (uint16_t)mep_f32_to_bf16_bits(acc[i][j][v]);
         }
       }
     }
@@ -697,6 +658,16 @@ constexpr int kSUnit = 32 * kRowBytes;     // 4 KB
 constexpr int kSLds = 160 * 1024;
 constexpr int kSParts = 2;                 // workgroups that share what a CU does
 
+// Two rows of a pair of neighbouring columns, one column a lane: the even lane stores both columns of the
+// first row, the odd lane both of the second.  c: the row and the first column of what this lane stores
+// (one value at a time: FFN forward of 64 tokens, 16 experts of 4096 x 2048 198 -> 195.6 us, of 18 tokens,
+// 4 experts of 3072 x 512 49 -> 47.6, of 106 tokens, 8 experts of 2816 x 256 36.7 -> 35).
+__device__ __forceinline__ void store_two_rows(uint16_t* c, float row0, float row1) {
+  const uint32_t w = mep_cvt_bf16x2(row0, row1);
+  const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0xB1, 0xf, 0xf, true);  // the pair's other lane
+  *(mep_u1_any*)c = __builtin_amdgcn_perm(o, w, threadIdx.x & 1 ? 0x03020706u : 0x05040100u);
+}
+
 template <int MODE, int NU>
 __device__ __forceinline__ void stream_tile(const GemmArgs& a, char* gsm, int m0, int g, int unit0) {
   constexpr bool SWIGLU = MODE == kModeSwiglu;
@@ -791,36 +762,154 @@ __device__ __forceinline__ void stream_tile(const GemmArgs& a, char* gsm, int m0
       // gate in the lanes 0 .. 15 of a half wave, up in 16 .. 31: the first take the rows of
       // v = 0 .. 7, the others of v = 8 .. 15, and hand each other what they lack
       const bool up = l31 >= 16;
-      const size_t first = (size_t)(m + (up ? 16 : 0)) * a.N + 16 * unit + (l31 & 15);
+      const size_t first = (size_t)(m + (up ? 16 : 0) + (lane & 1)) * a.N + 16 * unit + (l31 & 14);
 #pragma unroll
-      for (int v = 0; v < 8; ++v) {
-        const float mine = up ? acc[i][v + 8] : acc[i][v];
-        const float other = __shfl_xor(up ? acc[i][v] : acc[i][v + 8], 16);
-        const float gv = up ? other : mine, uv = up ? mine : other;
+      for (int v = 0; v < 8; v += 2) {
+        float gv[2], uv[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const float mine = up ? acc[i][v + 8 + e] : acc[i][v + e];
+          const float other = __shfl_xor(up ? acc[i][v + e] : acc[i][v + 8 + e], 16);
+          gv[e] = up ? other : mine;
+          uv[e] = up ? mine : other;
+        }
         const size_t o = first + (size_t)(8 * (v >> 2) + (v & 3)) * a.N;
-        a.C[o] = (uint16_t)mep_f32_to_bf16_bits(mep_silu(gv) * uv);
-        if (a.Cg) a.Cg[o] = (uint16_t)mep_f32_to_bf16_bits(gv);
-        if (a.Cu) a.Cu[o] = (uint16_t)mep_f32_to_bf16_bits(uv);
+        store_two_rows(a.C + o, mep_silu(gv[0]) * uv[0], mep_silu(gv[1]) * uv[1]);
+        if (a.Cg) store_two_rows(a.Cg + o, gv[0], gv[1]);
+        if (a.Cu) store_two_rows(a.Cu + o, uv[0], uv[1]);
       }
     } else {
-      uint16_t* c = a.C + (size_t)m * a.N + 32 * unit + l31;
+      uint16_t* c = a.C + (size_t)(m + (lane & 1)) * a.N + 32 * unit + (l31 & ~1);
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
+      for (int v = 0; v < 16; v += 2) {
         const int dr = 8 * (v >> 2) + (v & 3);
-        const float sc = a.scale ? a.scale[m + dr] : 1.0f;
-        c[(size_t)dr * a.N] = (uint16_t)mep_f32_to_bf16_bits(sc * acc[i][v]);
+        const float s0 = a.scale ? a.scale[m + dr] : 1.0f, s1 = a.scale ? a.scale[m + dr + 1] : 1.0f;
+        store_two_rows(c + (size_t)dr * a.N, s0 * acc[i][v], s1 * acc[i][v + 1]);
       }
     }
   }
 }
 
-template <int MODE>
+// The same for weights given as [K, N] (input gradients, alone or as a sum of two pairs).  A unit is 64
+// weight columns: a K step of it is 64 rows of 128 bytes in LDS, 16-byte vector v of row k at v ^ 2 (k & 3),
+// so that the two blocks of 4 x 16 which 32 lanes read with a transposing read cover all banks.  A wave
+// brings eight of the 64 rows and multiplies 32 rows by 32 columns of every unit.  us, dy * down and both
+// pairs, 128 x 256 tiles -> this: 4 blocks of K = 5632, 768 columns 97 / 181 -> 44 / 82; 12 of 1024 x 1024
+// 26 / 41 -> 13 / 21; 24 of 2048 x 4096 90 / 160 -> 88 / 155 (weights at 4.8 and 5.4 TB/s).
+constexpr int kSUnitsKn = 4;
+constexpr int kSUnitKn = 64 * kRowBytes;   // 8 KB
+
+template <int MODE, int NU>
+__device__ __forceinline__ void stream_tile_kn(const GemmArgs& a, char* gsm, int m0, int g, int unit0) {
+  constexpr bool DUAL = MODE == kModeDual;
+  constexpr int kStageBytes = kSA + NU * kSUnitKn;
+  constexpr int D = kSLds / kStageBytes < 8 ? kSLds / kStageBytes : 8;
+  static_assert(D >= 3 && (D - 1) * (2 + NU) < 64, "the loads on their way must fit the 6-bit counter");
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l31 = lane & 31, half = lane >> 5;
+  const int rb = wave & 3, uh = wave >> 2;
+  const size_t ldA = (size_t)a.K * 2, ldB = (size_t)a.N * 2;
+  const int KT1 = a.K / kBK, KT = DUAL ? 2 * KT1 : KT1;
+
+  const int r = lane >> 3, kv = lane & 7;
+  const size_t offA = (size_t)(m0 + 16 * wave) * ldA;
+  const size_t offB = ((size_t)g * a.K + 8 * wave) * ldB + (size_t)unit0 * kRowBytes;
+  const char* pA = mep_uniform((const char*)a.A + offA);
+  const char* pB = mep_uniform((const char*)a.B + offB);
+  uint32_t vA[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) vA[q] = (uint32_t)((8 * q + r) * ldA + ((kv ^ r ^ q) * 16));
+  const uint32_t vB = (uint32_t)(r * ldB + ((kv ^ (r & 3) << 1) * 16));
+  int kl = 0, ws = 0, rs = 0;
+  auto issue = [&]() {
+    if (DUAL && kl == KT1) {
+      pA = mep_uniform((const char*)a.A2 + offA);
+      pB = mep_uniform((const char*)a.B2 + offB);
+    }
+    const int bytes = __builtin_amdgcn_readfirstlane(kl < KT ? -1 : 0);  // past the last step: counted, but nothing is read
+    char* slot = gsm + ws;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) mep_load_lds16(pA, vA[q], 0, slot + (2 * wave + q) * 1024, bytes);
+#pragma unroll
+    for (int i = 0; i < NU; ++i)
+      mep_load_lds16<kNontemporal>(pB, vB, i * kRowBytes, slot + kSA + i * kSUnitKn + wave * 1024, bytes);
+    pA += kRowBytes;
+    pB += kBK * ldB;
+    ++kl;
+    ws = ws == (D - 1) * kStageBytes ? 0 : ws + kStageBytes;
+  };
+#pragma unroll
+  for (int k = 0; k < D - 1; ++k) issue();
+
+  mep_f32x16 acc[NU];
+#pragma unroll
+  for (int i = 0; i < NU; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[i][v] = 0.0f;
+  const int sw = (lane & 7) ^ ((lane >> 3) & 1);
+  int ad[4];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) ad[ks] = (32 * rb + l31) * kRowBytes + ((2 * ks + half) ^ sw) * 16;
+  // a block of sixteen lanes reads four rows of K by sixteen columns
+  const int ts = lane & 15, tb = (lane >> 4) & 1;
+  const int lds0 = (int)(uintptr_t)(__attribute__((address_space(3))) char*)gsm;
+  const int adB = lds0 + kSA + (8 * half + (ts >> 2)) * kRowBytes +
+                  (((4 * uh + 2 * tb + ((ts & 3) >> 1)) ^ (ts >> 2 << 1)) * 16) + (ts & 1) * 8;
+
+  for (int kt = 0; kt < KT; ++kt) {
+    // this wave's part of step kt is there; after the barrier everybody's, and the slot of the
+    // step before has been read by all
+    mep_wait_vm_lgkm0<(D - 2) * (2 + NU)>();
+    mep_bar();
+    mep_bf16x8 fa[4];
+    mep_s16x4 tw[4][NU][2];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      fa[ks] = *(const mep_bf16x8*)(gsm + rs + ad[ks]);
+#pragma unroll
+      for (int i = 0; i < NU; ++i)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) mep_tr_issue(tw[ks][i][u], adB + rs, i * kSUnitKn + ks * 2048 + u * 512);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    issue();
+    __builtin_amdgcn_sched_barrier(0);
+    mep_wait_lgkm0();
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+      for (int i = 0; i < NU; ++i) {
+        asm volatile("; arrived %0 %1" : "+v"(tw[ks][i][0]), "+v"(tw[ks][i][1]));
+        const mep_bf16x8 fb =
+            __builtin_bit_cast(mep_bf16x8, __builtin_shufflevector(tw[ks][i][0], tw[ks][i][1], 0, 1, 2, 3, 4, 5, 6, 7));
+        acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[ks], fb, acc[i], 0, 0, 0);
+      }
+    rs = rs == (D - 1) * kStageBytes ? 0 : rs + kStageBytes;
+  }
+  mep_wait_vm_lgkm0<0>();  // the loads past the last step write LDS, too
+  mep_bar();               // the next tile may be loaded
+
+  // acc[i][v] is row 32 rb + 8 (v / 4) + 4 half + v % 4, column 32 uh + l31 of unit i
+  const int m = m0 + 32 * rb + 4 * half;
+  uint16_t* c = a.C + (size_t)(m + (lane & 1)) * a.N + 64 * unit0 + 32 * uh + (l31 & ~1);
+#pragma unroll
+  for (int v = 0; v < 16; v += 2) {
+    const int dr = 8 * (v >> 2) + (v & 3);
+    float s0 = 1.0f, s1 = 1.0f;
+    if (!DUAL && a.scale) { s0 = a.scale[m + dr]; s1 = a.scale[m + dr + 1]; }
+#pragma unroll
+    for (int i = 0; i < NU; ++i) store_two_rows(c + (size_t)dr * a.N + 64 * i, s0 * acc[i][v], s1 * acc[i][v + 1]);
+  }
+}
+
+template <int MODE, bool KN>
 __global__ __launch_bounds__(kSThreads, 2) void gemm_stream_kernel(GemmArgs a) {
   extern __shared__ __attribute__((aligned(1024))) char gsm[];
-  const int per_block = a.N / (MODE == kModeSwiglu ? 16 : 32);
+  constexpr int kUnits = KN ? kSUnitsKn : kSUnits;
+  const int per_block = a.N / (KN ? 64 : MODE == kModeSwiglu ? 16 : 32);
   const int blocks = min(a.mtiles, a.cu[a.G - 1] / kBM);
   // `per` tiles of a block: as many as make the tiles of all blocks whole rounds of the CUs
-  const int least = (per_block + kSUnits - 1) / kSUnits;
+  const int least = (per_block + kUnits - 1) / kUnits;
   const int width = 8 * a.width;
   const int rounds = (blocks * least + width - 1) / width;
   const int per = min(per_block, rounds * width / max(blocks, 1));
@@ -846,16 +935,25 @@ __global__ __launch_bounds__(kSThreads, 2) void gemm_stream_kernel(GemmArgs a) {
     g = __builtin_amdgcn_readfirstlane(g);
     if (g < 0) break;  // cannot happen: the block lies below the last end
     const int m0 = mt * kBM;
-    switch (n) {
-      case 1: stream_tile<MODE, 1>(a, gsm, m0, g, unit0); break;
-      case 2: stream_tile<MODE, 2>(a, gsm, m0, g, unit0); break;
-      case 3: stream_tile<MODE, 3>(a, gsm, m0, g, unit0); break;
-      case 4: stream_tile<MODE, 4>(a, gsm, m0, g, unit0); break;
-      case 5: stream_tile<MODE, 5>(a, gsm, m0, g, unit0); break;
-      case 6: stream_tile<MODE, 6>(a, gsm, m0, g, unit0); break;
-      case 7: stream_tile<MODE, 7>(a, gsm, m0, g, unit0); break;
-      case 8: stream_tile<MODE, 8>(a, gsm, m0, g, unit0); break;
-      default: stream_tile<MODE, 9>(a, gsm, m0, g, unit0); break;
+    if constexpr (KN) {
+      switch (n) {
+        case 1: stream_tile_kn<MODE, 1>(a, gsm, m0, g, unit0); break;
+        case 2: stream_tile_kn<MODE, 2>(a, gsm, m0, g, unit0); break;
+        case 3: stream_tile_kn<MODE, 3>(a, gsm, m0, g, unit0); break;
+        default: stream_tile_kn<MODE, 4>(a, gsm, m0, g, unit0); break;
+      }
+    } else {
+      switch (n) {
+        case 1: stream_tile<MODE, 1>(a, gsm, m0, g, unit0); break;
+        case 2: stream_tile<MODE, 2>(a, gsm, m0, g, unit0); break;
+        case 3: stream_tile<MODE, 3>(a, gsm, m0, g, unit0); break;
+        case 4: stream_tile<MODE, 4>(a, gsm, m0, g, unit0); break;
+        case 5: stream_tile<MODE, 5>(a, gsm, m0, g, unit0); break;
+        case 6: stream_tile<MODE, 6>(a, gsm, m0, g, unit0); break;
+        case 7: stream_tile<MODE, 7>(a, gsm, m0, g, unit0); break;
+        case 8: stream_tile<MODE, 8>(a, gsm, m0, g, unit0); break;
+        default: stream_tile<MODE, 9>(a, gsm, m0, g, unit0); break;
+      }
     }
   }
   if (a.zero_tail) zero_tail_rows(a, blockIdx.x, gridDim.x, kSThreads);
@@ -1006,28 +1104,28 @@ int gemm_256_launch(GemmArgs a, hipStream_t st) {
 }
 
 // 144 KB of dynamic LDS: opted in by mep_init_gemm_kernels
-template <int MODE, bool BKN = false>
+template <int MODE>
 int gemm_launch(const GemmArgs& a, int64_t total, hipStream_t st) {
   MEP_REQUIRE(total > 0 && total < (1 << 30), MEP_ERR_UNSUPPORTED);
   const int per_xcd = (int)((total + 7) / 8) + (a.zero_tail ? 1 : 0);
   const size_t lds = (size_t)kStages * kStage;
   const int irc = mep_ensure_init();
   if (irc != MEP_OK) return irc;
-  hipLaunchKernelGGL((grouped_gemm_nt_kernel<MODE, BKN>), dim3(per_xcd * 8), dim3(kGemmThreads), lds, st, a);
+  hipLaunchKernelGGL((grouped_gemm_nt_kernel<MODE>), dim3(per_xcd * 8), dim3(kGemmThreads), lds, st, a);
   return mep_launch_status();
 }
 
-template <int MODE>
+template <int MODE, bool KN>
 int gemm_stream_launch(GemmArgs a, hipStream_t st) {
-  const int64_t units = (int64_t)a.mtiles * (a.N / (MODE == kModeSwiglu ? 16 : 32));
+  const int64_t units = (int64_t)a.mtiles * (a.N / (KN ? 64 : MODE == kModeSwiglu ? 16 : 32));
   MEP_REQUIRE(units > 0 && units < ((int64_t)1 << 30), MEP_ERR_UNSUPPORTED);
   // offsets inside a tile are 32 bits
-  MEP_REQUIRE((int64_t)32 * kSUnits * 2 * a.K < ((int64_t)1 << 31), MEP_ERR_UNSUPPORTED);
+  MEP_REQUIRE((int64_t)(KN ? 8 : 32 * kSUnits) * 2 * std::max(2 * a.K, KN ? a.N : 0) < ((int64_t)1 << 32), MEP_ERR_UNSUPPORTED);
   const int irc = mep_ensure_init();
   if (irc != MEP_OK) return irc;
   const int cus = mep_device_cu_count();
   a.width = (int)std::min<int64_t>((units + 7) / 8, std::max(cus > 0 ? cus / 8 : 32, 1));
-  hipLaunchKernelGGL((gemm_stream_kernel<MODE>), dim3(8 * a.width * kSParts), dim3(kSThreads), kSLds, st, a);
+  hipLaunchKernelGGL((gemm_stream_kernel<MODE, KN>), dim3(8 * a.width * kSParts), dim3(kSThreads), kSLds, st, a);
   return mep_launch_status();
 }
 
@@ -1088,13 +1186,30 @@ bool for_ranks(GemmArgs& a, int nranks) {
 // mep_set_gemm_row_tile(128 or 256) forces one side (tests run both on small shapes).
 std::atomic<int> g_forced_row_tile{0};
 
-bool use_256_tiles(const GemmArgs& a, bool forward) {
+bool use_256_tiles(const GemmArgs& a, bool forward, bool kn) {
   if (a.G != a.Gr) return true;  // several ranks
   const int forced = g_forced_row_tile.load(std::memory_order_relaxed);
   if (forced) return forced == 256;
   const int64_t rows = std::max((int64_t)a.M - (int64_t)(kBM - 1) * a.G, (int64_t)0);
-  // products of the backward pass: 256-row tiles unless half of their matrix work would be padding
-  if (!forward) return 2 * rows >= (int64_t)kBM * a.G;
+  // both pairs with weights along K: 256-row tiles unless half of their matrix work would be padding
+  if (!forward && !kn) return 2 * rows >= (int64_t)kBM * a.G;
+  const int64_t cus = std::max(mep_device_cu_count(), 8);
+  const int64_t blocks = std::max<int64_t>(a.G / 2 + 1, rows / kBM + a.G / 4);
+  const int64_t tiles = row_tiles_256(a) * a.ntiles, rounds = (tiles + cus - 1) / cus;
+  if (kn) {
+    // Input gradients: the time of either kernel in 10 ns, fitted to 172 products of 4 to 96 blocks of 8 to
+    // 96 groups, 256 .. 5632 by 256 .. 5632 (off by 9 and 12 %).  A round of streaming tiles of n units costs
+    // 6 + n us and 0.24 + 0.22 n a K step, one of 256 x 256 tiles 6 us and 0.9 to 1.5 a step.  us,
+    // streaming / 256 x 256 tiles, dy * down and both pairs: 4 blocks of K = 5632, 768 columns 44 / 76,
+    // 82 / 162; 12 of 1024 x 1024 13 / 20, 21 / 36; 17 of 2048 x 4096 68 / 85, 117 / 159; 24 of 2048 x 4096
+    // in 13 groups 88 / 56, 155 / 104; 96 of 1024 x 1024 52 / 34, 80 / 61.
+    const int64_t steps = (int64_t)a.K / kBK * (a.A2 ? 2 : 1);
+    const int64_t units = a.N / 64, least = (units + kSUnitsKn - 1) / kSUnitsKn;
+    const int64_t turns = (blocks * least + cus - 1) / cus, per = std::min(units, turns * cus / blocks);
+    const int64_t n = (units + per - 1) / per;
+    return 200 + 600 * rounds + steps * (90 * rounds + 64 * std::min(tiles, cus) / cus) <
+           turns * (600 + 100 * n + steps * (24 + 22 * n));
+  }
   // Forward products: what a K step costs either kernel.  The local experts (half of the groups)
   // and a slot or two have rows, the last block of each about half filled.  A round of 256 x 256
   // tiles takes 1.57 us a step whether it is full or not; the streaming kernel 0.21 us for each
@@ -1102,9 +1217,6 @@ bool use_256_tiles(const GemmArgs& a, bool forward) {
   // 4096 x 2048, E = 128, K = 8: 64 tokens 183 / 289, 256 245 .. 277 / 301; 512 404 / 302;
   // 7168 x 2048, E = 256: 256 tokens 597 / 738, 512 800 / 765; 1024 x 512, E = 64: 512 tokens
   // 44 / 51, 1024 76 / 53; 512 x 256, E = 16, K = 4, 2048 tokens: 34 / 40.
-  const int64_t cus = std::max(mep_device_cu_count(), 8);
-  const int64_t blocks = std::max<int64_t>(a.G / 2 + 1, rows / kBM + a.G / 4);
-  const int64_t rounds = (row_tiles_256(a) * a.ntiles + cus - 1) / cus;
   return 1570 * rounds * cus < 210 * blocks * 8 * a.ntiles;  // a tile is eight units wide
 }
 
@@ -1112,9 +1224,9 @@ bool use_256_tiles(const GemmArgs& a, bool forward) {
 template <int MODE, bool BKN>
 int row_tiled(const GemmArgs& a, hipStream_t st) {
   constexpr bool forward = !BKN && (MODE == kModeScale || MODE == kModeSwiglu);
-  if (use_256_tiles(a, forward)) return gemm_256_launch<MODE, BKN>(a, st);
-  if constexpr (forward) return gemm_stream_launch<MODE>(a, st);
-  else return gemm_launch<MODE, BKN>(a, (int64_t)a.mtiles * a.ntiles, st);
+  if (use_256_tiles(a, forward, BKN)) return gemm_256_launch<MODE, BKN>(a, st);
+  if constexpr (forward || BKN) return gemm_stream_launch<MODE, BKN>(a, st);
+  else return gemm_launch<MODE>(a, (int64_t)a.mtiles * a.ntiles, st);
 }
 
 int gemm_nt_forward(const void* A, const void* B, const void* B_up, const int32_t* cu, int G, void* C,
@@ -1204,12 +1316,12 @@ int mep_init_gemm_kernels() {
   const size_t ring = (size_t)kStages * kStage;
   int rc = MEP_OK;
 #define MEP_OPT(k, b) if (rc == MEP_OK) rc = opt_in_lds(k, b)
-  MEP_OPT((gemm_stream_kernel<kModeScale>), kSLds);
-  MEP_OPT((gemm_stream_kernel<kModeSwiglu>), kSLds);
-  MEP_OPT((grouped_gemm_nt_kernel<kModeDual, false>), ring);
-  MEP_OPT((grouped_gemm_nt_kernel<kModeWgrad, false>), ring);
-  MEP_OPT((grouped_gemm_nt_kernel<kModeScale, true>), ring);
-  MEP_OPT((grouped_gemm_nt_kernel<kModeDual, true>), ring);
+  MEP_OPT((gemm_stream_kernel<kModeScale, false>), kSLds);
+  MEP_OPT((gemm_stream_kernel<kModeSwiglu, false>), kSLds);
+  MEP_OPT((gemm_stream_kernel<kModeScale, true>), kSLds);
+  MEP_OPT((gemm_stream_kernel<kModeDual, true>), kSLds);
+  MEP_OPT((grouped_gemm_nt_kernel<kModeDual>), ring);
+  MEP_OPT((grouped_gemm_nt_kernel<kModeWgrad>), ring);
   MEP_OPT((gemm_pp_kernel<kModeScale, false, false>), kPLds);
   MEP_OPT((gemm_pp_kernel<kModeScale, false, false, true>), kPLds);
   MEP_OPT((gemm_pp_kernel<kModeDual, false, false>), kPLds);
