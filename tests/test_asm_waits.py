@@ -61,5 +61,5 @@ def test_the_gemm_kernels_as_they_are_compiled(tmp_path):
     path = str(tmp_path / "gemm.s")
     build.gemm_assembly(path)
     # 16 transposing reads in each kernel with [K, N] weights (3), 48 in the weight gradient, two
-    # scales in each of the scaled (2)
-    assert build.check_gemm_waits(path) == 3 * 16 + 48 + 2 * 2
+    # scales in each of the scaled (2); 8 for every unit of a streaming tile of 1 to 4, alone and in pairs
+    assert build.check_gemm_waits(path) == 3 * 16 + 48 + 2 * 2 + 2 * 8 * (1 + 2 + 3 + 4)
