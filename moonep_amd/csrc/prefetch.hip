@@ -22,30 +22,28 @@ constexpr int kVecPerThread = 4;                       // 16-byte vectors in fli
 constexpr int kTileBytes = kBlock * kVecPerThread * 16;  // 16 KiB per workgroup step
 constexpr int kMaxTensors = 6;
 
-// Slot table of `rank`: for each owned (local) expert the slots rb = d*epn+b
-// holding it, ascending.  LDS: e[R*epn], list[R*epn], off[epn+1], cur[epn],
-// active[epn], misc[2].  Built with LDS atomics for the counts and one wave
+// Slot table of `own` experts from expert `lo` on (one rank's, or several ranks'): for each of
+// them the slots rb = d*epn+b of the n = R*epn holding it, ascending.  LDS: e[n], list[n],
+// off[own+1], cur[own], active[own], misc[2].  Built with LDS atomics for the counts and one wave
 // walking the table 64 slots at a time (lanes holding the same expert are
 // found with one ballot per id bit), so a workgroup pays about a microsecond.
 struct SlotTable {
   int* e; int* list; int* off; int* cur; int* active; int* misc;
-  __device__ void carve(int* smem, int R, int epn) {
-    e = smem; list = e + R * epn; off = list + R * epn; cur = off + epn + 1;
-    active = cur + epn; misc = active + epn;
+  __device__ void carve(int* smem, int n, int own) {
+    e = smem; list = e + n; off = list + n; cur = off + own + 1;
+    active = cur + own; misc = active + own;
   }
   // All threads of the workgroup call this.  ORDERED: every expert's slots in ascending
   // order (the reduction adds them in that order); otherwise in any order (a copy to every
   // slot does not care), which all threads fill in at once instead of one wave walking the
   // table.
   template <bool ORDERED>
-  __device__ void build(const int* etc, int rank, int R, int epn) {
-    const int n = R * epn;
-    const int lo = rank * epn;
+  __device__ void build(const int* etc, int lo, int n, int own, int epn) {
     const int lane = threadIdx.x & 63;
-    for (int i = threadIdx.x; i <= epn; i += blockDim.x) off[i] = 0;
+    for (int i = threadIdx.x; i <= own; i += blockDim.x) off[i] = 0;
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
       const int v = etc[i] - lo;
-      e[i] = ((unsigned)v < (unsigned)epn) ? v : -1;
+      e[i] = ((unsigned)v < (unsigned)own) ? v : -1;
     }
     __syncthreads();
     for (int i = threadIdx.x; i < n; i += blockDim.x)
@@ -54,14 +52,14 @@ struct SlotTable {
     if (threadIdx.x < 64) {
       // exclusive prefix of the counts, list of experts with at least one slot
       int run = 0, na = 0;
-      for (int c = 0; c < epn; c += 64) {
+      for (int c = 0; c < own; c += 64) {
         const int le = c + lane;
-        const int cnt = le < epn ? off[le + 1] : 0;
+        const int cnt = le < own ? off[le + 1] : 0;
         const int incl = mep_wave_incl_scan(cnt);
         const uint64_t m = __ballot(cnt > 0);
         if (cnt > 0) active[na + __popcll(m & mep_lanes_lt())] = le;
         mep_wave_sync();
-        if (le < epn) { off[le + 1] = run + incl; cur[le] = run + incl - cnt; }
+        if (le < own) { off[le + 1] = run + incl; cur[le] = run + incl - cnt; }
         run += __builtin_amdgcn_readlane(incl, 63);
         na += __popcll(m);
       }
@@ -69,7 +67,7 @@ struct SlotTable {
       mep_wave_sync();
       if (ORDERED) {
         // slots in ascending order per expert
-        const int nbits = 32 - __clz(epn > 1 ? epn - 1 : 1);
+        const int nbits = 32 - __clz(own > 1 ? own - 1 : 1);
         for (int c = 0; c < n; c += 64) {
           const int le = c + lane < n ? e[c + lane] : -1;
           uint64_t same = __ballot(le >= 0);
@@ -102,9 +100,9 @@ struct SlotTable {
   }
 };
 
-__host__ __device__ inline int slot_table_ints(int R, int epn) { return 2 * R * epn + 3 * epn + 4; }
+__host__ __device__ inline int slot_table_ints(int n, int own) { return 2 * n + 3 * own + 4; }
 
-size_t slot_table_bytes(int R, int epn) { return (size_t)slot_table_ints(R, epn) * sizeof(int); }
+size_t slot_table_bytes(int n, int own) { return (size_t)slot_table_ints(n, own) * sizeof(int); }
 
 // Tile layout of both kernels.  A tile is 256 threads x 4 vectors of 16 bytes.
 // Where an expert's matrix allows it the four vectors of a thread lie 32 KiB
@@ -171,8 +169,8 @@ struct PrefetchTile {
 __global__ __launch_bounds__(kBlock) void prefetch_kernel(PrefetchArgs a) {
   extern __shared__ int smem[];
   SlotTable t;
-  t.carve(smem, a.R, a.epn);
-  t.build<false>(a.etc, a.rank, a.R, a.epn);
+  t.carve(smem, a.R * a.epn, a.epn);
+  t.build<false>(a.etc, a.rank * a.epn, a.R * a.epn, a.epn, a.epn);
   const unsigned n_active = (unsigned)__builtin_amdgcn_readfirstlane(t.misc[0]);
   if (n_active == 0) return;
   unsigned total = 0;
@@ -505,6 +503,7 @@ struct ReduceArgs {
   int64_t elems;        // per expert
   const int* etc;
   int rank, epn, R;
+  int own;              // experts summed, from rank * epn on: epn, or several ranks'
   unsigned flags;       // MEP_REDUCE_*
 };
 
@@ -512,20 +511,22 @@ constexpr int kMaxReduce = 3;
 
 // One launch sums several projections, one after the other with all workgroups on each (all at
 // once was 17 % slower: three times as many streams), over one slot table; a launch per projection
-// ends and begins with a few microseconds in which only part of the chip has work.  blockIdx.y is
-// the rank, for a caller that plays several.
+// ends and begins with a few microseconds in which only part of the chip has work.  For a caller
+// that plays several ranks their experts are one list: the experts that are hosted elsewhere belong
+// to few ranks (those of the popular ones), and workgroups dealt out by rank left most CUs idle.
+// us, by rank -> one list, three projections of 2048 x 1024, eight ranks of eight experts: seven slots
+// of one rank's experts 215 -> 76.5, five of one and two others 162 -> 77, four ranks' 105 -> 69, one
+// slot 30.5 -> 13, one slot of each rank 102 -> 100 (6.0 TB/s).
 struct ReduceBatch {
   float* local_grad[kMaxReduce];
   float* pool[kMaxReduce];
   int64_t rank_stride[kMaxReduce];
   int64_t elems[kMaxReduce];
   const int* etc;
-  int ntensors, rank0, epn, R;  // local_grad: a block of epn experts per rank
+  int ntensors, rank0, nranks, epn, R;  // local_grad: a block of epn experts per rank
   unsigned flags;
   __device__ __forceinline__ ReduceArgs of(int t) const {
-    const int r = blockIdx.y;
-    return ReduceArgs{local_grad[t] + (int64_t)r * epn * elems[t], pool[t], rank_stride[t], elems[t],
-                      etc, rank0 + r, epn, R, flags};
+    return ReduceArgs{local_grad[t], pool[t], rank_stride[t], elems[t], etc, rank0, epn, R, nranks * epn, flags};
   }
 };
 
@@ -560,7 +561,7 @@ __device__ __forceinline__ void reduce_tensor(const ReduceArgs& a, const SlotTab
   const SpreadTiles rt(a.elems * 4);
   const bool clear_as_read = a.flags == 0;  // own slots holding own experts, zeroed by their reader
   // where each entry of the slot lists starts in the pool, so that a tile only adds its offset
-  for (int i = threadIdx.x; i < t.off[a.epn]; i += kBlock) {
+  for (int i = threadIdx.x; i < t.off[a.own]; i += kBlock) {
     const int rb = t.list[i];
     const int src = rb / a.epn, b = rb - src * a.epn;
     sbase[i] = ((int64_t)src * a.rank_stride + (int64_t)b * a.elems) * 4;
@@ -594,7 +595,7 @@ __device__ __forceinline__ void reduce_tensor(const ReduceArgs& a, const SlotTab
   // 22.9, 37 MB 23.1 / 20.0, 235 MB 117 / 105, 245 MB 122 / 116, 470 MB 236 / 243, 700 MB 351 / 355 ..
   // 381.
   constexpr int64_t kLongStream = (int64_t)384 << 20;
-  const bool half = pieces > 0 && rt.bytes * (2 * n_active + t.off[a.epn] + n_clear) > kLongStream;
+  const bool half = pieces > 0 && rt.bytes * (2 * n_active + t.off[a.own] + n_clear) > kLongStream;
   const int nwg = half ? (int)((gridDim.x + 1) / 2) : (int)gridDim.x;
   if ((int)blockIdx.x >= nwg) return;
   const int64_t q = (pieces + work - 1) / work;  // pieces that follow every tile
@@ -716,9 +717,10 @@ __global__ __launch_bounds__(kBlock) void grad_reduce_kernel(ReduceBatch batch) 
   extern __shared__ int smem[];
   const ReduceArgs a = batch.of(0);
   SlotTable t;
-  t.carve(smem, a.R, a.epn);
-  int* occ = smem + slot_table_ints(a.R, a.epn);  // [epn] own slots holding foreign experts, [1] their number
-  int64_t* sbase = (int64_t*)(smem + ((slot_table_ints(a.R, a.epn) + a.epn + 2) & ~1));  // [R*epn] byte offset in the pool of list entry i
+  const int entries = a.R * a.epn, ints = slot_table_ints(entries, a.own);
+  t.carve(smem, entries, a.own);
+  int* occ = smem + ints;  // [epn] own slots holding foreign experts, [1] their number
+  int64_t* sbase = (int64_t*)(smem + ((ints + a.epn + 2) & ~1));  // [R*epn] byte offset in the pool of list entry i
   if (threadIdx.x < 64) {
     const int lane = threadIdx.x;
     const int lo = a.rank * a.epn;
@@ -735,7 +737,7 @@ __global__ __launch_bounds__(kBlock) void grad_reduce_kernel(ReduceBatch batch) 
     }
     if (lane == 0) occ[a.epn] = n;
   }
-  t.build<true>(a.etc, a.rank, a.R, a.epn);  // ends with a workgroup barrier
+  t.build<true>(a.etc, a.rank * a.epn, entries, a.own, a.epn);  // ends with a workgroup barrier
   const int n_active = (a.flags & MEP_REDUCE_CLEAR_ONLY) ? 0 : t.misc[0];
   const int n_clear = (a.flags & MEP_REDUCE_NO_CLEAR) ? 0 : occ[a.epn];
   int64_t before = 0;  // tiles of the tensors before
@@ -756,7 +758,7 @@ extern "C" int mep_prefetch(int ntensors, const void* const* local, void* const*
               MEP_ERR_INVALID_ARG);
   MEP_REQUIRE(ntensors > 0 && ntensors <= kMaxTensors, MEP_ERR_INVALID_ARG);
   MEP_REQUIRE(epn > 0 && R > 0 && rank >= 0 && rank < R, MEP_ERR_INVALID_ARG);
-  const size_t lds = slot_table_bytes(R, epn);
+  const size_t lds = slot_table_bytes(R * epn, epn);
   MEP_REQUIRE(lds <= 64 * 1024, MEP_ERR_UNSUPPORTED);
   PrefetchArgs a;
   a.ntensors = ntensors; a.rank = rank; a.epn = epn; a.R = R; a.etc = experts_to_copy;
@@ -891,24 +893,32 @@ int reduce_launch(int ntensors, float* const* local_grad, float* const* reduce_p
     if (rt.tiles > tiles) tiles = rt.tiles;
   }
   // slot table + own foreign-held slots + a pool offset per list entry
-  const size_t lds = slot_table_bytes(R, epn) + ((size_t)epn + 2) * sizeof(int) +
-                     (size_t)R * epn * sizeof(int64_t) + 8;
-  MEP_REQUIRE(lds <= kReduceLdsMax, MEP_ERR_UNSUPPORTED);
+  auto lds_of = [&](int ranks) {
+    return slot_table_bytes(R * epn, ranks * epn) + ((size_t)epn + 2) * sizeof(int) + (size_t)R * epn * sizeof(int64_t) + 8;
+  };
+  MEP_REQUIRE(lds_of(1) <= kReduceLdsMax, MEP_ERR_UNSUPPORTED);
+  int chunk = nranks;  // ranks of a launch
+  while (lds_of(chunk) > kReduceLdsMax) chunk = (chunk + 1) / 2;
+  const size_t lds = lds_of(chunk);
   if (lds > 64 * 1024) {  // large rank x slot tables: opted in by mep_init_stream_kernels
     const int irc = mep_ensure_init();
     if (irc != MEP_OK) return irc;
   }
-  a.etc = experts_to_copy; a.ntensors = ntensors; a.rank0 = rank0; a.epn = epn; a.R = R; a.flags = flags;
+  a.etc = experts_to_copy; a.ntensors = ntensors; a.epn = epn; a.R = R; a.flags = flags;
   const int cus = mep_device_cu_count();
   // Persistent workgroups, two per CU (the kernel halves that for a long stream with slots to fill),
   // fewer where all experts together have fewer tiles; three or four per CU lose 3-7 % on a table with
   // many slots.  As many as one expert has tiles, so that all took the same number of them, left most
   // CUs idle in small ones: 16 experts of 1792 x 256, 5 hosted elsewhere, 59.4 -> 20.0 us; 4 of 1024 x
   // 896, 3 hosted elsewhere, 42.3 -> 22.9.
-  int64_t cap = 2 * (int64_t)(cus > 0 ? cus : 256) / nranks;
-  if (cap < 1) cap = 1;
-  const int blocks = (int)std::min(cap, tiles * epn);
-  hipLaunchKernelGGL(grad_reduce_kernel, dim3(blocks, nranks), dim3(kBlock), lds, (hipStream_t)stream, a);
+  const int64_t cap = 2 * (int64_t)(cus > 0 ? cus : 256);
+  for (int r = 0; r < nranks; r += chunk) {
+    a.rank0 = rank0 + r;
+    a.nranks = std::min(chunk, nranks - r);
+    for (int i = 0; i < ntensors; ++i) a.local_grad[i] = local_grad[i] + (int64_t)r * epn * elems_per_expert[i];
+    const int blocks = (int)std::min(cap, tiles * epn * a.nranks);
+    hipLaunchKernelGGL(grad_reduce_kernel, dim3(blocks), dim3(kBlock), lds, (hipStream_t)stream, a);
+  }
   return mep_launch_status();
 }
 }  // namespace

@@ -100,6 +100,38 @@ def test_views_and_gradient_sums_of_a_group(cuda, R, epn, shapes):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("R,epn,elems,owner,rank0,nranks", [
+    (8, 8, 4096, 3, 0, 8),       # every hosted expert belongs to one rank
+    (4, 3, 36868, 0, 0, 4),      # experts past a 128 KiB block, few experts, the first rank's
+    (16, 5, 1028, 15, 9, 7),     # some of the ranks, the last rank's experts
+    (4, 2, 256, 1, 2, 2),        # none of theirs
+    (64, 96, 64, 37, 0, 64),     # a table that takes more than one launch
+])
+def test_sums_of_several_ranks_where_one_owns_the_hosted_experts(cuda, R, epn, elems, owner, rank0, nranks):
+    import ctypes as C
+
+    from moonep_amd import _lib
+    g = torch.Generator().manual_seed(R + epn)
+    etc = torch.full((R, epn), -1, dtype=torch.int32)
+    for d in range(min(R, 12)):
+        etc[d, d % epn] = owner * epn + int(torch.randint(0, min(epn, 3), (1,), generator=g))
+    own = torch.randn(nranks, epn, elems, generator=g)
+    pool = torch.randn(R, epn, elems, generator=g)
+    want = own.clone()
+    for d, b in (etc >= 0).nonzero().tolist():      # slots are added in ascending order, in fp32
+        e = int(etc[d, b])
+        if rank0 <= e // epn < rank0 + nranks:
+            want[e // epn - rank0, e % epn] += pool[d, b]
+    etc, got, slots = etc.to(cuda), own.to(cuda), pool.to(cuda)
+    arr_p, arr_i = C.c_void_p * 1, C.c_int64 * 1
+    rc = _lib.lib().mep_grad_reduce_batch(1, arr_p(got.data_ptr()), arr_p(slots.data_ptr()), arr_i(epn * elems),
+                                          arr_i(elems), etc.data_ptr(), rank0, nranks, epn, R, _lib.REDUCE_NO_CLEAR,
+                                          _lib.current_stream())
+    assert rc == 0
+    torch.cuda.synchronize()
+    assert torch.equal(got.cpu(), want) and torch.equal(slots.cpu(), pool)
+
+
 def _routed(cuda, R, E, S, K, H, seed):
     topk = torch.stack([routing.popularity_biased(S, K, E, R, r, 1.0, seed=seed) for r in range(R)])
     g = torch.Generator().manual_seed(seed)
