@@ -132,6 +132,37 @@ def test_sums_of_several_ranks_where_one_owns_the_hosted_experts(cuda, R, epn, e
     assert torch.equal(got.cpu(), want) and torch.equal(slots.cpu(), pool)
 
 
+@pytest.mark.parametrize("R,epn,nbytes,full,rank0,nranks", [
+    (8, 8, 16384, (5,), 0, 8),           # every occupied slot on one rank
+    (4, 3, 147472, (0, 3), 0, 4),        # experts past a 128 KiB block
+    (16, 70, 1040, (9, 15), 9, 7),       # some of the ranks, more slots than a wave has lanes
+    (4, 2, 256, (0, 1), 2, 2),           # no slot of theirs
+    (96, 86, 16, (0, 50, 95), 0, 96),    # a list that takes more than one launch
+])
+def test_slots_of_several_ranks_where_few_ranks_host(cuda, R, epn, nbytes, full, rank0, nranks):
+    import ctypes as C
+
+    from moonep_amd import _lib
+    g = torch.Generator().manual_seed(R + epn)
+    etc = torch.full((R, epn), -1, dtype=torch.int32)
+    for d in full:
+        etc[d, : epn - epn // 3] = torch.randint(0, R * epn, (epn - epn // 3,), generator=g).to(torch.int32)
+    local = torch.randint(0, 256, (R, epn, nbytes), dtype=torch.uint8, generator=g)
+    want = torch.randint(0, 256, (R, epn, nbytes), dtype=torch.uint8, generator=g)
+    src, got = local.to(cuda), want.to(cuda)
+    for d, b in (etc >= 0).nonzero().tolist():
+        if rank0 <= d < rank0 + nranks:
+            want[d, b] = local.view(-1, nbytes)[int(etc[d, b])]
+    etc = etc.to(cuda)
+    arr_p, arr_i = C.c_void_p * 1, C.c_int64 * 1
+    stride = arr_i(epn * nbytes)
+    rc = _lib.lib().mep_prefetch_pull_ranks(1, arr_p(src.data_ptr()), stride, arr_p(got.data_ptr()), stride, arr_i(nbytes),
+                                            etc.data_ptr(), rank0, nranks, epn, R, _lib.current_stream())
+    assert rc == 0
+    torch.cuda.synchronize()
+    assert torch.equal(got.cpu(), want) and torch.equal(src.cpu(), local)
+
+
 def _routed(cuda, R, E, S, K, H, seed):
     topk = torch.stack([routing.popularity_biased(S, K, E, R, r, 1.0, seed=seed) for r in range(R)])
     g = torch.Generator().manual_seed(seed)
