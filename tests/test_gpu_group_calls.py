@@ -170,6 +170,23 @@ def _routed(cuda, R, E, S, K, H, seed):
     return x, topk.to(cuda), routing.tokens_per_expert(topk, E).to(cuda)
 
 
+@pytest.mark.parametrize("used", ["rows", "slots", "both"])
+def test_dispatch_backward_where_only_some_outputs_are_used(cuda, used):
+    """An output that nobody used counts as one with a gradient of zeroes."""
+    R, epn, S, K, H, tp = 4, 2, 21, 3, 136, 16
+    group = moe.EmulatedGroup(S, H, K, R * epn, R, token_padding=tp)
+    x, topk, tpe = _routed(cuda, R, R * epn, S, K, H, seed=3)
+    w = torch.rand(R, S, K, device=cuda).requires_grad_()
+    rows, slots, _, _ = moe.group_dispatch(group, x, w, topk, tpe)
+    g_rows = torch.randn_like(rows) * (used != "slots")
+    g_slots = torch.randn_like(slots) * (used != "rows")
+    want = torch.autograd.grad((rows, slots), (x, w), (g_rows, g_slots), retain_graph=True)
+    outs = {"rows": ((rows,), (g_rows,)), "slots": ((slots,), (g_slots,)), "both": ((rows, slots), (g_rows, g_slots))}[used]
+    got = torch.autograd.grad(outs[0], (x, w), outs[1])
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
 def test_two_dispatches_of_a_group_in_flight(cuda, monkeypatch):
     """Micro-batches: the first one's combine and its backward work from the first one's plans."""
     R, epn, S, K, H, tp = 4, 2, 21, 3, 136, 16
