@@ -907,7 +907,15 @@ __global__ __launch_bounds__(kSThreads, 2) void gemm_stream_kernel(GemmArgs a) {
   extern __shared__ __attribute__((aligned(1024))) char gsm[];
   constexpr int kUnits = KN ? kSUnitsKn : kSUnits;
   const int per_block = a.N / (KN ? 64 : MODE == kModeSwiglu ? 16 : 32);
-  const int blocks = min(a.mtiles, a.cu[a.G - 1] / kBM);
+  // several ranks (at most 64, one a lane; input gradients only): their blocks are counted through
+  const bool ranks = KN && a.G != a.Gr;
+  auto rank_blocks = [&]() {
+    const int r = (int)(threadIdx.x & 63);
+    return r * a.Gr < a.G ? a.cu[r * a.Gr + a.Gr - 1] / kBM : 0;
+  };
+  int all = a.cu[a.G - 1] / kBM;
+  if (ranks) all = __builtin_amdgcn_readlane(mep_wave_incl_scan(rank_blocks()), 63);
+  const int blocks = min(a.mtiles, all);
   // `per` tiles of a block: as many as make the tiles of all blocks whole rounds of the CUs
   const int least = (per_block + kUnits - 1) / kUnits;
   const int width = 8 * a.width;
@@ -925,16 +933,26 @@ __global__ __launch_bounds__(kSThreads, 2) void gemm_stream_kernel(GemmArgs a) {
     const int mt = t / per, tl = t - mt * per;
     const int unit0 = tl * per_block / per;
     const int n = (tl + 1) * per_block / per - unit0;
-    // the group of this block: the first whose padded end lies beyond it
+    // its rank, and the block among that rank's
+    int rank = 0, mb = mt;
+    if (ranks) {
+      const int n_r = rank_blocks(), incl = mep_wave_incl_scan(n_r);
+      rank = __ffsll((unsigned long long)__ballot(incl > mt)) - 1;
+      if (rank < 0) break;  // cannot happen: the block lies below the sum
+      mb -= __builtin_amdgcn_readlane(incl - n_r, rank);
+    }
+    // the group of this block: the first of the rank whose padded end lies beyond it
+    const int* cu = a.cu + rank * a.Gr;
     int g = -1;
-    for (int c = 0; c < a.G && g < 0; c += 64) {
+    for (int c = 0; c < a.Gr && g < 0; c += 64) {
       const int gi = c + (int)(threadIdx.x & 63);
-      const uint64_t mask = __ballot(gi < a.G && a.cu[gi] > mt * kBM);
+      const uint64_t mask = __ballot(gi < a.Gr && cu[gi] > mb * kBM);
       if (mask) g = c + __ffsll((unsigned long long)mask) - 1;
     }
     g = __builtin_amdgcn_readfirstlane(g);
     if (g < 0) break;  // cannot happen: the block lies below the last end
-    const int m0 = mt * kBM;
+    g += rank * a.Gr;
+    const int m0 = rank * a.rank_rows + mb * kBM;
     if constexpr (KN) {
       switch (n) {
         case 1: stream_tile_kn<MODE, 1>(a, gsm, m0, g, unit0); break;
@@ -1187,7 +1205,8 @@ bool for_ranks(GemmArgs& a, int nranks) {
 std::atomic<int> g_forced_row_tile{0};
 
 bool use_256_tiles(const GemmArgs& a, bool forward, bool kn) {
-  if (a.G != a.Gr) return true;  // several ranks
+  const bool ranks = a.G != a.Gr;
+  if (ranks && (!kn || a.G / a.Gr > 64)) return true;  // the streaming kernel has a lane for each
   const int forced = g_forced_row_tile.load(std::memory_order_relaxed);
   if (forced) return forced == 256;
   const int64_t rows = std::max((int64_t)a.M - (int64_t)(kBM - 1) * a.G, (int64_t)0);
@@ -1196,6 +1215,14 @@ bool use_256_tiles(const GemmArgs& a, bool forward, bool kn) {
   const int64_t cus = std::max(mep_device_cu_count(), 8);
   const int64_t blocks = std::max<int64_t>(a.G / 2 + 1, rows / kBM + a.G / 4);
   const int64_t tiles = row_tiles_256(a) * a.ntiles, rounds = (tiles + cus - 1) / cus;
+  // Several ranks' input gradients: groups are many and tiles fill the chip either way; with less than
+  // a block a group most 256-row tiles are half empty.  us, backward pass (weight gradients included),
+  // streaming / 256 x 256: 8 ranks, 128 groups of 2048 x 1024 with 71 blocks 581 / 634, 95 676 / 721,
+  // 163 990 / 905; 16 ranks, 384 of 768 x 768 with 205 591 / 620, 512 of 1024 x 512 with 269 709 / 753;
+  // 4 ranks, 32 of 512 x 256 with 19 40 / 50; 8 ranks, 64 of 1024 x 512 with 38 115 / 111.  Forward
+  // passes of these: 246 / 252, 298 / 278, 535 / 358, 257 / 230, 311 / 274, 21 / 24, 52 / 38.
+  // Experts of more than 2048 x 1024 were not compared and stay.
+  if (ranks) return blocks >= a.G || (int64_t)a.N * a.K > 2048 * 1024;
   if (kn) {
     // Input gradients: the time of either kernel in 10 ns, fitted to 172 products of 4 to 96 blocks of 8 to
     // 96 groups, 256 .. 5632 by 256 .. 5632 (off by 9 and 12 %).  A round of streaming tiles of n units costs
