@@ -155,19 +155,24 @@ class _PlanTensors:
 def _rank_addresses(t):
     """Where each rank's part of a tensor with a leading rank dimension starts."""
     first, step = t.data_ptr(), t.stride(0) * t.element_size()
-    return range(first, first + step * t.shape[0], step)
+    return list(range(first, first + step * t.shape[0], step))
 
 
 def _plan_tensors(group, plans):
     """The stacked tensors of ``plans``: those they are views of, where a whole-group dispatch made
     them (any of those in flight: the plans carry them), else stacked here; the groups' ends are
     known to the former only."""
+    # the kernels read and write where the plans say, for as many ranks as the group has
+    R, sizes = group.R, (group.S * group.K, group.R, group.E, group.NvS, group.K)
+    assert len(plans) == R, f"a group of {R} ranks takes {R} plans, got {len(plans)}"
+    for r, p in enumerate(plans):
+        got = (p.N, p.R, p.E, p.NvS, p.K)
+        assert got == sizes, f"plan {r} must be of N, R, E, NvS, K = {sizes}, got {got}"
     own = getattr(plans[0].dst, "_group_tensors", None)
     # `own` holds its memory, so an equal address is the same memory
-    if own is None or len(plans) != group.R or any(
-            p.dst.data_ptr() != at for p, at in zip(plans, _rank_addresses(own.dst))):
+    if own is None or [p.dst.data_ptr() for p in plans] != _rank_addresses(own.dst):
         return _PlanTensors(torch.stack([p.dst for p in plans]), torch.stack([p.zero_fill_ranges for p in plans]), None)
-    if all(p.zero_fill_ranges.data_ptr() == at for p, at in zip(plans, _rank_addresses(own.zero_fill))):
+    if [p.zero_fill_ranges.data_ptr() for p in plans] == _rank_addresses(own.zero_fill):
         return own
     return _PlanTensors(own.dst, torch.stack([p.zero_fill_ranges for p in plans]), own.cu)
 
