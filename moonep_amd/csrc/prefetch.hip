@@ -23,80 +23,120 @@ constexpr int kTileBytes = kBlock * kVecPerThread * 16;  // 16 KiB per workgroup
 constexpr int kMaxTensors = 6;
 
 // Slot table of `own` experts from expert `lo` on (one rank's, or several ranks'): for each of
-// them the slots rb = d*epn+b of the n = R*epn holding it, ascending.  LDS: e[n], list[n],
-// off[own+1], cur[own], active[own], misc[2].  Built with LDS atomics for the counts and one wave
-// walking the table 64 slots at a time (lanes holding the same expert are
-// found with one ballot per id bit), so a workgroup pays about a microsecond.
+// them the slots rb = d*epn+b of the n = R*epn holding it.  LDS: e[n], list[n], off[own+1],
+// cur[own], active[own], misc[2].
 struct SlotTable {
   int* e; int* list; int* off; int* cur; int* active; int* misc;
   __device__ void carve(int* smem, int n, int own) {
     e = smem; list = e + n; off = list + n; cur = off + own + 1;
     active = cur + own; misc = active + own;
   }
-  // All threads of the workgroup call this.  ORDERED: every expert's slots in ascending
-  // order (the reduction adds them in that order); otherwise in any order (a copy to every
-  // slot does not care), which all threads fill in at once instead of one wave walking the
-  // table.
-  template <bool ORDERED>
-  __device__ void build(const int* etc, int lo, int n, int own, int epn) {
+  // One wave: where every expert's slots begin in the list, and the list of experts with at least one.
+  // Of an expert's slots at(w, le) come from part w of the table, before: those of the parts in front;
+  // the counts turn into where each part's begin.
+  template <int PARTS, class At>
+  __device__ void prefix(int own, At at) {
     const int lane = threadIdx.x & 63;
-    for (int i = threadIdx.x; i <= own; i += blockDim.x) off[i] = 0;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+    int run = 0, na = 0;
+    if (lane == 0) off[0] = 0;
+    for (int c = 0; c < own; c += 64) {
+      const int le = c + lane;
+      int part[PARTS], cnt = 0;
+#pragma unroll
+      for (int w = 0; w < PARTS; ++w) cnt += part[w] = le < own ? *at(w, le) : 0;
+      const uint64_t m = __ballot(cnt > 0);
+      int incl = 0;
+      if (m) {  // a wave's experts are often all without slots
+        incl = mep_wave_incl_scan(cnt);
+        if (cnt > 0) {
+          active[na + __popcll(m & mep_lanes_lt())] = le;
+          int begin = run + incl - cnt;
+#pragma unroll
+          for (int w = 0; w < PARTS; ++w) { *at(w, le) = begin; begin += part[w]; }
+        }
+        na += __popcll(m);
+      }
+      if (le < own) off[le + 1] = run + incl;
+      run += __builtin_amdgcn_readlane(incl, 63);
+    }
+    if (lane == 0) misc[0] = na;
+  }
+  // All threads of the workgroup call this.  Every expert's slots in any order (a copy to every slot
+  // does not care), as (rank << 16 | slot): the division is done here, once per slot.
+  __device__ void build(const int* etc, int lo, int n, int own, int epn) {
+    for (int i = threadIdx.x; i < own; i += kBlock) cur[i] = 0;
+    for (int i = threadIdx.x; i < n; i += kBlock) {
       const int v = etc[i] - lo;
       e[i] = ((unsigned)v < (unsigned)own) ? v : -1;
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < n; i += blockDim.x)
-      if (e[i] >= 0) atomicAdd(&off[e[i] + 1], 1);
+    for (int i = threadIdx.x; i < n; i += kBlock)
+      if (e[i] >= 0) atomicAdd(&cur[e[i]], 1);
     __syncthreads();
-    if (threadIdx.x < 64) {
-      // exclusive prefix of the counts, list of experts with at least one slot
-      int run = 0, na = 0;
-      for (int c = 0; c < own; c += 64) {
-        const int le = c + lane;
-        const int cnt = le < own ? off[le + 1] : 0;
-        const int incl = mep_wave_incl_scan(cnt);
-        const uint64_t m = __ballot(cnt > 0);
-        if (cnt > 0) active[na + __popcll(m & mep_lanes_lt())] = le;
-        mep_wave_sync();
-        if (le < own) { off[le + 1] = run + incl; cur[le] = run + incl - cnt; }
-        run += __builtin_amdgcn_readlane(incl, 63);
-        na += __popcll(m);
+    if (threadIdx.x < 64) prefix<1>(own, [&](int, int le) { return cur + le; });
+    __syncthreads();
+    for (int i = threadIdx.x; i < n; i += kBlock)
+      if (e[i] >= 0) {
+        const int d = i / epn;
+        list[atomicAdd(&cur[e[i]], 1)] = (d << 16) | (i - d * epn);
       }
-      if (lane == 0) misc[0] = na;
+    __syncthreads();
+  }
+  // The same with every expert's slots rb in ascending order (the reduction adds them in that order).
+  // Three waves take a third of the table each, 64 slots at a time; lanes holding the same expert are
+  // found with one ballot per id bit.  The counts of the second and third wave lie in `spare` [2*own].
+  // One wave for the whole table was slower than a list per rank where tables are large and experts
+  // small, since each doubling of the ranks is a ballot more (us of a launch with no slot in use, list
+  // per rank / one wave / three: 64 ranks of 48 experts 20 / 74 / 10.5, 16 of 48 7.5 / 10.8 / 6.7).
+  static constexpr int kWalkers = 3;
+  __device__ void build_ordered(const int* etc, int lo, int n, int own, int* spare) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int third = (n + 64 * kWalkers - 1) / (64 * kWalkers) * 64;
+    const int beg = wave * third, end = wave < kWalkers ? min(beg + third, n) : beg;
+    auto at = [&](int w, int le) { return (w == 0 ? cur : spare + (w - 1) * own) + le; };
+    constexpr int kAhead = 2;  // loads on their way
+    int v[kAhead];
+    auto load = [&](int c) {
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j) v[j] = c + 64 * j + lane < end ? etc[c + 64 * j + lane] - lo : -1;
+    };
+    load(beg);
+    if (wave < kWalkers)
+      for (int i = lane; i < own; i += 64) *at(wave, i) = 0;
+    mep_wave_sync();
+    for (int c = beg; c < end; c += 64 * kAhead) {
+      if (c > beg) load(c);
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j) {
+        const int i = c + 64 * j + lane;
+        const bool held = (unsigned)v[j] < (unsigned)own;
+        if (i < end) e[i] = held ? v[j] : -1;
+        if (held) atomicAdd(at(wave, v[j]), 1);
+      }
+    }
+    __syncthreads();
+    if (wave == 0) prefix<kWalkers>(own, at);
+    __syncthreads();
+    const int nbits = 32 - __clz(own > 1 ? own - 1 : 1);
+    for (int c = beg; c < end; c += 64) {
+      const int le = c + lane < end ? e[c + lane] : -1;
+      uint64_t same = __ballot(le >= 0);
+      if (!same) continue;
+      for (int b = 0; b < nbits; ++b) {
+        const bool bit = (le >> b) & 1;
+        const uint64_t bb = __ballot(bit);
+        same &= bit ? bb : ~bb;
+      }
+      int first = 0, pos = 0;
+      if (le >= 0) { first = *at(wave, le); pos = __popcll(same & mep_lanes_lt()); }
       mep_wave_sync();
-      if (ORDERED) {
-        // slots in ascending order per expert
-        const int nbits = 32 - __clz(own > 1 ? own - 1 : 1);
-        for (int c = 0; c < n; c += 64) {
-          const int le = c + lane < n ? e[c + lane] : -1;
-          uint64_t same = __ballot(le >= 0);
-          for (int b = 0; b < nbits; ++b) {
-            const bool bit = (le >> b) & 1;
-            const uint64_t bb = __ballot(bit);
-            same &= bit ? bb : ~bb;
-          }
-          int base = 0, pos = 0;
-          if (le >= 0) { base = cur[le]; pos = __popcll(same & mep_lanes_lt()); }
-          mep_wave_sync();
-          if (le >= 0) {
-            if (pos == 0) cur[le] = base + __popcll(same);
-            list[base + pos] = c + lane;
-          }
-          mep_wave_sync();
-        }
+      if (le >= 0) {
+        if (pos == 0) *at(wave, le) = first + __popcll(same);
+        list[first + pos] = c + lane;
       }
+      mep_wave_sync();
     }
     __syncthreads();
-    if (!ORDERED) {
-      // entries as (rank << 16 | slot): the division is done here, once per slot
-      for (int i = threadIdx.x; i < n; i += blockDim.x)
-        if (e[i] >= 0) {
-          const int d = i / epn;
-          list[atomicAdd(&cur[e[i]], 1)] = (d << 16) | (i - d * epn);
-        }
-      __syncthreads();
-    }
   }
 };
 
@@ -170,7 +210,7 @@ __global__ __launch_bounds__(kBlock) void prefetch_kernel(PrefetchArgs a) {
   extern __shared__ int smem[];
   SlotTable t;
   t.carve(smem, a.R * a.epn, a.epn);
-  t.build<false>(a.etc, a.rank * a.epn, a.R * a.epn, a.epn, a.epn);
+  t.build(a.etc, a.rank * a.epn, a.R * a.epn, a.epn, a.epn);
   const unsigned n_active = (unsigned)__builtin_amdgcn_readfirstlane(t.misc[0]);
   if (n_active == 0) return;
   unsigned total = 0;
@@ -508,6 +548,7 @@ struct ReduceArgs {
   const int* etc;
   int rank, epn, R;
   int own;              // experts summed, from rank * epn on: epn, or several ranks'
+  int over, over_half;  // whole experts that all workgroups, or half of them, step over
   unsigned flags;       // MEP_REDUCE_*
 };
 
@@ -520,7 +561,9 @@ constexpr int kMaxReduce = 3;
 // to few ranks (those of the popular ones), and workgroups dealt out by rank left most CUs idle.
 // us, by rank -> one list, three projections of 2048 x 1024, eight ranks of eight experts: seven slots
 // of one rank's experts 215 -> 76.5, five of one and two others 162 -> 77, four ranks' 105 -> 69, one
-// slot 30.5 -> 13, one slot of each rank 102 -> 100 (6.0 TB/s).
+// slot 30.5 -> 13, one slot of each rank 102 -> 100 (6.0 TB/s).  Small experts in large tables, by rank
+// -> one list, three tensors: 16 ranks of 48 experts of 16 KB with all slots in use 35 -> 25, one slot a
+// rank 12.6 -> 10.9; 64 of 48 of 43 KB, all slots 350 -> 158, one a rank 37 -> 23, none 20 -> 10.6.
 struct ReduceBatch {
   float* local_grad[kMaxReduce];
   float* pool[kMaxReduce];
@@ -528,9 +571,13 @@ struct ReduceBatch {
   int64_t elems[kMaxReduce];
   const int* etc;
   int ntensors, rank0, nranks, epn, R;  // local_grad: a block of epn experts per rank
+  int per;                              // ranks of a list; blockIdx.y is the list
+  int over[kMaxReduce], over_half[kMaxReduce];
   unsigned flags;
   __device__ __forceinline__ ReduceArgs of(int t) const {
-    return ReduceArgs{local_grad[t], pool[t], rank_stride[t], elems[t], etc, rank0, epn, R, nranks * epn, flags};
+    const int r = (int)blockIdx.y * per;
+    return ReduceArgs{local_grad[t] + (int64_t)r * epn * elems[t], pool[t], rank_stride[t], elems[t],
+                      etc, rank0 + r, epn, R, min(per, nranks - r) * epn, over[t], over_half[t], flags};
   }
 };
 
@@ -603,18 +650,27 @@ __device__ __forceinline__ void reduce_tensor(const ReduceArgs& a, const SlotTab
   const int nwg = half ? (int)((gridDim.x + 1) / 2) : (int)gridDim.x;
   if ((int)blockIdx.x >= nwg) return;
   const int64_t q = (pieces + work - 1) / work;  // pieces that follow every tile
-  // the workgroups' turns go on from the tensor before, so that none has more than one tile more
-  // than another over all of them
+  // the workgroups' turns go on from the tensor before: of tensors that use the same number of
+  // workgroups none has more than one tile more than another
   int first = (int)blockIdx.x - (int)(before % nwg);
   if (first < 0) first += nwg;
-  int ai = (int)(first / rt.tiles);
-  int64_t tile = first - (int64_t)ai * rt.tiles;
+  // from a tile to the workgroup's next: `over` experts and `on` tiles on
+  const int over = half ? a.over_half : a.over, on = (int)(nwg - over * rt.tiles);
+  int ai = 0, nai;
+  int64_t tile = first, ntile;
+  if (rt.tiles < nwg) {
+    const unsigned tiles = (unsigned)rt.tiles & 0xffffff;  // 24 bits: a short division
+    ai = (int)(((unsigned)first & 0xffffff) / tiles);
+    tile = first - ai * (int)tiles;
+  }
   // grad and first-slot vectors of the tile at hand, requested while the tile before it was
   // still being summed (a workgroup's loads then overlap its own stores)
   mep_f4 pacc[kVecPerThread], pv[kVecPerThread];
   bool ahead = false;
-  for (int64_t w = first; w < work; w += nwg, tile += nwg) {
-    while (tile >= rt.tiles) { tile -= rt.tiles; ++ai; }
+  for (int64_t w = first; w < work; w += nwg, tile = ntile, ai = nai) {
+    nai = ai + over;
+    ntile = tile + on;
+    if (ntile >= rt.tiles) { ntile -= rt.tiles; ++nai; }
     const int le = t.active[ai];
     int step;
     const int64_t o = rt.first(tile, &step);
@@ -645,9 +701,6 @@ __device__ __forceinline__ void reduce_tensor(const ReduceArgs& a, const SlotTab
       }
       // the tile this workgroup takes next
       {
-        int nai = ai;
-        int64_t ntile = tile + nwg;
-        while (ntile >= rt.tiles && nai < n_active) { ntile -= rt.tiles; ++nai; }
         ahead = w + nwg < work && rt.whole(ntile);
         if (ahead) {
           const int nle = t.active[nai];
@@ -725,8 +778,8 @@ __global__ __launch_bounds__(kBlock) void grad_reduce_kernel(ReduceBatch batch) 
   t.carve(smem, entries, a.own);
   int* occ = smem + ints;  // [epn] own slots holding foreign experts, [1] their number
   int64_t* sbase = (int64_t*)(smem + ((ints + a.epn + 2) & ~1));  // [R*epn] byte offset in the pool of list entry i
-  if (threadIdx.x < 64) {
-    const int lane = threadIdx.x;
+  if (threadIdx.x >= 64 * SlotTable::kWalkers) {  // the wave that does not walk the table
+    const int lane = threadIdx.x & 63;
     const int lo = a.rank * a.epn;
     int n = 0;
     for (int c = 0; c < a.epn; c += 64) {
@@ -741,7 +794,7 @@ __global__ __launch_bounds__(kBlock) void grad_reduce_kernel(ReduceBatch batch) 
     }
     if (lane == 0) occ[a.epn] = n;
   }
-  t.build<true>(a.etc, a.rank * a.epn, entries, a.own, a.epn);  // ends with a workgroup barrier
+  t.build_ordered(a.etc, a.rank * a.epn, entries, a.own, (int*)sbase);  // ends with a workgroup barrier
   const int n_active = (a.flags & MEP_REDUCE_CLEAR_ONLY) ? 0 : t.misc[0];
   const int n_clear = (a.flags & MEP_REDUCE_NO_CLEAR) ? 0 : occ[a.epn];
   int64_t before = 0;  // tiles of the tensors before
@@ -907,28 +960,31 @@ int reduce_launch(int ntensors, float* const* local_grad, float* const* reduce_p
     return slot_table_bytes(R * epn, ranks * epn) + ((size_t)epn + 2) * sizeof(int) + (size_t)R * epn * sizeof(int64_t) + 8;
   };
   MEP_REQUIRE(lds_of(1) <= kReduceLdsMax, MEP_ERR_UNSUPPORTED);
-  int chunk = nranks;  // ranks of a launch
-  while (lds_of(chunk) > kReduceLdsMax) chunk = (chunk + 1) / 2;
-  const size_t lds = lds_of(chunk);
+  // Ranks of a list: as many as leave room for two workgroups' tables on a CU.
+  int per = nranks;
+  while (per > 1 && lds_of(per) > 80 * 1024) per = (per + 1) / 2;
+  const int lists = (nranks + per - 1) / per;
+  const size_t lds = lds_of(per);
   if (lds > 64 * 1024) {  // large rank x slot tables: opted in by mep_init_stream_kernels
     const int irc = mep_ensure_init();
     if (irc != MEP_OK) return irc;
   }
-  a.etc = experts_to_copy; a.ntensors = ntensors; a.epn = epn; a.R = R; a.flags = flags;
+  a.etc = experts_to_copy; a.ntensors = ntensors; a.rank0 = rank0; a.nranks = nranks; a.per = per; a.epn = epn; a.R = R;
+  a.flags = flags;
   const int cus = mep_device_cu_count();
   // Persistent workgroups, two per CU (the kernel halves that for a long stream with slots to fill),
   // fewer where all experts together have fewer tiles; three or four per CU lose 3-7 % on a table with
   // many slots.  As many as one expert has tiles, so that all took the same number of them, left most
   // CUs idle in small ones: 16 experts of 1792 x 256, 5 hosted elsewhere, 59.4 -> 20.0 us; 4 of 1024 x
   // 896, 3 hosted elsewhere, 42.3 -> 22.9.
-  const int64_t cap = 2 * (int64_t)(cus > 0 ? cus : 256);
-  for (int r = 0; r < nranks; r += chunk) {
-    a.rank0 = rank0 + r;
-    a.nranks = std::min(chunk, nranks - r);
-    for (int i = 0; i < ntensors; ++i) a.local_grad[i] = local_grad[i] + (int64_t)r * epn * elems_per_expert[i];
-    const int blocks = (int)std::min(cap, tiles * epn * a.nranks);
-    hipLaunchKernelGGL(grad_reduce_kernel, dim3(blocks), dim3(kBlock), lds, (hipStream_t)stream, a);
+  const int64_t cap = std::max<int64_t>(2 * (int64_t)(cus > 0 ? cus : 256) / lists, 1);
+  const int blocks = (int)std::min(cap, tiles * epn * per);
+  for (int i = 0; i < ntensors; ++i) {
+    const SpreadTiles rt(elems_per_expert[i] * 4);
+    a.over[i] = (int)(blocks / rt.tiles);
+    a.over_half[i] = (int)((blocks + 1) / 2 / rt.tiles);
   }
+  hipLaunchKernelGGL(grad_reduce_kernel, dim3(blocks, lists), dim3(kBlock), lds, (hipStream_t)stream, a);
   return mep_launch_status();
 }
 }  // namespace

@@ -105,7 +105,7 @@ def test_views_and_gradient_sums_of_a_group(cuda, R, epn, shapes):
     (4, 3, 36868, 0, 0, 4),      # experts past a 128 KiB block, few experts, the first rank's
     (16, 5, 1028, 15, 9, 7),     # some of the ranks, the last rank's experts
     (4, 2, 256, 1, 2, 2),        # none of theirs
-    (64, 96, 64, 37, 0, 64),     # a table that takes more than one launch
+    (64, 96, 64, 37, 0, 64),     # a table that takes a list for each rank
 ])
 def test_sums_of_several_ranks_where_one_owns_the_hosted_experts(cuda, R, epn, elems, owner, rank0, nranks):
     import ctypes as C
