@@ -293,34 +293,62 @@ struct PullArgs {
 // The occupied slots of the ranks from `rank` on form the work list (slot b <- expert etc[rank, b]);
 // persistent workgroups walk (tensor, occupied slot, tile) in the tile layout of the push kernel, the
 // next tile's loads issued before the current tile's stores.  LDS: slot[nranks*epn] of the list,
-// expert[nranks*epn], n.
+// expert[nranks*epn], each wave's number of them.
 // Several ranks are one list: slots are few, and workgroups dealt out by rank were idle where a rank
 // hosts nothing.  us, by rank -> one list, three projections of 2048 x 1024, eight ranks: slots of one
 // rank 22 -> 10.5, of two 22.8 -> 14.1, three 24 -> 17.8, five 28 -> 25, seven or eight 33 and 35 as before.
+// All four waves read the table, four steps of it on their way: with one wave and a step at a time, 16
+// ranks of 48 experts of 262 KB with a slot a rank 6.4 -> 8.0 (now 6.7), all slots of 8 KB 11 -> 12.9
+// (11.0); only 64 ranks of 48 experts of 8 KB stay dearer, a slot a rank 4.8 -> 12.4 (6.4).
 __global__ __launch_bounds__(kBlock) void prefetch_pull_kernel(PullArgs a) {
   extern __shared__ int smem[];
   const int entries = a.nranks * a.epn;
-  int* s_slot = smem;
+  int* s_slot = smem;  // rank << 16 | slot: there are at most 8191
   int* s_exp = smem + entries;
-  int* s_n = s_exp + entries;
-  if (threadIdx.x < 64) {
-    const int lane = threadIdx.x;
-    int n = 0;
-    for (int c = 0; c < entries; c += 64) {
-      const int b = c + lane;
-      const int e = b < entries ? a.etc[a.rank * a.epn + b] : -1;
-      const bool ok = e >= 0 && e < a.R * a.epn;
-      const uint64_t m = __ballot(ok);
-      if (ok) {
-        const int i = n + __popcll(m & mep_lanes_lt());
-        s_slot[i] = b; s_exp[i] = e;
-      }
-      n += __popcll(m);
+  uint16_t* s_n = (uint16_t*)(s_exp + entries);
+  // a quarter of the table to a wave
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int quarter = (entries + kBlock - 1) / kBlock * 64;
+  const int beg = wave * quarter, end = min(beg + quarter, entries);
+  constexpr int kAhead = 4;  // loads on their way
+  int e[kAhead], n = 0;
+  auto fetch = [&](int c) {
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      const int i = c + 64 * j + lane, v = i < end ? a.etc[a.rank * a.epn + i] : -1;
+      e[j] = v < a.R * a.epn ? v : -1;
     }
-    if (lane == 0) *s_n = n;
+  };
+  const int steps = (quarter + 64 * kAhead - 1) / (64 * kAhead);
+  for (int k = 0; k < steps; ++k) {
+    fetch(beg + 64 * kAhead * k);
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) n += __popcll(__ballot(e[j] >= 0));
+  }
+  if (lane == 0) s_n[wave] = (uint16_t)n;
+  __syncthreads();
+  int at = 0, all = 0;
+#pragma unroll
+  for (int w = 0; w < kBlock / 64; ++w) {
+    if (w == wave) at = all;
+    all += s_n[w];
+  }
+  for (int k = steps - 1; k >= 0; --k) {  // the last step's are there
+    if (k < steps - 1) fetch(beg + 64 * kAhead * k);
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      const uint64_t m = __ballot(e[j] >= 0);
+      if (!m) continue;
+      if (e[j] >= 0) {
+        const int i = at + __popcll(m & mep_lanes_lt()), b = beg + 64 * (kAhead * k + j) + lane, r = b / a.epn;
+        s_slot[i] = r << 16 | (b - r * a.epn);
+        s_exp[i] = e[j];
+      }
+      at += __popcll(m);
+    }
   }
   __syncthreads();
-  const unsigned n_slots = (unsigned)__builtin_amdgcn_readfirstlane(*s_n);
+  const unsigned n_slots = (unsigned)__builtin_amdgcn_readfirstlane(all);
   if (n_slots == 0) return;
   unsigned total = 0;
   for (int ti = 0; ti < a.ntensors; ++ti) total += (unsigned)a.st[ti].tiles * n_slots;
@@ -352,7 +380,7 @@ __global__ __launch_bounds__(kBlock) void prefetch_pull_kernel(PullArgs a) {
   };
   auto store = [&](const Tile& p, const mep_u4* v) {
     const int64_t bytes = a.st[p.ti].bytes;
-    const int r = p.b / a.epn, b = p.b - r * a.epn;
+    const int r = p.b >> 16, b = p.b & 0xffff;
     char* dst = a.pool[p.ti] + (int64_t)(a.rank + r) * a.rank_stride[p.ti] + (int64_t)b * bytes + p.off;
     if (p.whole) {
 #pragma unroll
@@ -854,7 +882,7 @@ int pull_launch(int ntensors, const void* const* owners, const int64_t* owner_st
   MEP_REQUIRE(ntensors > 0 && ntensors <= kMaxTensors, MEP_ERR_INVALID_ARG);
   MEP_REQUIRE(epn > 0 && R > 0 && nranks > 0 && rank >= 0 && rank + nranks <= R, MEP_ERR_INVALID_ARG);
   // ranks of a launch: the list of slots in LDS and the 32 bits that number (tensor, slot, tile)
-  auto lds_of = [&](int ranks) { return (2 * (size_t)ranks * epn + 1) * sizeof(int); };
+  auto lds_of = [&](int ranks) { return (2 * (size_t)ranks * epn + 2) * sizeof(int); };
   MEP_REQUIRE(lds_of(1) <= 64 * 1024, MEP_ERR_UNSUPPORTED);
   PullArgs a;
   a.ntensors = ntensors; a.rank = rank; a.epn = epn; a.R = R; a.etc = experts_to_copy;

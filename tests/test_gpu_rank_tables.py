@@ -1,4 +1,4 @@
-"""Sums of several ranks' slots where the table is large: more than one list of ranks (and a
+"""Sums and copies of several ranks' slots where the table is large: more than one list of ranks (and a
 last one of fewer), more entries than a wave has lanes, experts in many slots, experts of less than a
 tile, so that a workgroup's next tile lies several experts on."""
 
@@ -49,3 +49,28 @@ def test_sums(cuda, R, epn, rank0, nranks, used):
     torch.cuda.synchronize()
     for a, b, c, d in zip(got, want, slots, pool):
         assert torch.equal(a.cpu(), b) and torch.equal(c.cpu(), d)
+
+
+@pytest.mark.parametrize("R,epn,rank0,nranks", [(64, 48, 0, 64), (64, 48, 3, 41), (16, 48, 0, 16), (3, 67, 1, 2),
+                                                (16, 17, 0, 16)])
+@pytest.mark.parametrize("used", [0.0, 0.02, 1.0])
+def test_copies(cuda, R, epn, rank0, nranks, used):
+    print(f"slots of ranks {rank0} + {nranks} of {R}, {epn} experts, {used} of them", flush=True)
+    g = torch.Generator().manual_seed(R + epn + nranks)
+    etc = _table(R, epn, used, g)
+    nbytes = 1040
+    local = torch.randint(0, 256, (R * epn, nbytes), dtype=torch.uint8, generator=g)
+    want = torch.randint(0, 256, (R, epn, nbytes), dtype=torch.uint8, generator=g)
+    src, got = local.to(cuda), want.to(cuda)
+    there = etc >= 0
+    there[:rank0] = False
+    there[rank0 + nranks:] = False
+    want[there] = local[etc[there].long()]
+    etc = etc.to(cuda)
+    arr_p, arr_i = C.c_void_p * 1, C.c_int64 * 1
+    stride = arr_i(epn * nbytes)
+    rc = _lib.lib().mep_prefetch_pull_ranks(1, arr_p(src.data_ptr()), stride, arr_p(got.data_ptr()), stride, arr_i(nbytes),
+                                            etc.data_ptr(), rank0, nranks, epn, R, _lib.current_stream())
+    _lib.check(rc, "mep_prefetch_pull_ranks")
+    torch.cuda.synchronize()
+    assert torch.equal(got.cpu(), want)
