@@ -1204,14 +1204,6 @@ bool for_ranks(GemmArgs& a, int nranks) {
 // mep_set_gemm_row_tile(128 or 256) forces one side (tests run both on small shapes).
 std::atomic<int> g_forced_row_tile{0};
 
-// how the streaming kernel would cut the N columns of `blocks` row blocks: rounds, units of a tile
-struct Streamed { int64_t turns, units; };
-Streamed streamed(int N, int64_t blocks, int64_t cus) {
-  const int64_t all = N / 64, least = (all + kSUnitsKn - 1) / kSUnitsKn;
-  const int64_t turns = (blocks * least + cus - 1) / cus, per = std::min(all, turns * cus / blocks);
-  return {turns, (all + per - 1) / per};
-}
-
 bool use_256_tiles(const GemmArgs& a, bool forward, bool kn) {
   const bool ranks = a.G != a.Gr;
   if (ranks && (!kn || a.G / a.Gr > 64)) return true;  // the streaming kernel has a lane for each
@@ -1223,25 +1215,14 @@ bool use_256_tiles(const GemmArgs& a, bool forward, bool kn) {
   const int64_t cus = std::max(mep_device_cu_count(), 8);
   const int64_t blocks = std::max<int64_t>(a.G / 2 + 1, rows / kBM + a.G / 4);
   const int64_t tiles = row_tiles_256(a) * a.ntiles, rounds = (tiles + cus - 1) / cus;
-  if (ranks) {
-    // Several ranks' input gradients: what either kernel makes of the time of a backward pass, in us (of both
-    // pairs, with what it costs the weight gradients behind it), fitted to 820 products of 4 to 1000 blocks of 8
-    // to 1024 groups (2 to 16 ranks), 256 .. 5120 by 256 .. 5120 (off by 10 %).  Unlike a single rank's below,
-    // the weights' bytes count (a group's are read by its few tiles alone) and the rows'.  550 passes, 140 of
-    // them not in the fit, are 0.5 % slower so than with the faster kernel for each product; streaming
-    // throughout 3, 256 x 256 throughout 12, streaming where blocks < groups and experts are at most
-    // 2048 x 1024 4.  Times of the products, us, streaming / 256 x 256 tiles, dy * down and both pairs: 8 ranks,
-    // 128 groups of 2048 x 1024 with 75 blocks 80 / 100, 161 / 179, with 100 92 / 109, 198 / 187, with 293
-    // 238 / 157, 569 / 324; 64 groups of 1024 x 512 with 37 18 / 25, 28 / 29, with 169 43 / 32, 80 / 62; 2 ranks,
-    // 8 groups of 512 x 256 with 12 9 / 17, 8 / 18, 4096 x 2048 with 9 47 / 81, 69 / 87; 4 ranks, 64 groups of
-    // 4096 x 2048 with 40 140 / 171, 281 / 306; 16 ranks, 512 of 768 x 768 with 275 98 / 99, 200 / 216.
-    const double pairs = a.A2 ? 2 : 1, steps = a.K / kBK * pairs;
-    const int64_t filled = std::min<int64_t>(a.G / 2 + a.G / 16 + 1, blocks);
-    const double weights = 2e-6 * filled * a.N * a.K * pairs, passed = 2e-6 * blocks * kBM * (a.K * pairs + a.N);  // MB
-    const Streamed s = streamed(a.N, blocks, cus);
-    return 1.4 + 6.1 * rounds + steps * (0.47 * tiles / cus + 0.8 * rounds) + 0.055 * weights + 0.089 * passed <
-           s.turns * (5.3 + 0.64 * s.units + steps * (0.216 + 0.204 * s.units)) + 0.066 * weights;
-  }
+  // Several ranks' input gradients: groups are many and tiles fill the chip either way; with less than
+  // a block a group most 256-row tiles are half empty.  us, backward pass (weight gradients included),
+  // streaming / 256 x 256: 8 ranks, 128 groups of 2048 x 1024 with 71 blocks 581 / 634, 95 676 / 721,
+  // 163 990 / 905; 16 ranks, 384 of 768 x 768 with 205 591 / 620, 512 of 1024 x 512 with 269 709 / 753;
+  // 4 ranks, 32 of 512 x 256 with 19 40 / 50; 8 ranks, 64 of 1024 x 512 with 38 115 / 111.  Forward
+  // passes of these: 246 / 252, 298 / 278, 535 / 358, 257 / 230, 311 / 274, 21 / 24, 52 / 38.
+  // Experts of more than 2048 x 1024 were not compared and stay.
+  if (ranks) return blocks >= a.G || (int64_t)a.N * a.K > 2048 * 1024;
   if (kn) {
     // Input gradients: the time of either kernel in 10 ns, fitted to 172 products of 4 to 96 blocks of 8 to
     // 96 groups, 256 .. 5632 by 256 .. 5632 (off by 9 and 12 %).  A round of streaming tiles of n units costs
@@ -1250,9 +1231,11 @@ bool use_256_tiles(const GemmArgs& a, bool forward, bool kn) {
     // 82 / 162; 12 of 1024 x 1024 13 / 20, 21 / 36; 17 of 2048 x 4096 68 / 85, 117 / 159; 24 of 2048 x 4096
     // in 13 groups 88 / 56, 155 / 104; 96 of 1024 x 1024 52 / 34, 80 / 61.
     const int64_t steps = (int64_t)a.K / kBK * (a.A2 ? 2 : 1);
-    const Streamed s = streamed(a.N, blocks, cus);
+    const int64_t units = a.N / 64, least = (units + kSUnitsKn - 1) / kSUnitsKn;
+    const int64_t turns = (blocks * least + cus - 1) / cus, per = std::min(units, turns * cus / blocks);
+    const int64_t n = (units + per - 1) / per;
     return 200 + 600 * rounds + steps * (90 * rounds + 64 * std::min(tiles, cus) / cus) <
-           s.turns * (600 + 100 * s.units + steps * (24 + 22 * s.units));
+           turns * (600 + 100 * n + steps * (24 + 22 * n));
   }
   // Forward products: what a K step costs either kernel.  The local experts (half of the groups)
   // and a slot or two have rows, the last block of each about half filled.  A round of 256 x 256
