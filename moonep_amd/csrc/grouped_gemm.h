@@ -114,11 +114,12 @@ __device__ __forceinline__ uint32_t mep_cvt_bf16x2(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
 }
 
-// Four K rows of a column block, transposed (see mep_tr_pair).  As an instruction of its own: in
-// front of the builtin the compiler waits for every load straight into LDS that is in flight.  The
-// result is there after the next wait for lgkmcnt(0); nothing may touch it before.  The compiler does
-// not know that: the build reads its assembly and fails where a register of a load in an asm
-// statement is touched before its wait, or where anything is spilled (moonep_amd/asm_waits.py).
+// Four K rows of a column block, transposed: sixteen lanes read a 4 x 16 block, 8 bytes of a row each,
+// and each receives one of its columns.  As an instruction of its own: in front of the builtin the
+// compiler waits for every load straight into LDS that is in flight.  The result is there after the next
+// wait for lgkmcnt(0); nothing may touch it before.  The compiler does not know that: the build reads its
+// assembly and fails where a register of a load in an asm statement is touched before its wait, or where
+// anything is spilled (moonep_amd/asm_waits.py).
 template <class T>
 __device__ __forceinline__ void mep_tr_issue(T& x, uint32_t lds, int offset) {
   asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(x) : "v"(lds), "n"(offset));

@@ -1215,13 +1215,16 @@ bool use_256_tiles(const GemmArgs& a, bool forward, bool kn) {
   const int64_t cus = std::max(mep_device_cu_count(), 8);
   const int64_t blocks = std::max<int64_t>(a.G / 2 + 1, rows / kBM + a.G / 4);
   const int64_t tiles = row_tiles_256(a) * a.ntiles, rounds = (tiles + cus - 1) / cus;
-  // Several ranks' input gradients: groups are many and tiles fill the chip either way; with less than
-  // a block a group most 256-row tiles are half empty.  us, backward pass (weight gradients included),
-  // streaming / 256 x 256: 8 ranks, 128 groups of 2048 x 1024 with 71 blocks 581 / 634, 95 676 / 721,
-  // 163 990 / 905; 16 ranks, 384 of 768 x 768 with 205 591 / 620, 512 of 1024 x 512 with 269 709 / 753;
-  // 4 ranks, 32 of 512 x 256 with 19 40 / 50; 8 ranks, 64 of 1024 x 512 with 38 115 / 111.  Forward
-  // passes of these: 246 / 252, 298 / 278, 535 / 358, 257 / 230, 311 / 274, 21 / 24, 52 / 38.
-  // Experts of more than 2048 x 1024 were not compared and stay.
+  // Several ranks' input gradients: with less than a block a group most 256-row tiles are half empty.  us,
+  // backward pass (weight gradients included), streaming / 256 x 256: 8 ranks, 128 groups of 2048 x 1024
+  // with 71 blocks 586 / 646, 99 697 / 723, 165 1003 / 916; 16 ranks, 384 of 768 x 768 with 205 617 / 641, 512
+  // of 1024 x 512 with 275 724 / 749; 4 ranks, 32 of 512 x 256 with 20 41 / 51; even at 8 ranks, 64 of
+  // 1024 x 512 with 41 and 43 126 / 123, 129 / 131.  By the kernels' times, 373 sizes with less than a block
+  // a group are 0.7 % off the faster kernel for each product, on 256 x 256 tiles 12 %.  Forward passes,
+  // which stay: 246 / 252, 298 / 278, 535 / 358, 257 / 230, 311 / 274, 21 / 24, 52 / 38.
+  // Neither bound is where the kernels cross: larger experts and more blocks stay with the 256 x 256 tiles,
+  // which are the faster ones for many blocks (4096 x 1024, 128 groups with 164, products 200 and 392 against
+  // 254 and 625) and lose where tiles are few (8 groups of 512 x 256 with 12, 17 and 18 against 9 and 8).
   if (ranks) return blocks >= a.G || (int64_t)a.N * a.K > 2048 * 1024;
   if (kn) {
     // Input gradients: the time of either kernel in 10 ns, fitted to 172 products of 4 to 96 blocks of 8 to
@@ -1424,7 +1427,8 @@ extern "C" int mep_grouped_gemm_wgrad(const void* At, const void* Bt, const int3
   a.skip_from = skip_empty_from;
   a.split = G;
   a.Gr = G;
-  // an expert's shapes: 256 x 256 tiles (whose lane offsets are 32 bits)
+  // an expert's shapes: 256 x 256 tiles (whose lane offsets are 32 bits).  Groups are experts and as many
+  // slots everywhere here, so G is even; the list of tiles would take an odd number, which was not compared.
   if (Ma % kPT == 0 && Nb % kPT == 0 && G % 2 == 0 && (uintptr_t)C % 16 == 0 && ld < ((int64_t)1 << 22)) {
     WgradMap map{};
     map.n = 1;

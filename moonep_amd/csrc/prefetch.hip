@@ -32,8 +32,7 @@ struct SlotTable {
     active = cur + own; misc = active + own;
   }
   // One wave: where every expert's slots begin in the list, and the list of experts with at least one.
-  // Of an expert's slots at(w, le) come from part w of the table, before: those of the parts in front;
-  // the counts turn into where each part's begin.
+  // at(w, le) is how many of the expert's slots part w of the table holds; it becomes where these begin.
   template <int PARTS, class At>
   __device__ void prefix(int own, At at) {
     const int lane = threadIdx.x & 63;

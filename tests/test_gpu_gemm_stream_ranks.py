@@ -68,3 +68,40 @@ def test_same_bits_as_the_256_row_kernels(cuda, ranks, H, Hp, slots):
         assert not y[r, end:].any() and not drows[r, end:].any()
         if end:
             assert y[r, :end].any()
+
+
+# ranks, experts of a rank, blocks of each of a rank's experts, H, H', does the streaming kernel run
+@pytest.mark.parametrize("n,epn,each,H,Hp,streaming", [(4, 2, 1, 512, 256, True),      # less than a block a group
+                                                       (4, 2, 2, 512, 256, False),
+                                                       (2, 2, 1, 2048, 1024, True),
+                                                       (2, 2, 1, 2304, 1024, False)])  # larger experts
+def test_the_kernel_of_these_sizes(cuda, n, epn, each, H, Hp, streaming):
+    """Which kernel brings both input gradients is a rule on sizes; the result is the other's to the bit."""
+    print(f"{n} ranks of {epn} experts, {each} blocks each, {H} x {Hp}", flush=True)
+    G, M = 2 * epn, 128 * (each * epn + 2 * epn)
+    g = torch.Generator(device="cuda").manual_seed(n)
+
+    def normal(*shape):
+        return torch.randn(*shape, device=cuda, generator=g).to(torch.bfloat16)
+
+    rows, dy, gate, up, down = normal(n, M, H), normal(n, M, H), normal(n, G, Hp, H), normal(n, G, Hp, H), normal(n, G, H, Hp)
+    cu = (128 * each * (torch.arange(G, device=cuda) + 1).clamp(max=epn)).to(torch.int32).expand(n, G).contiguous()
+    lib, p, s = _lib.lib(), _lib.ptr, _lib.current_stream()
+    drows = []
+    for tile in (0, 256 if streaming else 128):
+        mid = [normal(n, M, Hp) * 0 for _ in range(6)]
+        out = normal(n, M, H)
+        grads = [[torch.zeros(n, epn, *shape, device=cuda) for shape in ((Hp, H), (Hp, H), (H, Hp))] for _ in range(2)]
+        lib.mep_set_gemm_row_tile(tile)
+        try:
+            with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+                _lib.check(lib.mep_ffn_backward(
+                    p(dy), p(rows), None, p(cu), G, p(gate), p(up), p(down), p(rows), p(dy), *map(p, mid[:4]), None, p(out),
+                    *((ctypes.c_void_p * 3)(*map(p, t)) for t in grads), epn, n, M, H, Hp, G, s), "mep_ffn_backward")
+                torch.cuda.synchronize()
+        finally:
+            lib.mep_set_gemm_row_tile(0)
+        seen = sum(e.count for e in prof.key_averages() if "gemm_stream_kernel" in e.key)
+        assert seen == (2 if streaming == (tile == 0) else 0)
+        drows.append(out)
+    assert torch.equal(*drows) and drows[0].any()
