@@ -31,9 +31,14 @@ def test_bits_of_the_256_kernels(cuda, blocks, G, N, K):
     out = []
     for tile in (128, 256):
         _lib.check(_lib.lib().mep_set_gemm_row_tile(tile), "mep_set_gemm_row_tile")
-        out.append((ffn.launch_grouped_gemm_nn(a1, w1, ends), ffn.launch_grouped_gemm_nn(a1, w1, ends, row_scale=scale),
-                    ffn.launch_grouped_gemm_dual_nn(a1, w1, a2, w2, ends)))
-        torch.cuda.synchronize()
+        plain, scaled = (torch.full((M, N), 7.0, dtype=torch.bfloat16, device=cuda) for _ in range(2))
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+            ffn.launch_grouped_gemm_nn(a1, w1, ends, out=plain)
+            ffn.launch_grouped_gemm_nn(a1, w1, ends, out=scaled, row_scale=scale)
+            out.append((plain, scaled, ffn.launch_grouped_gemm_dual_nn(a1, w1, a2, w2, ends)))
+            torch.cuda.synchronize()
+        assert sum(e.count for e in prof.key_averages() if "gemm_stream_kernel" in e.key) == (3 if tile == 128 else 0)
     for what, x, y in zip(("plain", "scaled", "both pairs"), *out):
         assert torch.equal(x, y), what
     assert bool(out[0][0][:128 * blocks].any()) and not bool(out[0][2][128 * blocks:].any())
+    assert all(bool((x[128 * blocks:] == 7.0).all()) for x in out[0][:2])   # rows behind the last group

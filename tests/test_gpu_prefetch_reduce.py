@@ -416,3 +416,39 @@ def test_grad_reduce_batch_of_different_sizes_matches_oracle(cuda, shapes, plan)
         oo.grad_reduce(local[i], pools[i], etc, rank)
         assert torch.equal(dev_local[i].cpu().view(torch.int32), local[i].view(torch.int32)), f"sums of tensor {i}"
         assert torch.equal(dev_pools[i].cpu().view(torch.int32), pools[i].view(torch.int32)), f"slots of tensor {i}"
+
+
+@pytest.mark.parametrize("sizes", [(102400, 3407872, 40960), (3407872, 40960, 102400), (40960, 102400, 3407872)])
+def test_grad_reduce_batch_where_one_tensor_takes_half_of_the_workgroups(cuda, sizes):
+    """Slots are cleared beside the sums, and one of the three tensors (13.6 MB an expert, more than 384 MB
+    with its slots and clears) is summed by half of the workgroups, the others by all of them."""
+    import ctypes
+
+    from moonep_amd import _lib
+
+    print(f"grad_reduce halves {sizes}", flush=True)
+    R, epn, rank, n = 3, 8, 1, 3
+    lo = rank * epn
+    etc = torch.full((R, epn), -1, dtype=torch.int32)
+    etc[0] = torch.arange(lo, lo + epn)                                       # every expert of the rank at a peer
+    etc[rank] = torch.tensor([0, 1, 2, lo + 3, 4, 17, -1, 23])                # foreign, one own, one free
+    etc[2, 5] = lo + 3                                                        # an expert in three slots
+    g = torch.Generator(device=cuda).manual_seed(7)
+    local = [torch.randn(epn, s, device=cuda, generator=g) for s in sizes]
+    pools = [torch.randn(R, epn, s, device=cuda, generator=g) for s in sizes]
+    sums, after = [t.clone() for t in local], [t.clone() for t in pools]
+    for t, p, q in zip(sums, pools, after):
+        for d, b in (etc >= 0).nonzero().tolist():      # ascending, in fp32
+            if 0 <= int(etc[d, b]) - lo < epn:
+                t[int(etc[d, b]) - lo] += p[d, b]
+        q[rank, etc[rank].to(cuda) >= 0] = 0.0
+    etc_dev = etc.to(cuda)
+    rc = _lib.lib().mep_grad_reduce_batch(
+        n, (ctypes.c_void_p * n)(*[t.data_ptr() for t in local]), (ctypes.c_void_p * n)(*[t.data_ptr() for t in pools]),
+        (ctypes.c_int64 * n)(*[epn * s for s in sizes]), (ctypes.c_int64 * n)(*sizes), etc_dev.data_ptr(), rank, 1, epn, R, 0,
+        _lib.current_stream())
+    _lib.check(rc, "mep_grad_reduce_batch")
+    torch.cuda.synchronize()
+    for i in range(n):
+        assert torch.equal(local[i], sums[i]), f"sums of tensor {i}"
+        assert torch.equal(pools[i], after[i]), f"slots of tensor {i}"

@@ -1,10 +1,13 @@
 """Tile list of the weight gradients: products with fewer tiles than XCDs, numbers of tiles and groups that
-eight does not divide, three products in one launch, and more tiles than one workgroup lists."""
+eight does not divide, three products in one launch, several ranks' groups, and more tiles than one workgroup
+lists."""
+
+import ctypes
 
 import pytest
 import torch
 
-from moonep_amd import ffn
+from moonep_amd import _lib, ffn
 
 pytestmark = pytest.mark.gpu
 
@@ -59,6 +62,52 @@ def test_three_products_of_a_backward_are_the_single_ones(cuda, H, Hp, G):
     torch.cuda.synchronize()
     for what, a, b, c in zip(("gate", "up", "down"), (dg, du, dy), (rows, rows, hs), got):
         assert torch.equal(ffn.launch_grouped_gemm_wgrad_tn(a, b, ends), c), what
+
+
+# row blocks of each rank's groups: ends that differ between the ranks, empty groups on either side of the split
+RANKS = {"three": ((3, 0, 1, 2, 0, 1), (0, 0, 1, 1, 2, 0), (1, 2, 0, 0, 0, 0)),
+         "eleven": tuple(tuple((r + 3 * i) % 5 % 3 for i in range(10)) for r in range(11))}
+
+
+@pytest.mark.parametrize("ranks", list(RANKS))
+@pytest.mark.parametrize("H,Hp", [(768, 512), (2560, 1280), (256, 1024)])
+def test_several_ranks_are_the_single_ones(cuda, ranks, H, Hp):
+    """Each rank's six tensors of one backward call of all ranks: its own experts' and its slots', of
+    which the empty ones are left as they are."""
+    heights = RANKS[ranks]
+    n, G, M = len(heights), len(heights[0]), 128 * (max(map(sum, heights)) + 1)
+    split = G // 2
+    print(f"backward of {n} ranks {H}x{Hp}, {G} groups", flush=True)
+    g = torch.Generator(device=cuda).manual_seed(H + Hp + n)
+
+    def normal(*shape, scale=1.0):
+        return (torch.randn(*shape, device=cuda, generator=g) * scale).to(torch.bfloat16)
+
+    rows, dy = normal(n, M, H), normal(n, M, H)
+    gate, up = (normal(n, G, Hp, H, scale=H ** -0.5) for _ in range(2))
+    down = normal(n, G, H, Hp, scale=Hp ** -0.5)
+    gate_pre, up_pre = normal(n, M, Hp), normal(n, M, Hp)
+    cu = torch.tensor([[128 * sum(h[:i + 1]) for i in range(G)] for h in heights], dtype=torch.int32, device=cuda)
+    scale = torch.rand(n, M, device=cuda, generator=g) + 0.1
+    dh, dgate, dup, hs = (torch.zeros(n, M, Hp, dtype=torch.bfloat16, device=cuda) for _ in range(4))
+    drows, dslots = torch.zeros(n, M, H, dtype=torch.bfloat16, device=cuda), torch.zeros(n, M, device=cuda)
+    shapes = ((Hp, H), (Hp, H), (H, Hp))
+    grads = [[torch.full((n, k, *s), -3.0, device=cuda) for s in shapes] for k in (split, G - split)]
+    p = _lib.ptr
+    _lib.check(_lib.lib().mep_ffn_backward(
+        p(dy), p(rows), p(scale), p(cu), G, p(gate), p(up), p(down), p(gate_pre), p(up_pre), p(dh), p(dgate), p(dup), p(hs),
+        p(dslots), p(drows), *((ctypes.c_void_p * 3)(*map(p, t)) for t in grads), split, n, M, H, Hp, split,
+        _lib.current_stream()), "mep_ffn_backward")
+    torch.cuda.synchronize()
+    for r, lens in enumerate(heights):
+        for k, (x1, x2) in enumerate(((dgate, rows), (dup, rows), (dy, hs))):
+            one = torch.full((G, *shapes[k]), -3.0, device=cuda)
+            ffn.launch_grouped_gemm_wgrad_tn(x1[r], x2[r], cu[r], one, skip_empty_from=split)
+            got = torch.cat([grads[0][k][r], grads[1][k][r]])
+            assert torch.equal(got, one), (r, k)
+            for i, blocks in enumerate(lens):
+                kept = bool((got[i] == -3.0).all())
+                assert kept == (blocks == 0 and i >= split) and bool(got[i].any()) == (blocks > 0 or kept), (r, k, i)
 
 
 def test_more_tiles_than_a_workgroup_lists(cuda):
