@@ -575,7 +575,6 @@ struct ReduceArgs {
   const int* etc;
   int rank, epn, R;
   int own;              // experts summed, from rank * epn on: epn, or several ranks'
-  int over, over_half;  // whole experts that all workgroups, or half of them, step over
   unsigned flags;       // MEP_REDUCE_*
 };
 
@@ -599,12 +598,11 @@ struct ReduceBatch {
   const int* etc;
   int ntensors, rank0, nranks, epn, R;  // local_grad: a block of epn experts per rank
   int per;                              // ranks of a list; blockIdx.y is the list
-  int over[kMaxReduce], over_half[kMaxReduce];
   unsigned flags;
   __device__ __forceinline__ ReduceArgs of(int t) const {
     const int r = (int)blockIdx.y * per;
     return ReduceArgs{local_grad[t] + (int64_t)r * epn * elems[t], pool[t], rank_stride[t], elems[t],
-                      etc, rank0 + r, epn, R, min(per, nranks - r) * epn, over[t], over_half[t], flags};
+                      etc, rank0 + r, epn, R, min(per, nranks - r) * epn, flags};
   }
 };
 
@@ -682,22 +680,25 @@ __device__ __forceinline__ void reduce_tensor(const ReduceArgs& a, const SlotTab
   int first = (int)blockIdx.x - (int)(before % nwg);
   if (first < 0) first += nwg;
   // from a tile to the workgroup's next: `over` experts and `on` tiles on
-  const int over = half ? a.over_half : a.over, on = (int)(nwg - over * rt.tiles);
-  int ai = 0, nai;
-  int64_t tile = first, ntile;
+  int over = 0, on = nwg, ai = 0;
+  int64_t tile = first;
   if (rt.tiles < nwg) {
     const unsigned tiles = (unsigned)rt.tiles & 0xffffff;  // 24 bits: a short division
+    over = (int)(((unsigned)nwg & 0xffffff) / tiles);
+    on = nwg - over * (int)tiles;
     ai = (int)(((unsigned)first & 0xffffff) / tiles);
     tile = first - ai * (int)tiles;
   }
+  auto next = [&](int& expert, int64_t& t) {
+    expert += over;
+    t += on;
+    if (t >= rt.tiles) { t -= rt.tiles; ++expert; }
+  };
   // grad and first-slot vectors of the tile at hand, requested while the tile before it was
   // still being summed (a workgroup's loads then overlap its own stores)
   mep_f4 pacc[kVecPerThread], pv[kVecPerThread];
   bool ahead = false;
-  for (int64_t w = first; w < work; w += nwg, tile = ntile, ai = nai) {
-    nai = ai + over;
-    ntile = tile + on;
-    if (ntile >= rt.tiles) { ntile -= rt.tiles; ++nai; }
+  for (int64_t w = first; w < work; w += nwg, next(ai, tile)) {
     const int le = t.active[ai];
     int step;
     const int64_t o = rt.first(tile, &step);
@@ -728,6 +729,9 @@ __device__ __forceinline__ void reduce_tensor(const ReduceArgs& a, const SlotTab
       }
       // the tile this workgroup takes next
       {
+        int nai = ai;
+        int64_t ntile = tile;
+        next(nai, ntile);
         ahead = w + nwg < work && rt.whole(ntile);
         if (ahead) {
           const int nle = t.active[nai];
@@ -1006,11 +1010,6 @@ int reduce_launch(int ntensors, float* const* local_grad, float* const* reduce_p
   // 896, 3 hosted elsewhere, 42.3 -> 22.9.
   const int64_t cap = std::max<int64_t>(2 * (int64_t)(cus > 0 ? cus : 256) / lists, 1);
   const int blocks = (int)std::min(cap, tiles * epn * per);
-  for (int i = 0; i < ntensors; ++i) {
-    const SpreadTiles rt(elems_per_expert[i] * 4);
-    a.over[i] = (int)(blocks / rt.tiles);
-    a.over_half[i] = (int)((blocks + 1) / 2 / rt.tiles);
-  }
   hipLaunchKernelGGL(grad_reduce_kernel, dim3(blocks, lists), dim3(kBlock), lds, (hipStream_t)stream, a);
   return mep_launch_status();
 }
