@@ -125,102 +125,224 @@ __device__ __forceinline__ void mep_tr_issue(T& x, uint32_t lds, int offset) {
   asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(x) : "v"(lds), "n"(offset));
 }
 
-// Tile list of the weight gradients.  A group's T tiles, those of a row of the longer dimension behind
-// each other, are cut into eight runs of T / 8, and XCD x takes the run (x + group) mod 8: all XCDs
-// finish together whatever the groups' lengths (slots are often empty) and however few tiles an expert
-// has, and the tiles an XCD runs at one time lie in few rows and columns of one group.  (With whole rows
-// to an XCD the 3 x 3 tiles of 768 x 768 went to four of the eight: 192 such experts on 16 ranks of 692
-// tokens, K = 8, all three products 1140 -> 654 us.)  In eight consecutive groups every XCD has T tiles,
-// and its place among them is found without a table: it walks the runs x, x + 1, ... x + 7; run v begins
-// at v T / 8, from 8 on run v - 8 counted T further.
-// Up to three products whose outputs are M x N or N x M (the projections of an expert) are one list,
-// one product behind the other.
+// n / d for n >= 0, d > 0, in half the instructions of the general division (what a kernel runs once waits for its
+// instructions to be fetched): the quotient in fp32, that of what it leaves, and at most one more
+__device__ __forceinline__ int mep_quotient(int n, int d) {
+  const float inv = __builtin_amdgcn_rcpf((float)d);
+  int q = (int)((float)n * inv);
+  q += (int)((float)(n - q * d) * inv);
+  const int rest = n - q * d;
+  return q + (rest >= d) - (rest < 0);
+}
+
+// Tile list of the weight gradients: group by group (those with rows), a group's products (up to three, whose
+// outputs are M x N or N x M: the projections of an expert) behind each other, a product in bands of about four
+// tiles of the shorter dimension, a band row by row.  A group's T tiles are cut into eight runs of T / 8, and of
+// the k-th group XCD x takes the run (x + k) mod 8: all XCDs finish together whatever the groups' lengths and
+// however few tiles an expert has, the longest groups (local experts come first) early, and the tiles that an XCD
+// runs at one time are neighbours in one group, which all XCDs work on at that time.  In eight consecutive groups
+// every XCD has T tiles, and its place among them is found without a table: it walks the runs x, x + 1, ...
+// x + 7; run v begins at v T / 8, from 8 on run v - 8 counted T further.
+// (All groups of one product, then of the next, with the empty ones in their places, put long tiles last and wrote
+// the zeros at times when nobody multiplied.  us, that order -> this: 64 experts of 2048 x 1024 on 8 ranks, 512 rows
+// each 645 -> 545 (2.6 -> 1.4 GB fetched), 16 of 4096 x 2048 with 2048 rows each and as many empty slots 1730 -> 1640,
+// 4 of 2560 x 512 with 5443 250 -> 172.  An eighth of the whole list by work to each XCD fetches less, 0.8 instead of
+// 1.4 GB, and takes longer: 617, 1680, 172.  Sizes that are not faster: few tiles of few steps beside as many of
+// zeros, 34 groups of 512 x 512 with 128 rows and 30 empty 37 -> 41.)
 constexpr int kProducts = 3;
 struct WgradMap {
-  int tiles, other;   // T; tiles of the shorter dimension
-  int n;              // products
+  int tiles, rows, other;   // tiles of an output; of its longer dimension, of the shorter one
+  int bands;
+  int n;                    // products
   const uint16_t* A[kProducts];
   const uint16_t* B[kProducts];
   float* C[kProducts];   // [G, M, N]; the groups of a rank from a.split on go to C2
   float* C2[kProducts];
-  int M[kProducts], N[kProducts];
+  int tall;              // bit p: product p has the longer dimension as its rows
+  __host__ __device__ int M(int p) const { return (tall >> p & 1 ? rows : other) * kPT; }
+  __host__ __device__ int N(int p) const { return (tall >> p & 1 ? other : rows) * kPT; }
   // one of the three without an address, which would put the arguments into memory
   template <class T>
   __host__ __device__ static T pick(const T (&v)[kProducts], int p) { return p == 0 ? v[0] : p == 1 ? v[1] : v[2]; }
-  __host__ __device__ int begin(int v) const { return (int)((int64_t)v * tiles / 8); }
-  // an XCD's tiles of one product
-  __host__ __device__ int64_t count(int xcd, int groups) const {
-    return (int64_t)tiles * (groups >> 3) + begin(xcd + (groups & 7)) - begin(xcd);
+  // tile `item` of a product: its row of the longer dimension and its place in the shorter one
+  __device__ __forceinline__ void find(int item, int* row, int* place) const {
+    // the band that holds it: the last that begins at or before
+    const int band = mep_quotient(bands * (mep_quotient(item, rows) + 1) - 1, other);
+    const int first = mep_quotient(band * other, bands), width = mep_quotient((band + 1) * other, bands) - first;
+    const int at = item - first * rows;
+    *row = mep_quotient(at, width);
+    *place = first + at - *row * width;
   }
-  // the XCD's tile `item` of a product: its group, row of the longer dimension and place in it
-  __host__ __device__ void find(int xcd, int item, int* group, int* row, int* place) const {
-    const int octet = item / tiles;
-    const int pos = item - octet * tiles + begin(xcd);
-    const int v = (8 * pos + 7) / tiles;  // the last run that begins at or before this place
-    *group = 8 * octet + v - xcd;
-    const int first = begin(v), size = begin(v + 1) - first, rows = size / other;
-    int at = pos - first;
-    if (rows * other == size) at = at % rows * other + at / rows;  // whole rows: in columns (1 % at 16 x 8 tiles)
-    at += first - (v >= 8 ? tiles : 0);
-    *row = at / other;
-    *place = at - *row * other;
+  __device__ __forceinline__ int begin(int v) const { return (int)((int64_t)v * tiles * n >> 3); }  // of a run
+  // an XCD's tiles of the first k groups
+  __device__ __forceinline__ int count(int xcd, int k) const { return tiles * n * (k >> 3) + begin(xcd + (k & 7)) - begin(xcd); }
+  // where row `row` and place `place` of product p begin, in elements of M and of N
+  __device__ __forceinline__ void corner(int p, int row, int place, int* m0, int* n0) const {
+    *m0 = (tall >> p & 1 ? row : place) * kPT;
+    *n0 = (tall >> p & 1 ? place : row) * kPT;
   }
 };
 
 // The tiles of one workgroup of the weight gradients, one per lane: all that their divisions and table
 // lookups need is done once, side by side, and a change of tiles reads the lane (made anew by both
 // cursors at every change they were some hundred dependent instructions: three products of 64 experts of
-// 2048 x 1024, 512 rows each, 708 -> 652 us, of 16 of 4096 x 2048, 2048 rows each, 1890 -> 1778).  As in
-// PTiles, an XCD's workgroups take `rounds` tiles each in turn, moving on by one place from round to round.
-constexpr int kListed = 64;  // most rounds
+// 2048 x 1024, 512 rows each, 708 -> 652 us, of 16 of 4096 x 2048, 2048 rows each, 1890 -> 1778).  An XCD's
+// workgroups are sets of a.width that walk its tiles together, moving on by one place from round to round;
+// the sets share the rounds, whose number is only known here, evenly.
+constexpr int kListed = 64;           // most tiles of a workgroup
+constexpr int kTabled = 64 * 4096;    // most groups in the tables (100 KB)
 template <bool TN>
 struct WgradTiles {
+  const GemmArgs& a;
+  const WgradMap& map;
   int a0, a1, b0, b1, c0, c1;  // addresses: first K step of the operands, first element of the output
   int kp;                      // K steps, product
-  uint64_t left;               // the tiles to come
+  uint64_t left, empties;      // the tiles to come; tiles of zeros
   int KT, p, at;               // the present one
   static constexpr bool tall = true;
-  __device__ __forceinline__ WgradTiles(const GemmArgs& a, const WgradMap* of) {
-    const WgradMap& map = *of;
-    const int lane = threadIdx.x & 63, xcd = blockIdx.x & 7, q = blockIdx.x >> 3;
-    const int w = q % a.width, r = q / a.width * a.rounds + lane;
-    const int per = (int)map.count(xcd, a.G);
-    int item = r * a.width + (w + r) % a.width;
-    bool live = lane < a.rounds && item < per * map.n;
-    if (!live) item = 0;
-    const int pr = (item >= per) + (item >= 2 * per);
-    item -= pr * per;
-    int g, sl, u;
-    map.find(xcd, item, &g, &sl, &u);
-    if (!live) g = 0;
-    const int rank = g / a.Gr, l = g - rank * a.Gr;
-    const int first = l > 0 ? a.cu[g - 1] : 0;
-    const int steps = (a.cu[g] - first) / kBK;
-    const int64_t kbeg = (int64_t)rank * a.rank_rows + first;
-    live = live && (steps > 0 || l < a.skip_from);
-    int64_t M = 0, N = 0;
-    uint64_t A = 0, B = 0, C = 0;
+  // a group's first row among its rank's, and its K steps; -1: none, and it comes out as zeros
+  __device__ __forceinline__ int steps_of(int gi, int* beg) const {
+    *beg = 0;
+    if (gi >= a.G) return 0;
+    const int l = a.G == a.Gr ? gi : gi % a.Gr;
+    *beg = l > 0 ? a.cu[gi - 1] : 0;
+    const int steps = (a.cu[gi] - *beg) / kBK;
+    return steps > 0 ? steps : l < a.skip_from ? -1 : 0;
+  }
+  // the place of the k-th set bit
+  static __device__ __forceinline__ int nth(uint64_t mask, int k) {
+    int at = 0;
 #pragma unroll
-    for (int k = 0; k < kProducts; ++k) {
-      const uint64_t own = (uint64_t)map.C[k], other = (uint64_t)map.C2[k];
-      const uint64_t to = l < a.split ? own : other;
-      M = pr == k ? map.M[k] : M;
-      N = pr == k ? map.N[k] : N;
-      A = pr == k ? (uint64_t)map.A[k] : A;
-      B = pr == k ? (uint64_t)map.B[k] : B;
-      C = pr == k ? to : C;
+    for (int b = 32; b; b >>= 1) {
+      const int c = __popcll(mask >> at & ((1ull << b) - 1));
+      if (k >= c) { k -= c; at += b; }
     }
-    const int64_t m0 = (M >= N ? sl : u) * kPT, n0 = (M >= N ? u : sl) * kPT;
-    A += 2 * (TN ? kbeg * M + m0 : m0 * a.ld + kbeg);
-    B += 2 * (TN ? kbeg * N + n0 : n0 * a.ld + kbeg);
-    const int64_t row = (l < a.split ? (int64_t)rank * a.split + l : (int64_t)rank * (a.Gr - a.split) + l - a.split) * M + m0;
-    C += 4 * (row * N + n0);
+    return at;
+  }
+  // lds: the kernel's; free again when this returns in all waves
+  __device__ __forceinline__ WgradTiles(const GemmArgs& a_, const WgradMap* of, char* lds) : a(a_), map(*of) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int chunks = (a.G + 63) / 64;
+    int beg = 0, steps = steps_of(lane, &beg);
+    const int xcd = blockIdx.x & 7, q = blockIdx.x >> 3;
+    const int all_of = (int)(gridDim.x >> 3), sets = mep_quotient(all_of, a.width), set = mep_quotient(q, a.width), w = q - set * a.width;
+    // groups with rows and groups that come out as zeros: how many, and of every 64 groups which and how many in
+    // front of them.  More than 64 groups: each wave looks at its part of them (one after the other, 1536 groups
+    // would be 24 latencies of the memory).
+    uint64_t some = __ballot(steps > 0), none = __ballot(steps < 0);
+    int full = __popcll(some), empty = __popcll(none), sum = 0;
+    uint64_t* const masks = (uint64_t*)lds;                     // [2 chunks]
+    int2* const before = (int2*)(lds + 16 * (size_t)chunks);    // [chunks + 8], the waves' sums behind
+    // more groups than the tables hold: all are in the list, and those without rows are passed by or zeroed in their turn
+    const bool listed = a.G <= kTabled;
+    if (!listed) {
+      full = a.G;
+      empty = 0;
+    } else if (chunks > 1) {
+      full = empty = 0;
+      const int mine = wave * chunks / 8, end = (wave + 1) * chunks / 8;
+      for (int c = mine; c < end; ++c) {
+        steps = steps_of(64 * c + lane, &beg);
+        some = __ballot(steps > 0); none = __ballot(steps < 0);
+        if (lane == 0) { masks[2 * c] = some; masks[2 * c + 1] = none; before[c] = make_int2(full, empty); }
+        full += __popcll(some); empty += __popcll(none);
+      }
+      if (lane == 0) before[chunks + wave] = make_int2(full, empty);
+      __syncthreads();
+      full = empty = 0;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) { const int2 v = before[chunks + k]; full += v.x; empty += v.y; }
+      full = __builtin_amdgcn_readfirstlane(full); empty = __builtin_amdgcn_readfirstlane(empty);
+    } else {
+      sum = __builtin_amdgcn_readlane(mep_wave_incl_scan(max(steps, 0)), 63);
+    }
+    // This workgroup's tiles, a lane each.  The sets share the rounds of the groups with rows evenly, and all
+    // workgroups the tiles of zeros (as a tail of the list, when nothing is left to multiply, those of 15 of 32 groups
+    // of 4096 x 2048 are 100 us of 1750), but in a launch of one set the workgroups that have a tile less than the
+    // others first take as many of them as make up for it, a tile of zeros being the time of some six K steps.
+    const int tiles = map.count(xcd, full), blank = map.count(xcd, empty), total = mep_quotient(tiles + a.width - 1, a.width);
+    const int base = mep_quotient(total, sets), over = total - base * sets;
+    const int first_round = set * base + min(set, over), rounds = base + (set < over);
+    int extra = 0, place = q, from = 0, own = 0;
+    if (sets == 1 && blank) {
+      const int turned = max(total - 1, 0), more = tiles - turned * a.width, less = a.width - more;
+      place = w + turned - mep_quotient(w + turned, a.width) * a.width;
+      if (less) {
+        extra = min(blank, less * min(1 + mep_quotient(sum, 6 * max(full, 1)), kListed / 4));
+        const int each = mep_quotient(extra, less), more_of = extra - each * less, light = place - more;
+        if (light >= 0) {
+          from = light * each + min(light, more_of);
+          own = each + (light < more_of);
+        }
+      }
+    }
+    const int base2 = mep_quotient(blank - extra, all_of), over2 = blank - extra - base2 * all_of;
+    const int back = all_of - 1 - place;
+    const int from2 = extra + back * base2 + min(back, over2), own2 = base2 + (back < over2);
+    const int r = first_round + lane, z = lane - rounds;
+    const bool zero = z >= 0;
+    int at = zero ? (z < own ? from + z : from2 + z - own) : r * a.width + w + r - mep_quotient(w + r, a.width) * a.width;
+    bool live = zero ? z < own + own2 : at < tiles;
+    if (!live) at = 0;
+    // its group: among those with rows (zeros: without) the k-th
+    const int per = map.tiles * map.n, octet = mep_quotient(at, per), pos = at - octet * per + map.begin(xcd);
+    const int run = mep_quotient(8 * pos + 7, per);  // the last that begins at or before this place
+    int k = 8 * octet + run - xcd, g;
+    const int item = pos - map.begin(run) + map.begin(run & 7);
+    int first, length;
+    if (!listed) {
+      g = live ? k : 0;
+      length = steps_of(g, &first);
+      live = live && length;
+    } else if (chunks > 1) {
+      // the wave whose part holds it, the chunk in there
+      int c = 0, end = 0;
+#pragma unroll
+      for (int v = 0; v < 8; ++v) {
+        const int2 part = before[chunks + v];
+        const int n = zero ? part.y : part.x;
+        const bool here = c == end && k < n;
+        if (here) { c = v * chunks / 8; end = (v + 1) * chunks / 8; }
+        else if (c == end) k -= n;
+      }
+      while (end - c > 1) {  // the last chunk with no more than k in front of it
+        const int m = (c + end) / 2;
+        const int2 b = before[m];
+        if ((zero ? b.y : b.x) <= k) c = m;
+        else end = m;
+      }
+      const int2 b = before[c];
+      g = 64 * c + nth(masks[2 * c + zero], k - (zero ? b.y : b.x));
+      if (!live) g = 0;
+      length = steps_of(g, &first);
+      __syncthreads();  // the tables have been read
+    } else {
+      g = live ? nth(zero ? none : some, k) : 0;
+      first = __shfl(beg, g);
+      length = __shfl(steps, g);
+    }
+    const int pr = mep_quotient(item, map.tiles);
+    int sl, u, m0, n0;
+    map.find(item - pr * map.tiles, &sl, &u);
+    map.corner(pr, sl, u, &m0, &n0);
+    const int rank = a.G == a.Gr ? 0 : g / a.Gr;
+    const int64_t kbeg = (int64_t)rank * a.rank_rows + first;
+    const uint64_t A = (uint64_t)WgradMap::pick(map.A, pr) + 2 * (TN ? kbeg * map.M(pr) + m0 : m0 * a.ld + kbeg);
+    const uint64_t B = (uint64_t)WgradMap::pick(map.B, pr) + 2 * (TN ? kbeg * map.N(pr) + n0 : n0 * a.ld + kbeg);
+    const uint64_t C = (uint64_t)output(pr, g, m0, n0);
     a0 = (int)(uint32_t)A; a1 = (int)(A >> 32);
     b0 = (int)(uint32_t)B; b1 = (int)(B >> 32);
     c0 = (int)(uint32_t)C; c1 = (int)(C >> 32);
-    kp = steps * 4 + pr;
-    left = __ballot(live);
+    kp = max(length, 0) * 4 + pr;
+    left = __ballot(live && length > 0);
+    empties = __ballot(live && length < 0);
     KT = 0; p = 0; at = 0;
+  }
+  __device__ __forceinline__ float* output(int pr, int g, int m0, int n0) const {
+    const int rank = a.G == a.Gr ? 0 : g / a.Gr, l = g - rank * a.Gr;
+    const int64_t N = map.N(pr);
+    const int64_t row = (l < a.split ? (int64_t)rank * a.split + l : (int64_t)rank * (a.Gr - a.split) + l - a.split) * map.M(pr) + m0;
+    return (l < a.split ? WgradMap::pick(map.C, pr) : WgradMap::pick(map.C2, pr)) + row * N + n0;
   }
   __device__ __forceinline__ char* lane_pointer(int lo, int hi) const {
     return (char*)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane(hi, at) << 32) | (uint32_t)__builtin_amdgcn_readlane(lo, at));
@@ -228,7 +350,15 @@ struct WgradTiles {
   __device__ __forceinline__ const char* A() const { return lane_pointer(a0, a1); }
   __device__ __forceinline__ const char* B() const { return lane_pointer(b0, b1); }
   __device__ __forceinline__ float* C() const { return (float*)lane_pointer(c0, c1); }
-  // the next tile to write; false: no more
+  // f(first element, row length) for the workgroup's tiles of zeros
+  template <class F>
+  __device__ __forceinline__ void zeros(F&& f) {
+    for (uint64_t m = empties; m; m &= m - 1) {
+      at = __ffsll((unsigned long long)m) - 1;
+      f(C(), map.N(__builtin_amdgcn_readlane(kp, at) & 3));
+    }
+  }
+  // the next tile; false: no more
   __device__ __forceinline__ bool next() {
     if (!left) return false;
     at = __ffsll((unsigned long long)left) - 1;
@@ -254,7 +384,7 @@ struct PTiles {
   int incl, end, blocks;     // tiles up to and including the group, its end, its 128-row blocks
   int g, m0, n0, KT;
   bool tall;
-  __device__ __forceinline__ explicit PTiles(const GemmArgs& a_, const WgradMap* = nullptr) : a(a_) {
+  __device__ __forceinline__ explicit PTiles(const GemmArgs& a_, const WgradMap* = nullptr, char* = nullptr) : a(a_) {
     xcd = blockIdx.x & 7; nw = a.width; w = (int)(blockIdx.x >> 3) % nw;
     r = (int)(blockIdx.x >> 3) / nw * a.rounds; last = r + a.rounds;
     tall = true; KT = 0; g = 0; m0 = 0; n0 = 0;

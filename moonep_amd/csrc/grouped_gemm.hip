@@ -309,11 +309,14 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_nt_kernel(GemmAr
 //
 // Weight gradient at 34 688 rows in 33 groups, H = 7168, H' = 2048 (us, before -> now; before: one
 // 256-row kernel with two LDS stages that drained its loads every step): 1555 -> 1314 (1.1 GB of fp32
-// zeroes for unused groups included).  A step of it takes 1.9 us: 192 KB of transposing LDS reads, which
-// the LDS serves at half its rate, and 64 KB of loads into it.  gemm_wide_kernel reads 128 KB, but has
-// nothing beside its stores of fp32 and then meets the power limit: from equal (32 steps a tile) to
-// 15 % slower (8).  Stores of 16 bytes in pieces of 32, and waits that leave them in flight for the
-// first two steps of the next tile: 518 -> 550 at 33 792 rows, 4096 x 2048.
+// zeroes for unused groups included).  A step of it takes 1.2 to 1.6 us: 192 KB of transposing LDS reads (200
+// bytes a clock in this layout, half of the 2048 clocks of the matrix instructions) and 64 KB of loads.  What
+// it waits for is its own stores: 64 experts of 2048 x 1024, 512 rows each, take 624 us, without stores 395, with
+// stores but without loads 453 (loads that follow 256 KB of stores wait behind them, and loads that miss L2 longest).
+// gemm_wide_kernel reads 128 KB, but has nothing beside its stores of fp32: from equal (32 steps a tile) to
+// 15 % slower (8).  Not faster: stores of 16 bytes in pieces of 32 (6 % slower) or 64 (17 %), in whole 256 bytes
+// (0), plain ones (4 % slower) or written through (3 %), waits that leave them in flight for the next tile's first
+// steps (1 to 6 % slower), workgroups started a quarter of a tile apart (0), 16 x 16 x 32 instructions (0 to 5 % slower).
 //
 // LDS layouts.  Operand rows along K: 128 bytes per row and step, 16-byte vector q of row r at
 // position q ^ (r & 7) ^ ((r >> 3) & 1): sixteen consecutive lanes cover all banks.  Operands
@@ -351,8 +354,20 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
   size_t ldA = AT ? (size_t)a.M : (size_t)a.ld, ldB = BT ? (size_t)a.N : (size_t)a.ld;
   const int KT1 = WGRAD ? 0 : a.K / kBK;
   using Tiles = std::conditional_t<WGRAD, WgradTiles<AT>, PTiles<MODE>>;
-  Tiles ld(a, &map);
+  Tiles ld(a, &map, gsm);
   Tiles cp = ld;  // the tiles as they are multiplied; what describes them is read once for both
+  // Groups without rows: whole 1 KB rows of zeroes per wave instruction.  Every other workgroup writes its share in
+  // front of its tiles, so that the memory sees both kinds of work at one time.
+  const bool zeros_first = WGRAD && (blockIdx.x >> 3 & 1);
+  auto write_zeros = [&]() {
+    if constexpr (WGRAD)
+      cp.zeros([&](float* out, int N) {
+        const mep_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+        for (int row = wave; row < kPT; row += 8) __builtin_nontemporal_store(zero, (mep_f32x4*)(out + (size_t)row * N) + lane);
+      });
+  };
+  if (zeros_first) write_zeros();
   const char *pA, *pB;
   uint32_t halfA, halfB;
   int kl = 0;
@@ -372,8 +387,8 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
     if constexpr (WGRAD) {
       if (of != ld.p) {
         of = ld.p;
-        if (AT) ldA = (size_t)WgradMap::pick(map.M, of);
-        if (BT) ldB = (size_t)WgradMap::pick(map.N, of);
+        if (AT) ldA = (size_t)map.M(of);
+        if (BT) ldB = (size_t)map.N(of);
         lanes();
       }
       pA = ld.A();
@@ -386,8 +401,7 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
     halfA = __builtin_amdgcn_readfirstlane(ld.tall ? (AT ? 256u : (uint32_t)(128 * ldA * 2)) : 0u);
     halfB = BT ? 256u : (uint32_t)(128 * ldB * 2);
   };
-  bool more = true;
-  do { more = ld.next(); } while (more && ld.KT == 0);
+  bool more = ld.next();
   if (more) stand(0);
   auto advance = [&]() {
     if (!more) return;
@@ -398,7 +412,7 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
       pB += BT ? kBK * ldB * 2 : kBK * 2;
       return;
     }
-    do { more = ld.next(); } while (more && ld.KT == 0);
+    more = ld.next();
     if (more) { kl = 0; stand(0); }  // otherwise the last step is loaded again, for nobody
   };
   // slots are taken in turn: where the next half tile of each operand is written and read
@@ -516,19 +530,11 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
     float* cf = nullptr;
     if constexpr (WGRAD) {
       cf = cp.C();
-      N = WgradMap::pick(map.N, cp.p);
+      N = map.N(cp.p);
     } else {
       m0 = cp.m0; n0 = cp.n0;
     }
     if (SCALED) __builtin_assume(KT > 0);
-    if (WGRAD && KT == 0) {  // a group without rows: whole 1 KB rows of zeroes per wave instruction
-      typedef float f32x4 __attribute__((ext_vector_type(4)));
-      const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-      for (int row = wave; row < kPT; row += 8)
-        __builtin_nontemporal_store(zero, (f32x4*)(cf + (size_t)row * N) + lane);
-      continue;
-    }
     any = true;
 #pragma unroll
     for (int x = 0; x < 2; ++x)
@@ -624,6 +630,7 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
   }
   if (any && wave < 4) mep_bar();
   mep_wait_vmcnt<0>();  // the loads of steps nobody wanted write LDS, too
+  if (!zeros_first) write_zeros();
   if (!WGRAD && a.zero_tail) zero_tail_rows(a, blockIdx.x, gridDim.x, kPThreads);
 }
 // ---------------------------------------------------------------------------
@@ -1074,13 +1081,13 @@ __global__ __launch_bounds__(256) void swiglu_bwd_kernel(SwigluBwdArgs a) {
 // The grid of a kernel whose workgroups take a CU each, for at most `tiles` tiles per XCD of about
 // `steps` K steps: one workgroup per CU at one time (fewer where there are fewer tiles), each for
 // kPSteps steps.
-unsigned pp_split(GemmArgs& a, int64_t tiles, int64_t steps, int64_t most_rounds = INT32_MAX) {
+unsigned pp_split(GemmArgs& a, int64_t tiles, int64_t steps) {
   const int cus = mep_device_cu_count();
   const int64_t width = std::min<int64_t>(tiles, std::max(cus > 0 ? cus / 8 : 32, 1));
   const int64_t rounds = (tiles + width - 1) / width;
   steps = std::max<int64_t>(steps, 1);
   a.width = (int)width;
-  a.rounds = (int)std::min({rounds, std::max<int64_t>((kPSteps + steps / 2) / steps, 1), most_rounds});
+  a.rounds = (int)std::min(rounds, std::max<int64_t>((kPSteps + steps / 2) / steps, 1));
   return 8 * (unsigned)(width * ((rounds + a.rounds - 1) / a.rounds));
 }
 
@@ -1150,20 +1157,23 @@ int gemm_stream_launch(GemmArgs a, hipStream_t st) {
 // weight gradients on 256 x 256 tiles (M, N multiples of 256, a.G even)
 template <bool TN>
 int wgrad_pp_launch(GemmArgs a, WgradMap map, hipStream_t st) {
-  const int m = map.M[0], n = map.N[0];
-  MEP_REQUIRE((int64_t)(m / kPT) * (n / kPT) < (1 << 24), MEP_ERR_UNSUPPORTED);
-  map.tiles = (m / kPT) * (n / kPT);
-  map.other = std::min(m, n) / kPT;
-  int64_t per_xcd = 0;
-  for (int x = 0; x < 8; ++x) per_xcd = std::max(per_xcd, map.n * map.count(x, a.G));
-  MEP_REQUIRE(per_xcd > 0 && per_xcd < (1 << 27), MEP_ERR_UNSUPPORTED);
-  MEP_REQUIRE((int64_t)kPT * 2 * (TN ? (m > n ? m : n) : a.ld) < ((int64_t)1 << 31), MEP_ERR_UNSUPPORTED);
+  const int longer = map.rows * kPT;
+  MEP_REQUIRE((int64_t)map.rows * map.other < (1 << 24), MEP_ERR_UNSUPPORTED);
+  map.tiles = map.rows * map.other;
+  map.bands = std::max((map.other + 2) / 4, 1);
+  const int64_t per_xcd = ((int64_t)map.n * map.tiles * a.G + 7) / 8;
+  MEP_REQUIRE(per_xcd < (1 << 27), MEP_ERR_UNSUPPORTED);
+  MEP_REQUIRE((int64_t)kPT * 2 * (TN ? longer : a.ld) < ((int64_t)1 << 31), MEP_ERR_UNSUPPORTED);
   const int irc = mep_ensure_init();
   if (irc != MEP_OK) return irc;
-  // about half of the groups have rows
-  const int64_t steps = 2 * (a.rank_rows ? a.rank_rows : a.ld) / kBK / a.Gr;
-  hipLaunchKernelGGL((gemm_pp_kernel<kModeWgrad, TN, TN>), dim3(pp_split(a, per_xcd, steps, kListed)), dim3(kPThreads), kPLds,
-                     st, a, map);
+  // About half of the groups have rows, the local experts and a slot or two; the tiles of the others are skipped or
+  // are the time of a few K steps.  Sets of workgroups for some kPSteps steps each, and enough to list all tiles.
+  const int cus = mep_device_cu_count();
+  a.width = (int)std::min<int64_t>(per_xcd, std::max(cus > 0 ? cus / 8 : 32, 1));
+  const int64_t rounds = (per_xcd + a.width - 1) / a.width, per_group = (a.rank_rows ? a.rank_rows : a.ld) / kBK / a.Gr;
+  const int64_t steps = rounds * std::max<int64_t>(per_group + (a.skip_from < a.Gr ? 0 : 3), 1);
+  const int64_t sets = std::min(rounds, std::max((steps + kPSteps / 2) / kPSteps, rounds / (kListed * 3 / 4 - 4) + 1));
+  hipLaunchKernelGGL((gemm_pp_kernel<kModeWgrad, TN, TN>), dim3(8 * (unsigned)(a.width * sets)), dim3(kPThreads), kPLds, st, a, map);
   return mep_launch_status();
 }
 
@@ -1305,6 +1315,8 @@ int wgrad_tn(int n, const void* const* X1, const void* const* X2, const int32_t*
   MEP_REQUIRE(G % 2 == 0 && rows % kBM == 0 && rows * nranks <= INT32_MAX, MEP_ERR_UNSUPPORTED);
   WgradMap map{};
   map.n = n;
+  map.rows = std::max(M[0], N[0]) / kPT;
+  map.other = std::min(M[0], N[0]) / kPT;
   for (int i = 0; i < n; ++i) {
     MEP_REQUIRE(X1[i] && X2[i] && C[i] && C2[i] && M[i] > 0 && N[i] > 0, MEP_ERR_INVALID_ARG);
     MEP_REQUIRE(M[i] % kPT == 0 && N[i] % kPT == 0, MEP_ERR_UNSUPPORTED);
@@ -1317,8 +1329,7 @@ int wgrad_tn(int n, const void* const* X1, const void* const* X2, const int32_t*
     map.B[i] = (const uint16_t*)X2[i];
     map.C[i] = C[i];
     map.C2[i] = C2[i];
-    map.M[i] = M[i];
-    map.N[i] = N[i];
+    map.tall |= (M[i] >= N[i]) << i;
   }
   GemmArgs a{};
   a.cu = cu; a.split = split;
@@ -1432,7 +1443,8 @@ extern "C" int mep_grouped_gemm_wgrad(const void* At, const void* Bt, const int3
   if (Ma % kPT == 0 && Nb % kPT == 0 && G % 2 == 0 && (uintptr_t)C % 16 == 0 && ld < ((int64_t)1 << 22)) {
     WgradMap map{};
     map.n = 1;
-    map.A[0] = a.A; map.B[0] = a.B; map.C[0] = map.C2[0] = C; map.M[0] = Ma; map.N[0] = Nb;
+    map.A[0] = a.A; map.B[0] = a.B; map.C[0] = map.C2[0] = C;
+    map.rows = std::max(Ma, Nb) / kPT; map.other = std::min(Ma, Nb) / kPT; map.tall = Ma >= Nb;
     return wgrad_pp_launch<false>(a, map, (hipStream_t)stream);
   }
   a.mtiles = Ma / kBM;

@@ -1,0 +1,41 @@
+"""The weight gradients' list of tiles beside more groups than one wave looks at: which groups have rows, which
+come out as zeros and which are left alone."""
+
+import pytest
+import torch
+
+from moonep_amd import ffn
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("full", ["few", "half", "all", "last"])
+@pytest.mark.parametrize("G", [64, 66, 130, 1030])
+def test_groups_with_and_without_rows(cuda, G, full):
+    """Against the fp64 product: a sum of n products in fp32, in any order, is off by at most n 2^-24 of the
+    sum of their magnitudes."""
+    print(f"wgrad list, {G} groups, rows in {full}", flush=True)
+    g = torch.Generator().manual_seed(G)
+    share = {"few": 0.05, "half": 0.5, "all": 1.0, "last": 0.0}[full]
+    lens = ((torch.rand(G, generator=g) < share) * torch.randint(1, 3, (G,), generator=g)).tolist()
+    lens[-1] = 1
+    ends = (torch.tensor(lens).cumsum(0) * 128).to(torch.int32).to(cuda)
+    rows = 128 * (sum(lens) + 1)
+    gc = torch.Generator(device=cuda).manual_seed(G)
+    x1, x2 = (torch.randn(rows, n, generator=gc, device=cuda).to(torch.bfloat16) for n in (512, 256))
+    got = torch.full((G, 512, 256), float("nan"), device=cuda)
+    kept = got.clone()
+    ffn.launch_grouped_gemm_wgrad_tn(x1, x2, ends, got)
+    ffn.launch_grouped_gemm_wgrad_tn(x1, x2, ends, kept, skip_empty_from=G // 3)
+    torch.cuda.synchronize()
+    at = 0
+    for i, n in enumerate(lens):
+        if n:
+            a, b = (x[128 * at:128 * (at + n)].double() for x in (x1, x2))
+            assert bool(((got[i].double() - a.t() @ b).abs() <= 128 * n * 2.0 ** -24 * (a.abs().t() @ b.abs())).all()), f"group {i}"
+            at += n
+    empty = torch.tensor(lens, device=cuda) == 0
+    kept_alone = empty & (torch.arange(G, device=cuda) >= G // 3)
+    assert bool((got[empty] == 0).all())
+    assert torch.equal(kept[~kept_alone], got[~kept_alone])
+    assert bool(kept[kept_alone].isnan().all())
