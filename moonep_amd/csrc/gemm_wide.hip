@@ -112,8 +112,8 @@ __global__ __launch_bounds__(kWThreads, 1) void gemm_wide_kernel(GemmArgs a) {
   // asked for half a step after its weights
   const size_t ldA = (size_t)a.K, ldB = KN ? (size_t)a.N : (size_t)a.K;
   uint32_t stepA = kRowBytes, stepB = KN ? (uint32_t)(kBK * ldB * 2) : kRowBytes;
-  PTiles<MODE> ld(a);
-  PTiles<MODE> cp = ld;  // the tiles as they are multiplied
+  PTiles<MODE, true> ld(a);
+  PTiles<MODE, true> cp = ld;  // the tiles as they are multiplied
   const char *pA, *pB, *pB1, *qA;
   uint32_t halfA, halfB, qhalfA;
   int left = 0;         // K steps to the end of the tile, or of its first pair
