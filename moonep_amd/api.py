@@ -529,6 +529,8 @@ class Buffer:
         assert comm is not None, "MoonEP Buffer communication stream is not initialized"
         if self._limited_stream is None:
             self._record_streams(tensors, comm)
+        if self._native is not None:
+            _lib.host().comes_to_comm(self._native)
         comm.wait_event(main_stream.record_event())
         with torch.cuda.stream(comm):
             fn()

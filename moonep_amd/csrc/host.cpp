@@ -18,6 +18,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <algorithm>
 #include <initializer_list>
 #include <memory>
 #include <mutex>
@@ -39,15 +40,24 @@ struct Ctx {
   c10::Stream comm = c10::Stream(c10::Stream::UNSAFE, c10::Device(c10::kCPU), 0);
   hipStream_t comm_raw = nullptr;
   hipEvent_t order = nullptr;
-  std::mutex order_mutex;  // record and wait of `order` belong together
+  // A call's ordering and its launches belong together.  comm_used: something may be on the communication stream.
+  // beside: behind the last asynchronous call that stayed on its caller's stream, until the communication stream
+  // is ordered behind it.
+  std::mutex order_mutex;
+  bool comm_used = false, beside_open = false;
+  hipEvent_t beside = nullptr;
+  hipStream_t beside_on = nullptr;
   PyObject *plan_type = nullptr, *hidden_local_py = nullptr, *no_map_token = nullptr, *event_type = nullptr,
            *comm_py = nullptr, *empty = nullptr;
+  PyObject *current_stream = nullptr, *caller_py = nullptr;  // torch's function; what it answered for the stream caller_id
+  c10::StreamId caller_id = 0;
   PyObject *py_N = nullptr, *py_R = nullptr, *py_E = nullptr, *py_NvS = nullptr, *py_K = nullptr;
   ~Ctx() {
     for (PyObject* o : {plan_type, hidden_local_py, no_map_token, event_type, comm_py, empty, py_N, py_R, py_E,
-                        py_NvS, py_K})
+                        py_NvS, py_K, current_stream, caller_py})
       Py_XDECREF(o);
     if (order) (void)hipEventDestroy(order);
+    if (beside) (void)hipEventDestroy(beside);
   }
 };
 
@@ -96,23 +106,68 @@ struct NoGil {
   ~NoGil() { PyEval_RestoreThread(state); }
 };
 
-// ---- asynchronous calls: the work goes to the communication stream -----------------------
+// hipErrorNotReady is an answer: nobody is to find it as the last error
+hipError_t asked(hipError_t e) {
+  if (e == hipErrorNotReady) (void)hipGetLastError();
+  return e;
+}
+
+// Queries while another thread captures a stream, in whatever mode
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+// The most that an asynchronous call moves and stays on its caller's stream.  A crossing to the communication
+// stream and back takes 22 us of the GPU, and on the host some 40 a call: an event's record and the wait of
+// another stream for it, 16 us while the event has not come, and a record for every tensor that is freed after use on a
+// stream that is not its own.  Up to this size the call itself is no longer than the crossing.  us a pass of dispatch and
+// combine, each waited for, on the communication stream -> on the caller's, H = 2048, K = 8: 8 tokens 115 -> 35, 512 114 ->
+// 37, 1536 (48 MiB of copies) 117 -> 45; synchronous calls 12, 21 and 30.
+constexpr int64_t kBeside = (int64_t)64 << 20;
+
+// ---- asynchronous calls: the work goes to the communication stream, small calls' while that is idle to the caller's
 struct Async {
   Ctx& c;
-  bool on;
+  bool on, here = false;
   hipStream_t stream;
-  Async(Ctx& ctx, bool async) : c(ctx), on(async) {
+  std::unique_lock<std::mutex> lock;
+  // moved: bytes that the call reads or writes, whichever is more
+  Async(Ctx& ctx, bool async, int64_t moved = INT64_MAX) : c(ctx), on(async) {
     if (on && !c.comm_raw) {  // asked for by the first asynchronous call: the answer makes the stream exist
       PyObject* o = PyObject_GetAttrString(c.comm_py, "cuda_stream");
       c.comm_raw = o ? (hipStream_t)PyLong_AsVoidPtr(o) : nullptr;
       Py_XDECREF(o);
       if (PyErr_Occurred()) throw python_error();
     }
-    stream = on ? c.comm_raw : c10::hip::getCurrentHIPStream(c.hidden_buf.device().index()).stream();
+    here = on && moved <= kBeside;
+    stream = on ? c.comm_raw : callers();
+  }
+  hipStream_t callers() const { return c10::hip::getCurrentHIPStream(c.hidden_buf.device().index()).stream(); }
+  // `on_stream` behind the last call that stayed on its caller's stream
+  static hipError_t behind(Ctx& c, hipStream_t on_stream) {
+    if (!c.beside_open || c.beside_on == on_stream) return hipSuccess;
+    const RelaxedCapture relaxed;
+    const hipError_t e = asked(hipEventQuery(c.beside));
+    return e == hipErrorNotReady ? hipStreamWaitEvent(on_stream, c.beside, 0) : e;
   }
   // after the caller's work; the allocator must not reuse what the stream still works on
   int begin(std::initializer_list<const at::Tensor*> used) {
     if (!on) return MEP_OK;
+    hipStream_t main = callers();
+    lock = std::unique_lock<std::mutex>(c.order_mutex);
+    if (here && c.comm_used) {
+      const RelaxedCapture relaxed;
+      const hipError_t e = asked(hipStreamQuery(c.comm_raw));
+      if (e != hipSuccess && e != hipErrorNotReady) return (int)e;
+      here = e == hipSuccess;
+      c.comm_used = !here;
+    }
+    if (here) {
+      stream = main;
+      return (int)behind(c, main);
+    }
     const c10::StorageImpl* seen[24];
     int n = 0;
     for (const at::Tensor* t : used) {
@@ -124,18 +179,43 @@ struct Async {
       if (n < 24) seen[n++] = s;
       t->record_stream(c.comm);
     }
-    hipStream_t main = c10::hip::getCurrentHIPStream(c.hidden_buf.device().index()).stream();
-    std::lock_guard<std::mutex> lock(c.order_mutex);
+    c.comm_used = true;
     hipError_t e = c.order ? hipSuccess : hipEventCreateWithFlags(&c.order, hipEventDisableTiming);
     if (e == hipSuccess) e = hipEventRecord(c.order, main);
     if (e == hipSuccess) e = hipStreamWaitEvent(c.comm_raw, c.order, 0);
+    if (e == hipSuccess && c.beside_on != main) e = behind(c, c.comm_raw);
+    if (e == hipSuccess) c.beside_open = false;
     return (int)e;
+  }
+  // the call's work is on its stream
+  int launched(int rc) {
+    if (here && rc == MEP_OK) {
+      hipError_t e = c.beside ? hipSuccess : hipEventCreateWithFlags(&c.beside, hipEventDisableTiming);
+      if (e == hipSuccess) e = hipEventRecord(c.beside, stream);
+      c.beside_open = e == hipSuccess;
+      c.beside_on = stream;
+      rc = (int)e;
+    }
+    if (lock.owns_lock()) lock.unlock();
+    return rc;
+  }
+  // the caller's stream as a Python object (4 us when torch makes a new one for every event)
+  PyObject* caller() {
+    const c10::hip::HIPStream s = c10::hip::getCurrentHIPStream(c.hidden_buf.device().index());
+    if (!c.caller_py || c.caller_id != s.id()) {
+      PyObject* o = PyObject_CallFunction(c.current_stream, "i", (int)s.device_index());
+      if (!o) return nullptr;
+      Py_XSETREF(c.caller_py, o);
+      c.caller_id = s.id();
+    }
+    return c.caller_py;
   }
   // a new reference to the completion event
   PyObject* end() {
     PyObject* ev = PyObject_CallNoArgs(c.event_type);
     if (!ev) return nullptr;
-    PyObject* r = PyObject_CallMethodOneArg(ev, nm.record, c.comm_py);
+    PyObject* on_stream = here ? caller() : c.comm_py;
+    PyObject* r = on_stream ? PyObject_CallMethodOneArg(ev, nm.record, on_stream) : nullptr;
     if (!r) { Py_DECREF(ev); return nullptr; }
     Py_DECREF(r);
     return ev;
@@ -289,7 +369,8 @@ PyObject* py_dispatch(PyObject*, PyObject* const* args, Py_ssize_t n) {
   } else if (!read_plan(c, args[5], &plan)) {
     return new_none();
   }
-  Async as(c, async);
+  const int64_t row = (int64_t)c.H * 2, padded = std::min((int64_t)c.NvS, c.N + 2 * c.epn * (int64_t)(c.tp - 1));
+  Async as(c, async, padded * row + (zero_copy ? 0 : c.NvS * row));
   at::Tensor out, w_out;
   const char* what = kOrdering;
   int rc;
@@ -332,6 +413,7 @@ PyObject* py_dispatch(PyObject*, PyObject* const* args, Py_ssize_t n) {
                           zero_copy ? 0 : out.nbytes(), copy_w ? w_out.data_ptr() : nullptr,
                           copy_w ? w_local.data_ptr() : nullptr, copy_w ? (size_t)c.NvS : 0, as.stream);
     }
+    rc = as.launched(rc);
   }
   if (failed(rc, what)) return nullptr;
   PyObject* event = nullptr;
@@ -372,7 +454,7 @@ PyObject* py_combine(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const bool copy_w = w && w->data_ptr() != c.weights_local.data_ptr();
   if ((zero_copy && copy_h) || (w_zero_copy && copy_w)) return new_none();
   if (async && capturing(c)) return new_none();
-  Async as(c, async);
+  Async as(c, async, (c.N + (copy_h ? c.NvS : 0)) * (int64_t)c.H * 2);  // what it reads is more than what it writes
   at::Tensor out, out_w;
   const char* what = kOrdering;
   int rc;
@@ -395,6 +477,7 @@ PyObject* py_combine(PyObject*, PyObject* const* args, Py_ssize_t n) {
                        ptr<int>(plan.dst), out.data_ptr(), w ? ptr<float>(out_w) : nullptr, c.S, c.H, c.K, c.R, c.NvS,
                        MEP_COMBINE_TWO_LEVEL, as.stream);
     }
+    rc = as.launched(rc);
   }
   if (failed(rc, what)) return nullptr;
   PyObject* event = async ? as.end() : new_none();
@@ -490,6 +573,7 @@ PyObject* py_prefetch(PyObject*, PyObject* const* args, Py_ssize_t n) {
       what = "mep_prefetch";
       rc = mep_prefetch(m, src, dst, stride, bytes, ptr<int>(etc), c.rank, c.epn, c.R, as.stream);
     }
+    rc = as.launched(rc);
   }
   if (failed(rc, what)) return nullptr;
   if (async) return as.end();
@@ -529,6 +613,7 @@ PyObject* py_reduce(PyObject*, PyObject* const* args, Py_ssize_t n) {
       what = "mep_grad_reduce";
       rc = mep_grad_reduce_batch(3, lp, pp, stride, elems, ptr<int>(etc), c.rank, 1, c.epn, c.R, 0, as.stream);
     }
+    rc = as.launched(rc);
   }
   if (failed(rc, what)) return nullptr;
   if (async) return as.end();
@@ -722,10 +807,40 @@ PyObject* py_context(PyObject*, PyObject* const* args, Py_ssize_t n) {
   };
   c.comm = c10::Stream::unpack3(stream_num("stream_id"), (c10::DeviceIndex)stream_num("device_index"),
                                 (c10::DeviceType)stream_num("device_type"));
+  PyObject* cuda = PyImport_ImportModule("torch.cuda");
+  c.current_stream = cuda ? PyObject_GetAttrString(cuda, "current_stream") : nullptr;
+  Py_XDECREF(cuda);
   if (PyErr_Occurred()) return nullptr;
   PyObject* cap = PyCapsule_New(cptr.get(), kCapsule, free_ctx);
   if (cap) cptr.release();
   return cap;
+  END_HANDLE_TH_ERRORS
+}
+
+// comes_to_comm(ctx): the communication stream, which the caller is about to use, behind the last call that stayed on its
+// caller's stream
+PyObject* py_comes_to_comm(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Ctx* cp = n == 1 ? ctx_of(args[0]) : nullptr;
+  if (!cp) { if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "comes_to_comm takes a context"); return nullptr; }
+  Ctx& c = *cp;
+  Async as(c, true);
+  const bool captured = capturing(c);
+  hipError_t e = hipSuccess;
+  {
+    NoGil other_threads;
+    std::lock_guard<std::mutex> lock(c.order_mutex);
+    c.comm_used = true;
+    if (c.beside_open && captured) {  // a stream under capture cannot wait for what was not captured
+      const RelaxedCapture relaxed;
+      e = hipEventSynchronize(c.beside);
+    } else {
+      e = Async::behind(c, c.comm_raw);
+    }
+    if (e == hipSuccess) c.beside_open = false;
+  }
+  if (failed((int)e, kOrdering)) return nullptr;
+  Py_RETURN_NONE;
   END_HANDLE_TH_ERRORS
 }
 
@@ -735,6 +850,7 @@ PyMethodDef kMethods[] = {{"context", MEP_FAST(py_context)},
                           {"combine", MEP_FAST(py_combine)},
                           {"prefetch", MEP_FAST(py_prefetch)},
                           {"reduce_grad", MEP_FAST(py_reduce)},
+                          {"comes_to_comm", MEP_FAST(py_comes_to_comm)},
                           {"ffn_forward", MEP_FAST(py_ffn_forward)},
                           {"ffn_backward", MEP_FAST(py_ffn_backward)},
                           {nullptr, nullptr, 0, nullptr}};

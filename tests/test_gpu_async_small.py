@@ -1,0 +1,87 @@
+"""Small asynchronous calls, which stay on their caller's stream while the communication stream is idle: the same
+results as synchronous ones on both sides of the bound, and the order that one stream for all calls would give."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+E, K, R, TP = 32, 4, 4, 16
+
+
+def _make(cuda, S, H, seed=1):
+    from moonep_amd import Buffer, EmulatedWorld
+
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    topk = torch.topk(torch.randn(R, S, E, device=cuda, generator=g), K, dim=-1)[1].to(torch.int32)
+    counts = torch.zeros(R, E, dtype=torch.int32, device=cuda)
+    counts.scatter_add_(1, topk.reshape(R, -1).long(), torch.ones(R, S * K, dtype=torch.int32, device=cuda))
+    world = EmulatedWorld(S, H, K, E, R, TP)
+    world.hidden_buf.zero_()
+    buf = Buffer(S, H, K, E, R, token_padding=TP, rank=1, world=world)
+    xs = [torch.randn(S, H, device=cuda, generator=g).to(torch.bfloat16) for _ in range(2)]
+    return world, buf, xs, torch.rand(S, K, device=cuda, generator=g), topk, counts
+
+
+def _pass(buf, x, w, topk, counts, wait, zero_copy):
+    modes = dict(zero_copy=zero_copy, router_weights_zero_copy=zero_copy, async_finish=wait)
+    res = buf.dispatch(x, w, topk, counts, **modes)
+    if wait:
+        torch.cuda.current_stream().wait_event(res[4])
+    out = buf.combine(res[3], res[0], res[1], **modes)
+    if wait:
+        torch.cuda.current_stream().wait_event(out[2])
+    return res, out
+
+
+@pytest.mark.parametrize("S,H", [(1, 512), (300, 1024), (4000, 2048), (4200, 2048)])   # 64 MiB lie between the last
+@pytest.mark.parametrize("zero_copy", [True, False])
+def test_same_as_synchronous(cuda, S, H, zero_copy):
+    print(f"async {S} x {H} zero_copy={zero_copy}", flush=True)
+    world, buf, (x, _), w, topk, counts = _make(cuda, S, H)
+    got = []
+    for wait in (False, True, True):
+        world.hidden_buf.fill_(3)
+        res, out = _pass(buf, x, w, topk[1].contiguous(), counts, wait, zero_copy)
+        torch.cuda.synchronize()
+        got.append([t.clone() for t in (world.hidden_buf, res[1], res[2], res[3].dst, out[0], out[1])])
+    for other in got[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(got[0], other))
+
+
+def test_calls_from_several_streams_keep_their_order(cuda):
+    """A call whose stream is held comes before calls that are made later on other streams, small or through the
+    communication stream, as if all of them went through that one."""
+    S, H = 200, 1024
+    world, buf, (x, y), w, topk, counts = _make(cuda, S, H)
+    mine = topk[1].contiguous()
+    wants = []
+    for t in (x, y):
+        res, out = _pass(buf, t, w, mine, counts, False, True)
+        wants.append((res[0].clone(), out[0].clone()))
+    (rows_x, want_x), (rows_y, want_y) = wants
+    shard = res[0]
+    assert not torch.equal(rows_x, rows_y)
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    for rounds in range(3):
+        print(f"round {rounds}", flush=True)
+        torch.cuda.synchronize()
+        # held dispatch of x on one stream, combine on another
+        with torch.cuda.stream(a):
+            torch.cuda._sleep(20_000_000)
+            plan, ev = buf.dispatch(x, w, mine, counts, zero_copy=True, async_finish=True)[3:5]
+        with torch.cuda.stream(b):
+            out, _, done = buf.combine(plan, shard, zero_copy=True, async_finish=True)
+        done.synchronize()
+        assert ev.query() and torch.equal(out, want_x)
+        # held dispatch of x, then one of y whose routing is every rank's: that one goes through the communication stream
+        with torch.cuda.stream(b):
+            torch.cuda._sleep(20_000_000)
+            buf.dispatch(x, w, mine, counts, zero_copy=True, async_finish=True)
+        with torch.cuda.stream(a):
+            rows, _, _, plan, _ = buf.dispatch(y, w, topk, counts, zero_copy=True, async_finish=True)
+        with torch.cuda.stream(b):   # the communication stream is not idle
+            out, _, done = buf.combine(plan, shard, zero_copy=True, async_finish=True)
+        done.synchronize()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want_y) and torch.equal(rows, rows_y)
