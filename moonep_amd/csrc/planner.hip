@@ -712,21 +712,28 @@ struct PlanConfig {
   int groups;
 };
 
-// 0 on success
+// Ints of scratch per rank that a caller brings: two tables of E x R for every 256 threads' tokens where those and the
+// rest are more than a kernel's LDS without asking
+size_t plan_scratch_ints(int S, int K, int E, int R) {
+  if (plan_lds_bytes(256, E, R, true) <= kLdsDefaultLimit) return 0;
+  const int tok_per_wg = 256 / K;
+  return (size_t)((S + tok_per_wg - 1) / tok_per_wg) * 2 * (size_t)E * R;
+}
+
+// 0 on success.  1024 threads with all tables in LDS wherever that holds them, on a CU's whole LDS too: a workgroup
+// of 256 resolves a fourth of the tokens, so four times as many rebuild the plan, and tables in scratch memory are
+// latencies of the memory in its chain.  us, planner of 4096 tokens, K = 8 (cache warming included), 256 threads ->
+// 1024: E = 768, R = 16 30.3 -> 14.0.
 int plan_config(int S, int K, int E, int R, PlanConfig* c) {
-  c->opt_in = false;
-  if (plan_lds_bytes(1024, E, R, true) <= kLdsDefaultLimit) {
+  if (plan_lds_bytes(1024, E, R, true) <= kLdsOptInLimit) {
     c->nt = 1024; c->lds_tables = true;
-  } else if (plan_lds_bytes(256, E, R, true) <= kLdsDefaultLimit) {
-    c->nt = 256; c->lds_tables = true;
-  } else if (plan_lds_bytes(256, E, R, false) <= kLdsDefaultLimit) {
-    c->nt = 256; c->lds_tables = false;
   } else if (plan_lds_bytes(256, E, R, false) <= kLdsOptInLimit) {
-    c->nt = 256; c->lds_tables = false; c->opt_in = true;
+    c->nt = 256; c->lds_tables = false;
   } else {
     return MEP_ERR_UNSUPPORTED;
   }
   c->lds_bytes = plan_lds_bytes(c->nt, E, R, c->lds_tables);
+  c->opt_in = c->lds_bytes > kLdsDefaultLimit;
   c->tok_per_wg = c->nt / K;
   c->groups = (S + c->tok_per_wg - 1) / c->tok_per_wg;
   return MEP_OK;
@@ -737,8 +744,8 @@ int plan_config(int S, int K, int E, int R, PlanConfig* c) {
 extern "C" size_t mep_plan_scratch_bytes(int S, int K, int E, int R, int nranks) {
   PlanConfig c;
   if (S <= 0 || K <= 0 || K > 32 || E <= 0 || R <= 0 || nranks <= 0) return 0;
-  if (plan_config(S, K, E, R, &c) != MEP_OK || c.lds_tables) return 0;
-  return (size_t)c.groups * nranks * 2 * (size_t)E * R * sizeof(int);
+  if (plan_config(S, K, E, R, &c) != MEP_OK) return 0;
+  return plan_scratch_ints(S, K, E, R) * nranks * sizeof(int);
 }
 
 namespace {
@@ -825,8 +832,7 @@ int plan_launch(const int32_t* tpe_RE, const int32_t* topk_nSK, int rank0, int n
   PlanConfig c;
   int rc = plan_config(S, K, E, R, &c);
   if (rc != MEP_OK) return rc;
-  if (!c.lds_tables) {
-    const size_t need = (size_t)c.groups * nranks * 2 * (size_t)E * R * sizeof(int);
+  if (const size_t need = plan_scratch_ints(S, K, E, R) * nranks * sizeof(int)) {
     MEP_REQUIRE(scratch && scratch_bytes >= need, MEP_ERR_SCRATCH);
     MEP_REQUIRE((uintptr_t)scratch % 16 == 0, MEP_ERR_ALIGNMENT);
   }
@@ -859,17 +865,15 @@ int plan_launch(const int32_t* tpe_RE, const int32_t* topk_nSK, int rank0, int n
     warm_groups = (int)(want < cap ? want : cap);
   }
   dim3 grid(c.groups + warm_groups, nranks);
+  if (c.opt_in) {  // more dynamic LDS than the default limit: opted in by mep_init_planner_kernels
+    const int irc = mep_ensure_init();
+    if (irc != MEP_OK) return irc;
+  }
   if (c.nt == 1024) {
 #define MEP_PLAN(RC, KC) hipLaunchKernelGGL((plan_kernel<1024, true, RC, KC>), grid, dim3(1024), c.lds_bytes, st, a, NoCopy{})
     MEP_PLAN_VARIANT(R, K, MEP_PLAN);
 #undef MEP_PLAN
-  } else if (c.lds_tables) {
-    hipLaunchKernelGGL((plan_kernel<256, true>), grid, dim3(256), c.lds_bytes, st, a, NoCopy{});
   } else {
-    if (c.opt_in) {  // more dynamic LDS than the default limit: opted in by mep_init_planner_kernels
-      const int irc = mep_ensure_init();
-      if (irc != MEP_OK) return irc;
-    }
     hipLaunchKernelGGL((plan_kernel<256, false>), grid, dim3(256), c.lds_bytes, st, a, NoCopy{});
   }
   return mep_launch_status();
@@ -877,10 +881,14 @@ int plan_launch(const int32_t* tpe_RE, const int32_t* topk_nSK, int rank0, int n
 
 }  // namespace
 
-// LDS opt-in of the planner variant for very large expert counts, for the current device
+// LDS opt-ins of the planner variants that large expert counts take, for the current device
 int mep_init_planner_kernels() {
-  MEP_RETURN_IF_HIP(hipFuncSetAttribute((const void*)plan_kernel<256, false>,
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsOptInLimit));
+  for (const void* kernel : {(const void*)plan_kernel<256, false>, (const void*)plan_kernel<1024, true, 8, 8>,
+                             (const void*)plan_kernel<1024, true, 4, 8>, (const void*)plan_kernel<1024, true, 16, 8>,
+                             (const void*)plan_kernel<1024, true, 2, 0>, (const void*)plan_kernel<1024, true, 4, 0>,
+                             (const void*)plan_kernel<1024, true, 8, 0>, (const void*)plan_kernel<1024, true, 16, 0>,
+                             (const void*)plan_kernel<1024, true, 0, 0>})
+    MEP_RETURN_IF_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsOptInLimit));
   return MEP_OK;
 }
 
