@@ -33,9 +33,9 @@ struct DispatchArgs {
 // One wave per (token, k) copy: it reads the token row (the K waves of a token
 // share it through the caches) and streams it to its slot.  Waves that issue
 // one row of stores each keep the HBM write path busier than one wave issuing
-// K rows.  NV > 0: the row is exactly NV 16-byte vectors per lane and passes
-// through registers in one go; NV == 0: any H % 8 == 0, strided loop.
-template <int NV>
+// K rows.  A row passes through registers NV 16-byte vectors per lane at a time:
+// WHOLE: it is exactly those; otherwise any H % 8 == 0.
+template <int NV, bool WHOLE>
 __global__ __launch_bounds__(kBlock) void dispatch_kernel(DispatchArgs a) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -54,26 +54,30 @@ __global__ __launch_bounds__(kBlock) void dispatch_kernel(DispatchArgs a) {
     if (drank >= a.R) return;  // never write outside the shards
     if (a.w && lane == 0) a.wslots[(size_t)drank * a.wslot_stride + loff] = a.w[(size_t)blockIdx.y * a.S * a.K + gw];
     if (dv < 0 && !(a.flags & MEP_DISPATCH_WRITE_DUPS)) return;
-    const char* src = (const char*)a.hidden + ((size_t)blockIdx.y * a.S + s) * row_bytes + (size_t)lane * 16;
-    char* row = (char*)a.shards +
-                ((uint64_t)drank * (uint64_t)a.shard_stride_rows + (uint64_t)loff) * row_bytes +
-                (size_t)lane * 16;
-    if (NV > 0) {
-      mep_u4 v[NV > 0 ? NV : 1];
+    const char* src = (const char*)a.hidden + ((size_t)blockIdx.y * a.S + s) * row_bytes;
+    char* row = (char*)a.shards + ((uint64_t)drank * (uint64_t)a.shard_stride_rows + (uint64_t)loff) * row_bytes;
+    if (WHOLE) {
+      src += (size_t)lane * 16;
+      row += (size_t)lane * 16;
+      mep_u4 v[NV];
 #pragma unroll
       for (int i = 0; i < NV; ++i) v[i] = mep_ld16(src + (size_t)i * 1024);
 #pragma unroll
       for (int i = 0; i < NV; ++i) mep_st16_stream(row + (size_t)i * 1024, v[i]);
     } else {
+      // From the last 128-byte line that begins at or before the row: whole lines but for the row's ends.  (A KB from
+      // any 16-byte address leaves two lines of nine to be written in parts, a store each: 4096 tokens, K = 8, dispatch
+      // of H = 3000 57 -> 46 us, 4104 78 -> 60, 5000 96 -> 73, 7160 134 -> 100.  Plain stores for a row's two ends, whose
+      // lines other rows share: 62 at 5000, but the combine behind it 66 -> 80.)  No load waits for a condition: those
+      // past the row's end read its last vector.
       const int nvec = H / 8;
-      for (int c0 = 0; c0 < nvec; c0 += 4 * 64) {
-        mep_u4 v[4];
+      for (int c0 = lane - mep_line_offset(row) / 16; c0 - lane < nvec; c0 += NV * 64) {
+        mep_u4 v[NV];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (c0 + i * 64 + lane < nvec) v[i] = mep_ld16(src + (size_t)(c0 + i * 64) * 16);
+        for (int i = 0; i < NV; ++i) v[i] = mep_ld16(src + (size_t)min(max(c0 + i * 64, 0), nvec - 1) * 16);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (c0 + i * 64 + lane < nvec) mep_st16_stream(row + (size_t)(c0 + i * 64) * 16, v[i]);
+        for (int i = 0; i < NV; ++i)
+          if ((unsigned)(c0 + i * 64) < (unsigned)nvec) mep_st16_stream(row + (size_t)(c0 + i * 64) * 16, v[i]);
       }
     }
     return;
@@ -103,9 +107,12 @@ __global__ __launch_bounds__(kBlock) void dispatch_kernel(DispatchArgs a) {
   const mep_u4 zero = {0u, 0u, 0u, 0u};
   char* base = (char*)a.shards +
                ((uint64_t)rank * (uint64_t)a.shard_stride_rows + (uint64_t)pad_start) * row_bytes;
-  const size_t region = (size_t)n_pad * row_bytes;              // a multiple of 16 (H % 8 == 0)
+  const size_t before = mep_line_offset(base);  // whole lines, as above
+  base -= before;
+  const size_t region = (size_t)n_pad * row_bytes + before;     // a multiple of 16 (H % 8 == 0)
   const size_t step = (size_t)parts * kBlock * 16;
   for (size_t off = ((size_t)zb * kBlock + threadIdx.x) * 16; off < region; off += step) {
+    if (off < before) continue;
     if (a.through) mep_st16_through(base + off, zero);
     else mep_st16_stream(base + off, zero);
   }
@@ -391,19 +398,19 @@ int dispatch_launch(const void* hidden, const float* w, const int32_t* dst, cons
   a.zblocks = zblocks + a.tail_blocks;
   dim3 grid(a.tok_blocks + a.zblocks, nranks);
   hipStream_t st = (hipStream_t)stream;
-  // rows that are a whole number of 1-KiB wave tiles (H % 512 == 0, up to H = 8192) pass
-  // through registers in one go; any other H % 8 == 0 takes the strided loop
+  // rows that are a whole number of 1-KiB wave tiles (H % 512 == 0, up to H = 8192) pass through registers as they
+  // are; any other H % 8 == 0 from the line that holds its first byte, 4 KB at a time (as many as the row takes
+  // at once: the same time)
   const int nvec = H / 8;
-  const int tiles = nvec % 64 == 0 ? nvec / 64 : 0;
-  switch (tiles) {
+  switch (nvec % 64 == 0 ? nvec / 64 : 0) {
 #define MEP_DISPATCH_CASE(NV) \
-    case NV: hipLaunchKernelGGL(dispatch_kernel<NV>, grid, dim3(kBlock), 0, st, a); break;
+    case NV: hipLaunchKernelGGL((dispatch_kernel<NV, true>), grid, dim3(kBlock), 0, st, a); break;
     MEP_DISPATCH_CASE(1) MEP_DISPATCH_CASE(2) MEP_DISPATCH_CASE(3) MEP_DISPATCH_CASE(4)
     MEP_DISPATCH_CASE(5) MEP_DISPATCH_CASE(6) MEP_DISPATCH_CASE(7) MEP_DISPATCH_CASE(8)
     MEP_DISPATCH_CASE(9) MEP_DISPATCH_CASE(10) MEP_DISPATCH_CASE(11) MEP_DISPATCH_CASE(12)
     MEP_DISPATCH_CASE(13) MEP_DISPATCH_CASE(14) MEP_DISPATCH_CASE(15) MEP_DISPATCH_CASE(16)
 #undef MEP_DISPATCH_CASE
-    default: hipLaunchKernelGGL(dispatch_kernel<0>, grid, dim3(kBlock), 0, st, a); break;
+    default: hipLaunchKernelGGL((dispatch_kernel<4, false>), grid, dim3(kBlock), 0, st, a); break;
   }
   return mep_launch_status();
 }

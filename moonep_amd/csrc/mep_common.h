@@ -182,6 +182,8 @@ __device__ __forceinline__ mep_u4 mep_ld16_stream(const void* p) {
 __device__ __forceinline__ mep_u4 mep_ld16(const void* p) {
   return *(const mep_u4*)p;
 }
+// bytes from the beginning of the 128-byte line that holds it
+__device__ __forceinline__ int mep_line_offset(const void* p) { return (int)((uintptr_t)p & 127); }
 __device__ __forceinline__ void mep_st16_stream(void* p, mep_u4 v) {
   __builtin_nontemporal_store(v, (mep_u4*)p);
 }
