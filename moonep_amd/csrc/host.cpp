@@ -164,10 +164,9 @@ struct Async {
       here = e == hipSuccess;
       c.comm_used = !here;
     }
-    if (here) {
-      stream = main;
-      return (int)behind(c, main);
-    }
+    // on the caller's stream, too: a tensor may have been allocated on another (one of the same costs a look-up)
+    const c10::StreamId callers_id = c10::hip::getCurrentHIPStream(c.hidden_buf.device().index()).id();
+    const c10::Stream user = here ? c10::Stream(c10::Stream::UNSAFE, c.comm.device(), callers_id) : c.comm;
     const c10::StorageImpl* seen[24];
     int n = 0;
     for (const at::Tensor* t : used) {
@@ -177,7 +176,11 @@ struct Async {
       for (int i = 0; i < n; ++i) dup |= seen[i] == s;
       if (dup) continue;
       if (n < 24) seen[n++] = s;
-      t->record_stream(c.comm);
+      t->record_stream(user);
+    }
+    if (here) {
+      stream = main;
+      return (int)behind(c, main);
     }
     c.comm_used = true;
     hipError_t e = c.order ? hipSuccess : hipEventCreateWithFlags(&c.order, hipEventDisableTiming);

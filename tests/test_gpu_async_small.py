@@ -85,3 +85,25 @@ def test_calls_from_several_streams_keep_their_order(cuda):
         done.synchronize()
         torch.cuda.synchronize()
         assert torch.equal(out, want_y) and torch.equal(rows, rows_y)
+
+
+def test_memory_of_another_stream_outlives_the_call(cuda):
+    """Tensors that were allocated on a stream other than the caller's may be dropped as soon as the call returns: their
+    memory is not handed out again while the call's work is to come."""
+    S, H = 200, 1024
+    world, buf, (x, _), w, topk, counts = _make(cuda, S, H)
+    mine = topk[1].contiguous()
+    want = buf.dispatch(x, w, mine, counts, zero_copy=True)[0].clone()
+    side = torch.cuda.Stream()
+    for _ in range(3):
+        copy = x.clone()
+        place = copy.data_ptr()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            torch.cuda._sleep(20_000_000)
+            rows, _, _, _, done = buf.dispatch(copy, w, mine, counts, zero_copy=True, async_finish=True)
+        del copy
+        others = [torch.full_like(x, 7.0) for _ in range(4)]
+        assert not done.query() and place not in [t.data_ptr() for t in others]
+        done.synchronize()
+        assert torch.equal(rows, want)
