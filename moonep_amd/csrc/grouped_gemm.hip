@@ -309,7 +309,8 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_nt_kernel(GemmAr
 //
 // Weight gradient at 34 688 rows in 33 groups, H = 7168, H' = 2048 (us, before -> now; before: one
 // 256-row kernel with two LDS stages that drained its loads every step): 1555 -> 1314 (1.1 GB of fp32
-// zeroes for unused groups included).  A step of it takes 1.2 to 1.6 us: 192 KB of transposing LDS reads (200
+// zeroes for unused groups included; on another card 1358 -> 1303 with the list by groups, which spreads the zeroes
+// over the workgroups, 1052 -> 1027 without zeroes).  A step of it takes 1.2 to 1.6 us: 192 KB of transposing LDS reads (200
 // bytes a clock in this layout, half of the 2048 clocks of the matrix instructions) and 64 KB of loads.  What
 // it waits for is its own stores: 64 experts of 2048 x 1024, 512 rows each, take 624 us, without stores 395, with
 // stores but without loads 453 (loads that follow 256 KB of stores wait behind them, and loads that miss L2 longest).
