@@ -191,6 +191,7 @@ struct WgradMap {
 // the sets share the rounds, whose number is only known here, evenly.
 constexpr int kListed = 64;           // most tiles of a workgroup
 constexpr int kTabled = 64 * 4096;    // most groups in the tables (100 KB)
+typedef __attribute__((address_space(1))) float mep_global_f32;
 template <bool TN>
 struct WgradTiles {
   const GemmArgs& a;
@@ -349,7 +350,9 @@ struct WgradTiles {
   }
   __device__ __forceinline__ const char* A() const { return lane_pointer(a0, a1); }
   __device__ __forceinline__ const char* B() const { return lane_pointer(b0, b1); }
-  __device__ __forceinline__ float* C() const { return (float*)lane_pointer(c0, c1); }
+  // In global memory by its type: a store through a pointer of unknown kind counts among the LDS operations, too, and a wait
+  // for LDS reads then is one for the stores (C1).
+  __device__ __forceinline__ mep_global_f32* C() const { return (mep_global_f32*)lane_pointer(c0, c1); }
   // f(first element, row length) for the workgroup's tiles of zeros
   template <class F>
   __device__ __forceinline__ void zeros(F&& f) {

@@ -362,10 +362,11 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
   const bool zeros_first = WGRAD && (blockIdx.x >> 3 & 1);
   auto write_zeros = [&]() {
     if constexpr (WGRAD)
-      cp.zeros([&](float* out, int N) {
+      cp.zeros([&](mep_global_f32* out, int N) {
+        typedef __attribute__((address_space(1))) mep_f32x4 global_f32x4;
         const mep_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
-        for (int row = wave; row < kPT; row += 8) __builtin_nontemporal_store(zero, (mep_f32x4*)(out + (size_t)row * N) + lane);
+        for (int row = wave; row < kPT; row += 8) __builtin_nontemporal_store(zero, (global_f32x4*)(out + (size_t)row * N) + lane);
       });
   };
   if (zeros_first) write_zeros();
@@ -528,7 +529,7 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
     const int KT = cp.KT;
     const bool tall = cp.tall;
     int m0 = 0, n0 = 0, N = a.N;
-    float* cf = nullptr;
+    mep_global_f32* cf = nullptr;
     if constexpr (WGRAD) {
       cf = cp.C();
       N = map.N(cp.p);
@@ -592,7 +593,7 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
       for (int i = 0; i < 2; ++i) {
         const int m = m0 + 128 * x + 64 * wm + 32 * i + 4 * half;
         if (WGRAD) {
-          float* out = cf + (size_t)m * N + n0 + 32 * wn + l31;
+          mep_global_f32* out = cf + (size_t)m * N + n0 + 32 * wn + l31;
 #pragma unroll
           for (int v = 0; v < 16; ++v)
 #pragma unroll
