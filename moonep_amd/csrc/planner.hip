@@ -640,8 +640,9 @@ __global__ __launch_bounds__(NT, kPlanWavesPerSimd<Copy>) void plan_kernel(PlanA
       copy.wslots[(size_t)(dv / NvS) * copy.wslot_stride + dv % NvS] = copy.w[e0 + tid];
     __syncthreads();
     // from the line that holds the row's first byte, as dispatch_kernel does (8000 tokens at H = 520 31.3 -> 28.8 us, 600
-    // at 5000 19.9 -> 17.4)
-    const int pieces = (int)((row_bytes + (row_bytes & 127 ? 112 : 0) + 4095) >> 12);
+    // at 5000 19.9 -> 17.4); all rows begin at a line's beginning where the shards and a row's length do
+    const bool lines = ((row_bytes | (uintptr_t)copy.shards) & 127) == 0;
+    const int pieces = (int)((row_bytes + (lines ? 0 : 112) + 4095) >> 12);
     for (int i = wave; i < n * pieces; i += NW) {
       const int en = i / pieces, piece = i - en * pieces;
       const int raw = __builtin_amdgcn_readfirstlane(s_cd[en]);
