@@ -529,12 +529,17 @@ class Buffer:
         assert comm is not None, "MoonEP Buffer communication stream is not initialized"
         if self._limited_stream is None:
             self._record_streams(tensors, comm)
-        if self._native is not None:
-            _lib.host().comes_to_comm(self._native)
-        comm.wait_event(main_stream.record_event())
-        with torch.cuda.stream(comm):
-            fn()
-            done = comm.record_event()
+        native = self._native
+        if native is not None:
+            _lib.host().comes_to_comm(native)
+        try:
+            comm.wait_event(main_stream.record_event())
+            with torch.cuda.stream(comm):
+                fn()
+                done = comm.record_event()
+        finally:
+            if native is not None:
+                _lib.host().leaves_comm(native)
         if self._limited_stream is not None:
             # A CU-masked stream is the library's and gets destroyed at exit, so the
             # allocator must never hold it: instead of record_stream the tensors are kept

@@ -41,10 +41,11 @@ struct Ctx {
   hipStream_t comm_raw = nullptr;
   hipEvent_t order = nullptr;
   // A call's ordering and its launches belong together.  comm_used: something may be on the communication stream.
-  // beside: behind the last asynchronous call that stayed on its caller's stream, until the communication stream
+  // coming: callers of comes_to_comm whose work is not all there.  beside: behind the last asynchronous call that stayed on its caller's stream, until the communication stream
   // is ordered behind it.
   std::mutex order_mutex;
   bool comm_used = false, beside_open = false;
+  int coming = 0;
   hipEvent_t beside = nullptr;
   hipStream_t beside_on = nullptr;
   PyObject *plan_type = nullptr, *hidden_local_py = nullptr, *no_map_token = nullptr, *event_type = nullptr,
@@ -157,6 +158,7 @@ struct Async {
     if (!on) return MEP_OK;
     hipStream_t main = callers();
     lock = std::unique_lock<std::mutex>(c.order_mutex);
+    if (here && c.coming) here = false;  // the stream may be idle until another thread's launches
     if (here && c.comm_used) {
       const RelaxedCapture relaxed;
       const hipError_t e = asked(hipStreamQuery(c.comm_raw));
@@ -821,7 +823,7 @@ PyObject* py_context(PyObject*, PyObject* const* args, Py_ssize_t n) {
 }
 
 // comes_to_comm(ctx): the communication stream, which the caller is about to use, behind the last call that stayed on its
-// caller's stream
+// caller's stream; until the caller's leaves_comm(ctx) that stream counts as busy
 PyObject* py_comes_to_comm(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   Ctx* cp = n == 1 ? ctx_of(args[0]) : nullptr;
@@ -841,8 +843,23 @@ PyObject* py_comes_to_comm(PyObject*, PyObject* const* args, Py_ssize_t n) {
       e = Async::behind(c, c.comm_raw);
     }
     if (e == hipSuccess) c.beside_open = false;
+    if (e == hipSuccess) ++c.coming;
   }
   if (failed((int)e, kOrdering)) return nullptr;
+  Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
+
+// leaves_comm(ctx): all that the caller of comes_to_comm had for the communication stream is on it
+PyObject* py_leaves_comm(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Ctx* c = n == 1 ? ctx_of(args[0]) : nullptr;
+  if (!c) { if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "leaves_comm takes a context"); return nullptr; }
+  {
+    NoGil other_threads;
+    std::lock_guard<std::mutex> lock(c->order_mutex);
+    --c->coming;
+  }
   Py_RETURN_NONE;
   END_HANDLE_TH_ERRORS
 }
@@ -854,6 +871,7 @@ PyMethodDef kMethods[] = {{"context", MEP_FAST(py_context)},
                           {"prefetch", MEP_FAST(py_prefetch)},
                           {"reduce_grad", MEP_FAST(py_reduce)},
                           {"comes_to_comm", MEP_FAST(py_comes_to_comm)},
+                          {"leaves_comm", MEP_FAST(py_leaves_comm)},
                           {"ffn_forward", MEP_FAST(py_ffn_forward)},
                           {"ffn_backward", MEP_FAST(py_ffn_backward)},
                           {nullptr, nullptr, 0, nullptr}};

@@ -1,6 +1,9 @@
 """Small asynchronous calls, which stay on their caller's stream while the communication stream is idle: the same
 results as synchronous ones on both sides of the bound, and the order that one stream for all calls would give."""
 
+import threading
+import time
+
 import pytest
 import torch
 
@@ -85,6 +88,50 @@ def test_calls_from_several_streams_keep_their_order(cuda):
         done.synchronize()
         torch.cuda.synchronize()
         assert torch.equal(out, want_y) and torch.equal(rows, rows_y)
+
+
+def test_call_of_another_thread_while_one_comes_to_the_communication_stream(cuda):
+    """A dispatch with every rank's routing takes the communication stream in steps: first it is ordered, then the work
+    follows.  A small call of another thread in between finds that stream idle; the calls after both of them still come
+    behind the work."""
+    S, H = 200, 1024
+    world, buf, (x, y), w, topk, counts = _make(cuda, S, H)
+    mine = topk[1].contiguous()
+    rows, _, _, plan = buf.dispatch(y, w, topk, counts, zero_copy=True)
+    want = buf.combine(plan, rows, zero_copy=True)[0].clone()
+    a, streams = torch.cuda.Stream(), [torch.cuda.Stream() for _ in range(6)]   # some share a hardware queue
+    failures = []
+
+    def other():
+        try:
+            with torch.cuda.device(cuda), torch.cuda.stream(b):
+                buf.dispatch(x, w, mine, counts, zero_copy=True, async_finish=True)[4].synchronize()
+        except Exception as e:  # noqa: BLE001 - shown by the assertion below
+            failures.append(e)
+
+    run = buf._run_dispatch
+
+    def slowly(*args):
+        for _ in range(100):
+            time.sleep(0.001)
+            if buf._comm_stream.query():
+                break
+        thread = threading.Thread(target=other)
+        thread.start()
+        thread.join()
+        torch.cuda._sleep(20_000_000)
+        run(*args)
+
+    buf._run_dispatch = slowly
+    for b in streams:
+        torch.cuda.synchronize()
+        with torch.cuda.stream(a):
+            rows, _, _, plan, done = buf.dispatch(y, w, topk, counts, zero_copy=True, async_finish=True)
+        assert not failures
+        with torch.cuda.stream(b):
+            out, _, last = buf.combine(plan, rows, zero_copy=True, async_finish=True)
+        last.synchronize()
+        assert done.query() and torch.equal(out, want)
 
 
 def test_memory_of_another_stream_outlives_the_call(cuda):
