@@ -131,7 +131,7 @@ constexpr int64_t kBeside = (int64_t)64 << 20;
 // ---- asynchronous calls: the work goes to the communication stream, small calls' while that is idle to the caller's
 struct Async {
   Ctx& c;
-  bool on, here = false;
+  bool on, here = false, ordered = false;
   hipStream_t stream;
   std::unique_lock<std::mutex> lock;
   // moved: bytes that the call reads or writes, whichever is more
@@ -182,7 +182,9 @@ struct Async {
     }
     if (here) {
       stream = main;
-      return (int)behind(c, main);
+      const hipError_t e = behind(c, main);
+      ordered = e == hipSuccess;
+      return (int)e;
     }
     c.comm_used = true;
     hipError_t e = c.order ? hipSuccess : hipEventCreateWithFlags(&c.order, hipEventDisableTiming);
@@ -192,14 +194,14 @@ struct Async {
     if (e == hipSuccess) c.beside_open = false;
     return (int)e;
   }
-  // the call's work is on its stream
+  // the call's work is on its stream, or the part of it in front of the launch that failed
   int launched(int rc) {
-    if (here && rc == MEP_OK) {
+    if (here && ordered) {
       hipError_t e = c.beside ? hipSuccess : hipEventCreateWithFlags(&c.beside, hipEventDisableTiming);
       if (e == hipSuccess) e = hipEventRecord(c.beside, stream);
       c.beside_open = e == hipSuccess;
       c.beside_on = stream;
-      rc = (int)e;
+      if (rc == MEP_OK) rc = (int)e;
     }
     if (lock.owns_lock()) lock.unlock();
     return rc;

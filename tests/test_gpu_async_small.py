@@ -134,6 +134,30 @@ def test_call_of_another_thread_while_one_comes_to_the_communication_stream(cuda
         assert done.query() and torch.equal(out, want)
 
 
+def test_part_of_a_call_that_fails_keeps_its_place(cuda):
+    """A call whose second launch is refused leaves its first one on the caller's stream: later calls come behind it.
+    (The planner has run when the dispatch is refused: the context says that a rank's weight slots lie one apart.)"""
+    from moonep_amd.api import _native_context
+
+    S, H = 200, 1024
+    world, buf, (x, _), w, topk, counts = _make(cuda, S, H)
+    mine = topk[1].contiguous()
+    want = buf.dispatch(x, None, mine, counts, zero_copy=True)[0].clone()
+    buf._native = _native_context({**buf._ctx, "meta_chunk_padded": 1}, buf._comm_stream)
+    a = torch.cuda.Stream()
+    for b in [torch.cuda.Stream() for _ in range(6)]:   # some share a hardware queue with the first
+        torch.cuda.synchronize()
+        with torch.cuda.stream(a):
+            torch.cuda._sleep(20_000_000)
+            with pytest.raises(RuntimeError, match="mep_dispatch failed"):
+                buf.dispatch(x, w, mine, counts, zero_copy=True, async_finish=True)
+            first = a.record_event()
+        with torch.cuda.stream(b):
+            rows, _, _, _, done = buf.dispatch(x, None, mine, counts, zero_copy=True, async_finish=True)
+        done.synchronize()
+        assert first.query() and torch.equal(rows, want)
+
+
 def test_memory_of_another_stream_outlives_the_call(cuda):
     """Tensors that were allocated on a stream other than the caller's may be dropped as soon as the call returns: their
     memory is not handed out again while the call's work is to come."""
