@@ -142,8 +142,15 @@ struct Async {
       Py_XDECREF(o);
       if (PyErr_Occurred()) throw python_error();
     }
-    here = on && moved <= kBeside;
+    here = on && moved <= kBeside && !external();
     stream = on ? c.comm_raw : callers();
+  }
+  // A stream that torch did not make (its id is its handle) may end before the memory that is recorded on it, which the
+  // allocator then still touches it for, and before the calls that are to come behind its own: another of the
+  // same handle may have taken its place.  Nothing is kept by it.
+  bool external() const {
+    const c10::hip::HIPStream s = c10::hip::getCurrentHIPStream(c.hidden_buf.device().index());
+    return s.stream() && s.id() == (c10::StreamId)(intptr_t)s.stream();
   }
   hipStream_t callers() const { return c10::hip::getCurrentHIPStream(c.hidden_buf.device().index()).stream(); }
   // `on_stream` behind the last call that stayed on its caller's stream

@@ -1,11 +1,14 @@
 """Small asynchronous calls, which stay on their caller's stream while the communication stream is idle: the same
 results as synchronous ones on both sides of the bound, and the order that one stream for all calls would give."""
 
+import ctypes
 import threading
 import time
 
 import pytest
 import torch
+
+from moonep_amd import _lib
 
 pytestmark = pytest.mark.gpu
 
@@ -156,6 +159,34 @@ def test_part_of_a_call_that_fails_keeps_its_place(cuda):
             rows, _, _, _, done = buf.dispatch(x, None, mine, counts, zero_copy=True, async_finish=True)
         done.synchronize()
         assert first.query() and torch.equal(rows, want)
+
+
+def test_streams_of_others_may_end(cuda):
+    """Calls on a stream that torch did not make go through the communication stream: the allocator is not told of a stream that
+    may end before the memory does, and nothing is kept by its handle."""
+    S, H = 200, 1024
+    world, buf, (x, _), w, topk, counts = _make(cuda, S, H)
+    mine = topk[1].contiguous()
+    want = buf.dispatch(x, w, mine, counts, zero_copy=True)[0].clone()
+    lib = _lib.lib()
+    for _ in range(6):    # some share a hardware queue with the communication stream
+        handle = ctypes.c_void_p()
+        _lib.check(lib.mep_stream_create_limited(64, ctypes.byref(handle)), "mep_stream_create_limited")
+        copy, weights = x.clone(), w.clone()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(buf._comm_stream):
+            torch.cuda._sleep(20_000_000)
+            held = buf._comm_stream.record_event()
+        with torch.cuda.stream(torch.cuda.ExternalStream(handle.value)):
+            rows, _, _, _, done = buf.dispatch(copy, weights, mine, counts, zero_copy=True, async_finish=True)
+        done.synchronize()
+        assert held.query() and torch.equal(rows, want)
+        torch.cuda.synchronize()
+        _lib.check(lib.mep_stream_destroy(handle), "mep_stream_destroy")
+        del copy, weights
+        again = [torch.empty_like(x) for _ in range(4)]     # the allocator looks whether their memory is free
+        torch.cuda.synchronize()
+        del again
 
 
 def test_memory_of_another_stream_outlives_the_call(cuda):
