@@ -715,18 +715,12 @@ struct PlanConfig {
   int groups;
 };
 
-// Ints of scratch per rank that a caller brings: two tables of E x R for every 256 threads' tokens where those and the
-// rest are more than a kernel's LDS without asking
-size_t plan_scratch_ints(int S, int K, int E, int R) {
-  if (plan_lds_bytes(256, E, R, true) <= kLdsDefaultLimit) return 0;
-  const int tok_per_wg = 256 / K;
-  return (size_t)((S + tok_per_wg - 1) / tok_per_wg) * 2 * (size_t)E * R;
-}
-
 // 0 on success.  1024 threads with all tables in LDS wherever that holds them, on a CU's whole LDS too: a workgroup
 // of 256 resolves a fourth of the tokens, so four times as many rebuild the plan, and tables in scratch memory are
-// latencies of the memory in its chain.  us, planner of 4096 tokens, K = 8 (cache warming included), 256 threads ->
-// 1024: E = 768, R = 16 30.3 -> 14.0.
+// latencies of the memory in its chain.  us, 256 threads -> 1024, one rank planned (all ranks in one launch): tables
+// that 256 threads have in 64 KB, E = 224, R = 32, 64 tokens 25 -> 21 (25 -> 21), 4096 tokens 27 -> 24 (232 -> 89); tables in
+// scratch, E = 672, R = 24, 64 tokens 29 -> 17 (31 -> 18), 4096 tokens 37 -> 20 (291 -> 55).  Of 160 sizes, 1 to 16384 tokens, R = 1 to
+// 128, E from the smallest to the largest that the choice concerns, none is slower but for R = 1 (E = 1280 17.6 -> 18.1 at worst).
 int plan_config(int S, int K, int E, int R, PlanConfig* c) {
   if (plan_lds_bytes(1024, E, R, true) <= kLdsOptInLimit) {
     c->nt = 1024; c->lds_tables = true;
@@ -742,13 +736,18 @@ int plan_config(int S, int K, int E, int R, PlanConfig* c) {
   return MEP_OK;
 }
 
+// two tables of E x R for every workgroup whose LDS does not hold them
+size_t plan_scratch_bytes(const PlanConfig& c, int E, int R, int nranks) {
+  return c.lds_tables ? 0 : (size_t)c.groups * nranks * 2 * (size_t)E * R * sizeof(int);
+}
+
 }  // namespace
 
 extern "C" size_t mep_plan_scratch_bytes(int S, int K, int E, int R, int nranks) {
   PlanConfig c;
   if (S <= 0 || K <= 0 || K > 32 || E <= 0 || R <= 0 || nranks <= 0) return 0;
   if (plan_config(S, K, E, R, &c) != MEP_OK) return 0;
-  return plan_scratch_ints(S, K, E, R) * nranks * sizeof(int);
+  return plan_scratch_bytes(c, E, R, nranks);
 }
 
 namespace {
@@ -835,7 +834,7 @@ int plan_launch(const int32_t* tpe_RE, const int32_t* topk_nSK, int rank0, int n
   PlanConfig c;
   int rc = plan_config(S, K, E, R, &c);
   if (rc != MEP_OK) return rc;
-  if (const size_t need = plan_scratch_ints(S, K, E, R) * nranks * sizeof(int)) {
+  if (const size_t need = plan_scratch_bytes(c, E, R, nranks)) {
     MEP_REQUIRE(scratch && scratch_bytes >= need, MEP_ERR_SCRATCH);
     MEP_REQUIRE((uintptr_t)scratch % 16 == 0, MEP_ERR_ALIGNMENT);
   }

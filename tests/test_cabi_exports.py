@@ -43,7 +43,8 @@ def test_argument_validation_needs_no_device():
     assert lib.mep_combine(None, 0, None, 0, None, None, None, 4, 64, 2, 2, 64, 0, None) == -1
     assert lib.mep_grad_reduce(None, None, 0, None, 0, 4, 2, 16, 0, None) == -1
     assert lib.mep_plan_scratch_bytes(4096, 8, 256, 8, 1) == 0          # tables fit in LDS
-    assert lib.mep_plan_scratch_bytes(256, 1, 2050, 2, 2) > 0           # they do not
+    assert lib.mep_plan_scratch_bytes(256, 1, 2050, 2, 2) == 0          # in a CU's whole LDS
+    assert lib.mep_plan_scratch_bytes(256, 1, 2860, 2, 2) > 0           # they do not
     assert lib.mep_dedup_scratch_bytes(4096, 8) >= 4096 * 8 * 4
 
 
@@ -75,8 +76,8 @@ def test_error_codes_for_unsupported_shapes_alignment_and_scratch():
     assert plan(R=3) == -1                       # E not divisible by R
     assert plan(NvS=4) == -2                     # NvS below S*K
     assert plan(R=2, NvS=1 << 30) == -2          # R*NvS does not fit the int32 encoding
-    assert plan(E=2050, S=256, K=1, NvS=1024) == -3        # planner tables need caller scratch
-    assert plan(E=2050, S=256, K=1, NvS=1024, scratch=A + 4, sbytes=1 << 30) == -4   # misaligned scratch
+    assert plan(E=2860, S=256, K=1, NvS=1024) == -3        # planner tables need caller scratch
+    assert plan(E=2860, S=256, K=1, NvS=1024, scratch=A + 4, sbytes=1 << 30) == -4   # misaligned scratch
     assert plan(E=1 << 16, R=2, S=256, K=1, NvS=1024, scratch=A, sbytes=1 << 40) == -2  # beyond the LDS limit
     assert plan(E=5816, R=8, S=256, K=1, NvS=1024, scratch=A, sbytes=1 << 40) == -2     # one step beyond it (E = 5808 fills the 160 KB)
     assert lib.mep_plan_warm(A, A, 0, 4, 2, 8, 2, 8, 64, A, A, A, A, A, None, 0, A + 4, 64, None) == -4  # misaligned warm range

@@ -1,5 +1,5 @@
-"""The planner with more than 64 KB of tables: those that fill a CU's LDS, those just beyond it, and what of the
-scratch that callers bring for them is asked for as before."""
+"""The planner with more than 64 KB of tables: those that fill a CU's LDS and those just beyond it, the only ones
+that callers bring scratch for."""
 
 import numpy as np
 import pytest
@@ -26,8 +26,8 @@ def test_large_tables_match_the_oracle(cuda, S, K, E, R, tp):
     topk = torch.stack([routing.popularity_biased(S, K, E, R, r, 0.7, seed=5) for r in range(R)])
     tpe = routing.tokens_per_expert(topk, E)
     gp, plans, dst = oracle_world_plan(topk.numpy(), tpe.numpy(), tp)
-    old_tables = 4 * ((6 + 1) * E + 6 * R + 256 + 2 * E * R)
-    want = 0 if old_tables <= 65536 else -(-S // (256 // K)) * 2 * E * R * 4
+    tables = 4 * ((6 + 4) * E + 6 * R + 1024 + 2 * E * R)
+    want = 0 if tables <= 163840 else -(-S // (256 // K)) * 2 * E * R * 4
     assert _lib.lib().mep_plan_scratch_bytes(S, K, E, R, 1) == want
     buf = Buffer(S, 16, K, E, R, token_padding=tp, rank=0)
     dst_all, cu, etc, zfr, stats = launch_planning_all_ranks(buf._require_ctx(), topk.to(cuda), tpe.to(cuda))
