@@ -861,6 +861,15 @@ __device__ __forceinline__ void stream_tile_kn(const GemmArgs& a, char* gsm, int
     ++kl;
     ws = ws == (D - 1) * kStageBytes ? 0 : ws + kStageBytes;
   };
+  // row scales before all other loads, as in stream_tile (dy * down with them, 12 blocks of 1024 x 1024 13.9 -> 13.2 us, 4 of K =
+  // 5632, 768 columns 43.5 -> 42.6, 18 of K = 4096, 2048 columns 66.6 -> 65.3)
+  const int m = m0 + 32 * rb + 4 * half;
+  mep_f32x4 scale[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    scale[q] = mep_f32x4{1.0f, 1.0f, 1.0f, 1.0f};
+    if (!DUAL && a.scale) scale[q] = *(const mep_f32x4_any*)(a.scale + m + 8 * q);
+  }
 #pragma unroll
   for (int k = 0; k < D - 1; ++k) issue();
 
@@ -913,16 +922,13 @@ __device__ __forceinline__ void stream_tile_kn(const GemmArgs& a, char* gsm, int
   mep_bar();               // the next tile may be loaded
 
   // acc[i][v] is row 32 rb + 8 (v / 4) + 4 half + v % 4, column 32 uh + l31 of unit i
-  const int m = m0 + 32 * rb + 4 * half;
   uint16_t* c = a.C + (size_t)(m + (lane & 1)) * a.N + 64 * unit0 + 32 * uh + (l31 & ~1);
 #pragma unroll
-  for (int v = 0; v < 16; v += 2) {
-    const int dr = 8 * (v >> 2) + (v & 3);
-    float s0 = 1.0f, s1 = 1.0f;
-    if (!DUAL && a.scale) { s0 = a.scale[m + dr]; s1 = a.scale[m + dr + 1]; }
+  for (int v = 0; v < 16; v += 2)
 #pragma unroll
-    for (int i = 0; i < NU; ++i) store_two_rows(c + (size_t)dr * a.N + 64 * i, s0 * acc[i][v], s1 * acc[i][v + 1]);
-  }
+    for (int i = 0; i < NU; ++i)
+      store_two_rows(c + (size_t)(8 * (v >> 2) + (v & 3)) * a.N + 64 * i, scale[v >> 2][v & 3] * acc[i][v],
+                     scale[v >> 2][(v & 3) + 1] * acc[i][v + 1]);
 }
 
 template <int MODE, bool KN>
