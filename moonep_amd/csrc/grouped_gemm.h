@@ -147,8 +147,7 @@ __device__ __forceinline__ void mep_tr_issue(T& x, uint32_t lds, int offset) {
 // the zeros at times when nobody multiplied.  us, that order -> this: 64 experts of 2048 x 1024 on 8 ranks, 512 rows
 // each 645 -> 545 (2.6 -> 1.4 GB fetched), 16 of 4096 x 2048 with 2048 rows each and as many empty slots 1730 -> 1640,
 // 4 of 2560 x 512 with 5443 250 -> 172.  An eighth of the whole list by work to each XCD fetches less, 0.8 instead of
-// 1.4 GB, and takes longer: 617, 1680, 172.  Sizes that are not faster: few tiles of few steps beside as many of
-// zeros, 34 groups of 512 x 512 with 128 rows and 30 empty 37 -> 41.)
+// 1.4 GB, and takes longer: 617, 1680, 172.)
 constexpr int kProducts = 3;
 struct WgradMap {
   int tiles, rows, other;   // tiles of an output; of its longer dimension, of the shorter one
@@ -189,8 +188,14 @@ struct WgradMap {
 // 2048 x 1024, 512 rows each, 708 -> 652 us, of 16 of 4096 x 2048, 2048 rows each, 1890 -> 1778).  An XCD's
 // workgroups are sets of a.width that walk its tiles together, moving on by one place from round to round;
 // the sets share the rounds, whose number is only known here, evenly.
+// a.rounds: the tiles of all groups, with rows or without, stay in their places, as many for a set, and nobody
+// looks for the groups with rows first: what that takes, 1 to 3 us, is not made up for where a workgroup has one tile, of
+// whatever kind.  216 sizes of one round, 4 to 128 groups of 256 x 256 to 2048 x 1024, 128 to 1024 rows in an
+// eighth, half or all of them, against the order by products: the list 0.96 to 1.27 times its time, 1.03 on
+// average, this 0.72 to 1.09, 0.96 (4 of 256 x 256 with 128 rows 10.1, 13.0 and 9.6 us).  162 sizes of 2 to 16 rounds: the list
+// 0.94, 1.02 where all groups have rows, this 0.98.
 constexpr int kListed = 64;           // most tiles of a workgroup
-constexpr int kTabled = 64 * 4096;    // most groups in the tables (100 KB)
+constexpr int kTabled = 64 * 4096;    // most groups in the tables (100 KB); more stay in their places
 typedef __attribute__((address_space(1))) float mep_global_f32;
 template <bool TN>
 struct WgradTiles {
@@ -222,105 +227,111 @@ struct WgradTiles {
   }
   // lds: the kernel's; free again when this returns in all waves
   __device__ __forceinline__ WgradTiles(const GemmArgs& a_, const WgradMap* of, char* lds) : a(a_), map(*of) {
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const int chunks = (a.G + 63) / 64;
-    int beg = 0, steps = steps_of(lane, &beg);
-    const int xcd = blockIdx.x & 7, q = blockIdx.x >> 3;
-    const int all_of = (int)(gridDim.x >> 3), sets = mep_quotient(all_of, a.width), set = mep_quotient(q, a.width), w = q - set * a.width;
-    // groups with rows and groups that come out as zeros: how many, and of every 64 groups which and how many in
-    // front of them.  More than 64 groups: each wave looks at its part of them (one after the other, 1536 groups
-    // would be 24 latencies of the memory).
-    uint64_t some = __ballot(steps > 0), none = __ballot(steps < 0);
-    int full = __popcll(some), empty = __popcll(none), sum = 0;
-    uint64_t* const masks = (uint64_t*)lds;                     // [2 chunks]
-    int2* const before = (int2*)(lds + 16 * (size_t)chunks);    // [chunks + 8], the waves' sums behind
-    // more groups than the tables hold: all are in the list, and those without rows are passed by or zeroed in their turn
-    const bool listed = a.G <= kTabled;
-    if (!listed) {
-      full = a.G;
-      empty = 0;
-    } else if (chunks > 1) {
-      full = empty = 0;
-      const int mine = wave * chunks / 8, end = (wave + 1) * chunks / 8;
-      for (int c = mine; c < end; ++c) {
-        steps = steps_of(64 * c + lane, &beg);
-        some = __ballot(steps > 0); none = __ballot(steps < 0);
-        if (lane == 0) { masks[2 * c] = some; masks[2 * c + 1] = none; before[c] = make_int2(full, empty); }
-        full += __popcll(some); empty += __popcll(none);
-      }
-      if (lane == 0) before[chunks + wave] = make_int2(full, empty);
-      __syncthreads();
-      full = empty = 0;
-#pragma unroll
-      for (int k = 0; k < 8; ++k) { const int2 v = before[chunks + k]; full += v.x; empty += v.y; }
-      full = __builtin_amdgcn_readfirstlane(full); empty = __builtin_amdgcn_readfirstlane(empty);
-    } else {
-      sum = __builtin_amdgcn_readlane(mep_wave_incl_scan(max(steps, 0)), 63);
-    }
-    // This workgroup's tiles, a lane each.  The sets share the rounds of the groups with rows evenly, and all
-    // workgroups the tiles of zeros (as a tail of the list, when nothing is left to multiply, those of 15 of 32 groups
-    // of 4096 x 2048 are 100 us of 1750), but in a launch of one set the workgroups that have a tile less than the
-    // others first take as many of them as make up for it, a tile of zeros being the time of some six K steps.
-    const int tiles = map.count(xcd, full), blank = map.count(xcd, empty), total = mep_quotient(tiles + a.width - 1, a.width);
-    const int base = mep_quotient(total, sets), over = total - base * sets;
-    const int first_round = set * base + min(set, over), rounds = base + (set < over);
-    int extra = 0, place = q, from = 0, own = 0;
-    if (sets == 1 && blank) {
-      const int turned = max(total - 1, 0), more = tiles - turned * a.width, less = a.width - more;
-      place = w + turned - mep_quotient(w + turned, a.width) * a.width;
-      if (less) {
-        extra = min(blank, less * min(1 + mep_quotient(sum, 6 * max(full, 1)), kListed / 4));
-        const int each = mep_quotient(extra, less), more_of = extra - each * less, light = place - more;
-        if (light >= 0) {
-          from = light * each + min(light, more_of);
-          own = each + (light < more_of);
-        }
-      }
-    }
-    const int base2 = mep_quotient(blank - extra, all_of), over2 = blank - extra - base2 * all_of;
-    const int back = all_of - 1 - place;
-    const int from2 = extra + back * base2 + min(back, over2), own2 = base2 + (back < over2);
-    const int r = first_round + lane, z = lane - rounds;
-    const bool zero = z >= 0;
-    int at = zero ? (z < own ? from + z : from2 + z - own) : r * a.width + w + r - mep_quotient(w + r, a.width) * a.width;
-    bool live = zero ? z < own + own2 : at < tiles;
-    if (!live) at = 0;
-    // its group: among those with rows (zeros: without) the k-th
-    const int per = map.tiles * map.n, octet = mep_quotient(at, per), pos = at - octet * per + map.begin(xcd);
-    const int run = mep_quotient(8 * pos + 7, per);  // the last that begins at or before this place
-    int k = 8 * octet + run - xcd, g;
-    const int item = pos - map.begin(run) + map.begin(run & 7);
-    int first, length;
-    if (!listed) {
+    const int lane = threadIdx.x & 63, xcd = blockIdx.x & 7, q = blockIdx.x >> 3;
+    const int set = mep_quotient(q, a.width), w = q - set * a.width;
+    auto turn = [&](int r) { return r * a.width + w + r - mep_quotient(w + r, a.width) * a.width; };
+    const int per = map.tiles * map.n;
+    int k, g, item, first, length;
+    bool live;
+    // the XCD's tile `at` of a list: which of the groups, and its place among that group's
+    auto group = [&](int at) {
+      const int octet = mep_quotient(at, per), pos = at - octet * per + map.begin(xcd);
+      const int run = mep_quotient(8 * pos + 7, per);  // the last that begins at or before this place
+      k = 8 * octet + run - xcd;
+      item = pos - map.begin(run) + map.begin(run & 7);
+    };
+    if (a.rounds) {  // all groups in their places
+      const int r = set * a.rounds + lane, at = turn(r);
+      live = lane < a.rounds && at < map.count(xcd, a.G);
+      group(live ? at : 0);
       g = live ? k : 0;
       length = steps_of(g, &first);
       live = live && length;
-    } else if (chunks > 1) {
-      // the wave whose part holds it, the chunk in there
-      int c = 0, end = 0;
-#pragma unroll
-      for (int v = 0; v < 8; ++v) {
-        const int2 part = before[chunks + v];
-        const int n = zero ? part.y : part.x;
-        const bool here = c == end && k < n;
-        if (here) { c = v * chunks / 8; end = (v + 1) * chunks / 8; }
-        else if (c == end) k -= n;
-      }
-      while (end - c > 1) {  // the last chunk with no more than k in front of it
-        const int m = (c + end) / 2;
-        const int2 b = before[m];
-        if ((zero ? b.y : b.x) <= k) c = m;
-        else end = m;
-      }
-      const int2 b = before[c];
-      g = 64 * c + nth(masks[2 * c + zero], k - (zero ? b.y : b.x));
-      if (!live) g = 0;
-      length = steps_of(g, &first);
-      __syncthreads();  // the tables have been read
     } else {
-      g = live ? nth(zero ? none : some, k) : 0;
-      first = __shfl(beg, g);
-      length = __shfl(steps, g);
+      // groups with rows and groups that come out as zeros: how many, and of every 64 groups which and how many in
+      // front of them.  More than 64 groups: each wave looks at its part of them (one after the other, 1536 groups
+      // would be 24 latencies of the memory).
+      const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), chunks = (a.G + 63) / 64;
+      int beg = 0, steps = steps_of(lane, &beg);
+      uint64_t some = __ballot(steps > 0), none = __ballot(steps < 0);
+      int full = __popcll(some), empty = __popcll(none), sum = 0;
+      uint64_t* const masks = (uint64_t*)lds;                     // [2 chunks]
+      int2* const before = (int2*)(lds + 16 * (size_t)chunks);    // [chunks + 8], the waves' sums behind
+      if (chunks > 1) {
+        full = empty = 0;
+        const int mine = wave * chunks / 8, end = (wave + 1) * chunks / 8;
+        for (int c = mine; c < end; ++c) {
+          steps = steps_of(64 * c + lane, &beg);
+          some = __ballot(steps > 0); none = __ballot(steps < 0);
+          if (lane == 0) { masks[2 * c] = some; masks[2 * c + 1] = none; before[c] = make_int2(full, empty); }
+          full += __popcll(some); empty += __popcll(none);
+        }
+        if (lane == 0) before[chunks + wave] = make_int2(full, empty);
+        __syncthreads();
+        full = empty = 0;
+#pragma unroll
+        for (int v = 0; v < 8; ++v) { const int2 n = before[chunks + v]; full += n.x; empty += n.y; }
+        full = __builtin_amdgcn_readfirstlane(full); empty = __builtin_amdgcn_readfirstlane(empty);
+      } else {
+        sum = __builtin_amdgcn_readlane(mep_wave_incl_scan(max(steps, 0)), 63);
+      }
+      // This workgroup's tiles, a lane each.  The sets share the rounds of the groups with rows evenly, and all
+      // workgroups the tiles of zeros (as a tail of the list, when nothing is left to multiply, those of 15 of 32 groups
+      // of 4096 x 2048 are 100 us of 1750), but in a launch of one set the workgroups that have a tile less than the
+      // others first take as many of them as make up for it, a tile of zeros being the time of some six K steps.
+      const int all_of = (int)(gridDim.x >> 3), sets = mep_quotient(all_of, a.width);
+      const int tiles = map.count(xcd, full), blank = map.count(xcd, empty), total = mep_quotient(tiles + a.width - 1, a.width);
+      const int base = mep_quotient(total, sets), over = total - base * sets;
+      const int first_round = set * base + min(set, over), rounds = base + (set < over);
+      int extra = 0, place = q, from = 0, own = 0;
+      if (sets == 1 && blank) {
+        const int turned = max(total - 1, 0), more = tiles - turned * a.width, less = a.width - more;
+        place = w + turned - mep_quotient(w + turned, a.width) * a.width;
+        if (less) {
+          extra = min(blank, less * min(1 + mep_quotient(sum, 6 * max(full, 1)), kListed / 4));
+          const int each = mep_quotient(extra, less), more_of = extra - each * less, light = place - more;
+          if (light >= 0) {
+            from = light * each + min(light, more_of);
+            own = each + (light < more_of);
+          }
+        }
+      }
+      const int base2 = mep_quotient(blank - extra, all_of), over2 = blank - extra - base2 * all_of;
+      const int back = all_of - 1 - place;
+      const int from2 = extra + back * base2 + min(back, over2), own2 = base2 + (back < over2);
+      const int z = lane - rounds;
+      const bool zero = z >= 0;
+      const int at = zero ? (z < own ? from + z : from2 + z - own) : turn(first_round + lane);
+      live = zero ? z < own + own2 : at < tiles;
+      group(live ? at : 0);
+      // that group: among those with rows (zeros: without) the k-th
+      if (chunks > 1) {
+        // the wave whose part holds it, the chunk in there
+        int c = 0, end = 0;
+#pragma unroll
+        for (int v = 0; v < 8; ++v) {
+          const int2 part = before[chunks + v];
+          const int n = zero ? part.y : part.x;
+          const bool here = c == end && k < n;
+          if (here) { c = v * chunks / 8; end = (v + 1) * chunks / 8; }
+          else if (c == end) k -= n;
+        }
+        while (end - c > 1) {  // the last chunk with no more than k in front of it
+          const int m = (c + end) / 2;
+          const int2 b = before[m];
+          if ((zero ? b.y : b.x) <= k) c = m;
+          else end = m;
+        }
+        const int2 b = before[c];
+        g = 64 * c + nth(masks[2 * c + zero], k - (zero ? b.y : b.x));
+        if (!live) g = 0;
+        length = steps_of(g, &first);
+        __syncthreads();  // the tables have been read
+      } else {
+        g = live ? nth(zero ? none : some, k) : 0;
+        first = __shfl(beg, g);
+        length = __shfl(steps, g);
+      }
     }
     const int pr = mep_quotient(item, map.tiles);
     int sl, u, m0, n0;

@@ -1195,6 +1195,7 @@ int wgrad_pp_launch(GemmArgs a, WgradMap map, hipStream_t st) {
   const int64_t rounds = (per_xcd + a.width - 1) / a.width, per_group = (a.rank_rows ? a.rank_rows : a.ld) / kBK / a.Gr;
   const int64_t steps = rounds * std::max<int64_t>(per_group + (a.skip_from < a.Gr ? 0 : 3), 1);
   const int64_t sets = std::min(rounds, std::max((steps + kPSteps / 2) / kPSteps, rounds / (kListed * 3 / 4 - 4) + 1));
+  a.rounds = rounds == 1 || a.G > kTabled ? (int)((rounds + sets - 1) / sets) : 0;  // WgradTiles
   hipLaunchKernelGGL((gemm_pp_kernel<kModeWgrad, TN, TN>), dim3(8 * (unsigned)(a.width * sets)), dim3(kPThreads), kPLds, st, a, map);
   return mep_launch_status();
 }

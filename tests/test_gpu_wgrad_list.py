@@ -1,5 +1,5 @@
-"""The weight gradients' list of tiles beside more groups than one wave looks at: which groups have rows, which
-come out as zeros and which are left alone."""
+"""The weight gradients' list of tiles: which groups have rows, which come out as zeros and which are left alone.  Beside
+more groups than one wave looks at, of one round, where all groups stay in their places, and of several."""
 
 import pytest
 import torch
@@ -12,9 +12,19 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("full", ["few", "half", "all", "last"])
 @pytest.mark.parametrize("G", [64, 66, 130, 1030])
 def test_groups_with_and_without_rows(cuda, G, full):
+    check(cuda, G, full, 512, 256)
+
+
+@pytest.mark.parametrize("full", ["few", "half", "all", "last"])
+@pytest.mark.parametrize("G,M,N", [(32, 1024, 512), (34, 1024, 512), (64, 512, 1024), (66, 1024, 512), (256, 256, 256), (258, 256, 256)])
+def test_both_sides_of_one_round(cuda, G, M, N, full):
+    check(cuda, G, full, M, N)
+
+
+def check(cuda, G, full, M, N):
     """Against the fp64 product: a sum of n products in fp32, in any order, is off by at most n 2^-24 of the
     sum of their magnitudes."""
-    print(f"wgrad list, {G} groups, rows in {full}", flush=True)
+    print(f"wgrad list, {G} groups of {M} x {N}, rows in {full}", flush=True)
     g = torch.Generator().manual_seed(G)
     share = {"few": 0.05, "half": 0.5, "all": 1.0, "last": 0.0}[full]
     lens = ((torch.rand(G, generator=g) < share) * torch.randint(1, 3, (G,), generator=g)).tolist()
@@ -22,8 +32,8 @@ def test_groups_with_and_without_rows(cuda, G, full):
     ends = (torch.tensor(lens).cumsum(0) * 128).to(torch.int32).to(cuda)
     rows = 128 * (sum(lens) + 1)
     gc = torch.Generator(device=cuda).manual_seed(G)
-    x1, x2 = (torch.randn(rows, n, generator=gc, device=cuda).to(torch.bfloat16) for n in (512, 256))
-    got = torch.full((G, 512, 256), float("nan"), device=cuda)
+    x1, x2 = (torch.randn(rows, n, generator=gc, device=cuda).to(torch.bfloat16) for n in (M, N))
+    got = torch.full((G, M, N), float("nan"), device=cuda)
     kept = got.clone()
     ffn.launch_grouped_gemm_wgrad_tn(x1, x2, ends, got)
     ffn.launch_grouped_gemm_wgrad_tn(x1, x2, ends, kept, skip_empty_from=G // 3)
