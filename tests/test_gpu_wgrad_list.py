@@ -1,5 +1,6 @@
 """The weight gradients' list of tiles: which groups have rows, which come out as zeros and which are left alone.  Beside
-more groups than one wave looks at, of one round, where all groups stay in their places, and of several."""
+more groups than one wave looks at, of one round, where all groups stay in their places, and of several, and
+beside more groups than there are tables for."""
 
 import pytest
 import torch
@@ -49,3 +50,28 @@ def check(cuda, G, full, M, N):
     assert bool((got[empty] == 0).all())
     assert torch.equal(kept[~kept_alone], got[~kept_alone])
     assert bool(kept[kept_alone].isnan().all())
+
+
+@pytest.mark.parametrize("skip", [False, True])
+def test_more_groups_than_the_tables_hold(cuda, skip):
+    """262146 groups, five with rows: 69 GB of gradients, in which the others come out as zeros or are not touched."""
+    G, full = 262146, (0, 1, 70_000, 262_143, 262_145)
+    if torch.cuda.mem_get_info()[0] < 90 << 30:
+        pytest.skip("needs 69 GB")
+    print(f"wgrad list, {G} groups, skip={skip}", flush=True)
+    lens = torch.zeros(G, dtype=torch.int32)
+    lens[list(full)] = 128
+    ends = lens.cumsum(0).to(torch.int32).to(cuda)
+    g = torch.Generator(device=cuda).manual_seed(2)
+    x1, x2 = (torch.randn(128 * len(full), 256, generator=g, device=cuda).to(torch.bfloat16) for _ in range(2))
+    out = torch.full((G, 256, 256), 3.0, device=cuda)
+    ffn.launch_grouped_gemm_wgrad_tn(x1, x2, ends, out, skip_empty_from=0 if skip else None)
+    torch.cuda.synchronize()
+    for at, i in enumerate(full):
+        a, b = (x[128 * at:128 * (at + 1)].double() for x in (x1, x2))
+        assert bool(((out[i].double() - a.t() @ b).abs() <= 2.0 ** -17 * (a.abs().t() @ b.abs())).all()), f"group {i}"
+        out[i].fill_(3.0 if skip else 0.0)
+    low, high = torch.aminmax(out)
+    assert float(low) == float(high) == (3.0 if skip else 0.0)
+    del out
+    torch.cuda.empty_cache()
