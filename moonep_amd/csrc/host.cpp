@@ -41,13 +41,20 @@ struct Ctx {
   hipStream_t comm_raw = nullptr;
   hipEvent_t order = nullptr;
   // A call's ordering and its launches belong together.  comm_used: something may be on the communication stream.
-  // coming: callers of comes_to_comm whose work is not all there.  beside: behind the last asynchronous call that stayed on its caller's stream, until the communication stream
-  // is ordered behind it.
+  // coming: callers of comes_to_comm whose work is not all there.  beside_open: the last asynchronous call that stayed on its
+  // caller's stream, beside_on, until the communication stream is ordered behind it; beside, where it is recorded
+  // (beside_kept), lies behind that call.  several: such calls came from more than one stream.
   std::mutex order_mutex;
-  bool comm_used = false, beside_open = false;
+  bool comm_used = false, beside_open = false, beside_kept = false, several = false;
   int coming = 0;
   hipEvent_t beside = nullptr;
   hipStream_t beside_on = nullptr;
+  hipError_t keep_beside() {
+    hipError_t e = beside ? hipSuccess : hipEventCreateWithFlags(&beside, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipEventRecord(beside, beside_on);
+    beside_kept = e == hipSuccess;
+    return e;
+  }
   PyObject *plan_type = nullptr, *hidden_local_py = nullptr, *no_map_token = nullptr, *event_type = nullptr,
            *comm_py = nullptr, *empty = nullptr;
   PyObject *current_stream = nullptr, *caller_py = nullptr;  // torch's function; what it answered for the stream caller_id
@@ -124,8 +131,11 @@ struct RelaxedCapture {
 // stream and back takes 22 us of the GPU, and on the host some 40 a call: an event's record and the wait of
 // another stream for it, 16 us while the event has not come, and a record for every tensor that is freed after use on a
 // stream that is not its own.  Up to this size the call itself is no longer than the crossing.  us a pass of dispatch and
-// combine, each waited for, on the communication stream -> on the caller's, H = 2048, K = 8: 8 tokens 115 -> 35, 512 114 ->
-// 37, 1536 (48 MiB of copies) 117 -> 45; synchronous calls 12, 21 and 30.
+// combine, each waited for, H = 2048, K = 8, on the communication stream -> on the caller's, the default one, alone and with a
+// product of 60, 115 and 370 us of the caller's own behind each call, which the communication stream works beside: 8 tokens
+// 102 -> 30, 160 -> 131, 205 -> 204, 642 -> 643; 512 97 -> 29, 153 -> 135, 207 -> 208, 655 -> 651; 1536 (48 MiB of copies) 100 -> 36, 158 ->
+// 148, 223 -> 223, 670 -> 663; H = 7168 the same.  From another stream, whose calls record an event each: 8 tokens alone 36, with the
+// products 137, 211 and 649.  Synchronous calls alone: 8 tokens 16, 512 21, 1536 29.
 constexpr int64_t kBeside = (int64_t)64 << 20;
 
 // ---- asynchronous calls: the work goes to the communication stream, small calls' while that is idle to the caller's
@@ -157,7 +167,12 @@ struct Async {
   static hipError_t behind(Ctx& c, hipStream_t on_stream) {
     if (!c.beside_open || c.beside_on == on_stream) return hipSuccess;
     const RelaxedCapture relaxed;
-    const hipError_t e = asked(hipEventQuery(c.beside));
+    hipError_t e = hipSuccess;
+    if (!c.beside_kept) {
+      c.several = true;
+      if ((e = c.keep_beside()) != hipSuccess) return e;
+    }
+    e = asked(hipEventQuery(c.beside));
     return e == hipErrorNotReady ? hipStreamWaitEvent(on_stream, c.beside, 0) : e;
   }
   // after the caller's work; the allocator must not reuse what the stream still works on
@@ -204,10 +219,13 @@ struct Async {
   // the call's work is on its stream, or the part of it in front of the launch that failed
   int launched(int rc) {
     if (here && ordered) {
-      hipError_t e = c.beside ? hipSuccess : hipEventCreateWithFlags(&c.beside, hipEventDisableTiming);
-      if (e == hipSuccess) e = hipEventRecord(c.beside, stream);
-      c.beside_open = e == hipSuccess;
       c.beside_on = stream;
+      c.beside_kept = false;
+      // The default stream is there as long as the process and never under capture: behind its calls the event may be
+      // recorded when a call of another stream asks, for the first time then, since the later the more lies in front of it.
+      // (A record takes 4.5 us of the stream.)
+      const hipError_t e = !stream && !c.several ? hipSuccess : c.keep_beside();
+      c.beside_open = e == hipSuccess;
       if (rc == MEP_OK) rc = (int)e;
     }
     if (lock.owns_lock()) lock.unlock();
@@ -405,8 +423,9 @@ PyObject* py_dispatch(PyObject*, PyObject* const* args, Py_ssize_t n) {
                               c.hidden_buf.data_ptr(), c.NvS, w ? ptr<float>(c.meta_buf) : nullptr, c.wslot_stride,
                               ptr<void>(c.scratch), c.scratch.defined() ? c.scratch.nbytes() : 0, as.stream);
     } else if (rc == MEP_OK) {
-      // what is asynchronous runs beside kernels that hold CUs, GEMMs all of them: two launches even of a
-      // small call (has_all_cus in planner.hip has the figures)
+      // what is on the communication stream runs beside kernels that hold CUs, GEMMs all of them: two launches even of a
+      // small call (has_all_cus in planner.hip has the figures), and the same two where it stays on its caller's
+      // stream (one there: 8 tokens 30 -> 27 us a pass)
       what = "mep_plan";
       if (fresh)
         rc = mep_plan_fresh(ptr<int>(*tpe), ptr<int>(*topk), c.rank, c.S, c.K, c.E, c.R, c.tp, c.NvS,
@@ -831,8 +850,8 @@ PyObject* py_context(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// comes_to_comm(ctx): the communication stream, which the caller is about to use, behind the last call that stayed on its
-// caller's stream; until the caller's leaves_comm(ctx) that stream counts as busy
+// comes_to_comm(ctx): the communication stream, which the caller is about to use behind its own stream, behind the last
+// call that stayed on another; until the caller's leaves_comm(ctx) that stream counts as busy
 PyObject* py_comes_to_comm(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   Ctx* cp = n == 1 ? ctx_of(args[0]) : nullptr;
@@ -847,12 +866,15 @@ PyObject* py_comes_to_comm(PyObject*, PyObject* const* args, Py_ssize_t n) {
     c.comm_used = true;
     if (c.beside_open && captured) {  // a stream under capture cannot wait for what was not captured
       const RelaxedCapture relaxed;
-      e = hipEventSynchronize(c.beside);
-    } else {
+      if (!c.beside_kept) e = c.keep_beside();
+      if (e == hipSuccess) e = hipEventSynchronize(c.beside);
+    } else if (c.beside_on != as.callers()) {
       e = Async::behind(c, c.comm_raw);
     }
-    if (e == hipSuccess) c.beside_open = false;
-    if (e == hipSuccess) ++c.coming;
+    if (e == hipSuccess) {
+      c.beside_open = false;
+      ++c.coming;
+    }
   }
   if (failed((int)e, kOrdering)) return nullptr;
   Py_RETURN_NONE;

@@ -209,3 +209,68 @@ def test_memory_of_another_stream_outlives_the_call(cuda):
         assert not done.query() and place not in [t.data_ptr() for t in others]
         done.synchronize()
         assert torch.equal(rows, want)
+
+
+@pytest.mark.parametrize("way", ["small", "prefetch", "all ranks"])
+def test_calls_behind_those_of_the_default_stream(cuda, way):
+    """A call on the default stream, then one on another: on that stream itself, where the first call of another stream finds
+    no event behind the held one yet, and through the communication stream, as a prefetch and as a dispatch that knows every
+    rank's routing."""
+    S, H = 200, 1024
+    world, buf, (x, y), w, topk, counts = _make(cuda, S, H)
+    mine = topk[1].contiguous()
+    want = {}
+    for name, t in (("x", x), ("y", y)):
+        res, out = _pass(buf, t, w, mine, counts, False, True)
+        want[name] = res[0].clone(), out[0].clone()
+    shard = res[0]
+    local = torch.ones(E // R, 128, 128, dtype=torch.bfloat16, device=cuda)
+    pools = [torch.zeros(R, E // R, 128, 128, dtype=torch.bfloat16, device=cuda) for _ in range(3)]
+    for rounds, b in enumerate([torch.cuda.Stream() for _ in range(5)]):     # some share the default stream's hardware queue
+        print(f"{way} round {rounds}", flush=True)
+        torch.cuda.synchronize()
+        torch.cuda._sleep(20_000_000)
+        plan, ev = buf.dispatch(x, w, mine, counts, zero_copy=True, async_finish=True)[3:5]
+        expect = want["x"]
+        with torch.cuda.stream(b):
+            if way == "prefetch":
+                buf.prefetch_weight(plan, True, local_gate_weight=local, local_up_weight=local, local_down_weight=local,
+                                    gate_prefetch_buffer=pools[0], up_prefetch_buffer=pools[1], down_prefetch_buffer=pools[2])
+            elif way == "all ranks":
+                plan = buf.dispatch(y, w, topk, counts, zero_copy=True, async_finish=True)[3]
+                expect = want["y"]
+            out, _, done = buf.combine(plan, shard, zero_copy=True, async_finish=True)
+        done.synchronize()
+        assert ev.query() and torch.equal(out, expect[1])
+        torch.cuda.synchronize()
+        assert torch.equal(shard, expect[0])
+
+
+def test_capture_behind_a_call_of_the_default_stream(cuda):
+    """A call is captured while one on the default stream is still running, and without the wait that torch.cuda.graph
+    begins with: replays give what an eager call gives, and later calls keep their order."""
+    S, H = 200, 1024
+    world, buf, (x, y), w, topk, counts = _make(cuda, S, H)
+    mine = topk[1].contiguous()
+    rows_y = _pass(buf, y, w, mine, counts, True, True)[0][0].clone()
+    rows_x = _pass(buf, x, w, mine, counts, True, True)[0][0].clone()
+    a, held = torch.cuda.Stream(), x.clone()
+    with torch.cuda.stream(a):
+        buf.dispatch(y, w, mine, counts, zero_copy=True, async_finish=True)[4].wait()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda._sleep(20_000_000)
+    ev = buf.dispatch(x, w, mine, counts, zero_copy=True, async_finish=True)[4]
+    with torch.cuda.stream(a):
+        graph.capture_begin()
+        buf.dispatch(y, w, mine, counts, zero_copy=True, async_finish=True)[4].wait()
+        graph.capture_end()
+    ev.synchronize()
+    shard = buf.hidden_nvsh_buffer_view
+    for _ in range(3):
+        torch.cuda.synchronize()
+        assert torch.equal(shard, rows_x)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(shard, rows_y)
+        buf.dispatch(x, w, mine, counts, zero_copy=True, async_finish=True)[4].synchronize()
