@@ -399,9 +399,11 @@ int dispatch_launch(const void* hidden, const float* w, const int32_t* dst, cons
   dim3 grid(a.tok_blocks + a.zblocks, nranks);
   hipStream_t st = (hipStream_t)stream;
   // rows that are a whole number of 1-KiB wave tiles (H % 512 == 0, up to H = 8192) pass through registers as they
-  // are; any other H % 8 == 0 from the line that holds its first byte, 4 KB at a time (as many as the row takes
-  // at once: the same time)
+  // are; any other H % 8 == 0 from the line that holds its first byte, at most 4 KB at a time (as many as the row takes
+  // at once: the same time) and no more than the row takes (4096 tokens, K = 8, always 4 KB -> as many: H = 64 10.3 -> 8.6 us,
+  // 448 10.8 -> 8.9, 576 11.0 -> 9.9)
   const int nvec = H / 8;
+  const int pieces = (2 * H + (((uintptr_t)shards | 2 * H) & 127 ? 112 : 0) + 1023) / 1024;  // KB from a line's beginning on
   switch (nvec % 64 == 0 ? nvec / 64 : 0) {
 #define MEP_DISPATCH_CASE(NV) \
     case NV: hipLaunchKernelGGL((dispatch_kernel<NV, true>), grid, dim3(kBlock), 0, st, a); break;
@@ -410,7 +412,11 @@ int dispatch_launch(const void* hidden, const float* w, const int32_t* dst, cons
     MEP_DISPATCH_CASE(9) MEP_DISPATCH_CASE(10) MEP_DISPATCH_CASE(11) MEP_DISPATCH_CASE(12)
     MEP_DISPATCH_CASE(13) MEP_DISPATCH_CASE(14) MEP_DISPATCH_CASE(15) MEP_DISPATCH_CASE(16)
 #undef MEP_DISPATCH_CASE
-    default: hipLaunchKernelGGL((dispatch_kernel<4, false>), grid, dim3(kBlock), 0, st, a); break;
+    default:
+      if (pieces == 1) hipLaunchKernelGGL((dispatch_kernel<1, false>), grid, dim3(kBlock), 0, st, a);
+      else if (pieces == 2) hipLaunchKernelGGL((dispatch_kernel<2, false>), grid, dim3(kBlock), 0, st, a);
+      else hipLaunchKernelGGL((dispatch_kernel<4, false>), grid, dim3(kBlock), 0, st, a);
+      break;
   }
   return mep_launch_status();
 }

@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("base", [0, 16, 64, 112])
-@pytest.mark.parametrize("H", [8, 520, 1024, 2048, 2880, 4096, 4104, 6144, 8192])   # 16 bytes .. four whole pieces of 4 KB
+# 16 bytes to four whole pieces of 4 KB; both sides of what a row takes in one and in two KB from a line's beginning on
+@pytest.mark.parametrize("H", [8, 448, 456, 464, 520, 960, 968, 976, 1024, 2048, 2880, 4096, 4104, 6144, 8192])
 @pytest.mark.parametrize("one_launch", [False, True])
 def test_every_byte_of_the_shards(cuda, H, base, one_launch):
     S, K, E, R, rank, tp = 21, 3, 8, 2, 1, 16
