@@ -17,7 +17,8 @@ def test_groups_with_and_without_rows(cuda, G, full):
 
 
 @pytest.mark.parametrize("full", ["few", "half", "all", "last"])
-@pytest.mark.parametrize("G,M,N", [(32, 1024, 512), (34, 1024, 512), (64, 512, 1024), (66, 1024, 512), (256, 256, 256), (258, 256, 256)])
+@pytest.mark.parametrize("G,M,N", [(32, 1024, 512), (34, 1024, 512), (64, 512, 1024), (66, 1024, 512), (256, 256, 256), (258, 256, 256),
+                                   (30, 1280, 512), (34, 768, 768), (66, 256, 1280)])    # numbers of tiles that eight does not divide
 def test_both_sides_of_one_round(cuda, G, M, N, full):
     check(cuda, G, full, M, N)
 
