@@ -89,6 +89,19 @@ __device__ __forceinline__ void mep_acc_taken() {
 constexpr int mep_row_block(int n) { return n >> 4 << 1 | ((n ^ n >> 1) & 1); }
 constexpr int mep_weight_block(int n) { return (n >> 4 & 1 ? ~n : n) >> 1 & 7; }
 
+// Four lanes of sixteen, bank 0 .. 3: x of the banks with bit S against y of those without, at the same place in the bank.
+typedef uint32_t mep_u4 __attribute__((ext_vector_type(4)));
+template <int S>
+__device__ __forceinline__ void mep_trade(mep_u4& x, mep_u4& y) {
+  constexpr int kUp = 0x120 + (S ? 8 : 4), kDown = 0x120 + (S ? 8 : 12);  // row_ror
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const uint32_t was = x[d];
+    x[d] = (uint32_t)__builtin_amdgcn_update_dpp((int)was, (int)y[d], kUp, 0xf, S ? 0xc : 0xa, false);
+    y[d] = (uint32_t)__builtin_amdgcn_update_dpp((int)y[d], (int)was, kDown, 0xf, S ? 0x3 : 0x5, false);
+  }
+}
+
 // f(0), f(1) .. f(N - 1), the numbers as constants
 template <class F, int... I>
 __device__ __forceinline__ void mep_each(F&& f, std::integer_sequence<int, I...>) {
@@ -152,9 +165,10 @@ __global__ __launch_bounds__(kWThreads, 1) void gemm_wide_kernel(GemmArgs a) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int j = 4 * wave + q;
-      vA[q] = (uint32_t)((8 * j + r) * ldA * 2 + (kv ^ (r & 6)) * 16);
-      vB[q] = KN ? (uint32_t)((4 * j + lq) * ldB * 2 + (l15 ^ (lq << 2) ^ (q >> 1 << 1)) * 16)
-                 : (uint32_t)((8 * j + r) * ldB * 2 + (kv ^ (r & 2) ^ (q >> 1 << 2)) * 16);
+      // less what the instruction adds (no less than that: K and N are at least 64 and 128)
+      vA[q] = (uint32_t)((8 * j + r) * ldA * 2 + (kv ^ (r & 6)) * 16) - q * 1024;
+      vB[q] = (KN ? (uint32_t)((4 * j + lq) * ldB * 2 + (l15 ^ (lq << 2) ^ (q >> 1 << 1)) * 16)
+                  : (uint32_t)((8 * j + r) * ldB * 2 + (kv ^ (r & 2) ^ (q >> 1 << 2)) * 16)) - q * 1024;
     }
   }
   // where the next step of each operand is written and read
@@ -162,11 +176,13 @@ __global__ __launch_bounds__(kWThreads, 1) void gemm_wide_kernel(GemmArgs a) {
   int wA = 0, wB = kWFirstB, rA = 0, rB = kWFirstB;
   auto turnA = [](int& s) MEP_INLINE { s ^= kWStep; };
   auto turnB = [](int& s) MEP_INLINE { s = s == kWLds - kWStep ? kWFirstB : s + kWStep; };
-  auto issueA = [&](int n) MEP_INLINE {  // n = 0 .. 7
-    mep_load_lds16(qA, vA[n & 3], n >> 2 ? qhalfA : 0u, lds_w + wA + (n >> 2) * kWHalf + (n & 3) * 1024);
+  auto issueA = [&](auto c) MEP_INLINE {  // 0 .. 7
+    constexpr int n = c;
+    mep_load_lds16<0, (n & 3) * 1024>(qA, vA[n & 3], n >> 2 ? qhalfA : 0u, lds_w + wA + (n >> 2) * kWHalf);
   };
-  auto issueB = [&](int n) MEP_INLINE {
-    mep_load_lds16(n >> 2 ? pB1 : pB, vB[n & 3], n >> 2 ? halfB : 0u, lds_w + wB + (n >> 2) * kWHalf + (n & 3) * 1024);
+  auto issueB = [&](auto c) MEP_INLINE {
+    constexpr int n = c;
+    mep_load_lds16<0, (n & 3) * 1024>(n >> 2 ? pB1 : pB, vB[n & 3], n >> 2 ? halfB : 0u, lds_w + wB + (n >> 2) * kWHalf);
   };
 
   // ---- fragments: set s holds half s of a K step
@@ -218,10 +234,8 @@ __global__ __launch_bounds__(kWThreads, 1) void gemm_wide_kernel(GemmArgs a) {
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       qA = pA; qhalfA = halfA;
-#pragma unroll
-      for (int n = 0; n < 8; ++n) issueA(n);
-#pragma unroll
-      for (int n = 0; n < 8; ++n) issueB(n);
+      mep_each<8>(issueA);
+      mep_each<8>(issueB);
       turnA(wA); turnB(wB);
       on();
       if (--left == 0) turned();
@@ -270,7 +284,7 @@ __global__ __launch_bounds__(kWThreads, 1) void gemm_wide_kernel(GemmArgs a) {
       mep_each<NM>([&](auto c) MEP_INLINE {
         constexpr int n = c;
         if constexpr (n % R == 0) { read(1, n / R, at_rows); __builtin_amdgcn_sched_barrier(0); }
-        if constexpr (n % L == L / 2 + 1) { issueB(n / L); __builtin_amdgcn_sched_barrier(0); }
+        if constexpr (n % L == L / 2 + 1) { issueB(std::integral_constant<int, n / L>{}); __builtin_amdgcn_sched_barrier(0); }
         if constexpr (n == NM - 2) {
           turnA(rA); turnB(rB);
           at_rows = (kt + 1 < KT ? at_cur : at_next) + rA;
@@ -291,7 +305,7 @@ __global__ __launch_bounds__(kWThreads, 1) void gemm_wide_kernel(GemmArgs a) {
         if constexpr (n == 1) { qA = pA; qhalfA = halfA; __builtin_amdgcn_sched_barrier(0); }
         if constexpr (n == 2) { on(); --left; __builtin_amdgcn_sched_barrier(0); }
         if constexpr (n % R == 0) { read(0, n / R, at_rows); __builtin_amdgcn_sched_barrier(0); }
-        if constexpr (n % L == L / 2 + 1) { issueA(n / L); __builtin_amdgcn_sched_barrier(0); }
+        if constexpr (n % L == L / 2 + 1) { issueA(std::integral_constant<int, n / L>{}); __builtin_amdgcn_sched_barrier(0); }
         if constexpr (n == NM - 1) { turnA(wA); __builtin_amdgcn_sched_barrier(0); }
         constexpr int i = mep_row_block(n), j = mep_weight_block(n);
         mep_acc_mul<8 * i + j, false>(fw[1][j], fr[1][i]);
@@ -318,30 +332,46 @@ __global__ __launch_bounds__(kWThreads, 1) void gemm_wide_kernel(GemmArgs a) {
     auto store_rows = [&](auto ii) MEP_INLINE {
       constexpr int i = ii;
       __builtin_amdgcn_sched_barrier(0);
-      const size_t row = (size_t)(m0 + (tall ? 128 : 64) * wm + 16 * i + l15) * a.N + n0 + (SWIGLU ? 64 : 128) * wn + 8 * lq;
+      // row and column of what this lane stores first
+      const int c0 = l15 >> 2;
+      const size_t first = (size_t)(m0 + (tall ? 128 : 64) * wm + 16 * i + (l15 & (SWIGLU ? 11 : 3))) * a.N + n0 + (SWIGLU ? 64 : 128) * wn +
+                           32 * (SWIGLU ? c0 & 1 : c0) + 8 * lq;
       auto pack = [](const mep_f32x4& x, const mep_f32x4& y) MEP_INLINE {
-        return mep_u4_any{mep_cvt_bf16x2(x[0], x[1]), mep_cvt_bf16x2(x[2], x[3]), mep_cvt_bf16x2(y[0], y[1]), mep_cvt_bf16x2(y[2], y[3])};
+        return mep_u4{mep_cvt_bf16x2(x[0], x[1]), mep_cvt_bf16x2(x[2], x[3]), mep_cvt_bf16x2(y[0], y[1]), mep_cvt_bf16x2(y[2], y[3])};
       };
       if constexpr (SWIGLU) {
+        auto put = [&](uint16_t* out, mep_u4 x, mep_u4 y) MEP_INLINE {
+          mep_trade<0>(x, y);
+          __builtin_nontemporal_store((mep_u4_any)x, (mep_u4_any*)(out + first));
+          __builtin_nontemporal_store((mep_u4_any)y, (mep_u4_any*)(out + first + 4 * (size_t)a.N));
+        };
+        mep_u4 h[2], g[2], u[2];
         mep_each<2>([&](auto c) MEP_INLINE {
           const mep_f32x4 g0 = mep_acc_get<8 * i + 2 * c>(), g1 = mep_acc_get<8 * i + 2 * c + 1>();
           const mep_f32x4 u0 = mep_acc_get<8 * i + 2 * c + 4>(), u1 = mep_acc_get<8 * i + 2 * c + 5>();
           auto act = [](const mep_f32x4& g, const mep_f32x4& u) MEP_INLINE {
             return mep_f32x4{mep_silu(g[0]) * u[0], mep_silu(g[1]) * u[1], mep_silu(g[2]) * u[2], mep_silu(g[3]) * u[3]};
           };
-          const size_t at = row + 32 * c;
-          *(mep_u4_any*)(a.C + at) = pack(act(g0, u0), act(g1, u1));
-          if (a.Cg) *(mep_u4_any*)(a.Cg + at) = pack(g0, g1);
-          if (a.Cu) *(mep_u4_any*)(a.Cu + at) = pack(u0, u1);
+          h[c] = pack(act(g0, u0), act(g1, u1));
+          g[c] = pack(g0, g1);
+          u[c] = pack(u0, u1);
         });
+        put(a.C, h[0], h[1]);
+        if (a.Cg) put(a.Cg, g[0], g[1]);
+        if (a.Cu) put(a.Cu, u[0], u[1]);
       } else {
         float sc = 1.0f;
         if (SCALED) sc = __int_as_float(__builtin_amdgcn_ds_bpermute(4 * (16 * (i & 3) + l15), __float_as_int(i < 4 ? scl0 : scl1)));
+        mep_u4 x[4];
         mep_each<4>([&](auto c) MEP_INLINE {
-          mep_f32x4 x = mep_acc_get<8 * i + 2 * c>(), y = mep_acc_get<8 * i + 2 * c + 1>();
-          if (SCALED) { x *= sc; y *= sc; }
-          *(mep_u4_any*)(a.C + row + 32 * c) = pack(x, y);
+          mep_f32x4 lo = mep_acc_get<8 * i + 2 * c>(), hi = mep_acc_get<8 * i + 2 * c + 1>();
+          if (SCALED) { lo *= sc; hi *= sc; }
+          x[c] = pack(lo, hi);
         });
+        mep_trade<0>(x[0], x[1]); mep_trade<0>(x[2], x[3]);
+        mep_trade<1>(x[0], x[2]); mep_trade<1>(x[1], x[3]);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) __builtin_nontemporal_store((mep_u4_any)x[c], (mep_u4_any*)(a.C + first + 4 * c * (size_t)a.N));
       }
     };
     mep_each<4>(store_rows);

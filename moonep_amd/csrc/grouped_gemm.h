@@ -86,10 +86,11 @@ constexpr int kNontemporal = 2;  // cache policy of a buffer load
 
 // 16 bytes per lane straight into LDS: lane offsets voff from a uniform base.  bytes = 0: nothing
 // is read (every offset is past the end) and the lanes' LDS vectors come out undefined.
-template <int AUX = 0>
+// AT: added to both addresses, in the instruction.
+template <int AUX = 0, int AT = 0>
 __device__ __forceinline__ void mep_load_lds16(const char* base, uint32_t voff, uint32_t soff, char* lds, int bytes = -1) {
   __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes, 0x00020000);
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, soff, 0, AUX);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, soff, AT, AUX);
 }
 template <int VM>
 __device__ __forceinline__ void mep_wait_vm_lgkm0() {
