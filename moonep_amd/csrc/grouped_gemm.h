@@ -384,6 +384,23 @@ struct WgradTiles {
   }
 };
 
+// The order of the K steps of the streaming kernel's forward products (rows and weights along K).  At a pitch that is a
+// multiple of 4 KB the 128 bytes that all CUs ask for in one step lie, of every row, on the same few channels of the L2
+// and the memory; the steps of a 4 KB piece of the rows then alternate between its halves, so that the two or three that are on
+// their way at one time use twice as many.  Otherwise they go up.  The order is that of the shape alone, the same for all tiles.
+// us, up -> this, 17 blocks of 128 rows (in brackets the time of 128 more columns, which go up): down 4096 x 2048
+// 67.7 (54.6) -> 53.8, 4096 x 4096 122.5 -> 97.9, 2048 x 4096 64.3 -> 57.6, SwiGLU 2048 x 2048 68.4 -> 53.7, 2048 x 4096 97.1 -> 96.7.
+// Tiles that begin at 2, 4 or 16 different places take as long as this (55.8, 56.1, 57.0 for the first), with sums whose order
+// depends on the tile.  At a pitch of 2 KB (K = 1024) beginning at different places gains nothing, and the 256 x 256 kernels lose 0.5
+// to 1 % with this order, to the cursor's instructions between the matrix instructions, so their steps go up.
+constexpr int kFold = 32;   // K steps of 4 KB
+__device__ __forceinline__ bool mep_folds(int K) { return K % (kFold * kBK) == 0; }
+// bytes from step k of a folded product to the next one
+__device__ __forceinline__ int mep_fold_step(int k) {
+  k &= kFold - 1;
+  return k & 1 ? (k == kFold - 1 ? 1 : 1 - kFold / 2) * kRowBytes : kFold / 2 * kRowBytes;
+}
+
 // The tiles of one workgroup, in order.  XCD x (workgroups x, x + 8, ...) walks a contiguous
 // eighth of the list, `width` workgroups in turn for `rounds` tiles each, then the next ones, so the
 // tiles that run on an XCD at one time are neighbours in the list.  Row-tiled products: the list goes group by group, inside a group weight

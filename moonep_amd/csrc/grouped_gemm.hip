@@ -707,6 +707,7 @@ __device__ __forceinline__ void stream_tile(const GemmArgs& a, char* gsm, int m0
 #pragma unroll
   for (int q = 0; q < 2; ++q) vA[q] = (uint32_t)((8 * q + r) * ld + ((kv ^ r ^ q) * 16));
   const uint32_t vB = (uint32_t)(r * ld + ((kv ^ r ^ (wave & 1)) * 16));
+  const bool fold = mep_folds(a.K);
   int kl = 0, ws = 0, rs = 0;
   auto issue = [&]() {
     const int bytes = __builtin_amdgcn_readfirstlane(kl < KT ? -1 : 0);  // past the last step: counted, but nothing is read
@@ -716,7 +717,8 @@ __device__ __forceinline__ void stream_tile(const GemmArgs& a, char* gsm, int m0
 #pragma unroll
     for (int i = 0; i < kLo; ++i) mep_load_lds16<kNontemporal>(pB, vB, i * strideB, slot + kSA + (wave + 8 * i) * 1024, bytes);
     if (kHi > kLo && lower) mep_load_lds16<kNontemporal>(pB, vB, kLo * strideB, slot + kSA + (wave + 8 * kLo) * 1024, bytes);
-    pA += kRowBytes; pB += kRowBytes;
+    const int step = fold ? mep_fold_step(kl) : kRowBytes;
+    pA += step; pB += step;
     ++kl;
     ws = ws == (D - 1) * kStageBytes ? 0 : ws + kStageBytes;
   };
