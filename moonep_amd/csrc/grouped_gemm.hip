@@ -745,12 +745,16 @@ __device__ __forceinline__ void stream_tile(const GemmArgs& a, char* gsm, int m0
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks) ad[ks] = l31 * kRowBytes + ((2 * ks + half) ^ sw) * 16;
 
-  for (int kt = 0; kt < KT; ++kt) {
-    // this wave's part of step kt is there; after the barrier everybody's, and the slot of the
-    // step before has been read by all
+  // this wave's part of the next step is there
+  auto next_in = [&]() {
     if (kHi == kLo || lower) mep_wait_vm_lgkm0<(D - 2) * (2 + kHi)>();
     else mep_wait_vm_lgkm0<(D - 2) * (2 + kLo)>();
-    mep_bar();
+  };
+  next_in();
+  mep_bar();
+  if (!lower) mep_bar();
+  for (int kt = 0; kt < KT; ++kt) {
+    // everybody's part of step kt is there, and the slot of the step before has been read by all
     const char* sa = gsm + rs + rb * 32 * kRowBytes;
     const char* sb = gsm + rs + kSA + uh * kSUnit;
     mep_bf16x8 fa[4], fb[4][kHi];
@@ -763,7 +767,10 @@ __device__ __forceinline__ void stream_tile(const GemmArgs& a, char* gsm, int m0
     }
     __builtin_amdgcn_sched_barrier(0);
     issue();
-    __builtin_amdgcn_sched_barrier(0);
+    mep_wait_lgkm0();
+    if (!lower) next_in();
+    mep_bar();
+    __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
 #pragma unroll
@@ -772,8 +779,12 @@ __device__ __forceinline__ void stream_tile(const GemmArgs& a, char* gsm, int m0
       if (kHi > kLo && lower)
         acc[kHi - 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[ks], fb[ks][kHi - 1], acc[kHi - 1], 0, 0, 0);
     }
+    __builtin_amdgcn_s_setprio(0);
     rs = rs == (D - 1) * kStageBytes ? 0 : rs + kStageBytes;
+    if (lower) next_in();
+    mep_bar();
   }
+  if (lower) mep_bar();
   mep_wait_vm_lgkm0<0>();  // the loads past the last step write LDS, too
   mep_bar();               // the next tile may be loaded
 
