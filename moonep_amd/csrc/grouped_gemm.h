@@ -365,13 +365,16 @@ struct WgradTiles {
   // In global memory by its type: a store through a pointer of unknown kind counts among the LDS operations, too, and a wait
   // for LDS reads then is one for the stores (C1).
   __device__ __forceinline__ mep_global_f32* C() const { return (mep_global_f32*)lane_pointer(c0, c1); }
-  // f(first element, row length) for the workgroup's tiles of zeros
-  template <class F>
-  __device__ __forceinline__ void zeros(F&& f) {
-    for (uint64_t m = empties; m; m &= m - 1) {
-      at = __ffsll((unsigned long long)m) - 1;
-      f(C(), map.N(__builtin_amdgcn_readlane(kp, at) & 3));
-    }
+  // the next of the workgroup's tiles of zeros: its first element, its row length; false: no more
+  __device__ __forceinline__ bool blank(mep_global_f32** out, int* N) {
+    if (!empties) return false;
+    const int now = at;
+    at = __ffsll((unsigned long long)empties) - 1;
+    empties &= empties - 1;
+    *out = C();
+    *N = map.N(__builtin_amdgcn_readlane(kp, at) & 3);
+    at = now;
+    return true;
   }
   // the next tile; false: no more
   __device__ __forceinline__ bool next() {

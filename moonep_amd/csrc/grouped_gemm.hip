@@ -357,19 +357,23 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
   using Tiles = std::conditional_t<WGRAD, WgradTiles<AT>, PTiles<MODE>>;
   Tiles ld(a, &map, gsm);
   Tiles cp = ld;  // the tiles as they are multiplied; what describes them is read once for both
-  // Groups without rows: whole 1 KB rows of zeroes per wave instruction.  Every other workgroup writes its share in
-  // front of its tiles, so that the memory sees both kinds of work at one time.
-  const bool zeros_first = WGRAD && (blockIdx.x >> 3 & 1);
-  auto write_zeros = [&]() {
-    if constexpr (WGRAD)
-      cp.zeros([&](mep_global_f32* out, int N) {
+  // Groups without rows: whole 1 KB rows of zeroes per wave instruction, between the K steps of the workgroup's tiles, as
+  // many tiles of zeros to each and not at the same time on all CUs: a CU alone writes 50 bytes a clock, all together 15
+  // each.  (16 groups of 4096 x 2048 with 2048 rows and as many without, us: half of the workgroups in front of
+  // their tiles, half behind them 1587, this 1549; a row per wave and K step, among the loads, whose waits then are for stores, too, 1617;
+  // without zeros 1440 to 1500.)
+  auto write_zeros = [&](int tiles) {
+    if constexpr (WGRAD) {
+      mep_global_f32* out;
+      int N;
+      for (; tiles > 0 && cp.blank(&out, &N); --tiles) {
         typedef __attribute__((address_space(1))) mep_f32x4 global_f32x4;
         const mep_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
         for (int row = wave; row < kPT; row += 8) __builtin_nontemporal_store(zero, (global_f32x4*)(out + (size_t)row * N) + lane);
-      });
+      }
+    }
   };
-  if (zeros_first) write_zeros();
   const char *pA, *pB;
   uint32_t halfA, halfB;
   int kl = 0;
@@ -381,6 +385,8 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
       const int j = 2 * wave + q;
       vA[q] = AT ? (uint32_t)((4 * j + lk) * ldA * 2 + ((lv ^ (lk << 2)) * 16)) : (uint32_t)((8 * j + r) * ldA * 2 + ((kv ^ r ^ q) * 16));
       vB[q] = BT ? (uint32_t)((4 * j + lk) * ldB * 2 + ((lv ^ (lk << 2)) * 16)) : (uint32_t)((8 * j + r) * ldB * 2 + ((kv ^ r ^ q) * 16));
+      vA[q] -= q * 1024;  // what the instruction adds to both addresses (never more than is there: K is at least 64, M and N 256)
+      vB[q] -= q * 1024;
     }
   };
   if (!WGRAD) lanes();
@@ -422,13 +428,13 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
   auto turn = [](int& slot, int first) { slot = slot == first + (kPSlots - 1) * kPHalf ? first : slot + kPHalf; };
   char* lds_w = gsm + wave * 2048;
   auto issueA = [&](int h) {
-#pragma unroll
-    for (int q = 0; q < 2; ++q) mep_load_lds16(pA, vA[q], h ? halfA : 0u, lds_w + wA + q * 1024);
+    mep_load_lds16(pA, vA[0], h ? halfA : 0u, lds_w + wA);
+    mep_load_lds16<0, 1024>(pA, vA[1], h ? halfA : 0u, lds_w + wA);
     turn(wA, 0);
   };
   auto issueB = [&](int h) {
-#pragma unroll
-    for (int q = 0; q < 2; ++q) mep_load_lds16(pB, vB[q], h ? halfB : 0u, lds_w + wB + q * 1024);
+    mep_load_lds16(pB, vB[0], h ? halfB : 0u, lds_w + wB);
+    mep_load_lds16<0, 1024>(pB, vB[1], h ? halfB : 0u, lds_w + wB);
     turn(wB, kPOperand);
   };
 
@@ -555,7 +561,14 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
       asm volatile("global_load_dword %0, %1, off" : "=v"(scl0) : "v"(sp));
       asm volatile("global_load_dword %0, %1, off" : "=v"(scl1) : "v"(sp + (tall ? 128 : 0)));
     }
+    int zeros_at = -1, zeros = 0;
+    if constexpr (WGRAD) {
+      const int tiles = 1 + __popcll(cp.left);
+      zeros = mep_quotient(__popcll(cp.empties) + tiles - 1, tiles);
+      zeros_at = (int)(blockIdx.x >> 3 & 7) * KT >> 3;
+    }
     for (int kt = 0; kt < KT; ++kt) {
+      if (WGRAD && kt == zeros_at) write_zeros(zeros);
       readA();
       readB(fb0, tb0);
       readB(fb1, tb1);
@@ -632,7 +645,7 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
   }
   if (any && wave < 4) mep_bar();
   mep_wait_vmcnt<0>();  // the loads of steps nobody wanted write LDS, too
-  if (!zeros_first) write_zeros();
+  write_zeros(1 << 30);
   if (!WGRAD && a.zero_tail) zero_tail_rows(a, blockIdx.x, gridDim.x, kPThreads);
 }
 // ---------------------------------------------------------------------------
@@ -644,13 +657,18 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
 // however many groups have rows (whole 128 x 256 tiles leave 17 blocks of 4096 weight rows with
 // 272 tiles for 256 CUs: a second round for sixteen of them) and the rows come from L2 once for up
 // to 288 weight rows.  A K step of 64 is 16 KB of rows and 4 KB a unit; the whole LDS holds D of
-// them, D - 1 on their way (72 KB of weights per CU at nine units) while one is multiplied, with
-// one barrier a step.  8 waves: 32 rows each, every other unit.  All of a step's fragments are
+// them, D - 1 on their way (72 KB of weights per CU at nine units) while one is multiplied.
+// 8 waves: 32 rows each, every other unit.  The waves 4 .. 7 run one barrier behind the waves 0 .. 3,
+// so that one wave of a SIMD multiplies while the other reads: a step's 160 to 192 KB of LDS reads
+// take about as long as its matrix instructions, and one after the other, with one barrier a step, the
+// two were 1.17 us a step of eight units and 1.33 of nine, however few of the CUs were still at work
+// (us, before -> now, 17 blocks: down 4096 x 4096 102 -> 96, 4096 x 7168 176 -> 169, 2048 x 4096
+// 61 -> 57, SwiGLU 2048 x 4096 100 -> 98, down 4096 x 2048 the same; the [K, N] form below is 0 to 5 %
+// slower that way).  All of a step's fragments are
 // asked for before the next loads are issued (behind them they waited: 78 against 54 us where a
 // tile has one or two units); weights are loaded nontemporal, so that the rows stay in L2 (183
-// against 202 us at 17 blocks).  K goes up in every tile as in the other kernels: the order of a
-// sum does not depend on where its tile lies.  (Workgroups that start at different K steps, and
-// so do not all read the same column of rows of one pitch, took 168 us.)
+// against 202 us at 17 blocks).  The order of the K steps is that of the shape (mep_fold_step): the
+// order of a sum does not depend on where its tile lies.
 //
 // The tiles of a block divide its units evenly and are as many as fill whole rounds of the grid:
 // cut where a CU's even share of the list ends, a tile in two blocks ran its K loop twice with
@@ -662,6 +680,7 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
 // The forward of 17 blocks on another card 211 -> 202 us with the epilogue's selects of two values and the row scales read
 // before the loads, of 18 232 -> 219, of 24 314 -> 298, 7168 x 2048 with 33 583 -> 558.  What a tile takes beside its
 // K steps now: 1.2 us to its group, 0.8 to the last of the first loads, 2 to 3 to their arrival, 1.4 (down) to 4 (SwiGLU) to store.
+// With the order of the K steps and the waves' two shifts, 64 tokens at 17 blocks: 190 -> 161.
 // ---------------------------------------------------------------------------
 typedef float mep_f32x4_any __attribute__((ext_vector_type(4), aligned(4)));  // at any element
 constexpr int kSThreads = 512;
