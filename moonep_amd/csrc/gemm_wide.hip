@@ -17,7 +17,9 @@
 //    slot of the next step is made in there, too.  In front of the matrix instructions of 16 rows
 //    instead, two reads and a load cost 10 %; a branch for every four of them (to skip the rows that
 //    a short tile does not have) 9 %, so there are two copies of a step, 256 rows and 128.
-// Loads go straight into LDS: the weights' tile (32 KB a step) has three slots, the rows' two.  A K
+// Loads go straight into LDS: the weights' tile (32 KB a step) has three slots, the rows' two.  Four
+// loads in a row take their place from one M0 and the offset in the instruction, which counts for both
+// addresses (an M0 each: 0.2 % slower).  A K
 // step goes in two halves (K 0 .. 31, 32 .. 63); while one half's fragments are multiplied, the other
 // half's are read.  When the second half's have arrived, one barrier says that the step's slots are
 // free and that the next step's are full.  Waiting for older or for younger loads there made no
@@ -27,6 +29,15 @@
 // The first operand of the matrix instruction is the weights: a lane then holds four neighbouring
 // columns of one row, and the fragments 2 c and 2 c + 1 take the weight rows 8 a + b and 8 a + 4 + b
 // (a, b = 0 .. 3) of a block of 32, so that they make eight neighbouring columns, one 16-byte store.
+// Before they are stored, lanes four rows apart trade these 16 bytes for two blocks of columns, so that an
+// instruction stores 128 neighbouring bytes of eight rows instead of 64 of sixteen; and the stores are
+// nontemporal.  When all CUs store at one time, as they do after tiles of equal length, 128 KB a CU take
+// 9000 cycles as plain stores, 9500 to 11 000 nontemporal in pieces of 64 bytes and 6800 in pieces of
+// 128 or 256 (one CU alone: 2500), with the matrix cores idle.  us, before -> now: 36 864 rows in 96
+// groups, 2048 x 1024: SwiGLU 297 -> 291, down 161 -> 157, dy * down 154 -> 150, both pairs 287 -> 284;
+// 32 768 rows in 32 groups, 2048 x 1024 columns 118 -> 108; 7168 x 2048, which power bounds, 1333 ->
+// 1324, 716 -> 714, 670 -> 666, 1347 -> 1342 (with the loads below).  Workgroups that begin a quarter of
+// the stores' time apart are no faster.
 //
 // LDS layouts.  The hardware serves 16-byte reads in groups of the lanes 0-3, 12-15, 20-27 (and
 // 4-11, 16-19, 28-31), not of sixteen neighbours.  Rows: 128 bytes each, vector q of row r at
@@ -89,16 +100,16 @@ __device__ __forceinline__ void mep_acc_taken() {
 constexpr int mep_row_block(int n) { return n >> 4 << 1 | ((n ^ n >> 1) & 1); }
 constexpr int mep_weight_block(int n) { return (n >> 4 & 1 ? ~n : n) >> 1 & 7; }
 
-// Four lanes of sixteen, bank 0 .. 3: x of the banks with bit S against y of those without, at the same place in the bank.
+// x and y are two blocks of columns of a lane's row.  Of eight lanes the first four take the last four's x for their y: they then
+// have one block of their row and of the row four lanes on, the others the other block of the same two.
 typedef uint32_t mep_u4 __attribute__((ext_vector_type(4)));
-template <int S>
 __device__ __forceinline__ void mep_trade(mep_u4& x, mep_u4& y) {
-  constexpr int kUp = 0x120 + (S ? 8 : 4), kDown = 0x120 + (S ? 8 : 12);  // row_ror
+  constexpr int kFromBelow = 0x124, kFromAbove = 0x12c;  // row_ror by four lanes and by twelve
 #pragma unroll
   for (int d = 0; d < 4; ++d) {
-    const uint32_t was = x[d];
-    x[d] = (uint32_t)__builtin_amdgcn_update_dpp((int)was, (int)y[d], kUp, 0xf, S ? 0xc : 0xa, false);
-    y[d] = (uint32_t)__builtin_amdgcn_update_dpp((int)y[d], (int)was, kDown, 0xf, S ? 0x3 : 0x5, false);
+    const int was = (int)x[d];
+    x[d] = (uint32_t)__builtin_amdgcn_update_dpp(was, (int)y[d], kFromBelow, 0xf, 0xa, false);
+    y[d] = (uint32_t)__builtin_amdgcn_update_dpp((int)y[d], was, kFromAbove, 0xf, 0x5, false);
   }
 }
 
@@ -115,7 +126,7 @@ __device__ __forceinline__ void mep_each(F&& f) {
 // KN: the weights are given as [K, columns].  SCALED: scale mode with row scales.
 template <int MODE, bool KN, bool SCALED>
 __global__ __launch_bounds__(kWThreads, 1) void gemm_wide_kernel(GemmArgs a) {
-  constexpr bool SWIGLU = MODE == kModeSwiglu, DUAL = MODE == kModeDual;
+  constexpr bool SWIGLU = MODE == kModeSwiglu, DUAL = MODE == kModeDual, FORWARD = !DUAL && !KN;
   static_assert(!(SWIGLU && KN) && (!SCALED || MODE == kModeScale) && MODE != kModeWgrad, "no such product");
   extern __shared__ __attribute__((aligned(1024))) char gsm[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -124,27 +135,54 @@ __global__ __launch_bounds__(kWThreads, 1) void gemm_wide_kernel(GemmArgs a) {
   // ---- loads: a cursor over (tile, K step).  It moves on once a step; the rows of a step (qA) are
   // asked for half a step after its weights
   const size_t ldA = (size_t)a.K, ldB = KN ? (size_t)a.N : (size_t)a.K;
-  uint32_t stepA = kRowBytes, stepB = KN ? (uint32_t)(kBK * ldB * 2) : kRowBytes;
   PTiles<MODE, true> ld(a);
   PTiles<MODE, true> cp = ld;  // the tiles as they are multiplied
-  const char *pA, *pB, *pB1, *qA;
-  uint32_t halfA, halfB, qhalfA;
+  // A tile's operands as the loads take them; a step moves them along K by an offset.  (As addresses, which move on by 64
+  // bits and are made into the loads' four words again between the matrix instructions: 32 768 rows, 7168 x 2048,
+  // SwiGLU 1334 -> 1329 us, down 719 -> 716; on zeroes, where power bounds less, 1145 -> 1141, 582 -> 580.)
+  __amdgpu_buffer_rsrc_t dA = mep_rsrc((const char*)a.A), dB = dA, dB1 = dA;
+  uint32_t kA = 0, qkA = 0, halfA = 0, qhalfA = 0;
+  uint32_t step = kRowBytes, both = 2 * kRowBytes;  // to the next step; to the one behind it
+  const bool fold = FORWARD && mep_folds(a.K);
+  int pieces = 0;       // of a folded tile, behind the one that `left` counts
+  const uint32_t stepB = KN ? (uint32_t)(kBK * ldB * 2) : 0;
+  const uint32_t halfB = SWIGLU ? 0u : KN ? 256u : (uint32_t)(128 * ldB * 2);
+  const char* pB = nullptr;
   int left = 0;         // K steps to the end of the tile, or of its first pair
   bool second = false;  // dual: at the second pair
   auto stand = [&]() MEP_INLINE {  // at the first K step of the tile (of its second pair)
     const size_t offA = (size_t)ld.m0 * ldA;
     const size_t offB = (size_t)ld.g * a.N * a.K + (KN ? (size_t)ld.n0 : (size_t)ld.n0 * ldB);
-    pA = mep_uniform((const char*)((DUAL && second ? a.A2 : a.A) + offA));
+    dA = mep_rsrc(mep_uniform((const char*)((DUAL && second ? a.A2 : a.A) + offA)));
     pB = mep_uniform((const char*)((DUAL && second ? a.B2 : a.B) + offB));
-    pB1 = SWIGLU ? mep_uniform((const char*)(a.B2 + offB)) : pB;
+    if (!KN) dB = mep_rsrc(pB);
+    if (SWIGLU) dB1 = mep_rsrc(mep_uniform((const char*)(a.B2 + offB)));
+    kA = 0;
     halfA = __builtin_amdgcn_readfirstlane(ld.tall ? (uint32_t)(128 * ldA * 2) : 0u);
-    halfB = SWIGLU ? 0u : KN ? 256u : (uint32_t)(128 * ldB * 2);
-    left = __builtin_amdgcn_readfirstlane(a.K / kBK);
+    left = __builtin_amdgcn_readfirstlane(fold ? kFold : a.K / kBK);
+    if (FORWARD) {
+      pieces = __builtin_amdgcn_readfirstlane(fold ? a.K / kBK / kFold - 1 : 0);
+      step = fold ? (uint32_t)mep_fold_step(0) : kRowBytes;
+      both = fold ? kRowBytes : 2 * kRowBytes;
+    }
   };
+  // more than one tile a workgroup: the next tile's loads wait behind the stores (one: 20 groups of 1792 x 768, down 18.8 us
+  // as plain stores, 20 nontemporal)
+  const int rounds = __builtin_amdgcn_readfirstlane((int)(ld.count > ld.nw));
   const int some = __builtin_amdgcn_readfirstlane((int)ld.next());
   if (some) stand();
-  auto on = [&]() MEP_INLINE { pA += stepA; pB += stepB; if (SWIGLU) pB1 += stepB; else pB1 = pB; };
-  auto turned = [&]() MEP_INLINE {  // the cursor has left its tile
+  auto on = [&]() MEP_INLINE {
+    kA += step;
+    if (FORWARD) step = both - step;
+    if (KN && step) pB += stepB;
+  };
+  auto turned = [&]() MEP_INLINE {  // the cursor has left its tile, or a piece of it
+    if (FORWARD && pieces > 0) {
+      --pieces;
+      left = kFold;
+      kA += kRowBytes - (both - step);
+      return;
+    }
     if (DUAL && !second) {
       second = true;
       stand();
@@ -154,8 +192,9 @@ __global__ __launch_bounds__(kWThreads, 1) void gemm_wide_kernel(GemmArgs a) {
     if (__builtin_amdgcn_readfirstlane((int)ld.next())) {
       stand();
     } else {  // the last step is loaded again, for nobody
-      pA -= stepA; pB -= stepB; pB1 = SWIGLU ? pB1 - stepB : pB;
-      stepA = stepB = 0;
+      kA -= FORWARD ? both - step : step;
+      pB -= stepB;
+      step = both = 0;
       left = 1 << 30;
     }
   };
@@ -171,6 +210,8 @@ __global__ __launch_bounds__(kWThreads, 1) void gemm_wide_kernel(GemmArgs a) {
                   : (uint32_t)((8 * j + r) * ldB * 2 + (kv ^ (r & 2) ^ (q >> 1 << 2)) * 16)) - q * 1024;
     }
   }
+  __amdgpu_buffer_rsrc_t dqA = dA;  // the rows' step, behind the weights'
+  auto hold = [&]() MEP_INLINE { dqA = dA; qkA = kA; qhalfA = kA + halfA; };
   // where the next step of each operand is written and read
   char* lds_w = gsm + wave * 4096;
   int wA = 0, wB = kWFirstB, rA = 0, rB = kWFirstB;
@@ -178,11 +219,12 @@ __global__ __launch_bounds__(kWThreads, 1) void gemm_wide_kernel(GemmArgs a) {
   auto turnB = [](int& s) MEP_INLINE { s = s == kWLds - kWStep ? kWFirstB : s + kWStep; };
   auto issueA = [&](auto c) MEP_INLINE {  // 0 .. 7
     constexpr int n = c;
-    mep_load_lds16<0, (n & 3) * 1024>(qA, vA[n & 3], n >> 2 ? qhalfA : 0u, lds_w + wA + (n >> 2) * kWHalf);
+    mep_load_lds16<0, (n & 3) * 1024>(dqA, vA[n & 3], n >> 2 ? qhalfA : qkA, lds_w + wA + (n >> 2) * kWHalf);
   };
   auto issueB = [&](auto c) MEP_INLINE {
     constexpr int n = c;
-    mep_load_lds16<0, (n & 3) * 1024>(n >> 2 ? pB1 : pB, vB[n & 3], n >> 2 ? halfB : 0u, lds_w + wB + (n >> 2) * kWHalf);
+    if (KN) mep_load_lds16<0, (n & 3) * 1024>(pB, vB[n & 3], n >> 2 ? halfB : 0u, lds_w + wB + (n >> 2) * kWHalf);
+    else mep_load_lds16<0, (n & 3) * 1024>(SWIGLU && n >> 2 ? dB1 : dB, vB[n & 3], SWIGLU || !(n >> 2) ? kA : kA + halfB, lds_w + wB + (n >> 2) * kWHalf);
   };
 
   // ---- fragments: set s holds half s of a K step
@@ -233,7 +275,7 @@ __global__ __launch_bounds__(kWThreads, 1) void gemm_wide_kernel(GemmArgs a) {
   if (some) {
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-      qA = pA; qhalfA = halfA;
+      hold();
       mep_each<8>(issueA);
       mep_each<8>(issueB);
       turnA(wA); turnB(wB);
@@ -302,7 +344,7 @@ __global__ __launch_bounds__(kWThreads, 1) void gemm_wide_kernel(GemmArgs a) {
       mep_bar();
       mep_each<NM>([&](auto c) MEP_INLINE {
         constexpr int n = c;
-        if constexpr (n == 1) { qA = pA; qhalfA = halfA; __builtin_amdgcn_sched_barrier(0); }
+        if constexpr (n == 1) { hold(); __builtin_amdgcn_sched_barrier(0); }
         if constexpr (n == 2) { on(); --left; __builtin_amdgcn_sched_barrier(0); }
         if constexpr (n % R == 0) { read(0, n / R, at_rows); __builtin_amdgcn_sched_barrier(0); }
         if constexpr (n % L == L / 2 + 1) { issueA(std::integral_constant<int, n / L>{}); __builtin_amdgcn_sched_barrier(0); }
@@ -333,18 +375,24 @@ __global__ __launch_bounds__(kWThreads, 1) void gemm_wide_kernel(GemmArgs a) {
       constexpr int i = ii;
       __builtin_amdgcn_sched_barrier(0);
       // row and column of what this lane stores first
-      const int c0 = l15 >> 2;
-      const size_t first = (size_t)(m0 + (tall ? 128 : 64) * wm + 16 * i + (l15 & (SWIGLU ? 11 : 3))) * a.N + n0 + (SWIGLU ? 64 : 128) * wn +
-                           32 * (SWIGLU ? c0 & 1 : c0) + 8 * lq;
+      const size_t first = (size_t)(m0 + (tall ? 128 : 64) * wm + 16 * i + (l15 & 11)) * a.N + n0 + (SWIGLU ? 64 : 128) * wn +
+                           8 * (l15 & 4) + 8 * lq;
       auto pack = [](const mep_f32x4& x, const mep_f32x4& y) MEP_INLINE {
         return mep_u4{mep_cvt_bf16x2(x[0], x[1]), mep_cvt_bf16x2(x[2], x[3]), mep_cvt_bf16x2(y[0], y[1]), mep_cvt_bf16x2(y[2], y[3])};
       };
+      auto put = [&](uint16_t* out, mep_u4 x, mep_u4 y) MEP_INLINE {
+        mep_trade(x, y);
+        mep_u4_any* const at = (mep_u4_any*)(out + first);
+        mep_u4_any* const below = (mep_u4_any*)(out + first + 4 * (size_t)a.N);
+        if (rounds) {
+          __builtin_nontemporal_store((mep_u4_any)x, at);
+          __builtin_nontemporal_store((mep_u4_any)y, below);
+        } else {
+          *at = x;
+          *below = y;
+        }
+      };
       if constexpr (SWIGLU) {
-        auto put = [&](uint16_t* out, mep_u4 x, mep_u4 y) MEP_INLINE {
-          mep_trade<0>(x, y);
-          __builtin_nontemporal_store((mep_u4_any)x, (mep_u4_any*)(out + first));
-          __builtin_nontemporal_store((mep_u4_any)y, (mep_u4_any*)(out + first + 4 * (size_t)a.N));
-        };
         mep_u4 h[2], g[2], u[2];
         mep_each<2>([&](auto c) MEP_INLINE {
           const mep_f32x4 g0 = mep_acc_get<8 * i + 2 * c>(), g1 = mep_acc_get<8 * i + 2 * c + 1>();
@@ -368,10 +416,8 @@ __global__ __launch_bounds__(kWThreads, 1) void gemm_wide_kernel(GemmArgs a) {
           if (SCALED) { lo *= sc; hi *= sc; }
           x[c] = pack(lo, hi);
         });
-        mep_trade<0>(x[0], x[1]); mep_trade<0>(x[2], x[3]);
-        mep_trade<1>(x[0], x[2]); mep_trade<1>(x[1], x[3]);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) __builtin_nontemporal_store((mep_u4_any)x[c], (mep_u4_any*)(a.C + first + 4 * c * (size_t)a.N));
+        put(a.C, x[0], x[1]);
+        put(a.C + 64, x[2], x[3]);
       }
     };
     mep_each<4>(store_rows);

@@ -92,6 +92,13 @@ __device__ __forceinline__ void mep_load_lds16(const char* base, uint32_t voff, 
   __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes, 0x00020000);
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, soff, AT, AUX);
 }
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t mep_rsrc(const char* base) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, -1, 0x00020000);
+}
+template <int AUX = 0, int AT = 0>
+__device__ __forceinline__ void mep_load_lds16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, char* lds) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, soff, AT, AUX);
+}
 template <int VM>
 __device__ __forceinline__ void mep_wait_vm_lgkm0() {
   __builtin_amdgcn_s_waitcnt((VM & 15) | (7 << 4) | ((VM >> 4) << 14));
@@ -387,17 +394,17 @@ struct WgradTiles {
   }
 };
 
-// The order of the K steps of the streaming kernel's forward products (rows and weights along K).  At a pitch that is a
-// multiple of 4 KB the 128 bytes that all CUs ask for in one step lie, of every row, on the same few channels of the L2
-// and the memory; the steps of a 4 KB piece of the rows then alternate between its halves, so that the two or three that are on
-// their way at one time use twice as many.  Otherwise they go up.  The order is that of the shape alone, the same for all tiles.
-// us, up -> this, 17 blocks of 128 rows (in brackets the time of 128 more columns, which go up): down 4096 x 2048
-// 67.7 (54.6) -> 53.8, 4096 x 4096 122.5 -> 97.9, 2048 x 4096 64.3 -> 57.6, SwiGLU 2048 x 2048 68.4 -> 53.7, 2048 x 4096 97.1 -> 96.7.
-// Tiles that begin at 2, 4 or 16 different places take as long as this (55.8, 56.1, 57.0 for the first), with sums whose order
-// depends on the tile.  At a pitch of 2 KB (K = 1024) beginning at different places gains nothing, and the 256 x 256 kernels lose 0.5
-// to 1 % with this order, to the cursor's instructions between the matrix instructions, so their steps go up.
+// The order of the K steps of forward products (rows and weights along K), the same in every kernel that makes them: the
+// forms agree to the bit.  At a pitch that is a multiple of 4 KB the 128 bytes that all CUs ask for in one step lie, of
+// every row, on the same few channels of the L2 and the memory; the steps of a 4 KB piece of the rows then alternate between its
+// halves, so that the two or three that are on their way at one time use twice as many.  Otherwise they go up.  The order
+// is that of the shape alone.  us, up -> this, streaming kernel, 17 blocks of 128 rows (in brackets the time of 128 more columns,
+// which go up): down 4096 x 2048 67.7 (54.6) -> 53.8, 4096 x 4096 122.5 -> 97.9, 2048 x 4096 64.3 -> 57.6, SwiGLU 2048 x 2048
+// 68.4 -> 53.7, 2048 x 4096 97.1 -> 96.7.  Tiles that begin at 2, 4 or 16 different places take as long as this (55.8, 56.1, 57.0
+// for the first), with sums whose order depends on the tile.  At a pitch of 2 KB (K = 1024) beginning at different places gains
+// nothing.  The 256 x 256 kernels, whose operands come from the L2 several times, take the same time with either order.
 constexpr int kFold = 32;   // K steps of 4 KB
-__device__ __forceinline__ bool mep_folds(int K) { return K % (kFold * kBK) == 0; }
+__host__ __device__ __forceinline__ bool mep_folds(int K) { return K % (kFold * kBK) == 0; }
 // bytes from step k of a folded product to the next one
 __device__ __forceinline__ int mep_fold_step(int k) {
   k &= kFold - 1;

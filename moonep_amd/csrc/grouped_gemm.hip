@@ -343,7 +343,7 @@ constexpr int kPSteps = 128;
 // AT, BT: the operand is given as [K, columns].  SCALED: scale mode with row scales.
 template <int MODE, bool AT, bool BT, bool SCALED = false>
 __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, WgradMap map) {
-  constexpr bool DUAL = MODE == kModeDual, WGRAD = MODE == kModeWgrad;
+  constexpr bool DUAL = MODE == kModeDual, WGRAD = MODE == kModeWgrad, FORWARD = MODE == kModeScale && !BT;
   static_assert(!AT || WGRAD, "rows of the other products lie along K");
   static_assert(MODE != kModeSwiglu, "gemm_wide_kernel has it");
   extern __shared__ __attribute__((aligned(1024))) char gsm[];
@@ -354,6 +354,7 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
   // pitches; of a weight gradient's operands, [rows, M] and [rows, N], those of the product at hand
   size_t ldA = AT ? (size_t)a.M : (size_t)a.ld, ldB = BT ? (size_t)a.N : (size_t)a.ld;
   const int KT1 = WGRAD ? 0 : a.K / kBK;
+  [[maybe_unused]] const bool fold = FORWARD && mep_folds(a.K);
   using Tiles = std::conditional_t<WGRAD, WgradTiles<AT>, PTiles<MODE>>;
   Tiles ld(a, &map, gsm);
   Tiles cp = ld;  // the tiles as they are multiplied; what describes them is read once for both
@@ -416,8 +417,11 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
     if (kl + 1 < ld.KT) {
       ++kl;
       if (DUAL && kl == KT1) { stand(1); return; }
-      pA += AT ? kBK * ldA * 2 : kBK * 2;
-      pB += BT ? kBK * ldB * 2 : kBK * 2;
+      const int step = FORWARD && fold ? mep_fold_step(kl - 1) : kRowBytes;
+      if (AT) pA += kBK * ldA * 2;
+      else pA += step;
+      if (BT) pB += kBK * ldB * 2;
+      else pB += step;
       return;
     }
     more = ld.next();
@@ -667,8 +671,8 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
 // slower that way).  All of a step's fragments are
 // asked for before the next loads are issued (behind them they waited: 78 against 54 us where a
 // tile has one or two units); weights are loaded nontemporal, so that the rows stay in L2 (183
-// against 202 us at 17 blocks).  The order of the K steps is that of the shape (mep_fold_step): the
-// order of a sum does not depend on where its tile lies.
+// against 202 us at 17 blocks).  The order of the K steps is that of the shape (mep_fold_step), as in the
+// other kernels: the order of a sum does not depend on where its tile lies.
 //
 // The tiles of a block divide its units evenly and are as many as fill whole rounds of the grid:
 // cut where a CU's even share of the list ends, a tile in two blocks ran its K loop twice with
@@ -700,11 +704,12 @@ __device__ __forceinline__ void store_two_rows(uint16_t* c, float row0, float ro
   *(mep_u1_any*)c = __builtin_amdgcn_perm(o, w, threadIdx.x & 1 ? 0x03020706u : 0x05040100u);
 }
 
-template <int MODE, int NU>
+template <int MODE, int NU, bool FOLD>
 __device__ __forceinline__ void stream_tile(const GemmArgs& a, char* gsm, int m0, int g, int unit0) {
   constexpr bool SWIGLU = MODE == kModeSwiglu;
   constexpr int kStageBytes = kSA + NU * kSUnit;
   constexpr int D = kSLds / kStageBytes < 8 ? kSLds / kStageBytes : 8;
+  constexpr bool kShift = NU >= 7;                // the waves 4 .. 7 run one barrier behind the others
   constexpr int kHi = (NU + 1) / 2, kLo = NU / 2;  // units of the waves 0 .. 3 and 4 .. 7; as many pieces to load
   static_assert(D >= 3 && (D - 1) * (2 + kHi) < 64, "the loads on their way must fit the 6-bit counter");
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -726,7 +731,6 @@ __device__ __forceinline__ void stream_tile(const GemmArgs& a, char* gsm, int m0
 #pragma unroll
   for (int q = 0; q < 2; ++q) vA[q] = (uint32_t)((8 * q + r) * ld + ((kv ^ r ^ q) * 16));
   const uint32_t vB = (uint32_t)(r * ld + ((kv ^ r ^ (wave & 1)) * 16));
-  const bool fold = mep_folds(a.K);
   int kl = 0, ws = 0, rs = 0;
   auto issue = [&]() {
     const int bytes = __builtin_amdgcn_readfirstlane(kl < KT ? -1 : 0);  // past the last step: counted, but nothing is read
@@ -736,7 +740,7 @@ __device__ __forceinline__ void stream_tile(const GemmArgs& a, char* gsm, int m0
 #pragma unroll
     for (int i = 0; i < kLo; ++i) mep_load_lds16<kNontemporal>(pB, vB, i * strideB, slot + kSA + (wave + 8 * i) * 1024, bytes);
     if (kHi > kLo && lower) mep_load_lds16<kNontemporal>(pB, vB, kLo * strideB, slot + kSA + (wave + 8 * kLo) * 1024, bytes);
-    const int step = fold ? mep_fold_step(kl) : kRowBytes;
+    const int step = FOLD ? mep_fold_step(kl) : kRowBytes;
     pA += step; pB += step;
     ++kl;
     ws = ws == (D - 1) * kStageBytes ? 0 : ws + kStageBytes;
@@ -769,10 +773,16 @@ __device__ __forceinline__ void stream_tile(const GemmArgs& a, char* gsm, int m0
     if (kHi == kLo || lower) mep_wait_vm_lgkm0<(D - 2) * (2 + kHi)>();
     else mep_wait_vm_lgkm0<(D - 2) * (2 + kLo)>();
   };
-  next_in();
-  mep_bar();
-  if (!lower) mep_bar();
+  if (kShift) {
+    next_in();
+    mep_bar();
+    if (!lower) mep_bar();
+  }
   for (int kt = 0; kt < KT; ++kt) {
+    if (!kShift) {
+      next_in();
+      mep_bar();
+    }
     // everybody's part of step kt is there, and the slot of the step before has been read by all
     const char* sa = gsm + rs + rb * 32 * kRowBytes;
     const char* sb = gsm + rs + kSA + uh * kSUnit;
@@ -786,10 +796,13 @@ __device__ __forceinline__ void stream_tile(const GemmArgs& a, char* gsm, int m0
     }
     __builtin_amdgcn_sched_barrier(0);
     issue();
-    mep_wait_lgkm0();
-    if (!lower) next_in();
-    mep_bar();
-    __builtin_amdgcn_s_setprio(1);
+    __builtin_amdgcn_sched_barrier(0);
+    if (kShift) {
+      mep_wait_lgkm0();
+      if (!lower) next_in();
+      mep_bar();
+      __builtin_amdgcn_s_setprio(1);
+    }
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
 #pragma unroll
@@ -798,12 +811,14 @@ __device__ __forceinline__ void stream_tile(const GemmArgs& a, char* gsm, int m0
       if (kHi > kLo && lower)
         acc[kHi - 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[ks], fb[ks][kHi - 1], acc[kHi - 1], 0, 0, 0);
     }
-    __builtin_amdgcn_s_setprio(0);
     rs = rs == (D - 1) * kStageBytes ? 0 : rs + kStageBytes;
-    if (lower) next_in();
-    mep_bar();
+    if (kShift) {
+      __builtin_amdgcn_s_setprio(0);
+      if (lower) next_in();
+      mep_bar();
+    }
   }
-  if (lower) mep_bar();
+  if (kShift && lower) mep_bar();
   mep_wait_vm_lgkm0<0>();  // the loads past the last step write LDS, too
   mep_bar();               // the next tile may be loaded
 
@@ -963,7 +978,8 @@ __device__ __forceinline__ void stream_tile_kn(const GemmArgs& a, char* gsm, int
                      scale[v >> 2][(v & 3) + 1] * acc[i][v + 1]);
 }
 
-template <int MODE, bool KN>
+// FOLD: a forward product with mep_folds(K).  (As a choice in the kernel it cost the products of few tiles and steps 0.3 to 0.4 us each.)
+template <int MODE, bool KN, bool FOLD = false>
 __global__ __launch_bounds__(kSThreads, 2) void gemm_stream_kernel(GemmArgs a) {
   extern __shared__ __attribute__((aligned(1024))) char gsm[];
   constexpr int kUnits = KN ? kSUnitsKn : kSUnits;
@@ -1023,15 +1039,15 @@ __global__ __launch_bounds__(kSThreads, 2) void gemm_stream_kernel(GemmArgs a) {
       }
     } else {
       switch (n) {
-        case 1: stream_tile<MODE, 1>(a, gsm, m0, g, unit0); break;
-        case 2: stream_tile<MODE, 2>(a, gsm, m0, g, unit0); break;
-        case 3: stream_tile<MODE, 3>(a, gsm, m0, g, unit0); break;
-        case 4: stream_tile<MODE, 4>(a, gsm, m0, g, unit0); break;
-        case 5: stream_tile<MODE, 5>(a, gsm, m0, g, unit0); break;
-        case 6: stream_tile<MODE, 6>(a, gsm, m0, g, unit0); break;
-        case 7: stream_tile<MODE, 7>(a, gsm, m0, g, unit0); break;
-        case 8: stream_tile<MODE, 8>(a, gsm, m0, g, unit0); break;
-        default: stream_tile<MODE, 9>(a, gsm, m0, g, unit0); break;
+        case 1: stream_tile<MODE, 1, FOLD>(a, gsm, m0, g, unit0); break;
+        case 2: stream_tile<MODE, 2, FOLD>(a, gsm, m0, g, unit0); break;
+        case 3: stream_tile<MODE, 3, FOLD>(a, gsm, m0, g, unit0); break;
+        case 4: stream_tile<MODE, 4, FOLD>(a, gsm, m0, g, unit0); break;
+        case 5: stream_tile<MODE, 5, FOLD>(a, gsm, m0, g, unit0); break;
+        case 6: stream_tile<MODE, 6, FOLD>(a, gsm, m0, g, unit0); break;
+        case 7: stream_tile<MODE, 7, FOLD>(a, gsm, m0, g, unit0); break;
+        case 8: stream_tile<MODE, 8, FOLD>(a, gsm, m0, g, unit0); break;
+        default: stream_tile<MODE, 9, FOLD>(a, gsm, m0, g, unit0); break;
       }
     }
   }
@@ -1204,7 +1220,14 @@ int gemm_stream_launch(GemmArgs a, hipStream_t st) {
   if (irc != MEP_OK) return irc;
   const int cus = mep_device_cu_count();
   a.width = (int)std::min<int64_t>((units + 7) / 8, std::max(cus > 0 ? cus / 8 : 32, 1));
-  hipLaunchKernelGGL((gemm_stream_kernel<MODE, KN>), dim3(8 * a.width * kSParts), dim3(kSThreads), kSLds, st, a);
+  const dim3 grid(8 * a.width * kSParts), threads(kSThreads);
+  if constexpr (!KN) {
+    if (mep_folds(a.K)) {
+      hipLaunchKernelGGL((gemm_stream_kernel<MODE, KN, true>), grid, threads, kSLds, st, a);
+      return mep_launch_status();
+    }
+  }
+  hipLaunchKernelGGL((gemm_stream_kernel<MODE, KN>), grid, threads, kSLds, st, a);
   return mep_launch_status();
 }
 
@@ -1414,6 +1437,8 @@ int mep_init_gemm_kernels() {
 #define MEP_OPT(k, b) if (rc == MEP_OK) rc = opt_in_lds(k, b)
   MEP_OPT((gemm_stream_kernel<kModeScale, false>), kSLds);
   MEP_OPT((gemm_stream_kernel<kModeSwiglu, false>), kSLds);
+  MEP_OPT((gemm_stream_kernel<kModeScale, false, true>), kSLds);
+  MEP_OPT((gemm_stream_kernel<kModeSwiglu, false, true>), kSLds);
   MEP_OPT((gemm_stream_kernel<kModeScale, true>), kSLds);
   MEP_OPT((gemm_stream_kernel<kModeDual, true>), kSLds);
   MEP_OPT((grouped_gemm_nt_kernel<kModeDual>), ring);
