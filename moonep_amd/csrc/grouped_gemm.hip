@@ -662,7 +662,8 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
 // 272 tiles for 256 CUs: a second round for sixteen of them) and the rows come from L2 once for up
 // to 288 weight rows.  A K step of 64 is 16 KB of rows and 4 KB a unit; the whole LDS holds D of
 // them, D - 1 on their way (72 KB of weights per CU at nine units) while one is multiplied.
-// 8 waves: 32 rows each, every other unit.  The waves 4 .. 7 run one barrier behind the waves 0 .. 3,
+// 8 waves: 32 rows each, every other unit.  In tiles of seven units and more (fewer have little to read in
+// a step: 2816 x 256 12.0 us that way, 11.6 in step) the waves 4 .. 7 run one barrier behind the waves 0 .. 3,
 // so that one wave of a SIMD multiplies while the other reads: a step's 160 to 192 KB of LDS reads
 // take about as long as its matrix instructions, and one after the other, with one barrier a step, the
 // two were 1.17 us a step of eight units and 1.33 of nine, however few of the CUs were still at work
@@ -684,7 +685,7 @@ __global__ __launch_bounds__(kPThreads, 2) void gemm_pp_kernel(GemmArgs a, Wgrad
 // The forward of 17 blocks on another card 211 -> 202 us with the epilogue's selects of two values and the row scales read
 // before the loads, of 18 232 -> 219, of 24 314 -> 298, 7168 x 2048 with 33 583 -> 558.  What a tile takes beside its
 // K steps now: 1.2 us to its group, 0.8 to the last of the first loads, 2 to 3 to their arrival, 1.4 (down) to 4 (SwiGLU) to store.
-// With the order of the K steps and the waves' two shifts, 64 tokens at 17 blocks: 190 -> 161.
+// With the order of the K steps and the waves' two shifts, 64 tokens at 17 blocks: 190 -> 161 and 170 -> 158 on two cards.
 // ---------------------------------------------------------------------------
 typedef float mep_f32x4_any __attribute__((ext_vector_type(4), aligned(4)));  // at any element
 constexpr int kSThreads = 512;
